@@ -5,10 +5,11 @@
 // from the request's state slot (or from zero when the request has no tokens behind it) and leaving the state there:
 // a prompt portion, the next portion and single decoded tokens all go through this one kernel.
 //
-// Two kernels: gla_col_kernel (key sizes up to 128: one state column per thread, see there) and gla_kernel for wider
-// states, where thread (part, v) keeps the state entries S[part + parts * i][v], i < DPT, in registers and the o_t
+// Steps that bring prompts run sixteen tokens at a time on the matrix cores (chunk_scan.h).  Single tokens and the sizes
+// that kernel does not serve walk token by token: gla_col_kernel (key sizes up to 128: one state column per thread, see
+// there) and gla_kernel for wider states, where thread (part, v) keeps the state entries S[part + parts * i][v], i < DPT, in registers and the o_t
 // column sums over the parts go through LDS.  The decay is evaluated as exp(log(sigmoid(z)) / tau) with log(sigmoid) in its stable form.
-#include "anyt.h"
+#include "chunk_scan.h"
 
 namespace {
 
@@ -260,12 +261,56 @@ extern "C" int nv_gla_recurrent(const float* proj, int64_t proj_row_stride, int 
                                 const int32_t* past_lens, const int32_t* state_slots, const void* norm_w, void* out,
                                 int num_seqs, int heads, int dim, int vdim, float tau, float q_scale, float eps,
                                 int dtype, nv_stream_t stream) {
+  return nv_gla_recurrent_batch(proj, proj_row_stride, q_off, k_off, v_off, g_off, z, z_row_stride, state, cu_q, past_lens,
+                                state_slots, norm_w, out, 0, num_seqs, heads, dim, vdim, tau, q_scale, eps, dtype, stream);
+}
+
+extern "C" int nv_gla_recurrent_batch(const float* proj, int64_t proj_row_stride, int q_off, int k_off, int v_off, int g_off,
+                                      const float* z, int64_t z_row_stride, float* state, const int32_t* cu_q,
+                                      const int32_t* past_lens, const int32_t* state_slots, const void* norm_w, void* out,
+                                      int64_t tokens, int num_seqs, int heads, int dim, int vdim, float tau, float q_scale,
+                                      float eps, int dtype, nv_stream_t stream) {
   NV_CHECK_ARG(proj && z && state && cu_q && past_lens && state_slots && norm_w && out, "nv_gla_recurrent: null pointer");
   NV_CHECK_ARG(dtype == NV_BF16 || dtype == NV_F32, "nv_gla_recurrent: bad dtype %d", dtype);
   NV_CHECK_ARG(heads > 0 && heads <= 65535 && dim > 0 && vdim > 0 && vdim <= 1024 && num_seqs >= 0 && num_seqs <= 65535,
                "nv_gla_recurrent: bad shape heads=%d dim=%d vdim=%d seqs=%d", heads, dim, vdim, num_seqs);
   NV_CHECK_ARG(tau > 0.0f, "nv_gla_recurrent: tau must be positive");
   if (num_seqs == 0) return NV_OK;
+  if (tokens > num_seqs) {     // somebody brings more than one token
+    chunk_scan::Args c{};
+    c.q = proj + q_off;
+    c.k = proj + k_off;
+    c.v = proj + v_off;
+    c.g = proj + g_off;
+    c.q_rs = c.k_rs = c.v_rs = c.g_rs = proj_row_stride;
+    c.s0 = z;
+    c.s_rs = z_row_stride;
+    c.w0 = norm_w;
+    c.state = state;
+    c.per_head = (int64_t)dim * vdim;
+    c.cu_q = cu_q;
+    c.past = past_lens;
+    c.slots = state_slots;
+    c.out = out;
+    c.out_rs = (int64_t)heads * vdim;
+    c.H = heads;
+    c.heads_per_group = 1;
+    c.dim = dim;
+    c.vdim = vdim;
+    c.q_scale = q_scale;
+    c.k_scale = 1.0f;
+    c.c0 = 1.0f / tau;
+    c.eps = eps;
+    if (chunk_scan::serves(c) && z_row_stride % 4 == 0 && (uintptr_t)z % 16 == 0) {
+      hipError_t e;
+      NV_DISPATCH_T(dtype, e = chunk_scan::launch<chunk_scan::GLA, T>(c, num_seqs, (hipStream_t)stream));
+      if (e != hipSuccess) {
+        nv_set_error("nv_gla_recurrent: %s", hipGetErrorString(e));
+        return NV_ERR_LAUNCH;
+      }
+      return NV_OK;
+    }
+  }
   if (dim <= 128) {     // one state column per thread (or per CS threads)
     int dmax = 16;
     while (dmax < dim) dmax *= 2;

@@ -624,9 +624,9 @@ def gla_recurrent(proj, offsets, z, state, cu_q, past_lens, state_slots, norm_w,
     assert cu_q.numel() == B + 1 and state_slots.numel() == B
     out = torch.empty(T, heads * vdim, dtype=norm_w.dtype, device=proj.device) if out is None else out
     q_off, k_off, v_off, g_off = offsets
-    check(lib().nv_gla_recurrent(ptr(proj), proj.stride(0), q_off, k_off, v_off, g_off, ptr(z), z.stride(0), ptr(state),
-                                 ptr(cu_q), ptr(past_lens), ptr(state_slots), ptr(norm_w), ptr(out), B, heads, dim, vdim,
-                                 tau, q_scale, eps, _code32(norm_w.dtype), stream()), "nv_gla_recurrent")
+    check(lib().nv_gla_recurrent_batch(ptr(proj), proj.stride(0), q_off, k_off, v_off, g_off, ptr(z), z.stride(0), ptr(state),
+                                       ptr(cu_q), ptr(past_lens), ptr(state_slots), ptr(norm_w), ptr(out), T, B, heads, dim,
+                                       vdim, tau, q_scale, eps, _code32(norm_w.dtype), stream()), "nv_gla_recurrent_batch")
     return out
 
 

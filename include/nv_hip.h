@@ -435,6 +435,13 @@ int nv_gla_recurrent(const float* proj, int64_t proj_row_stride, int q_off, int 
                      const float* z, int64_t z_row_stride, float* state, const int32_t* cu_q, const int32_t* past_lens,
                      const int32_t* state_slots, const void* norm_w, void* out, int num_seqs, int heads, int dim,
                      int vdim, float tau, float q_scale, float eps, int dtype, nv_stream_t stream);
+/* The same with the number of tokens of the whole step: with more than one per request they are worked on sixteen at a time on
+ * the matrix cores where the sizes and alignments allow it (csrc/chunk_scan.h). */
+int nv_gla_recurrent_batch(const float* proj, int64_t proj_row_stride, int q_off, int k_off, int v_off, int g_off,
+                           const float* z, int64_t z_row_stride, float* state, const int32_t* cu_q,
+                           const int32_t* past_lens, const int32_t* state_slots, const void* norm_w, void* out,
+                           int64_t tokens, int num_seqs, int heads, int dim, int vdim, float tau, float q_scale, float eps,
+                           int dtype, nv_stream_t stream);
 
 /* Matrix memories with one decay per head and token (csrc/memory.hip): S_t = keep_t S_(t-1) + take_t k_t v_t^T,
  * o_t = S_t^T q_t over this step's tokens of each request, state carried in fp32 slots of nv_matrix_memory_state_size
