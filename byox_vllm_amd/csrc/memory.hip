@@ -29,7 +29,7 @@
 //   S  <- decay^n S + sum_j decay^(n-1-j) k_j v_j^T,
 // so a chunk costs three short phases instead of C dependent steps.  Each power of the decay is formed on its own (no
 // quotients of powers: nothing overflows or cancels, however small the decay).
-#include "anyt.h"
+#include "chunk_scan.h"
 
 namespace {
 
@@ -715,6 +715,43 @@ extern "C" int nv_matrix_memory(const float* proj, int64_t proj_row_stride, int 
       return NV_ERR_LAUNCH;
     }
     return NV_OK;
+  }
+  // prompts in the gated form: sixteen tokens at a time (two tokens already cost the walk a whole staged chunk)
+  if (mode == MEM_EXPGATE && max_q > 1 && !silu && rot_dims == 0 && getenv("NV_MATRIX_MEMORY_STEPS") == nullptr &&
+      getenv("NV_MATRIX_MEMORY_GENERIC") == nullptr) {
+    chunk_scan::Args c{};
+    c.q = proj + q_off;
+    c.k = proj + k_off;
+    c.v = proj + v_off;
+    c.q_rs = c.k_rs = c.v_rs = c.s_rs = proj_row_stride;
+    c.s0 = proj + i_off;
+    c.s1 = proj + f_off;
+    const int item = dtype == NV_BF16 ? 2 : 4;
+    c.w0 = bias ? reinterpret_cast<const char*>(bias) + (int64_t)i_off * item : nullptr;
+    c.w1 = bias ? reinterpret_cast<const char*>(bias) + (int64_t)f_off * item : nullptr;
+    c.state = state;
+    c.per_head = p.per_head;
+    c.cu_q = cu_q;
+    c.past = past_lens;
+    c.slots = state_slots;
+    c.out = out;
+    c.out_rs = out_row_stride;
+    c.H = heads;
+    c.heads_per_group = 1;
+    c.dim = dim;
+    c.vdim = vdim;
+    c.q_scale = q_scale;
+    c.k_scale = k_scale;
+    c.c0 = cap;
+    if (chunk_scan::serves(c)) {
+      hipError_t e;
+      NV_DISPATCH_T(dtype, e = chunk_scan::launch<chunk_scan::EXPGATE, T>(c, num_seqs, (hipStream_t)stream));
+      if (e != hipSuccess) {
+        nv_set_error("nv_matrix_memory: %s", hipGetErrorString(e));
+        return NV_ERR_LAUNCH;
+      }
+      return NV_OK;
+    }
   }
   if (dmax > 256 || slices > 65535 || getenv("NV_MATRIX_MEMORY_GENERIC") != nullptr) {
     const size_t glds = ((size_t)2 * dim + 4 + 32) * sizeof(float);

@@ -153,4 +153,4 @@ class MLSTM(_MatrixMemoryMixer):
         return kernels.matrix_memory(proj, (self.at["q"], self.at["k"], self.at["v"]), state, ctx.cu_seqlens_q,
                                      ctx.past_lens, ctx.state_slots, self.heads, self.dim, self.vdim, self.mode,
                                      bias=self.inp.bias.data, gate_offsets=(self.at["i"], self.at["f"]),
-                                     cap=self.gate_cap, q_scale=self.dim ** -0.5)
+                                     cap=self.gate_cap, q_scale=self.dim ** -0.5, max_q=ctx.max_seqlen_q)

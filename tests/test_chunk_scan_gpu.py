@@ -89,3 +89,59 @@ def test_gated_linear_attention(H, d, dv, decay):
     check(lib().nv_gla_recurrent(ptr(p), p.stride(0), *offs, ptr(zz), zz.stride(0), ptr(dev2), *map(ptr, args), ptr(ww), ptr(out2),
                                  len(LENS), H, d, dv, tau, d ** -0.5, eps, 2, stream()), "nv_gla_recurrent")
     close(got, out2, "rows against the walk")
+
+
+@pytest.mark.parametrize("H,d,dv", [(2, 64, 128), (1, 128, 128), (3, 32, 64), (2, 20, 24), (1, 4, 4), (2, 100, 68), (1, 36, 128)])
+@pytest.mark.parametrize("forget", [4.0, 0.0, -30.0])
+def test_exponential_gates(H, d, dv, forget, monkeypatch):
+    from byox_vllm_amd import kernels
+    torch.manual_seed(H * 1000 + d + dv)
+    cu, past, slots = batch()
+    T, cap, copies = cu[-1], 15.0, -(-dv // 64)
+    cols = 2 * H * d + H * dv
+    proj, bias = torch.randn(T, cols + 2 * H + (-(cols + 2 * H)) % 4), torch.zeros(cols + 2 * H)
+    proj[:, cols:] *= 3.0
+    bias[cols:cols + H], bias[cols + H:] = -1.0, forget
+
+    def start():
+        n, m = torch.randn(H, d), torch.randn(H, 1)
+        return torch.cat([torch.randn(H, d * dv)] + [n, m] * copies, 1)
+    state = pool(cu, past, slots, (H, d * dv + copies * (d + 1)), start)
+    q, k, v = (proj[:, o:o + n].double().view(T, H, -1) for o, n in ((0, H * d), (H * d, H * d), (2 * H * d, H * dv)))
+    i, f = (cap * torch.tanh((proj[:, o:o + H] + bias[o:o + H]).double() / cap) for o in (cols, cols + H))
+    f = torch.nn.functional.logsigmoid(f)
+
+    def unpack(b, fresh):
+        if fresh:
+            return [torch.zeros(s, dtype=torch.float64) for s in ((H, d, dv), (H, d), (H,))]
+        s = state[slots[b]].double()
+        return [s[:, :d * dv].reshape(H, d, dv), s[:, d * dv:d * dv + d], s[:, d * dv + d]]
+
+    def step(s, t):
+        S, n, m = s
+        top = torch.maximum(f[t] + m, i[t])
+        keep, take = torch.exp(f[t] + m - top), torch.exp(i[t] - top)
+        S = S * keep[:, None, None] + take[:, None, None] * k[t][..., None] * v[t][:, None]
+        n = n * keep[:, None] + take[:, None] * k[t]
+        below = torch.maximum((n * q[t]).sum(-1).abs() * d ** -0.5, torch.exp(-top)) + 1e-6
+        # a sum n . q that nearly cancels is divided by: its terms' errors come out enlarged
+        magnified[t] = ((n * q[t]).abs().sum(-1) * d ** -0.5 / below).clamp_min(1.0)
+        return [S, n, top], ((S * q[t][..., None]).sum(1) * d ** -0.5 / below[:, None]).reshape(-1)
+    magnified = torch.ones(T, H, dtype=torch.float64)
+    want, ends = walk(cu, past, unpack, step, H * dv)
+    ends = torch.stack([torch.cat([S.reshape(H, -1)] + [n, m[:, None]] * copies, 1) for S, n, m in ends])
+
+    def run():
+        dev = state.to(DEV)
+        out = kernels.matrix_memory(proj.to(DEV), (0, H * d, 2 * H * d), dev, i32(cu), i32(past), i32(slots), H, d, dv,
+                                    kernels.MEM_EXPGATE, bias=bias.to(DEV), gate_offsets=(cols, cols + H), cap=cap,
+                                    q_scale=d ** -0.5, max_q=max(LENS))
+        return out, torch.stack([dev[s] for s in slots])
+    got, state_got = run()
+    monkeypatch.setenv("NV_MATRIX_MEMORY_STEPS", "1")
+    steps, state_steps = run()
+    magnified = magnified.repeat_interleave(dv, 1)
+    close(got, want, "rows", magnified)
+    close(got, steps, "rows against the walk", magnified)
+    close(state_got, ends, "states")
+    close(state_got, state_steps, "states against the walk")
