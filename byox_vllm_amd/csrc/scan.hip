@@ -10,7 +10,7 @@
 //               out = S * silu(g): the minimal gated recurrent unit, whose gates read the current token only.
 // ssd_scan:     per head, S [N, P]:  S = exp(-exp(A_log) dt) S + dt B x^T,  y = S^T C + D x,  dt = softplus(raw + bias);
 //               out = y * silu(z): the selective state-space recurrence of Mamba-2 in its token-by-token form.
-#include "anyt.h"
+#include "chunk_scan.h"
 
 namespace {
 
@@ -569,6 +569,46 @@ extern "C" int nv_ssd_scan(const float* xbc, int64_t xbc_row_stride, const float
   }
   float* ws_state = reinterpret_cast<float*>(workspace);
   float* ws_decay = runs > 1 ? ws_state + (size_t)num_seqs * heads * runs * state_size * vdim : nullptr;
+  if (max_q > 1) {
+    chunk_scan::Args c{};
+    const int inner = heads * vdim;
+    c.q = xbc + inner + groups * state_size;
+    c.k = xbc + inner;
+    c.v = xbc;
+    c.g = z;
+    c.q_rs = c.k_rs = c.v_rs = xbc_row_stride;
+    c.g_rs = z_row_stride;
+    c.s0 = dt;
+    c.s_rs = dt_row_stride;
+    c.w0 = dt_bias;
+    c.w1 = A_log;
+    c.w2 = D;
+    c.state = state;
+    c.per_head = (int64_t)state_size * vdim;
+    c.cu_q = cu_q;
+    c.past = past_lens;
+    c.slots = state_slots;
+    c.out = out;
+    c.out_rs = inner;
+    c.H = heads;
+    c.heads_per_group = heads / groups;
+    c.dim = state_size;
+    c.vdim = vdim;
+    c.q_scale = c.k_scale = 1.0f;
+    c.ws_state = ws_state;
+    c.ws_decay = ws_decay;
+    c.runs = runs;
+    c.run_len = run_len;
+    if (chunk_scan::serves(c)) {
+      hipError_t e;
+      NV_DISPATCH_T(dtype, e = chunk_scan::launch_ssd<T>(c, num_seqs, (hipStream_t)stream));
+      if (e != hipSuccess) {
+        nv_set_error("nv_ssd_scan: %s", hipGetErrorString(e));
+        return NV_ERR_LAUNCH;
+      }
+      return NV_OK;
+    }
+  }
   SsdArgs p{xbc, xbc_row_stride, z, z_row_stride, dt, dt_row_stride, dt_bias, A_log, D, state, cu_q, past_lens,
             state_slots, out, heads, groups, state_size, vdim, parts, ws_state, ws_decay, runs, run_len, 1};
   const int threads = ((parts * vdim + 63) / 64) * 64;

@@ -145,3 +145,57 @@ def test_exponential_gates(H, d, dv, forget, monkeypatch):
     close(got, steps, "rows against the walk", magnified)
     close(state_got, ends, "states")
     close(state_got, state_steps, "states against the walk")
+
+
+@pytest.mark.parametrize("H,G,n,dv", [(4, 1, 128, 64), (4, 2, 64, 64), (2, 2, 16, 128), (2, 1, 20, 24), (6, 3, 4, 4), (2, 1, 100, 68)])
+@pytest.mark.parametrize("scale", [0.1, 3.0, 100.0])
+def test_state_space(H, G, n, dv, scale):
+    from byox_vllm_amd import kernels
+    torch.manual_seed(H * 1000 + n + dv)
+    cu, past, slots = batch()
+    T, inner = cu[-1], H * dv
+    xbc, z, dt = torch.randn(T, inner + 2 * G * n), torch.randn(T, inner), torch.randn(T, H)
+    dt_bias, A_log, D = torch.randn(H), torch.randn(H) + torch.tensor(scale).log(), torch.randn(H)
+    state = pool(cu, past, slots, (H, n, dv), lambda: torch.randn(H, n, dv))
+    x = xbc[:, :inner].double().view(T, H, dv)
+    B, C = (xbc[:, inner + o:inner + o + G * n].double().view(T, G, n).repeat_interleave(H // G, 1) for o in (0, G * n))
+    step_size = torch.nn.functional.softplus(dt.double() + dt_bias.double())
+    keep = torch.exp(-torch.exp(A_log.double()) * step_size)
+
+    def step(S, t):
+        S = S * keep[t][:, None, None] + (step_size[t][:, None] * B[t])[..., None] * x[t][:, None]
+        y = ((S * C[t][..., None]).sum(1) + D.double()[:, None] * x[t]).reshape(-1)
+        return S, y * torch.nn.functional.silu(z[t].double())
+    want, ends = walk(cu, past, lambda b, fresh: torch.zeros(H, n, dv, dtype=torch.float64) if fresh else state[slots[b]].double(),
+                      step, inner)
+    runs = []
+    for max_q in (max(LENS), 1):            # chunks; the walk
+        dev = state.to(DEV)
+        out = kernels.ssd_scan(xbc.to(DEV), z.to(DEV), dt.to(DEV), dt_bias.to(DEV), A_log.to(DEV), D.to(DEV), dev, i32(cu),
+                               i32(past), i32(slots), H, G, n, dv, max_q=max_q)
+        runs.append((out, torch.stack([dev[s] for s in slots])))
+    close(runs[0][0], want, "rows")
+    close(runs[0][1], torch.stack(ends), "states")
+    close(runs[0][0], runs[1][0], "rows against the walk")
+
+
+@pytest.mark.parametrize("lens,past", [([256], [0]), ([257, 3], [5, 0]), ([511, 128, 129, 1], [0, 9, 0, 4])])
+def test_state_space_runs(lens, past):
+    """Few requests with long prompts: runs side by side against one walk over the same tokens."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(sum(lens))
+    H, G, n, dv = 2, 1, 64, 64
+    cu = [0]
+    for m in lens:
+        cu.append(cu[-1] + m)
+    T, inner = cu[-1], H * dv
+    data = [torch.randn(s, device=DEV) for s in ((T, inner + 2 * G * n), (T, inner), (T, H), (H,), (H,), (H,))]
+    data[4] = data[4] - 2.0
+    state = torch.randn(len(lens), H, n, dv, device=DEV)
+    runs = []
+    for max_q in (max(lens), 1):
+        dev = state.clone()
+        out = kernels.ssd_scan(*data, dev, i32(cu), i32(past), i32(list(range(len(lens)))), H, G, n, dv, max_q=max_q)
+        runs.append((out, dev))
+    close(runs[0][0], runs[1][0], "rows")
+    close(runs[0][1], runs[1][1], "states")
