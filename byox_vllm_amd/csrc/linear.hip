@@ -473,6 +473,8 @@ int launch_epi(const LinArgs& p, int epi, dim3 grid, hipStream_t s) {
   return 0;
 }
 
+#include "linear_wide.h"
+
 }  // namespace
 
 extern "C" int nv_linear(const void* a, int64_t a_row_stride, const int32_t* a_rows, const void* w, int64_t w_row_stride,
@@ -490,6 +492,18 @@ extern "C" int nv_linear_scaled(const void* a, int64_t a_row_stride, const int32
                          int batch, int64_t a_batch_stride, int64_t w_batch_stride, int64_t out_batch_stride,
                          int64_t bias_batch_stride, const int32_t* group_offsets, int epilogue, int act,
                          const float* epi_ptr, int64_t epi_row_stride, float epi_const, const float* row_scale, int dtype,
+                         nv_stream_t stream) {
+  return nv_linear_rows(a, a_row_stride, a_rows, w, w_row_stride, bias, out, out_row_stride, out_dtype, M, N, K, batch,
+                        a_batch_stride, w_batch_stride, out_batch_stride, bias_batch_stride, group_offsets, epilogue, act,
+                        epi_ptr, epi_row_stride, epi_const, row_scale, group_offsets ? M * batch : M, dtype, stream);
+}
+
+extern "C" int nv_linear_rows(const void* a, int64_t a_row_stride, const int32_t* a_rows, const void* w, int64_t w_row_stride,
+                         const void* bias, void* out, int64_t out_row_stride, int out_dtype, int64_t M, int N, int K,
+                         int batch, int64_t a_batch_stride, int64_t w_batch_stride, int64_t out_batch_stride,
+                         int64_t bias_batch_stride, const int32_t* group_offsets, int epilogue, int act,
+                         const float* epi_ptr, int64_t epi_row_stride, float epi_const, const float* row_scale,
+                         int64_t total_rows, int dtype,
                          nv_stream_t stream) {
   NV_CHECK_ARG(a && w && out, "nv_linear: null pointer");
   NV_CHECK_ARG(dtype == NV_BF16 || dtype == NV_F32, "nv_linear: dtype %d is neither bf16 nor fp32", dtype);
@@ -512,6 +526,27 @@ extern "C" int nv_linear_scaled(const void* a, int64_t a_row_stride, const int32
   p.vec_w = (uintptr_t)w % 16 == 0 && w_row_stride % per == 0 && (w_batch_stride * esz) % 16 == 0;
   dim3 grid((unsigned)((N + 63) / 64), (unsigned)mtiles, (unsigned)batch);
   hipStream_t s = (hipStream_t)stream;
+  // more than 64 rows that split into K blocks of 128 bytes: the wide tiles
+  if (M > 64 && p.vec_a && p.vec_w && (K * esz) % 128 == 0 && getenv("NV_LINEAR_TILE_OFF") == nullptr) {
+    const int cols = epilogue == EPI_GLU ? 2 * N : N;
+    int tile = pick_wide_tile(M, total_rows, cols, batch, group_offsets != nullptr, dtype == NV_BF16);
+    if (const char* force = getenv("NV_LINEAR_TILE")) tile = atoi(force);
+    if (wide_tiles(64, 128, M, total_rows + 64 * batch, cols, batch, group_offsets != nullptr) < (1 << 30)) {
+      hipError_t e;
+      if (dtype == NV_BF16) {
+        e = out_dtype == NV_BF16 ? launch_wide<bf16_t, bf16_t>(p, epilogue, total_rows, batch, tile, s)
+                                 : launch_wide<bf16_t, float>(p, epilogue, total_rows, batch, tile, s);
+      } else {
+        e = out_dtype == NV_BF16 ? launch_wide<float, bf16_t>(p, epilogue, total_rows, batch, tile, s)
+                                 : launch_wide<float, float>(p, epilogue, total_rows, batch, tile, s);
+      }
+      if (e != hipSuccess) {
+        nv_set_error("nv_linear: %s", hipGetErrorString(e));
+        return NV_ERR_LAUNCH;
+      }
+      return NV_OK;
+    }
+  }
   // more than 64 rows of 16-byte-aligned bf16: the LDS-tiled kernel (a group's rows are not known here: M bounds them)
   if (dtype == NV_BF16 && M > 64 && p.vec_a && p.vec_w && K % 8 == 0 && getenv("NV_LINEAR_TILE_OFF") == nullptr) {
     if (out_dtype == NV_BF16) launch_tile<bf16_t>(p, epilogue, batch, s);

@@ -1,0 +1,303 @@
+// nv_linear for many rows: tiles of BM x BN outputs with both operands in LDS, filled by LDS-DMA.  Included by linear.hip.
+//
+// What bounds it: at 2048 rows per expert the products are 2 x 128 flops per byte that a 256 x 256 tile moves, so the matrix
+// cores; the kernel it replaces there (128 x 128 tiles, K in blocks of 32 through registers) reached a quarter of their
+// rate, waiting at a barrier every 16 matrix instructions.  Here
+//   * a K block is 128 bytes of every row (64 bf16, 32 fp32): 64 matrix instructions per wavefront and barrier at 256 x 256;
+//   * the following blocks' rows go from L2 straight into the other LDS buffers (global_load_lds, 16 bytes per lane) while a
+//     block is multiplied; no staging registers, no LDS store instructions.  Two buffers fit beside 256 x 256 outputs; the
+//     smaller tiles have three, because there a block is multiplied faster than one arrives;
+//   * LDS rows are 128 bytes apart and their 16-byte pieces are dealt by XOR with half the row number, through the DMA's
+//     source addresses, so the 16 rows that one read phase touches lie in 16 different bank groups;
+//   * fragments of the next step of K are read while the current step's matrix instructions run (two register sets);
+//   * workgroups that share operands run on one XCD: tile numbers are dealt to the XCDs in contiguous eighths.
+// Groups (experts) of unknown size: the grid covers the largest possible number of tiles, every workgroup finds its group
+// from the offsets with one wavefront-wide prefix sum, and the surplus leaves at once.
+#pragma once
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// value(s) of one output -> what is stored (bias, activation, gate)
+template <typename T, int EPI>
+__device__ __forceinline__ float lin_finish(const LinArgs& p, const T* bias, float v, float u, float rsc, int64_t s, int n, int z) {
+  v *= rsc;
+  if (bias) v += ld_f32<T>(bias + n);
+  if constexpr (EPI == EPI_GLU) {
+    u *= rsc;
+    if (bias) u += ld_f32<T>(bias + p.N + n);
+    v = glu_act(v, u, p.act, p.epi_c);
+  } else if constexpr (EPI == EPI_SOFTCAP) {
+    v = p.epi_c * tanhf(v / p.epi_c);
+  } else if constexpr (EPI == EPI_ROW_GATE) {
+    v *= sigmoid_f32(p.epi_ptr[s * p.epi_rs + (p.act ? (int64_t)z * p.N + n : z)]);
+  } else if constexpr (EPI == EPI_ACT) {
+    v = unary_act(v, p.act, p.epi_ptr, p.epi_c);
+  }
+  return v;
+}
+
+__device__ __forceinline__ f32x16 mma32(const u32x4& a, const u32x4& b, f32x16 c, bf16_t) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x16 mma32(const u32x4& a, const u32x4& b, f32x16 c, float) {
+  // step m takes number 4 half + m of the eight that the two half-wavefronts hold
+#pragma unroll
+  for (int m = 0; m < 4; ++m) c = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[m]), __uint_as_float(b[m]), c, 0, 0, 0);
+  return c;
+}
+
+// MT x 2 tiles of 32 x 32 per wavefront, WM wavefronts along the rows, WN along the columns
+template <typename T, typename TO, int EPI, int MT, int WM, int WN, int STAGES>
+__global__ __launch_bounds__(64 * WM * WN, 2) void linear_wide_kernel(LinArgs p, int mt_max, int nt_all) {
+  constexpr bool GLU = EPI == EPI_GLU;
+  constexpr int NW = WM * WN, BM = 32 * MT * WM, BN = 64 * WN, NOUT = GLU ? BN / 2 : BN;
+  constexpr int PER = 16 / sizeof(T), BK = 8 * PER;                 // numbers per 16-byte piece; per K block
+  constexpr int AG = BM / 8 / NW, WG = BN / 8 / NW;                 // DMA instructions (8 rows each) per wavefront
+  static_assert(AG >= 1 && WG >= 1 && AG * 8 * NW == BM && WG * 8 * NW == BN, "the tile splits into whole DMA instructions");
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wv % WM, wn = wv / WM;
+
+  // -------- which tile
+  int z = blockIdx.z, n_tile, m_tile;
+  int64_t lo = 0, hi = p.M;
+  {
+    int tile = blockIdx.x;
+    if (p.group_off) {
+      const int groups = mt_max;       // grouped: the number of groups
+      int real = 0;
+      for (int base = 0; base < groups; base += 64) {
+        const int g = base + lane;
+        int mt = g < groups ? (p.group_off[g + 1] - p.group_off[g] + BM - 1) / BM : 0;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) mt += __shfl_xor(mt, o, 64);
+        real += mt;
+      }
+      real = __builtin_amdgcn_readfirstlane(real) * nt_all;
+      const int share = (real + 7) / 8, slot = tile >> 3;
+      tile = (tile & 7) * share + slot;
+      if (slot >= share || tile >= real) return;
+      int before = 0;
+      z = -1;
+      for (int base = 0; base < groups && z < 0; base += 64) {
+        const int g = base + lane;
+        const int mine = g < groups ? (p.group_off[g + 1] - p.group_off[g] + BM - 1) / BM : 0;
+        int upto = mine;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const int x = __shfl_up(upto, o, 64);
+          if (lane >= o) upto += x;
+        }
+        const uint64_t hit = __ballot(tile < (before + upto) * nt_all);
+        if (hit) {
+          const int l = __ffsll((unsigned long long)hit) - 1;
+          z = base + l;
+          const int count = __builtin_amdgcn_readlane(mine, l);
+          const int local = tile - (before + __builtin_amdgcn_readlane(upto, l) - count) * nt_all;
+          m_tile = local % count;
+          n_tile = local / count;
+        } else {
+          before += __builtin_amdgcn_readlane(upto, 63);
+        }
+      }
+      lo = p.group_off[z];
+      hi = p.group_off[z + 1];
+    } else {
+      const int real = mt_max * nt_all, share = (real + 7) / 8, slot = tile >> 3;
+      tile = (tile & 7) * share + slot;
+      if (slot >= share || tile >= real) return;
+      m_tile = tile % mt_max;
+      n_tile = tile / mt_max;
+    }
+  }
+  const int64_t mbase = lo + (int64_t)m_tile * BM;
+  const int n0 = n_tile * NOUT;
+  const T* A = reinterpret_cast<const T*>(p.a) + z * p.a_bs;
+  const T* W = reinterpret_cast<const T*>(p.w) + z * p.w_bs;
+
+  // -------- DMA: instruction i of this wavefront fills rows 8 (wv + NW i) .. + 7; lane l the piece l & 7 of row l >> 3
+  const int dr = lane >> 3, dp = lane & 7;
+  const T* ap[AG];
+  const T* wp[WG];
+#pragma unroll
+  for (int i = 0; i < AG; ++i) {
+    const int r = 8 * (wv + NW * i) + dr;
+    int64_t s = mbase + r;
+    if (s >= hi) s = hi - 1;                                        // rows past the end repeat the last one
+    ap[i] = A + (int64_t)(p.a_rows ? p.a_rows[s] : s) * p.a_rs + PER * (dp ^ ((r >> 1) & 7));
+  }
+#pragma unroll
+  for (int i = 0; i < WG; ++i) {
+    const int r = 8 * (wv + NW * i) + dr;
+    int row;
+    if constexpr (GLU) row = r < BN / 2 ? min(n0 + r, p.N - 1) : p.N + min(n0 + r - BN / 2, p.N - 1);
+    else row = min(n0 + r, p.N - 1);
+    wp[i] = W + (int64_t)row * p.w_rs + PER * (dp ^ ((r >> 1) & 7));
+  }
+  typedef __attribute__((address_space(1))) void global_void;
+  typedef __attribute__((address_space(3))) void lds_void;
+  auto fill = [&](int buf) {
+    unsigned char* b = lds_raw + buf * (BM + BN) * 128;
+#pragma unroll
+    for (int i = 0; i < AG; ++i) {
+      __builtin_amdgcn_global_load_lds((global_void*)ap[i], (lds_void*)(b + (wv + NW * i) * 1024), 16, 0, 0);
+      ap[i] += BK;
+    }
+#pragma unroll
+    for (int i = 0; i < WG; ++i) {
+      __builtin_amdgcn_global_load_lds((global_void*)wp[i], (lds_void*)(b + BM * 128 + (wv + NW * i) * 1024), 16, 0, 0);
+      wp[i] += BK;
+    }
+  };
+
+  const int fr = lane & 31, fh = lane >> 5;
+  int a_row[MT], w_row[2];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) a_row[i] = 32 * (MT * wm + i) + fr;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) w_row[j] = BM + (GLU ? (BN / 2) * j + 32 * wn : 64 * wn + 32 * j) + fr;
+  const int sw = (fr >> 1) & 7;                                     // every tile starts at a multiple of 32 rows
+  auto piece = [&](const unsigned char* b, int row, int step) {
+    return *reinterpret_cast<const u32x4*>(b + row * 128 + (((2 * step + fh) ^ sw) << 4));
+  };
+
+  f32x16 acc[2][MT];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[j][i][r] = 0.0f;
+
+  const int blocks = p.K / BK;
+#pragma unroll
+  for (int i = 0; i < STAGES - 1; ++i)
+    if (i < blocks) fill(i);
+  int buf = 0;
+  for (int t = 0; t < blocks; ++t) {
+    // this wavefront's part of block t has arrived (later blocks may still be on their way), then everybody's has; the
+    // barrier also says that block t - 1 is no longer read
+    if (STAGES > 2 && t + 1 < blocks) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 2) * (AG + WG)) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (t + STAGES - 1 < blocks) fill(buf == 0 ? STAGES - 1 : buf - 1);
+    const unsigned char* b = lds_raw + buf * (BM + BN) * 128;
+    buf = buf + 1 == STAGES ? 0 : buf + 1;
+    u32x4 wf[2][2], af[2][MT];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) wf[0][j] = piece(b, w_row[j], 0);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) af[0][i] = piece(b, a_row[i], 0);
+#pragma unroll
+    for (int step = 0; step < 4; ++step) {
+      const int cur = step & 1, nxt = cur ^ 1;
+      if (step < 3) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) wf[nxt][j] = piece(b, w_row[j], step + 1);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) af[nxt][i] = piece(b, a_row[i], step + 1);
+      }
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[j][i] = mma32(wf[cur][j], af[cur][i], acc[j][i], T{});
+      // one fragment of the next step is requested behind each of this step's first products; left alone, the compiler
+      // puts the reads right before their use
+      if constexpr (sizeof(T) == 2) {
+#pragma unroll
+        for (int i = 0; i < 2 * MT; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          if (step < 3 && i < MT + 2) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+      }
+    }
+  }
+
+  // -------- results: lane holds row fr of each row tile, columns 8 g + 4 fh + r of each column tile
+  TO* O = reinterpret_cast<TO*>(p.out) + z * p.out_bs;
+  const T* bias = p.bias ? reinterpret_cast<const T*>(p.bias) + z * p.bias_bs : nullptr;
+  typedef typename Pack4<TO>::type P4;
+  const bool vec = p.N % 4 == 0 && p.out_rs % 4 == 0 && p.out_bs % 4 == 0 && (uintptr_t)p.out % 16 == 0;
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const int64_t s = mbase + 32 * (MT * wm + i) + fr;
+    if (s >= hi) continue;
+    const float rsc = p.row_scale ? p.row_scale[s] : 1.0f;
+#pragma unroll
+    for (int j = 0; j < (GLU ? 1 : 2); ++j) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int n = n0 + (GLU ? 32 * wn : 64 * wn + 32 * j) + 8 * g + 4 * fh;
+        if (n >= p.N) continue;
+        f32x4 v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          v[r] = n + r < p.N ? lin_finish<T, EPI>(p, bias, acc[j][i][4 * g + r], GLU ? acc[1][i][4 * g + r] : 0.0f, rsc, s, n + r, z)
+                             : 0.0f;
+        TO* o = O + s * p.out_rs + n;
+        if (vec) {
+          *reinterpret_cast<P4*>(o) = Pack4<TO>::narrow(v);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (n + r < p.N) st_f32<TO>(o + r, v[r]);
+        }
+      }
+    }
+  }
+}
+
+template <typename T, typename TO, int EPI, int MT, int WM, int WN, int STAGES>
+hipError_t launch_wide_one(const LinArgs& p, int64_t total_rows, int batch, hipStream_t s) {
+  constexpr int BM = 32 * MT * WM, BN = 64 * WN, NOUT = EPI == EPI_GLU ? BN / 2 : BN;
+  constexpr size_t lds = STAGES * (size_t)(BM + BN) * 128;
+  if (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&linear_wide_kernel<T, TO, EPI, MT, WM, WN, STAGES>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  const int64_t nt = (p.N + NOUT - 1) / NOUT;
+  const int64_t mt = p.group_off ? total_rows / BM + batch : (p.M + BM - 1) / BM;      // at most this many row tiles
+  const dim3 grid((unsigned)((mt * nt + 7) / 8 * 8), 1, p.group_off ? 1 : batch);
+  linear_wide_kernel<T, TO, EPI, MT, WM, WN, STAGES><<<grid, dim3(64 * WM * WN), lds, s>>>(p, p.group_off ? batch : (int)mt, (int)nt);
+  return hipGetLastError();
+}
+
+// Which tile: the one whose launch takes the fewest chip-wide rounds of tile area, each by what it reaches when the chip is
+// full (bf16, 32768 rows by 6144 columns of K 2048 in 16 groups: 917, 742 and 608 TFLOP/s; a workgroup of 256 x 256 has a CU
+// to itself, of the others two share one).  fp32 has the two smaller ones: its slower matrix instructions hide the loads.
+enum { TILE_256 = 2, TILE_128 = 1, TILE_64 = 0 };
+inline int64_t wide_tiles(int bm, int bn, int64_t m, int64_t total_rows, int cols, int batch, bool grouped) {
+  // groups end inside a tile: half a tile each on average
+  return (grouped ? (total_rows + bm - 1) / bm + batch / 2 : (m + bm - 1) / bm * batch) * ((cols + bn - 1) / bn);
+}
+inline int pick_wide_tile(int64_t m, int64_t total_rows, int cols, int batch, bool grouped, bool has_256) {
+  auto cost = [&](int bm, int bn, int per_cu, double reached) {
+    const int64_t slots = 256 * per_cu, rounds = (wide_tiles(bm, bn, m, total_rows, cols, batch, grouped) + slots - 1) / slots;
+    return (double)rounds * per_cu * bm * bn / reached;
+  };
+  const double c64 = cost(64, 128, 2, 608), c128 = cost(128, 128, 2, 742), c256 = cost(256, 256, 1, 917);
+  if (has_256 && c256 < c128 && c256 < c64) return TILE_256;
+  return c128 < c64 ? TILE_128 : TILE_64;
+}
+
+template <typename T, typename TO, int EPI>
+hipError_t launch_wide_epi(const LinArgs& p, int64_t total_rows, int batch, int tile, hipStream_t s) {
+  if constexpr (sizeof(T) == 2) {
+    if (tile == TILE_256) return launch_wide_one<T, TO, EPI, 4, 2, 4, 2>(p, total_rows, batch, s);
+  }
+  if (tile == TILE_128) return launch_wide_one<T, TO, EPI, 2, 2, 2, 2>(p, total_rows, batch, s);
+  return launch_wide_one<T, TO, EPI, 1, 2, 2, 3>(p, total_rows, batch, s);
+}
+
+template <typename T, typename TO>
+hipError_t launch_wide(const LinArgs& p, int epi, int64_t total_rows, int batch, int tile, hipStream_t s) {
+  switch (epi) {
+    case EPI_NONE: return launch_wide_epi<T, TO, EPI_NONE>(p, total_rows, batch, tile, s);
+    case EPI_GLU: return launch_wide_epi<T, TO, EPI_GLU>(p, total_rows, batch, tile, s);
+    case EPI_SOFTCAP: return launch_wide_epi<T, TO, EPI_SOFTCAP>(p, total_rows, batch, tile, s);
+    case EPI_ACT: return launch_wide_epi<T, TO, EPI_ACT>(p, total_rows, batch, tile, s);
+    default: return launch_wide_epi<T, TO, EPI_ROW_GATE>(p, total_rows, batch, tile, s);
+  }
+}

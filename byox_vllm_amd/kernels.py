@@ -506,10 +506,10 @@ def linear(x, w, bias=None, out=None, out_dtype=None, *, rows=None, a_rows=None,
     if a_rows is not None:
         assert a_rows.dtype == torch.int32
     bias_stride = n * (2 if epilogue == EPI_GLU else 1) if bias is not None and batch > 1 else 0
-    check(lib().nv_linear_scaled(ptr(x), x.stride(0), ptr(a_rows), ptr(w), w.stride(-2), ptr(bias), ptr(out), out.stride(0),
-                                 _code32(out_dtype), grid_rows, n, K, batch, a_batch_stride, w_batch_stride,
-                                 out_batch_stride, bias_stride, ptr(group_offsets), epilogue, act, ptr(gate), gate_stride,
-                                 cap, ptr(row_scale), _code32(x.dtype), stream()), "nv_linear_scaled")
+    check(lib().nv_linear_rows(ptr(x), x.stride(0), ptr(a_rows), ptr(w), w.stride(-2), ptr(bias), ptr(out), out.stride(0),
+                               _code32(out_dtype), grid_rows, n, K, batch, a_batch_stride, w_batch_stride,
+                               out_batch_stride, bias_stride, ptr(group_offsets), epilogue, act, ptr(gate), gate_stride,
+                               cap, ptr(row_scale), M, _code32(x.dtype), stream()), "nv_linear_rows")
     return out
 
 

@@ -359,6 +359,13 @@ int nv_linear_scaled(const void* a, int64_t a_row_stride, const int32_t* a_rows,
                      int64_t a_batch_stride, int64_t w_batch_stride, int64_t out_batch_stride, int64_t bias_batch_stride,
                      const int32_t* group_offsets, int epilogue, int act, const float* epi_ptr, int64_t epi_row_stride,
                      float epi_const, const float* row_scale, int dtype, nv_stream_t stream);
+/* ... with the number of output rows of all groups together (grouped products; M bounds one group's): the grid then covers
+ * total_rows instead of M rows for every group. */
+int nv_linear_rows(const void* a, int64_t a_row_stride, const int32_t* a_rows, const void* w, int64_t w_row_stride,
+                   const void* bias, void* out, int64_t out_row_stride, int out_dtype, int64_t M, int N, int K, int batch,
+                   int64_t a_batch_stride, int64_t w_batch_stride, int64_t out_batch_stride, int64_t bias_batch_stride,
+                   const int32_t* group_offsets, int epilogue, int act, const float* epi_ptr, int64_t epi_row_stride,
+                   float epi_const, const float* row_scale, int64_t total_rows, int dtype, nv_stream_t stream);
 
 /* out[t] = table[ids[t]] * scale as fp32 rows (the residual stream's first value). */
 int nv_embed_scale(const int64_t* ids, const void* table, float* out, int64_t tokens, int width, int64_t vocab,

@@ -1,0 +1,85 @@
+"""nv_linear's wide tiles (csrc/linear_wide.h) at the edges of their row, column and K tiles, in every tile size, against
+float64; groups that are empty, end on a tile and end inside one; and K sizes the tiles leave to the other kernels."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def close(got, want, K, dtype, out_dtype):
+    # fp32 accumulation of K products that are exact (16-bit operands) or rounded once (fp32), then one rounding
+    tol = K * 2.0 ** -24 + (2.0 ** -8 if out_dtype == torch.bfloat16 else 2.0 ** -22)
+    got, want = got.double().cpu(), want.double().cpu()
+    scale = want.pow(2).mean().sqrt()
+    off = ((got - want).abs() / torch.maximum(scale, want.abs())).max()
+    assert torch.isfinite(got).all() and off < tol, f"off by {off:.3g}, {tol:.3g} allowed"
+
+
+@pytest.mark.parametrize("tile", ["0", "1", "2", None])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K", [(65, 4, 64), (129, 127, 128), (255, 130, 192), (256, 256, 64), (300, 513, 320), (200, 96, 96),
+                                   (90, 61, 40)])
+def test_edges(M, N, K, dtype, tile, monkeypatch):
+    from byox_vllm_amd import kernels
+    if tile is not None:
+        monkeypatch.setenv("NV_LINEAR_TILE", tile)
+    torch.manual_seed(M + N + K)
+    x, w = torch.randn(M, K + 8).to(dtype)[:, :K], torch.randn(N, K).to(dtype) * 0.1
+    b = torch.randn(N).to(dtype)
+    want = x.double() @ w.double().t() + b.double()
+    for out_dtype in (dtype, torch.float32):
+        got = kernels.linear(x.to(DEV), w.to(DEV), b.to(DEV), out_dtype=out_dtype)
+        close(got, want, K, dtype, out_dtype)
+    wide = torch.zeros(M, N + 3, dtype=torch.float32, device=DEV)         # rows that do not split into 16-byte pieces
+    kernels.linear(x.to(DEV), w.to(DEV), b.to(DEV), out=wide[:, :N], out_dtype=torch.float32)
+    close(wide[:, :N], want, K, dtype, torch.float32)
+    assert not wide[:, N:].any()
+
+
+@pytest.mark.parametrize("tile", ["0", "1", "2", None])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("sizes,N,K", [([0, 128, 1, 0, 257, 64, 0], 68, 64), ([300], 256, 128), ([5] * 70, 36, 64),
+                                       ([0, 0, 256, 256, 3], 130, 192)])
+def test_groups(sizes, N, K, dtype, tile, monkeypatch):
+    from byox_vllm_amd import kernels
+    if tile is not None:
+        monkeypatch.setenv("NV_LINEAR_TILE", tile)
+    torch.manual_seed(sum(sizes) + N)
+    E, rows, T = len(sizes), sum(sizes), 90
+    off = torch.tensor([0] + list(torch.tensor(sizes).cumsum(0)), dtype=torch.int32)
+    x = torch.randn(T, K).to(dtype)
+    token = torch.randint(0, T, (rows,), dtype=torch.int32)
+    gu, scale = torch.randn(E, 2 * N, K).to(dtype) * 0.1, torch.rand(rows) + 0.5
+    d = lambda t: t.to(DEV)  # noqa: E731
+    args = dict(rows=rows, a_rows=d(token), batch=E, group_offsets=d(off), max_group_rows=max(65, max(sizes)))
+    hidden = kernels.linear(d(x), d(gu), w_batch_stride=2 * N * K, epilogue=kernels.EPI_GLU, row_scale=d(scale),
+                            out_dtype=torch.float32, **args)
+    plain = kernels.linear(d(x), d(gu), w_batch_stride=2 * N * K, out_dtype=torch.float32, n=2 * N, **args)
+    want_h, want_p = torch.zeros(rows, N, dtype=torch.float64), torch.zeros(rows, 2 * N, dtype=torch.float64)
+    for e in range(E):
+        a, b = off[e], off[e + 1]
+        y = x[token[a:b].long()].double() @ gu[e].double().t()
+        want_p[a:b] = y
+        g, u = (y * scale[a:b, None].double()).chunk(2, -1)
+        want_h[a:b] = torch.nn.functional.silu(g) * u
+    close(plain, want_p, K, dtype, torch.float32)
+    close(hidden, want_h, 2 * K, dtype, torch.float32)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_batches_and_gates(dtype):
+    """One product per head side by side, with the row gate, the soft cap and the element-wise epilogues."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(3)
+    M, H, K, n = 150, 3, 128, 72
+    x, w, gate = torch.randn(M, H * K).to(dtype), torch.randn(H, n, K).to(dtype) * 0.1, torch.randn(M, H)
+    want = torch.einsum("mhk,hnk->mhn", x.double().view(M, H, K), w.double())
+    args = dict(batch=H, a_batch_stride=K, w_batch_stride=n * K, out_batch_stride=n, n=n, out_dtype=torch.float32)
+    run = lambda **kw: kernels.linear(x.to(DEV), w.to(DEV), **args, **kw).view(M, H, n)  # noqa: E731
+    close(run(), want, K, dtype, torch.float32)
+    close(run(epilogue=kernels.EPI_ROW_GATE, gate=gate.to(DEV), gate_stride=H), want * torch.sigmoid(gate.double())[..., None], K,
+          dtype, torch.float32)
+    close(run(epilogue=kernels.EPI_SOFTCAP, cap=2.0), 2.0 * torch.tanh(want / 2.0), K, dtype, torch.float32)
+    close(run(epilogue=kernels.EPI_ACT, act=kernels.ACT_SILU), torch.nn.functional.silu(want), K, dtype, torch.float32)
