@@ -1,0 +1,281 @@
+// Prompt attention over paged bf16 rows, included by window_attn.hip (WAttnArgs, close_softmax): the walk of
+// window_attn_mfma_kernel for heads of 64 or 128 numbers, arranged for many query rows per key.
+//
+// What bounded the older kernel at 0.1 PFLOP/s: 64 query rows per staged tile of 64 keys, V written transposed into LDS two
+// bytes at a time, three workgroup barriers per tile and no load under the arithmetic.  Here
+//   * a workgroup holds 128 query rows (128 / R tokens times the R heads of a key head), 32 per wavefront;
+//   * keys and values travel as whole rows into LDS by LDS-DMA, the next tile under the current one's arithmetic, with one
+//     barrier per tile; their 16-byte pieces are dealt by XOR with the row so that fragment reads meet no bank conflicts;
+//   * S^T = K Q^T: a lane owns one query row and sixteen keys of a 32 x 32 product, so maxima and sums are lane-local but for
+//     one exchange between the wavefront's halves, and P^T is the operand of O^T = V^T P^T as it lies in the registers;
+//     V^T fragments come from transposing LDS reads (ds_read_b64_tr_b16);
+//   * tiles that every row of the wavefront sees whole take no mask, and the outputs are rescaled only when some row's
+//     maximum grew.
+// Scores, maxima, sums and outputs are fp32; q and P enter the products as bf16, as before.  Measured, 8 prompts of 2048
+// tokens, 16 heads of 128: window 512 beside 16 kept keys, two heads per key head, 554 -> 179 us; 16 key heads, ragged, every
+// earlier key, 549 -> 181 us.  What is left is the softmax: about 250 VALU instructions per 32 matrix instructions.
+#pragma once
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int PA_ROWS = 128, PA_KEYS = 64;
+
+template <int D, bool EXT>
+__global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int tiles, int bs_shift) {
+  constexpr int KS = D / 16, DT = D / 32, ROWB = 2 * D, TILE = PA_KEYS * ROWB;      // bytes of one operand's tile
+  constexpr int RPI = 1024 / ROWB, NI = PA_KEYS / RPI / 4;                          // rows per DMA instruction; instructions per wavefront
+  constexpr float L2E = 1.4426950408889634f;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[2][2 * TILE];
+  typedef __attribute__((address_space(1))) const void global_void;
+  typedef __attribute__((address_space(3))) void lds_void;
+  typedef short v4s __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) v4s lds_v4s;
+  // tiles that share keys run on one XCD; late tiles of a request, which see the most keys, first
+  int g, tile;
+  {
+    const int total = tiles * p.G, share = (total + 7) / 8, slot = blockIdx.x >> 3, id = (blockIdx.x & 7) * share + slot;
+    if (slot >= share || id >= total) return;
+    g = id / tiles;
+    tile = tiles - 1 - id % tiles;
+  }
+  const int R = p.H / p.G;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 31, lh = lane >> 5;
+  const int64_t t_begin = (int64_t)tile * p.TQ;
+  const int64_t t_end = min(p.tokens, t_begin + p.TQ);
+  const char* k_base = reinterpret_cast<const char*>(p.cache) + (int64_t)g * ROWB;
+  const char* v_base = reinterpret_cast<const char*>(p.cache) + ((int64_t)p.v_col + (int64_t)g * D) * 2;
+  const int64_t row_bytes = (int64_t)p.cw * 2;
+  const bf16_t* sink = reinterpret_cast<const bf16_t*>(p.sink);
+  auto k_swz = [](int r) { return D == 128 ? r & 15 : (r >> 1) & 7; };
+  auto v_swz = [](int r) { return D == 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); };
+
+  // this lane's part of the DMA: row RPI * (wv * NI + i) + lane / (64 / RPI) of the tile, piece lane % (64 / RPI)
+  constexpr int PIECES = 64 / RPI;                 // 16-byte pieces of a row
+  const int dma_r = lane / PIECES, dma_p = lane % PIECES;
+  int k_off[NI], v_off[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int r = RPI * (wv * NI + i) + dma_r;
+    k_off[i] = (dma_p ^ k_swz(r)) << 4;
+    v_off[i] = (dma_p ^ v_swz(r)) << 4;
+  }
+  // fragment addresses inside a tile: K row lr of a 32-row tile, piece 2 ks + lh; V^T: four tokens by sixteen numbers per
+  // sixteen lanes, rows 4 lh + (lane & 15) / 4 (and 8 further), numbers 16 (lr >> 4) + 4 (lane & 3)
+  const int ksw = k_swz(lr);
+  const int vq = (lane & 15) >> 2, vr = 4 * lh + vq, vsw = v_swz(vr);
+  auto v_at = [&](int dt) { return vr * ROWB + (((4 * dt + 2 * (lr >> 4) + ((lane & 3) >> 1)) ^ vsw) << 4) + (lane & 1) * 8; };
+
+  for (int64_t ts = t_begin; ts < t_end;) {
+    const int b = p.seq_of[ts];
+    const int64_t te = min(t_end, (int64_t)p.cu_q[b + 1]);
+    const int nq = (int)(te - ts), rows = nq * R;
+    const int p0 = p.past[b] + (int)(ts - p.cu_q[b]);
+    const int32_t* table = p.tables + (int64_t)b * p.table_cols;
+    const int row0 = 32 * wv, rr = row0 + lr;
+    const bool valid = rr < rows, wave_on = row0 < rows;
+    const int tok = valid ? rr / R : 0, head = g * R + (valid ? rr % R : 0);
+    const int pos = p0 + tok;
+    // queries: lane holds numbers 16 ks + 8 lh .. + 7 of its row
+    bf16x8 qf[KS];
+    {
+      const float* qrow = p.q + ((ts + tok) * p.H + head) * D + 8 * lh;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const f32x4 a = *reinterpret_cast<const f32x4*>(qrow + 16 * ks), c = *reinterpret_cast<const f32x4*>(qrow + 16 * ks + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          qf[ks][e] = (bf16_t)(valid ? a[e] : 0.0f);
+          qf[ks][4 + e] = (bf16_t)(valid ? c[e] : 0.0f);
+        }
+      }
+    }
+    f32x16 o[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[dt][r] = 0.0f;
+    float m_run = -INFINITY, l_run = 0.0f;
+    // first key of the row's window or chunk
+    const int low = max(p.window > 0 ? pos - p.window + 1 : 0, EXT && p.chunk > 0 ? pos / p.chunk * p.chunk : 0);
+    const int wpos_lo = p0 + row0 / R, wpos_hi = p0 + min(rows - 1, row0 + 31) / R;
+
+    const int lo_w = p.window > 0 ? max(0, p0 - p.window + 1) : 0;
+    const int lo = EXT && p.chunk > 0 ? max(lo_w, p0 / p.chunk * p.chunk) : lo_w, hi = p0 + nq - 1;
+    // kept keys: the walk is over c = c_first .. hi; c < lo means key c - c_first (those ahead of the window), else key c
+    const int c_first = EXT ? lo - min(p.keep, lo) : lo;
+    auto key_of = [&](int c) { return EXT && c < lo ? c - c_first : c; };
+    // pages of this lane's part of a tile (places past the last key repeat it: they are masked).  They are asked for a tile
+    // ahead and turned into addresses only when the tile is fetched, so nothing waits for them.
+    int page[NI], in_page[NI];
+    auto look_up = [&](int j0) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int kp = key_of(min(j0 + RPI * (wv * NI + i) + dma_r, hi));
+        const int n = bs_shift >= 0 ? kp >> bs_shift : kp / p.block_size;
+        in_page[i] = kp - n * p.block_size;
+        page[i] = table[n];
+      }
+    };
+    auto fill = [&](int buf) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int64_t at = ((int64_t)page[i] * p.block_size + in_page[i]) * row_bytes;
+        unsigned char* dst = lds[buf] + (wv * NI + i) * 1024;
+        __builtin_amdgcn_global_load_lds((global_void*)(k_base + at + k_off[i]), (lds_void*)dst, 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((global_void*)(v_base + at + v_off[i]), (lds_void*)(dst + TILE), 16, 0, 0);
+      }
+    };
+    __builtin_amdgcn_s_barrier();            // an earlier request's walk through this tile has read its last buffer
+    look_up(c_first);
+    fill(0);
+    look_up(c_first + PA_KEYS);              // page numbers a tile ahead of their use
+    int buf = 0;
+    for (int j0 = c_first; j0 <= hi; j0 += PA_KEYS, buf ^= 1) {
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (j0 + PA_KEYS <= hi) {
+        fill(buf ^ 1);
+        look_up(j0 + 2 * PA_KEYS);
+      }
+      // keys that this wavefront's rows can see at all, and whether all its rows see all of the tile
+      bool need = wave_on && j0 <= wpos_hi && (p.window <= 0 || j0 + PA_KEYS - 1 > wpos_lo - p.window);
+      bool all = j0 + PA_KEYS - 1 <= wpos_lo && (p.window <= 0 || wpos_hi - j0 < p.window);
+      if constexpr (EXT) {
+        need = wave_on && key_of(j0) <= wpos_hi && (need || key_of(j0) < p.keep) &&
+               (p.chunk <= 0 || j0 + PA_KEYS - 1 >= wpos_lo / p.chunk * p.chunk);
+        all = all && j0 >= lo && (p.chunk <= 0 || j0 >= wpos_hi / p.chunk * p.chunk);
+      }
+      if (!need) continue;
+      const unsigned char* kt = lds[buf];
+      f32x16 s[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[t][r] = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const bf16x8 kf = *reinterpret_cast<const bf16x8*>(kt + (32 * t + lr) * ROWB + (((2 * ks + lh) ^ ksw) << 4));
+          s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], s[t], 0, 0, 0);
+        }
+      }
+      // four fragments ahead of the products that use them
+      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+      for (int i = 0; i < 2 * KS; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (i < 2 * KS - 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      if (!all) {
+        // place k of the lane's keys shows key c = j0 + 4 lh + k of the walk: kept keys (c < lo), then those from the row's
+        // first to its own position, or below `keep`
+        const int c0 = j0 + 4 * lh, last = pos - c0, first = low - c0, kept = (EXT ? lo : 0) - c0, low_kept = p.keep - c0;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int k = 32 * t + 8 * (r >> 2) + (r & 3);
+            bool vis = k <= last && k >= first;
+            if constexpr (EXT) vis = vis || k < kept || (k < low_kept && k <= last);
+            s[t][r] = vis ? s[t][r] : -INFINITY;
+          }
+      }
+      float mx[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        mx[e] = fmaxf(s[0][e], s[1][e]);
+#pragma unroll
+        for (int r = 4; r < 16; r += 4) mx[e] = fmaxf(mx[e], fmaxf(s[0][r + e], s[1][r + e]));
+      }
+      float m_lo, m_hi;
+      rows_pair32(fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3])), m_lo, m_hi);
+      const float m_new = fmaxf(m_run, fmaxf(m_lo, m_hi));
+      const float m_use = m_new == -INFINITY ? 0.0f : m_new * L2E;
+      if (__any(m_new != m_run)) {
+        const float corr = __builtin_amdgcn_exp2f(fmaf(m_run, L2E, -m_use));       // exp2(-inf) = 0 at the first tile
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[dt][r] *= corr;
+        l_run *= corr;
+        m_run = m_new;
+      }
+      float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      bf16x8 pf[4];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float e = __builtin_amdgcn_exp2f(fmaf(s[t][r], L2E, -m_use));
+          sum[r & 3] += e;
+          pf[2 * t + (r >> 3)][r & 7] = (bf16_t)e;
+        }
+      l_run += (sum[0] + sum[1]) + (sum[2] + sum[3]);
+      const unsigned char* vt = kt + TILE;
+#pragma unroll
+      for (int ss = 0; ss < 4; ++ss)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          const unsigned char* a = vt + 16 * ss * ROWB + v_at(dt);
+          const v4s x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)a);
+          const v4s y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(a + 8 * ROWB));
+          const u32x2 x2 = __builtin_bit_cast(u32x2, x), y2 = __builtin_bit_cast(u32x2, y);
+          const bf16x8 vf = __builtin_bit_cast(bf16x8, u32x4{x2[0], x2[1], y2[0], y2[1]});
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[ss], o[dt], 0, 0, 0);
+        }
+      __builtin_amdgcn_sched_group_barrier(0x100, 6, 1);
+#pragma unroll
+      for (int i = 0; i < 4 * DT; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
+        if (i < 4 * DT - 3) __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
+      }
+    }
+    if (wave_on) {
+      float l_lo, l_hi;
+      rows_pair32(l_run, l_lo, l_hi);
+      if (valid) {
+        float fs, den;
+        close_softmax(m_run, l_lo + l_hi, sink != nullptr, sink ? ld_f32<bf16_t>(sink + head) : 0.0f, fs, den);
+        float f = p.out_scale * fs / den;
+        const float* grow = p.gate ? p.gate + (ts + tok) * p.gate_rs : nullptr;
+        if (EXT && p.gate_head) {
+          if (grow) f *= sigmoid_f32(grow[head]);
+          grow = nullptr;
+        }
+        bf16_t* orow = reinterpret_cast<bf16_t*>(p.out) + (ts + tok) * p.out_rs + (int64_t)head * D + 4 * lh;
+        if (grow) grow += (int64_t)head * D + 4 * lh;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {           // register 4 q + r produced number 32 dt + 8 q + 4 lh + r
+            f32x4 v;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              v[r] = o[dt][4 * q + r] * f * (grow ? sigmoid_f32(grow[32 * dt + 8 * q + r]) : 1.0f);
+            *reinterpret_cast<uint2*>(orow + 32 * dt + 8 * q) = Pack4<bf16_t>::narrow(v);
+          }
+      }
+    }
+    ts = te;
+  }
+}
+
+template <int D>
+hipError_t launch_prompt_attn(WAttnArgs p, hipStream_t s) {
+  p.TQ = PA_ROWS / (p.H / p.G);
+  const int64_t tiles = (p.tokens + p.TQ - 1) / p.TQ;
+  int shift = -1;
+  if ((p.block_size & (p.block_size - 1)) == 0)
+    for (shift = 0; (1 << shift) < p.block_size;) ++shift;
+  const dim3 grid((unsigned)((tiles * p.G + 7) / 8 * 8));
+  if (p.chunk > 0 || p.keep > 0 || (p.gate && p.gate_head)) prompt_attn_kernel<D, true><<<grid, dim3(256), 0, s>>>(p, (int)tiles, shift);
+  else prompt_attn_kernel<D, false><<<grid, dim3(256), 0, s>>>(p, (int)tiles, shift);
+  return hipGetLastError();
+}
+
+// The kernel's sizes: heads of 64 or 128 for keys and values alike, 16-byte rows, scores without cap and distance term.
+inline bool prompt_attn_serves(const WAttnArgs& p) {
+  return (p.d == 64 || p.d == 128) && p.dv == p.d && p.H / p.G <= PA_ROWS && p.softcap <= 0.0f && !p.slope_on &&
+         (uintptr_t)p.q % 16 == 0 && (uintptr_t)p.out % 8 == 0 && p.out_rs % 4 == 0;
+}

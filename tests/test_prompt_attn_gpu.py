@@ -1,0 +1,103 @@
+"""Prompt attention over paged rows (csrc/prompt_attn.h) against float64: heads of 64 and 128, one to five query heads per key
+head, portions that end inside tiles and continue from cached tokens, pages of a power of two and not, windows, kept first
+keys, chunks, sinks, gates, values that are the keys; and the rotating page store in its four-numbers-per-access form."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+CASES = [  # window, keep, chunk, sink, gate ("", "head", "number"), values are keys
+    (0, 0, 0, False, "", False), (70, 0, 0, False, "head", False), (33, 5, 0, True, "head", False),
+    (0, 0, 64, False, "number", False), (0, 0, 0, True, "number", True), (200, 300, 0, False, "", False)]
+
+
+def i32(v):
+    return torch.tensor(v, dtype=torch.int32, device=DEV)
+
+
+@pytest.mark.parametrize("options", CASES)
+@pytest.mark.parametrize("D,R,G,block", [(128, 2, 2, 64), (64, 1, 3, 48), (128, 4, 1, 16), (64, 3, 2, 256), (128, 5, 1, 80)])
+def test_against_float64(D, R, G, block, options):
+    from byox_vllm_amd import kernels
+    window, keep, chunk, with_sink, gate_form, same = options
+    torch.manual_seed(D + R + G + window)
+    new, past = [1, 63, 64, 65, 150, 2], [100, 0, 7, 64, 33, 0]
+    H, width = R * G, G * D if same else 2 * G * D
+    pages = [-(-(a + b) // block) for a, b in zip(new, past)]
+    order, tables = torch.randperm(sum(pages) + 2).tolist(), []
+    for n in pages:
+        tables.append([order.pop() for _ in range(n)])
+    cache = torch.randn((sum(pages) + 2) * block, width).to(torch.bfloat16)
+    cu = [0]
+    for n in new:
+        cu.append(cu[-1] + n)
+    T = cu[-1]
+    q = torch.randn(T, H * D) * D ** -0.5 * 2.0
+    sink = torch.randn(H).to(torch.bfloat16) if with_sink else None
+    gate = torch.randn(T, H if gate_form == "head" else H * D) if gate_form else None
+    want = torch.zeros(T, H, D, dtype=torch.float64)
+    for b, t in enumerate(tables):
+        n = past[b] + new[b]
+        rows = torch.cat([cache[p * block:(p + 1) * block] for p in t])[:n].double()
+        k = rows[:, :G * D].view(n, G, D)
+        v = k if same else rows[:, G * D:].view(n, G, D)
+        i, j = torch.arange(past[b], n)[:, None], torch.arange(n)[None]
+        seen = j <= i
+        if window:
+            seen &= (i - j < window) | (j < keep)
+        if chunk:
+            seen &= i // chunk == j // chunk
+        for h in range(H):
+            s = q[cu[b]:cu[b + 1]].to(torch.bfloat16).double().view(-1, H, D)[:, h] @ k[:, h // R].t()
+            s = s.masked_fill(~seen, float("-inf"))
+            top = s.amax(-1, keepdim=True)
+            e = torch.exp(s - top)
+            below = e.sum(-1, keepdim=True) + (torch.exp(sink[h].double() - top) if with_sink else 0.0)
+            want[cu[b]:cu[b + 1], h] = e / below @ v[:, h // R]
+    if gate_form:
+        want = want * torch.sigmoid(gate.double()).view(T, H, -1)
+    out = torch.zeros(T, H * D + 8, dtype=torch.bfloat16, device=DEV)
+    cols = max(pages)
+    kernels.paged_softmax_attn(q.to(DEV), cache.to(DEV), i32([t + [0] * (cols - len(t)) for t in tables]), i32(cu), i32(past),
+                               i32([b for b, n in enumerate(new) for _ in range(n)]), max(new), H, G, D, D, block, out,
+                               window=window, keep_first=keep, chunk=chunk, sink=None if sink is None else sink.to(DEV),
+                               gate=None if gate is None else gate.to(DEV), gate_per_head=gate_form == "head",
+                               values_are_keys=same)
+    got = out[:, :H * D].double().cpu().view(T, H, D)
+    # probabilities rounded to 8 bits of mantissa (their sum is not), values exact, one rounding of the result: a row's error
+    # is at most 2^-9 of sum p |v| <= max |v| twice over, here three units of the result's scale at most
+    assert torch.isfinite(got).all()
+    off = (got - want).abs().amax(-1)
+    bound = 2.0 ** -8 * want.abs().amax(-1) + 2.0 ** -9 * 4.0
+    assert (off <= bound).all(), float((off - bound).max())
+    assert (got - want).norm() <= 2.0 ** -8 * want.norm()
+    assert not out[:, H * D:].any()
+
+
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("dim,vdim,rot", [(64, 64, 32), (128, 64, 128), (20, 12, 8), (24, 24, 12), (16, 8, 0)])
+def test_rotating_store(dim, vdim, rot, interleaved):
+    from byox_vllm_amd import kernels
+    torch.manual_seed(dim + rot)
+    T, H, G = 37, 4, 2
+    cols = (H + G) * dim + G * vdim
+    proj = torch.randn(T, cols + 4)
+    positions = torch.randint(0, 3000, (T,))
+    freq = (1.0 / 10000.0 ** (torch.arange(0, max(rot, 2), 2).float() / max(rot, 2)))[:rot // 2]
+    cache = torch.zeros(T + 3, G * (dim + vdim), device=DEV)
+    slots = torch.randperm(T + 3)[:T].to(torch.int32)
+    q = kernels.qk_rotate_store(proj.to(DEV), (0, H * dim, (H + G) * dim), positions.to(DEV), 0.3, slots.to(DEV), cache, H, G, dim,
+                                vdim, inv_freq=freq.to(DEV) if rot else None, rot_dims=rot, interleaved=interleaved)
+
+    def turn(x):          # [T, heads, dim]
+        x, angle = x.double().clone(), (positions.float()[:, None] * freq[None]).double()[:, None]     # angles are fp32 products
+        a, b = (slice(0, rot, 2), slice(1, rot, 2)) if interleaved else (slice(0, rot // 2), slice(rot // 2, rot))
+        u, v = x[..., a].clone(), x[..., b].clone()
+        x[..., a], x[..., b] = u * angle.cos() - v * angle.sin(), v * angle.cos() + u * angle.sin()
+        return x
+    heads = turn(proj[:, :(H + G) * dim].view(T, H + G, dim)) if rot else proj[:, :(H + G) * dim].double().view(T, H + G, dim)
+    assert torch.allclose(q.double().cpu().view(T, H, dim), heads[:, :H] * 0.3, rtol=1e-6, atol=1e-6)
+    rows = cache.double().cpu()[slots.long()]
+    assert torch.allclose(rows[:, :G * dim].view(T, G, dim), heads[:, H:], rtol=1e-6, atol=2e-6)
+    assert torch.equal(rows[:, G * dim:], proj[:, (H + G) * dim:cols].double())
