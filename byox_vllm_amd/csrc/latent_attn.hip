@@ -6,7 +6,8 @@
 //
 //   nv_latent_kv_store : RMS norm of the latent, rotation of the shared key part, store into the token's cache row
 //   nv_latent_q_rope   : rotation of the per-head query parts into the absorbed-query buffer
-//   nv_latent_attn     : sliding-window softmax attention, one workgroup per (token, group of heads)
+//   nv_latent_attn     : sliding-window softmax attention, one workgroup per (token, group of heads); single tokens of a
+//                        request take latent_token.h
 //   nv_latent_gather, nv_latent_expand, nv_latent_q_rows : the pieces of the EXPANDED form that long prompt portions
 //                        take: the step's requests' cache rows gathered in order, keys and values of every head written
 //                        out from their up-projections, whole query rows; ordinary paged attention reads the result
@@ -499,6 +500,8 @@ hipError_t launch_mfma_attn(const MfmaAttnArgs& q, dim3 grid, size_t lds, hipStr
   return hipSuccess;
 }
 
+#include "latent_token.h"
+
 }  // namespace
 
 extern "C" int nv_latent_kv_store(const float* kv, int64_t kv_row_stride, const void* norm_w, const int64_t* positions,
@@ -586,6 +589,24 @@ extern "C" int nv_latent_attn_split(const float* qa, const void* cache, const in
     if (max_q == 1 && workspace) {
       const int k = latent_attn_key_splits(tokens, heads);
       if (k > 1 && workspace_bytes >= (size_t)tokens * heads * k * (rank + 2) * sizeof(float)) q.ksplit = k;
+    }
+    // single tokens whose rows split into 64-byte units: every wavefront on its own tiles of 32 keys.  Sixteen workgroups per
+    // token put 2048 keys under way at once; more of them only lengthen the join.
+    if (max_q == 1 && Dk % 32 == 0 && Dk <= 544 && (uintptr_t)cache % 16 == 0 && (uintptr_t)qa % 16 == 0 && (uintptr_t)out % 8 == 0) {
+      if (q.ksplit > 16) q.ksplit = 16;
+      const hipError_t e = Dk <= 160   ? launch_latent_token<5>(q, tokens, (hipStream_t)stream)
+                           : Dk <= 288 ? launch_latent_token<9>(q, tokens, (hipStream_t)stream)
+                                       : launch_latent_token<17>(q, tokens, (hipStream_t)stream);
+      if (e != hipSuccess) {
+        nv_set_error("nv_latent_attn: %s", hipGetErrorString(e));
+        return NV_ERR_LAUNCH;
+      }
+      if (q.ksplit > 1) {
+        latent_attn_join_kernel<<<dim3((unsigned)(tokens * heads)), dim3(256), 0, (hipStream_t)stream>>>(
+            q.partial, reinterpret_cast<bf16_t*>(out), q.ksplit, rank);
+        NV_CHECK_LAUNCH();
+      }
+      return NV_OK;
     }
     const int Dq = q.Dkp + 8;
     auto lds_for = [&](int keys) {
