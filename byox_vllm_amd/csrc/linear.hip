@@ -334,133 +334,6 @@ int launch_tile(const LinArgs& p, int epi, int batch, hipStream_t s) {
   return 0;
 }
 
-
-// Up to 64 rows per (group of) product: the launch is bound by how many weight loads are in flight, so the four
-// wavefronts of a workgroup share ONE 16-column tile and split K between them (four times the workgroups of the
-// general kernel, a quarter of the dependent rounds each); the partial sums meet in LDS and wavefront 0 finishes.
-// NSUB = 16-row sub-tiles (1: at most 16 rows, 4: at most 64).  Grouped products of 17 to 64 rows take NSUB 2 and a second
-// workgroup for rows past the 32nd: a group rarely has so many, and half the registers let twice the loads be in flight.
-template <typename T, typename TO, int EPI, int NSUB>
-__global__ __launch_bounds__(256) void linear_fewrow_kernel(LinArgs p) {
-  typedef typename Frag<T>::type F;
-  constexpr int KS = Frag<T>::KS, PER = Frag<T>::PER, UNR = 4;
-  constexpr bool GLU = EPI == EPI_GLU;
-  __shared__ float part[GLU ? 2 : 1][4][NSUB][256];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int c = lane & 15, g = lane >> 4;
-  const int z = blockIdx.z;
-  int64_t lo = 0, hi = p.M;
-  if (p.group_off) {
-    lo = p.group_off[z];
-    hi = p.group_off[z + 1];
-  }
-  lo += (int64_t)blockIdx.y * (16 * NSUB);
-  if (lo >= hi) return;
-  const int nsub = (int)((hi - lo + 15) / 16 < NSUB ? (hi - lo + 15) / 16 : NSUB);
-  const int n0 = blockIdx.x * 16;
-  const T* A = reinterpret_cast<const T*>(p.a) + z * p.a_bs;
-  const T* W = reinterpret_cast<const T*>(p.w) + z * p.w_bs;
-  const T* wrow = (n0 + c < p.N) ? W + (int64_t)(n0 + c) * p.w_rs : nullptr;
-  const T* urow = nullptr;
-  if constexpr (GLU) urow = (n0 + c < p.N) ? W + (int64_t)(p.N + n0 + c) * p.w_rs : nullptr;
-  const T* arow[NSUB];
-#pragma unroll
-  for (int i = 0; i < NSUB; ++i) {
-    const int64_t s = lo + 16 * i + c;
-    arow[i] = s < hi ? A + (int64_t)(p.a_rows ? p.a_rows[s] : s) * p.a_rs : nullptr;
-  }
-  // this wavefront's share of K, in whole rounds
-  const int round = KS * UNR;
-  const int rounds = (p.K + round - 1) / round;
-  const int k_lo = ((rounds * wv) / 4) * round, k_hi = min(p.K, ((rounds * (wv + 1)) / 4) * round);
-  f32x4 acc[NSUB], accu[NSUB];
-#pragma unroll
-  for (int i = 0; i < NSUB; ++i) acc[i] = accu[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = k_lo; k0 < k_hi; k0 += round) {
-    F wf[UNR], uf[UNR], xf[NSUB][UNR];
-#pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-      const int k = k0 + u * KS + PER * g;
-      wf[u] = load_frag<T>(wrow, k, k_hi, p.vec_w);
-      if constexpr (GLU) uf[u] = load_frag<T>(urow, k, k_hi, p.vec_w);
-#pragma unroll
-      for (int i = 0; i < NSUB; ++i)
-        if (i < nsub) xf[i][u] = load_frag<T>(arow[i], k, k_hi, p.vec_a);
-    }
-#pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-#pragma unroll
-      for (int i = 0; i < NSUB; ++i) {
-        if (i < nsub) {
-          acc[i] = mma(wf[u], xf[i][u], acc[i]);
-          if constexpr (GLU) accu[i] = mma(uf[u], xf[i][u], accu[i]);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < NSUB; ++i) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      part[0][wv][i][4 * lane + r] = acc[i][r];
-      if constexpr (GLU) part[1][wv][i][4 * lane + r] = accu[i][r];
-    }
-  }
-  __syncthreads();
-  if (wv != 0) return;
-  TO* O = reinterpret_cast<TO*>(p.out) + z * p.out_bs;
-  const T* bias = p.bias ? reinterpret_cast<const T*>(p.bias) + z * p.bias_bs : nullptr;
-#pragma unroll
-  for (int i = 0; i < NSUB; ++i) {
-    const int64_t s = lo + 16 * i + c;
-    if (i >= nsub || s >= hi) continue;
-    const float rsc = p.row_scale ? p.row_scale[s] : 1.0f;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int n = n0 + 4 * g + r;
-      if (n >= p.N) continue;
-      const int e = 4 * lane + r;
-      float v = (part[0][0][i][e] + part[0][1][i][e] + part[0][2][i][e] + part[0][3][i][e]) * rsc;
-      if (bias) v += ld_f32<T>(bias + n);
-      if constexpr (GLU) {
-        float u = (part[1][0][i][e] + part[1][1][i][e] + part[1][2][i][e] + part[1][3][i][e]) * rsc;
-        if (bias) u += ld_f32<T>(bias + p.N + n);
-        v = glu_act(v, u, p.act, p.epi_c);
-      } else if constexpr (EPI == EPI_SOFTCAP) {
-        v = p.epi_c * tanhf(v / p.epi_c);
-      } else if constexpr (EPI == EPI_ROW_GATE) {
-        v *= sigmoid_f32(p.epi_ptr[s * p.epi_rs + (p.act ? (int64_t)z * p.N + n : z)]);
-      } else if constexpr (EPI == EPI_ACT) {
-        v = unary_act(v, p.act, p.epi_ptr, p.epi_c);
-      }
-      st_f32<TO>(O + s * p.out_rs + n, v);
-    }
-  }
-}
-
-template <typename T, typename TO, int NSUB>
-int launch_fewrow(const LinArgs& p, int epi, dim3 grid, hipStream_t s) {
-  switch (epi) {
-    case EPI_NONE: linear_fewrow_kernel<T, TO, EPI_NONE, NSUB><<<grid, dim3(256), 0, s>>>(p); break;
-    case EPI_GLU: linear_fewrow_kernel<T, TO, EPI_GLU, NSUB><<<grid, dim3(256), 0, s>>>(p); break;
-    case EPI_SOFTCAP: linear_fewrow_kernel<T, TO, EPI_SOFTCAP, NSUB><<<grid, dim3(256), 0, s>>>(p); break;
-    case EPI_ACT: linear_fewrow_kernel<T, TO, EPI_ACT, NSUB><<<grid, dim3(256), 0, s>>>(p); break;
-    default: linear_fewrow_kernel<T, TO, EPI_ROW_GATE, NSUB><<<grid, dim3(256), 0, s>>>(p); break;
-  }
-  return 0;
-}
-
-template <int NSUB>
-void launch_fewrow_any(const LinArgs& p, int epi, dim3 grid, int dtype, int out_dtype, hipStream_t s) {
-  if (dtype == NV_BF16) {
-    if (out_dtype == NV_BF16) launch_fewrow<bf16_t, bf16_t, NSUB>(p, epi, grid, s);
-    else launch_fewrow<bf16_t, float, NSUB>(p, epi, grid, s);
-  } else {
-    if (out_dtype == NV_BF16) launch_fewrow<float, bf16_t, NSUB>(p, epi, grid, s);
-    else launch_fewrow<float, float, NSUB>(p, epi, grid, s);
-  }
-}
-
 template <typename T, typename TO>
 int launch_epi(const LinArgs& p, int epi, dim3 grid, hipStream_t s) {
   switch (epi) {
@@ -473,6 +346,7 @@ int launch_epi(const LinArgs& p, int epi, dim3 grid, hipStream_t s) {
   return 0;
 }
 
+#include "linear_few.h"
 #include "linear_wide.h"
 
 }  // namespace
@@ -556,10 +430,13 @@ extern "C" int nv_linear_rows(const void* a, int64_t a_row_stride, const int32_t
   }
   // at most 64 rows per product and a K worth splitting: one 16-column tile per workgroup, K split over its wavefronts
   if (M <= 64 && K >= 256 && (N + 15) / 16 <= 1048576) {
-    dim3 g16((unsigned)((N + 15) / 16), 1, (unsigned)batch);
-    if (M <= 16) launch_fewrow_any<1>(p, epilogue, g16, dtype, out_dtype, s);
-    else if (group_offsets) launch_fewrow_any<2>(p, epilogue, dim3(g16.x, (unsigned)((M + 31) / 32), g16.z), dtype, out_dtype, s);
-    else launch_fewrow_any<4>(p, epilogue, g16, dtype, out_dtype, s);
+    if (dtype == NV_BF16) {
+      if (out_dtype == NV_BF16) launch_few<bf16_t, bf16_t>(p, epilogue, batch, s);
+      else launch_few<bf16_t, float>(p, epilogue, batch, s);
+    } else {
+      if (out_dtype == NV_BF16) launch_few<float, bf16_t>(p, epilogue, batch, s);
+      else launch_few<float, float>(p, epilogue, batch, s);
+    }
     NV_CHECK_LAUNCH();
     return NV_OK;
   }
