@@ -89,7 +89,8 @@ _PROTOS = {
     "nv_sample_f32": (_i, [_p, _i64, _p, _p, _i, _i, _u64, _p]),
     "nv_gla_recurrent": (_i, [_p, _i64, _i, _i, _i, _i, _p, _i64, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _f, _f, _f, _i, _p]),
     "nv_gla_recurrent_batch": (_i, [_p, _i64, _i, _i, _i, _i, _p, _i64, _p, _p, _p, _p, _p, _p, _i64, _i, _i, _i, _i, _f, _f,
-                                    _f, _i, _p]),
+                                    _f, _i, _p, _sz, _i, _p]),
+    "nv_gla_recurrent_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "nv_matrix_memory_state_size": (_i64, [_i, _i, _i]),
     "nv_matrix_memory": (_i, [_p, _i64, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _i64, _i, _i, _i, _i, _i, _i, _f, _f,
                               _p, _i, _f, _i, _i, _p]),

@@ -16,6 +16,12 @@
 // m of a four-number sum taking the numbers {16 kk + 4 g + m}, an accumulator of S (rows 4 g + m of tile kk, column c) IS
 // the operand fragment of the next chunk's q . S.  The serial chain of a prompt is one chunk of about 40 matrix
 // instructions per wavefront; the walk it replaces is bound by the issue of 2 dim FMAs per column and token.
+//
+// Measured against that walk: channel decays, 8 x 2048 tokens, 16 heads of 64 x 128: 2560 us then, 316 now (542 MB of operands:
+// 1.7 TB/s); exponential gates, 64 requests of about 256 tokens, 8 heads of 64 x 128: 477 and 82; one decay per token, 4 requests
+// of about 1000 tokens, 32 heads of 128 x 64: 645 and 136.  What bounds it now, with two workgroups on a CU: matrix
+// instructions 37 % of the time and the vector instructions around them half, next to no overlap of the two (32768 tokens: 400 us;
+// a third fewer vector instructions gained 4 %).  Registers are held to 128 up to 64 channels for the sake of the second workgroup.
 #pragma once
 #include "anyt.h"
 
@@ -46,9 +52,9 @@ struct Args {
   int64_t out_rs;
   int H, heads_per_group, dim, vdim;
   float q_scale, k_scale, c0, eps;      // c0: GLA 1 / tau, EXPGATE the gate cap
-  // SSD, long prompts of few requests: runs of run_len tokens side by side, in two passes (see launch_ssd)
+  // GLA, SSD: long prompts of few requests as runs of run_len tokens side by side, in two passes (see launch_runs)
   float* ws_state;       // [B * H * runs][dim * vdim] state at the end of each run
-  float* ws_decay;       // [B * H * runs] product of the run's decays
+  float* ws_decay;       // SSD [B * H * runs], GLA [B * H * runs][dim]: product of the run's decays
   int runs, run_len, pass;
 };
 
@@ -164,7 +170,7 @@ __device__ __forceinline__ float silu(float z) {
 }
 
 template <int MODE, typename T, int D, int NW>
-__global__ __launch_bounds__(64 * NW) void chunk_scan_kernel(Args p) {
+__global__ __launch_bounds__(64 * NW, D <= 64 ? 4 : 1) void chunk_scan_kernel(Args p) {
   constexpr int DP = D + 4, DT = D / 16, CPL = D / (4 * NW), NP = DT < 2 ? 2 : DT;
   static_assert(CPL >= 1 && CPL <= 8 && NW % 4 == 0 && D * CP >= TOK * DP, "every lane stages whole channels");
   constexpr int BUF = 2 * TOK * DP + D * CP + D + 6 * TOK;
@@ -177,15 +183,16 @@ __global__ __launch_bounds__(64 * NW) void chunk_scan_kernel(Args p) {
   const int h = blockIdx.x, b = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, lc = lane & 15, lg = lane >> 4;
   int t0 = p.cu_q[b], t1 = p.cu_q[b + 1];
-  const int t_end = t1, j = MODE == SSD ? (int)blockIdx.z + (p.pass == 2 ? 1 : 0) : 0;
-  if constexpr (MODE == SSD) {
+  const int t_end = t1, j = MODE != EXPGATE ? (int)blockIdx.z + (p.pass == 2 ? 1 : 0) : 0;
+  if constexpr (MODE != EXPGATE) {
     if (p.runs > 1) {
       t0 += j * p.run_len;
-      t1 = min(t1, t0 + p.run_len);
+      if (j + 1 < p.runs) t1 = min(t1, t0 + p.run_len);
     }
   }
   if (t1 <= t0) return;
-  const bool emit = MODE != SSD || j == 0 || p.pass == 2;      // else: the first pass of a later run, its end state alone
+  const bool emit = MODE == EXPGATE || j == 0 || p.pass == 2;      // else: the first pass of a later run, its end state alone
+  if (!emit && t1 == t_end) return;      // which nobody needs behind the last run
   const int64_t run0 = ((int64_t)b * p.H + h) * p.runs;
   const int d = p.dim, vd = p.vdim, ch0 = (4 * wv + lg) * CPL, col = 16 * wv + lc;
   const bool own = col < vd;             // a column of the state
@@ -210,23 +217,32 @@ __global__ __launch_bounds__(64 * NW) void chunk_scan_kernel(Args p) {
   }
 
   f32x4 S[DT];
+  const int s_at = own ? (4 * lg * vd + col) * 4 : ABSENT;       // rows from d on lie past the end
+  {
+    const auto r_s = rows_of(S_g, (MODE == EXPGATE || j == 0) && !fresh ? d * vd * 4 : 0);
 #pragma unroll
-  for (int i = 0; i < DT; ++i)
+    for (int i = 0; i < DT; ++i)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * i + 4 * lg + r;
-      const bool mine = own && row < d;
-      if (MODE != SSD || j == 0) S[i][r] = (!fresh && mine) ? S_g[(int64_t)row * vd + col] : 0.0f;
-      else if (p.pass == 1 || !mine) S[i][r] = 0.0f;
-      else {             // what the runs ahead left: E_0, then D_i S + E_i
-        const int64_t per = (int64_t)d * vd;
-        const float* E = p.ws_state + run0 * per + (int64_t)row * vd + col;
-        float x = E[0];
-        for (int i2 = 1; i2 < j; ++i2) x = p.ws_decay[run0 + i2] * x + E[i2 * per];
-        S[i][r] = x;
+      for (int r = 0; r < 4; ++r) S[i][r] = load_1(r_s, s_at + (16 * i + r) * vd * 4);
+  }
+  if (MODE != EXPGATE && p.pass == 2) {       // what the runs ahead left: S <- D_i S + E_i in turn
+    for (int64_t run = run0; run < run0 + j; ++run) {
+      const auto r_s = rows_of(p.ws_state + run * d * vd, d * vd * 4);
+      const auto r_d = rows_of(p.ws_decay + (MODE == GLA ? run * d : run), MODE == GLA ? d * 4 : 4);
+#pragma unroll
+      for (int i = 0; i < DT; ++i) {
+        float f[4];
+        if constexpr (MODE == GLA) load_n(f, r_d, (16 * i + 4 * lg) * 4, d - 16 * i - 4 * lg);
+        else f[0] = f[1] = f[2] = f[3] = load_1(r_d, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[i][r] = f[r] * S[i][r] + load_1(r_s, s_at + (16 * i + r) * vd * 4);
       }
     }
+  }
   double run_lf = 0.0;                   // SSD: the run's log decay
+  float run_e[MODE == GLA ? CPL : 1];    // GLA: the run's decays of this lane's channels
+#pragma unroll
+  for (int i = 0; i < (MODE == GLA ? CPL : 1); ++i) run_e[i] = 1.0f;
   float n0[CPL], m_run = 0.0f;           // EXPGATE: normaliser of this lane's channels, running maximum (every lane)
   if constexpr (MODE == EXPGATE) {
     const float* n_g = S_g + (int64_t)d * vd;
@@ -246,20 +262,35 @@ __global__ __launch_bounds__(64 * NW) void chunk_scan_kernel(Args p) {
     o_at[m] = own ? (int)((4 * lg + m) * p.out_rs + col) * OUT : ABSENT;
   }
   float q[CPL], k[CPL], z[MODE == GLA ? CPL : 1], vn[4], gn[4];
+#pragma unroll
+  for (int i = 0; i < CPL; ++i) q[i] = 0.0f;
+#pragma unroll
+  for (int m = 0; m < 4; ++m) gn[m] = 0.0f;
+  // the next chunk's rows; the pointers advance with it
+  const float *q_p = p.q + t0 * p.q_rs + hq * d, *k_p = p.k + t0 * p.k_rs + hq * d, *v_p = p.v + t0 * p.v_rs + h * vd;
+  const float* g_p = MODE != EXPGATE ? p.g + t0 * p.g_rs + h * vd : nullptr;
+  const float* z_p = MODE == GLA ? p.s0 + t0 * p.s_rs + h * d : nullptr;
   auto fetch = [&](int c0) {
-    const int64_t last = min(TOK, t1 - c0) - 1, c = c0;
-    load_n(q, rows_of(p.q + c * p.q_rs + hq * d, (last * p.q_rs + d) * 4), qk_at[0], left);
-    load_n(k, rows_of(p.k + c * p.k_rs + hq * d, (last * p.k_rs + d) * 4), qk_at[1], left);
-    if constexpr (MODE == GLA) load_n(z, rows_of(p.s0 + c * p.s_rs + h * d, (last * p.s_rs + d) * 4), qk_at[2], left);
-    const auto rv = rows_of(p.v + c * p.v_rs + h * vd, (last * p.v_rs + vd) * 4);
+    const int last = min(TOK, t1 - c0) - 1;      // 64 rows within 2 GB: 32 bits hold every size
+    if (emit) load_n(q, rows_of(q_p, (last * (int)p.q_rs + d) * 4), qk_at[0], left);
+    load_n(k, rows_of(k_p, (last * (int)p.k_rs + d) * 4), qk_at[1], left);
+    if constexpr (MODE == GLA) load_n(z, rows_of(z_p, (last * (int)p.s_rs + d) * 4), qk_at[2], left);
+    const auto rv = rows_of(v_p, (last * (int)p.v_rs + vd) * 4);
 #pragma unroll
     for (int m = 0; m < 4; ++m) vn[m] = load_1(rv, v_at[m]);
-    if constexpr (MODE != EXPGATE) {
-      const auto rg = rows_of(p.g + c * p.g_rs + h * vd, (last * p.g_rs + vd) * 4);
+    if (MODE != EXPGATE && emit) {
+      const auto rg = rows_of(g_p, (last * (int)p.g_rs + vd) * 4);
 #pragma unroll
       for (int m = 0; m < 4; ++m) gn[m] = load_1(rg, g_at[m]);
     }
+    q_p += TOK * p.q_rs;
+    k_p += TOK * p.k_rs;
+    v_p += TOK * p.v_rs;
+    if constexpr (MODE != EXPGATE) g_p += TOK * p.g_rs;
+    if constexpr (MODE == GLA) z_p += TOK * p.s_rs;
   };
+  char* out_p = reinterpret_cast<char*>(p.out) + (t0 * p.out_rs + h * vd) * OUT;
+  const float inv_vd = 1.0f / (float)vd;
   // the gates of 64 tokens, one per lane, for four chunks in turn
   float s_in = 0.0f, f_in = 0.0f, s_gate = 0.0f, s_lf = 0.0f;
   auto fetch_gates = [&](int c0) {
@@ -323,14 +354,21 @@ __global__ __launch_bounds__(64 * NW) void chunk_scan_kernel(Args p) {
       for (int i = 0; i < CPL; ++i) {
         q[i] *= p.q_scale;
         k[i] *= p.k_scale;
-        qs[i] = q[i] * __builtin_amdgcn_exp2f(raw_f[i]);
-        ks[i] = k[i] * __builtin_amdgcn_exp2f(-raw_f[i]);
         skT[(ch0 + i) * CP + lc] = k[i] * __builtin_amdgcn_exp2f(back[i]);
-        if (lc == 15) se[ch0 + i] = __builtin_amdgcn_exp2f(end[i]);
+        const float e = __builtin_amdgcn_exp2f(end[i]);
+        run_e[i] *= e;
+        if (lc == 15) se[ch0 + i] = e;
       }
-      store_n(sq + lc * DP + ch0, qs);
-      store_n(sk + lc * DP + ch0, ks);
-      if (lane == 0) sflag[cur * NW + wv] = any ? 1.0f : 0.0f;
+      if (emit) {
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) {
+          qs[i] = q[i] * __builtin_amdgcn_exp2f(raw_f[i]);
+          ks[i] = k[i] * __builtin_amdgcn_exp2f(-raw_f[i]);
+        }
+        store_n(sq + lc * DP + ch0, qs);
+        store_n(sk + lc * DP + ch0, ks);
+        if (lane == 0) sflag[cur * NW + wv] = any ? 1.0f : 0.0f;
+      }
     } else {
       if (quarter == 0) {
         gates();
@@ -399,7 +437,7 @@ __global__ __launch_bounds__(64 * NW) void chunk_scan_kernel(Args p) {
     __syncthreads();
     // -------- scores q_t . k_s of the chunk, shares of sixteen channels dealt to the wavefronts
     bool slow = false;
-    if constexpr (MODE == GLA) {
+    if (MODE == GLA && emit) {
 #pragma unroll
       for (int w = 0; w < NW; ++w) slow |= sflag[cur * NW + w] != 0.0f;
     }
@@ -435,6 +473,7 @@ __global__ __launch_bounds__(64 * NW) void chunk_scan_kernel(Args p) {
       const int pair = tid & 255, part = tid >> 8, t = pair >> 4, s = pair & 15;
       float x = 0.0f;
       if (s <= t) {
+#pragma unroll 2
         for (int c = part * CH; c < (part + 1) * CH; ++c)
           x += rq[t * DP + c] * sk[s * DP + c] * __builtin_amdgcn_exp2f((rf[t * DP + c] - rf[s * DP + c]) + (rr[t * DP + c] - rr[s * DP + c]));
       }
@@ -472,40 +511,34 @@ __global__ __launch_bounds__(64 * NW) void chunk_scan_kernel(Args p) {
       }
       S[i] = step4(at4(skT + (16 * i + lc) * CP + 4 * lg), vv, S[i]);
     }
+    if (!emit) continue;                 // the next chunk goes to the other buffer: one barrier a chunk
     __syncthreads();
-    if (!emit) continue;
     // -------- what the chunk's own tokens contribute
-    f32x4 P = zero;
+    f32x4 P = at4(sp + lc * CP + 4 * lg);
 #pragma unroll
-    for (int w = 0; w < NP; ++w) {
+    for (int w = 1; w < NP; ++w) {
       const f32x4 x = at4(sp + (w * TOK + lc) * CP + 4 * lg);
 #pragma unroll
       for (int r = 0; r < 4; ++r) P[r] += x[r];
     }
     o = step4(P, vv, o);
-    const auto ro = rows_of(reinterpret_cast<char*>(p.out) + ((int64_t)c0 * p.out_rs + h * vd) * OUT,
-                            ((n - 1) * p.out_rs + vd) * OUT);
+    const auto ro = rows_of(out_p, ((n - 1) * (int)p.out_rs + vd) * OUT);
+    out_p += TOK * p.out_rs * OUT;
     if constexpr (MODE == GLA) {
+      f32x4 share;                       // columns that are not there hold zeros
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float ss = lanes_sum<16>(own ? o[r] * o[r] : 0.0f);
-        if (lc == 0) sred[wv * TOK + 4 * lg + r] = ss;
-      }
+      for (int r = 0; r < 4; ++r) share[r] = lanes_sum<16>(o[r] * o[r]);
+      if (lc == 0) *reinterpret_cast<f32x4*>(sred + wv * TOK + 4 * lg) = share;
       __syncthreads();
-      f32x4 ss = zero;
+      // token lc's norm, then those of this lane's four rows
+      float ss = sred[lc];
 #pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        const f32x4 x = at4(sred + w * TOK + 4 * lg);
+      for (int w = 1; w < NW; ++w) ss += sred[w * TOK + lc];
+      const float var = ss * inv_vd + p.eps;
+      float inv = __builtin_amdgcn_rsqf(var);                          // and one Newton step
+      inv *= fmaf(-0.5f * var * inv, inv, 1.5f);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) ss[r] += x[r];
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float var = ss[r] / (float)vd + p.eps;
-        float inv = __builtin_amdgcn_rsqf(var);                        // and one Newton step
-        inv *= fmaf(-0.5f * var * inv, inv, 1.5f);
-        store_1<T>(ro, o_at[r], o[r] * inv * nw * silu(gate[r]));
-      }
+      for (int r = 0; r < 4; ++r) store_1<T>(ro, o_at[r], o[r] * __shfl(inv, 4 * lg + r, 64) * nw * silu(gate[r]));
     } else if constexpr (MODE == EXPGATE) {
       // n_t . q_t of token lc: the scores' row and the normaliser ahead of the chunk
       float a, bb, nq = (P[0] + P[1]) + (P[2] + P[3]);
@@ -525,7 +558,7 @@ __global__ __launch_bounds__(64 * NW) void chunk_scan_kernel(Args p) {
     }
   }
   if (own) {
-    const bool to_slot = emit && t1 == t_end, to_ws = MODE == SSD && p.runs > 1 && p.pass == 1;
+    const bool to_slot = emit && t1 == t_end, to_ws = MODE != EXPGATE && p.runs > 1 && p.pass == 1 && t1 < t_end;
     float* E = p.ws_state + (run0 + j) * d * vd;
 #pragma unroll
     for (int i = 0; i < DT; ++i)
@@ -537,7 +570,14 @@ __global__ __launch_bounds__(64 * NW) void chunk_scan_kernel(Args p) {
           if (to_ws) E[(int64_t)row * vd + col] = S[i][r];
         }
       }
-    if (to_ws && tid == 0) p.ws_decay[run0 + j] = expf((float)run_lf);
+    if (MODE == SSD && to_ws && tid == 0) p.ws_decay[run0 + j] = expf((float)run_lf);
+  }
+  if constexpr (MODE == GLA) {
+    if (p.runs > 1 && p.pass == 1 && t1 < t_end && lc == 0) {
+#pragma unroll
+      for (int i = 0; i < CPL; ++i)
+        if (ch0 + i < d) p.ws_decay[(run0 + j) * d + ch0 + i] = run_e[i];
+    }
   }
   if constexpr (MODE == EXPGATE) {
     for (int c = 0; c < (vd + 63) / 64; ++c) {
@@ -584,18 +624,18 @@ hipError_t launch(const Args& p, int num_seqs, hipStream_t s, int runs = 1) {
   return launch_one<MODE, T, 128, 8>(p, num_seqs, runs, s);
 }
 
-// With one scalar decay per token a run of tokens maps the state affinely, S -> D S + E, so the long prompts of few requests
-// are cut into runs that are walked side by side.  First pass: run 0 starts from the slot and is final; every other run
-// starts from zero and leaves its end state E and the product D of its decays.  Second pass: run j >= 1 folds those of the
-// runs ahead of it into its start and walks again, writing its rows; the run with the step's last token leaves the state in
-// the slot (which nobody reads in the second pass).
-template <typename T>
-hipError_t launch_ssd(Args& p, int num_seqs, hipStream_t s) {
+// Decays per token (SSD) or per token and channel (GLA) make a run of tokens an affine map of the state, S -> D S + E, so the
+// long prompts of few requests are cut into runs that are walked side by side.  First pass: run 0 starts from the slot and is
+// final; the runs between it and the last start from zero and leave their end state E and the product D of their decays.  Second
+// pass: run j >= 1 folds those of the runs ahead of it into its start and walks its tokens, writing their rows; the run with the
+// step's last token leaves the state in the slot (which nobody reads in the second pass).
+template <int MODE, typename T>
+hipError_t launch_runs(Args& p, int num_seqs, hipStream_t s) {
   p.pass = 1;
-  const hipError_t e = launch<SSD, T>(p, num_seqs, s, p.runs);
+  const hipError_t e = launch<MODE, T>(p, num_seqs, s, p.runs);
   if (e != hipSuccess || p.runs == 1) return e;
   p.pass = 2;
-  return launch<SSD, T>(p, num_seqs, s, p.runs - 1);
+  return launch<MODE, T>(p, num_seqs, s, p.runs - 1);
 }
 
 }  // namespace chunk_scan

@@ -262,14 +262,40 @@ extern "C" int nv_gla_recurrent(const float* proj, int64_t proj_row_stride, int 
                                 int num_seqs, int heads, int dim, int vdim, float tau, float q_scale, float eps,
                                 int dtype, nv_stream_t stream) {
   return nv_gla_recurrent_batch(proj, proj_row_stride, q_off, k_off, v_off, g_off, z, z_row_stride, state, cu_q, past_lens,
-                                state_slots, norm_w, out, 0, num_seqs, heads, dim, vdim, tau, q_scale, eps, dtype, stream);
+                                state_slots, norm_w, out, 0, num_seqs, heads, dim, vdim, tau, q_scale, eps, 1, nullptr, 0, dtype,
+                                stream);
+}
+
+// Runs that a request of up to max_q tokens is cut into.  A run between the first and the last is walked twice, so runs pay while
+// the (request, head) pairs leave CUs idle: two workgroups per CU up to 64 key channels, one beyond, twice over so that a round's
+// end is small; past sixteen the folding of the runs ahead costs more than it gives.  Whole layers, without runs and with them (dim
+// 64): 8 requests of 2048 tokens, 16 heads 987 and 823 us; 10 of them 1123 and 1018; 16 of them 1509 and 1507, so no runs there;
+// 1 of 4096 tokens, 8 heads 887 and 194.  Dim 128: 4 of 2000 tokens, 16 heads 1004 and 655 (n = 4: 704).
+static void gla_runs(int num_seqs, int heads, int dim, int max_q, int* runs, int* run_len) {
+  *runs = 1;
+  *run_len = max_q > 0 ? max_q : 1;
+  const int64_t groups = (int64_t)num_seqs * heads;
+  if (max_q < 256 || groups == 0) return;
+  int64_t n = (dim <= 64 ? 1024 : 512) / groups;
+  if (n < (dim <= 64 ? 5 : 3)) return;
+  if (n > 16) n = 16;
+  if (n > max_q / 64) n = max_q / 64;
+  *run_len = (int)(((max_q + n - 1) / n + 15) / 16 * 16);
+  *runs = (max_q + *run_len - 1) / *run_len;
+}
+
+extern "C" size_t nv_gla_recurrent_workspace_bytes(int num_seqs, int heads, int dim, int vdim, int max_q) {
+  int runs, len;
+  gla_runs(num_seqs, heads, dim, max_q, &runs, &len);
+  return runs > 1 ? (size_t)num_seqs * heads * runs * dim * ((size_t)vdim + 1) * sizeof(float) : 0;
 }
 
 extern "C" int nv_gla_recurrent_batch(const float* proj, int64_t proj_row_stride, int q_off, int k_off, int v_off, int g_off,
                                       const float* z, int64_t z_row_stride, float* state, const int32_t* cu_q,
                                       const int32_t* past_lens, const int32_t* state_slots, const void* norm_w, void* out,
                                       int64_t tokens, int num_seqs, int heads, int dim, int vdim, float tau, float q_scale,
-                                      float eps, int dtype, nv_stream_t stream) {
+                                      float eps, int max_q, void* workspace, size_t workspace_bytes, int dtype,
+                                      nv_stream_t stream) {
   NV_CHECK_ARG(proj && z && state && cu_q && past_lens && state_slots && norm_w && out, "nv_gla_recurrent: null pointer");
   NV_CHECK_ARG(dtype == NV_BF16 || dtype == NV_F32, "nv_gla_recurrent: bad dtype %d", dtype);
   NV_CHECK_ARG(heads > 0 && heads <= 65535 && dim > 0 && vdim > 0 && vdim <= 1024 && num_seqs >= 0 && num_seqs <= 65535,
@@ -302,8 +328,13 @@ extern "C" int nv_gla_recurrent_batch(const float* proj, int64_t proj_row_stride
     c.c0 = 1.0f / tau;
     c.eps = eps;
     if (chunk_scan::serves(c) && z_row_stride % 4 == 0 && (uintptr_t)z % 16 == 0) {
+      gla_runs(num_seqs, heads, dim, max_q, &c.runs, &c.run_len);
+      const size_t need = nv_gla_recurrent_workspace_bytes(num_seqs, heads, dim, vdim, max_q);
+      if (!workspace || workspace_bytes < need) c.runs = 1;
+      c.ws_state = reinterpret_cast<float*>(workspace);
+      c.ws_decay = c.ws_state + (size_t)num_seqs * heads * c.runs * dim * vdim;
       hipError_t e;
-      NV_DISPATCH_T(dtype, e = chunk_scan::launch<chunk_scan::GLA, T>(c, num_seqs, (hipStream_t)stream));
+      NV_DISPATCH_T(dtype, e = (chunk_scan::launch_runs<chunk_scan::GLA, T>(c, num_seqs, (hipStream_t)stream)));
       if (e != hipSuccess) {
         nv_set_error("nv_gla_recurrent: %s", hipGetErrorString(e));
         return NV_ERR_LAUNCH;

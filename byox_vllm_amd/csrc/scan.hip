@@ -10,6 +10,8 @@
 //               out = S * silu(g): the minimal gated recurrent unit, whose gates read the current token only.
 // ssd_scan:     per head, S [N, P]:  S = exp(-exp(A_log) dt) S + dt B x^T,  y = S^T C + D x,  dt = softplus(raw + bias);
 //               out = y * silu(z): the selective state-space recurrence of Mamba-2 in its token-by-token form.
+#include <algorithm>
+
 #include "chunk_scan.h"
 
 namespace {
@@ -525,21 +527,27 @@ extern "C" int nv_mingru_scan(const float* proj, int64_t proj_row_stride, int z_
   return NV_OK;
 }
 
-// runs a request of max_q tokens is cut into, and their length.  Runs cost every token a second walk, so they pay only
-// while (requests x heads) leaves most of the chip idle.
-static void ssd_runs(int num_seqs, int heads, int max_q, int* runs, int* run_len) {
+// Runs a request of max_q tokens is cut into, and their length.  A run between the first and the last is walked twice, so runs pay
+// only while (requests x heads) leaves CUs idle.  Token by token: runs of 128 below 128 pairs.  In chunks: as many as make 1024
+// workgroups, four per CU, up to 256 pairs (whole fp32 layers of 1024 tokens, 32 heads, state 128, without runs and with them:
+// 4 requests 787 and 675 us, 6 of them 1060 and 1001, 8 of them 1225 and 1203; runs for 512 workgroups: 693, 1061, 1226).
+static void ssd_runs(bool chunks, int num_seqs, int heads, int max_q, int* runs, int* run_len) {
   *runs = 1;
   *run_len = max_q > 0 ? max_q : 1;
-  if (max_q < 256 || (int64_t)num_seqs * heads >= 128) return;
-  int len = 128;
-  if ((max_q + len - 1) / len > 64) len = ((max_q + 63) / 64 + 15) / 16 * 16;
-  *run_len = len;
-  *runs = (max_q + len - 1) / len;
+  const int64_t pairs = (int64_t)num_seqs * heads;
+  if (max_q < 256 || pairs == 0 || pairs > (chunks ? 256 : 127)) return;
+  int64_t n = chunks ? std::min<int64_t>(1024 / pairs, max_q / 64) : (max_q + 127) / 128;
+  if (n > 64) n = 64;
+  const int unit = chunks || n == 64 ? 16 : 128;
+  *run_len = (int)(((max_q + n - 1) / n + unit - 1) / unit * unit);
+  *runs = (max_q + *run_len - 1) / *run_len;
 }
 
 extern "C" size_t nv_ssd_scan_workspace_bytes(int num_seqs, int heads, int state_size, int vdim, int max_q) {
-  int runs, len;
-  ssd_runs(num_seqs, heads, max_q, &runs, &len);
+  int runs, more, len;
+  ssd_runs(false, num_seqs, heads, max_q, &runs, &len);
+  ssd_runs(true, num_seqs, heads, max_q, &more, &len);
+  runs = std::max(runs, more);
   return runs > 1 ? (size_t)num_seqs * heads * runs * ((size_t)state_size * vdim + 1) * sizeof(float) : 0;
 }
 
@@ -562,13 +570,18 @@ extern "C" int nv_ssd_scan(const float* xbc, int64_t xbc_row_stride, const float
   const int per = (state_size + parts - 1) / parts;
   NV_CHECK_ARG(per <= 64, "nv_ssd_scan: a state of %d x %d exceeds one workgroup's registers", state_size, vdim);
   int runs, run_len;
-  ssd_runs(num_seqs, heads, max_q, &runs, &run_len);
-  if (runs > 1) {
-    NV_CHECK_ARG(workspace && workspace_bytes >= nv_ssd_scan_workspace_bytes(num_seqs, heads, state_size, vdim, max_q),
-                 "nv_ssd_scan: %d runs need a workspace of nv_ssd_scan_workspace_bytes", runs);
+  ssd_runs(false, num_seqs, heads, max_q, &runs, &run_len);
+  const size_t per_run = (size_t)num_seqs * heads * ((size_t)state_size * vdim + 1) * sizeof(float);
+  NV_CHECK_ARG(runs == 1 || (workspace && workspace_bytes >= per_run * runs),
+               "nv_ssd_scan: %d runs need a workspace of nv_ssd_scan_workspace_bytes", runs);
+  const int walk_runs = runs, walk_len = run_len;
+  ssd_runs(true, num_seqs, heads, max_q, &runs, &run_len);
+  if (runs > 1 && (!workspace || workspace_bytes < per_run * runs)) {      // room for the walk's runs only
+    runs = walk_runs;
+    run_len = walk_len;
   }
   float* ws_state = reinterpret_cast<float*>(workspace);
-  float* ws_decay = runs > 1 ? ws_state + (size_t)num_seqs * heads * runs * state_size * vdim : nullptr;
+  auto decays = [&](int n) { return n > 1 ? ws_state + (size_t)num_seqs * heads * n * state_size * vdim : nullptr; };
   if (max_q > 1) {
     chunk_scan::Args c{};
     const int inner = heads * vdim;
@@ -596,12 +609,12 @@ extern "C" int nv_ssd_scan(const float* xbc, int64_t xbc_row_stride, const float
     c.vdim = vdim;
     c.q_scale = c.k_scale = 1.0f;
     c.ws_state = ws_state;
-    c.ws_decay = ws_decay;
+    c.ws_decay = decays(runs);
     c.runs = runs;
     c.run_len = run_len;
     if (chunk_scan::serves(c)) {
       hipError_t e;
-      NV_DISPATCH_T(dtype, e = chunk_scan::launch_ssd<T>(c, num_seqs, (hipStream_t)stream));
+      NV_DISPATCH_T(dtype, e = chunk_scan::launch_runs<chunk_scan::SSD, T>(c, num_seqs, (hipStream_t)stream));
       if (e != hipSuccess) {
         nv_set_error("nv_ssd_scan: %s", hipGetErrorString(e));
         return NV_ERR_LAUNCH;
@@ -609,8 +622,10 @@ extern "C" int nv_ssd_scan(const float* xbc, int64_t xbc_row_stride, const float
       return NV_OK;
     }
   }
+  runs = walk_runs;
+  run_len = walk_len;
   SsdArgs p{xbc, xbc_row_stride, z, z_row_stride, dt, dt_row_stride, dt_bias, A_log, D, state, cu_q, past_lens,
-            state_slots, out, heads, groups, state_size, vdim, parts, ws_state, ws_decay, runs, run_len, 1};
+            state_slots, out, heads, groups, state_size, vdim, parts, ws_state, decays(runs), runs, run_len, 1};
   const int threads = ((parts * vdim + 63) / 64) * 64;
   // tokens per stage: as many as fit 48 KB of LDS, at most 16
   auto need = [&](int tc) { return (size_t)tc * (2 * state_size + vdim + parts * vdim + 2) * sizeof(float); };

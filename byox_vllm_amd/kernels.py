@@ -612,9 +612,10 @@ def sample_f32(logits, temperatures, seed=0, out=None):
 
 
 def gla_recurrent(proj, offsets, z, state, cu_q, past_lens, state_slots, norm_w, heads, dim, vdim, tau, q_scale, eps,
-                  out=None):
+                  out=None, max_q=1):
     """Gated linear attention over the step's tokens; ``proj`` fp32 [T, *] holds q | k | v | g at ``offsets``; ``state``
-    fp32 [slots, heads, dim, vdim] is read (unless the request starts) and written back."""
+    fp32 [slots, heads, dim, vdim] is read (unless the request starts) and written back.  ``max_q`` > 1 bounds the tokens one
+    request brings: long prompts of few requests are then walked in parallel runs through a workspace."""
     require_gpu(proj, "gla_recurrent")
     T = proj.size(0)
     assert proj.dtype == z.dtype == state.dtype == torch.float32 and proj.stride(1) == 1 and z.stride(1) == 1
@@ -624,9 +625,12 @@ def gla_recurrent(proj, offsets, z, state, cu_q, past_lens, state_slots, norm_w,
     assert cu_q.numel() == B + 1 and state_slots.numel() == B
     out = torch.empty(T, heads * vdim, dtype=norm_w.dtype, device=proj.device) if out is None else out
     q_off, k_off, v_off, g_off = offsets
+    nbytes = lib().nv_gla_recurrent_workspace_bytes(B, heads, dim, vdim, max_q)
+    ws = workspace(nbytes, proj.device, "gla_recurrent") if nbytes else None
     check(lib().nv_gla_recurrent_batch(ptr(proj), proj.stride(0), q_off, k_off, v_off, g_off, ptr(z), z.stride(0), ptr(state),
                                        ptr(cu_q), ptr(past_lens), ptr(state_slots), ptr(norm_w), ptr(out), T, B, heads, dim,
-                                       vdim, tau, q_scale, eps, _code32(norm_w.dtype), stream()), "nv_gla_recurrent_batch")
+                                       vdim, tau, q_scale, eps, max_q, ptr(ws), nbytes, _code32(norm_w.dtype), stream()),
+          "nv_gla_recurrent_batch")
     return out
 
 

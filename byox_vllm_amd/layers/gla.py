@@ -38,5 +38,6 @@ class GatedLinearAttention(nn.Module):
         proj = self.qkvg(h, out_dtype=torch.float32)
         z = self.a2(self.a1(h), out_dtype=torch.float32)
         o = kernels.gla_recurrent(proj, self.offsets, z, self.state, ctx.cu_seqlens_q, ctx.past_lens, ctx.state_slots,
-                                  self.norm.data, self.heads, self.dim, self.vdim, self.tau, self.dim ** -0.5, self.eps)
+                                  self.norm.data, self.heads, self.dim, self.vdim, self.tau, self.dim ** -0.5, self.eps,
+                                  max_q=ctx.max_seqlen_q)
         return self.o(o, out_dtype=torch.float32)

@@ -448,7 +448,10 @@ int nv_gla_recurrent_batch(const float* proj, int64_t proj_row_stride, int q_off
                            const float* z, int64_t z_row_stride, float* state, const int32_t* cu_q,
                            const int32_t* past_lens, const int32_t* state_slots, const void* norm_w, void* out,
                            int64_t tokens, int num_seqs, int heads, int dim, int vdim, float tau, float q_scale, float eps,
-                           int dtype, nv_stream_t stream);
+                           int max_q, void* workspace, size_t workspace_bytes, int dtype, nv_stream_t stream);
+/* fp32 scratch with which the long prompts of few requests are walked in parallel runs; 0 where that does not pay.  max_q
+ * bounds the tokens one request brings. */
+size_t nv_gla_recurrent_workspace_bytes(int num_seqs, int heads, int dim, int vdim, int max_q);
 
 /* Matrix memories with one decay per head and token (csrc/memory.hip): S_t = keep_t S_(t-1) + take_t k_t v_t^T,
  * o_t = S_t^T q_t over this step's tokens of each request, state carried in fp32 slots of nv_matrix_memory_state_size

@@ -36,12 +36,12 @@ def walk(cu, past, start, step, width):
     return out, states
 
 
-def batch():
+def batch(lens=LENS):
     cu = [0]
-    for n in LENS:
+    for n in lens:
         cu.append(cu[-1] + n)
-    past = [0 if i % 3 else 7 for i in range(len(LENS))]
-    slots = [(5 * i + 2) % (len(LENS) + 1) for i in range(len(LENS))]      # a permutation with one slot left out
+    past = [0 if i % 3 else 7 for i in range(len(lens))]
+    slots = [(5 * i + 2) % (len(lens) + 1) for i in range(len(lens))]      # a permutation with one slot left out
     assert len(set(slots)) == len(slots)
     return cu, past, slots
 
@@ -57,10 +57,11 @@ def pool(cu, past, slots, shape, make):
 
 @pytest.mark.parametrize("H,d,dv", [(2, 64, 128), (1, 128, 128), (3, 32, 64), (2, 20, 24), (1, 4, 4), (2, 100, 68), (1, 36, 128)])
 @pytest.mark.parametrize("decay", ["slow", "mixed", "hard"])
-def test_gated_linear_attention(H, d, dv, decay):
+@pytest.mark.parametrize("lens", [LENS, [400], [63, 64, 65, 257, 2], [1, 129, 300]])       # the last three: runs side by side
+def test_gated_linear_attention(H, d, dv, decay, lens):
     from byox_vllm_amd import kernels
     torch.manual_seed(H * 1000 + d + dv)
-    cu, past, slots = batch()
+    cu, past, slots = batch(lens)
     T, tau, eps = cu[-1], 4.0, 1e-5
     proj = torch.randn(T, 2 * H * d + 2 * H * dv + 4)
     offs = (0, H * d, 2 * H * d, 2 * H * d + H * dv)
@@ -79,7 +80,7 @@ def test_gated_linear_attention(H, d, dv, decay):
                       step, H * dv)
     dev = state.to(DEV)
     got = kernels.gla_recurrent(proj.to(DEV), offs, z.to(DEV), dev, i32(cu), i32(past), i32(slots), w.to(DEV), H, d, dv, tau,
-                                d ** -0.5, eps)
+                                d ** -0.5, eps, max_q=max(lens))
     close(got, want, "rows")
     close(torch.stack([dev[s] for s in slots]), torch.stack(ends), "states")
     # the token-by-token kernel on the same arguments
@@ -87,7 +88,7 @@ def test_gated_linear_attention(H, d, dv, decay):
     dev2, out2 = state.to(DEV), torch.empty_like(got)
     p, zz, ww, args = proj.to(DEV), z.to(DEV), w.to(DEV), [i32(cu), i32(past), i32(slots)]
     check(lib().nv_gla_recurrent(ptr(p), p.stride(0), *offs, ptr(zz), zz.stride(0), ptr(dev2), *map(ptr, args), ptr(ww), ptr(out2),
-                                 len(LENS), H, d, dv, tau, d ** -0.5, eps, 2, stream()), "nv_gla_recurrent")
+                                 len(lens), H, d, dv, tau, d ** -0.5, eps, 2, stream()), "nv_gla_recurrent")
     close(got, out2, "rows against the walk")
 
 
