@@ -1,5 +1,6 @@
-"""Products of at most 64 rows (csrc/linear_few.h) against float64: rows and columns around the sixteen of a tile, K around the
-pieces, rounds and wavefronts that share it, rows that are not aligned, groups that are empty and full, every epilogue."""
+"""Products of at most 64 rows (csrc/linear_few.h) and of many rows by a short K (csrc/linear_short.h) against float64: rows and
+columns around the sixteen of a tile, K around the pieces, rounds and wavefronts that share it, rows that are not aligned, groups
+that are empty and full, the epilogues."""
 
 import pytest
 import torch
@@ -60,3 +61,34 @@ def test_groups(dtype, N, K, sizes, epilogue):
         a, b = int(off[e]), int(off[e + 1])
         if a < b:
             check(got[a:b], x[at[a:b].long()], w[e], None, epilogue, K)
+
+
+@pytest.mark.parametrize("dtype,K", [(torch.bfloat16, 8), (torch.bfloat16, 24), (torch.bfloat16, 32), (torch.bfloat16, 40),
+                                     (torch.bfloat16, 64), (torch.float32, 4), (torch.float32, 16), (torch.float32, 20),
+                                     (torch.float32, 32)])
+@pytest.mark.parametrize("M", [65, 128, 2100])
+@pytest.mark.parametrize("N", [1, 63, 256, 1000])
+@pytest.mark.parametrize("epilogue", [0, 2])
+def test_short_k(dtype, M, N, K, epilogue):
+    from byox_vllm_amd import kernels
+    torch.manual_seed(M + N + K)
+    x = torch.randn(M, K + 8, device=DEV).to(dtype)[:, :K]
+    w = torch.randn(N, K, device=DEV).to(dtype)
+    bias = torch.randn(N, device=DEV).to(dtype) if N % 2 else None
+    got = kernels.linear(x, w, bias, out_dtype=torch.float32 if M % 2 else dtype, epilogue=epilogue, cap=3.0)
+    check(got, x, w, bias, epilogue, K)
+
+
+def test_short_k_batched_gated_rows():
+    from byox_vllm_amd import kernels
+    torch.manual_seed(0)
+    M, N, K, H = 130, 96, 32, 5
+    x, w = torch.randn(M, H * K, device=DEV).bfloat16(), torch.randn(H, N, K, device=DEV).bfloat16()
+    at, gate = torch.randperm(M, device=DEV).int(), torch.randn(M, H, device=DEV)
+    out = torch.empty(M, H * N, device=DEV)
+    kernels.linear(x, w, out=out, out_dtype=torch.float32, rows=M, a_rows=at, batch=H, a_batch_stride=K, w_batch_stride=N * K, out_batch_stride=N,
+                   epilogue=kernels.EPI_ROW_GATE, act=0, gate=gate, gate_stride=H, n=N)
+    rows = x[at.long()].view(M, H, K).double()
+    want = torch.stack([rows[:, h] @ w[h].double().t() for h in range(H)], 1) * torch.sigmoid(gate.double())[..., None]
+    size = torch.stack([rows[:, h].abs() @ w[h].double().abs().t() for h in range(H)], 1)
+    assert ((out.view(M, H, N).double() - want).abs() <= (K / 16 + 24) * 2.0 ** -24 * size).all()
