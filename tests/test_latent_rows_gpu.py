@@ -1,0 +1,40 @@
+"""The copies of the expanded latent form (csrc/latent_attn.hip): whole rows of keys and values and whole rotated query rows, with
+heads that split into 16-byte pieces and that do not."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,dim,rot,vdim,rank", [(16, 96, 32, 128, 512), (3, 8, 8, 16, 24), (2, 12, 4, 20, 36), (3, 7, 2, 5, 9), (2, 8, 0, 8, 8)])
+def test_expand(dtype, H, dim, rot, vdim, rank):
+    from byox_vllm_amd._C import check, dtype_code, lib, ptr, stream
+    rows = 37
+    kv, c = torch.randn(rows, H * (dim + vdim), device=DEV).to(dtype), torch.randn(rows, rank + rot, device=DEV).to(dtype)
+    out = torch.empty(rows, H * (dim + rot + vdim), device=DEV, dtype=dtype)
+    check(lib().nv_latent_expand(ptr(kv), ptr(c), ptr(out), rows, H, dim, rot, vdim, rank, dtype_code(dtype, allow_f32=True),
+                                 stream()), "nv_latent_expand")
+    k = torch.cat([kv[:, :H * dim].view(rows, H, dim), c[:, None, rank:].expand(rows, H, rot)], -1).reshape(rows, -1)
+    assert torch.equal(out, torch.cat([k, kv[:, H * dim:]], -1))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("H,dim,rot,rot_dims", [(16, 96, 32, 32), (3, 8, 8, 6), (2, 7, 2, 2), (1, 20, 600, 600)])
+def test_query_rows(dtype, interleaved, H, dim, rot, rot_dims):
+    from byox_vllm_amd import kernels
+    T, scale, mag = 11, 0.3, 1.25
+    q = torch.randn(T, H * (dim + rot), device=DEV).to(dtype)
+    pos = torch.randint(0, 5000, (T,), device=DEV)
+    freq = (10000.0 ** (-torch.arange(rot_dims // 2, device=DEV) / max(1, rot_dims // 2))).float()
+    got = kernels.latent_q_rows(q, pos, freq, mag, H, dim, rot, rot_dims, scale, interleaved).view(T, H, dim + rot).double()
+    want = q.double().view(T, H, dim + rot).clone()
+    a = (pos.float()[:, None] * freq).double()[:, None]          # the angle is rounded to fp32
+    x = want[..., dim:dim + rot_dims].clone()
+    u, v = (x[..., 0::2], x[..., 1::2]) if interleaved else x.chunk(2, -1)
+    y, z = u * a.cos() - v * a.sin(), v * a.cos() + u * a.sin()
+    want[..., dim:dim + rot_dims] = mag * (torch.stack([y, z], -1).flatten(-2) if interleaved else torch.cat([y, z], -1))
+    assert ((got - want * scale).abs() <= 8 * 2.0 ** -24 * (want * scale).abs().max()).all()
