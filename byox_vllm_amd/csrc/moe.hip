@@ -438,20 +438,36 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const float* __restrict_
   scatter_pairs(cnt, choice, p);
 }
 
+// V columns per thread: four where rows split into 16-byte pieces (bound by memory: 16384 rows of 2048, two choices each, 402 MB:
+// 119 us in single numbers, 69 in fours).  The rows of four choices are under way together.
+template <int V>
 __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restrict__ y, const int32_t* __restrict__ slot_of,
                                                           const float* __restrict__ wt, int top,
                                                           const float* __restrict__ shared, const float* __restrict__ sg,
                                                           int64_t sg_rs, float* __restrict__ out, int width) {
+  typedef float vec __attribute__((ext_vector_type(V)));
   const int64_t t = blockIdx.x;
   const float gate = !shared ? 0.0f : sg ? sigmoid_f32(sg[t * sg_rs]) : 1.0f;   // no gate logits: a plain addend
-  for (int c = threadIdx.x; c < width; c += blockDim.x) {
-    float a = 0.0f;
-    for (int j = 0; j < top; ++j) {
-      const int slot = slot_of[t * top + j];
-      if (slot >= 0) a += wt[t * top + j] * y[(int64_t)slot * width + c];
+  for (int c = threadIdx.x * V; c < width; c += blockDim.x * V) {
+    vec a = 0.0f;
+    for (int j = 0; j < top; j += 4) {
+      vec row[4];
+      float w[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int slot = j + i < top ? slot_of[t * top + j + i] : -1;
+        row[i] = 0.0f;
+        w[i] = 0.0f;
+        if (slot >= 0) {
+          w[i] = wt[t * top + j + i];
+          row[i] = *reinterpret_cast<const vec*>(y + (int64_t)slot * width + c);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) a += w[i] * row[i];
     }
-    if (shared) a += gate * shared[t * width + c];
-    out[t * width + c] = a;
+    if (shared) a += gate * *reinterpret_cast<const vec*>(shared + t * width + c);
+    *reinterpret_cast<vec*>(out + t * width + c) = a;
   }
 }
 
@@ -546,9 +562,13 @@ extern "C" int nv_moe_combine(const float* y, const int32_t* slot_of, const floa
   NV_CHECK_ARG(y && slot_of && weights && out, "nv_moe_combine: null pointer");
   NV_CHECK_ARG(tokens >= 0 && top > 0 && width > 0, "nv_moe_combine: bad shape");
   if (tokens == 0) return NV_OK;
-  moe_combine_kernel<<<dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream>>>(y, slot_of, weights, top, shared,
-                                                                                   shared_gate, shared_gate_stride, out,
-                                                                                   width);
+  const bool fours = width % 4 == 0 && ((uintptr_t)y | (uintptr_t)shared | (uintptr_t)out) % 16 == 0;
+  if (fours)
+    moe_combine_kernel<4><<<dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream>>>(y, slot_of, weights, top, shared, shared_gate,
+                                                                                        shared_gate_stride, out, width);
+  else
+    moe_combine_kernel<1><<<dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream>>>(y, slot_of, weights, top, shared, shared_gate,
+                                                                                        shared_gate_stride, out, width);
   NV_CHECK_LAUNCH();
   return NV_OK;
 }
