@@ -13,6 +13,10 @@
 //   * workgroups that share operands run on one XCD: tile numbers are dealt to the XCDs in contiguous eighths.
 // Groups (experts) of unknown size: the grid covers the largest possible number of tiles, every workgroup finds its group
 // from the offsets with one wavefront-wide prefix sum, and the surplus leaves at once.
+//
+// Measured, before and after: sixteen experts, 32768 rows of them, gated up 2048 -> 2 x 3072 1467 and 940 us (0.88 PFLOP/s; groups
+// of equal size 907: a group that ends inside a 256-row tile costs a round), down 786 and 502; fp32, 3135 rows 1024 -> 4416 without
+// LDS 543 and 270 us (105 TFLOP/s); bf16, 1000 rows 2048 -> 1024 23 us with two LDS buffers on 128 x 128 tiles, 18.6 with three.
 #pragma once
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));

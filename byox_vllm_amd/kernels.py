@@ -648,8 +648,8 @@ def matrix_memory(proj, offsets, state, cu_q, past_lens, state_slots, heads, dim
     """Matrix memory with one decay per head and token over the step's tokens; ``proj`` fp32 [T, *] holds q | k | v at
     ``offsets`` (and, MEM_EXPGATE, one input-gate and one forget-gate logit per head at ``gate_offsets``, to which
     ``bias`` over proj's columns is added); ``rot`` fp32 [T, dims]: cosines and sines (rotation_table) by which the first
-    dims numbers of every q and k head turn, i with i + dims / 2; ``max_q`` bounds the tokens one request brings (MEM_CONST
-    works on prompts in chunks); ``state`` fp32 [slots, heads, state size] is read (unless
+    dims numbers of every q and k head turn, i with i + dims / 2; ``max_q`` bounds the tokens one request brings (prompts
+    are worked on in chunks); ``state`` fp32 [slots, heads, state size] is read (unless
     the request starts) and written back.  -> fp32 [T, heads * vdim]."""
     require_gpu(proj, "matrix_memory")
     T = proj.size(0)
