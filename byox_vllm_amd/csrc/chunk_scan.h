@@ -21,7 +21,8 @@
 // 1.7 TB/s); exponential gates, 64 requests of about 256 tokens, 8 heads of 64 x 128: 477 and 82; one decay per token, 4 requests
 // of about 1000 tokens, 32 heads of 128 x 64: 645 and 136.  What bounds it now, with two workgroups on a CU: matrix
 // instructions 37 % of the time and the vector instructions around them half, next to no overlap of the two (32768 tokens: 400 us;
-// a third fewer vector instructions gained 4 %).  Registers are held to 128 up to 64 channels for the sake of the second workgroup.
+// a third fewer vector instructions gained 4 %).  Registers are held to 128 up to 64 channels, and for wide
+// state-space heads, for the sake of the second workgroup.
 #pragma once
 #include "anyt.h"
 
@@ -170,7 +171,7 @@ __device__ __forceinline__ float silu(float z) {
 }
 
 template <int MODE, typename T, int D, int NW>
-__global__ __launch_bounds__(64 * NW, D <= 64 ? 4 : 1) void chunk_scan_kernel(Args p) {
+__global__ __launch_bounds__(64 * NW, D <= 64 || (MODE == SSD && NW == 8) ? 4 : 1) void chunk_scan_kernel(Args p) {
   constexpr int DP = D + 4, DT = D / 16, CPL = D / (4 * NW), NP = DT < 2 ? 2 : DT;
   static_assert(CPL >= 1 && CPL <= 8 && NW % 4 == 0 && D * CP >= TOK * DP, "every lane stages whole channels");
   constexpr int BUF = 2 * TOK * DP + D * CP + D + 6 * TOK;
@@ -434,6 +435,10 @@ __global__ __launch_bounds__(64 * NW, D <= 64 ? 4 : 1) void chunk_scan_kernel(Ar
       v[m] = vn[m];
       gate[m] = MODE == EXPGATE ? 0.0f : gn[m];
     }
+    bool odd = false;                    // of this wavefront's values, is one not finite?
+#pragma unroll
+    for (int m = 0; m < 4; ++m) odd |= __builtin_amdgcn_classf(v[m], 0x207);         // NaNs and infinities
+    odd = __any(odd);
     __syncthreads();
     // -------- scores q_t . k_s of the chunk, shares of sixteen channels dealt to the wavefronts
     bool slow = false;
@@ -521,7 +526,22 @@ __global__ __launch_bounds__(64 * NW, D <= 64 ? 4 : 1) void chunk_scan_kernel(Ar
 #pragma unroll
       for (int r = 0; r < 4; ++r) P[r] += x[r];
     }
-    o = step4(P, vv, o);
+    // A score of a later token is 0, but 0 times an infinity or a NaN is not: with such a value in the chunk its terms are summed one
+    // by one, so that a token's row depends on the tokens up to it alone.
+    if (!odd) {
+      o = step4(P, vv, o);
+    } else {
+#pragma unroll 1
+      for (int s = 0; s < TOK; ++s) {
+        const float vs = __shfl(s & 2 ? (s & 1 ? vv[3] : vv[2]) : (s & 1 ? vv[1] : vv[0]), 16 * (s >> 2) + lc, 64);
+        const float ps = s & 2 ? (s & 1 ? P[3] : P[2]) : (s & 1 ? P[1] : P[0]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float x = __shfl(ps, 16 * (s >> 2) + 4 * lg + r, 64);
+          if (s <= 4 * lg + r) o[r] = fmaf(x, vs, o[r]);
+        }
+      }
+    }
     const auto ro = rows_of(out_p, ((n - 1) * (int)p.out_rs + vd) * OUT);
     out_p += TOK * p.out_rs * OUT;
     if constexpr (MODE == GLA) {

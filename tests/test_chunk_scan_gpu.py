@@ -200,3 +200,41 @@ def test_state_space_runs(lens, past):
         runs.append((out, dev))
     close(runs[0][0], runs[1][0], "rows")
     close(runs[0][1], runs[1][1], "states")
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("at", [0, 5, 15, 20, 38])
+def test_a_value_that_is_not_finite_stays_out_of_earlier_rows(bad, at):
+    """One number of one token's value row is an infinity or a NaN: the rows ahead of it, and the other request's, are what they
+    are without it; the token's own row is not finite."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(at)
+    H, d, dv, lens = 2, 64, 64, [39, 20]
+    cu, T = [0, 39, 59], 59
+    ints = i32(cu), i32([0, 0]), i32([0, 1])
+    rows = torch.randn(T, 2 * H * d + 2 * H * dv + 2 * H, device=DEV)
+    z, w = torch.randn(T, H * d, device=DEV), torch.ones(dv, device=DEV)
+    vectors = [torch.randn(H, device=DEV) for _ in range(3)]
+    at_v = 2 * H * d
+
+    def gla(p):
+        return kernels.gla_recurrent(p, (0, H * d, at_v, at_v + H * dv), z, torch.zeros(2, H, d, dv, device=DEV), *ints, w, H, d, dv,
+                                     4.0, 1.0, 1e-5, max_q=39)
+
+    def gates(p):
+        state = torch.zeros(2, H, d * dv + d + 1, device=DEV)
+        return kernels.matrix_memory(p, (0, H * d, at_v), state, *ints, H, d, dv, kernels.MEM_EXPGATE, max_q=39, cap=15.0,
+                                     gate_offsets=(at_v + 2 * H * dv, at_v + 2 * H * dv + H))
+
+    def ssd(p):          # values first in this layout
+        xbc = torch.cat([p[:, at_v:at_v + H * dv], p[:, :2 * d]], 1).contiguous()
+        return kernels.ssd_scan(xbc, p[:, at_v + H * dv:at_v + 2 * H * dv], p[:, -H:], *vectors, torch.zeros(2, H, d, dv, device=DEV),
+                                *ints, H, 1, d, dv, max_q=39)
+    for name, f in (("channel decays", gla), ("exponential gates", gates), ("state space", ssd)):
+        want = f(rows)
+        spoilt = rows.clone()
+        spoilt[at, at_v + 3] = bad
+        got = f(spoilt)
+        close(got[:at] if at else got[39:], want[:at] if at else want[39:], f"{name}: rows ahead")
+        close(got[39:], want[39:], f"{name}: the other request")
+        assert not torch.isfinite(got[at]).all(), name
