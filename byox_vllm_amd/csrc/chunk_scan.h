@@ -71,7 +71,8 @@ constexpr size_t lds_floats() {
 
 // Rows are read and written through buffer descriptors over the chunk's tokens: tokens and channels that are not there lie
 // past the end and read as zeros (writes are dropped), so no access needs a branch or a clamped address.
-constexpr int ABSENT = 0x7ffffff0;       // an offset past every end
+constexpr int ABSENT = 0x7ff00000;       // an offset past every end, with room for what is added to it
+static_assert((int64_t)ABSENT + 128 * 128 * 4 <= INT32_MAX, "an absent state column's rows stay within an int");
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_of(const void* p, int64_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);
 }
