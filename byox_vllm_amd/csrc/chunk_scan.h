@@ -625,12 +625,13 @@ hipError_t launch_one(const Args& p, int num_seqs, int runs, hipStream_t s) {
 }
 
 // Sizes and alignments that the kernel serves: rows that split into 16-byte pieces, keys and values up to 128 numbers per
-// head, 64 rows within the 2 GB of a buffer descriptor's offsets.
+// head, 64 rows within the 2 GB of a buffer descriptor's offsets.  Key rows must not overlap: those past a request's end are zeros
+// because they start past the last row's end (a row expanded over the tokens, with a stride of 0, goes to the walk).
 constexpr int64_t FAR = 1 << 22;
 inline bool serves(const Args& p) {
   auto al16 = [](const void* q) { return (uintptr_t)q % 16 == 0; };
-  return p.dim % 4 == 0 && p.dim <= 128 && p.vdim <= 128 && p.q_rs % 4 == 0 && p.k_rs % 4 == 0 && al16(p.q) && al16(p.k) && p.q_rs < FAR && p.k_rs < FAR && p.v_rs < FAR &&
-         p.g_rs < FAR && p.s_rs < FAR && p.out_rs < FAR;
+  return p.dim % 4 == 0 && p.dim <= 128 && p.vdim <= 128 && p.q_rs % 4 == 0 && p.k_rs % 4 == 0 && al16(p.q) && al16(p.k) &&
+         p.k_rs >= p.dim && p.q_rs < FAR && p.k_rs < FAR && p.v_rs < FAR && p.g_rs < FAR && p.s_rs < FAR && p.out_rs < FAR;
 }
 
 template <int MODE, typename T>

@@ -238,3 +238,30 @@ def test_a_value_that_is_not_finite_stays_out_of_earlier_rows(bad, at):
         close(got[:at] if at else got[39:], want[:at] if at else want[39:], f"{name}: rows ahead")
         close(got[39:], want[39:], f"{name}: the other request")
         assert not torch.isfinite(got[at]).all(), name
+
+
+def test_one_row_for_every_token():
+    """Rows expanded over the tokens (a row stride of 0) give what copies of the row give."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(2)
+    H, d, dv, lens = 2, 64, 64, [21, 5]
+    cu, T = [0, 21, 26], 26
+    ints = i32(cu), i32([0, 0]), i32([0, 1])
+    row = torch.randn(1, 2 * H * d + 2 * H * dv, device=DEV).expand(T, -1)
+    xbc = torch.randn(1, H * dv + 2 * d, device=DEV).expand(T, -1)
+    z, dt, w = torch.randn(T, H * d, device=DEV), torch.randn(T, H, device=DEV), torch.ones(dv, device=DEV)
+    vectors = [torch.randn(H, device=DEV) for _ in range(3)]
+    gates = torch.randn(T, H * dv, device=DEV)
+    for name in ("channel decays", "state space"):
+        runs = []
+        for copy in (False, True):
+            state = torch.zeros(2, H, d, dv, device=DEV)
+            if name == "state space":
+                out = kernels.ssd_scan(xbc.contiguous() if copy else xbc, gates, dt, *vectors, state, *ints, H, 1, d, dv,
+                                       max_q=max(lens))
+            else:
+                out = kernels.gla_recurrent(row.contiguous() if copy else row, (0, H * d, 2 * H * d, 2 * H * d + H * dv), z, state,
+                                            *ints, w, H, d, dv, 4.0, 1.0, 1e-5, max_q=max(lens))
+            runs.append((out, state))
+        close(runs[0][0], runs[1][0], f"{name}: rows")
+        close(runs[0][1], runs[1][1], f"{name}: states")
