@@ -1155,12 +1155,26 @@ extern "C" int nv_paged_softmax_attn(const float* q, const void* cache, const in
                                      int distance_term, int values_are_keys, const void* sink, const float* gate,
                                      int64_t gate_row_stride, int gate_per_head, void* workspace, size_t workspace_bytes,
                                      int dtype, nv_stream_t stream) {
+  return nv_paged_softmax_attn_batch(q, cache, block_tables, table_cols, cu_q, past_lens, seq_of_token, out, out_row_stride,
+                                     tokens, 0, max_q, heads, kv_heads, dim, vdim, block_size, window, chunk, keep_first, softcap,
+                                     out_scale, distance_term, values_are_keys, sink, gate, gate_row_stride, gate_per_head,
+                                     workspace, workspace_bytes, dtype, stream);
+}
+
+extern "C" int nv_paged_softmax_attn_batch(const float* q, const void* cache, const int32_t* block_tables, int table_cols,
+                                           const int32_t* cu_q, const int32_t* past_lens, const int32_t* seq_of_token,
+                                           void* out, int64_t out_row_stride, int64_t tokens, int num_seqs, int max_q,
+                                           int heads, int kv_heads, int dim, int vdim, int block_size, int window, int chunk,
+                                           int keep_first, float softcap, float out_scale, int distance_term,
+                                           int values_are_keys, const void* sink, const float* gate, int64_t gate_row_stride,
+                                           int gate_per_head, void* workspace, size_t workspace_bytes, int dtype,
+                                           nv_stream_t stream) {
   NV_CHECK_ARG(q && cache && block_tables && cu_q && past_lens && seq_of_token && out, "nv_window_attn: null pointer");
   NV_CHECK_ARG(!values_are_keys || vdim == dim, "nv_window_attn: values that are the keys have the keys' size");
   const int cw = values_are_keys ? kv_heads * dim : kv_heads * (dim + vdim), v_col = values_are_keys ? 0 : kv_heads * dim;
   NV_CHECK_ARG(dtype == NV_BF16 || dtype == NV_F32, "nv_window_attn: bad dtype %d", dtype);
   NV_CHECK_ARG(tokens >= 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && dim > 0 && vdim > 0 &&
-                   block_size > 0 && window >= 0 && chunk >= 0 && keep_first >= 0 && table_cols > 0,
+                   block_size > 0 && window >= 0 && chunk >= 0 && keep_first >= 0 && table_cols > 0 && num_seqs >= 0,
                "nv_window_attn: bad shape");
   NV_CHECK_ARG(chunk == 0 || keep_first == 0, "nv_window_attn: chunks and kept first keys exclude each other");
   if (tokens == 0) return NV_OK;
@@ -1187,7 +1201,7 @@ extern "C" int nv_paged_softmax_attn(const float* q, const void* cache, const in
       const int wide = dim > vdim ? dim : vdim;
       if (max_q > 1 && prompt_attn_serves(pm) && (tokens * (int64_t)kv_heads + 7) / 8 * 8 < (1 << 30) &&
           getenv("NV_WINDOW_ATTN_PROMPT_OFF") == nullptr) {
-        const hipError_t e = dim == 64 ? launch_prompt_attn<64>(pm, st) : launch_prompt_attn<128>(pm, st);
+        const hipError_t e = dim == 64 ? launch_prompt_attn<64>(pm, num_seqs, st) : launch_prompt_attn<128>(pm, num_seqs, st);
         if (e != hipSuccess) {
           nv_set_error("nv_window_attn: %s", hipGetErrorString(e));
           return NV_ERR_LAUNCH;

@@ -1093,13 +1093,14 @@ def paged_softmax_attn(q, cache, block_tables, cu_q, past_lens, seq_of_token, ma
     # by the warm-up run of the same shape)
     nbytes = lib().nv_paged_softmax_attn_workspace_bytes(T, max_q, heads, kv_heads, vdim) if cache.dtype == torch.bfloat16 else 0
     ws = workspace(nbytes, q.device, "paged_softmax_attn") if nbytes else None
-    check(lib().nv_paged_softmax_attn(ptr(q), ptr(cache), ptr(block_tables), block_tables.size(1), ptr(cu_q),
-                                      ptr(past_lens), ptr(seq_of_token), ptr(out), out.stride(0), T, max_q, heads, kv_heads,
-                                      dim, vdim, block_size, window, int(chunk), int(keep_first), float(softcap or 0.0), out_scale,
-                                      int(distance_term), int(values_are_keys), ptr(sink), ptr(gate),
-                                      gate.stride(0) if gate is not None else 0, int(gate_per_head), ptr(ws), nbytes,
-                                      _code32(cache.dtype), stream()),
-          "nv_paged_softmax_attn")
+    check(lib().nv_paged_softmax_attn_batch(ptr(q), ptr(cache), ptr(block_tables), block_tables.size(1), ptr(cu_q),
+                                            ptr(past_lens), ptr(seq_of_token), ptr(out), out.stride(0), T,
+                                            min(cu_q.numel() - 1, past_lens.numel()), max_q, heads, kv_heads, dim, vdim,
+                                            block_size, window, int(chunk), int(keep_first), float(softcap or 0.0), out_scale,
+                                            int(distance_term), int(values_are_keys), ptr(sink), ptr(gate),
+                                            gate.stride(0) if gate is not None else 0, int(gate_per_head), ptr(ws), nbytes,
+                                            _code32(cache.dtype), stream()),
+          "nv_paged_softmax_attn_batch")
     return out
 
 

@@ -606,6 +606,15 @@ int nv_paged_softmax_attn(const float* q, const void* cache, const int32_t* bloc
                           int block_size, int window, int chunk, int keep_first, float softcap, float out_scale,
                           int distance_term, int values_are_keys, const void* sink, const float* gate, int64_t gate_row_stride,
                           int gate_per_head, void* workspace, size_t workspace_bytes, int dtype, nv_stream_t stream);
+/* nv_paged_softmax_attn with the number of requests (cu_q has one entry more): prompts are then dealt to workgroups request by
+ * request, so that no workgroup walks the contexts of several decoding requests in turn.  0: not known. */
+int nv_paged_softmax_attn_batch(const float* q, const void* cache, const int32_t* block_tables, int table_cols,
+                                const int32_t* cu_q, const int32_t* past_lens, const int32_t* seq_of_token, void* out,
+                                int64_t out_row_stride, int64_t tokens, int num_seqs, int max_q, int heads, int kv_heads,
+                                int dim, int vdim, int block_size, int window, int chunk, int keep_first, float softcap,
+                                float out_scale, int distance_term, int values_are_keys, const void* sink, const float* gate,
+                                int64_t gate_row_stride, int gate_per_head, void* workspace, size_t workspace_bytes, int dtype,
+                                nv_stream_t stream);
 int nv_qk_rotate_store(const float* proj, const void* bias, int64_t proj_row_stride, int q_off, int k_off, int v_off,
                        const void* q_norm, const void* k_norm, int norm_whole, const void* temp, const int64_t* positions,
                        float temp_coef, int temp_every, const float* inv_freq, int rot_dims, int interleaved, float mscale,

@@ -75,6 +75,53 @@ def test_against_float64(D, R, G, block, options):
     assert not out[:, H * D:].any()
 
 
+@pytest.mark.parametrize("window,keep", [(0, 0), (50, 4)])
+@pytest.mark.parametrize("D,R,G", [(128, 1, 2), (64, 2, 2), (64, 3, 1), (128, 8, 1)])
+def test_steps_of_single_tokens_and_pieces(D, R, G, window, keep):
+    """Decoding requests beside prompt pieces, more requests than a wavefront has lanes, one of them without tokens, pieces at
+    the edges of a tile of 128 / R tokens: against float64, and the entry that is not told how many requests there are."""
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd._C import check, dtype_code, lib, ptr, stream
+    torch.manual_seed(D + R)
+    TQ, H, block = 128 // R, R * G, 32
+    new = [1] * 70 + [0, TQ, TQ + 1, 1, TQ - 1, 2 * TQ, 3]
+    past = [(37 * i) % 90 for i in range(70)] + [5, 0, 64, 200, 7, 31, 0]
+    pages = [-(-(a + b) // block) for a, b in zip(new, past)]
+    order, tables = torch.randperm(sum(pages)).tolist(), []
+    for n in pages:
+        tables.append([order.pop() for _ in range(n)])
+    cache = torch.randn(sum(pages) * block, 2 * G * D).to(torch.bfloat16)
+    cu = [0]
+    for n in new:
+        cu.append(cu[-1] + n)
+    T = cu[-1]
+    q = torch.randn(T, H * D) * D ** -0.5 * 2.0
+    want = torch.zeros(T, H, D, dtype=torch.float64)
+    for b, t in enumerate(tables):
+        n = past[b] + new[b]
+        rows = torch.cat([cache[p * block:(p + 1) * block] for p in t])[:n].double()
+        i, j = torch.arange(past[b], n)[:, None], torch.arange(n)[None]
+        seen = (j <= i) & ((i - j < window) | (j < keep)) if window else j <= i
+        for h in range(H):
+            g = h // R
+            s = q[cu[b]:cu[b + 1]].to(torch.bfloat16).double().view(-1, H, D)[:, h] @ rows[:, g * D:(g + 1) * D].t()
+            want[cu[b]:cu[b + 1], h] = torch.softmax(s.masked_fill(~seen, float("-inf")), -1) @ rows[:, (G + g) * D:(G + g + 1) * D]
+    q, cache, tables, ints = q.to(DEV), cache.to(DEV), i32([t + [0] * (max(pages) - len(t)) for t in tables]), (
+        i32(cu), i32(past), i32([b for b, n in enumerate(new) for _ in range(n)]))
+    out = torch.full((T, H * D), float("nan"), dtype=torch.bfloat16, device=DEV)
+    kernels.paged_softmax_attn(q, cache, tables, *ints, max(new), H, G, D, D, block, out, window=window, keep_first=keep)
+    untold = torch.full_like(out, float("nan"))
+    check(lib().nv_paged_softmax_attn(ptr(q), ptr(cache), ptr(tables), tables.size(1), *map(ptr, ints), ptr(untold), H * D, T, max(new),
+                                      H, G, D, D, block, window, 0, keep, 0.0, 1.0, 0, 0, ptr(None), ptr(None), 0, 0, ptr(None), 0,
+                                      dtype_code(out.dtype), stream()), "nv_paged_softmax_attn")
+    for got in (out, untold):
+        got = got.double().cpu().view(T, H, D)
+        assert torch.isfinite(got).all()
+        # as above: probabilities rounded to 8 bits of mantissa, one rounding of the result
+        assert ((got - want).abs().amax(-1) <= 2.0 ** -8 * want.abs().amax(-1) + 2.0 ** -9 * 4.0).all()
+        assert (got - want).norm() <= 2.0 ** -8 * want.norm()
+
+
 @pytest.mark.parametrize("interleaved", [False, True])
 @pytest.mark.parametrize("dim,vdim,rot", [(64, 64, 32), (128, 64, 128), (20, 12, 8), (24, 24, 12), (16, 8, 0)])
 def test_rotating_store(dim, vdim, rot, interleaved):
