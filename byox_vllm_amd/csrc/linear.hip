@@ -450,11 +450,11 @@ extern "C" int nv_linear_rows(const void* a, int64_t a_row_stride, const int32_t
   // at most 64 rows per product and a K worth splitting: one 16-column tile per workgroup, K split over its wavefronts
   if (M <= 64 && K >= 256 && (N + 15) / 16 <= 1048576) {
     if (dtype == NV_BF16) {
-      if (out_dtype == NV_BF16) launch_few<bf16_t, bf16_t>(p, epilogue, batch, s);
-      else launch_few<bf16_t, float>(p, epilogue, batch, s);
+      if (out_dtype == NV_BF16) launch_few<bf16_t, bf16_t>(p, epilogue, total_rows, batch, s);
+      else launch_few<bf16_t, float>(p, epilogue, total_rows, batch, s);
     } else {
-      if (out_dtype == NV_BF16) launch_few<float, bf16_t>(p, epilogue, batch, s);
-      else launch_few<float, float>(p, epilogue, batch, s);
+      if (out_dtype == NV_BF16) launch_few<float, bf16_t>(p, epilogue, total_rows, batch, s);
+      else launch_few<float, float>(p, epilogue, total_rows, batch, s);
     }
     NV_CHECK_LAUNCH();
     return NV_OK;

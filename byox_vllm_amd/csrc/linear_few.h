@@ -62,15 +62,16 @@ __device__ __forceinline__ void few_mma(const FewRound<T, GLU, NS>& r, f32x4* ac
 }
 
 // a wavefront's share [k_lo, k_hi) of K, both whole rounds but for the end of K; rows point at the lane's piece of k = 0
-template <typename T, bool GLU, int NS>
+template <typename T, bool GLU, bool AHEAD, int NS>
 __device__ __forceinline__ void few_sum(const T* wrow, const T* urow, const T* const (&arow)[NS], int k_lo, int k_hi, int K, int piece,
                                         f32x4* acc, f32x4* accu) {
   constexpr int ROUND = 4 * Frag<T>::KS;
   if (k_lo >= k_hi) return;
   const int lim = K - piece;        // this lane's pieces below here are inside K
-  // gate and up rows fill half again as many registers: there a second round in flight costs more in wavefronts per SIMD than it
-  // brings (64 rows over 16 experts of 6.3 MB: 30 us with it, 26 without; their down rows, of one kind: 16.4 with it, 18 without)
-  if constexpr (GLU) {
+  // AHEAD: a second round in flight.  Gate and up rows fill half again as many registers: there it costs more in wavefronts per SIMD
+  // than it brings (64 rows over 16 experts of 6.3 MB: 30 us with it, 26 without; their down rows, of one kind: 16.4 with it, 18
+  // without)
+  if constexpr (!AHEAD) {
     for (int k = k_lo; k < k_hi; k += ROUND) {
       FewRound<T, GLU, NS> r;
       few_load<T, GLU, NS>(r, wrow, urow, arow, k, lim, k + ROUND > K);
@@ -90,7 +91,7 @@ __device__ __forceinline__ void few_sum(const T* wrow, const T* urow, const T* c
 }
 
 // VEC: rows are 16-byte aligned and K a multiple of 16 bytes
-template <typename T, typename TO, int EPI, int NSUB, int NW, bool VEC>
+template <typename T, typename TO, int EPI, int NSUB, int NW, bool VEC, bool AHEAD>
 __global__ __launch_bounds__(64 * NW) void linear_few_kernel(LinArgs p) {
   typedef typename Frag<T>::type F;
   constexpr int KS = Frag<T>::KS, PER = Frag<T>::PER, ROUND = 4 * KS;
@@ -132,9 +133,9 @@ __global__ __launch_bounds__(64 * NW) void linear_few_kernel(LinArgs p) {
     for (int i = 0; i < NSUB; ++i) arow[i] += PER * g;
     if (NSUB > 1 && nsub == 1) {
       const T* const one[1] = {arow[0]};
-      few_sum<T, GLU, 1>(wrow, urow, one, k_lo, k_hi, p.K, PER * g, acc, accu);
+      few_sum<T, GLU, AHEAD, 1>(wrow, urow, one, k_lo, k_hi, p.K, PER * g, acc, accu);
     } else {
-      few_sum<T, GLU, NSUB>(wrow, urow, arow, k_lo, k_hi, p.K, PER * g, acc, accu);
+      few_sum<T, GLU, AHEAD, NSUB>(wrow, urow, arow, k_lo, k_hi, p.K, PER * g, acc, accu);
     }
   } else {
     for (int k0 = k_lo; k0 < k_hi; k0 += KS) {
@@ -191,24 +192,27 @@ __global__ __launch_bounds__(64 * NW) void linear_few_kernel(LinArgs p) {
   }
 }
 
-template <typename T, typename TO, int NSUB, int NW, bool VEC>
+template <typename T, typename TO, int NSUB, int NW, bool VEC, bool AHEAD = VEC>
 void launch_few_as(const LinArgs& p, int epi, dim3 grid, hipStream_t s) {
   grid.y = (unsigned)((p.M + 16 * NSUB - 1) / (16 * NSUB));
   switch (epi) {
-    case EPI_NONE: linear_few_kernel<T, TO, EPI_NONE, NSUB, NW, VEC><<<grid, dim3(64 * NW), 0, s>>>(p); break;
-    case EPI_GLU: linear_few_kernel<T, TO, EPI_GLU, NSUB, NW, VEC><<<grid, dim3(64 * NW), 0, s>>>(p); break;
-    case EPI_SOFTCAP: linear_few_kernel<T, TO, EPI_SOFTCAP, NSUB, NW, VEC><<<grid, dim3(64 * NW), 0, s>>>(p); break;
-    case EPI_ACT: linear_few_kernel<T, TO, EPI_ACT, NSUB, NW, VEC><<<grid, dim3(64 * NW), 0, s>>>(p); break;
-    default: linear_few_kernel<T, TO, EPI_ROW_GATE, NSUB, NW, VEC><<<grid, dim3(64 * NW), 0, s>>>(p); break;
+    case EPI_NONE: linear_few_kernel<T, TO, EPI_NONE, NSUB, NW, VEC, AHEAD><<<grid, dim3(64 * NW), 0, s>>>(p); break;
+    case EPI_GLU: linear_few_kernel<T, TO, EPI_GLU, NSUB, NW, VEC, false><<<grid, dim3(64 * NW), 0, s>>>(p); break;
+    case EPI_SOFTCAP: linear_few_kernel<T, TO, EPI_SOFTCAP, NSUB, NW, VEC, AHEAD><<<grid, dim3(64 * NW), 0, s>>>(p); break;
+    case EPI_ACT: linear_few_kernel<T, TO, EPI_ACT, NSUB, NW, VEC, AHEAD><<<grid, dim3(64 * NW), 0, s>>>(p); break;
+    default: linear_few_kernel<T, TO, EPI_ROW_GATE, NSUB, NW, VEC, AHEAD><<<grid, dim3(64 * NW), 0, s>>>(p); break;
   }
 }
 
 // At most 64 rows.  As many sub-tiles per workgroup as leave the chip a workgroup per CU (each further workgroup reads the weights
 // again): 64 rows by 1024 columns of K = 1024 take 24 us in 64 workgroups of four sub-tiles, 7 in 256 of one.  A group of rows
 // seldom has more than 32.  Sixteen wavefronts share K where even single sub-tiles leave CUs idle and every wavefront still gets a
-// round (8 rows by 1024 columns of K = 1024 in fp32: 9.0 us on four, 6.3 on sixteen).
+// round (8 rows by 1024 columns of K = 1024 in fp32: 9.0 us on four, 6.3 on sixteen).  Where all groups together have at most 8 rows,
+// few of them have any, and the registers of a second round in flight cost more than it brings (mean over routings of 1 to 8 rows, 16
+// experts of 2048 x 3072: 13.4 us with it, 11.7 without, 32 of 1024 x 1536 6.7 and 6.1; over all sizes measured 2 to 8 rows 2 to 5 %
+// shorter without it, 10 the same, 12 to 39 2 to 4 % longer).
 template <typename T, typename TO>
-void launch_few(const LinArgs& p, int epi, int batch, hipStream_t s) {
+void launch_few(const LinArgs& p, int epi, int64_t total_rows, int batch, hipStream_t s) {
   const dim3 grid((unsigned)((p.N + 15) / 16), 1, (unsigned)batch);
   if (!p.vec_a || !p.vec_w || p.K % Frag<T>::PER) {
     if (p.M <= 16) launch_few_as<T, TO, 1, 4, false>(p, epi, grid, s);
@@ -220,5 +224,6 @@ void launch_few(const LinArgs& p, int epi, int batch, hipStream_t s) {
   if (p.M > 32 && !p.group_off && groups(4) >= 256) launch_few_as<T, TO, 4, 4, true>(p, epi, grid, s);
   else if (p.M > 16 && groups(2) >= 256) launch_few_as<T, TO, 2, 4, true>(p, epi, grid, s);
   else if (groups(1) <= 256 && p.K >= 16 * 4 * Frag<T>::KS) launch_few_as<T, TO, 1, 16, true>(p, epi, grid, s);
+  else if (p.group_off && total_rows <= 8) launch_few_as<T, TO, 1, 4, true, false>(p, epi, grid, s);
   else launch_few_as<T, TO, 1, 4, true>(p, epi, grid, s);
 }

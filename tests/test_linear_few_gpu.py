@@ -63,6 +63,26 @@ def test_groups(dtype, N, K, sizes, epilogue):
             check(got[a:b], x[at[a:b].long()], w[e], None, epilogue, K)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,K", [(48, 512), (1040, 264), (40, 1160), (1040, 3080)])
+@pytest.mark.parametrize("sizes", [[1, 0, 0, 0], [0, 1, 5, 2], [3, 0, 5, 1]])          # eight rows and the nine beyond the rule
+@pytest.mark.parametrize("epilogue", [0, 1])
+def test_groups_of_a_few_rows_in_all(dtype, N, K, sizes, epilogue):
+    from byox_vllm_amd import kernels
+    torch.manual_seed(N + K)
+    n, T, rows = 2 * N if epilogue else N, 6, sum(sizes)
+    x = torch.randn(T, K, device=DEV).to(dtype)
+    w = (torch.randn(4, n, K, device=DEV) * K ** -0.5).to(dtype)
+    at = torch.randint(0, T, (rows,), dtype=torch.int32, device=DEV)
+    off = torch.tensor([0] + torch.tensor(sizes).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+    got = kernels.linear(x, w, out_dtype=torch.float32, rows=rows, a_rows=at, batch=4, w_batch_stride=n * K, group_offsets=off,
+                         max_group_rows=T, epilogue=epilogue, act=kernels.ACT_SILU)
+    for e in range(4):
+        a, b = int(off[e]), int(off[e + 1])
+        if a < b:
+            check(got[a:b], x[at[a:b].long()], w[e], None, epilogue, K)
+
+
 @pytest.mark.parametrize("dtype,K", [(torch.bfloat16, 8), (torch.bfloat16, 24), (torch.bfloat16, 32), (torch.bfloat16, 40),
                                      (torch.bfloat16, 64), (torch.float32, 4), (torch.float32, 16), (torch.float32, 20),
                                      (torch.float32, 32)])
