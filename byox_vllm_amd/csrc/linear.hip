@@ -404,10 +404,8 @@ extern "C" int nv_linear_rows(const void* a, int64_t a_row_stride, const int32_t
   p.vec_w = (uintptr_t)w % 16 == 0 && w_row_stride % per == 0 && (w_batch_stride * esz) % 16 == 0;
   dim3 grid((unsigned)((N + 63) / 64), (unsigned)mtiles, (unsigned)batch);
   hipStream_t s = (hipStream_t)stream;
-  // more than 64 rows by all of K in one or two fragments: nothing to stage.  (fp32 takes eight matrix instructions per tile from
-  // 17 numbers on, which few rows do not hide: 200 rows by 512 of K = 32 6.7 us on the tiles, 7.0 there; 4000 rows 9.3 and 8.2.)
+  // more than 64 rows by all of K in one or two fragments: nothing to stage
   if (M > 64 && p.vec_a && p.vec_w && K % per == 0 && K * esz <= 128 && !group_offsets && epilogue != EPI_GLU &&
-      (dtype == NV_BF16 || K <= 16 || M >= 2048) &&
       getenv("NV_LINEAR_TILE_OFF") == nullptr) {
     if (dtype == NV_BF16) {
       if (out_dtype == NV_BF16) launch_short<bf16_t, bf16_t>(p, epilogue, batch, s);

@@ -112,3 +112,18 @@ def test_short_k_batched_gated_rows():
     want = torch.stack([rows[:, h] @ w[h].double().t() for h in range(H)], 1) * torch.sigmoid(gate.double())[..., None]
     size = torch.stack([rows[:, h].abs() @ w[h].double().abs().t() for h in range(H)], 1)
     assert ((out.view(M, H, N).double() - want).abs() <= (K / 16 + 24) * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("dtype,K", [(torch.bfloat16, 40), (torch.bfloat16, 64), (torch.float32, 20), (torch.float32, 32)])
+@pytest.mark.parametrize("M,N", [(4170, 1000), (8200, 257), (66, 257)])          # 256 columns per workgroup; one workgroup short of it
+@pytest.mark.parametrize("epilogue", [0, 3])
+def test_short_k_four_tiles_per_wavefront(dtype, K, M, N, epilogue):
+    from byox_vllm_amd import kernels
+    torch.manual_seed(M + N + K)
+    x, w = torch.randn(M, K, device=DEV).to(dtype), torch.randn(N, K, device=DEV).to(dtype)
+    gate = torch.randn(M, 1, device=DEV) if epilogue else None
+    got = kernels.linear(x, w, out_dtype=torch.float32, epilogue=epilogue, gate=gate, gate_stride=1)
+    want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    if epilogue:
+        want = want * torch.sigmoid(gate.double())
+    assert ((got.double() - want).abs() <= (K / 16 + 24) * 2.0 ** -24 * size).all()
