@@ -21,9 +21,10 @@
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// value(s) of one output -> what is stored (bias, activation, gate)
+// value(s) of one output -> what is stored (bias, activation, gate); `gate`: the row's, where there is one for all of it
 template <typename T, int EPI>
-__device__ __forceinline__ float lin_finish(const LinArgs& p, const T* bias, float v, float u, float rsc, int64_t s, int n, int z) {
+__device__ __forceinline__ float lin_finish(const LinArgs& p, const T* bias, float v, float u, float rsc, float gate, int64_t s, int n,
+                                            int z) {
   v *= rsc;
   if (bias) v += ld_f32<T>(bias + n);
   if constexpr (EPI == EPI_GLU) {
@@ -33,7 +34,7 @@ __device__ __forceinline__ float lin_finish(const LinArgs& p, const T* bias, flo
   } else if constexpr (EPI == EPI_SOFTCAP) {
     v = p.epi_c * tanhf(v / p.epi_c);
   } else if constexpr (EPI == EPI_ROW_GATE) {
-    v *= sigmoid_f32(p.epi_ptr[s * p.epi_rs + (p.act ? (int64_t)z * p.N + n : z)]);
+    v *= p.act ? sigmoid_f32(p.epi_ptr[s * p.epi_rs + (int64_t)z * p.N + n]) : gate;
   } else if constexpr (EPI == EPI_ACT) {
     v = unary_act(v, p.act, p.epi_ptr, p.epi_c);
   }
@@ -228,6 +229,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void linear_wide_kernel(LinArgs p,
     const int64_t s = mbase + 32 * (MT * wm + i) + fr;
     if (s >= hi) continue;
     const float rsc = p.row_scale ? p.row_scale[s] : 1.0f;
+    const float gate = EPI == EPI_ROW_GATE && !p.act ? sigmoid_f32(p.epi_ptr[s * p.epi_rs + z]) : 1.0f;
 #pragma unroll
     for (int j = 0; j < (GLU ? 1 : 2); ++j) {
 #pragma unroll
@@ -237,7 +239,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void linear_wide_kernel(LinArgs p,
         f32x4 v;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          v[r] = n + r < p.N ? lin_finish<T, EPI>(p, bias, acc[j][i][4 * g + r], GLU ? acc[1][i][4 * g + r] : 0.0f, rsc, s, n + r, z)
+          v[r] = n + r < p.N ? lin_finish<T, EPI>(p, bias, acc[j][i][4 * g + r], GLU ? acc[1][i][4 * g + r] : 0.0f, rsc, gate, s, n + r,
+                                                z)
                              : 0.0f;
         TO* o = O + s * p.out_rs + n;
         if (vec) {

@@ -83,3 +83,19 @@ def test_batches_and_gates(dtype):
           dtype, torch.float32)
     close(run(epilogue=kernels.EPI_SOFTCAP, cap=2.0), 2.0 * torch.tanh(want / 2.0), K, dtype, torch.float32)
     close(run(epilogue=kernels.EPI_ACT, act=kernels.ACT_SILU), torch.nn.functional.silu(want), K, dtype, torch.float32)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,K", [(150, 128), (150, 32), (40, 256)])          # the wide tiles, the short products, the few rows
+@pytest.mark.parametrize("per_number", [False, True])
+def test_gates_of_rows_and_of_numbers(dtype, M, K, per_number):
+    from byox_vllm_amd import kernels
+    torch.manual_seed(M + K)
+    H, n = 3, 70
+    x, w = torch.randn(M, H * K).to(dtype), torch.randn(H, n, K).to(dtype) * 0.1
+    gate = torch.randn(M, H * n if per_number else H)
+    got = kernels.linear(x.to(DEV), w.to(DEV), batch=H, a_batch_stride=K, w_batch_stride=n * K, out_batch_stride=n, n=n,
+                         out_dtype=torch.float32, epilogue=kernels.EPI_ROW_GATE, act=kernels.GATE_PER_NUMBER if per_number else 0,
+                         gate=gate.to(DEV), gate_stride=gate.size(1)).view(M, H, n)
+    want = torch.matmul(x.double().view(M, H, K).transpose(0, 1), w.double().transpose(1, 2)).transpose(0, 1)
+    close(got, want * torch.sigmoid(gate.double()).view(M, H, -1), K, dtype, torch.float32)
