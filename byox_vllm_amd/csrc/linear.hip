@@ -417,8 +417,16 @@ extern "C" int nv_linear_rows(const void* a, int64_t a_row_stride, const int32_t
     NV_CHECK_LAUNCH();
     return NV_OK;
   }
-  // more than 64 rows that split into K blocks of 128 bytes: the wide tiles
-  if (M > 64 && p.vec_a && p.vec_w && (K * esz) % 128 == 0 && getenv("NV_LINEAR_TILE_OFF") == nullptr) {
+  // more than 64 rows that split into K blocks of 128 bytes: the wide tiles.  In fp32 a wide tile costs whatever of it is used, and its
+  // wavefronts form twice as many results each as those of linear_kernel, so two kinds of product stay there: at most 32 columns
+  // whose short K brings more tiles than the chip holds (32 heads of 32 columns, 4000 rows, K = 128: 33.8 us there, 50 in wide tiles;
+  // 1000 rows, 512 tiles: 15.7 and 14.9), and element-wise functions of a product of two K blocks that leaves CUs idle (130 rows by
+  // 1500 columns, K = 64, soft cap: 11.4 and 13.9; K = 128: 15.3 and 16.2; 4000 rows by 512: 14.4 and 13.0).
+  const int64_t tiles64 = wide_tiles(64, 128, M, total_rows, epilogue == EPI_GLU ? 2 * N : N, batch, group_offsets != nullptr);
+  const bool stays = dtype == NV_F32 && !group_offsets && epilogue != EPI_GLU &&
+                     (N <= 32 ? K <= 128 && tiles64 > 512
+                              : (epilogue == EPI_SOFTCAP || epilogue == EPI_ACT) && K <= 64 && tiles64 < 96);
+  if (M > 64 && p.vec_a && p.vec_w && (K * esz) % 128 == 0 && !stays && getenv("NV_LINEAR_TILE_OFF") == nullptr) {
     const int cols = epilogue == EPI_GLU ? 2 * N : N;
     int tile = pick_wide_tile(M, total_rows, cols, batch, group_offsets != nullptr, dtype == NV_BF16);
     if (const char* force = getenv("NV_LINEAR_TILE")) tile = atoi(force);

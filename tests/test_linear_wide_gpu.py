@@ -99,3 +99,17 @@ def test_gates_of_rows_and_of_numbers(dtype, M, K, per_number):
                          gate=gate.to(DEV), gate_stride=gate.size(1)).view(M, H, n)
     want = torch.matmul(x.double().view(M, H, K).transpose(0, 1), w.double().transpose(1, 2)).transpose(0, 1)
     close(got, want * torch.sigmoid(gate.double()).view(M, H, -1), K, dtype, torch.float32)
+
+
+@pytest.mark.parametrize("M,N,K,H,softcap", [(1100, 32, 128, 32, False), (1000, 32, 128, 32, False), (1100, 33, 96, 8, False),
+                                             (1300, 5, 64, 30, True), (130, 200, 64, 1, True), (200, 3100, 64, 1, True)])
+def test_fp32_products_on_both_sides_of_the_rule(M, N, K, H, softcap):
+    """Narrow and short fp32 products that stay with the kernel for any shape, and their neighbours in wide tiles."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(M + N)
+    x, w = torch.randn(M, H * K), torch.randn(H, N, K) * 0.1
+    args = dict(batch=H, a_batch_stride=K, w_batch_stride=N * K, out_batch_stride=N, n=N) if H > 1 else {}
+    got = kernels.linear(x.to(DEV), (w if H > 1 else w[0]).to(DEV), out_dtype=torch.float32, cap=2.0,
+                         epilogue=kernels.EPI_SOFTCAP if softcap else kernels.EPI_NONE, **args).view(M, H, N)
+    want = torch.matmul(x.double().view(M, H, K).transpose(0, 1), w.double().transpose(1, 2)).transpose(0, 1)
+    close(got, 2.0 * torch.tanh(want / 2.0) if softcap else want, K, torch.float32, torch.float32)
