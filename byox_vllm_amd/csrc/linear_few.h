@@ -137,6 +137,24 @@ __global__ __launch_bounds__(64 * NW) void linear_few_kernel(LinArgs p) {
     } else {
       few_sum<T, GLU, AHEAD, NSUB>(wrow, urow, arow, k_lo, k_hi, p.K, PER * g, acc, accu);
     }
+  } else if constexpr (NSUB == 1 && sizeof(T) == 4) {
+    // numbers one by one: rows that are not there are not read, and a round's loads precede its products (one row by 777 columns of
+    // K = 1030: 11.1 us so, 12.2 step by step with every lane reading; 64 rows 40.2 and 32.9, bf16 12.9 and 12.3: below)
+    for (int k0 = k_lo; k0 < k_hi; k0 += ROUND) {
+      F w[4], u[GLU ? 4 : 1], x[4];
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        const int k = k0 + f * KS + PER * g;
+        w[f] = load_frag<T>(wrow, k, p.K, p.vec_w);
+        if constexpr (GLU) u[f] = load_frag<T>(urow, k, p.K, p.vec_w);
+        x[f] = load_frag<T>(lo + c < hi ? arow[0] : nullptr, k, p.K, p.vec_a);
+      }
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        acc[0] = mma(w[f], x[f], acc[0]);
+        if constexpr (GLU) accu[0] = mma(u[f], x[f], accu[0]);
+      }
+    }
   } else {
     for (int k0 = k_lo; k0 < k_hi; k0 += KS) {
       const int k = k0 + PER * g;
