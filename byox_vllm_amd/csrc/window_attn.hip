@@ -158,10 +158,10 @@ __global__ __launch_bounds__(256) void qk_norm_store_kernel(QkArgs p) {
 }
 
 // The case without norms, temperatures, biases and blended values: a thread takes four consecutive numbers of q | k | v per
-// access.  Interleaved rotations need nothing else; in the other form the four partners half the rotated numbers away are one
-// more access, for the rotated numbers alone (8 x 2048 tokens, 32 heads of 128, 32 numbers turned:
-// 245 us in the general kernel, 111 us here).
-template <typename T>
+// access.  Interleaved rotations need nothing else; in the other form (HALVES) the four partners half the rotated numbers away are
+// one more access, for the rotated numbers alone (8 x 2048 tokens, 32 heads of 128, 32 numbers turned:
+// 245 us in the general kernel, 111 us here).  One kernel for both forms cost the interleaved one 2 to 4 % at any size.
+template <typename T, bool HALVES>
 __global__ __launch_bounds__(256) void qk_pairs_store_kernel(QkArgs p) {
   typedef typename Pack4<T>::type P;
   __shared__ float s_cs[128], s_sn[128];
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(256) void qk_pairs_store_kernel(QkArgs p) {
     f32x4 x = *reinterpret_cast<const f32x4*>(row + (is_q ? p.q_off : is_v ? p.v_off : p.k_off) + rel);
     if (!is_v) {
       const int e = rel % p.d;
-      if (!p.interleaved) {
+      if constexpr (HALVES) {
         if (e < p.rot_dims) {
           const bool first = e < half;
           const int i = first ? e : e - half;
@@ -193,13 +193,14 @@ __global__ __launch_bounds__(256) void qk_pairs_store_kernel(QkArgs p) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) x[j] = first ? x[j] * s_cs[i + j] - y[j] * s_sn[i + j] : x[j] * s_cs[i + j] + y[j] * s_sn[i + j];
         }
-      } else
+      } else {
 #pragma unroll
-      for (int j = 0; j < 4; j += 2) {
-        if (e + j < p.rot_dims) {
-          const float cs = s_cs[(e + j) >> 1], sn = s_sn[(e + j) >> 1], u = x[j], v = x[j + 1];
-          x[j] = u * cs - v * sn;
-          x[j + 1] = v * cs + u * sn;
+        for (int j = 0; j < 4; j += 2) {
+          if (e + j < p.rot_dims) {
+            const float cs = s_cs[(e + j) >> 1], sn = s_sn[(e + j) >> 1], u = x[j], v = x[j + 1];
+            x[j] = u * cs - v * sn;
+            x[j + 1] = v * cs + u * sn;
+          }
         }
       }
     }
@@ -1081,8 +1082,10 @@ extern "C" int nv_qk_rotate_store(const float* proj, const void* bias, int64_t p
   QkArgs p{proj, bias, proj_row_stride, q_off, k_off, v_off, q_norm, k_norm, temp, positions, temp_coef, temp_every,
            slot_mapping, cache, q_out, heads, kv_heads, dim, vdim, scale, eps, norm_whole, inv_freq, rot_dims, mscale,
            v_first, v_first_row_stride, vmix, interleaved};
-  if (pairs)
-    NV_DISPATCH_T(dtype, qk_pairs_store_kernel<T><<<dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream>>>(p));
+  if (pairs && (interleaved || rot_dims == 0))
+    NV_DISPATCH_T(dtype, qk_pairs_store_kernel<T, false><<<dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream>>>(p));
+  else if (pairs)
+    NV_DISPATCH_T(dtype, qk_pairs_store_kernel<T, true><<<dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream>>>(p));
   else
     NV_DISPATCH_T(dtype, qk_norm_store_kernel<T><<<dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream>>>(p));
   NV_CHECK_LAUNCH();
