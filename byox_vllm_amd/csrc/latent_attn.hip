@@ -56,8 +56,10 @@ __global__ __launch_bounds__(256) void latent_kv_store_kernel(const float* __res
 
 // q [tokens, H * (dim + rot_dim)] in storage type -> qa[t, h, rank .. rank + rot_dim) fp32, rotated
 constexpr int TURNS = 256;
-// One workgroup per token: its cosines and sines once in LDS (per head and number they were most of the kernel), the numbers in
-// front in fours where rows split into them (`quads`).  53 us for 11013 tokens of 16 heads of 96 + 32 then, 38 now (135 MB).
+// One workgroup per token: its cosines and sines once in LDS where a thread has more than one rotated number (per head and number
+// they were most of the kernel), the numbers in front in fours where rows split into them (`quads`).  53 us for 11013 tokens of 16
+// heads of 96 + 32 then, 38 now (135 MB).  With one number per thread the table and its barrier only cost: 16384 tokens of 4 such
+// heads 21.2 us with it, 18.7 without.
 template <typename T>
 __global__ __launch_bounds__(256) void latent_q_rope_kernel(const T* __restrict__ q, int64_t q_rs,
                                                             const int64_t* __restrict__ positions,
@@ -73,7 +75,9 @@ __global__ __launch_bounds__(256) void latent_q_rope_kernel(const T* __restrict_
     const float a = pos * inv_freq[i];
     return make_float2(cosf(a) * mscale, sinf(a) * mscale);
   };
-  for (int i = threadIdx.x; i < min(half, TURNS); i += blockDim.x) turn[i] = angle(i);
+  const bool table = H * rot_dim > (int)blockDim.x;
+  if (table)
+    for (int i = threadIdx.x; i < min(half, TURNS); i += blockDim.x) turn[i] = angle(i);
   if (copy_front && quads) {          // the unrotated numbers in front of the rotated ones (rank == dim): a whole query row
     const int per = dim / 4;
     for (int idx = threadIdx.x; idx < H * per; idx += blockDim.x) {
@@ -89,7 +93,7 @@ __global__ __launch_bounds__(256) void latent_q_rope_kernel(const T* __restrict_
       qa[(t * H + h) * (rank + rot_dim) + j] = ld_f32<T>(q + t * q_rs + (int64_t)h * (dim + rot_dim) + j) * factor;
     }
   }
-  __syncthreads();
+  if (table) __syncthreads();
   for (int idx = threadIdx.x; idx < H * rot_dim; idx += blockDim.x) {
     const int h = idx / rot_dim, j = idx % rot_dim;
     const T* src = q + t * q_rs + (int64_t)h * (dim + rot_dim) + dim;
@@ -97,7 +101,7 @@ __global__ __launch_bounds__(256) void latent_q_rope_kernel(const T* __restrict_
     if (j < rot_dims) {
       const bool first = interleaved ? (j & 1) == 0 : j < half;
       const int i = interleaved ? j >> 1 : (first ? j : j - half);
-      const float2 a = i < TURNS ? turn[i] : angle(i);
+      const float2 a = table && i < TURNS ? turn[i] : angle(i);
       const float other = ld_f32<T>(src + (interleaved ? j ^ 1 : (first ? j + half : j - half)));
       v = first ? v * a.x - other * a.y : v * a.x + other * a.y;
     }
