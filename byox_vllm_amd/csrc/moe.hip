@@ -439,8 +439,9 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const float* __restrict_
 }
 
 // V columns per thread: four where rows split into 16-byte pieces (bound by memory: 16384 rows of 2048, two choices each, 402 MB:
-// 119 us in single numbers, 69 in fours).  The rows of four choices are under way together.
-template <int V>
+// 119 us in single numbers, 69 in fours).  The rows of N choices are under way together: four, or one where a token has no more
+// (8 tokens by 7001 numbers of one choice: 9.3 us in fours, 8.0 alone).
+template <int V, int N>
 __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restrict__ y, const int32_t* __restrict__ slot_of,
                                                           const float* __restrict__ wt, int top,
                                                           const float* __restrict__ shared, const float* __restrict__ sg,
@@ -450,11 +451,11 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restric
   const float gate = !shared ? 0.0f : sg ? sigmoid_f32(sg[t * sg_rs]) : 1.0f;   // no gate logits: a plain addend
   for (int c = threadIdx.x * V; c < width; c += blockDim.x * V) {
     vec a = 0.0f;
-    for (int j = 0; j < top; j += 4) {
-      vec row[4];
-      float w[4];
+    for (int j = 0; j < top; j += N) {
+      vec row[N];
+      float w[N];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < N; ++i) {
         const int slot = j + i < top ? slot_of[t * top + j + i] : -1;
         row[i] = 0.0f;
         w[i] = 0.0f;
@@ -464,7 +465,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restric
         }
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a += w[i] * row[i];
+      for (int i = 0; i < N; ++i) a += w[i] * row[i];
     }
     if (shared) a += gate * *reinterpret_cast<const vec*>(shared + t * width + c);
     *reinterpret_cast<vec*>(out + t * width + c) = a;
@@ -563,12 +564,10 @@ extern "C" int nv_moe_combine(const float* y, const int32_t* slot_of, const floa
   NV_CHECK_ARG(tokens >= 0 && top > 0 && width > 0, "nv_moe_combine: bad shape");
   if (tokens == 0) return NV_OK;
   const bool fours = width % 4 == 0 && ((uintptr_t)y | (uintptr_t)shared | (uintptr_t)out) % 16 == 0;
-  if (fours)
-    moe_combine_kernel<4><<<dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream>>>(y, slot_of, weights, top, shared, shared_gate,
-                                                                                        shared_gate_stride, out, width);
-  else
-    moe_combine_kernel<1><<<dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream>>>(y, slot_of, weights, top, shared, shared_gate,
-                                                                                        shared_gate_stride, out, width);
+  auto kernel = fours ? (top > 1 ? moe_combine_kernel<4, 4> : moe_combine_kernel<4, 1>)
+                      : (top > 1 ? moe_combine_kernel<1, 4> : moe_combine_kernel<1, 1>);
+  kernel<<<dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream>>>(y, slot_of, weights, top, shared, shared_gate,
+                                                                       shared_gate_stride, out, width);
   NV_CHECK_LAUNCH();
   return NV_OK;
 }
