@@ -544,6 +544,26 @@ static void ssd_runs(bool chunks, int num_seqs, int heads, int max_q, int* runs,
   *runs = (max_q + *run_len - 1) / *run_len;
 }
 
+// From how many tokens of the longest request on a step goes to the chunks.  They give every (request, head) pair a workgroup of 64
+// columns and of the state's rows rounded up to 32, 64 or 128, whatever it uses of them and also for a single token; the walk costs
+// what the state holds, and about 0.5 us for each token of the longest request.  So steps of many decoding requests beside a short
+// piece stay with the walk while the pairs' excess outweighs the piece.  Walk and chunks, for 16 heads and 128 + 1 requests: 128 x 16
+// numbers 17.4 and 41.3 us with 2 tokens, 34.6 and 45.1 with 32; 32 x 16 7.6 and 13.8, 16.4 and 15.9; 128 x 48 24 % more with 2, 8 %
+// less with 32; 64 x 32 and 64 requests 3 % more with 2, 11 % less with 8; 64 x 48 and 64 x 128 from 2 on 30 to 45 % less.
+static int ssd_chunk_tokens(int dim, int vdim, int64_t pairs) {
+  int64_t n = 2;
+  if (vdim > 64) {
+    if (dim > 64 && pairs < 200) n = 3;
+  } else if (dim > 64) {
+    n = vdim > 32 ? 4 + std::min<int64_t>(24, pairs / 130) : pairs <= 300 ? 4 + pairs / 150 : std::min<int64_t>(64, pairs / 30);
+  } else if (dim > 32) {
+    if (vdim <= 32) n = vdim > 16 ? std::min<int64_t>(8, pairs / 300) : std::min<int64_t>(32, pairs / 130);
+  } else if (vdim <= 48) {
+    n = vdim > 32 ? 3 : std::min<int64_t>(48, 1 + pairs / 64);
+  }
+  return (int)std::max<int64_t>(2, n);
+}
+
 extern "C" size_t nv_ssd_scan_workspace_bytes(int num_seqs, int heads, int state_size, int vdim, int max_q) {
   int runs, more, len;
   ssd_runs(false, num_seqs, heads, max_q, &runs, &len);
@@ -583,7 +603,7 @@ extern "C" int nv_ssd_scan(const float* xbc, int64_t xbc_row_stride, const float
   }
   float* ws_state = reinterpret_cast<float*>(workspace);
   auto decays = [&](int n) { return n > 1 ? ws_state + (size_t)num_seqs * heads * n * state_size * vdim : nullptr; };
-  if (max_q > 1) {
+  if (max_q >= ssd_chunk_tokens(state_size, vdim, (int64_t)num_seqs * heads)) {
     chunk_scan::Args c{};
     const int inner = heads * vdim;
     c.q = xbc + inner + groups * state_size;

@@ -180,6 +180,26 @@ def test_state_space(H, G, n, dv, scale):
     close(runs[0][0], runs[1][0], "rows against the walk")
 
 
+@pytest.mark.parametrize("H,n,dv", [(8, 128, 16), (8, 128, 64), (8, 32, 16), (8, 64, 32), (2, 128, 128)])
+@pytest.mark.parametrize("longest", [2, 3, 17, 70])
+def test_state_space_steps_of_single_tokens_and_a_piece(H, n, dv, longest):
+    """Many decoding requests beside one piece, whichever of the two forms the step takes, against the walk asked for by max_q 1."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(n + dv + longest)
+    lens = [1] * 70 + [longest]
+    cu, past, slots = batch(lens)
+    T, inner = cu[-1], H * dv
+    data = [torch.randn(s, device=DEV) for s in ((T, inner + 2 * n), (T, inner), (T, H), (H,), (H,), (H,))]
+    state = pool(cu, past, slots, (H, n, dv), lambda: torch.randn(H, n, dv)).to(DEV)
+    runs = []
+    for max_q in (longest, 1):
+        dev = state.clone()
+        out = kernels.ssd_scan(*data, dev, i32(cu), i32(past), i32(slots), H, 1, n, dv, max_q=max_q)
+        runs.append((out, torch.stack([dev[s] for s in slots])))
+    close(runs[0][0], runs[1][0], "rows")
+    close(runs[0][1], runs[1][1], "states")
+
+
 @pytest.mark.parametrize("lens,past", [([256], [0]), ([257, 3], [5, 0]), ([511, 128, 129, 1], [0, 9, 0, 4])])
 def test_state_space_runs(lens, past):
     """Few requests with long prompts: runs side by side against one walk over the same tokens."""
