@@ -225,10 +225,11 @@ void launch_few_as(const LinArgs& p, int epi, dim3 grid, hipStream_t s) {
 // At most 64 rows.  As many sub-tiles per workgroup as leave the chip a workgroup per CU (each further workgroup reads the weights
 // again): 64 rows by 1024 columns of K = 1024 take 24 us in 64 workgroups of four sub-tiles, 7 in 256 of one.  A group of rows
 // seldom has more than 32.  Sixteen wavefronts share K where even single sub-tiles leave CUs idle and every wavefront still gets a
-// round (8 rows by 1024 columns of K = 1024 in fp32: 9.0 us on four, 6.3 on sixteen).  Where all groups together have at most 8 rows,
-// few of them have any, and the registers of a second round in flight cost more than it brings (mean over routings of 1 to 8 rows, 16
-// experts of 2048 x 3072: 13.4 us with it, 11.7 without, 32 of 1024 x 1536 6.7 and 6.1; over all sizes measured 2 to 8 rows 2 to 5 %
-// shorter without it, 10 the same, 12 to 39 2 to 4 % longer).
+// round (8 rows by 1024 columns of K = 1024 in fp32: 9.0 us on four, 6.3 on sixteen).  Of groups, few may have rows, and then the
+// registers of a second round in flight cost more than it brings, unless K is long: with at most 8 rows in all (mean over routings of
+// 1 to 8 rows, 16 experts of 2048 x 3072: 13.4 us with it, 11.7 without, 32 of 1024 x 1536 6.7 and 6.1), up to 16 rows per group below
+// K = 3072 (16 rows over 64 experts of 512 x 2048: 12.4 and 10.2 us; 10 to 39 rows over 16 of 2048 x 3072 2 to 4 % longer without),
+// of more rows below K = 2048 (64 over 64 experts of 2048 x 768: 32.5 and 26.5 us; over 16 of 512 x 2048 11 % longer without).
 template <typename T, typename TO>
 void launch_few(const LinArgs& p, int epi, int64_t total_rows, int batch, hipStream_t s) {
   const dim3 grid((unsigned)((p.N + 15) / 16), 1, (unsigned)batch);
@@ -237,11 +238,15 @@ void launch_few(const LinArgs& p, int epi, int64_t total_rows, int batch, hipStr
     else launch_few_as<T, TO, 4, 4, false>(p, epi, grid, s);
     return;
   }
+  constexpr int ROUND = 4 * Frag<T>::KS;
   const int64_t tiles = (int64_t)grid.x * batch;
   auto groups = [&](int nsub) { return tiles * ((p.M + 16 * nsub - 1) / (16 * nsub)); };
   if (p.M > 32 && !p.group_off && groups(4) >= 256) launch_few_as<T, TO, 4, 4, true>(p, epi, grid, s);
-  else if (p.M > 16 && groups(2) >= 256) launch_few_as<T, TO, 2, 4, true>(p, epi, grid, s);
-  else if (groups(1) <= 256 && p.K >= 16 * 4 * Frag<T>::KS) launch_few_as<T, TO, 1, 16, true>(p, epi, grid, s);
-  else if (p.group_off && total_rows <= 8) launch_few_as<T, TO, 1, 4, true, false>(p, epi, grid, s);
+  else if (p.M > 16 && groups(2) >= 256) {
+    if (p.group_off && p.K < 16 * ROUND) launch_few_as<T, TO, 2, 4, true, false>(p, epi, grid, s);
+    else launch_few_as<T, TO, 2, 4, true>(p, epi, grid, s);
+  }
+  else if (groups(1) <= 256 && p.K >= 16 * ROUND) launch_few_as<T, TO, 1, 16, true>(p, epi, grid, s);
+  else if (p.group_off && (total_rows <= 8 || p.K < 24 * ROUND)) launch_few_as<T, TO, 1, 4, true, false>(p, epi, grid, s);
   else launch_few_as<T, TO, 1, 4, true>(p, epi, grid, s);
 }
