@@ -25,6 +25,79 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int PA_ROWS = 128, PA_KEYS = 64;
 
+// A weight of 0 times an infinity or a NaN is NaN: a value row that is not finite reaches the rows that meet it in a tile without
+// seeing it, those ahead of it among them.  Rows that came out so (bit i of `rest`: row row0 + i of the tile's tokens from ts on) are
+// formed again by one wavefront from the keys that they see, one by one.
+template <int D, bool EXT>
+__device__ __forceinline__ void prompt_rows_again(const WAttnArgs& a, uint32_t rest, int row0, int64_t ts, int b, int g, int bs_shift) {
+  constexpr float LOG2E = 1.4426950408889634f;
+  const int lane = threadIdx.x & 63, heads = a.H / a.G, first_pos = a.past[b] + (int)(ts - a.cu_q[b]);
+  const int32_t* table = a.tables + (int64_t)b * a.table_cols;
+  const char* k_base = reinterpret_cast<const char*>(a.cache) + (int64_t)g * (2 * D);
+  const char* v_base = reinterpret_cast<const char*>(a.cache) + ((int64_t)a.v_col + (int64_t)g * D) * 2;
+#pragma unroll 1
+  for (; rest != 0; rest &= rest - 1) {
+    const int row = row0 + __ffs(rest) - 1, row_tok = row / heads, row_head = g * heads + row % heads, row_pos = first_pos + row_tok;
+    const int first = max(a.window > 0 ? row_pos - a.window + 1 : 0, EXT && a.chunk > 0 ? row_pos / a.chunk * a.chunk : 0);
+    const int from = max(first, 0), kept = EXT ? min(a.keep, from) : 0, count = kept + row_pos + 1 - from;
+    const float* qrow = a.q + ((ts + row_tok) * a.H + row_head) * D;
+    auto row_at = [&](int c) {             // byte offset of the row's c-th visible key
+      const int key = c < kept ? c : from + c - kept, n = bs_shift >= 0 ? key >> bs_shift : key / a.block_size;
+      return ((int64_t)table[n] * a.block_size + (key - n * a.block_size)) * (2 * (int64_t)a.cw);
+    };
+    auto score = [&](int c) {
+      const char* k = k_base + row_at(c);
+      float sum = 0.0f;
+#pragma unroll 1
+      for (int e = 0; e < D; e += 8) {
+        const bf16x8 x = *reinterpret_cast<const bf16x8*>(k + 2 * e);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sum = fmaf((float)(bf16_t)qrow[e + j], (float)x[j], sum);
+      }
+      return sum;
+    };
+    float m = -INFINITY;
+    bool undefined = false;
+#pragma unroll 1
+    for (int c0 = 0; c0 < count; c0 += 64) {
+      const float x = score(min(c0 + lane, count - 1));
+      m = fmaxf(m, x);
+      undefined |= x != x || x == INFINITY;
+    }
+    if (__any(undefined)) continue;        // all of the row is NaN, as stored
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+    const float m_use = m == -INFINITY ? 0.0f : m * LOG2E;
+    float l = 0.0f, acc[D / 64];
+#pragma unroll
+    for (int i = 0; i < D / 64; ++i) acc[i] = 0.0f;
+#pragma unroll 1
+    for (int c0 = 0; c0 < count; c0 += 64) {
+      const float e = c0 + lane < count ? __builtin_amdgcn_exp2f(fmaf(score(min(c0 + lane, count - 1)), LOG2E, -m_use)) : 0.0f;
+      l += e;
+#pragma unroll 1
+      for (int c = c0; c < min(c0 + 64, count); ++c) {
+        const float w = (float)(bf16_t)__shfl(e, c - c0, 64);
+        const bf16_t* v = reinterpret_cast<const bf16_t*>(v_base + row_at(c)) + lane;
+#pragma unroll
+        for (int i = 0; i < D / 64; ++i) acc[i] += w * (float)v[64 * i];
+      }
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) l += __shfl_xor(l, d, 64);
+    float fs, den;
+    close_softmax(m, l, a.sink != nullptr, a.sink ? ld_f32<bf16_t>(reinterpret_cast<const bf16_t*>(a.sink) + row_head) : 0.0f, fs, den);
+    const float f = a.out_scale * fs / den;
+    const float* gates = a.gate ? a.gate + (ts + row_tok) * a.gate_rs : nullptr;
+#pragma unroll
+    for (int i = 0; i < D / 64; ++i) {
+      const int n = row_head * D + lane + 64 * i;
+      const float on = !gates ? 1.0f : sigmoid_f32(gates[EXT && a.gate_head ? row_head : n]);
+      reinterpret_cast<bf16_t*>(a.out)[(ts + row_tok) * a.out_rs + n] = (bf16_t)(acc[i] * f * on);
+    }
+  }
+}
+
 template <int D, bool EXT>
 __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int tiles, int num_seqs, int bs_shift) {
   constexpr int KS = D / 16, DT = D / 32, ROWB = 2 * D, TILE = PA_KEYS * ROWB;      // bytes of one operand's tile
@@ -261,6 +334,13 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
       }
     }
     if (wave_on) {
+      float none[4] = {0.0f, 0.0f, 0.0f, 0.0f};       // 0 times every number: NaN where one is not finite
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) none[r & 3] = fmaf(o[dt][r], 0.0f, none[r & 3]);
+      const bool odd = !((none[0] + none[1]) + (none[2] + none[3]) == 0.0f);
+      const uint64_t odd_lanes = __ballot(odd && valid);
       float l_lo, l_hi;
       rows_pair32(l_run, l_lo, l_hi);
       if (valid) {
@@ -284,6 +364,12 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
               v[r] = o[dt][4 * q + r] * f * (grow ? sigmoid_f32(grow[32 * dt + 8 * q + r]) : 1.0f);
             *reinterpret_cast<uint2*>(orow + 32 * dt + 8 * q) = Pack4<bf16_t>::narrow(v);
           }
+      }
+      if (odd_lanes != 0) {
+        uint64_t args = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(args));         // read again: kept in registers, the arguments slow the walk
+        prompt_rows_again<D, EXT>(*reinterpret_cast<const WAttnArgs*>(args), (uint32_t)(odd_lanes | odd_lanes >> 32), row0, ts, b, g,
+                                  bs_shift);
       }
     }
     ts = te;

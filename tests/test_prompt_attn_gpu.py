@@ -122,6 +122,54 @@ def test_steps_of_single_tokens_and_pieces(D, R, G, window, keep):
         assert (got - want).norm() <= 2.0 ** -8 * want.norm()
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("options", CASES)
+@pytest.mark.parametrize("D,R,G", [(128, 2, 2), (64, 3, 1)])
+def test_a_value_that_is_not_finite_stays_out_of_rows_that_do_not_see_it(D, R, G, options, bad):
+    """One number of one token's value row is an infinity or a NaN: tokens ahead of it, and those it is out of the window or the
+    chunk of, keep their rows; the others have one number per head that is not finite."""
+    from byox_vllm_amd import kernels
+    window, keep, chunk, with_sink, gate_form, same = options
+    torch.manual_seed(D + R)
+    block, H, past, new = 48, R * G, [70, 0], [180, 40]
+    pages = [-(-(a + b) // block) for a, b in zip(new, past)]
+    order, tables = torch.randperm(sum(pages)).tolist(), []
+    for n in pages:
+        tables.append([order.pop() for _ in range(n)])
+    cache = torch.randn(sum(pages) * block, G * D if same else 2 * G * D).to(torch.bfloat16)
+    T, cols = sum(new), max(pages)
+    q = torch.randn(T, H * D, device=DEV) * D ** -0.5 * 2.0
+    sink = torch.randn(H, device=DEV).to(torch.bfloat16) if with_sink else None
+    gate = torch.randn(T, H if gate_form == "head" else H * D, device=DEV) if gate_form else None
+    ints = (i32([t + [0] * (cols - len(t)) for t in tables]), i32([0, new[0], T]), i32(past), i32([0] * new[0] + [1] * new[1]))
+
+    def rows(c):
+        out = torch.zeros(T, H * D, dtype=torch.bfloat16, device=DEV)
+        kernels.paged_softmax_attn(q, c.to(DEV), *ints, max(new), H, G, D, D, block, out, window=window, keep_first=keep, chunk=chunk,
+                                   sink=sink, gate=gate, gate_per_head=gate_form == "head", values_are_keys=same)
+        return out.double().cpu().view(T, H, D)
+    want = rows(cache)
+    for at in (0, 69, 70, 133, 200, 249):               # position in the first request
+        spoilt = cache.clone()
+        spoilt[tables[0][at // block] * block + at % block, (0 if same else G * D) + 5] = bad       # head 0's sixth number
+        got = rows(spoilt)
+        i = torch.arange(past[0], past[0] + new[0])
+        sees = i >= at
+        if window:
+            sees &= (i - at < window) | (at < keep)
+        if chunk:
+            sees &= i // chunk == at // chunk
+        sees = torch.cat([sees, torch.zeros(new[1], dtype=torch.bool)])
+        # probabilities of rows formed again are summed in another order; one rounding of the result
+        near = (got - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -9
+        assert near[~sees].all(), at
+        assert near[:, R:].all(), at
+        assert not torch.isfinite(got[sees][:, :R, 5]).any(), at
+        if not same:                                    # (a key that is not finite spoils the row's scores)
+            others = [n for n in range(D) if n != 5]
+            assert near[sees][:, :R][..., others].all(), at
+
+
 @pytest.mark.parametrize("interleaved", [False, True])
 @pytest.mark.parametrize("dim,vdim,rot", [(64, 64, 32), (128, 64, 128), (20, 12, 8), (24, 24, 12), (16, 8, 0)])
 def test_rotating_store(dim, vdim, rot, interleaved):
