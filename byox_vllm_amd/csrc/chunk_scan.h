@@ -25,6 +25,7 @@
 // state-space heads, for the sake of the second workgroup.
 #pragma once
 #include "anyt.h"
+#include "lds_limit.h"
 
 namespace chunk_scan {
 
@@ -616,8 +617,8 @@ hipError_t launch_one(const Args& p, int num_seqs, int runs, hipStream_t s) {
   constexpr size_t lds = lds_floats<D, NW>() * sizeof(float);
   static_assert(lds <= 160 * 1024, "the chunk fits the LDS");
   if (lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&chunk_scan_kernel<MODE, T, D, NW>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    static std::atomic<uint64_t> devices{0};
+    const hipError_t e = allow_lds(reinterpret_cast<const void*>(&chunk_scan_kernel<MODE, T, D, NW>), lds, devices);
     if (e != hipSuccess) return e;
   }
   chunk_scan_kernel<MODE, T, D, NW><<<dim3(p.H, num_seqs, runs), dim3(64 * NW), lds, s>>>(p);

@@ -16,6 +16,7 @@
 // is position * inv_freq[i] in fp32, and both cosine and sine are multiplied by `mscale` (the caller folds frequency
 // scaling into inv_freq and mscale).
 #include "anyt.h"
+#include "lds_limit.h"
 
 namespace {
 

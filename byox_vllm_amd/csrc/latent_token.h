@@ -205,8 +205,8 @@ template <int KS>
 hipError_t launch_latent_token(const MfmaAttnArgs& q, int64_t tokens, hipStream_t s) {
   constexpr size_t lds = (size_t)4 * KS * 2048;
   if (lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_token_kernel<KS>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    static std::atomic<uint64_t> devices{0};
+    const hipError_t e = allow_lds(reinterpret_cast<const void*>(&latent_token_kernel<KS>), lds, devices);
     if (e != hipSuccess) return e;
   }
   int shift = -1;

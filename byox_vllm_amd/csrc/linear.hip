@@ -14,6 +14,7 @@
 #include <stdlib.h>
 
 #include "anyt.h"
+#include "lds_limit.h"
 
 namespace {
 

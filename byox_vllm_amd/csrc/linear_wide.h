@@ -260,8 +260,8 @@ hipError_t launch_wide_one(const LinArgs& p, int64_t total_rows, int batch, hipS
   constexpr int BM = 32 * MT * WM, BN = 64 * WN, NOUT = EPI == EPI_GLU ? BN / 2 : BN;
   constexpr size_t lds = STAGES * (size_t)(BM + BN) * 128;
   if (lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&linear_wide_kernel<T, TO, EPI, MT, WM, WN, STAGES>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    static std::atomic<uint64_t> devices{0};
+    const hipError_t e = allow_lds(reinterpret_cast<const void*>(&linear_wide_kernel<T, TO, EPI, MT, WM, WN, STAGES>), lds, devices);
     if (e != hipSuccess) return e;
   }
   const int64_t nt = (p.N + NOUT - 1) / NOUT;
