@@ -1,7 +1,7 @@
 // nv_linear, up to 64 rows per (group of) product; included by linear.hip.
 //
 // Such a launch is bound by how many weight loads are in flight.  A workgroup owns ONE 16-column tile and its NW wavefronts split K
-// between them; the partial sums meet in LDS and wavefront 0 finishes.  Rows and columns that are not there read the first one's
+// between them; the partial sums meet in LDS and wavefront i finishes the i-th sixteen rows.  Rows and columns that are not there read the first one's
 // numbers instead (their products are never stored), so the loop carries no branch and the loads of a round are all under way
 // together.  Tested per lane and piece, every load was waited for by itself (K 1024 and 2048, bf16 but for the second): 64 rows by
 // 16 columns 11.4 us then, 4.2 now; by 1024 columns in fp32 24.3 and 7.1; by 2 x 8192 gated columns 65.6 and 29.5; 8 rows by the
@@ -224,12 +224,14 @@ void launch_few_as(const LinArgs& p, int epi, dim3 grid, hipStream_t s) {
 
 // At most 64 rows.  As many sub-tiles per workgroup as leave the chip a workgroup per CU (each further workgroup reads the weights
 // again): 64 rows by 1024 columns of K = 1024 take 24 us in 64 workgroups of four sub-tiles, 7 in 256 of one.  A group of rows
-// seldom has more than 32.  Sixteen wavefronts share K where even single sub-tiles leave CUs idle and every wavefront still gets a
-// round (8 rows by 1024 columns of K = 1024 in fp32: 9.0 us on four, 6.3 on sixteen).  Of groups, few may have rows, and then the
+// seldom has more than 32 (two sub-tiles for up to 32 rows also where they leave a quarter of the CUs idle: 20 rows over 4 experts of
+// 2 x 768 x 1024 7.4 us in single ones, 5.8; in 128 workgroups 6.3 and 8.0).  Sixteen wavefronts share K where even single
+// sub-tiles leave CUs idle and every wavefront still gets a round (8 rows by 1024 columns of K = 1024 in fp32: 9.0 us on four, 6.3 on sixteen).  Of groups, few may have rows, and then the
 // registers of a second round in flight cost more than it brings, unless K is long: with at most 8 rows in all (mean over routings of
 // 1 to 8 rows, 16 experts of 2048 x 3072: 13.4 us with it, 11.7 without, 32 of 1024 x 1536 6.7 and 6.1), up to 16 rows per group below
 // K = 3072 (16 rows over 64 experts of 512 x 2048: 12.4 and 10.2 us; 10 to 39 rows over 16 of 2048 x 3072 2 to 4 % longer without),
-// of more rows below K = 2048 (64 over 64 experts of 2048 x 768: 32.5 and 26.5 us; over 16 of 512 x 2048 11 % longer without).
+// of more rows below K = 1024, or 1536 from 32 groups on (64 over 64 experts of 2048 x 768: 32.5 and 26.5 us; 16 experts of 768 x 1024
+// 3 to 12 % longer without, 32 of them 6 % shorter).
 template <typename T, typename TO>
 void launch_few(const LinArgs& p, int epi, int64_t total_rows, int batch, hipStream_t s) {
   const dim3 grid((unsigned)((p.N + 15) / 16), 1, (unsigned)batch);
@@ -242,8 +244,8 @@ void launch_few(const LinArgs& p, int epi, int64_t total_rows, int batch, hipStr
   const int64_t tiles = (int64_t)grid.x * batch;
   auto groups = [&](int nsub) { return tiles * ((p.M + 16 * nsub - 1) / (16 * nsub)); };
   if (p.M > 32 && !p.group_off && groups(4) >= 256) launch_few_as<T, TO, 4, 4, true>(p, epi, grid, s);
-  else if (p.M > 16 && groups(2) >= 256) {
-    if (p.group_off && p.K < 16 * ROUND) launch_few_as<T, TO, 2, 4, true, false>(p, epi, grid, s);
+  else if (p.M > 16 && groups(2) >= (p.group_off && p.M <= 32 ? 192 : 256)) {
+    if (p.group_off && p.K < (batch < 32 ? 8 : 12) * ROUND) launch_few_as<T, TO, 2, 4, true, false>(p, epi, grid, s);
     else launch_few_as<T, TO, 2, 4, true>(p, epi, grid, s);
   }
   else if (groups(1) <= 256 && p.K >= 16 * ROUND) launch_few_as<T, TO, 1, 16, true>(p, epi, grid, s);
