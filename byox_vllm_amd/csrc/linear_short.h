@@ -7,7 +7,8 @@
 // 300 rows by 256 columns of K = 16 with a soft cap: 13.8 us with four tiles, 5.5 with one, 8.6 in the kernel for any K).  Four,
 // 256 columns per workgroup, where every CU has a workgroup all the same and the rows' fragments are two: they are read once for all
 // the columns then (bf16, 16384 rows by 2048 columns of K = 64: 43.6 us with one tile, 34.3 with four; K = 32: 25.0 and 28.7).
-// 16384 rows by 1000 columns of K = 32 in bf16, fp32 result, alone: 54.9 us on the LDS tiles, 20.5 with four tiles per wavefront, 16.3
+// 16384 rows by 1000 columns of K = 32 in bf16, fp32 result, alone (21 us inside a layer, where the result finds other rows in the
+// caches): 54.9 us on the LDS tiles, 20.5 with four tiles per wavefront, 16.3
 // with one (67 MB: 4.1 TB/s).
 #pragma once
 

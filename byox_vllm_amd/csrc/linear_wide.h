@@ -5,8 +5,9 @@
 // rate, waiting at a barrier every 16 matrix instructions.  Here
 //   * a K block is 128 bytes of every row (64 bf16, 32 fp32): 64 matrix instructions per wavefront and barrier at 256 x 256;
 //   * the following blocks' rows go from L2 straight into the other LDS buffers (global_load_lds, 16 bytes per lane) while a
-//     block is multiplied; no staging registers, no LDS store instructions.  Two buffers fit beside 256 x 256 outputs; the
-//     smaller tiles have three, because there a block is multiplied faster than one arrives;
+//     block is multiplied; no staging registers, no LDS store instructions.  Two buffers fit where tiles of 256 x 256
+//     have a CU each and those of 128 x 128 share one in pairs; tiles of 64 x 128 have three, because there a block is
+//     multiplied faster than one arrives;
 //   * LDS rows are 128 bytes apart and their 16-byte pieces are dealt by XOR with half the row number, through the DMA's
 //     source addresses, so the 16 rows that one read phase touches lie in 16 different bank groups;
 //   * fragments of the next step of K are read while the current step's matrix instructions run (two register sets);
@@ -14,9 +15,10 @@
 // Groups (experts) of unknown size: the grid covers the largest possible number of tiles, every workgroup finds its group
 // from the offsets with one wavefront-wide prefix sum, and the surplus leaves at once.
 //
-// Measured, before and after: sixteen experts, 32768 rows of them, gated up 2048 -> 2 x 3072 1467 and 940 us (0.88 PFLOP/s; groups
-// of equal size 907: a group that ends inside a 256-row tile costs a round), down 786 and 502; fp32, 3135 rows 1024 -> 4416 without
-// LDS 543 and 270 us (105 TFLOP/s); bf16, 1000 rows 2048 -> 1024 23 us with two LDS buffers on 128 x 128 tiles, 18.6 with three.
+// Measured alone, before and after: sixteen experts, 32768 rows of them, gated up 2048 -> 2 x 3072 1467 and 1005 us (0.82 PFLOP/s; groups
+// of equal size 910: a group that ends inside a 256-row tile costs a round), down 786 and 497; fp32, 3135 rows 1024 -> 4416 without
+// LDS 543 and 275 us (103 TFLOP/s); bf16, 1000 rows 2048 -> 1024 27 us on tiles of 128 x 128, 19 on 64 x 128.  Inside a layer under
+// the profiler the first two take 1140 and 565 us, the third 297.
 #pragma once
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
