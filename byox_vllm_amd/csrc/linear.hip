@@ -3,7 +3,7 @@
 // (nv_gemm) does not take: K or N that are no multiples of its tiles, fp32 models, batched products with one weight
 // per head, grouped products with one weight per expert over gathered rows, and the gated epilogues.
 //
-// linear_wide.h serves more than 64 rows whose K splits into 128-byte blocks, linear_short.h many rows by a K below that,
+// linear_stream.h and linear_wide.h serve more than 64 rows whose K splits into 128-byte blocks, linear_short.h many rows by a K below that,
 // linear_few.h up to 64 rows; linear_tile_kernel below the other aligned bf16 products of many rows, linear_kernel the rest.
 //
 // linear_kernel: a workgroup owns a 64 x 64 tile of the output: wavefront w the 16 columns n0 + 16 w .. and all four 16-row
@@ -429,8 +429,9 @@ extern "C" int nv_linear_rows(const void* a, int64_t a_row_stride, const int32_t
                               : (epilogue == EPI_SOFTCAP || epilogue == EPI_ACT) && K <= 64 && tiles64 < 96);
   if (M > 64 && p.vec_a && p.vec_w && (K * esz) % 128 == 0 && !stays && getenv("NV_LINEAR_TILE_OFF") == nullptr) {
     const int cols = epilogue == EPI_GLU ? 2 * N : N;
-    int tile = pick_wide_tile(M, total_rows, cols, batch, group_offsets != nullptr, dtype == NV_BF16);
-    if (const char* force = getenv("NV_LINEAR_TILE")) tile = atoi(force);
+    const bool has_256 = dtype == NV_BF16 && stream_takes(p, total_rows, batch, cols);
+    int tile = pick_wide_tile(M, total_rows, cols, batch, group_offsets != nullptr, has_256);
+    if (const char* force = getenv("NV_LINEAR_TILE")) tile = atoi(force) == TILE_256 && !has_256 ? TILE_128 : atoi(force);
     if (wide_tiles(64, 128, M, total_rows + 64 * batch, cols, batch, group_offsets != nullptr) < (1 << 30)) {
       hipError_t e;
       if (dtype == NV_BF16) {

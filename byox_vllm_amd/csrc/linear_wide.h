@@ -1,13 +1,11 @@
-// nv_linear for many rows: tiles of BM x BN outputs with both operands in LDS, filled by LDS-DMA.  Included by linear.hip.
+// nv_linear for many rows: tiles of BM x BN outputs with both operands in LDS, filled by LDS-DMA.  Included by linear.hip.  These
+// serve fp32, and 16 bits where tiles of 256 x 256 (linear_stream.h) would leave much of the chip idle.
 //
-// What bounds it: at 2048 rows per expert the products are 2 x 128 flops per byte that a 256 x 256 tile moves, so the matrix
-// cores; the kernel it replaces there (128 x 128 tiles, K in blocks of 32 through registers) reached a quarter of their
-// rate, waiting at a barrier every 16 matrix instructions.  Here
-//   * a K block is 128 bytes of every row (64 bf16, 32 fp32): 64 matrix instructions per wavefront and barrier at 256 x 256;
+// What bounds it: the matrix cores, and for small products the latency of one round of tiles.
+//   * A K block is 128 bytes of every row (64 bf16, 32 fp32);
 //   * the following blocks' rows go from L2 straight into the other LDS buffers (global_load_lds, 16 bytes per lane) while a
-//     block is multiplied; no staging registers, no LDS store instructions.  Two buffers fit where tiles of 256 x 256
-//     have a CU each and those of 128 x 128 share one in pairs; tiles of 64 x 128 have three, because there a block is
-//     multiplied faster than one arrives;
+//     block is multiplied; no staging registers, no LDS store instructions.  Tiles of 128 x 128 share a CU in pairs with two buffers
+//     each; tiles of 64 x 128 have three, because there a block is multiplied faster than one arrives;
 //   * LDS rows are 128 bytes apart and their 16-byte pieces are dealt by XOR with half the row number, through the DMA's
 //     source addresses, so the 16 rows that one read phase touches lie in 16 different bank groups;
 //   * fragments of the next step of K are read while the current step's matrix instructions run (two register sets);
@@ -15,33 +13,12 @@
 // Groups (experts) of unknown size: the grid covers the largest possible number of tiles, every workgroup finds its group
 // from the offsets with one wavefront-wide prefix sum, and the surplus leaves at once.
 //
-// Measured alone, before and after: sixteen experts, 32768 rows of them, gated up 2048 -> 2 x 3072 1467 and 1005 us (0.82 PFLOP/s; groups
-// of equal size 910: a group that ends inside a 256-row tile costs a round), down 786 and 497; fp32, 3135 rows 1024 -> 4416 without
-// LDS 543 and 275 us (103 TFLOP/s); bf16, 1000 rows 2048 -> 1024 27 us on tiles of 128 x 128, 19 on 64 x 128.  Inside a layer under
-// the profiler the first two take 1140 and 565 us, the third 297.
+// Measured alone, before (without LDS) and after: fp32, 3135 rows 1024 -> 4416 543 and 275 us (103 TFLOP/s; 297 inside a layer under the
+// profiler); bf16, 1000 rows 2048 -> 1024 27 us on tiles of 128 x 128, 19 on 64 x 128.
 #pragma once
+#include "linear_stream.h"
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-// value(s) of one output -> what is stored (bias, activation, gate); `gate`: the row's, where there is one for all of it
-template <typename T, int EPI>
-__device__ __forceinline__ float lin_finish(const LinArgs& p, const T* bias, float v, float u, float rsc, float gate, int64_t s, int n,
-                                            int z) {
-  v *= rsc;
-  if (bias) v += ld_f32<T>(bias + n);
-  if constexpr (EPI == EPI_GLU) {
-    u *= rsc;
-    if (bias) u += ld_f32<T>(bias + p.N + n);
-    v = glu_act(v, u, p.act, p.epi_c);
-  } else if constexpr (EPI == EPI_SOFTCAP) {
-    v = p.epi_c * tanhf(v / p.epi_c);
-  } else if constexpr (EPI == EPI_ROW_GATE) {
-    v *= p.act ? sigmoid_f32(p.epi_ptr[s * p.epi_rs + (int64_t)z * p.N + n]) : gate;
-  } else if constexpr (EPI == EPI_ACT) {
-    v = unary_act(v, p.act, p.epi_ptr, p.epi_c);
-  }
-  return v;
-}
 
 __device__ __forceinline__ f32x16 mma32(const u32x4& a, const u32x4& b, f32x16 c, bf16_t) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
@@ -274,8 +251,10 @@ hipError_t launch_wide_one(const LinArgs& p, int64_t total_rows, int batch, hipS
 }
 
 // Which tile: the one whose launch takes the fewest chip-wide rounds of tile area, each by what it reaches when the chip is
-// full (bf16, 32768 rows by 6144 columns of K 2048 in 16 groups: 917, 742 and 608 TFLOP/s; a workgroup of 256 x 256 has a CU
-// to itself, of the others two share one).  fp32 has the two smaller ones: its slower matrix instructions hide the loads.
+// full (bf16, 32768 rows by 6144 columns of K 2048: 1150 TFLOP/s in the streams of 256 x 256, which have a CU to themselves; 742 and
+// 608 in the others, of which two share one).  A last round of 256 x 256 that half of the chip would have is dealt in halves and
+// costs 0.85 of a round (12000 rows by 2048, K 1024, 1.5 rounds: 65 us, 128 x 128 93, 64 x 128 88; 4096 by 2048, half a round:
+// 29.4, 29.3, 33; 5000 by 1536, K 1536: 38, 34, 43).  fp32 has the two smaller ones: its slower matrix instructions hide the loads.
 enum { TILE_256 = 2, TILE_128 = 1, TILE_64 = 0 };
 inline int64_t wide_tiles(int bm, int bn, int64_t m, int64_t total_rows, int cols, int batch, bool grouped) {
   // groups end inside a tile: half a tile each on average
@@ -283,10 +262,11 @@ inline int64_t wide_tiles(int bm, int bn, int64_t m, int64_t total_rows, int col
 }
 inline int pick_wide_tile(int64_t m, int64_t total_rows, int cols, int batch, bool grouped, bool has_256) {
   auto cost = [&](int bm, int bn, int per_cu, double reached) {
-    const int64_t slots = 256 * per_cu, rounds = (wide_tiles(bm, bn, m, total_rows, cols, batch, grouped) + slots - 1) / slots;
-    return (double)rounds * per_cu * bm * bn / reached;
+    const int64_t slots = 256 * per_cu, tiles = wide_tiles(bm, bn, m, total_rows, cols, batch, grouped), over = tiles % slots;
+    const double last = over == 0 ? 0.0 : bm == 256 && 2 * over <= slots ? 0.85 : 1.0;
+    return ((double)(tiles / slots) + last) * per_cu * bm * bn / reached;
   };
-  const double c64 = cost(64, 128, 2, 608), c128 = cost(128, 128, 2, 742), c256 = cost(256, 256, 1, 917);
+  const double c64 = cost(64, 128, 2, 608), c128 = cost(128, 128, 2, 742), c256 = cost(256, 256, 1, 1150);
   if (has_256 && c256 < c128 && c256 < c64) return TILE_256;
   return c128 < c64 ? TILE_128 : TILE_64;
 }
@@ -294,7 +274,7 @@ inline int pick_wide_tile(int64_t m, int64_t total_rows, int cols, int batch, bo
 template <typename T, typename TO, int EPI>
 hipError_t launch_wide_epi(const LinArgs& p, int64_t total_rows, int batch, int tile, hipStream_t s) {
   if constexpr (sizeof(T) == 2) {
-    if (tile == TILE_256) return launch_wide_one<T, TO, EPI, 4, 2, 4, 2>(p, total_rows, batch, s);
+    if (tile == TILE_256) return launch_stream_epi<TO, EPI>(p, total_rows, batch, s);
   }
   if (tile == TILE_128) return launch_wide_one<T, TO, EPI, 2, 2, 2, 2>(p, total_rows, batch, s);
   return launch_wide_one<T, TO, EPI, 1, 2, 2, 3>(p, total_rows, batch, s);

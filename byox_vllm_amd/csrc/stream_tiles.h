@@ -1,0 +1,265 @@
+// Products of many rows, 16-bit operands: a workgroup per CU walks tiles of 32 MT x 64 NT outputs whose K blocks form one stream.
+//
+// What bounds it: the matrix cores and, on this part, their power: at 8192 x 8192 x 8192 the loop that this one replaced (a block
+// fetched, waited for and multiplied behind one barrier, 32 x 32 products) kept them 56 % busy at 1.76 GHz, the vendor library's
+// 87 % at 1.59.  What the loop spent beside them, from copies that leave one activity out (8192^3, us): whole 882, operands always
+// from the same cache lines 719, no LDS reads 716, no DMA 669, none of these and no barriers 505.  So
+//   * 16 x 16 x 32 products: a lane's results lie where whole 64-byte pieces of rows can be stored (14592 rows by 4096, K 1024: 143
+//     us with 32 x 32 products, 125 with these);
+//   * the barrier stands before the block's last step of K, whose fragments are in registers: behind it the first fragments of the
+//     next block are read under that step's products, and the buffer just left is refilled, one DMA instruction behind every few
+//     products (with all of them behind the reads: 846 us at 8192^3, so 796);
+//   * the order of products, LDS reads and DMA is fixed in the source (sched_barrier); left alone, the compiler puts the reads
+//     behind two thirds of the products and waits for them at once;
+//   * workgroups stay: the first two blocks of the next tile are on their way while the results of a tile are stored, and nothing
+//     waits for those stores but the second block after them (14592 by 4096, K 1024: 129 us with a workgroup per tile, so 117).
+//     Their tiles are found once, by a thread each, and kept in LDS: found in the loop they cost it its registers.
+// Measured, before and after: sixteen experts, 32768 rows of them, gated up 2048 -> 2 x 3072 and down, the layer 1584 and 1418 us;
+// 16384 rows 2048 -> 6144 into fp32 429 and 372 us (1110 TFLOP/s).
+// LDS rows are 128 bytes, their 16-byte pieces dealt by XOR with half the row number (through the DMA's source addresses): the 16
+// rows that a read touches lie in 16 bank groups.  Tiles go to the XCDs in contiguous eighths, within them in bands of eight row
+// tiles, so the 32 workgroups of an XCD share 8 row and 4 column panels in its L2.  A group's short last row tile stays in its band
+// (at the end of everything, its column panels come from memory again: the experts' layer 1450 us against 1418).
+//
+// Job (what is multiplied and what becomes of it) provides:
+//   T, NSTORE (stores of one wavefront for a whole tile), K (elements, a multiple of 64, at least 128)
+//   int count(lane)                       how many tiles there are
+//   StreamTile find(tile, lane)           which rows and columns the thread's tile has (every thread of a wavefront calls it)
+//   const void* a_base(tile); uint32_t a_row(tile, r); uint32_t a_stride()      row r of the tile's A rows (those past the end
+//                                         repeat a real one) lies at base + row * stride bytes, its K in 16-byte pieces
+//   w_base, w_row, w_stride               the same of row r of the W tile in LDS
+//   uint32_t w_lane(r, piece), w_step()   bytes from the row to its piece 0..7 of the first K block; and to the next K block
+//   bool whole(tile)                      every store of a wavefront is executed for this tile
+//   void store<NT, MT>(tile, first row, first column's wavefront, lane, acc)
+#pragma once
+#include "anyt.h"
+#include "lds_limit.h"
+
+struct alignas(16) StreamTile {
+  int lo, hi;       // first row of the tile; end of the rows it may touch
+  int n0, z;        // first column; which product of a batch or which group
+};
+constexpr int STREAM_LIST = 512;      // tiles of one workgroup at most
+
+__device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x4 c, bf16_t) {
+  return mfma16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c);
+}
+__device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x4 c, f16_t) {
+  return mfma16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c);
+}
+
+// column, within 32, of LDS row r: 16-bit results are stored eight to a lane, from two products of the same rows
+template <bool PAIRED> __device__ __forceinline__ int stream_column(int r) {
+  if constexpr (!PAIRED) return r;
+  return 8 * ((r & 15) >> 2) + 4 * (r >> 4) + (r & 3);
+}
+
+// place `in` of a group of `rows` row tiles by `cols` column tiles: bands of eight row tiles (the last of up to fifteen), rows first
+__device__ __forceinline__ void stream_order(int in, int rows, int cols, int& m_tile, int& n_tile) {
+  const int bands = max(1, rows >> 3), band = min(in / (8 * cols), bands - 1), first = 8 * band;
+  const int wide = band == bands - 1 ? rows - first : 8;
+  in -= first * cols;
+  m_tile = first + in % wide;
+  n_tile = in / wide;
+}
+
+// the lane's number, formed where it is used: what depends on it alone is not kept in registers through the loop over blocks
+__device__ __forceinline__ int stream_lane() {
+  uint32_t all = ~0u;
+  asm volatile("" : "+s"(all));
+  return (int)__builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0));
+}
+
+template <int MT, int NT, typename Job>
+__global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef typename Job::T T;
+  constexpr int BM = 32 * MT, BN = 64 * NT, BO = (BM + BN) * 128;       // BO: bytes of one buffer
+  constexpr int AG = BM / 64, WG = BN / 64, D = AG + WG;                // DMA instructions (8 rows each) of a wavefront per block
+  constexpr int P = MT * NT, R = MT + NT;                               // products and fragment reads of a step
+  typedef __attribute__((address_space(1))) void global_void;
+  typedef __attribute__((address_space(3))) void lds_void;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+  const int lane = stream_lane(), wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wv >> 2, wn = wv & 3;                                  // a SIMD has one wavefront of each half of the rows
+
+  // -------- this workgroup's tiles: every per-th of its XCD's.  A last round that at most half of the workgroups would have is dealt
+  // as tiles of half the rows.  One thread finds one tile; the list is in LDS.
+  StreamTile* const list = reinterpret_cast<StreamTile*>(lds_raw + 2 * BO);
+  int tiles;
+  {
+    const int per = gridDim.x >> 3, xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int64_t all = job.count(lane);
+    const int first = (int)(all * xcd >> 3), mine_all = (int)(all * (xcd + 1) >> 3) - first, over = mine_all % per;
+    const int halves = 2 * over <= per ? 2 * over : 0, rounds = halves ? mine_all - over : mine_all, end = rounds + halves;
+    tiles = slot < end ? (end - slot + per - 1) / per : 0;
+    if (tiles == 0) return;
+    const int t = min(slot + (int)threadIdx.x * per, end - 1), h = t - rounds;
+    StreamTile mine = job.find(first + (h < 0 ? t : rounds + (h >> 1)), lane);
+    if (h >= 0) {
+      mine.lo += (h & 1) * (BM / 2);
+      mine.hi = min(mine.hi, mine.lo + BM / 2);      // the second half of a short tile has no rows
+    }
+    list[threadIdx.x] = mine;
+    __syncthreads();
+  }
+  auto listed = [&](int n) {
+    const StreamTile at = list[n];
+    return StreamTile{__builtin_amdgcn_readfirstlane(at.lo), __builtin_amdgcn_readfirstlane(at.hi),
+                      __builtin_amdgcn_readfirstlane(at.n0), __builtin_amdgcn_readfirstlane(at.z)};
+  };
+
+  // -------- the stream of blocks
+  const uint32_t a_stride = job.a_stride(), w_stride = job.w_stride(), w_step = job.w_step();
+  uint32_t arow[AG], wrow[WG];
+  uint64_t apos, wpos;            // where the next K block begins, less what depends on the lane
+  auto point = [&](const StreamTile& at) {
+
+    const int r0 = 8 * wv + (stream_lane() >> 3);
+#pragma unroll
+    for (int i = 0; i < AG; ++i) arow[i] = job.a_row(at, r0 + 64 * i);
+#pragma unroll
+    for (int i = 0; i < AG; ++i) asm volatile("" : "+v"(arow[i]));      // a gathered row's number is waited for here, not at each fetch
+#pragma unroll
+    for (int i = 0; i < WG; ++i) wrow[i] = job.w_row(at, r0 + 64 * i);
+    apos = reinterpret_cast<uint64_t>(job.a_base(at));
+    wpos = reinterpret_cast<uint64_t>(job.w_base(at));
+  };
+  // DMA instruction i fills LDS rows 8 (wv + 8 i) + l / 8, whose place among the XORs is the same for every i
+  uint32_t alane, wlane;
+  auto lanes = [&]() {
+    const int l = stream_lane(), r0 = 8 * wv + (l >> 3), piece = (l & 7) ^ ((r0 >> 1) & 7);
+    alane = 16 * piece;
+    wlane = job.w_lane(r0, piece);
+  };
+  auto fill = [&](int bo, int i) {
+    if (i < AG) {
+      const int q = i < AG ? i : 0;
+      __builtin_amdgcn_global_load_lds((global_void*)(apos + (uint64_t)arow[q] * a_stride + alane), (lds_void*)(lds_raw + bo + (wv + 8 * q) * 1024),
+                                       16, 0, 0);
+    } else {
+      const int q = i < AG ? 0 : i - AG;
+      __builtin_amdgcn_global_load_lds((global_void*)(wpos + (uint64_t)wrow[q] * w_stride + wlane),
+                                       (lds_void*)(lds_raw + bo + BM * 128 + (wv + 8 * q) * 1024), 16, 0, 0);
+    }
+    if (i == AG - 1) apos += 128;
+    if (i == D - 1) wpos += w_step;
+  };
+  // where this lane's first fragments of W and A lie in the buffer at `bo`; formed for every step anew (registers).  Every fragment
+  // starts at a multiple of 16 rows.
+  auto fragments = [&](int bo, int step, int& wat, int& aat) {
+    const int l = stream_lane(), fr = l & 15, in = bo + fr * 128 + 16 * (((4 * step + (l >> 4)) ^ (fr >> 1)) & 7);
+    wat = in + (BM + 16 * NT * wn) * 128;
+    aat = in + 16 * MT * wm * 128;
+  };
+  u32x4 wf[2][NT], af[2][MT];
+  auto read = [&](int wat, int aat, int r, int set) {
+    if (r < NT) wf[set][r < NT ? r : 0] = *reinterpret_cast<const u32x4*>(lds_raw + wat + 2048 * r);
+    else af[set][r < NT ? 0 : r - NT] = *reinterpret_cast<const u32x4*>(lds_raw + aat + 2048 * (r - NT));
+  };
+
+  f32x4 acc[NT][MT];
+  auto clear = [&]() {
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int i = 0; i < MT; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  clear();
+
+  const int blocks = job.K / 64;
+  StreamTile at = listed(0), ahead = at;
+  point(at);
+  lanes();
+#pragma unroll
+  for (int i = 0; i < D; ++i) fill(0, i);
+#pragma unroll
+  for (int i = 0; i < D; ++i) fill(BO, i);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(D) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  int wat, aat;
+  fragments(0, 0, wat, aat);
+#pragma unroll
+  for (int r = 0; r < R; ++r) read(wat, aat, r, 0);
+  int fetched = 2, left = blocks, tile = 0, next = 0, bo = 0;
+  bool stored = false, live = at.lo + 16 * MT * wm < at.hi;
+
+  for (;;) {
+    if (fetched == blocks) {        // the stream goes on with the next tile; behind the last one with that one again, unused
+      fetched = 0;
+      if (next + 1 < tiles) ahead = listed(++next);
+      point(ahead);
+    }
+    if (live) {
+      fragments(bo, 1, wat, aat);
+#pragma unroll
+      for (int m = 0; m < P; ++m) {
+        acc[m % NT][m / NT] = stream_mma(wf[0][m % NT], af[0][m / NT], acc[m % NT][m / NT], T{});
+        if (m == 0) __builtin_amdgcn_sched_barrier(0);       // or the first product waits for the first of these reads
+        if (m < R) read(wat, aat, m, 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {       // the second set holds nothing then: said so, or its registers stay taken around the loop
+#pragma unroll
+      for (int j = 0; j < NT; ++j) asm volatile("" : "=v"(wf[1][j]));
+#pragma unroll
+      for (int i = 0; i < MT; ++i) asm volatile("" : "=v"(af[1][i]));
+    }
+    // this wavefront's part of the next block has arrived and it has read the last of this one; then everybody has.  Behind a
+    // whole tile's stores only what came before them is waited for: loads and stores are counted in the order of their issue.
+    if (stored) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(Job::NSTORE) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    fragments(BO - bo, 0, wat, aat);
+    lanes();
+    if (live) {
+      constexpr int EVERY = P / D;
+#pragma unroll
+      for (int m = 0; m < P; ++m) {
+        acc[m % NT][m / NT] = stream_mma(wf[1][m % NT], af[1][m / NT], acc[m % NT][m / NT], T{});
+        if (m == 0) __builtin_amdgcn_sched_barrier(0);       // or the first product waits for the first of these reads
+        if (m < R) read(wat, aat, m, 0);
+        if (m % EVERY == 0 && m / EVERY < D) fill(bo, m / EVERY);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; ++r) read(wat, aat, r, 0);
+#pragma unroll
+      for (int i = 0; i < D; ++i) fill(bo, i);
+    }
+    ++fetched;
+    bo = BO - bo;
+    stored = false;
+    if (--left > 0) continue;
+
+    left = blocks;
+    if (live) {
+  
+      job.template store<MT, NT>(at, at.lo + 16 * MT * wm, wn, stream_lane(), acc);
+      stored = job.template whole<BM, BN>(at);
+      clear();
+    }
+    if (++tile == tiles) break;
+    fragments(bo, 0, wat, aat);
+#pragma unroll
+    for (int r = 0; r < R; ++r) read(wat, aat, r, 0);       // again: their registers were the epilogue's
+    at = ahead;       // with at least two blocks to a tile the stream is there already
+    live = at.lo + 16 * MT * wm < at.hi;
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");     // no DMA outlives the workgroup's LDS
+#endif
+}
+
+template <int MT, int NT, typename Job>
+hipError_t launch_stream_tiles(const Job& job, int64_t max_tiles, hipStream_t s) {
+  constexpr size_t lds = 2 * (32 * MT + 64 * NT) * 128 + STREAM_LIST * sizeof(StreamTile);
+  static std::atomic<uint64_t> devices{0};
+  const hipError_t e = allow_lds(reinterpret_cast<const void*>(&stream_tiles_kernel<MT, NT, Job>), lds, devices);
+  if (e != hipSuccess) return e;
+  const unsigned grid = (unsigned)(max_tiles < 256 ? (max_tiles + 7) / 8 * 8 : 256);
+  stream_tiles_kernel<MT, NT, Job><<<dim3(grid), dim3(512), lds, s>>>(job);
+  return hipGetLastError();
+}

@@ -68,6 +68,33 @@ def test_groups(sizes, N, K, dtype, tile, monkeypatch):
     close(hidden, want_h, 2 * K, dtype, torch.float32)
 
 
+@pytest.mark.parametrize("M,N,K,act", [(256 * 70 + 12, 1000, 128, None), (256 * 72, 1024, 192, 0), (256 * 33, 2048, 128, 1),
+                                       (256 * 140 + 130, 512, 128, 4), (256 * 128 + 1, 515, 256, 2)])
+def test_streams_of_tiles(M, N, K, act, monkeypatch):
+    """More 256 x 256 tiles than workgroups: whole rounds, a last round dealt in halves of tiles, remainders of rows."""
+    from byox_vllm_amd import kernels
+    monkeypatch.setenv("NV_LINEAR_TILE", "2")
+    kernels.block_many_rows(True)
+    try:
+        torch.manual_seed(M + N)
+        x, w = torch.randn(M, K, device=DEV).bfloat16(), (torch.randn(N, K, device=DEV) * 0.1).bfloat16()
+        coefficients = torch.tensor([0.8, 0.4], device=DEV)
+        for out_dtype in (torch.bfloat16, torch.float32):
+            args = {} if act is None else dict(epilogue=kernels.EPI_ACT, act=act, gate=coefficients if act == 2 else None)
+            got = kernels.linear(x, w, out_dtype=out_dtype, **args)
+            for lo in range(0, M, 8192):
+                want = x[lo:lo + 8192].double() @ w.double().t()
+                if act == 2:
+                    want = torch.where(want > 0, 0.8 * want * want + 0.5 * want,
+                                       0.4 * (torch.special.expm1(want) - want) + 0.5 * want)
+                elif act is not None:
+                    want = {0: torch.nn.functional.silu, 1: lambda v: torch.nn.functional.gelu(v, approximate="tanh"),
+                            4: torch.nn.functional.gelu}[act](want)
+                close(got[lo:lo + 8192], want, 4 * K, torch.bfloat16, out_dtype)
+    finally:
+        kernels.block_many_rows(False)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_batches_and_gates(dtype):
     """One product per head side by side, with the row gate, the soft cap and the element-wise epilogues."""
