@@ -38,6 +38,8 @@ _PROTOS = {
     "nv_paged_attn_decode_static": (_i, [_p, _i64, _p, _p, _p, _i, _p, _p, _i64, _i, _i, _i, _i, _i, _f, _i, _i, _p]),
     "nv_attn_prefill": (_i, [_p, _i64, _p, _p, _i64, _p, _p, _p, _i, _p, _i64, _i, _i, _i, _i, _i, _i, _f, _i, _p]),
     "nv_silu_mul": (_i, [_p, _p, _i64, _i, _i, _p]),
+    "nv_gemm_stream": (_i, [_p, _i64, _p, _p, _p, _i64, _i, _i, _i, _i, _i, _i, _p]),
+    "nv_gemm_stream_rope_kv_store": (_i, [_p, _i64, _p, _p, _p, _i64, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _f, _i, _i, _i, _i, _p]),
     "nv_gemm_lt_available": (_i, []),
     "nv_gemm_lt": (_i, [_p, _i64, _p, _p, _p, _i64, _i, _i, _i, _i, _p, _sz, _p]),
     "nv_gemm_lt_f32out": (_i, [_p, _i64, _p, _p, _i64, _i, _i, _i, _i, _p, _sz, _p]),

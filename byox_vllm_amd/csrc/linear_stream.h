@@ -2,10 +2,14 @@
 // linear.hip.  Groups (experts) of unknown size: every workgroup counts the tiles from the offsets with one wavefront-wide prefix
 // sum; a group that ends in the upper half of a tile's rows costs the half.
 #pragma once
+#include <type_traits>
+
 #include "stream_tiles.h"
 
 // value(s) of one output -> what is stored (bias, activation, gate); `gate`: the row's, where there is one for all of it
-template <typename T, int EPI, int ACT = -1>
+// SHORT: the result is rounded to 16 bits next; SiLU then comes from the hardware's exp2 and reciprocal, each within about 1 ulp of
+// fp32 (expf and a division are 30 instructions per result)
+template <typename T, int EPI, int ACT = -1, bool SHORT = false>
 __device__ __forceinline__ float lin_finish(const LinArgs& p, const T* bias, float v, float u, float rsc, float gate, int64_t s, int n,
                                             int z) {
   v *= rsc;
@@ -13,7 +17,8 @@ __device__ __forceinline__ float lin_finish(const LinArgs& p, const T* bias, flo
   if constexpr (EPI == EPI_GLU) {
     u *= rsc;
     if (bias) u += ld_f32<T>(bias + p.N + n);
-    v = glu_act(v, u, p.act, p.epi_c);
+    if (SHORT && p.act == 0) v = v * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * v)) * u;
+    else v = glu_act(v, u, p.act, p.epi_c);
   } else if constexpr (EPI == EPI_SOFTCAP) {
     v = p.epi_c * tanhf(v / p.epi_c);
   } else if constexpr (EPI == EPI_ROW_GATE) {
@@ -29,10 +34,12 @@ __device__ __forceinline__ u32x4 pack8(const float* v) {
   return u32x4{pack2<bf16_t>(v[0], v[1]), pack2<bf16_t>(v[2], v[3]), pack2<bf16_t>(v[4], v[5]), pack2<bf16_t>(v[6], v[7])};
 }
 
-template <typename TO, int EPI, int BM>
+template <typename TO, int EPI>
 struct LinearJob {
   typedef bf16_t T;
+  static constexpr int BM = STREAM_BM, MT = 8, NT = 4;              // four wavefronts along the columns
   static constexpr bool GLU = EPI == EPI_GLU, PAIRED = sizeof(TO) == 2;
+  typedef std::conditional_t<PAIRED, StreamPaired, StreamNatural> Order;
   static constexpr int NOUT = GLU ? 128 : 256;                      // columns of results per tile
   static constexpr int NSTORE = BM / 32 * (PAIRED ? 2 : 4) / (GLU ? 2 : 1);
   LinArgs p;
@@ -91,32 +98,28 @@ struct LinearJob {
   __device__ __forceinline__ uint32_t w_stride() const { return (uint32_t)p.w_rs * 2; }
   __device__ __forceinline__ uint32_t w_row(const StreamTile& at, int r) const {
     // a wavefront's 64 rows: 64 columns, or 32 columns' gates and the same columns' ups
-    if constexpr (GLU) return min(at.n0 + 32 * (r >> 6) + stream_column<PAIRED>(r & 31), p.N - 1) + ((r & 32) ? p.N : 0);
-    else return min(at.n0 + (r & ~31) + stream_column<PAIRED>(r & 31), p.N - 1);
+    if constexpr (GLU) return min(at.n0 + 32 * (r >> 6) + (r & 31), p.N - 1) + ((r & 32) ? p.N : 0);
+    else return min(at.n0 + r, p.N - 1);
   }
-  __device__ __forceinline__ uint32_t w_lane(int r, int piece) const { return 16 * piece; }
   __device__ __forceinline__ uint32_t w_step() const { return 128; }
-  template <int BMX, int BNX>
   __device__ __forceinline__ bool whole(const StreamTile& at) const {
     return vec && at.lo + BM <= at.hi && at.n0 + NOUT <= p.N;
   }
-  template <int MT, int NT>
   __device__ __forceinline__ void store(const StreamTile& at, int64_t row0, int wn, int lane, const f32x4 (&acc)[NT][MT]) const {
     if constexpr (EPI == EPI_ACT) {      // one function per copy: with the choice inside, the loops would not unroll
       switch (p.act) {
-        case 0: return store_as<MT, NT, 0>(at, row0, wn, lane, acc);
-        case 1: return store_as<MT, NT, 1>(at, row0, wn, lane, acc);
-        case 2: return store_as<MT, NT, 2>(at, row0, wn, lane, acc);
-        case 4: return store_as<MT, NT, 4>(at, row0, wn, lane, acc);
-        default: return store_as<MT, NT, 3>(at, row0, wn, lane, acc);
+        case 0: return store_as<0>(at, row0, wn, lane, acc);
+        case 1: return store_as<1>(at, row0, wn, lane, acc);
+        case 2: return store_as<2>(at, row0, wn, lane, acc);
+        case 4: return store_as<4>(at, row0, wn, lane, acc);
+        default: return store_as<3>(at, row0, wn, lane, acc);
       }
     } else {
-      store_as<MT, NT, -1>(at, row0, wn, lane, acc);
+      store_as<-1>(at, row0, wn, lane, acc);
     }
   }
-  template <int MT, int NT, int ACT>
+  template <int ACT>
   __device__ __forceinline__ void store_as(const StreamTile& at, int64_t row0, int wn, int lane, const f32x4 (&acc)[NT][MT]) const {
-    static_assert(NT == 4 && 32 * MT == BM, "");
     const int fr = lane & 15, g = lane >> 4;
     TO* O = reinterpret_cast<TO*>(p.out) + at.z * p.out_bs;
     const T* bias = p.bias ? reinterpret_cast<const T*>(p.bias) + at.z * p.bias_bs : nullptr;
@@ -130,7 +133,7 @@ struct LinearJob {
       const float gate = EPI == EPI_ROW_GATE && !p.act ? sigmoid_f32(p.epi_ptr[s * p.epi_rs + at.z]) : 1.0f;
       auto result = [&](int q, int e, int n) {
         const int j = q * (LEN / 4) + e / 4;
-        return lin_finish<T, EPI, ACT>(p, bias, acc[j][i][e & 3], GLU ? acc[(j + UP) % NT][i][e & 3] : 0.0f, rsc, gate, s, n + e, at.z);
+        return lin_finish<T, EPI, ACT, PAIRED>(p, bias, acc[j][i][e & 3], GLU ? acc[(j + UP) % NT][i][e & 3] : 0.0f, rsc, gate, s, n + e, at.z);
       };
       TO* o = O + s * p.out_rs;
 #pragma unroll
@@ -162,13 +165,10 @@ inline bool stream_takes(const LinArgs& p, int64_t total_rows, int batch, int co
 
 template <typename TO, int EPI>
 hipError_t launch_stream_epi(const LinArgs& p, int64_t total_rows, int batch, hipStream_t s) {
-  constexpr int BM = 256;
-  typedef LinearJob<TO, EPI, BM> Job;
+  typedef LinearJob<TO, EPI> Job;
   constexpr int64_t unit = sizeof(TO) == 2 ? 8 : 4;
   const int nt = (p.N + Job::NOUT - 1) / Job::NOUT;
   const int vec = p.N % unit == 0 && p.out_rs % unit == 0 && p.out_bs % unit == 0 && (uintptr_t)p.out % 16 == 0;
   const Job job{p, p.K, p.group_off ? batch : 0, batch, nt, vec};
-  // tiles of half the rows among them
-  const int64_t most = 2 * (p.group_off ? total_rows / BM + batch : (p.M + BM - 1) / BM * batch) * nt;
-  return launch_stream_tiles<BM / 32, 4>(job, most, s);
+  return launch_stream_tiles<4>(job, (p.group_off ? total_rows / Job::BM + batch : (p.M + Job::BM - 1) / Job::BM * batch) * nt, s);
 }

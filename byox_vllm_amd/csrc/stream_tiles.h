@@ -1,4 +1,4 @@
-// Products of many rows, 16-bit operands: a workgroup per CU walks tiles of 32 MT x 64 NT outputs whose K blocks form one stream.
+// Products of many rows, 16-bit operands: a workgroup per CU walks tiles of 256 x 256 outputs whose K blocks form one stream.
 //
 // What bounds it: the matrix cores and, on this part, their power: at 8192 x 8192 x 8192 the loop that this one replaced (a block
 // fetched, waited for and multiplied behind one barrier, 32 x 32 products) kept them 56 % busy at 1.76 GHz, the vendor library's
@@ -16,21 +16,21 @@
 //     Their tiles are found once, by a thread each, and kept in LDS: found in the loop they cost it its registers.
 // Measured, before and after: sixteen experts, 32768 rows of them, gated up 2048 -> 2 x 3072 and down, the layer 1584 and 1418 us;
 // 16384 rows 2048 -> 6144 into fp32 429 and 372 us (1110 TFLOP/s).
-// LDS rows are 128 bytes, their 16-byte pieces dealt by XOR with half the row number (through the DMA's source addresses): the 16
-// rows that a read touches lie in 16 bank groups.  Tiles go to the XCDs in contiguous eighths, within them in bands of eight row
+// LDS rows are 128 bytes, their 16-byte pieces dealt by XOR (through the DMA's source addresses) so that the 16 rows a read touches lie
+// in 16 bank groups.  Tiles go to the XCDs in contiguous eighths, within them in bands of eight row
 // tiles, so the 32 workgroups of an XCD share 8 row and 4 column panels in its L2.  A group's short last row tile stays in its band
 // (at the end of everything, its column panels come from memory again: the experts' layer 1450 us against 1418).
 //
 // Job (what is multiplied and what becomes of it) provides:
-//   T, NSTORE (stores of one wavefront for a whole tile), K (elements, a multiple of 64, at least 128)
+//   T, Order (how W lies, below), NSTORE, K (elements, a multiple of 64, at least 128)
 //   int count(lane)                       how many tiles there are
 //   StreamTile find(tile, lane)           which rows and columns the thread's tile has (every thread of a wavefront calls it)
 //   const void* a_base(tile); uint32_t a_row(tile, r); uint32_t a_stride()      row r of the tile's A rows (those past the end
 //                                         repeat a real one) lies at base + row * stride bytes, its K in 16-byte pieces
-//   w_base, w_row, w_stride               the same of row r of the W tile in LDS
-//   uint32_t w_lane(r, piece), w_step()   bytes from the row to its piece 0..7 of the first K block; and to the next K block
-//   bool whole(tile)                      every store of a wavefront is executed for this tile
-//   void store<NT, MT>(tile, first row, first column's wavefront, lane, acc)
+//   w_base, w_row, w_stride, w_step()     the same of row r of the W tile in LDS, or of its 16-row tile r; bytes to the next K block
+//   bool whole(tile)                      NSTORE stores of a wavefront at least are executed for this tile
+//   void store(tile, first row, wn, lane, acc)   acc[j][i]: row 16 i + lane % 16 of the wavefront's, fragment row 4 (lane / 16) + r of product j
+// WN wavefronts lie along the columns, 8 / WN along the rows.
 #pragma once
 #include "anyt.h"
 #include "lds_limit.h"
@@ -40,6 +40,8 @@ struct alignas(16) StreamTile {
   int n0, z;        // first column; which product of a batch or which group
 };
 constexpr int STREAM_LIST = 512;      // tiles of one workgroup at most
+constexpr int STREAM_BM = 256, STREAM_BN = 256;
+constexpr int STREAM_BUFFER = (STREAM_BM + STREAM_BN) * 128 + 1024;      // a K block of both, and what lies between W's tiles
 
 __device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x4 c, bf16_t) {
   return mfma16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c);
@@ -48,11 +50,42 @@ __device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x
   return mfma16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c);
 }
 
-// column, within 32, of LDS row r: 16-bit results are stored eight to a lane, from two products of the same rows
-template <bool PAIRED> __device__ __forceinline__ int stream_column(int r) {
-  if constexpr (!PAIRED) return r;
-  return 8 * ((r & 15) >> 2) + 4 * (r >> 4) + (r & 3);
-}
+// Where W lies in LDS and which of its rows a fragment has.  W stays in the order it has in memory, so that neighbouring lanes of a
+// DMA instruction fetch whole lines of it; the fragments choose which results a lane gets (frag and off, in bytes).  In rows: row r is
+// 128 bytes, its pieces XORed with key(r); of the 16 rows that a fragment reads no two of the same parity share a key, and row
+// frag / 128 + off / 128 has key (fr >> 1) & 7.  In tiles (TILED; nv_gemm's layout): 16 rows by 32 of K are 1 KB, row c's K piece g at
+// 16 (16 g + c); tile t lies at place(t), 2 KB apart and a little more, so that the parts of tiles which one fragment reads meet in
+// different banks.
+struct StreamNatural {      // four consecutive columns to a lane and product: 16 bytes of fp32
+  static constexpr bool TILED = false;
+  static __device__ __forceinline__ int frag(int fr) { return 128 * fr; }
+  static __host__ __device__ constexpr int off(int j) { return 2048 * j; }
+  static __device__ __forceinline__ int key(int r) { return (r >> 1) & 7; }
+};
+struct StreamPaired {       // eight consecutive columns to a lane and pair of products: 16 bytes of 16-bit results
+  static constexpr bool TILED = false;
+  static __device__ __forceinline__ int frag(int fr) { return 128 * (8 * (fr >> 2) + (fr & 3)); }
+  static __host__ __device__ constexpr int off(int j) { return 128 * (32 * (j >> 1) + 4 * (j & 1)); }
+  static __device__ __forceinline__ int key(int r) { return ((r >> 1) & 1) | (((r >> 3) & 3) << 1); }
+};
+struct StreamQuads {        // rows (gate 2 i, gate 2 i + 1, up 2 i, up 2 i + 1): gates in products 0 and 1, ups in 2 and 3, as pairs
+  static constexpr bool TILED = false;
+  static __device__ __forceinline__ int frag(int fr) { return 128 * (16 * (fr >> 2) + 4 * ((fr >> 1) & 1) + (fr & 1)); }
+  static __host__ __device__ constexpr int off(int j) { return 128 * (8 * (j & 1) + 2 * (j >> 1)); }
+  static __device__ __forceinline__ int key(int r) { return ((r >> 2) & 1) | (((r >> 4) & 3) << 1); }
+};
+struct StreamPairedTiled {
+  static constexpr bool TILED = true;
+  static __host__ __device__ constexpr int place(int t) { return 2112 * t; }
+  static __device__ __forceinline__ int frag(int fr) { return place(fr >> 3) + 16 * (8 * ((fr >> 2) & 1) + (fr & 3)); }
+  static __host__ __device__ constexpr int off(int j) { return place(2 * (j >> 1)) + 64 * (j & 1); }
+};
+struct StreamQuadsTiled {
+  static constexpr bool TILED = true;
+  static __host__ __device__ constexpr int place(int t) { return 2048 * t + 32 * (t & 1) + 128 * ((t >> 1) & 1) + 256 * (t >> 2); }
+  static __device__ __forceinline__ int frag(int fr) { return place(fr >> 2) + 16 * (4 * ((fr >> 1) & 1) + (fr & 1)); }
+  static __host__ __device__ constexpr int off(int j) { return 128 * (j & 1) + 32 * (j >> 1); }
+};
 
 // place `in` of a group of `rows` row tiles by `cols` column tiles: bands of eight row tiles (the last of up to fifteen), rows first
 __device__ __forceinline__ void stream_order(int in, int rows, int cols, int& m_tile, int& n_tile) {
@@ -70,18 +103,20 @@ __device__ __forceinline__ int stream_lane() {
   return (int)__builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0));
 }
 
-template <int MT, int NT, typename Job>
+template <int WN, typename Job>
 __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef typename Job::T T;
-  constexpr int BM = 32 * MT, BN = 64 * NT, BO = (BM + BN) * 128;       // BO: bytes of one buffer
+  constexpr int WM = 8 / WN, MT = STREAM_BM / 16 / WM, NT = STREAM_BN / 16 / WN;
+  typedef typename Job::Order Order;
+  constexpr int BM = STREAM_BM, BN = STREAM_BN, BO = STREAM_BUFFER;     // BO: bytes of one buffer
   constexpr int AG = BM / 64, WG = BN / 64, D = AG + WG;                // DMA instructions (8 rows each) of a wavefront per block
   constexpr int P = MT * NT, R = MT + NT;                               // products and fragment reads of a step
   typedef __attribute__((address_space(1))) void global_void;
   typedef __attribute__((address_space(3))) void lds_void;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   const int lane = stream_lane(), wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wv >> 2, wn = wv & 3;                                  // a SIMD has one wavefront of each half of the rows
+  const int wm = wv / WN, wn = wv % WN;                                 // a SIMD has one wavefront of each half of the rows
 
   // -------- this workgroup's tiles: every per-th of its XCD's.  A last round that at most half of the workgroups would have is dealt
   // as tiles of half the rows.  One thread finds one tile; the list is in LDS.
@@ -121,16 +156,21 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
 #pragma unroll
     for (int i = 0; i < AG; ++i) asm volatile("" : "+v"(arow[i]));      // a gathered row's number is waited for here, not at each fetch
 #pragma unroll
-    for (int i = 0; i < WG; ++i) wrow[i] = job.w_row(at, r0 + 64 * i);
+    for (int i = 0; i < WG; ++i) wrow[i] = job.w_row(at, Order::TILED ? (wv >> 1) + 4 * i : r0 + 64 * i);
     apos = reinterpret_cast<uint64_t>(job.a_base(at));
     wpos = reinterpret_cast<uint64_t>(job.w_base(at));
   };
   // DMA instruction i fills LDS rows 8 (wv + 8 i) + l / 8, whose place among the XORs is the same for every i
   uint32_t alane, wlane;
   auto lanes = [&]() {
-    const int l = stream_lane(), r0 = 8 * wv + (l >> 3), piece = (l & 7) ^ ((r0 >> 1) & 7);
-    alane = 16 * piece;
-    wlane = job.w_lane(r0, piece);
+    const int l = stream_lane(), r0 = 8 * wv + (l >> 3);
+    alane = 16 * ((l & 7) ^ ((r0 >> 1) & 7));
+    if constexpr (Order::TILED) wlane = 1024 * (wv & 1) + 16 * l;
+    else wlane = 16 * ((l & 7) ^ Order::key(r0));
+  };
+  auto wplace = [&](int i) {
+    if constexpr (Order::TILED) return Order::place((wv >> 1) + 4 * i) + 1024 * (wv & 1);
+    else return 1024 * (wv + 8 * i);
   };
   auto fill = [&](int bo, int i) {
     if (i < AG) {
@@ -140,7 +180,7 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
     } else {
       const int q = i < AG ? 0 : i - AG;
       __builtin_amdgcn_global_load_lds((global_void*)(wpos + (uint64_t)wrow[q] * w_stride + wlane),
-                                       (lds_void*)(lds_raw + bo + BM * 128 + (wv + 8 * q) * 1024), 16, 0, 0);
+                                       (lds_void*)(lds_raw + bo + BM * 128 + wplace(q)), 16, 0, 0);
     }
     if (i == AG - 1) apos += 128;
     if (i == D - 1) wpos += w_step;
@@ -148,13 +188,14 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
   // where this lane's first fragments of W and A lie in the buffer at `bo`; formed for every step anew (registers).  Every fragment
   // starts at a multiple of 16 rows.
   auto fragments = [&](int bo, int step, int& wat, int& aat) {
-    const int l = stream_lane(), fr = l & 15, in = bo + fr * 128 + 16 * (((4 * step + (l >> 4)) ^ (fr >> 1)) & 7);
-    wat = in + (BM + 16 * NT * wn) * 128;
-    aat = in + 16 * MT * wm * 128;
+    const int l = stream_lane(), fr = l & 15, in = bo + 16 * (((4 * step + (l >> 4)) ^ (fr >> 1)) & 7);
+    if constexpr (Order::TILED) wat = bo + BM * 128 + Order::place(NT * wn) + Order::frag(fr) + 1024 * step + 256 * (l >> 4);
+    else wat = in + (BM + 16 * NT * wn) * 128 + Order::frag(fr);
+    aat = in + (16 * MT * wm + fr) * 128;
   };
   u32x4 wf[2][NT], af[2][MT];
   auto read = [&](int wat, int aat, int r, int set) {
-    if (r < NT) wf[set][r < NT ? r : 0] = *reinterpret_cast<const u32x4*>(lds_raw + wat + 2048 * r);
+    if (r < NT) wf[set][r < NT ? r : 0] = *reinterpret_cast<const u32x4*>(lds_raw + wat + Order::off(r < NT ? r : 0));
     else af[set][r < NT ? 0 : r - NT] = *reinterpret_cast<const u32x4*>(lds_raw + aat + 2048 * (r - NT));
   };
 
@@ -238,8 +279,8 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
     left = blocks;
     if (live) {
   
-      job.template store<MT, NT>(at, at.lo + 16 * MT * wm, wn, stream_lane(), acc);
-      stored = job.template whole<BM, BN>(at);
+      job.store(at, at.lo + 16 * MT * wm, wn, stream_lane(), acc);
+      stored = job.whole(at);
       clear();
     }
     if (++tile == tiles) break;
@@ -253,13 +294,14 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
 #endif
 }
 
-template <int MT, int NT, typename Job>
+template <int WN, typename Job>
 hipError_t launch_stream_tiles(const Job& job, int64_t max_tiles, hipStream_t s) {
-  constexpr size_t lds = 2 * (32 * MT + 64 * NT) * 128 + STREAM_LIST * sizeof(StreamTile);
+  constexpr size_t lds = 2 * STREAM_BUFFER + STREAM_LIST * sizeof(StreamTile);
   static std::atomic<uint64_t> devices{0};
-  const hipError_t e = allow_lds(reinterpret_cast<const void*>(&stream_tiles_kernel<MT, NT, Job>), lds, devices);
+  const hipError_t e = allow_lds(reinterpret_cast<const void*>(&stream_tiles_kernel<WN, Job>), lds, devices);
   if (e != hipSuccess) return e;
-  const unsigned grid = (unsigned)(max_tiles < 256 ? (max_tiles + 7) / 8 * 8 : 256);
-  stream_tiles_kernel<MT, NT, Job><<<dim3(grid), dim3(512), lds, s>>>(job);
+  // with few tiles there is a workgroup for each half of one
+  const unsigned grid = (unsigned)(max_tiles < 128 ? (2 * max_tiles + 7) / 8 * 8 : 256);
+  stream_tiles_kernel<WN, Job><<<dim3(grid), dim3(512), lds, s>>>(job);
   return hipGetLastError();
 }

@@ -253,7 +253,7 @@ def pick_split_k(M, N, K, wfmt=_C.W_INT4):
 
 
 # Rows from which a product goes through the vendor library (nv_gemm_lt) instead of nv_gemm's decode-shaped tiles:
-# prefill steps.  Measured on the layer shapes of Qwen3-0.6B, Qwen2-0.5B and Qwen2-7B, weight expansion included
+# prefill steps; from the same number on, what gemm_many_rows keeps on this library's own tiles.  Measured on the layer shapes of Qwen3-0.6B, Qwen2-0.5B and Qwen2-7B, weight expansion included
 # (scripts/r03_dense_prefill_gemm.py): at 1024 rows nv_gemm wins everywhere, at 2048 the two trade places by shape,
 # from 4096 on the library wins or ties (1.3-1.7 times faster from 8192).  NV_GEMM_LT_ROWS=0 switches the path off.
 MANY_ROWS = int(os.environ.get("NV_GEMM_LT_ROWS", "4096"))
@@ -271,13 +271,71 @@ def expand_weight(w, gate_up_rows=False, out=None):
     return out
 
 
-def gemm_many_rows(x, w, bias=None, out=None, silu_mul=False):
-    """gemm() for prefill-sized x: the weight written out row-major into scratch, one vendor-library product, and for
-    gate/up weights the SiluAndMul pass over its result (same roundings as the fused epilogue: the product rounded to
-    the model dtype, silu rounded, the product with up rounded)."""
+def _rows_weight(w):
+    """A LinearWeight as nv_gemm_stream reads it -> (data, format): 16-bit weights as they are, quantised ones expanded in order."""
+    if w.fmt in (_C.W_DENSE, _C.W_DENSE_TILED):
+        return w.data, w.fmt
+    N, K = w.out_features, w.in_features
+    wr = workspace(N * K * 2, w.data.device, "gemm_lt_weight")[:N * K * 2].view(w.dtype).view(N, K)
+    return expand_weight(w, out=wr), _C.W_DENSE
+
+
+def streams(x, w, *others):
+    """Whether nv_gemm_stream takes this product: 16-byte aligned rows, K of two blocks, a list of tiles that fits."""
+    return x.stride(0) % 8 == 0 and w.in_features % 64 == 0 and w.in_features >= 128 and \
+        (-(-x.size(0) // 256)) * (-(-w.out_features // 256)) <= 256 * 510 and \
+        all(t is None or t.data_ptr() % 16 == 0 for t in (x, w.data) + others)
+
+
+def gemm_stream_rope_kv_store(x, w, bias, positions, cos_sin, num_heads, num_kv_heads, head_dim, slot_mapping=None,
+                              k_cache=None, v_cache=None, q_norm_w=None, k_norm_w=None, eps=1e-6):
+    """gemm_rope_kv_store() for prefill-sized x (nv_gemm_stream_rope_kv_store)."""
+    require_gpu(x, "gemm_stream_rope_kv_store")
+    _require_device_weight(w, "gemm_stream_rope_kv_store")
+    T, K = x.shape
+    N = (num_heads + 2 * num_kv_heads) * head_dim
+    assert K == w.in_features and N == w.out_features and x.stride(1) == 1 and x.dtype == w.dtype
+    assert positions.dtype == torch.int64 and positions.numel() == T and positions.is_contiguous()
+    assert cos_sin.dtype == torch.float32 and cos_sin.is_contiguous() and cos_sin.size(-1) == head_dim
+    assert bias is None or (bias.numel() == N and bias.dtype == x.dtype)
+    if k_cache is not None:
+        assert slot_mapping is not None and slot_mapping.dtype == torch.int32 and slot_mapping.numel() == T
+        assert k_cache.is_contiguous() and v_cache.is_contiguous() and k_cache.dtype == x.dtype
+        assert k_cache.size(-1) == head_dim and k_cache.size(-2) == num_kv_heads
+    data, fmt = _rows_weight(w)
+    out = torch.empty(T, N, dtype=x.dtype, device=x.device)
+    check(lib().nv_gemm_stream_rope_kv_store(ptr(x), x.stride(0), ptr(data), ptr(bias), ptr(out), out.stride(0), T, K, fmt,
+                                             ptr(positions), ptr(cos_sin), ptr(slot_mapping), ptr(k_cache), ptr(v_cache),
+                                             ptr(q_norm_w), ptr(k_norm_w), eps, num_heads, num_kv_heads, head_dim,
+                                             dtype_code(x.dtype), stream()), "nv_gemm_stream_rope_kv_store")
+    return out
+
+
+def gemm_stream(x, w, bias=None, out=None, silu_mul=False):
+    """gemm() for prefill-sized x on this library's own tiles (nv_gemm_stream)."""
+    M, K = x.shape
+    N = w.out_features
+    data, fmt = _rows_weight(w)
+    cols = N // 2 if silu_mul else N
+    out = torch.empty(M, cols, dtype=x.dtype, device=x.device) if out is None else out
+    assert out.stride(1) == 1 and out.shape == (M, cols)
+    check(lib().nv_gemm_stream(ptr(x), x.stride(0), ptr(data), ptr(bias), ptr(out), out.stride(0), M, N, K, fmt, int(silu_mul),
+                               dtype_code(x.dtype), stream()), "nv_gemm_stream")
+    return out
+
+
+def gemm_many_rows(x, w, bias=None, out=None, silu_mul=False, rope=None):
+    """gemm() for prefill-sized x.  Gate/up weights, and products of a K below 1024, on this library's tiles (nv_gemm_stream); the
+    others as the weight written out row-major into scratch and one vendor-library product.  14.6 k rows, vendor route and
+    nv_gemm_stream: 1024 -> 2 x 3072 with SiluAndMul 208 and 169 us, 896 -> 2 x 4864 332 and 235; 896 -> 896 42 and 30;
+    2048 -> 1024 51 and 55, 3072 -> 1024 70 and 79.  ``rope``: arguments of gemm_stream_rope_kv_store, whose result this is then."""
     M, K = x.shape
     N = w.out_features
     dev = x.device
+    if rope is not None:
+        return gemm_stream_rope_kv_store(x, w, bias, **rope)
+    if streams(x, w, bias, out) and (out is None or out.stride(0) % 8 == 0) and (bias is None if silu_mul else 512 <= K < 1024):
+        return gemm_stream(x, w, bias, out, silu_mul)
     if w.fmt == _C.W_DENSE and not silu_mul:
         wr = w.data
     else:
@@ -331,6 +389,11 @@ def gemm(x, w, bias=None, out=None, split_k=None, silu_mul=False, partial_out=Fa
     if split_k is None:
         if use_many_rows_path(M, K, N) and (out is None or out.is_contiguous() or not silu_mul):
             return gemm_many_rows(x, w, bias, out, silu_mul)
+        # gate/up from half as many rows on where the weight is read as it lies (2048 rows, nv_gemm and the streamed tiles:
+        # 1024 -> 2 x 3072 37 and 33 us, 896 -> 2 x 4864 61 and 46; 1024 rows: 23 and 30)
+        if silu_mul and bias is None and M >= MANY_ROWS // 2 and w.fmt in (_C.W_DENSE, _C.W_DENSE_TILED) and \
+                use_many_rows_path(max(M, MANY_ROWS), K, N) and streams(x, w, out) and (out is None or out.stride(0) % 8 == 0):
+            return gemm_stream(x, w, None, out, True)
         split_k = 1 if silu_mul else pick_split_k(M, N, K, w.fmt)
     split_k = max(1, min(split_k, K // 128))
     if split_k == 1:

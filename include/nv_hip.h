@@ -163,6 +163,19 @@ int nv_gemm_lt(const void* x, int64_t x_row_stride, const void* w_rowmajor, cons
                int64_t out_row_stride, int M, int N, int K, int dtype, void* workspace, size_t workspace_bytes,
                nv_stream_t stream);
 
+/* The same many-row products on this library's own tiles, with what follows them; W in a 16-bit format of nv_gemm (NV_W_DENSE,
+ * NV_W_DENSE_TILED), read as it lies.  nv_gemm_stream: out = x * W^T (+ bias), or with silu_mul the rows of nv_gemm's silu(gate)*up
+ * epilogue (gate 2i, gate 2i+1, up 2i, up 2i+1; no bias; out [M, N / 2], nanovllm/layers/activation.py:10-13).
+ * nv_gemm_stream_rope_kv_store: arguments and results of nv_gemm_rope_kv_store.  K >= 128, pointers 16-byte aligned, row strides
+ * multiples of 8.  No workspace; may be captured. */
+int nv_gemm_stream(const void* x, int64_t x_row_stride, const void* w, const void* bias, void* out, int64_t out_row_stride,
+                   int M, int N, int K, int wfmt, int silu_mul, int dtype, nv_stream_t stream);
+int nv_gemm_stream_rope_kv_store(const void* x, int64_t x_row_stride, const void* w, const void* bias, void* qkv,
+                                 int64_t qkv_row_stride, int M, int K, int wfmt, const int64_t* positions,
+                                 const float* cos_sin, const int32_t* slot_mapping, void* k_cache, void* v_cache,
+                                 const void* q_norm_w, const void* k_norm_w, float eps, int H, int Hkv, int D, int dtype,
+                                 nv_stream_t stream);
+
 /* Weight of any nv_gemm format (NV_W_*) -> row-major [N, K] in the model dtype: tiled layouts un-tiled, int4 / int8
  * dequantised as (u - 8) * s resp. q * s in fp32, rounded once (the oracle's dequantisation, so nv_gemm_lt on the result
  * is "dequantise, then F.linear").  gate_up_rows != 0: the rows are stored in the order of nv_gemm's silu(gate)*up

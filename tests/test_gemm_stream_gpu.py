@@ -1,0 +1,94 @@
+"""nv_gemm_stream and its rotating form (csrc/gemm_stream.hip) at the edges of their 256 x 256 tiles: ragged row tiles, last
+rounds dealt in halves, columns that end inside a tile, both 16-bit weight layouts, both head sizes."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+DT = {"bf16": torch.bfloat16, "fp16": torch.float16}
+
+
+def weight(w, tiled):
+    from byox_vllm_amd.layers.quant import LinearWeight
+    return LinearWeight.dense_tiled(w) if tiled else LinearWeight.dense(w)
+
+
+def close(got, want, dt, K, ulps=1.0):
+    # `ulps` roundings to 16 bits, and K roundings of fp32 partial sums of a few units where the products cancel
+    eps = torch.finfo(dt).eps
+    got, want = got.double(), want.double()
+    bad = (got - want).abs() > ulps * eps * want.abs() + 8.0 * K ** 0.5 * 2.0 ** -24
+    assert torch.isfinite(got).all() and not bad.any(), f"{int(bad.sum())} of {bad.numel()} off, max {(got - want).abs().max()}"
+
+
+SHAPES = [(1, 16, 128), (255, 272, 128), (257, 640, 256), (4100, 528, 384), (256 * 66 + 3, 1024, 128), (2300, 4096, 256)]
+
+
+@pytest.mark.parametrize("name", ["bf16", "fp16"])
+@pytest.mark.parametrize("tiled", [True, False])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_plain(M, N, K, tiled, name):
+    from byox_vllm_amd import kernels
+    torch.manual_seed(M + N)
+    dt = DT[name]
+    x, w, b = torch.randn(M, K, device=DEV).to(dt), (torch.randn(N, K, device=DEV) * 0.05).to(dt), torch.randn(N, device=DEV).to(dt)
+    want = x.double() @ w.double().t()
+    out = torch.zeros(M, N + 8, dtype=dt, device=DEV)
+    got = kernels.gemm_stream(x, weight(w, tiled), b, out=out[:, :N])
+    close(got, want + b.double(), dt, K)
+    assert not out[:, N:].any()
+    close(kernels.gemm_stream(x, weight(w, tiled)), want, dt, K)
+
+
+@pytest.mark.parametrize("name", ["bf16", "fp16"])
+@pytest.mark.parametrize("tiled", [True, False])
+@pytest.mark.parametrize("M,inter,K", [(1, 16, 128), (255, 272, 128), (300, 1536, 256), (2100, 1040, 384), (256 * 66 + 3, 512, 128)])
+def test_silu_mul(M, inter, K, tiled, name):
+    """Gate and up rows as the kernels store them, against the product's, SiLU's and the last rounding taken one by one."""
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.layers.quant import interleave_gate_up
+    torch.manual_seed(M + inter)
+    dt = DT[name]
+    x, w = torch.randn(M, K, device=DEV).to(dt), (torch.randn(2 * inter, K, device=DEV) * 0.05).to(dt)
+    got = kernels.gemm_stream(x, weight(interleave_gate_up(w), tiled), silu_mul=True)
+    gate, up = (x.double() @ w.double().t()).to(dt).double().chunk(2, -1)
+    want = torch.nn.functional.silu(gate).to(dt).double() * up
+    close(got, want, dt, K, ulps=3.0)      # a gate on the other side of a rounding moves two more
+
+
+@pytest.mark.parametrize("name", ["bf16", "fp16"])
+@pytest.mark.parametrize("tiled", [True, False])
+@pytest.mark.parametrize("T,H,Hkv,D,norms", [(1, 1, 1, 64, False), (257, 14, 2, 64, False), (300, 3, 1, 64, True), (513, 16, 8, 128, True),
+                                             (4100, 5, 1, 128, False), (256 * 34 + 5, 4, 2, 128, True)])
+def test_rope_kv_store(T, H, Hkv, D, norms, tiled, name):
+    """The launch against the product and nv_rope_kv_store in two: the same roundings, so equal up to the order of the norm's sum."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(T + H)
+    dt, K, N = DT[name], 256, (H + 2 * Hkv) * D
+    x, w = torch.randn(T, K, device=DEV).to(dt), (torch.randn(N, K, device=DEV) * 0.1).to(dt)
+    bias = None if norms else torch.randn(N, device=DEV).to(dt)
+    qn, kn = ((torch.rand(D, device=DEV) + 0.5).to(dt) if norms else None for _ in range(2))
+    pos = torch.randint(0, 500, (T,), device=DEV)
+    cos_sin = torch.randn(500, D, device=DEV)
+    pages = -(-T // 16) + 1
+    slots = torch.randperm(pages * 16, device=DEV)[:T].int()
+    slots[T // 2] = -1 if T > 1 else slots[0]                 # a token that is not kept
+    caches = [torch.zeros(pages, 16, Hkv, D, dtype=dt, device=DEV) for _ in range(4)]
+    args = dict(slot_mapping=slots, q_norm_w=qn, k_norm_w=kn, eps=1e-6)
+    got = kernels.gemm_stream_rope_kv_store(x, weight(w, tiled), bias, pos, cos_sin, H, Hkv, D, k_cache=caches[0], v_cache=caches[1], **args)
+    qkv = kernels.gemm_stream(x, weight(w, tiled), bias)
+    close(qkv, x.double() @ w.double().t() + (0 if bias is None else bias.double()), dt, K)
+    want = kernels.rope_kv_store(qkv, pos, cos_sin, H, Hkv, D, k_cache=caches[2], v_cache=caches[3], **args)
+    for a, b in ((got, want), (caches[0], caches[2]), (caches[1], caches[3])):
+        if norms:
+            # one rounding of the normed number, another of its product with the weight, turned by |(cos, sin)| up to 6, and its own
+            scale = torch.finfo(dt).eps * 8.0 * 6.0
+            assert ((a.double() - b.double()).abs() <= scale * (1 + b.double().abs())).all()
+            assert (a != b).float().mean() < 1e-3
+        else:
+            # the same fp32 numbers (a compiler may contract a product of up to 32 into the sum: 2^-19) rounded once
+            assert ((a.double() - b.double()).abs() <= torch.finfo(dt).eps * b.double().abs() + 2.0 ** -19).all()
+            assert (a != b).float().mean() < 1e-3
+    bare = kernels.gemm_stream_rope_kv_store(x, weight(w, tiled), bias, pos, cos_sin, H, Hkv, D, q_norm_w=qn, k_norm_w=kn)
+    assert torch.equal(bare, got)
