@@ -526,28 +526,15 @@ def linear(x, w, bias=None, out=None, out_dtype=None, *, rows=None, a_rows=None,
     if n is None:
         n = w.size(-2) // (2 if epilogue == EPI_GLU else 1)
     M = x.size(0) if rows is None else rows
-    # prefill-sized plain products of a 16-bit model go where the engine sends its other many-row products: the vendor
-    # library, here with the result left in fp32
-    if (epilogue in (EPI_NONE, EPI_GLU, EPI_ACT) and batch == 1 and group_offsets is None and a_rows is None
-            and (bias is None or (epilogue != EPI_NONE and (out_dtype or x.dtype) == x.dtype)) and out is None
-            and row_scale is None
+    # prefill-sized plain products of a 16-bit model go where the engine sends its other many-row products: the vendor library, here
+    # with the result left in fp32.  Not those with an epilogue, which nv_linear forms on the way (16384 rows 2048 -> 2 x 6144, SiLU:
+    # 714 us, the library and a pass over its result 928; 4096 rows 1024 -> 4096 48 and 65), nor those of a short K whose columns do
+    # not split into the library's tiles (12300 rows 1024 -> 3088: 95 and 110; 512 -> 1552: 42 and 49; 2048 -> 4112: 325 and 290).
+    if (epilogue == EPI_NONE and batch == 1 and group_offsets is None and a_rows is None and bias is None and out is None
+            and row_scale is None and not (K <= 1024 and n > 1024 and n % 256)
             and rows is None and x.dtype == torch.bfloat16 and (out_dtype or x.dtype) in (torch.float32, torch.bfloat16)
             and w.dim() == 2 and w.is_contiguous() and x.stride(0) % 8 == 0 and use_many_rows_path(M, K, n) and K % 8 == 0
             and n % 8 == 0 and x.data_ptr() % 16 == 0):
-        if epilogue == EPI_GLU:      # [gate | up] rows from the library, activation and product in one pass over them
-            y = _linear_many_rows(x, w, M, 2 * n, K, torch.float32)
-            out = torch.empty(M, n, dtype=out_dtype or x.dtype, device=x.device)
-            assert bias is None or (bias.dtype == x.dtype and bias.numel() == 2 * n and bias.is_contiguous())
-            check(lib().nv_bias_act_mul_f32(ptr(y), ptr(bias), ptr(out), M, n, act, cap, _code32(out.dtype), stream()),
-                  "nv_bias_act_mul_f32")
-            return out
-        if epilogue == EPI_ACT:      # the element-wise function in one pass over the library's fp32 result
-            y = _linear_many_rows(x, w, M, n, K, torch.float32)
-            out = torch.empty(M, n, dtype=out_dtype or x.dtype, device=x.device)
-            assert bias is None or (bias.dtype == x.dtype and bias.numel() == n and bias.is_contiguous())
-            check(lib().nv_bias_act_f32(ptr(y), ptr(bias), n, ptr(out), M * n, act, ptr(gate), cap, _code32(out.dtype),
-                                        stream()), "nv_bias_act_f32")
-            return out
         return _linear_many_rows(x, w, M, n, K, out_dtype or x.dtype)
     grid_rows = M if group_offsets is None else (max_group_rows if max_group_rows is not None else M)
     out_dtype = out_dtype or x.dtype
