@@ -40,6 +40,9 @@ _PROTOS = {
     "nv_silu_mul": (_i, [_p, _p, _i64, _i, _i, _p]),
     "nv_gemm_stream": (_i, [_p, _i64, _p, _p, _p, _i64, _i, _i, _i, _i, _i, _i, _p]),
     "nv_gemm_stream_rope_kv_store": (_i, [_p, _i64, _p, _p, _p, _i64, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _f, _i, _i, _i, _i, _p]),
+    "nv_norm_gemm_silu": (_i, [_p, _p, _i, _p, _p, _p, _f, _p, _p, _i64, _i, _i, _i, _i, _p]),
+    "nv_norm_gemm_rope_kv_store": (_i, [_p, _p, _i, _p, _p, _p, _f, _p, _p, _p, _i64, _i, _i, _p, _p, _p, _p, _p, _p, _p, _f, _i, _i,
+                                        _i, _i, _p]),
     "nv_gemm_lt_available": (_i, []),
     "nv_gemm_lt": (_i, [_p, _i64, _p, _p, _p, _i64, _i, _i, _i, _i, _p, _sz, _p]),
     "nv_gemm_lt_f32out": (_i, [_p, _i64, _p, _p, _i64, _i, _i, _i, _i, _p, _sz, _p]),

@@ -160,6 +160,61 @@ def gemm_rope_kv_store(x, w, bias, positions, cos_sin, num_heads, num_kv_heads, 
     return out
 
 
+# Rows up to which a norm is formed in the product that reads it.  A decode step of 24 layers, norms apart and in the product, us:
+# Qwen2-0.5B 1 row 951 and 858, 4 rows 976 and 929, 6 rows 985 and 1021; Qwen3-0.6B 1037 and 923, 1054 and 992, 1071 and 1086.
+NORM_GEMM_ROWS = 4
+
+
+def takes_norm(x, residual, w, norm_w) -> bool:
+    """Whether the norm of these rows can be formed in the product of ``w`` (nv_norm_gemm_*): few rows, 16-bit tiled weights."""
+    rows, cols = (x.rows, x.cols) if isinstance(x, Partials) else x.shape if torch.is_tensor(x) else (0, 0)
+    return (0 < rows <= NORM_GEMM_ROWS and cols == w.in_features and w.fmt == _C.W_DENSE_TILED and cols <= 2048
+            and rows * (2 * cols + 16) <= 48 << 10 and norm_w.dtype == w.dtype and norm_w.data_ptr() % 16 == 0
+            and (x.bias is None and residual is not None if isinstance(x, Partials)
+                 else x.dtype == w.dtype and x.is_contiguous() and x.data_ptr() % 16 == 0)
+            and (residual is None or (residual.dtype == w.dtype and residual.is_contiguous() and residual.data_ptr() % 16 == 0)))
+
+
+def _norm_rows(x, residual, w):
+    """The first arguments of nv_norm_gemm_* for rows that are a tensor or Partials -> (arguments, the new residual, M, K)."""
+    _require_device_weight(w, "nv_norm_gemm")
+    M, K = (x.rows, x.cols) if isinstance(x, Partials) else x.shape
+    assert residual is None or residual.shape == (M, K)
+    new = None if residual is None else torch.empty_like(residual)
+    head = (None, ptr(x.slabs), x.n) if isinstance(x, Partials) else (ptr(x), None, 0)
+    return head + (ptr(residual), ptr(new)), (x if residual is None else new), M, K
+
+
+def norm_gemm_silu(x, residual, norm_w, eps, w):
+    """RMSNorm(x + residual) -> gate/up product -> SiLU(gate) * up in one launch -> ([M, N / 2], the new residual)."""
+    args, new, M, K = _norm_rows(x, residual, w)
+    N = w.out_features
+    out = torch.empty(M, N // 2, dtype=w.dtype, device=w.data.device)
+    check(lib().nv_norm_gemm_silu(*args, ptr(norm_w), eps, ptr(w.data), ptr(out), out.stride(0), M, N, K, dtype_code(w.dtype),
+                                  stream()), "nv_norm_gemm_silu")
+    return out, new
+
+
+def norm_gemm_rope_kv_store(x, residual, norm_w, norm_eps, w, bias, positions, cos_sin, num_heads, num_kv_heads, head_dim,
+                            slot_mapping=None, k_cache=None, v_cache=None, q_norm_w=None, k_norm_w=None, eps=1e-6):
+    """RMSNorm(x + residual) and gemm_rope_kv_store() in one launch -> (qkv, the new residual)."""
+    args, new, M, K = _norm_rows(x, residual, w)
+    N = (num_heads + 2 * num_kv_heads) * head_dim
+    assert N == w.out_features and positions.dtype == torch.int64 and positions.numel() == M and positions.is_contiguous()
+    assert cos_sin.dtype == torch.float32 and cos_sin.is_contiguous() and cos_sin.size(-1) == head_dim
+    assert bias is None or (bias.numel() == N and bias.dtype == w.dtype)
+    if k_cache is not None:
+        assert slot_mapping is not None and slot_mapping.dtype == torch.int32 and slot_mapping.numel() == M
+        assert k_cache.is_contiguous() and v_cache.is_contiguous() and k_cache.dtype == w.dtype
+        assert k_cache.size(-1) == head_dim and k_cache.size(-2) == num_kv_heads
+    out = torch.empty(M, N, dtype=w.dtype, device=w.data.device)
+    check(lib().nv_norm_gemm_rope_kv_store(*args, ptr(norm_w), norm_eps, ptr(w.data), ptr(bias), ptr(out), out.stride(0), M, K,
+                                           ptr(positions), ptr(cos_sin), ptr(slot_mapping), ptr(k_cache), ptr(v_cache),
+                                           ptr(q_norm_w), ptr(k_norm_w), eps, num_heads, num_kv_heads, head_dim,
+                                           dtype_code(w.dtype), stream()), "nv_norm_gemm_rope_kv_store")
+    return out, new
+
+
 def kv_store(key, value, k_cache, v_cache, slot_mapping):
     """store_kvcache: key/value [T, Hkv, D] (may be strided views of a qkv buffer)."""
     require_gpu(key, "kv_store")

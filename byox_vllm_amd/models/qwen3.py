@@ -58,7 +58,8 @@ class Qwen3Attention(nn.Module):
             self.q_norm = RMSNorm(self.head_dim, eps=rms_norm_eps)
             self.k_norm = RMSNorm(self.head_dim, eps=rms_norm_eps)
 
-    def forward(self, positions: torch.Tensor, hidden_states: torch.Tensor) -> torch.Tensor:
+    def forward(self, positions: torch.Tensor, hidden_states: torch.Tensor, norm=None, residual=None):
+        """``norm``: the layer's input norm, still to be taken of ``hidden_states`` and ``residual`` -> (result, new residual)."""
         context = get_context()
         attn = self.attn
         has_cache = attn.k_cache.numel() > 0
@@ -69,6 +70,19 @@ class Qwen3Attention(nn.Module):
         proj = self.qkv_proj
         if proj.packed is None:
             proj.finalize(None)
+        bias = None if proj.bias is None else proj.bias.data
+        if norm is not None:
+            if self.fuse_qkv_rope and self.head_dim in (64, 128) and \
+                    kernels.takes_norm(hidden_states, residual, proj.packed, norm.weight.data):
+                qkv, residual = kernels.norm_gemm_rope_kv_store(
+                    hidden_states, residual, norm.weight.data, norm.eps, proj.packed, bias, positions,
+                    self.rotary_emb.cos_sin_cache, self.num_heads, self.num_kv_heads, self.head_dim, **rope)
+                return self._attend(qkv), residual
+            if residual is None:
+                hidden_states, residual = norm(hidden_states), hidden_states
+            else:
+                hidden_states, residual = norm(hidden_states, residual)
+            return self.forward(positions, hidden_states), residual
         rows = hidden_states.size(0)
         # Decode rows run inside a captured graph, where the library's estimate of GPU time decides.  A prefill step
         # is launched eagerly and is bound by the host up to about 2 k tokens (5.4 ms for 24 layers whatever the
@@ -80,7 +94,6 @@ class Qwen3Attention(nn.Module):
                                                           self.num_heads, self.num_kv_heads, self.head_dim))
         # From prefill sizes on, the streamed tiles do the same where a product is short: 14.6 k rows, vendor product + RoPE pass
         # and one launch: K 1024 165 and 148 us, K 896 70 and 61; 8 k rows of K 3584: 246 and 264.
-        bias = None if proj.bias is None else proj.bias.data
         if many_rows and not fused and self.fuse_qkv_rope and proj.packed.in_features <= 2048 and self.head_dim in (64, 128) and \
                 kernels.streams(hidden_states, proj.packed, bias, self.rotary_emb.cos_sin_cache, rope["k_cache"], rope["v_cache"],
                                 rope["q_norm_w"], rope["k_norm_w"]):
@@ -95,11 +108,14 @@ class Qwen3Attention(nn.Module):
             qkv = self.qkv_proj(hidden_states, partial_out=True)   # split-K slabs + bias, summed inside the RoPE kernel
             qkv = kernels.rope_kv_store(qkv, positions, self.rotary_emb.cos_sin_cache, self.num_heads,
                                         self.num_kv_heads, self.head_dim, **rope)
+        return self._attend(qkv)
+
+    def _attend(self, qkv):
         q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
         q = q.view(-1, self.num_heads, self.head_dim)
         k = k.view(-1, self.num_kv_heads, self.head_dim)
         v = v.view(-1, self.num_kv_heads, self.head_dim)
-        o = attn.forward_fused(q, k, v)
+        o = self.attn.forward_fused(q, k, v)
         return self.o_proj(o.view(o.size(0), -1), partial_out=True)
 
 
@@ -114,7 +130,15 @@ class Qwen3MLP(nn.Module):
         assert hidden_act == "silu"
         self.act_fn = SiluAndMul()
 
-    def forward(self, x):
+    def forward(self, x, norm=None, residual=None):
+        """``norm``: as in Qwen3Attention.forward."""
+        if norm is not None:
+            proj = self.gate_up_proj
+            if proj.packed is not None and proj.fused_silu and kernels.takes_norm(x, residual, proj.packed, norm.weight.data):
+                act, residual = kernels.norm_gemm_silu(x, residual, norm.weight.data, norm.eps, proj.packed)
+                return self.down_proj(act, partial_out=True), residual
+            x, residual = norm(x, residual)
+            return self.forward(x), residual
         if self.gate_up_proj.fused_silu:
             act = self.gate_up_proj.forward_silu_mul(x)
         else:
@@ -141,14 +165,9 @@ class Qwen3DecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(config.hidden_size, eps=config.rms_norm_eps)
 
     def forward(self, positions, hidden_states, residual):
-        if residual is None:
-            hidden_states, residual = self.input_layernorm(hidden_states), hidden_states
-        else:
-            hidden_states, residual = self.input_layernorm(hidden_states, residual)
-        hidden_states = self.self_attn(positions, hidden_states)
-        hidden_states, residual = self.post_attention_layernorm(hidden_states, residual)
-        hidden_states = self.mlp(hidden_states)
-        return hidden_states, residual
+        # each half takes its own norm: a few rows' is formed in the product that reads it (kernels.takes_norm)
+        hidden_states, residual = self.self_attn(positions, hidden_states, self.input_layernorm, residual)
+        return self.mlp(hidden_states, self.post_attention_layernorm, residual)
 
 
 class Qwen3Model(nn.Module):

@@ -176,6 +176,20 @@ int nv_gemm_stream_rope_kv_store(const void* x, int64_t x_row_stride, const void
                                  const void* q_norm_w, const void* k_norm_w, float eps, int H, int Hkv, int D, int dtype,
                                  nv_stream_t stream);
 
+/* A residual add and RMSNorm (RMSNorm.add_rms_forward, nanovllm/layers/layernorm.py:31-41) inside the product that follows, for up to 16
+ * rows.  x [M, K], or the fp32 slabs of a split-K product (x NULL); residual NULL: the norm alone; residual_out: another buffer than
+ * residual.  w_tiled: NV_W_DENSE_TILED, K a multiple of 128 up to 2048, M rows of which fit 48 KB.
+ * nv_norm_gemm_silu: gate/up rows as nv_gemm's silu(gate)*up epilogue wants them, out [M, N / 2];
+ * nv_norm_gemm_rope_kv_store: the rest as in nv_gemm_rope_kv_store, `head_eps` for the per-head norms. */
+int nv_norm_gemm_silu(const void* x, const float* partials, int num_partials, const void* residual, void* residual_out,
+                      const void* norm_w, float eps, const void* w_tiled, void* out, int64_t out_row_stride, int M, int N, int K,
+                      int dtype, nv_stream_t stream);
+int nv_norm_gemm_rope_kv_store(const void* x, const float* partials, int num_partials, const void* residual, void* residual_out,
+                               const void* norm_w, float eps, const void* w_tiled, const void* bias, void* qkv,
+                               int64_t qkv_row_stride, int M, int K, const int64_t* positions, const float* cos_sin,
+                               const int32_t* slot_mapping, void* k_cache, void* v_cache, const void* q_norm_w,
+                               const void* k_norm_w, float head_eps, int H, int Hkv, int D, int dtype, nv_stream_t stream);
+
 /* Weight of any nv_gemm format (NV_W_*) -> row-major [N, K] in the model dtype: tiled layouts un-tiled, int4 / int8
  * dequantised as (u - 8) * s resp. q * s in fp32, rounded once (the oracle's dequantisation, so nv_gemm_lt on the result
  * is "dequantise, then F.linear").  gate_up_rows != 0: the rows are stored in the order of nv_gemm's silu(gate)*up

@@ -1,0 +1,106 @@
+"""nv_norm_gemm_* (csrc/norm_gemm.hip): a few rows' residual add and RMSNorm inside the product that reads them, against the same
+steps in launches of their own (which have tests against the oracle)."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+DT = {"bf16": torch.bfloat16, "fp16": torch.float16}
+
+
+def inputs(M, K, dt, form):
+    """form: the rows alone, rows and residual, or split-K slabs and residual -> (x for the fused call, x as rows, residual)"""
+    from byox_vllm_amd import kernels
+    res = None if form == "first" else torch.randn(M, K, device=DEV).to(dt)
+    if not form.startswith("slabs"):
+        x = torch.randn(M, K, device=DEV).to(dt)
+        return x, x, res
+    n = int(form[5:])
+    slabs = torch.randn(n, M, K, device=DEV) * n ** -0.5
+    total = slabs[0].clone()
+    for z in range(1, n):
+        total += slabs[z]
+    return kernels.Partials(slabs, n, M, K, None, dt), total.to(dt), res
+
+
+def normed(rows, res, w):
+    from byox_vllm_amd import kernels
+    if res is None:
+        return kernels.rms_norm(rows, w, 1e-6), rows
+    return kernels.add_rms_norm(rows, res, w, 1e-6)
+
+
+def close(got, want, dt, what):
+    # the norms' sums in another order move a normed number over a rounding now and then; products of K of them, rounded
+    scale = want.double().pow(2).mean().sqrt()
+    off = ((got.double() - want.double()).abs() / torch.maximum(want.double().abs(), scale)).max()
+    assert torch.isfinite(got).all() and off < 4 * torch.finfo(dt).eps, f"{what}: off by {off:.3g}"
+
+
+@pytest.mark.parametrize("name", ["bf16", "fp16"])
+@pytest.mark.parametrize("form", ["first", "rows", "slabs1", "slabs3", "slabs11"])
+@pytest.mark.parametrize("M,K,inter", [(1, 896, 4864), (1, 128, 8), (3, 1024, 3072), (7, 256, 24), (8, 2048, 520), (16, 1024, 40)])
+def test_silu(M, K, inter, form, name):
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.layers.quant import LinearWeight, interleave_gate_up
+    torch.manual_seed(M + K)
+    dt = DT[name]
+    x, rows, res = inputs(M, K, dt, form)
+    nw = (torch.rand(K, device=DEV) + 0.5).to(dt)
+    w = LinearWeight.dense_tiled(interleave_gate_up((torch.randn(2 * inter, K, device=DEV) * K ** -0.5).to(dt)))
+    if inter % 16 == 0:
+        h, new = normed(rows, res, nw)
+        want = kernels.gemm(h, w, silu_mul=True)
+    else:
+        h, new = normed(rows, res, nw)
+        want = kernels.gemm_stream(h, w, silu_mul=True) if w.out_features % 32 == 0 else None
+    before = None if res is None else res.clone()
+    got, kept = kernels.norm_gemm_silu(x, res, nw, 1e-6, w)
+    assert torch.equal(kept, new) and (res is None or torch.equal(res, before))
+    if want is None:
+        y = (h.double() @ w.logical_dense().double().t()).to(dt).double().view(M, -1, 4)
+        want = (torch.nn.functional.silu(y[..., :2]).to(dt).double() * y[..., 2:]).reshape(M, -1).to(dt)
+    close(got, want, dt, "silu")
+
+
+@pytest.mark.parametrize("name", ["bf16", "fp16"])
+@pytest.mark.parametrize("form", ["first", "rows", "slabs5"])
+@pytest.mark.parametrize("M,K,H,Hkv,D,norms", [(1, 896, 14, 2, 64, False), (1, 1024, 16, 8, 128, True), (5, 896, 14, 2, 64, False),
+                                               (8, 256, 3, 1, 64, True), (7, 2048, 2, 1, 128, False), (16, 1024, 1, 1, 128, True)])
+def test_rope_kv_store(M, K, H, Hkv, D, norms, form, name):
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.layers.quant import LinearWeight
+    torch.manual_seed(M + K + H)
+    dt, N = DT[name], (H + 2 * Hkv) * D
+    x, rows, res = inputs(M, K, dt, form)
+    nw = (torch.rand(K, device=DEV) + 0.5).to(dt)
+    w = LinearWeight.dense_tiled((torch.randn(N, K, device=DEV) * K ** -0.5).to(dt))
+    bias = None if norms else torch.randn(N, device=DEV).to(dt)
+    qn, kn = ((torch.rand(D, device=DEV) + 0.5).to(dt) if norms else None for _ in range(2))
+    pos = torch.randint(0, 100, (M,), device=DEV)
+    angle = torch.rand(100, D // 2, device=DEV) * 6.28
+    cos_sin = torch.cat([angle.cos(), angle.sin()], -1).contiguous()
+    slots = torch.randperm(3 * 16, device=DEV)[:M].int()
+    if M > 1:
+        slots[M // 2] = -1
+    caches = [torch.zeros(3, 16, Hkv, D, dtype=dt, device=DEV) for _ in range(4)]
+    args = dict(slot_mapping=slots, q_norm_w=qn, k_norm_w=kn, eps=1e-6)
+    got, kept = kernels.norm_gemm_rope_kv_store(x, res, nw, 1e-6, w, bias, pos, cos_sin, H, Hkv, D, k_cache=caches[0], v_cache=caches[1],
+                                                **args)
+    h, new = normed(rows, res, nw)
+    want = kernels.rope_kv_store(kernels.gemm(h, w, bias), pos, cos_sin, H, Hkv, D, k_cache=caches[2], v_cache=caches[3], **args)
+    assert torch.equal(kept, new)
+    for a, b, what in ((got, want, "q/k/v"), (caches[0], caches[2], "keys"), (caches[1], caches[3], "values")):
+        close(a, b, dt, what)
+
+
+def test_refuses_what_it_cannot_hold():
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.layers.quant import LinearWeight
+    w = LinearWeight.dense_tiled(torch.zeros(32, 2048, dtype=torch.bfloat16, device=DEV))
+    x, nw = torch.zeros(12, 2048, dtype=torch.bfloat16, device=DEV), torch.ones(2048, dtype=torch.bfloat16, device=DEV)
+    assert kernels.takes_norm(x[:4], None, w, nw) and not kernels.takes_norm(x[:5], None, w, nw)
+    assert not kernels.takes_norm(x, None, w, nw)
+    with pytest.raises(RuntimeError):
+        kernels.norm_gemm_silu(x, None, nw, 1e-6, w)
