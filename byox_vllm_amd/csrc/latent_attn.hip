@@ -4,7 +4,8 @@
 // kernel returns sum_j p_j c_j per head; the caller applies W_uv[h] afterwards.  Every head of a token reads the same
 // key rows, so a workgroup stages a tile of them in LDS once and serves all its heads from it.
 //
-//   nv_latent_kv_store : RMS norm of the latent, rotation of the shared key part, store into the token's cache row
+//   nv_latent_kv_store : RMS norm of the latent, rotation of the shared key part, store into the token's cache row;
+//   nv_latent_norms      with it the query latent's RMS norm, in workgroups beside (launches of 5.7 and 5.8 us for 8 tokens)
 //   nv_latent_q_rope   : rotation of the per-head query parts into the absorbed-query buffer
 //   nv_latent_attn     : sliding-window softmax attention, one workgroup per (token, group of heads); single tokens of a
 //                        request take latent_token.h
@@ -20,6 +21,52 @@
 
 namespace {
 
+// Rows whose norm is taken beside the latent's, in workgroups of their own (blockIdx.y == 1)
+struct NormRows {
+  const float* x;          // or null
+  int64_t rs;
+  const void* w;
+  void* out;
+  int n, quads;
+};
+
+// out[j] = x[j] / rms(x) * w[j] by one workgroup; `store`: whether there is a place for it.  In fours (aligned rows of at most 4096) a
+// row is read once and kept in registers.
+template <typename T>
+__device__ __forceinline__ void norm_row(const float* x, const T* w, T* out, int n, float eps, bool quads, bool store, float* red) {
+  typedef typename Pack4<T>::type P;
+  float ss = 0.0f;
+  if (quads) {
+    f32x4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int j = 4 * (threadIdx.x + 256 * k);
+      v[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      if (j < n) v[k] = *reinterpret_cast<const f32x4*>(x + j);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ss += v[k][r] * v[k][r];
+    }
+    ss = block_sum(ss, red);
+    if (!store) return;
+    const float inv = 1.0f / sqrtf(ss / (float)n + eps);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int j = 4 * (threadIdx.x + 256 * k);
+      if (j >= n) continue;
+      const f32x4 f = Pack4<T>::widen(*reinterpret_cast<const P*>(w + j));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[k][r] = v[k][r] * inv * f[r];
+      *reinterpret_cast<P*>(out + j) = Pack4<T>::narrow(v[k]);
+    }
+  } else {
+    for (int j = threadIdx.x; j < n; j += blockDim.x) ss += x[j] * x[j];
+    ss = block_sum(ss, red);
+    if (!store) return;
+    const float inv = 1.0f / sqrtf(ss / (float)n + eps);
+    for (int j = threadIdx.x; j < n; j += blockDim.x) st_f32<T>(out + j, x[j] * inv * ld_f32<T>(w + j));
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void latent_kv_store_kernel(const float* __restrict__ kv, int64_t kv_rs,
                                                               const T* __restrict__ norm_w,
@@ -27,18 +74,18 @@ __global__ __launch_bounds__(256) void latent_kv_store_kernel(const float* __res
                                                               const float* __restrict__ inv_freq, float mscale,
                                                               const int32_t* __restrict__ slot_mapping,
                                                               T* __restrict__ cache, int rank, int rot_dim, int rot_dims,
-                                                              float eps, int interleaved) {
+                                                              float eps, int interleaved, int quads, NormRows q) {
   __shared__ float red[32];
   const int64_t t = blockIdx.x;
+  if (blockIdx.y) {
+    norm_row<T>(q.x + t * q.rs, reinterpret_cast<const T*>(q.w), reinterpret_cast<T*>(q.out) + t * q.n, q.n, eps, q.quads, true, red);
+    return;
+  }
   const int32_t slot = slot_mapping[t];
   const float* row = kv + t * kv_rs;
-  float ss = 0.0f;
-  for (int j = threadIdx.x; j < rank; j += blockDim.x) ss += row[j] * row[j];
-  ss = block_sum(ss, red);
+  T* dst = cache + (int64_t)(slot < 0 ? 0 : slot) * (rank + rot_dim);
+  norm_row<T>(row, norm_w, dst, rank, eps, quads, slot >= 0, red);
   if (slot < 0) return;
-  const float inv = 1.0f / sqrtf(ss / (float)rank + eps);
-  T* dst = cache + (int64_t)slot * (rank + rot_dim);
-  for (int j = threadIdx.x; j < rank; j += blockDim.x) st_f32<T>(dst + j, row[j] * inv * ld_f32<T>(norm_w + j));
   const float pos = (float)positions[t];
   const int half = rot_dims / 2;
   for (int j = threadIdx.x; j < rot_dim; j += blockDim.x) {
@@ -534,14 +581,28 @@ extern "C" int nv_latent_kv_store(const float* kv, int64_t kv_row_stride, const 
                                   const float* inv_freq, float mscale, const int32_t* slot_mapping, void* cache,
                                   int64_t tokens, int rank, int rot_dim, int rot_dims, int interleaved, float eps,
                                   int dtype, nv_stream_t stream) {
+  return nv_latent_norms(kv, kv_row_stride, norm_w, positions, inv_freq, mscale, slot_mapping, cache, tokens, rank, rot_dim, rot_dims,
+                         interleaved, nullptr, 0, nullptr, nullptr, 0, eps, dtype, stream);
+}
+
+extern "C" int nv_latent_norms(const float* kv, int64_t kv_row_stride, const void* norm_w, const int64_t* positions,
+                               const float* inv_freq, float mscale, const int32_t* slot_mapping, void* cache, int64_t tokens,
+                               int rank, int rot_dim, int rot_dims, int interleaved, const float* q, int64_t q_row_stride,
+                               const void* q_norm_w, void* q_out, int q_rank, float eps, int dtype, nv_stream_t stream) {
   NV_CHECK_ARG(kv && norm_w && positions && inv_freq && slot_mapping && cache, "nv_latent_kv_store: null pointer");
+  NV_CHECK_ARG(!q || (q_norm_w && q_out && q_rank > 0), "nv_latent_norms: null pointer");
   NV_CHECK_ARG(dtype == NV_BF16 || dtype == NV_F32, "nv_latent_kv_store: bad dtype %d", dtype);
   NV_CHECK_ARG(tokens >= 0 && rank > 0 && rot_dim >= 0 && rot_dims >= 0 && rot_dims <= rot_dim && rot_dims % 2 == 0,
                "nv_latent_kv_store: bad shape rank=%d rot_dim=%d rot_dims=%d", rank, rot_dim, rot_dims);
   if (tokens == 0) return NV_OK;
-  NV_DISPATCH_T(dtype, latent_kv_store_kernel<T><<<dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream>>>(
+  auto quads = [](const float* x, int64_t rs, const void* w, const void* out, int n, int out_row) {
+    return n <= 4096 && n % 4 == 0 && rs % 4 == 0 && out_row % 4 == 0 && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 == 0;
+  };
+  const NormRows rows{q, q_row_stride, q_norm_w, q_out, q_rank, q ? quads(q, q_row_stride, q_norm_w, q_out, q_rank, q_rank) : 0};
+  const int kv_quads = quads(kv, kv_row_stride, norm_w, cache, rank, rank + rot_dim);
+  NV_DISPATCH_T(dtype, latent_kv_store_kernel<T><<<dim3((unsigned)tokens, q ? 2 : 1), dim3(256), 0, (hipStream_t)stream>>>(
                            kv, kv_row_stride, (const T*)norm_w, positions, inv_freq, mscale, slot_mapping, (T*)cache,
-                           rank, rot_dim, rot_dims, eps, interleaved));
+                           rank, rot_dim, rot_dims, eps, interleaved, kv_quads, rows));
   NV_CHECK_LAUNCH();
   return NV_OK;
 }

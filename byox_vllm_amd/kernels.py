@@ -837,16 +837,24 @@ def residual_pair(x, x0, dtype, delta=None):
 
 
 def latent_kv_store(kv, norm_w, positions, inv_freq, mscale, slot_mapping, cache, rank, rot_dim, rot_dims, eps,
-                    interleaved=False):
-    """``interleaved``: dimension 2i turns with 2i + 1 instead of i with i + rot_dims / 2."""
+                    interleaved=False, q=None, q_norm_w=None):
+    """``interleaved``: dimension 2i turns with 2i + 1 instead of i with i + rot_dims / 2.  ``q`` fp32 [T, q_rank]: its RMS norm
+    in the same launch, times ``q_norm_w`` -> rows of the cache's dtype."""
     require_gpu(kv, "latent_kv_store")
     assert kv.dtype == torch.float32 and kv.stride(1) == 1 and kv.size(1) == rank + rot_dim
     assert positions.dtype == torch.int64 and slot_mapping.dtype == torch.int32 and inv_freq.dtype == torch.float32
     assert cache.is_contiguous() and cache.size(-1) == rank + rot_dim and cache.dtype == norm_w.dtype
     assert positions.numel() == slot_mapping.numel() == kv.size(0) and inv_freq.numel() * 2 >= rot_dims
-    check(lib().nv_latent_kv_store(ptr(kv), kv.stride(0), ptr(norm_w), ptr(positions), ptr(inv_freq), mscale,
-                                   ptr(slot_mapping), ptr(cache), kv.size(0), rank, rot_dim, rot_dims, int(interleaved),
-                                   eps, _code32(cache.dtype), stream()), "nv_latent_kv_store")
+    out = None
+    if q is not None:
+        assert q.dtype == torch.float32 and q.stride(1) == 1 and q.size(0) == kv.size(0)
+        assert q_norm_w.dtype == cache.dtype and q_norm_w.numel() == q.size(1)
+        out = torch.empty(q.shape, dtype=cache.dtype, device=q.device)
+    check(lib().nv_latent_norms(ptr(kv), kv.stride(0), ptr(norm_w), ptr(positions), ptr(inv_freq), mscale, ptr(slot_mapping),
+                                ptr(cache), kv.size(0), rank, rot_dim, rot_dims, int(interleaved), ptr(q),
+                                0 if q is None else q.stride(0), ptr(q_norm_w), ptr(out), 0 if q is None else q.size(1), eps,
+                                _code32(cache.dtype), stream()), "nv_latent_norms")
+    return out
 
 
 def latent_q_rope(q, positions, inv_freq, mscale, qa, heads, dim, rot_dim, rot_dims, rank, interleaved=False):

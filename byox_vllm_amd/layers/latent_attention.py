@@ -66,11 +66,14 @@ class LatentAttention(nn.Module):
         H, d, r, R = self.heads, self.dim, self.rot_dim, self.kv_rank
         inv_freq = self.inv_freq if self.inv_freq.dtype == torch.float32 else self.inv_freq.float()
         dn = self.down(h, out_dtype=torch.float32)
-        q = self.uq(kernels.rms_norm_f32(dn[:, :self.q_rank], self.dq_norm.data, self.eps))
         if self.own_kv:
             at = self.down.offset("dkv")
-            kernels.latent_kv_store(dn[:, at: at + R + r], self.dkv_norm.data, positions, inv_freq, self.magnitude,
-                                    ctx.slot_mapping, self.cache, R, r, self.rot_dims, self.eps, self.interleaved)
+            dq = kernels.latent_kv_store(dn[:, at: at + R + r], self.dkv_norm.data, positions, inv_freq, self.magnitude,
+                                         ctx.slot_mapping, self.cache, R, r, self.rot_dims, self.eps, self.interleaved,
+                                         q=dn[:, :self.q_rank], q_norm_w=self.dq_norm.data)
+        else:
+            dq = kernels.rms_norm_f32(dn[:, :self.q_rank], self.dq_norm.data, self.eps)
+        q = self.uq(dq)
         src = self if self.own_kv else self.kv_source
         T = h.size(0)
         if self._expands(ctx, h):

@@ -515,6 +515,11 @@ int nv_rotation_table(const int64_t* positions, const double* inv_freq, float* o
 int nv_latent_kv_store(const float* kv, int64_t kv_row_stride, const void* norm_w, const int64_t* positions,
                        const float* inv_freq, float mscale, const int32_t* slot_mapping, void* cache, int64_t tokens,
                        int rank, int rot_dim, int rot_dims, int interleaved, float eps, int dtype, nv_stream_t stream);
+/* nv_latent_kv_store, and in the same launch q_out[t] = rms_norm(q[t]) * q_norm_w over rows of q_rank (q NULL: that alone is left out) */
+int nv_latent_norms(const float* kv, int64_t kv_row_stride, const void* norm_w, const int64_t* positions, const float* inv_freq,
+                    float mscale, const int32_t* slot_mapping, void* cache, int64_t tokens, int rank, int rot_dim, int rot_dims,
+                    int interleaved, const float* q, int64_t q_row_stride, const void* q_norm_w, void* q_out, int q_rank, float eps,
+                    int dtype, nv_stream_t stream);
 int nv_latent_q_rope(const void* q, int64_t q_row_stride, const int64_t* positions, const float* inv_freq, float mscale,
                      float* qa, int64_t tokens, int heads, int dim, int rot_dim, int rot_dims, int interleaved, int rank,
                      int dtype, nv_stream_t stream);

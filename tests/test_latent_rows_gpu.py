@@ -38,3 +38,35 @@ def test_query_rows(dtype, interleaved, H, dim, rot, rot_dims):
     y, z = u * a.cos() - v * a.sin(), v * a.cos() + u * a.sin()
     want[..., dim:dim + rot_dims] = mag * (torch.stack([y, z], -1).flatten(-2) if interleaved else torch.cat([y, z], -1))
     assert ((got - want * scale).abs() <= 8 * 2.0 ** -24 * (want * scale).abs().max()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rank,rot,q_rank", [(512, 32, 1024), (24, 8, 36), (9, 2, 7), (4100, 4, 4096), (8, 0, 4104), (512, 30, 1022)])
+def test_norms_of_both_latents(dtype, rank, rot, q_rank):
+    """The latent's norm and store with the query latent's norm beside it, in fours and one by one; an unkept token."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(rank)
+    T, eps = 9, 1e-5
+    dn = torch.randn(T, q_rank + rank + rot + 5, device=DEV)
+    w, qw = (torch.rand(rank, device=DEV) + 0.5).to(dtype), (torch.rand(q_rank, device=DEV) + 0.5).to(dtype)
+    slots = torch.randperm(16, device=DEV)[:T].int()
+    slots[4] = -1
+    cache = torch.zeros(16, rank + rot, dtype=dtype, device=DEV)
+    pos = torch.zeros(T, dtype=torch.int64, device=DEV)
+    freq = torch.ones(max(1, rot // 2), device=DEV)
+    kv, q = dn[:, q_rank:q_rank + rank + rot], dn[:, :q_rank]
+    got = kernels.latent_kv_store(kv, w, pos, freq, 1.0, slots, cache, rank, rot, rot, eps, q=q, q_norm_w=qw)
+
+    def rms(x, f):
+        x = x.double()
+        return x * torch.rsqrt((x * x).mean(-1, keepdim=True) + eps) * f.double()
+    # the sum of squares in fp32 in any order, then the reciprocal root, two products and the storage type's rounding
+    tol = (rank + q_rank) ** 0.5 * 2.0 ** -24 + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -21)
+    keep = slots >= 0
+    rows = cache[slots[keep].long()].double()
+    for a, b in ((got.double(), rms(q, qw)), (rows[:, :rank], rms(kv[keep][:, :rank], w))):
+        assert ((a - b).abs() <= tol * b.abs()).all()
+    assert torch.equal(rows[:, rank:], kv[keep][:, rank:].to(dtype).double())          # position 0: nothing turns
+    empty = torch.ones(16, dtype=torch.bool, device=DEV)
+    empty[slots[keep].long()] = False
+    assert not cache[empty].any()
