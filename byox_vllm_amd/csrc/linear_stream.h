@@ -1,4 +1,4 @@
-// nv_linear for many rows in bf16: the products, groups and epilogues of LinArgs on the tiles of stream_tiles.h.  Included by
+// nv_linear for many rows: the products, groups and epilogues of LinArgs on the tiles of stream_tiles.h.  Included by
 // linear.hip.  Groups (experts) of unknown size: every workgroup counts the tiles from the offsets with one wavefront-wide prefix
 // sum; a group that ends in the upper half of a tile's rows costs the half.
 #pragma once
@@ -34,9 +34,9 @@ __device__ __forceinline__ u32x4 pack8(const float* v) {
   return u32x4{pack2<bf16_t>(v[0], v[1]), pack2<bf16_t>(v[2], v[3]), pack2<bf16_t>(v[4], v[5]), pack2<bf16_t>(v[6], v[7])};
 }
 
-template <typename TO, int EPI>
+template <typename TT, typename TO, int EPI>
 struct LinearJob {
-  typedef bf16_t T;
+  typedef TT T;
   static constexpr int BM = STREAM_BM, MT = 8, NT = 4;              // four wavefronts along the columns
   static constexpr bool GLU = EPI == EPI_GLU, PAIRED = sizeof(TO) == 2;
   typedef std::conditional_t<PAIRED, StreamPaired, StreamNatural> Order;
@@ -89,13 +89,13 @@ struct LinearJob {
     return at;
   }
   __device__ __forceinline__ const void* a_base(const StreamTile& at) const { return reinterpret_cast<const T*>(p.a) + at.z * p.a_bs; }
-  __device__ __forceinline__ uint32_t a_stride() const { return (uint32_t)p.a_rs * 2; }
+  __device__ __forceinline__ uint32_t a_stride() const { return (uint32_t)p.a_rs * sizeof(T); }
   __device__ __forceinline__ uint32_t a_row(const StreamTile& at, int r) const {
     const int s = min(at.lo + r, at.hi - 1);
     return (uint32_t)(p.a_rows ? p.a_rows[s] : s);
   }
   __device__ __forceinline__ const void* w_base(const StreamTile& at) const { return reinterpret_cast<const T*>(p.w) + at.z * p.w_bs; }
-  __device__ __forceinline__ uint32_t w_stride() const { return (uint32_t)p.w_rs * 2; }
+  __device__ __forceinline__ uint32_t w_stride() const { return (uint32_t)p.w_rs * sizeof(T); }
   __device__ __forceinline__ uint32_t w_row(const StreamTile& at, int r) const {
     // a wavefront's 64 rows: 64 columns, or 32 columns' gates and the same columns' ups
     if constexpr (GLU) return min(at.n0 + 32 * (r >> 6) + (r & 31), p.N - 1) + ((r & 32) ? p.N : 0);
@@ -157,15 +157,15 @@ struct LinearJob {
 };
 
 // two K blocks at least, row strides whose bytes are 32-bit numbers, tiles that fit the workgroups' lists
-inline bool stream_takes(const LinArgs& p, int64_t total_rows, int batch, int cols) {
+inline bool stream_takes(const LinArgs& p, int esz, int64_t total_rows, int batch, int cols) {
   const int64_t rows = p.group_off ? total_rows / 256 + batch : (p.M + 255) / 256 * batch;
   if (total_rows >= ((int64_t)1 << 31) || rows * ((cols + 255) / 256) > 256 * (STREAM_LIST - 2)) return false;
-  return p.K >= 128 && p.K % 64 == 0 && p.a_rs >= 0 && p.w_rs >= 0 && p.a_rs < ((int64_t)1 << 31) && p.w_rs < ((int64_t)1 << 31);
+  return p.K * esz >= 256 && p.K * esz % 128 == 0 && p.a_rs >= 0 && p.w_rs >= 0 && p.a_rs < ((int64_t)1 << 30) && p.w_rs < ((int64_t)1 << 30);
 }
 
-template <typename TO, int EPI>
+template <typename T, typename TO, int EPI>
 hipError_t launch_stream_epi(const LinArgs& p, int64_t total_rows, int batch, hipStream_t s) {
-  typedef LinearJob<TO, EPI> Job;
+  typedef LinearJob<T, TO, EPI> Job;
   constexpr int64_t unit = sizeof(TO) == 2 ? 8 : 4;
   const int nt = (p.N + Job::NOUT - 1) / Job::NOUT;
   const int vec = p.N % unit == 0 && p.out_rs % unit == 0 && p.out_bs % unit == 0 && (uintptr_t)p.out % 16 == 0;

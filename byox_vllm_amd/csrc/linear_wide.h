@@ -1,5 +1,5 @@
 // nv_linear for many rows: tiles of BM x BN outputs with both operands in LDS, filled by LDS-DMA.  Included by linear.hip.  These
-// serve fp32, and 16 bits where tiles of 256 x 256 (linear_stream.h) would leave much of the chip idle.
+// serve what tiles of 256 x 256 (linear_stream.h) would leave much of the chip idle for.
 //
 // What bounds it: the matrix cores, and for small products the latency of one round of tiles.
 //   * A K block is 128 bytes of every row (64 bf16, 32 fp32);
@@ -254,28 +254,31 @@ hipError_t launch_wide_one(const LinArgs& p, int64_t total_rows, int batch, hipS
 // full (bf16, 32768 rows by 6144 columns of K 2048: 1150 TFLOP/s in the streams of 256 x 256, which have a CU to themselves; 742 and
 // 608 in the others, of which two share one).  A last round of 256 x 256 that half of the chip would have is dealt in halves and
 // costs 0.85 of a round (12000 rows by 2048, K 1024, 1.5 rounds: 65 us, 128 x 128 93, 64 x 128 88; 4096 by 2048, half a round:
-// 29.4, 29.3, 33; 5000 by 1536, K 1536: 38, 34, 43).  fp32 has the two smaller ones: its slower matrix instructions hide the loads.
+// 29.4, 29.3, 33; 5000 by 1536, K 1536: 38, 34, 43).
+// fp32 is bound by its matrix instructions alone: a workgroup that has a CU to itself is twice as fast as one of two, so rounds count
+// tiles per CU, and half a tile costs little more than half (reached when full 135, 130 and 121; 256, 128 and 64 rows: 3135 by 4416,
+// K 1024 256, 271 and 265 us; 4096 by 4416 383, 340, 343; 2000 by 2208, K 512 73, 73, 60; 2500 by 6144 256, 267, 281).
 enum { TILE_256 = 2, TILE_128 = 1, TILE_64 = 0 };
 inline int64_t wide_tiles(int bm, int bn, int64_t m, int64_t total_rows, int cols, int batch, bool grouped) {
   // groups end inside a tile: half a tile each on average
   return (grouped ? (total_rows + bm - 1) / bm + batch / 2 : (m + bm - 1) / bm * batch) * ((cols + bn - 1) / bn);
 }
-inline int pick_wide_tile(int64_t m, int64_t total_rows, int cols, int batch, bool grouped, bool has_256) {
-  auto cost = [&](int bm, int bn, int per_cu, double reached) {
+inline int pick_wide_tile(int64_t m, int64_t total_rows, int cols, int batch, bool grouped, bool fp32, bool has_256) {
+  auto cost = [&](int bm, int bn, int per_cu, double reached, double half) {
     const int64_t slots = 256 * per_cu, tiles = wide_tiles(bm, bn, m, total_rows, cols, batch, grouped), over = tiles % slots;
-    const double last = over == 0 ? 0.0 : bm == 256 && 2 * over <= slots ? 0.85 : 1.0;
+    const double last = over == 0 ? 0.0 : bm == 256 && 2 * over <= slots ? half : 1.0;
     return ((double)(tiles / slots) + last) * per_cu * bm * bn / reached;
   };
-  const double c64 = cost(64, 128, 2, 608), c128 = cost(128, 128, 2, 742), c256 = cost(256, 256, 1, 1150);
+  const int pair = fp32 ? 1 : 2;
+  const double c64 = cost(64, 128, pair, fp32 ? 121 : 608, 1.0), c128 = cost(128, 128, pair, fp32 ? 130 : 742, 1.0);
+  const double c256 = cost(256, 256, 1, fp32 ? 135 : 1150, fp32 ? 0.55 : 0.85);
   if (has_256 && c256 < c128 && c256 < c64) return TILE_256;
   return c128 < c64 ? TILE_128 : TILE_64;
 }
 
 template <typename T, typename TO, int EPI>
 hipError_t launch_wide_epi(const LinArgs& p, int64_t total_rows, int batch, int tile, hipStream_t s) {
-  if constexpr (sizeof(T) == 2) {
-    if (tile == TILE_256) return launch_stream_epi<TO, EPI>(p, total_rows, batch, s);
-  }
+  if (tile == TILE_256) return launch_stream_epi<T, TO, EPI>(p, total_rows, batch, s);
   if (tile == TILE_128) return launch_wide_one<T, TO, EPI, 2, 2, 2, 2>(p, total_rows, batch, s);
   return launch_wide_one<T, TO, EPI, 1, 2, 2, 3>(p, total_rows, batch, s);
 }

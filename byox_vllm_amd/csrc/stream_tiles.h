@@ -1,4 +1,4 @@
-// Products of many rows, 16-bit operands: a workgroup per CU walks tiles of 256 x 256 outputs whose K blocks form one stream.
+// Products of many rows: a workgroup per CU walks tiles of 256 x 256 outputs whose K blocks form one stream.
 //
 // What bounds it: the matrix cores and, on this part, their power: at 8192 x 8192 x 8192 the loop that this one replaced (a block
 // fetched, waited for and multiplied behind one barrier, 32 x 32 products) kept them 56 % busy at 1.76 GHz, the vendor library's
@@ -22,7 +22,7 @@
 // (at the end of everything, its column panels come from memory again: the experts' layer 1450 us against 1418).
 //
 // Job (what is multiplied and what becomes of it) provides:
-//   T, Order (how W lies, below), NSTORE, K (elements, a multiple of 64, at least 128)
+//   T, Order (how W lies, below), NSTORE, K (elements, two blocks of 128 bytes at least)
 //   int count(lane)                       how many tiles there are
 //   StreamTile find(tile, lane)           which rows and columns the thread's tile has (every thread of a wavefront calls it)
 //   const void* a_base(tile); uint32_t a_row(tile, r); uint32_t a_stride()      row r of the tile's A rows (those past the end
@@ -48,6 +48,12 @@ __device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x
 }
 __device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x4 c, f16_t) {
   return mfma16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c);
+}
+__device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x4 c, float) {
+  // product e takes number 4 g + e of the sixteen that the four groups of lanes hold
+#pragma unroll
+  for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[e]), __uint_as_float(b[e]), c, 0, 0, 0);
+  return c;
 }
 
 // Where W lies in LDS and which of its rows a fragment has.  W stays in the order it has in memory, so that neighbouring lanes of a
@@ -208,7 +214,7 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
   };
   clear();
 
-  const int blocks = job.K / 64;
+  const int blocks = job.K / (128 / (int)sizeof(T));
   StreamTile at = listed(0), ahead = at;
   point(at);
   lanes();

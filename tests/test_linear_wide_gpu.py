@@ -95,6 +95,18 @@ def test_streams_of_tiles(M, N, K, act, monkeypatch):
         kernels.block_many_rows(False)
 
 
+@pytest.mark.parametrize("M,N,K", [(256 * 70 + 12, 1000, 64), (256 * 33, 2048, 96), (256 * 40 + 130, 515, 160), (300, 260, 64)])
+def test_streams_of_fp32_tiles(M, N, K, monkeypatch):
+    from byox_vllm_amd import kernels
+    monkeypatch.setenv("NV_LINEAR_TILE", "2")
+    torch.manual_seed(M + N)
+    x, w, b = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV) * 0.1, torch.randn(N, device=DEV)
+    for out_dtype in (torch.bfloat16, torch.float32):
+        got = kernels.linear(x, w, b, out_dtype=out_dtype)
+        for lo in range(0, M, 8192):
+            close(got[lo:lo + 8192], x[lo:lo + 8192].double() @ w.double().t() + b.double(), K, torch.float32, out_dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_batches_and_gates(dtype):
     """One product per head side by side, with the row gate, the soft cap and the element-wise epilogues."""
