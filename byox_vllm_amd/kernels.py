@@ -584,9 +584,10 @@ def linear(x, w, bias=None, out=None, out_dtype=None, *, rows=None, a_rows=None,
     # prefill-sized plain products of a 16-bit model go where the engine sends its other many-row products: the vendor library, here
     # with the result left in fp32.  Not those with an epilogue, which nv_linear forms on the way (16384 rows 2048 -> 2 x 6144, SiLU:
     # 714 us, the library and a pass over its result 928; 4096 rows 1024 -> 4096 48 and 65), nor those of a short K whose columns do
-    # not split into the library's tiles (12300 rows 1024 -> 3088: 95 and 110; 512 -> 1552: 42 and 49; 2048 -> 4112: 325 and 290).
+    # not split into the library's tiles, where the results fill 0.7 of nv_linear's rounds of 256 x 256 (12300 rows 1024 -> 3088, 0.75:
+    # 95 and 110; 5500 rows, 0.5: a layer 136 and 129; 12300 rows 2048 -> 4112: 325 and 290).
     if (epilogue == EPI_NONE and batch == 1 and group_offsets is None and a_rows is None and bias is None and out is None
-            and row_scale is None and not (K <= 1024 and n > 1024 and n % 256)
+            and row_scale is None and not (K <= 1024 and n > 1024 and n % 256 and _fills_rounds(M, n))
             and rows is None and x.dtype == torch.bfloat16 and (out_dtype or x.dtype) in (torch.float32, torch.bfloat16)
             and w.dim() == 2 and w.is_contiguous() and x.stride(0) % 8 == 0 and use_many_rows_path(M, K, n) and K % 8 == 0
             and n % 8 == 0 and x.data_ptr() % 16 == 0):
@@ -616,6 +617,11 @@ def linear(x, w, bias=None, out=None, out_dtype=None, *, rows=None, a_rows=None,
                                out_batch_stride, bias_stride, ptr(group_offsets), epilogue, act, ptr(gate), gate_stride,
                                cap, ptr(row_scale), M, _code32(x.dtype), stream()), "nv_linear_rows")
     return out
+
+
+def _fills_rounds(M, n) -> bool:
+    """Whether M x n results take up 0.7 of the chip-wide rounds of 256 tiles of 256 x 256 that hold them."""
+    return M * n >= 0.7 * 65536 * 256 * -(-(-(-M // 256) * -(-n // 256)) // 256)
 
 
 def _linear_many_rows(x, w, M, N, K, out_dtype):
