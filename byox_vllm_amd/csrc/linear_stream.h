@@ -7,9 +7,7 @@
 #include "stream_tiles.h"
 
 // value(s) of one output -> what is stored (bias, activation, gate); `gate`: the row's, where there is one for all of it
-// SHORT: the result is rounded to 16 bits next; SiLU then comes from the hardware's exp2 and reciprocal, each within about 1 ulp of
-// fp32 (expf and a division are 30 instructions per result)
-template <typename T, int EPI, int ACT = -1, bool SHORT = false>
+template <typename T, int EPI, int ACT = -1>
 __device__ __forceinline__ float lin_finish(const LinArgs& p, const T* bias, float v, float u, float rsc, float gate, int64_t s, int n,
                                             int z) {
   v *= rsc;
@@ -17,8 +15,7 @@ __device__ __forceinline__ float lin_finish(const LinArgs& p, const T* bias, flo
   if constexpr (EPI == EPI_GLU) {
     u *= rsc;
     if (bias) u += ld_f32<T>(bias + p.N + n);
-    if (SHORT && p.act == 0) v = v * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * v)) * u;
-    else v = glu_act(v, u, p.act, p.epi_c);
+    v = glu_act(v, u, p.act, p.epi_c);
   } else if constexpr (EPI == EPI_SOFTCAP) {
     v = p.epi_c * tanhf(v / p.epi_c);
   } else if constexpr (EPI == EPI_ROW_GATE) {
@@ -133,7 +130,7 @@ struct LinearJob {
       const float gate = EPI == EPI_ROW_GATE && !p.act ? sigmoid_f32(p.epi_ptr[s * p.epi_rs + at.z]) : 1.0f;
       auto result = [&](int q, int e, int n) {
         const int j = q * (LEN / 4) + e / 4;
-        return lin_finish<T, EPI, ACT, PAIRED>(p, bias, acc[j][i][e & 3], GLU ? acc[(j + UP) % NT][i][e & 3] : 0.0f, rsc, gate, s, n + e, at.z);
+        return lin_finish<T, EPI, ACT>(p, bias, acc[j][i][e & 3], GLU ? acc[(j + UP) % NT][i][e & 3] : 0.0f, rsc, gate, s, n + e, at.z);
       };
       TO* o = O + s * p.out_rs;
 #pragma unroll

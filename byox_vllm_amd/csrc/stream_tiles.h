@@ -14,8 +14,7 @@
 //   * workgroups stay: the first two blocks of the next tile are on their way while the results of a tile are stored, and nothing
 //     waits for those stores but the second block after them (14592 by 4096, K 1024: 129 us with a workgroup per tile, so 117).
 //     Their tiles are found once, by a thread each, and kept in LDS: found in the loop they cost it its registers.
-// Measured, before and after: sixteen experts, 32768 rows of them, gated up 2048 -> 2 x 3072 and down, the layer 1584 and 1418 us (1382 with
-// linear_stream.h's shorter SiLU);
+// Measured, before and after: sixteen experts, 32768 rows of them, gated up 2048 -> 2 x 3072 and down, the layer 1582 and 1428 us;
 // 16384 rows 2048 -> 6144 into fp32 429 and 372 us (1110 TFLOP/s).
 // LDS rows are 128 bytes, their 16-byte pieces dealt by XOR (through the DMA's source addresses) so that the 16 rows a read touches lie
 // in 16 bank groups.  Tiles go to the XCDs in contiguous eighths, within them in bands of eight row

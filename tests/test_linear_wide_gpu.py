@@ -152,3 +152,29 @@ def test_fp32_products_on_both_sides_of_the_rule(M, N, K, H, softcap):
                          epilogue=kernels.EPI_SOFTCAP if softcap else kernels.EPI_NONE, **args).view(M, H, N)
     want = torch.matmul(x.double().view(M, H, K).transpose(0, 1), w.double().transpose(1, 2)).transpose(0, 1)
     close(got, 2.0 * torch.tanh(want / 2.0) if softcap else want, K, torch.float32, torch.float32)
+
+
+def correctly_rounded(got, want, dtype, ulps):
+    """|got - want| within half a unit of the 16-bit type and ``ulps`` units of fp32 (of the numbers before that rounding)."""
+    bits = 8 if dtype == torch.bfloat16 else 11
+    spacing = torch.exp2(torch.floor(torch.log2(want.abs().clamp_min(2.0 ** -126))) + 1 - bits)
+    bad = (got.double().cpu() - want).abs() > 0.5 * spacing + ulps * 2.0 ** -23 * want.abs()
+    assert not bad.any(), f"{int(bad.sum())} of {bad.numel()} off, the first at {want[bad][0]:.6g}: {got.double().cpu()[bad][0]:.6g}"
+
+
+@pytest.mark.parametrize("tile", ["0", "1", "2"])
+def test_gated_unit_is_exact_in_fp32(tile, monkeypatch):
+    """SiLU(gate) * up of gates and ups that the products give exactly, down to where exp(-gate) nearly overflows: the exponential
+    within 1 unit of fp32, a sum, a quotient and a product within half of one each, then bf16's rounding - in every tile size."""
+    from byox_vllm_amd import kernels
+    monkeypatch.setenv("NV_LINEAR_TILE", tile)
+    torch.manual_seed(7)
+    M, N, K = 300, 1024, 128
+    x, w = torch.zeros(M, K), torch.zeros(2 * N, K)
+    x[:, 0], x[:, 1] = 1.0, 1.0 + torch.rand(M)
+    w[:N, 0], w[N:, 1] = torch.linspace(-88.5, 20.0, N), 1.0 + torch.rand(N)
+    x, w = x.bfloat16(), w.bfloat16()
+    gate, up = (x.double() @ w.double().t()).chunk(2, -1)
+    got = kernels.linear(x.to(DEV), w.to(DEV), epilogue=kernels.EPI_GLU)
+    assert got.dtype == torch.bfloat16
+    correctly_rounded(got, gate / (1.0 + torch.exp(-gate)) * up, torch.bfloat16, 3.0)
