@@ -80,9 +80,9 @@ struct RowsJob {
         float v[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          // dtype(dtype(silu(dtype(gate))) * dtype(up)), with the hardware's exp2 and reciprocal (each about 1 ulp of fp32)
+          // dtype(dtype(silu(dtype(gate))) * dtype(up)), as nv_silu_mul takes it
           const float gt = rounded(acc[e >> 2][i][e & 3]), up = rounded(acc[2 + (e >> 2)][i][e & 3]);
-          v[e] = rounded(gt * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * gt))) * up;
+          v[e] = rounded(gt / (1.0f + expf(-gt))) * up;
         }
         *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(p.out) + s * p.os + n) = pack(v);
       } else {

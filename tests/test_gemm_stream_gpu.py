@@ -58,6 +58,22 @@ def test_silu_mul(M, inter, K, tiled, name):
 
 
 @pytest.mark.parametrize("name", ["bf16", "fp16"])
+def test_silu_mul_has_the_bits_of_the_pass_over_rows(name):
+    """Gates and ups that the products give exactly, down to where exp(-gate) nearly overflows: nv_silu_mul's bits."""
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.layers.quant import interleave_gate_up
+    torch.manual_seed(7)
+    M, inter, K, dt = 300, 1024, 128, DT[name]
+    x, w = torch.zeros(M, K), torch.zeros(2 * inter, K)
+    x[:, 0], x[:, 1] = 1.0, 1.0 + torch.rand(M)
+    w[:inter, 0], w[inter:, 1] = torch.linspace(-88.5, 20.0, inter), 1.0 + torch.rand(inter)
+    x, w = x.to(dt).to(DEV), w.to(dt).to(DEV)
+    rows = (x.double() @ w.double().t()).to(dt)
+    got = kernels.gemm_stream(x, weight(interleave_gate_up(w), True), silu_mul=True)
+    assert torch.equal(got, kernels.silu_mul(rows))
+
+
+@pytest.mark.parametrize("name", ["bf16", "fp16"])
 @pytest.mark.parametrize("tiled", [True, False])
 @pytest.mark.parametrize("T,H,Hkv,D,norms", [(1, 1, 1, 64, False), (257, 14, 2, 64, False), (300, 3, 1, 64, True), (513, 16, 8, 128, True),
                                              (4100, 5, 1, 128, False), (256 * 34 + 5, 4, 2, 128, True)])
