@@ -167,27 +167,35 @@ NORM_GEMM_ROWS = 4
 
 def takes_norm(x, residual, w, norm_w) -> bool:
     """Whether the norm of these rows can be formed in the product of ``w`` (nv_norm_gemm_*): few rows, 16-bit tiled weights."""
-    rows, cols = (x.rows, x.cols) if isinstance(x, Partials) else x.shape if torch.is_tensor(x) else (0, 0)
+    rows, cols = (x.rows, x.cols) if isinstance(x, Partials) else x.shape if torch.is_tensor(x) and x.dim() == 2 else (0, 0)
     return (0 < rows <= NORM_GEMM_ROWS and cols == w.in_features and w.fmt == _C.W_DENSE_TILED and cols <= 2048
-            and rows * (2 * cols + 16) <= 48 << 10 and norm_w.dtype == w.dtype and norm_w.data_ptr() % 16 == 0
+            and rows * (2 * cols + 16) <= 48 << 10
+            and norm_w.dtype == w.dtype and norm_w.numel() == cols and norm_w.is_contiguous() and norm_w.data_ptr() % 16 == 0
             and (x.bias is None and residual is not None if isinstance(x, Partials)
-                 else x.dtype == w.dtype and x.is_contiguous() and x.data_ptr() % 16 == 0)
-            and (residual is None or (residual.dtype == w.dtype and residual.is_contiguous() and residual.data_ptr() % 16 == 0)))
+                 else x.is_cuda and x.dtype == w.dtype and x.is_contiguous() and x.data_ptr() % 16 == 0)
+            and (residual is None or (residual.is_cuda and residual.dtype == w.dtype and residual.shape == (rows, cols)
+                                      and residual.is_contiguous() and residual.data_ptr() % 16 == 0)))
 
 
-def _norm_rows(x, residual, w):
+def _norm_rows(x, residual, norm_w, w):
     """The first arguments of nv_norm_gemm_* for rows that are a tensor or Partials -> (arguments, the new residual, M, K)."""
     _require_device_weight(w, "nv_norm_gemm")
-    M, K = (x.rows, x.cols) if isinstance(x, Partials) else x.shape
-    assert residual is None or residual.shape == (M, K)
+    slabs = isinstance(x, Partials)
+    M, K = (x.rows, x.cols) if slabs else x.shape
+    for t in (x.slabs if slabs else x, residual, norm_w):
+        if t is not None:
+            require_gpu(t, "nv_norm_gemm")
+    assert K == w.in_features and x.dtype == w.dtype and (x.bias is None if slabs else x.is_contiguous())
+    assert norm_w.numel() == K and norm_w.dtype == w.dtype and norm_w.is_contiguous()
+    assert residual is None or (residual.shape == (M, K) and residual.dtype == w.dtype and residual.is_contiguous())
     new = None if residual is None else torch.empty_like(residual)
-    head = (None, ptr(x.slabs), x.n) if isinstance(x, Partials) else (ptr(x), None, 0)
+    head = (None, ptr(x.slabs), x.n) if slabs else (ptr(x), None, 0)
     return head + (ptr(residual), ptr(new)), (x if residual is None else new), M, K
 
 
 def norm_gemm_silu(x, residual, norm_w, eps, w):
     """RMSNorm(x + residual) -> gate/up product -> SiLU(gate) * up in one launch -> ([M, N / 2], the new residual)."""
-    args, new, M, K = _norm_rows(x, residual, w)
+    args, new, M, K = _norm_rows(x, residual, norm_w, w)
     N = w.out_features
     out = torch.empty(M, N // 2, dtype=w.dtype, device=w.data.device)
     check(lib().nv_norm_gemm_silu(*args, ptr(norm_w), eps, ptr(w.data), ptr(out), out.stride(0), M, N, K, dtype_code(w.dtype),
@@ -198,7 +206,7 @@ def norm_gemm_silu(x, residual, norm_w, eps, w):
 def norm_gemm_rope_kv_store(x, residual, norm_w, norm_eps, w, bias, positions, cos_sin, num_heads, num_kv_heads, head_dim,
                             slot_mapping=None, k_cache=None, v_cache=None, q_norm_w=None, k_norm_w=None, eps=1e-6):
     """RMSNorm(x + residual) and gemm_rope_kv_store() in one launch -> (qkv, the new residual)."""
-    args, new, M, K = _norm_rows(x, residual, w)
+    args, new, M, K = _norm_rows(x, residual, norm_w, w)
     N = (num_heads + 2 * num_kv_heads) * head_dim
     assert N == w.out_features and positions.dtype == torch.int64 and positions.numel() == M and positions.is_contiguous()
     assert cos_sin.dtype == torch.float32 and cos_sin.is_contiguous() and cos_sin.size(-1) == head_dim
@@ -368,12 +376,16 @@ def gemm_stream_rope_kv_store(x, w, bias, positions, cos_sin, num_heads, num_kv_
 
 def gemm_stream(x, w, bias=None, out=None, silu_mul=False):
     """gemm() for prefill-sized x on this library's own tiles (nv_gemm_stream)."""
+    require_gpu(x, "gemm_stream")
+    _require_device_weight(w, "gemm_stream")
     M, K = x.shape
     N = w.out_features
+    assert K == w.in_features and x.stride(1) == 1 and x.dtype == w.dtype
+    assert bias is None or (bias.numel() == N and bias.dtype == x.dtype and bias.is_cuda)
     data, fmt = _rows_weight(w)
     cols = N // 2 if silu_mul else N
     out = torch.empty(M, cols, dtype=x.dtype, device=x.device) if out is None else out
-    assert out.stride(1) == 1 and out.shape == (M, cols)
+    assert out.stride(1) == 1 and out.shape == (M, cols) and out.is_cuda
     check(lib().nv_gemm_stream(ptr(x), x.stride(0), ptr(data), ptr(bias), ptr(out), out.stride(0), M, N, K, fmt, int(silu_mul),
                                dtype_code(x.dtype), stream()), "nv_gemm_stream")
     return out
@@ -853,6 +865,7 @@ def latent_kv_store(kv, norm_w, positions, inv_freq, mscale, slot_mapping, cache
     assert positions.numel() == slot_mapping.numel() == kv.size(0) and inv_freq.numel() * 2 >= rot_dims
     out = None
     if q is not None:
+        require_gpu(q, "latent_kv_store")
         assert q.dtype == torch.float32 and q.stride(1) == 1 and q.size(0) == kv.size(0)
         assert q_norm_w.dtype == cache.dtype and q_norm_w.numel() == q.size(1)
         out = torch.empty(q.shape, dtype=cache.dtype, device=q.device)

@@ -577,3 +577,20 @@ def test_next_step_is_certain_counts_down_to_boundaries_and_limits():
     assert not runner._next_step_is_certain(seqs, cache, [6, 6], [7, 7])      # the second reaches max_tokens with this token
     cache = {"sure": None}
     assert runner._next_step_is_certain(seqs, cache, [6, 5], [7, 7]) and cache["sure"] == 0
+
+
+def test_rows_in_host_memory_do_not_take_the_norm_into_the_product():
+    """kernels.takes_norm is False for what the norm in a launch of its own refuses - rows or a residual in host memory, a norm
+    weight of another size - so a layer called with them raises there instead of handing a kernel a host pointer."""
+    import pytest
+
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.layers.quant import LinearWeight
+    w = LinearWeight.dense_tiled(torch.zeros(64, 896, dtype=torch.bfloat16))
+    rows, nw = torch.zeros(2, 896, dtype=torch.bfloat16), torch.ones(896, dtype=torch.bfloat16)
+    assert not kernels.takes_norm(rows, None, w, nw) and not kernels.takes_norm(rows, rows, w, nw)
+    slabs = kernels.Partials(torch.zeros(3, 2, 896), 3, 2, 896, None, torch.bfloat16)
+    assert not kernels.takes_norm(slabs, rows, w, nw) and not kernels.takes_norm(rows, None, w, nw[:64])
+    for call in (kernels.gemm_stream, lambda x, w: kernels.norm_gemm_silu(x, None, nw, 1e-6, w)):
+        with pytest.raises(RuntimeError, match="no CPU compute path|must be device memory"):
+            call(rows, w)

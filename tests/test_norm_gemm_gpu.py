@@ -104,3 +104,28 @@ def test_refuses_what_it_cannot_hold():
     assert not kernels.takes_norm(x, None, w, nw)
     with pytest.raises(RuntimeError):
         kernels.norm_gemm_silu(x, None, nw, 1e-6, w)
+
+
+def test_refuses_operands_before_any_launch(monkeypatch):
+    """Rows or a residual in host memory, weights of another size or type: an error of the wrapper, no launch."""
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.layers.quant import LinearWeight
+
+    def launched():
+        raise SystemError("reached the library")
+    w = LinearWeight.dense_tiled(torch.zeros(32, 896, dtype=torch.bfloat16, device=DEV))
+    x, nw = torch.zeros(2, 896, dtype=torch.bfloat16, device=DEV), torch.ones(896, dtype=torch.bfloat16, device=DEV)
+    slabs = torch.zeros(2, 2, 896, device=DEV)
+    assert kernels.takes_norm(x, x, w, nw)
+    parts = lambda s: kernels.Partials(s, 2, 2, 896, None, torch.bfloat16)  # noqa: E731
+    monkeypatch.setattr(kernels, "lib", launched)
+    for rows, res, weight in ((x.cpu(), None, nw), (x, x.cpu(), nw), (x, x, nw[:64]), (x, x[:1], nw), (x.half(), None, nw),
+                              (x, x.half(), nw), (x, x, nw.half()), (x[:, :512], None, nw[:512]), (x, None, nw.cpu()),
+                              (parts(slabs.cpu()), x, nw), (parts(slabs), x, nw[:64])):
+        # (a weight or slabs in host memory: no other path has a check for them, so it is the wrapper that raises)
+        assert weight.is_cpu or getattr(rows, "slabs", nw).is_cpu or not kernels.takes_norm(rows, res, w, weight)
+        with pytest.raises((RuntimeError, AssertionError)):
+            kernels.norm_gemm_silu(rows, res, weight, 1e-6, w)
+    for rows, bias in ((x.cpu(), None), (x.half(), None), (x[:, :512], None), (x.t().contiguous().t(), None), (x, nw[:31]), (x, nw[:32].half())):
+        with pytest.raises((RuntimeError, AssertionError)):
+            kernels.gemm_stream(rows, w, bias)
