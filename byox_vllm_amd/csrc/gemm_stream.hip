@@ -75,7 +75,7 @@ struct RowsJob {
       __builtin_amdgcn_sched_barrier(0);       // one row's results at a time: registers
       const int s = row0 + 16 * i + fr;
       if constexpr (SILU) {
-        const int n = at.n0 + 32 * wn + 8 * g;
+        const int n = at.n0 + 32 * wn + 8 * g;        // a lane's eight results come from 16 rows of W: N is a multiple of that
         if (s >= at.hi || 2 * n >= p.N) continue;
         float v[8];
 #pragma unroll
@@ -218,7 +218,7 @@ int rows_launch(const char* name, const RowsArgs& p, const RopeArgs& ra, int wha
 
 extern "C" int nv_gemm_stream(const void* x, int64_t x_row_stride, const void* w, const void* bias, void* out, int64_t out_row_stride,
                               int M, int N, int K, int wfmt, int silu_mul, int dtype, nv_stream_t stream) {
-  NV_CHECK_ARG(!silu_mul || (!bias && N % 32 == 0), "nv_gemm_stream: gate and up rows come in fours of 32 without a bias");
+  NV_CHECK_ARG(!silu_mul || !bias, "nv_gemm_stream: the silu*up epilogue takes no bias");
   const RowsArgs p{x, w, bias, out, x_row_stride, out_row_stride, M, N, K, wfmt == NV_W_DENSE_TILED};
   return rows_launch("nv_gemm_stream", p, RopeArgs{}, silu_mul ? ROWS_SILU : ROWS_PLAIN, wfmt, dtype, stream);
 }

@@ -43,7 +43,8 @@ def test_plain(M, N, K, tiled, name):
 
 @pytest.mark.parametrize("name", ["bf16", "fp16"])
 @pytest.mark.parametrize("tiled", [True, False])
-@pytest.mark.parametrize("M,inter,K", [(1, 16, 128), (255, 272, 128), (300, 1536, 256), (2100, 1040, 384), (256 * 66 + 3, 512, 128)])
+@pytest.mark.parametrize("M,inter,K", [(1, 16, 128), (255, 272, 128), (300, 1536, 256), (2100, 1040, 384), (256 * 66 + 3, 512, 128),
+                                       (1, 8, 128), (700, 24, 256), (300, 1000, 128)])
 def test_silu_mul(M, inter, K, tiled, name):
     """Gate and up rows as the kernels store them, against the product's, SiLU's and the last rounding taken one by one."""
     from byox_vllm_amd import kernels
@@ -108,3 +109,19 @@ def test_rope_kv_store(T, H, Hkv, D, norms, tiled, name):
             assert (a != b).float().mean() < 1e-3
     bare = kernels.gemm_stream_rope_kv_store(x, weight(w, tiled), bias, pos, cos_sin, H, Hkv, D, q_norm_w=qn, k_norm_w=kn)
     assert torch.equal(bare, got)
+
+
+@pytest.mark.parametrize("M", [300, 2100, 4100])
+@pytest.mark.parametrize("inter", [24, 40])
+@pytest.mark.parametrize("fmt", [None, "w4a16"])
+def test_gate_up_of_any_width_at_every_row_count(M, inter, fmt):
+    """Gate/up products whose 2 * inter columns are a multiple of 16 but not of 32: from 2048 and 4096 rows on too."""
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.layers.quant import LinearWeight, interleave_gate_up
+    torch.manual_seed(M + inter)
+    K, dt = 256, torch.bfloat16
+    x, w = torch.randn(M, K, device=DEV).to(dt), (torch.randn(2 * inter, K, device=DEV) * 0.05).to(dt)
+    lw = LinearWeight.make(interleave_gate_up(w), fmt)
+    assert (2 * inter) % 32
+    gate, up = (x.double() @ kernels.expand_weight(lw, gate_up_rows=True).double().t()).to(dt).double().chunk(2, -1)
+    close(kernels.gemm(x, lw, silu_mul=True), torch.nn.functional.silu(gate).to(dt).double() * up, dt, K, ulps=3.0)
