@@ -344,8 +344,8 @@ def _rows_weight(w):
 
 
 def streams(x, w, *others):
-    """Whether nv_gemm_stream takes this product: 16-byte aligned rows, K of two blocks, a list of tiles that fits."""
-    return x.stride(0) % 8 == 0 and w.in_features % 64 == 0 and w.in_features >= 128 and \
+    """Whether nv_gemm_stream takes this product: 16-byte aligned rows that lie apart, K of two blocks, a list of tiles that fits."""
+    return x.stride(0) % 8 == 0 and x.stride(0) >= w.in_features and w.in_features % 64 == 0 and w.in_features >= 128 and \
         (-(-x.size(0) // 256)) * (-(-w.out_features // 256)) <= 256 * 510 and \
         all(t is None or t.data_ptr() % 16 == 0 for t in (x, w.data) + others)
 

@@ -125,3 +125,18 @@ def test_gate_up_of_any_width_at_every_row_count(M, inter, fmt):
     assert (2 * inter) % 32
     gate, up = (x.double() @ kernels.expand_weight(lw, gate_up_rows=True).double().t()).to(dt).double().chunk(2, -1)
     close(kernels.gemm(x, lw, silu_mul=True), torch.nn.functional.silu(gate).to(dt).double() * up, dt, K, ulps=3.0)
+
+
+@pytest.mark.parametrize("stride", [0, 64])
+def test_rows_that_overlap_stay_with_nv_gemm(stride):
+    """One row expanded over all, and windows of one buffer that overlap: as at 2047 rows, so at 2048."""
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.layers.quant import interleave_gate_up
+    torch.manual_seed(3)
+    M, K, inter, dt = 2048, 256, 64, torch.bfloat16
+    x = torch.randn(K + M * 64, device=DEV).to(dt).as_strided((M, K), (stride, 1))
+    lw = weight(interleave_gate_up((torch.randn(2 * inter, K, device=DEV) * 0.05).to(dt)), True)
+    gate, up = (x.double() @ kernels.expand_weight(lw, gate_up_rows=True).double().t()).to(dt).double().chunk(2, -1)
+    want = torch.nn.functional.silu(gate).to(dt).double() * up
+    for rows in (2047, 2048):
+        close(kernels.gemm(x[:rows], lw, silu_mul=True), want[:rows], dt, K, ulps=3.0)
