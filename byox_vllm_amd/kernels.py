@@ -350,6 +350,12 @@ def streams(x, w, *others):
         all(t is None or t.data_ptr() % 16 == 0 for t in (x, w.data) + others)
 
 
+def _streams_into(out, x, cols):
+    """Whether nv_gemm_stream may write its rows to ``out`` (or allocate them: None)."""
+    return out is None or (out.shape == (x.size(0), cols) and out.dtype == x.dtype and out.stride(1) == 1
+                           and out.stride(0) % 8 == 0 and out.stride(0) >= cols)
+
+
 def gemm_stream_rope_kv_store(x, w, bias, positions, cos_sin, num_heads, num_kv_heads, head_dim, slot_mapping=None,
                               k_cache=None, v_cache=None, q_norm_w=None, k_norm_w=None, eps=1e-6):
     """gemm_rope_kv_store() for prefill-sized x (nv_gemm_stream_rope_kv_store)."""
@@ -385,7 +391,7 @@ def gemm_stream(x, w, bias=None, out=None, silu_mul=False):
     data, fmt = _rows_weight(w)
     cols = N // 2 if silu_mul else N
     out = torch.empty(M, cols, dtype=x.dtype, device=x.device) if out is None else out
-    assert out.stride(1) == 1 and out.shape == (M, cols) and out.is_cuda
+    assert _streams_into(out, x, cols) and out.is_cuda
     check(lib().nv_gemm_stream(ptr(x), x.stride(0), ptr(data), ptr(bias), ptr(out), out.stride(0), M, N, K, fmt, int(silu_mul),
                                dtype_code(x.dtype), stream()), "nv_gemm_stream")
     return out
@@ -401,7 +407,7 @@ def gemm_many_rows(x, w, bias=None, out=None, silu_mul=False, rope=None):
     dev = x.device
     if rope is not None:
         return gemm_stream_rope_kv_store(x, w, bias, **rope)
-    if streams(x, w, bias, out) and (out is None or out.stride(0) % 8 == 0) and (bias is None if silu_mul else 512 <= K < 1024):
+    if streams(x, w, bias, out) and _streams_into(out, x, N // 2 if silu_mul else N) and (bias is None if silu_mul else 512 <= K < 1024):
         return gemm_stream(x, w, bias, out, silu_mul)
     if w.fmt == _C.W_DENSE and not silu_mul:
         wr = w.data
@@ -459,7 +465,7 @@ def gemm(x, w, bias=None, out=None, split_k=None, silu_mul=False, partial_out=Fa
         # gate/up from half as many rows on where the weight is read as it lies (2048 rows, nv_gemm and the streamed tiles:
         # 1024 -> 2 x 3072 37 and 33 us, 896 -> 2 x 4864 61 and 46; 1024 rows: 23 and 30)
         if silu_mul and bias is None and M >= MANY_ROWS // 2 and w.fmt in (_C.W_DENSE, _C.W_DENSE_TILED) and \
-                use_many_rows_path(max(M, MANY_ROWS), K, N) and streams(x, w, out) and (out is None or out.stride(0) % 8 == 0):
+                use_many_rows_path(max(M, MANY_ROWS), K, N) and streams(x, w, out) and _streams_into(out, x, N // 2):
             return gemm_stream(x, w, None, out, True)
         split_k = 1 if silu_mul else pick_split_k(M, N, K, w.fmt)
     split_k = max(1, min(split_k, K // 128))

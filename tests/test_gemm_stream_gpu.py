@@ -140,3 +140,18 @@ def test_rows_that_overlap_stay_with_nv_gemm(stride):
     want = torch.nn.functional.silu(gate).to(dt).double() * up
     for rows in (2047, 2048):
         close(kernels.gemm(x[:rows], lw, silu_mul=True), want[:rows], dt, K, ulps=3.0)
+
+
+def test_outputs_with_spare_rows_stay_with_nv_gemm():
+    """A result buffer of more rows than the product has: its first rows are written from 2048 rows on too, the others left."""
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.layers.quant import interleave_gate_up
+    torch.manual_seed(4)
+    K, inter, dt = 256, 64, torch.bfloat16
+    x = torch.randn(2100, K, device=DEV).to(dt)
+    lw = weight(interleave_gate_up((torch.randn(2 * inter, K, device=DEV) * 0.05).to(dt)), True)
+    gate, up = (x.double() @ kernels.expand_weight(lw, gate_up_rows=True).double().t()).to(dt).double().chunk(2, -1)
+    out = torch.zeros(2200, inter, dtype=dt, device=DEV)
+    kernels.gemm(x, lw, out=out, silu_mul=True)
+    close(out[:2100], torch.nn.functional.silu(gate).to(dt).double() * up, dt, K, ulps=3.0)
+    assert not out[2100:].any()
