@@ -581,6 +581,9 @@ GLU_CLAMPED = 2      # EPI_GLU only: g sigmoid(1.702 g) (u + 1) with g = min(gat
 ROUTE_CHOSEN, ROUTE_ALL, ROUTE_SIGMOID, ROUTE_SOFTMAX = 0, 1, 2, 3
 
 
+LINEAR_ROWS = 65535 * 64     # rows of one nv_linear launch
+
+
 def _code32(dt) -> int:
     return dtype_code(dt, allow_f32=True)
 
@@ -604,12 +607,19 @@ def linear(x, w, bias=None, out=None, out_dtype=None, *, rows=None, a_rows=None,
     # 714 us, the library and a pass over its result 928; 4096 rows 1024 -> 4096 48 and 65), nor those of a short K whose columns do
     # not split into the library's tiles, where the results fill 0.7 of nv_linear's rounds of 256 x 256 (12300 rows 1024 -> 3088, 0.75:
     # 95 and 110; 5500 rows, 0.5: a layer 136 and 129; 12300 rows 2048 -> 4112: 325 and 290).
-    if (epilogue == EPI_NONE and batch == 1 and group_offsets is None and a_rows is None and bias is None and out is None
-            and row_scale is None and not (K <= 1024 and n > 1024 and n % 256 and _fills_rounds(M, n))
-            and rows is None and x.dtype == torch.bfloat16 and (out_dtype or x.dtype) in (torch.float32, torch.bfloat16)
+    if (M >= MANY_ROWS and batch == 1 and group_offsets is None and a_rows is None and out is None and row_scale is None and rows is None
+            and x.dtype == torch.bfloat16 and (out_dtype or x.dtype) in (torch.float32, torch.bfloat16)
             and w.dim() == 2 and w.is_contiguous() and x.stride(0) % 8 == 0 and use_many_rows_path(M, K, n) and K % 8 == 0
             and n % 8 == 0 and x.data_ptr() % 16 == 0):
-        return _linear_many_rows(x, w, M, n, K, out_dtype or x.dtype)
+        one_launch = M <= LINEAR_ROWS
+        if epilogue == EPI_NONE and bias is None and not (K <= 1024 and n > 1024 and n % 256 and one_launch and _fills_rounds(M, n)):
+            return _linear_many_rows(x, w, M, n, K, out_dtype or x.dtype)
+        if epilogue in (EPI_GLU, EPI_ACT) and not one_launch:
+            out = torch.empty(M, n, dtype=out_dtype or x.dtype, device=x.device)
+            for lo in range(0, M, LINEAR_ROWS):
+                linear(x[lo:lo + LINEAR_ROWS], w, bias, out[lo:lo + LINEAR_ROWS], out.dtype, epilogue=epilogue, act=act, gate=gate,
+                       cap=cap, n=n)
+            return out
     grid_rows = M if group_offsets is None else (max_group_rows if max_group_rows is not None else M)
     out_dtype = out_dtype or x.dtype
     if out is None:

@@ -178,3 +178,23 @@ def test_gated_unit_is_exact_in_fp32(tile, monkeypatch):
     got = kernels.linear(x.to(DEV), w.to(DEV), epilogue=kernels.EPI_GLU)
     assert got.dtype == torch.bfloat16
     correctly_rounded(got, gate / (1.0 + torch.exp(-gate)) * up, torch.bfloat16, 3.0)
+
+
+@pytest.mark.parametrize("epilogue,n", [("GLU", 16), ("ACT", 16), ("NONE", 1040)])
+def test_more_rows_than_one_launch_holds(epilogue, n):
+    """65535 * 64 rows and some: gated and element-wise epilogues in pieces of rows, plain products through the library."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(5)
+    M, K = kernels.LINEAR_ROWS + 300, 128
+    x = torch.randn(8192, K, device=DEV).bfloat16().repeat(-(-M // 8192), 1)[:M]
+    w = (torch.randn(n * (2 if epilogue == "GLU" else 1), K, device=DEV) * 0.1).bfloat16()
+    got = kernels.linear(x, w, epilogue=getattr(kernels, "EPI_" + epilogue))
+    assert got.shape == (M, n) and got.dtype == torch.bfloat16
+    for lo, hi in ((0, 500), (kernels.LINEAR_ROWS - 300, kernels.LINEAR_ROWS + 300)):
+        want = x[lo:hi].double() @ w.double().t()
+        if epilogue == "GLU":
+            gate, up = want.chunk(2, -1)
+            want = torch.nn.functional.silu(gate) * up
+        elif epilogue == "ACT":
+            want = torch.nn.functional.silu(want)
+        close(got[lo:hi], want, 2 * K, torch.bfloat16, torch.bfloat16)
