@@ -16,6 +16,7 @@ import os
 
 import torch
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from byox_vllm_amd import kernels
 from byox_vllm_amd.layers.activation import SiluAndMul
@@ -25,6 +26,12 @@ from byox_vllm_amd.layers.layernorm import RMSNorm
 from byox_vllm_amd.layers.linear import MergedColumnParallelLinear, QKVParallelLinear, RowParallelLinear
 from byox_vllm_amd.layers.rotary_embedding import get_rope
 from byox_vllm_amd.utils.context import get_context
+
+
+def plain(module: nn.Module, cls: type) -> bool:
+    """Whether ``module`` is a ``cls`` whose call can be left out: no subclass, no forward of its own, nobody's hooks."""
+    return type(module) is cls and "forward" not in module.__dict__ and not (
+        module._forward_hooks or module._forward_pre_hooks or _has_any_global_hook())
 
 
 class Qwen3Attention(nn.Module):
@@ -58,31 +65,35 @@ class Qwen3Attention(nn.Module):
             self.q_norm = RMSNorm(self.head_dim, eps=rms_norm_eps)
             self.k_norm = RMSNorm(self.head_dim, eps=rms_norm_eps)
 
-    def forward(self, positions: torch.Tensor, hidden_states: torch.Tensor, norm=None, residual=None):
-        """``norm``: the layer's input norm, still to be taken of ``hidden_states`` and ``residual`` -> (result, new residual)."""
-        context = get_context()
-        attn = self.attn
+    def _rope_args(self) -> dict:
+        context, attn = get_context(), self.attn
         has_cache = attn.k_cache.numel() > 0
-        rope = dict(slot_mapping=context.slot_mapping if has_cache else None,
+        return dict(slot_mapping=context.slot_mapping if has_cache else None,
                     k_cache=attn.k_cache if has_cache else None, v_cache=attn.v_cache if has_cache else None,
                     q_norm_w=None if self.qkv_bias else self.q_norm.weight.data,
                     k_norm_w=None if self.qkv_bias else self.k_norm.weight.data, eps=self.rms_norm_eps)
+
+    def with_norm(self, positions: torch.Tensor, hidden_states, residual, norm: RMSNorm):
+        """forward() of norm(hidden_states, residual) -> (result, new residual) where the norm can be formed in the projection (a few
+        rows) and nobody listens for the calls this leaves out, else None."""
+        proj = self.qkv_proj
+        if proj.packed is None:
+            proj.finalize(None)
+        if not (self.fuse_qkv_rope and self.head_dim in (64, 128) and plain(self, Qwen3Attention) and plain(norm, RMSNorm) and
+                plain(proj, QKVParallelLinear) and kernels.takes_norm(hidden_states, residual, proj.packed, norm.weight.data)):
+            return None
+        qkv, residual = kernels.norm_gemm_rope_kv_store(
+            hidden_states, residual, norm.weight.data, norm.eps, proj.packed, None if proj.bias is None else proj.bias.data, positions,
+            self.rotary_emb.cos_sin_cache, self.num_heads, self.num_kv_heads, self.head_dim, **self._rope_args())
+        return self._attend(qkv), residual
+
+    def forward(self, positions: torch.Tensor, hidden_states: torch.Tensor) -> torch.Tensor:
+        context = get_context()
+        rope = self._rope_args()
         proj = self.qkv_proj
         if proj.packed is None:
             proj.finalize(None)
         bias = None if proj.bias is None else proj.bias.data
-        if norm is not None:
-            if self.fuse_qkv_rope and self.head_dim in (64, 128) and \
-                    kernels.takes_norm(hidden_states, residual, proj.packed, norm.weight.data):
-                qkv, residual = kernels.norm_gemm_rope_kv_store(
-                    hidden_states, residual, norm.weight.data, norm.eps, proj.packed, bias, positions,
-                    self.rotary_emb.cos_sin_cache, self.num_heads, self.num_kv_heads, self.head_dim, **rope)
-                return self._attend(qkv), residual
-            if residual is None:
-                hidden_states, residual = norm(hidden_states), hidden_states
-            else:
-                hidden_states, residual = norm(hidden_states, residual)
-            return self.forward(positions, hidden_states), residual
         rows = hidden_states.size(0)
         # Decode rows run inside a captured graph, where the library's estimate of GPU time decides.  A prefill step
         # is launched eagerly and is bound by the host up to about 2 k tokens (5.4 ms for 24 layers whatever the
@@ -130,15 +141,16 @@ class Qwen3MLP(nn.Module):
         assert hidden_act == "silu"
         self.act_fn = SiluAndMul()
 
-    def forward(self, x, norm=None, residual=None):
-        """``norm``: as in Qwen3Attention.forward."""
-        if norm is not None:
-            proj = self.gate_up_proj
-            if proj.packed is not None and proj.fused_silu and kernels.takes_norm(x, residual, proj.packed, norm.weight.data):
-                act, residual = kernels.norm_gemm_silu(x, residual, norm.weight.data, norm.eps, proj.packed)
-                return self.down_proj(act, partial_out=True), residual
-            x, residual = norm(x, residual)
-            return self.forward(x), residual
+    def with_norm(self, x, residual, norm: RMSNorm):
+        """As Qwen3Attention.with_norm."""
+        proj = self.gate_up_proj
+        if proj.packed is None or not (proj.fused_silu and plain(self, Qwen3MLP) and plain(norm, RMSNorm) and
+                                       kernels.takes_norm(x, residual, proj.packed, norm.weight.data)):
+            return None
+        act, residual = kernels.norm_gemm_silu(x, residual, norm.weight.data, norm.eps, proj.packed)
+        return self.down_proj(act, partial_out=True), residual
+
+    def forward(self, x):
         if self.gate_up_proj.fused_silu:
             act = self.gate_up_proj.forward_silu_mul(x)
         else:
@@ -165,9 +177,20 @@ class Qwen3DecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(config.hidden_size, eps=config.rms_norm_eps)
 
     def forward(self, positions, hidden_states, residual):
-        # each half takes its own norm: a few rows' is formed in the product that reads it (kernels.takes_norm)
-        hidden_states, residual = self.self_attn(positions, hidden_states, self.input_layernorm, residual)
-        return self.mlp(hidden_states, self.post_attention_layernorm, residual)
+        done = self.self_attn.with_norm(positions, hidden_states, residual, self.input_layernorm)
+        if done is not None:
+            hidden_states, residual = done
+        else:
+            if residual is None:
+                hidden_states, residual = self.input_layernorm(hidden_states), hidden_states
+            else:
+                hidden_states, residual = self.input_layernorm(hidden_states, residual)
+            hidden_states = self.self_attn(positions, hidden_states)
+        done = self.mlp.with_norm(hidden_states, residual, self.post_attention_layernorm)
+        if done is not None:
+            return done
+        hidden_states, residual = self.post_attention_layernorm(hidden_states, residual)
+        return self.mlp(hidden_states), residual
 
 
 class Qwen3Model(nn.Module):

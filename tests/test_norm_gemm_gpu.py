@@ -129,3 +129,81 @@ def test_refuses_operands_before_any_launch(monkeypatch):
     for rows, bias in ((x.cpu(), None), (x.half(), None), (x[:, :512], None), (x.t().contiguous().t(), None), (x, nw[:31]), (x, nw[:32].half())):
         with pytest.raises((RuntimeError, AssertionError)):
             kernels.gemm_stream(rows, w, bias)
+
+
+@pytest.fixture()
+def layer():
+    """A decoder layer with a KV cache, ready for a step of two tokens -> (the layer, its call)"""
+    from types import SimpleNamespace
+
+    from byox_vllm_amd.models.qwen3 import Qwen3DecoderLayer
+    from byox_vllm_amd.utils.context import reset_context, set_context
+    cfg = SimpleNamespace(hidden_size=256, num_attention_heads=4, num_key_value_heads=2, max_position_embeddings=64, rms_norm_eps=1e-6,
+                          attention_bias=False, head_dim=64, intermediate_size=512, hidden_act="silu")
+    torch.manual_seed(11)
+    torch.set_default_dtype(torch.bfloat16)
+    try:
+        with torch.device(DEV):
+            made = Qwen3DecoderLayer(cfg)
+    finally:
+        torch.set_default_dtype(torch.float32)
+    for name, p in made.named_parameters():
+        p.data.copy_(torch.rand_like(p) + 0.5 if "norm" in name else torch.randn_like(p) * 0.06)
+    made.mlp.gate_up_proj.finalize(None, fuse_silu=True)
+    cache = torch.zeros(2, 1, 16, 2, 64, dtype=torch.bfloat16, device=DEV)
+    made.self_attn.attn.k_cache, made.self_attn.attn.v_cache = cache[0], cache[1]
+    ints = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+
+    def call(first):
+        x = torch.randn(2, 256, generator=torch.Generator(device=DEV).manual_seed(2), device=DEV).bfloat16()
+        res = None if first else torch.randn(2, 256, generator=torch.Generator(device=DEV).manual_seed(3), device=DEV).bfloat16()
+        set_context(True, ints(0, 2), ints(0, 2), 2, 2, ints(0, 1))
+        try:
+            out, res = made(torch.arange(2, device=DEV), x, res)
+        finally:
+            reset_context()
+        if not torch.is_tensor(out):                  # split-K slabs, for the next layer's norm to sum
+            out = out.slabs.view(torch.float32)[:out.n * 512].view(out.n, 2, 256).sum(0).bfloat16()
+        return out, res
+    return made, call
+
+
+def count(monkeypatch, *names):
+    """How often each of the library's functions is launched from here on."""
+    from byox_vllm_amd import kernels
+    real, calls = kernels.lib(), dict.fromkeys(names, 0)
+
+    class Counting:
+        def __getattr__(self, name):
+            if name in calls:
+                calls[name] += 1
+            return getattr(real, name)
+    monkeypatch.setattr(kernels, "lib", Counting)
+    return calls
+
+
+@pytest.mark.parametrize("first", [True, False])
+@pytest.mark.parametrize("where", ["input_layernorm", "post_attention_layernorm", "self_attn", "mlp"])
+def test_hooks_on_a_layers_modules_are_called(layer, where, first, monkeypatch):
+    """A module with a hook is called as a module: its hook sees a tensor, or slabs, as from five rows on, and not a pair."""
+    made, call = layer
+    want = call(first)
+    calls = count(monkeypatch, "nv_norm_gemm_silu", "nv_norm_gemm_rope_kv_store")
+    call(first)
+    assert calls == dict(nv_norm_gemm_silu=1, nv_norm_gemm_rope_kv_store=1)
+    seen = []
+    handle = getattr(made, where).register_forward_hook(lambda m, args, out: seen.append(out))
+    got = call(first)
+    handle.remove()
+    assert len(seen) == 1 and calls["nv_norm_gemm_silu"] + calls["nv_norm_gemm_rope_kv_store"] == 3
+    assert isinstance(seen[0], tuple) == (where.endswith("norm") and not (first and where == "input_layernorm"))
+    for a, b, what in zip(got, want, ("result", "residual")):
+        close(a, b, torch.bfloat16, what)
+    every = []
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda m, args, out: every.append(m))
+    call(first)
+    handle.remove()
+    assert getattr(made, where) in every
+    getattr(made, where).forward = lambda *a, **k: type(getattr(made, where)).forward(getattr(made, where), *a, **k)
+    call(first)
+    assert calls["nv_norm_gemm_silu"] + calls["nv_norm_gemm_rope_kv_store"] == 4
