@@ -79,8 +79,9 @@ class Qwen3Attention(nn.Module):
         proj = self.qkv_proj
         if proj.packed is None:
             proj.finalize(None)
-        if not (self.fuse_qkv_rope and self.head_dim in (64, 128) and plain(self, Qwen3Attention) and plain(norm, RMSNorm) and
-                plain(proj, QKVParallelLinear) and kernels.takes_norm(hidden_states, residual, proj.packed, norm.weight.data)):
+        if not (self.fuse_qkv_rope and not self.force_fuse_qkv_rope and self.head_dim in (64, 128) and
+                plain(self, Qwen3Attention) and plain(norm, RMSNorm) and plain(proj, QKVParallelLinear) and
+                kernels.takes_norm(hidden_states, residual, proj.packed, norm.weight.data)):
             return None
         qkv, residual = kernels.norm_gemm_rope_kv_store(
             hidden_states, residual, norm.weight.data, norm.eps, proj.packed, None if proj.bias is None else proj.bias.data, positions,

@@ -207,3 +207,13 @@ def test_hooks_on_a_layers_modules_are_called(layer, where, first, monkeypatch):
     getattr(made, where).forward = lambda *a, **k: type(getattr(made, where)).forward(getattr(made, where), *a, **k)
     call(first)
     assert calls["nv_norm_gemm_silu"] + calls["nv_norm_gemm_rope_kv_store"] == 4
+
+
+@pytest.mark.parametrize("force", [False, True])
+def test_forced_rotation_behind_the_product(layer, force, monkeypatch):
+    """NV_FUSE_QKV_ROPE=2 (read when the layer is made) sends every row count to nv_gemm_rope_kv_store."""
+    made, call = layer
+    made.self_attn.force_fuse_qkv_rope = force
+    calls = count(monkeypatch, "nv_gemm_rope_kv_store", "nv_norm_gemm_rope_kv_store")
+    call(False)
+    assert calls == dict(nv_gemm_rope_kv_store=int(force), nv_norm_gemm_rope_kv_store=int(not force))
