@@ -602,23 +602,34 @@ def linear(x, w, bias=None, out=None, out_dtype=None, *, rows=None, a_rows=None,
     if n is None:
         n = w.size(-2) // (2 if epilogue == EPI_GLU else 1)
     M = x.size(0) if rows is None else rows
-    # prefill-sized plain products of a 16-bit model go where the engine sends its other many-row products: the vendor library, here
-    # with the result left in fp32.  Not those with an epilogue, which nv_linear forms on the way (16384 rows 2048 -> 2 x 6144, SiLU:
-    # 714 us, the library and a pass over its result 928; 4096 rows 1024 -> 4096 48 and 65), nor those of a short K whose columns do
-    # not split into the library's tiles, where the results fill 0.7 of nv_linear's rounds of 256 x 256 (12300 rows 1024 -> 3088, 0.75:
-    # 95 and 110; 5500 rows, 0.5: a layer 136 and 129; 12300 rows 2048 -> 4112: 325 and 290).
-    if (M >= MANY_ROWS and batch == 1 and group_offsets is None and a_rows is None and out is None and row_scale is None and rows is None
-            and x.dtype == torch.bfloat16 and (out_dtype or x.dtype) in (torch.float32, torch.bfloat16)
+    # prefill-sized products of a 16-bit model go where the engine sends its other many-row products: the vendor library, here with the
+    # result left in fp32, and with an epilogue a pass over that result.  nv_linear keeps, as far as one launch holds the rows,
+    #  * those with an epilogue that fill its rounds of 256 x 256 tiles (16384 rows 2048 -> 2 x 4096, SiLU, share 1.0: 489 us, the
+    #    library and a pass 588; 6000 rows 4096 -> 2 x 1024, 0.73: 107 and 92; 4100 rows 1024 -> 1024, 0.29: 42 and 26; of 650 shapes
+    #    above the line one is more than 3 % slower, by 3.1);
+    #  * plain ones of a short K whose columns do not split into the library's tiles (12300 rows 1024 -> 3088, share 0.79: 95 and 110;
+    #    5500 rows, 0.55: a layer 136 and 129; 12300 rows 2048 -> 4112: 325 and 290).
+    if (epilogue in (EPI_NONE, EPI_GLU, EPI_ACT) and M >= MANY_ROWS and batch == 1 and group_offsets is None and a_rows is None
+            and (bias is None or (epilogue != EPI_NONE and (out_dtype or x.dtype) == x.dtype)) and out is None
+            and row_scale is None and rows is None and x.dtype == torch.bfloat16
+            and (out_dtype or x.dtype) in (torch.float32, torch.bfloat16)
             and w.dim() == 2 and w.is_contiguous() and x.stride(0) % 8 == 0 and use_many_rows_path(M, K, n) and K % 8 == 0
             and n % 8 == 0 and x.data_ptr() % 16 == 0):
-        one_launch = M <= LINEAR_ROWS
-        if epilogue == EPI_NONE and bias is None and not (K <= 1024 and n > 1024 and n % 256 and one_launch and _fills_rounds(M, n)):
-            return _linear_many_rows(x, w, M, n, K, out_dtype or x.dtype)
-        if epilogue in (EPI_GLU, EPI_ACT) and not one_launch:
+        share = tile_share(M, 2 * n if epilogue == EPI_GLU else n) if M <= LINEAR_ROWS else 0.0
+        if epilogue == EPI_NONE:
+            if not (K <= 1024 and n > 1024 and n % 256 and share >= 0.7):
+                return _linear_many_rows(x, w, M, n, K, out_dtype or x.dtype)
+        elif share < (0.7 if K <= 512 else 0.8):
+            cols = 2 * n if epilogue == EPI_GLU else n
+            assert bias is None or (bias.dtype == x.dtype and bias.numel() == cols and bias.is_contiguous())
+            y = _linear_many_rows(x, w, M, cols, K, torch.float32)
             out = torch.empty(M, n, dtype=out_dtype or x.dtype, device=x.device)
-            for lo in range(0, M, LINEAR_ROWS):
-                linear(x[lo:lo + LINEAR_ROWS], w, bias, out[lo:lo + LINEAR_ROWS], out.dtype, epilogue=epilogue, act=act, gate=gate,
-                       cap=cap, n=n)
+            if epilogue == EPI_GLU:      # [gate | up] rows from the library, activation and product in one pass over them
+                check(lib().nv_bias_act_mul_f32(ptr(y), ptr(bias), ptr(out), M, n, act, cap, _code32(out.dtype), stream()),
+                      "nv_bias_act_mul_f32")
+            else:                        # the element-wise function in one pass over the library's fp32 result
+                check(lib().nv_bias_act_f32(ptr(y), ptr(bias), n, ptr(out), M * n, act, ptr(gate), cap, _code32(out.dtype),
+                                            stream()), "nv_bias_act_f32")
             return out
     grid_rows = M if group_offsets is None else (max_group_rows if max_group_rows is not None else M)
     out_dtype = out_dtype or x.dtype
@@ -647,9 +658,12 @@ def linear(x, w, bias=None, out=None, out_dtype=None, *, rows=None, a_rows=None,
     return out
 
 
-def _fills_rounds(M, n) -> bool:
-    """Whether M x n results take up 0.7 of the chip-wide rounds of 256 tiles of 256 x 256 that hold them."""
-    return M * n >= 0.7 * 65536 * 256 * -(-(-(-M // 256) * -(-n // 256)) // 256)
+def tile_share(M, n) -> float:
+    """Which part of the chip-wide rounds of 256 tiles of 256 x 256 M x n results take up.  A last round that half of the chip would have
+    is dealt in halves of tiles and costs 0.85 of one."""
+    tiles = -(-M // 256) * -(-n // 256)
+    over = tiles % 256
+    return M * n / (65536 * 256 * (tiles // 256 + (0.0 if over == 0 else 0.85 if over <= 128 else 1.0)))
 
 
 def _linear_many_rows(x, w, M, N, K, out_dtype):
