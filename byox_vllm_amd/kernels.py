@@ -398,16 +398,23 @@ def gemm_stream(x, w, bias=None, out=None, silu_mul=False):
 
 
 def gemm_many_rows(x, w, bias=None, out=None, silu_mul=False, rope=None):
-    """gemm() for prefill-sized x.  Gate/up weights, and products of a K below 1024, on this library's tiles (nv_gemm_stream); the
-    others as the weight written out row-major into scratch and one vendor-library product.  14.6 k rows, vendor route and
-    nv_gemm_stream: 1024 -> 2 x 3072 with SiluAndMul 208 and 169 us, 896 -> 2 x 4864 332 and 235; 896 -> 896 42 and 30;
-    2048 -> 1024 51 and 55, 3072 -> 1024 70 and 79.  ``rope``: arguments of gemm_stream_rope_kv_store, whose result this is then."""
+    """gemm() for prefill-sized x: the weight written out row-major into scratch and one vendor-library product, with a SiluAndMul pass
+    over its result for gate/up weights; or, where that is not slower, this library's tiles (nv_gemm_stream).  Those have
+     * gate/up weights of a K below 4096, or below 2048 where the weight has to be expanded, without a bias (16384 rows, both routes:
+       1024 -> 2 x 3072 217 and 197 us, int4 216 and 204; 2048 -> 2 x 6144 690 and 706, 6000 rows 351 and 271; 4096 rows 4096 -> 2 x
+       12288 645 and 651, int4 653 and 723);
+     * products of a K below 1024: 14.6 k rows 896 -> 896 42 and 30; 2048 -> 1024 51 and 55, 3072 -> 1024 70 and 79.
+    ``rope``: arguments of gemm_stream_rope_kv_store, whose result this is then."""
     M, K = x.shape
     N = w.out_features
     dev = x.device
     if rope is not None:
         return gemm_stream_rope_kv_store(x, w, bias, **rope)
-    if streams(x, w, bias, out) and _streams_into(out, x, N // 2 if silu_mul else N) and (bias is None if silu_mul else 512 <= K < 1024):
+    if silu_mul:
+        own = bias is None and K < (4096 if w.fmt == _C.W_DENSE_TILED else 2048)
+    else:
+        own = 512 <= K < 1024
+    if own and streams(x, w, bias, out) and _streams_into(out, x, N // 2 if silu_mul else N):
         return gemm_stream(x, w, bias, out, silu_mul)
     if w.fmt == _C.W_DENSE and not silu_mul:
         wr = w.data
@@ -462,9 +469,11 @@ def gemm(x, w, bias=None, out=None, split_k=None, silu_mul=False, partial_out=Fa
     if split_k is None:
         if use_many_rows_path(M, K, N) and (out is None or out.is_contiguous() or not silu_mul):
             return gemm_many_rows(x, w, bias, out, silu_mul)
-        # gate/up from half as many rows on where the weight is read as it lies (2048 rows, nv_gemm and the streamed tiles:
-        # 1024 -> 2 x 3072 37 and 33 us, 896 -> 2 x 4864 61 and 46; 1024 rows: 23 and 30)
-        if silu_mul and bias is None and M >= MANY_ROWS // 2 and w.fmt in (_C.W_DENSE, _C.W_DENSE_TILED) and \
+        # gate/up from half as many rows on where the tiled weight is read as it lies and there are tiles for five CUs in eight (2048
+        # rows, nv_gemm and the streamed tiles: 896 -> 2 x 4864 60 and 50 us, 2048 -> 2 x 6144 118 and 99; 3000 rows 512 -> 2 x 1408, 132
+        # tiles: 23 and 24, 2048 rows 256 -> 2 x 512, 32 tiles: 5 and 12; 1024 rows 1024 -> 2 x 3072: 23 and 30)
+        if silu_mul and bias is None and M >= MANY_ROWS // 2 and w.fmt == _C.W_DENSE_TILED and \
+                -(-M // 256) * -(-N // 256) >= 160 and \
                 use_many_rows_path(max(M, MANY_ROWS), K, N) and streams(x, w, out) and _streams_into(out, x, N // 2):
             return gemm_stream(x, w, None, out, True)
         split_k = 1 if silu_mul else pick_split_k(M, N, K, w.fmt)

@@ -55,3 +55,27 @@ def test_linear_of_many_rows(M, K, n, epilogue, want, out_dtype, launched):
     elif epilogue == "ACT":
         y = torch.nn.functional.silu(y)
     close(got, y, K, out_dtype)
+
+
+OWN, OTHER, LT = ["nv_gemm_stream"], ["nv_gemm"], ["nv_weight_expand", "nv_gemm_lt", "nv_silu_mul"]
+
+
+@pytest.mark.parametrize("M,K,inter,fmt,want", [
+    (2047, 512, 5120, None, OTHER), (2048, 512, 5120, None, OWN), (2048, 512, 2432, None, OTHER), (2048, 512, 2560, None, OWN),
+    (2048, 512, 5120, "w4a16", OTHER), (4095, 256, 512, None, OTHER), (4096, 256, 512, None, OWN), (4096, 256, 512, "w8a16", ["nv_weight_expand"] + OWN),
+    (4096, 3968, 256, None, OWN), (4096, 4096, 256, None, LT), (4096, 1920, 256, "w4a16", ["nv_weight_expand"] + OWN),
+    (4096, 2048, 256, "w4a16", LT)])
+def test_gate_up_of_many_rows(M, K, inter, fmt, want, launched):
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.layers.quant import LinearWeight, interleave_gate_up
+    torch.manual_seed(M + K)
+    dt = torch.bfloat16
+    x = torch.randn(M, K, device=DEV).to(dt)
+    lw = LinearWeight.make(interleave_gate_up((torch.randn(2 * inter, K, device=DEV) * K ** -0.5).to(dt)), fmt)
+    got = kernels.gemm(x, lw, silu_mul=True)
+    assert launched == want
+    gate, up = (x.double() @ kernels.expand_weight(lw, gate_up_rows=True).double().t()).to(dt).double().chunk(2, -1)
+    # the product, SiLU's and the last number rounded to 16 bits; a gate on the other side of a rounding moves two more
+    want = torch.nn.functional.silu(gate).to(dt).double() * up
+    off = (got.double() - want).abs() - 3.0 * torch.finfo(dt).eps * want.abs()
+    assert torch.isfinite(got).all() and (off <= 8.0 * K ** 0.5 * 2.0 ** -24).all()
