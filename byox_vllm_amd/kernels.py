@@ -403,7 +403,9 @@ def gemm_many_rows(x, w, bias=None, out=None, silu_mul=False, rope=None):
      * gate/up weights of a K below 4096, or below 2048 where the weight has to be expanded, without a bias (16384 rows, both routes:
        1024 -> 2 x 3072 217 and 197 us, int4 216 and 204; 2048 -> 2 x 6144 690 and 706, 6000 rows 351 and 271; 4096 rows 4096 -> 2 x
        12288 645 and 651, int4 653 and 723);
-     * products of a K below 1024: 14.6 k rows 896 -> 896 42 and 30; 2048 -> 1024 51 and 55, 3072 -> 1024 70 and 79.
+     * products of 512 <= K < 1024 without a bias whose columns do not split into tiles and whose results fill 0.6 of their rounds, 0.8
+       where the weight has to be expanded (tile_share; 16384 rows 896 -> 896, share 0.88: 43 and 30 us, int4 43 and 33; 11000 rows
+       896 -> 640, 0.42: 21 and 27; whole tiles: 16384 rows 896 -> 8192 198 and 223, 2048 -> 1024 51 and 55).
     ``rope``: arguments of gemm_stream_rope_kv_store, whose result this is then."""
     M, K = x.shape
     N = w.out_features
@@ -413,7 +415,7 @@ def gemm_many_rows(x, w, bias=None, out=None, silu_mul=False, rope=None):
     if silu_mul:
         own = bias is None and K < (4096 if w.fmt == _C.W_DENSE_TILED else 2048)
     else:
-        own = 512 <= K < 1024
+        own = bias is None and 512 <= K < 1024 and N % 256 != 0 and tile_share(M, N) >= (0.6 if w.fmt == _C.W_DENSE_TILED else 0.8)
     if own and streams(x, w, bias, out) and _streams_into(out, x, N // 2 if silu_mul else N):
         return gemm_stream(x, w, bias, out, silu_mul)
     if w.fmt == _C.W_DENSE and not silu_mul:

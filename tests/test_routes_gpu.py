@@ -79,3 +79,22 @@ def test_gate_up_of_many_rows(M, K, inter, fmt, want, launched):
     want = torch.nn.functional.silu(gate).to(dt).double() * up
     off = (got.double() - want).abs() - 3.0 * torch.finfo(dt).eps * want.abs()
     assert torch.isfinite(got).all() and (off <= 8.0 * K ** 0.5 * 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("M,K,N,fmt,bias,want", [
+    (16384, 896, 896, None, False, OWN), (16384, 896, 896, "w4a16", False, ["nv_weight_expand"] + OWN),
+    (16384, 896, 896, None, True, ["nv_weight_expand", "nv_gemm_lt"]), (11000, 896, 640, None, False, ["nv_weight_expand", "nv_gemm_lt"]),
+    (14600, 896, 896, None, False, OWN), (14600, 896, 896, "w8a16", False, ["nv_weight_expand", "nv_gemm_lt"]),
+    (16384, 896, 1024, None, False, ["nv_weight_expand", "nv_gemm_lt"]), (16384, 384, 896, None, False, ["nv_weight_expand", "nv_gemm_lt"]),
+    (16384, 1024, 896, None, False, ["nv_weight_expand", "nv_gemm_lt"])])
+def test_products_of_many_rows(M, K, N, fmt, bias, want, launched):
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.layers.quant import LinearWeight
+    torch.manual_seed(M + K)
+    dt = torch.bfloat16
+    x = torch.randn(M, K, device=DEV).to(dt)
+    lw = LinearWeight.make((torch.randn(N, K, device=DEV) * 0.05).to(dt), fmt)
+    b = torch.randn(N, device=DEV).to(dt) if bias else None
+    got = kernels.gemm(x, lw, b)
+    assert launched == want
+    close(got, x.double() @ kernels.expand_weight(lw).double().t() + (b.double() if bias else 0.0), K, dt)
