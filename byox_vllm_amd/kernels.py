@@ -350,6 +350,18 @@ def streams(x, w, *others):
         all(t is None or t.data_ptr() % 16 == 0 for t in (x, w.data) + others)
 
 
+def rotation_streams(M, w) -> bool:
+    """Whether gemm_stream_rope_kv_store is not slower than the library's product and rope_kv_store for M prefill rows: the results fill
+    their rounds of tiles (tile_share), by less where their width does not split into the library's; K up to 2048, 1024 where the weight
+    has to be expanded.  Both routes, us: 16384 rows 1024 -> 4096, share 1.0: 183 and 155; 14600 rows 896 -> 1152, 0.54: 69 and 62; 5000
+    rows, 0.40: 27 and 37; 4100 rows 2048 -> 4096, 0.54: 93 and 102; int4, 11000 rows 1024 -> 4096, 0.90: 140 and 123, 16384 rows
+    2048 -> 4096, 1.0: 249 and 255."""
+    N, odd = w.out_features, w.out_features % 256 != 0
+    if w.fmt == _C.W_DENSE_TILED:
+        return w.in_features <= 2048 and tile_share(M, N) >= (0.5 if odd else 0.75)
+    return w.in_features <= 1024 and tile_share(M, N) >= (0.6 if odd else 0.8)
+
+
 def _streams_into(out, x, cols):
     """Whether nv_gemm_stream may write its rows to ``out`` (or allocate them: None)."""
     return out is None or (out.shape == (x.size(0), cols) and out.dtype == x.dtype and out.stride(1) == 1
@@ -397,7 +409,7 @@ def gemm_stream(x, w, bias=None, out=None, silu_mul=False):
     return out
 
 
-def gemm_many_rows(x, w, bias=None, out=None, silu_mul=False, rope=None):
+def gemm_many_rows(x, w, bias=None, out=None, silu_mul=False):
     """gemm() for prefill-sized x: the weight written out row-major into scratch and one vendor-library product, with a SiluAndMul pass
     over its result for gate/up weights; or, where that is not slower, this library's tiles (nv_gemm_stream).  Those have
      * gate/up weights of a K below 4096, or below 2048 where the weight has to be expanded, without a bias (16384 rows, both routes:
@@ -405,13 +417,10 @@ def gemm_many_rows(x, w, bias=None, out=None, silu_mul=False, rope=None):
        12288 645 and 651, int4 653 and 723);
      * products of 512 <= K < 1024 without a bias whose columns do not split into tiles and whose results fill 0.6 of their rounds, 0.8
        where the weight has to be expanded (tile_share; 16384 rows 896 -> 896, share 0.88: 43 and 30 us, int4 43 and 33; 11000 rows
-       896 -> 640, 0.42: 21 and 27; whole tiles: 16384 rows 896 -> 8192 198 and 223, 2048 -> 1024 51 and 55).
-    ``rope``: arguments of gemm_stream_rope_kv_store, whose result this is then."""
+       896 -> 640, 0.42: 21 and 27; whole tiles: 16384 rows 896 -> 8192 198 and 223, 2048 -> 1024 51 and 55)."""
     M, K = x.shape
     N = w.out_features
     dev = x.device
-    if rope is not None:
-        return gemm_stream_rope_kv_store(x, w, bias, **rope)
     if silu_mul:
         own = bias is None and K < (4096 if w.fmt == _C.W_DENSE_TILED else 2048)
     else:

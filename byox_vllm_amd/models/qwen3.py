@@ -104,14 +104,12 @@ class Qwen3Attention(nn.Module):
             self.force_fuse_qkv_rope or (context.is_prefill and 16 <= rows <= 4096 and not many_rows) or
             kernels.lib().nv_gemm_rope_kv_store_is_faster(rows, proj.packed.in_features, proj.packed.fmt,
                                                           self.num_heads, self.num_kv_heads, self.head_dim))
-        # From prefill sizes on, the streamed tiles do the same where a product is short: 14.6 k rows, vendor product + RoPE pass
-        # and one launch: K 1024 165 and 148 us, K 896 70 and 61; 8 k rows of K 3584: 246 and 264.
-        if many_rows and not fused and self.fuse_qkv_rope and proj.packed.in_features <= 2048 and self.head_dim in (64, 128) and \
+        if many_rows and not fused and self.fuse_qkv_rope and self.head_dim in (64, 128) and \
+                kernels.rotation_streams(rows, proj.packed) and \
                 kernels.streams(hidden_states, proj.packed, bias, self.rotary_emb.cos_sin_cache, rope["k_cache"], rope["v_cache"],
                                 rope["q_norm_w"], rope["k_norm_w"]):
-            qkv = kernels.gemm_many_rows(hidden_states, proj.packed, bias, rope=dict(
-                positions=positions, cos_sin=self.rotary_emb.cos_sin_cache, num_heads=self.num_heads,
-                num_kv_heads=self.num_kv_heads, head_dim=self.head_dim, **rope))
+            qkv = kernels.gemm_stream_rope_kv_store(hidden_states, proj.packed, bias, positions, self.rotary_emb.cos_sin_cache,
+                                                    self.num_heads, self.num_kv_heads, self.head_dim, **rope)
         elif fused:
             # projection, bias, head norms, RoPE and the KV-cache store in one launch (one workgroup per head)
             qkv = kernels.gemm_rope_kv_store(hidden_states, proj.packed, bias, positions, self.rotary_emb.cos_sin_cache,

@@ -770,6 +770,7 @@ def test_gemm_many_rows_through_the_vendor_library(name, M, N, K, fmt, monkeypat
 @pytest.mark.parametrize("M", [640, 2100])
 @pytest.mark.parametrize("vendor", [True, False])
 def test_gemm_many_rows_silu_mul(M, vendor, monkeypatch):
+    """Beside the vendor's products (from MANY_ROWS rows on the streamed tiles have gate/up of this K), and without them."""
     from byox_vllm_amd import kernels
     monkeypatch.setattr(kernels, "MANY_ROWS", 2048 if vendor else 0)
     from byox_vllm_amd.layers.quant import LinearWeight, interleave_gate_up

@@ -667,7 +667,7 @@ def test_generate_with_steps_launched_ahead_equals_generate_on_demand(golden, mo
 @pytest.mark.parametrize("quant,bits", [(None, 0), ("w8a16", 8), ("w4a16", 4)])
 def test_prefill_of_many_rows_through_the_vendor_library_vs_oracle(golden, quant, bits, monkeypatch):
     """A prefill step of 4 500 tokens: every linear of the step goes through kernels.gemm_many_rows (weight written out
-    row-major, hipBLASLt product, SiluAndMul pass for gate/up), the q/k/v projection as an unfused launch.  Last-token
+    row-major and a hipBLASLt product; gate/up on the streamed tiles), the q/k/v projection as an unfused launch.  Last-token
     logits against the oracle (dequantised dense weights), and against the same step with the path switched off."""
     from byox_vllm_amd import kernels
     g, key, weights = _golden_weights(golden, "qwen2")

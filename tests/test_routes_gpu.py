@@ -98,3 +98,59 @@ def test_products_of_many_rows(M, K, N, fmt, bias, want, launched):
     got = kernels.gemm(x, lw, b)
     assert launched == want
     close(got, x.double() @ kernels.expand_weight(lw).double().t() + (b.double() if bias else 0.0), K, dt)
+
+
+def attention(K, H, Hkv, D, fmt, norms):
+    from byox_vllm_amd.models.qwen3 import Qwen3Attention
+    torch.set_default_dtype(torch.bfloat16)
+    try:
+        with torch.device(DEV):
+            made = Qwen3Attention(K, H, Hkv, max_position=32768, head_dim=D, qkv_bias=not norms)
+    finally:
+        torch.set_default_dtype(torch.float32)
+    for name, p in made.named_parameters():
+        p.data.copy_(torch.rand_like(p) + 0.5 if "norm" in name else torch.randn_like(p) * 0.05)
+    made.qkv_proj.finalize(fmt)
+    return made
+
+
+@pytest.mark.parametrize("M,K,H,Hkv,D,fmt,own", [
+    (8192, 1024, 16, 8, 128, None, True), (4100, 1024, 16, 8, 128, None, False), (8192, 1024, 16, 8, 128, "w4a16", True),
+    (14600, 896, 14, 2, 64, None, True), (14600, 896, 14, 2, 64, "w4a16", False), (5000, 896, 14, 2, 64, None, False),
+    (11000, 896, 14, 2, 64, "w8a16", True), (8192, 2048, 16, 8, 128, None, True), (8192, 2048, 16, 8, 128, "w4a16", False),
+    (8192, 2176, 8, 4, 128, None, False)])
+def test_rotation_behind_the_product(M, K, H, Hkv, D, fmt, own, launched, monkeypatch):
+    """q/k/v of many rows: one launch or two by the share of its rounds; rotated rows and the cache against float64."""
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.utils.context import reset_context, set_context
+    torch.manual_seed(M + K)
+    dt = torch.bfloat16
+    made = attention(K, H, Hkv, D, fmt, norms=D == 128)
+    x = torch.randn(M, K, device=DEV).to(dt)
+    cache = torch.zeros(2, -(-M // 16), 16, Hkv, D, dtype=dt, device=DEV)
+    made.attn.k_cache, made.attn.v_cache = cache[0], cache[1]
+    pos, slots = torch.arange(M, device=DEV), torch.arange(M, device=DEV, dtype=torch.int32)
+    monkeypatch.setattr(made, "_attend", lambda qkv: qkv)
+    set_context(True, slot_mapping=slots)
+    try:
+        got = made(pos, x)
+    finally:
+        reset_context()
+    assert ("nv_gemm_stream_rope_kv_store" in launched) == own and ("nv_rope_kv_store" in launched) != own
+    y = x.double() @ kernels.expand_weight(made.qkv_proj.packed).double().t()
+    if made.qkv_proj.bias is not None:
+        y += made.qkv_proj.bias.data.double()
+    y = y.view(M, H + 2 * Hkv, D)
+    turned = y[:, :H + Hkv]
+    if D == 128:
+        turned = turned * torch.rsqrt((turned * turned).mean(-1, keepdim=True) + 1e-6)
+        turned = torch.cat([turned[:, :H] * made.q_norm.weight.data.double(), turned[:, H:] * made.k_norm.weight.data.double()], 1)
+    cos, sin = made.rotary_emb.cos_sin_cache[:M].view(M, 1, D).double().chunk(2, -1)
+    a, b = turned.chunk(2, -1)
+    want = torch.cat([torch.cat([a * cos - b * sin, b * cos + a * sin], -1), y[:, H + Hkv:]], 1)
+    # roundings to eight bits, each up to 2^-8: the product's, with head norms two more ahead of the turn, and the last.  A turn adds two
+    # numbers' errors: of a head's largest number, where the turned ones cancel.
+    size = torch.maximum(want.abs(), torch.cat([turned, y[:, H + Hkv:]], 1).abs().amax(-1, keepdim=True))
+    assert ((got.view(M, -1, D).double() - want).abs() <= 2.0 ** -8 * (1 + 2 ** 0.5 * (3 if D == 128 else 1)) * size + 1e-4).all()
+    kv = got.view(M, -1, D)[:, H:].reshape(M, 2, Hkv, D)
+    assert torch.equal(cache.view(2, -1, Hkv, D)[:, :M], kv.transpose(0, 1))
