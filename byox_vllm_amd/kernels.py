@@ -160,9 +160,23 @@ def gemm_rope_kv_store(x, w, bias, positions, cos_sin, num_heads, num_kv_heads, 
     return out
 
 
-# Rows up to which a norm is formed in the product that reads it.  A decode step of 24 layers, norms apart and in the product, us:
-# Qwen2-0.5B 1 row 951 and 858, 4 rows 976 and 929, 6 rows 985 and 1021; Qwen3-0.6B 1037 and 923, 1054 and 992, 1071 and 1086.
+# Rows up to which a norm is formed in the product that reads it
 NORM_GEMM_ROWS = 4
+
+
+def norm_gemm_pays(x, w, head_dim=None) -> bool:
+    """Whether the norm of these rows inside the product of ``w`` (with rotation: ``head_dim``) is not slower than in a launch of its own.
+    A workgroup norms the rows it has wavefronts for at once, 8 / ceil(K / 256), and each further pass costs it about 1.5 us; heads of 128
+    have one wavefront per 16 columns and its whole K, and with many columns several workgroups per CU repeat the norm.  Both ways in a
+    captured graph, a split-K product ahead of each, us: gate/up, 1024 -> 2 x 3072 2 rows (one pass) 10.9 and 8.4, 4 rows (two) 10.8 and
+    10.0; 896 -> 2 x 4864 4 rows 11.2 and 11.7; 1536 -> 2 x 8960 2 rows (two) 19.9 and 22.2, 4 rows (four) 19.9 and 28.6; 256 -> 2 x 8960
+    1 row 8.7 and 9.6.  q/k/v, heads of 64, 896 -> 1152 4 rows (two) 10.7 and 10.1, 2048 -> 3072 1 row 12.8 and 11.3; heads of 128, 1024
+    -> 4096 1 row 12.2 and 11.1, 4 rows (two) 12.1 and 12.8, 2048 -> 4096 1 row 13.6 and 14.3."""
+    rows, K = x.rows if isinstance(x, Partials) else x.size(0), w.in_features
+    passes = -(-rows // (8 // -(-K // 256)))
+    if head_dim is not None:
+        return passes == 1 and (K <= 1024 or head_dim == 64) or passes == 2 and K <= 1024 and head_dim == 64
+    return passes == 1 and K >= 512 or passes <= 3 and w.out_features <= 8192
 
 
 def takes_norm(x, residual, w, norm_w) -> bool:

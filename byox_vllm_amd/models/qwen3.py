@@ -81,7 +81,8 @@ class Qwen3Attention(nn.Module):
             proj.finalize(None)
         if not (self.fuse_qkv_rope and not self.force_fuse_qkv_rope and self.head_dim in (64, 128) and
                 plain(self, Qwen3Attention) and plain(norm, RMSNorm) and plain(proj, QKVParallelLinear) and
-                kernels.takes_norm(hidden_states, residual, proj.packed, norm.weight.data)):
+                kernels.takes_norm(hidden_states, residual, proj.packed, norm.weight.data) and
+                kernels.norm_gemm_pays(hidden_states, proj.packed, self.head_dim)):
             return None
         qkv, residual = kernels.norm_gemm_rope_kv_store(
             hidden_states, residual, norm.weight.data, norm.eps, proj.packed, None if proj.bias is None else proj.bias.data, positions,
@@ -144,7 +145,8 @@ class Qwen3MLP(nn.Module):
         """As Qwen3Attention.with_norm."""
         proj = self.gate_up_proj
         if proj.packed is None or not (proj.fused_silu and plain(self, Qwen3MLP) and plain(norm, RMSNorm) and
-                                       kernels.takes_norm(x, residual, proj.packed, norm.weight.data)):
+                                       kernels.takes_norm(x, residual, proj.packed, norm.weight.data) and
+                                       kernels.norm_gemm_pays(x, proj.packed)):
             return None
         act, residual = kernels.norm_gemm_silu(x, residual, norm.weight.data, norm.eps, proj.packed)
         return self.down_proj(act, partial_out=True), residual

@@ -154,3 +154,45 @@ def test_rotation_behind_the_product(M, K, H, Hkv, D, fmt, own, launched, monkey
     assert ((got.view(M, -1, D).double() - want).abs() <= 2.0 ** -8 * (1 + 2 ** 0.5 * (3 if D == 128 else 1)) * size + 1e-4).all()
     kv = got.view(M, -1, D)[:, H:].reshape(M, 2, Hkv, D)
     assert torch.equal(cache.view(2, -1, Hkv, D)[:, :M], kv.transpose(0, 1))
+
+
+def decoder_layer(K, H, Hkv, D, inter):
+    from types import SimpleNamespace
+
+    from byox_vllm_amd.models.qwen3 import Qwen3DecoderLayer
+    cfg = SimpleNamespace(hidden_size=K, num_attention_heads=H, num_key_value_heads=Hkv, max_position_embeddings=64, rms_norm_eps=1e-6,
+                          attention_bias=D == 64, head_dim=D, intermediate_size=inter, hidden_act="silu")
+    torch.set_default_dtype(torch.bfloat16)
+    try:
+        with torch.device(DEV):
+            made = Qwen3DecoderLayer(cfg)
+    finally:
+        torch.set_default_dtype(torch.float32)
+    for name, p in made.named_parameters():
+        p.data.copy_(torch.rand_like(p) + 0.5 if "norm" in name else torch.randn_like(p) * 0.02)
+    made.mlp.gate_up_proj.finalize(None, fuse_silu=True)
+    return made
+
+
+@pytest.mark.parametrize("rows,K,H,Hkv,D,inter,attn,mlp", [
+    (1, 896, 14, 2, 64, 4864, True, True), (2, 896, 14, 2, 64, 4864, True, True), (4, 896, 14, 2, 64, 4864, True, False),
+    (5, 896, 14, 2, 64, 1024, False, False), (2, 1024, 16, 8, 128, 3072, True, True), (3, 1024, 16, 8, 128, 3072, False, True),
+    (1, 1536, 12, 2, 128, 8960, False, True), (2, 1536, 12, 2, 128, 8960, False, False), (1, 2048, 32, 8, 64, 6144, True, True),
+    (3, 2048, 32, 8, 64, 3072, False, True), (4, 2048, 32, 8, 64, 3072, False, False), (1, 256, 4, 2, 64, 8960, True, False),
+    (4, 512, 8, 2, 64, 1024, True, True), (1, 2176, 4, 2, 128, 1024, False, False)])
+def test_norms_of_a_few_rows(rows, K, H, Hkv, D, inter, attn, mlp, launched):
+    """A decoder layer's two norms, each inside the product behind it or in a launch of its own."""
+    from byox_vllm_amd.utils.context import reset_context, set_context
+    torch.manual_seed(K + rows)
+    made = decoder_layer(K, H, Hkv, D, inter)
+    cache = torch.zeros(2, 1, 16, Hkv, D, dtype=torch.bfloat16, device=DEV)
+    made.self_attn.attn.k_cache, made.self_attn.attn.v_cache = cache[0], cache[1]
+    ints = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    x, res = (torch.randn(rows, K, device=DEV).bfloat16() for _ in range(2))
+    set_context(True, ints(0, rows), ints(0, rows), rows, rows, ints(*range(rows)))
+    try:
+        made(torch.arange(rows, device=DEV), x, res)
+    finally:
+        reset_context()
+    assert ("nv_norm_gemm_rope_kv_store" in launched, "nv_norm_gemm_silu" in launched) == (attn, mlp), launched
+    assert sum(n.startswith("nv_add_rmsnorm") for n in launched) == 2 - attn - mlp
