@@ -255,24 +255,33 @@ hipError_t launch_wide_one(const LinArgs& p, int64_t total_rows, int batch, hipS
 // 608 in the others, of which two share one).  A last round of 256 x 256 that half of the chip would have is dealt in halves and
 // costs 0.85 of a round (12000 rows by 2048, K 1024, 1.5 rounds: 65 us, 128 x 128 93, 64 x 128 88; 4096 by 2048, half a round:
 // 29.4, 29.3, 33; 5000 by 1536, K 1536: 38, 34, 43).
-// fp32 is bound by its matrix instructions alone: a workgroup that has a CU to itself is twice as fast as one of two, so rounds count
-// tiles per CU, and half a tile costs little more than half (reached when full 135, 130 and 121; 256, 128 and 64 rows: 3135 by 4416,
-// K 1024 256, 271 and 265 us; 4096 by 4416 383, 340, 343; 2000 by 2208, K 512 73, 73, 60; 2500 by 6144 256, 267, 281).
+// fp32 is bound by its matrix instructions alone: a workgroup that has a CU to itself is twice as fast as one of two.  So, from K 256 on
+// (us of 256 x 256, 128 x 128 and 64 x 128; a tile's beginning and end weigh more below):
+//   * 256 x 256 where the results fill 0.9 of its rounds, a halved last one as 0.55 (2500 by 6144, K 1024, share 0.91: 256, 266, 281;
+//     8000 by 2048, K 512, 0.98: 137, 149, 150; 4000 by 4096 gated, K 512, 0.68 - 0.88: up to 15 % slower than 128 x 128);
+//   * 64 x 128 where they take fewer rounds per CU than two for each of 128 x 128 (2500 by 2048, K 1024, 3 and 2 x 2: 134, 135, 111;
+//     3135 by 4416, 7 and 2 x 4: 255, 265, 247);
+//   * else as in 16 bits.  Of 1430 shapes none is over 3 % slower than with the last rule alone.
 enum { TILE_256 = 2, TILE_128 = 1, TILE_64 = 0 };
 inline int64_t wide_tiles(int bm, int bn, int64_t m, int64_t total_rows, int cols, int batch, bool grouped) {
   // groups end inside a tile: half a tile each on average
   return (grouped ? (total_rows + bm - 1) / bm + batch / 2 : (m + bm - 1) / bm * batch) * ((cols + bn - 1) / bn);
 }
-inline int pick_wide_tile(int64_t m, int64_t total_rows, int cols, int batch, bool grouped, bool fp32, bool has_256) {
-  auto cost = [&](int bm, int bn, int per_cu, double reached, double half) {
-    const int64_t slots = 256 * per_cu, tiles = wide_tiles(bm, bn, m, total_rows, cols, batch, grouped), over = tiles % slots;
-    const double last = over == 0 ? 0.0 : bm == 256 && 2 * over <= slots ? half : 1.0;
-    return ((double)(tiles / slots) + last) * per_cu * bm * bn / reached;
+inline int pick_wide_tile(int64_t m, int64_t total_rows, int cols, int K, int batch, bool grouped, bool fp32, bool has_256) {
+  auto tiles = [&](int bm, int bn) { return wide_tiles(bm, bn, m, total_rows, cols, batch, grouped); };
+  auto rounds = [&](int bm, int bn, int64_t slots, double half) {
+    const int64_t n = tiles(bm, bn), over = n % slots;
+    return (double)(n / slots) + (over == 0 ? 0.0 : bm == 256 && 2 * over <= slots ? half : 1.0);
   };
-  const int pair = fp32 ? 1 : 2;
-  const double c64 = cost(64, 128, pair, fp32 ? 121 : 608, 1.0), c128 = cost(128, 128, pair, fp32 ? 130 : 742, 1.0);
-  const double c256 = cost(256, 256, 1, fp32 ? 135 : 1150, fp32 ? 0.55 : 0.85);
-  if (has_256 && c256 < c128 && c256 < c64) return TILE_256;
+  const double c64 = rounds(64, 128, 512, 1.0) * 2 * 64 * 128 / 608, c128 = rounds(128, 128, 512, 1.0) * 2 * 128 * 128 / 742;
+  if (fp32) {
+    const double results = (double)(grouped ? total_rows : m * batch) * cols;
+    if (has_256 && K >= 256 && results >= 0.9 * 65536 * 256 * rounds(256, 256, 256, 0.55)) return TILE_256;
+    if (K >= 256 && rounds(64, 128, 256, 1.0) < 2 * rounds(128, 128, 256, 1.0)) return TILE_64;
+  } else {
+    const double c256 = rounds(256, 256, 256, 0.85) * 256 * 256 / 1150;
+    if (has_256 && c256 < c128 && c256 < c64) return TILE_256;
+  }
   return c128 < c64 ? TILE_128 : TILE_64;
 }
 

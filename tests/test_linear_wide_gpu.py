@@ -107,6 +107,22 @@ def test_streams_of_fp32_tiles(M, N, K, monkeypatch):
             close(got[lo:lo + 8192], x[lo:lo + 8192].double() @ w.double().t() + b.double(), K, torch.float32, out_dtype)
 
 
+@pytest.mark.parametrize("M,N,K", [(2500, 6144, 256), (2500, 6144, 224), (2500, 2048, 256), (2500, 2048, 224), (8000, 2048, 256),
+                                   (4000, 4096, 256), (1500, 2048, 512), (16384, 64, 256)])
+@pytest.mark.parametrize("glu", [False, True])
+def test_fp32_on_both_sides_of_each_line(M, N, K, glu):
+    """Sizes where fp32 products take 256 x 256, 64 x 128 and 128 x 128 tiles, and just below the K from which they do."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(M + N)
+    x, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV) * 0.1
+    got = kernels.linear(x, w, epilogue=kernels.EPI_GLU if glu else kernels.EPI_NONE)
+    want = x.double() @ w.double().t()
+    if glu:
+        gate, up = want.chunk(2, -1)
+        want = torch.nn.functional.silu(gate) * up
+    close(got, want, 2 * K, torch.float32, torch.float32)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_batches_and_gates(dtype):
     """One product per head side by side, with the row gate, the soft cap and the element-wise epilogues."""
