@@ -649,12 +649,11 @@ def linear(x, w, bias=None, out=None, out_dtype=None, *, rows=None, a_rows=None,
             and (out_dtype or x.dtype) in (torch.float32, torch.bfloat16)
             and w.dim() == 2 and w.is_contiguous() and x.stride(0) % 8 == 0 and use_many_rows_path(M, K, n) and K % 8 == 0
             and n % 8 == 0 and x.data_ptr() % 16 == 0):
-        share = tile_share(M, 2 * n if epilogue == EPI_GLU else n) if M <= LINEAR_ROWS else 0.0
+        cols = 2 * n if epilogue == EPI_GLU else n
         if epilogue == EPI_NONE:
-            if not (K <= 1024 and n > 1024 and n % 256 and share >= 0.7):
+            if not (K <= 1024 and n > 1024 and n % 256 and M <= LINEAR_ROWS and tile_share(M, n) >= 0.7):
                 return _linear_many_rows(x, w, M, n, K, out_dtype or x.dtype)
-        elif share < (0.7 if K <= 512 else 0.8):
-            cols = 2 * n if epilogue == EPI_GLU else n
+        elif M > LINEAR_ROWS or tile_share(M, cols) < (0.7 if K <= 512 else 0.8):
             assert bias is None or (bias.dtype == x.dtype and bias.numel() == cols and bias.is_contiguous())
             y = _linear_many_rows(x, w, M, cols, K, torch.float32)
             out = torch.empty(M, n, dtype=out_dtype or x.dtype, device=x.device)
