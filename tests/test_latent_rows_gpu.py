@@ -70,3 +70,24 @@ def test_norms_of_both_latents(dtype, rank, rot, q_rank):
     empty = torch.ones(16, dtype=torch.bool, device=DEV)
     empty[slots[keep].long()] = False
     assert not cache[empty].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rank,rot", [(512, 32), (508, 4), (514, 2), (4096, 8), (4100, 4), (9, 2)])
+def test_the_latent_alone(dtype, rank, rot):
+    """Without a query latent: in fours from 512 numbers on, else one by one; the same cache as beside one."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(rank)
+    T, eps = 9, 1e-5
+    kv, q = torch.randn(T, rank + rot, device=DEV), torch.randn(T, 64, device=DEV)
+    w, qw = (torch.rand(rank, device=DEV) + 0.5).to(dtype), torch.ones(64, device=DEV).to(dtype)
+    slots, pos = torch.randperm(16, device=DEV)[:T].int(), torch.zeros(T, dtype=torch.int64, device=DEV)
+    slots[4] = -1
+    freq = torch.ones(max(1, rot // 2), device=DEV)
+    alone, beside = (torch.zeros(16, rank + rot, dtype=dtype, device=DEV) for _ in range(2))
+    assert kernels.latent_kv_store(kv, w, pos, freq, 1.0, slots, alone, rank, rot, rot, eps) is None
+    kernels.latent_kv_store(kv, w, pos, freq, 1.0, slots, beside, rank, rot, rot, eps, q=q, q_norm_w=qw)
+    # the same sum of squares in another order, then the reciprocal root and the storage type's rounding
+    tol = rank ** 0.5 * 2.0 ** -24 + (2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -21)
+    assert ((alone.double() - beside.double()).abs() <= tol * beside.double().abs()).all()
+    assert (alone.abs().sum(-1) > 0).sum() == T - 1
