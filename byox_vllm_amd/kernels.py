@@ -181,8 +181,10 @@ def norm_gemm_pays(x, w, head_dim=None) -> bool:
 
 def takes_norm(x, residual, w, norm_w) -> bool:
     """Whether the norm of these rows can be formed in the product of ``w`` (nv_norm_gemm_*): few rows, 16-bit tiled weights."""
+    if w.fmt != _C.W_DENSE_TILED:
+        return False
     rows, cols = (x.rows, x.cols) if isinstance(x, Partials) else x.shape if torch.is_tensor(x) and x.dim() == 2 else (0, 0)
-    return (0 < rows <= NORM_GEMM_ROWS and cols == w.in_features and w.fmt == _C.W_DENSE_TILED and cols <= 2048
+    return (0 < rows <= NORM_GEMM_ROWS and cols == w.in_features and cols <= 2048
             and rows * (2 * cols + 16) <= 48 << 10
             and norm_w.dtype == w.dtype and norm_w.numel() == cols and norm_w.is_contiguous() and norm_w.data_ptr() % 16 == 0
             and (x.bias is None and residual is not None if isinstance(x, Partials)

@@ -19,6 +19,7 @@ from torch import nn
 from torch.nn.modules.module import _has_any_global_hook
 
 from byox_vllm_amd import kernels
+from byox_vllm_amd._C import W_DENSE_TILED
 from byox_vllm_amd.layers.activation import SiluAndMul
 from byox_vllm_amd.layers.attention import Attention
 from byox_vllm_amd.layers.embed_head import ParallelLMHead, VocabParallelEmbedding
@@ -65,8 +66,8 @@ class Qwen3Attention(nn.Module):
             self.q_norm = RMSNorm(self.head_dim, eps=rms_norm_eps)
             self.k_norm = RMSNorm(self.head_dim, eps=rms_norm_eps)
 
-    def _rope_args(self) -> dict:
-        context, attn = get_context(), self.attn
+    def _rope_args(self, context) -> dict:
+        attn = self.attn
         has_cache = attn.k_cache.numel() > 0
         return dict(slot_mapping=context.slot_mapping if has_cache else None,
                     k_cache=attn.k_cache if has_cache else None, v_cache=attn.v_cache if has_cache else None,
@@ -79,23 +80,24 @@ class Qwen3Attention(nn.Module):
         proj = self.qkv_proj
         if proj.packed is None:
             proj.finalize(None)
-        if not (self.fuse_qkv_rope and not self.force_fuse_qkv_rope and self.head_dim in (64, 128) and
-                plain(self, Qwen3Attention) and plain(norm, RMSNorm) and plain(proj, QKVParallelLinear) and
-                kernels.takes_norm(hidden_states, residual, proj.packed, norm.weight.data) and
-                kernels.norm_gemm_pays(hidden_states, proj.packed, self.head_dim)):
+        w = proj.packed
+        if w.fmt != W_DENSE_TILED or not self.fuse_qkv_rope or self.force_fuse_qkv_rope or self.head_dim not in (64, 128):
+            return None
+        norm_w = norm.weight.data
+        if not (kernels.takes_norm(hidden_states, residual, w, norm_w) and kernels.norm_gemm_pays(hidden_states, w, self.head_dim) and
+                plain(self, Qwen3Attention) and plain(norm, RMSNorm) and plain(proj, QKVParallelLinear)):
             return None
         qkv, residual = kernels.norm_gemm_rope_kv_store(
-            hidden_states, residual, norm.weight.data, norm.eps, proj.packed, None if proj.bias is None else proj.bias.data, positions,
-            self.rotary_emb.cos_sin_cache, self.num_heads, self.num_kv_heads, self.head_dim, **self._rope_args())
+            hidden_states, residual, norm_w, norm.eps, w, None if proj.bias is None else proj.bias.data, positions,
+            self.rotary_emb.cos_sin_cache, self.num_heads, self.num_kv_heads, self.head_dim, **self._rope_args(get_context()))
         return self._attend(qkv), residual
 
     def forward(self, positions: torch.Tensor, hidden_states: torch.Tensor) -> torch.Tensor:
         context = get_context()
-        rope = self._rope_args()
+        rope = self._rope_args(context)
         proj = self.qkv_proj
         if proj.packed is None:
             proj.finalize(None)
-        bias = None if proj.bias is None else proj.bias.data
         rows = hidden_states.size(0)
         # Decode rows run inside a captured graph, where the library's estimate of GPU time decides.  A prefill step
         # is launched eagerly and is bound by the host up to about 2 k tokens (5.4 ms for 24 layers whatever the
@@ -105,6 +107,7 @@ class Qwen3Attention(nn.Module):
             self.force_fuse_qkv_rope or (context.is_prefill and 16 <= rows <= 4096 and not many_rows) or
             kernels.lib().nv_gemm_rope_kv_store_is_faster(rows, proj.packed.in_features, proj.packed.fmt,
                                                           self.num_heads, self.num_kv_heads, self.head_dim))
+        bias = proj.bias.data if (many_rows or fused) and proj.bias is not None else None
         if many_rows and not fused and self.fuse_qkv_rope and self.head_dim in (64, 128) and \
                 kernels.rotation_streams(rows, proj.packed) and \
                 kernels.streams(hidden_states, proj.packed, bias, self.rotary_emb.cos_sin_cache, rope["k_cache"], rope["v_cache"],
@@ -144,11 +147,14 @@ class Qwen3MLP(nn.Module):
     def with_norm(self, x, residual, norm: RMSNorm):
         """As Qwen3Attention.with_norm."""
         proj = self.gate_up_proj
-        if proj.packed is None or not (proj.fused_silu and plain(self, Qwen3MLP) and plain(norm, RMSNorm) and
-                                       kernels.takes_norm(x, residual, proj.packed, norm.weight.data) and
-                                       kernels.norm_gemm_pays(x, proj.packed)):
+        w = proj.packed
+        if w is None or w.fmt != W_DENSE_TILED or not proj.fused_silu:
             return None
-        act, residual = kernels.norm_gemm_silu(x, residual, norm.weight.data, norm.eps, proj.packed)
+        norm_w = norm.weight.data
+        if not (kernels.takes_norm(x, residual, w, norm_w) and kernels.norm_gemm_pays(x, w) and
+                plain(self, Qwen3MLP) and plain(norm, RMSNorm)):
+            return None
+        act, residual = kernels.norm_gemm_silu(x, residual, norm_w, norm.eps, w)
         return self.down_proj(act, partial_out=True), residual
 
     def forward(self, x):
@@ -178,20 +184,23 @@ class Qwen3DecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(config.hidden_size, eps=config.rms_norm_eps)
 
     def forward(self, positions, hidden_states, residual):
-        done = self.self_attn.with_norm(positions, hidden_states, residual, self.input_layernorm)
+        few = positions.size(0) <= kernels.NORM_GEMM_ROWS       # asked once: an eager step of some hundred tokens waits for the host
+        norm, attn = self.input_layernorm, self.self_attn
+        done = attn.with_norm(positions, hidden_states, residual, norm) if few else None
         if done is not None:
             hidden_states, residual = done
         else:
             if residual is None:
-                hidden_states, residual = self.input_layernorm(hidden_states), hidden_states
+                hidden_states, residual = norm(hidden_states), hidden_states
             else:
-                hidden_states, residual = self.input_layernorm(hidden_states, residual)
-            hidden_states = self.self_attn(positions, hidden_states)
-        done = self.mlp.with_norm(hidden_states, residual, self.post_attention_layernorm)
+                hidden_states, residual = norm(hidden_states, residual)
+            hidden_states = attn(positions, hidden_states)
+        norm, mlp = self.post_attention_layernorm, self.mlp
+        done = mlp.with_norm(hidden_states, residual, norm) if few else None
         if done is not None:
             return done
-        hidden_states, residual = self.post_attention_layernorm(hidden_states, residual)
-        return self.mlp(hidden_states), residual
+        hidden_states, residual = norm(hidden_states, residual)
+        return mlp(hidden_states), residual
 
 
 class Qwen3Model(nn.Module):
