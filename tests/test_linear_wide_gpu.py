@@ -107,6 +107,63 @@ def test_streams_of_fp32_tiles(M, N, K, monkeypatch):
             close(got[lo:lo + 8192], x[lo:lo + 8192].double() @ w.double().t() + b.double(), K, torch.float32, out_dtype)
 
 
+def gated(y, act, cap=0.0):
+    """[.., gate | up] -> act(gate) * up, the clamped form for act 2."""
+    g, u = y.chunk(2, -1)
+    if act == 2:
+        g, u = g.clamp(max=cap), u.clamp(-cap, cap)
+        return g * torch.sigmoid(1.702 * g) * (u + 1)
+    return (torch.nn.functional.silu(g) if act == 0 else torch.nn.functional.gelu(g, approximate="tanh")) * u
+
+
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K,act,biased", [(256 * 70 + 12, 520, 128, 0, True), (256 * 66, 512, 192, 1, False), (256 * 33 + 130, 1027, 128, 2, True),
+                                              (256 * 140 + 1, 256, 256, 0, False), (300, 136, 128, 1, True)])
+def test_streams_of_gated_tiles(M, N, K, act, biased, out_dtype, monkeypatch):
+    """Gate and up rows side by side in a wavefront: 16-byte pieces of 16- and 32-bit results and columns that do not split into them, several
+    whole tiles per workgroup, last rounds in halves, remainders of rows and columns."""
+    from byox_vllm_amd import kernels
+    monkeypatch.setenv("NV_LINEAR_TILE", "2")
+    kernels.block_many_rows(True)
+    try:
+        torch.manual_seed(M + N)
+        x, w = torch.randn(M, K, device=DEV).bfloat16(), (torch.randn(2 * N, K, device=DEV) * 0.1).bfloat16()
+        b = torch.randn(2 * N, device=DEV).bfloat16() if biased else None
+        got = kernels.linear(x, w, b, out_dtype=out_dtype, epilogue=kernels.EPI_GLU, act=act, cap=1.5)
+        for lo in range(0, M, 8192):
+            want = gated(x[lo:lo + 8192].double() @ w.double().t() + (b.double() if biased else 0.0), act, 1.5)
+            close(got[lo:lo + 8192], want, 4 * K, torch.bfloat16, out_dtype)
+    finally:
+        kernels.block_many_rows(False)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("sizes,N,K", [([4096, 0, 5000, 255, 300, 8192, 1, 1023], 1032, 128), ([700] * 40, 640, 192),
+                                       ([33000, 0, 0, 129], 499, 128), ([256, 512] * 70, 264, 128)])
+def test_streams_of_grouped_tiles(sizes, N, K, dtype, monkeypatch):
+    """Experts' products whose workgroups walk several whole tiles, over gathered rows with a factor per row: gated into 16 and 32 bits, and
+    plain."""
+    from byox_vllm_amd import kernels
+    monkeypatch.setenv("NV_LINEAR_TILE", "2")
+    torch.manual_seed(sum(sizes) + N)
+    E, rows, T = len(sizes), sum(sizes), 3000
+    off = torch.tensor([0] + list(torch.tensor(sizes).cumsum(0)), dtype=torch.int32)
+    tiles = sum(-(-n // 256) for n in sizes) * -(-2 * N // 256)
+    assert tiles > 512
+    x, token = torch.randn(T, K, device=DEV).to(dtype), torch.randint(0, T, (rows,), dtype=torch.int32, device=DEV)
+    gu, scale = (torch.randn(E, 2 * N, K, device=DEV) * 0.1).to(dtype), torch.rand(rows, device=DEV) + 0.5
+    args = dict(rows=rows, a_rows=token, batch=E, group_offsets=off.to(DEV), max_group_rows=max(sizes), row_scale=scale, w_batch_stride=2 * N * K)
+    outs = [(o, kernels.linear(x, gu, epilogue=kernels.EPI_GLU, out_dtype=o, **args)) for o in (torch.bfloat16, torch.float32)]
+    plain = kernels.linear(x, gu, out_dtype=torch.float32, n=2 * N, **args)
+    for e in range(E):
+        for lo in range(off[e], off[e + 1], 8192):
+            hi = min(lo + 8192, int(off[e + 1]))
+            y = (x[token[lo:hi].long()].double() @ gu[e].double().t()) * scale[lo:hi, None].double()
+            close(plain[lo:hi], y, 2 * K, dtype, torch.float32)
+            for o, got in outs:
+                close(got[lo:hi], gated(y, 0), 4 * K, dtype, o)
+
+
 @pytest.mark.parametrize("M,N,K", [(2500, 6144, 256), (2500, 6144, 224), (2500, 2048, 256), (2500, 2048, 224), (8000, 2048, 256),
                                    (4000, 4096, 256), (1500, 2048, 512), (16384, 64, 256)])
 @pytest.mark.parametrize("glu", [False, True])

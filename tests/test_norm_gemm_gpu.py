@@ -95,6 +95,44 @@ def test_rope_kv_store(M, K, H, Hkv, D, norms, form, name):
         close(a, b, dt, what)
 
 
+def norm64(x, res, w, eps, dt):
+    """RMSNorm of x + residual in float64 with the roundings the storage type makes: the sum, the normed row, its product with the weight."""
+    total = x.double() if res is None else (x.double() + res.double()).to(dt).double()
+    normed = (total * torch.rsqrt((total * total).mean(-1, keepdim=True) + eps)).to(dt).double()
+    return (normed * w.double()).to(dt).double()
+
+
+@pytest.mark.parametrize("name", ["bf16", "fp16"])
+@pytest.mark.parametrize("form", ["first", "rows", "slabs3"])
+@pytest.mark.parametrize("M,K,H,Hkv,D,inter", [(1, 896, 14, 2, 64, 4864), (4, 1024, 3, 1, 128, 520), (2, 2048, 2, 1, 64, 24), (3, 256, 1, 1, 128, 136)])
+def test_against_float64(M, K, H, Hkv, D, inter, form, name):
+    """Both products of normed rows, SiLU's and the rotation's ends, from the sums to the last rounding in float64."""
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.layers.quant import LinearWeight, interleave_gate_up
+    torch.manual_seed(M + K)
+    dt, N, u = DT[name], (H + 2 * Hkv) * D, torch.finfo(DT[name]).eps / 2
+    x, rows, res = inputs(M, K, dt, form)
+    nw = (torch.rand(K, device=DEV) + 0.5).to(dt)
+    h = norm64(rows, res, nw, 1e-6, dt)
+    # a row's normed numbers may lie on the other side of a rounding: sums of K products of N(0, 1) by N(0, 1 / K) with some of their
+    # terms off by two roundings stay within two of a unit number; each result then has its own roundings
+    gu = (torch.randn(2 * inter, K, device=DEV) * K ** -0.5).to(dt)
+    got, _ = kernels.norm_gemm_silu(x, res, nw, 1e-6, LinearWeight.dense_tiled(interleave_gate_up(gu)))
+    gate, up = (h @ gu.double().t()).chunk(2, -1)
+    assert ((got.double() - torch.nn.functional.silu(gate) * up).abs() <= 5 * u * (1 + gate.abs()) * (1 + up.abs())).all()
+
+    w, bias = (torch.randn(N, K, device=DEV) * K ** -0.5).to(dt), torch.randn(N, device=DEV).to(dt)
+    pos, angle = torch.randint(0, 100, (M,), device=DEV), torch.rand(100, D // 2, device=DEV) * 6.28
+    cos_sin = torch.cat([angle.cos(), angle.sin()], -1).contiguous()
+    qkv, _ = kernels.norm_gemm_rope_kv_store(x, res, nw, 1e-6, LinearWeight.dense_tiled(w), bias, pos, cos_sin, H, Hkv, D)
+    y = (h @ w.double().t() + bias.double()).view(M, -1, D)
+    a, b = y[:, :H + Hkv].chunk(2, -1)
+    c, s = cos_sin[pos].double().view(M, 1, D).chunk(2, -1)
+    want = torch.cat([torch.cat([a * c - b * s, b * c + a * s], -1), y[:, H + Hkv:]], 1)
+    size = 1 + torch.maximum(want.abs(), y.abs().amax(-1, keepdim=True))
+    assert ((qkv.view(M, -1, D).double() - want).abs() <= 5 * u * size).all()
+
+
 def test_refuses_what_it_cannot_hold():
     from byox_vllm_amd import kernels
     from byox_vllm_amd.layers.quant import LinearWeight
