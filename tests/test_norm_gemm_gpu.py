@@ -6,6 +6,20 @@ import torch
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
+
+
+@pytest.fixture(autouse=True)
+def one_rank(monkeypatch):
+    """Layers of one rank and rotation tables of their own, whatever ran before."""
+    from byox_vllm_amd.layers import linear
+    from byox_vllm_amd.layers.rotary_embedding import get_rope
+    monkeypatch.setattr(linear, "_TP_STATE", (0, 1, None))
+    monkeypatch.setattr(linear, "_COMM", None)
+    get_rope.cache_clear()
+    yield
+    get_rope.cache_clear()
+
+
 DT = {"bf16": torch.bfloat16, "fp16": torch.float16}
 
 

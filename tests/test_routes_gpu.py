@@ -8,6 +8,20 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
+@pytest.fixture(autouse=True)
+def one_rank(monkeypatch):
+    """Layers of one rank and rotation tables of their own, whatever ran before."""
+    from byox_vllm_amd.layers import linear
+    from byox_vllm_amd.layers.rotary_embedding import get_rope
+    monkeypatch.setattr(linear, "_TP_STATE", (0, 1, None))
+    monkeypatch.setattr(linear, "_COMM", None)
+    get_rope.cache_clear()
+    yield
+    get_rope.cache_clear()
+
+
+
+
 @pytest.fixture()
 def launched(monkeypatch):
     """The library's functions that are called, in their order, without the questions asked of it."""
@@ -196,3 +210,24 @@ def test_norms_of_a_few_rows(rows, K, H, Hkv, D, inter, attn, mlp, launched):
         reset_context()
     assert ("nv_norm_gemm_rope_kv_store" in launched, "nv_norm_gemm_silu" in launched) == (attn, mlp), launched
     assert sum(n.startswith("nv_add_rmsnorm") for n in launched) == 2 - attn - mlp
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,n", [(1, 4), (37, 516), (3, 7)])
+def test_passes_over_a_products_rows(rows, n, dtype):
+    """The passes behind the library's products, with a bias and in the forms without one (which only C callers use)."""
+    from byox_vllm_amd._C import check, dtype_code, lib, ptr, stream
+    torch.manual_seed(rows + n)
+    y, b = torch.randn(rows, 2 * n, device=DEV), torch.randn(2 * n, device=DEV).to(dtype)
+    code = dtype_code(dtype, allow_f32=True)
+    for bias in (None, b):
+        x = y.double() + (0.0 if bias is None else bias.double())
+        out, half = torch.empty(rows, 2 * n, dtype=dtype, device=DEV), torch.empty(rows, n, dtype=dtype, device=DEV)
+        if bias is None:
+            check(lib().nv_act_f32(ptr(y), ptr(out), rows * 2 * n, 1, None, 0.0, code, stream()), "nv_act_f32")
+            check(lib().nv_act_mul_f32(ptr(y), ptr(half), rows, n, 0, 0.0, code, stream()), "nv_act_mul_f32")
+        else:
+            check(lib().nv_bias_act_f32(ptr(y), ptr(bias), 2 * n, ptr(out), rows * 2 * n, 1, None, 0.0, code, stream()), "nv_bias_act_f32")
+            check(lib().nv_bias_act_mul_f32(ptr(y), ptr(bias), ptr(half), rows, n, 0, 0.0, code, stream()), "nv_bias_act_mul_f32")
+        close(out, torch.nn.functional.gelu(x, approximate="tanh"), 4, dtype)
+        close(half, torch.nn.functional.silu(x[:, :n]) * x[:, n:], 4, dtype)
