@@ -4,7 +4,8 @@
 //
 // What bounded these steps: the vendor library's product, then a pass over its whole result that moves it twice.  14.6 k rows of 1024
 // (Qwen3-0.6B): gate and up 157 us and SiluAndMul 53, q/k/v 105 and rotation with the store 61, and 5 - 7 us before each for the
-// weight as rows.
+// weight as rows.  Here 190 and 151 us; SiLU by exp and quotient, as in the pass, is 20 of the first.  Which sizes this pays for:
+// kernels.gemm_many_rows and kernels.rotation_streams.
 #include <type_traits>
 
 #include "rope_common.h"

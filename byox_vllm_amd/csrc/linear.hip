@@ -3,8 +3,8 @@
 // (nv_gemm) does not take: K or N that are no multiples of its tiles, fp32 models, batched products with one weight
 // per head, grouped products with one weight per expert over gathered rows, and the gated epilogues.
 //
-// linear_stream.h and linear_wide.h serve more than 64 rows whose K splits into 128-byte blocks, linear_short.h many rows by a K below that,
-// linear_few.h up to 64 rows; linear_tile_kernel below the other aligned bf16 products of many rows, linear_kernel the rest.
+// linear_stream.h and linear_wide.h serve more than 64 rows whose K splits into 128-byte blocks, linear_short.h many rows by a K below
+// that, linear_few.h up to 64 rows; linear_tile_kernel below the other aligned bf16 products of many rows, linear_kernel the rest.
 //
 // linear_kernel: a workgroup owns a 64 x 64 tile of the output: wavefront w the 16 columns n0 + 16 w .. and all four 16-row
 // sub-tiles.  Operands go from memory straight into MFMA fragments (both are K-contiguous rows, which is the fragment

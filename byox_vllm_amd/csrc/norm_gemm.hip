@@ -5,9 +5,9 @@
 // norm and the rotation are two of them around a product whose weights do not depend on them.  Here every workgroup forms the norm of
 // all rows itself (a few KB), four numbers to a thread, while its weights are already on their way: 16 rows by 32 of K
 // per wavefront and register set, the whole K of a tile of 16 outputs dealt to PARTS wavefronts.  Only the first workgroup writes the
-// new residual, to another buffer than the one the others may still be reading.  Qwen2-0.5B, one row: norm 3.7 + product 8.3 us and
-// 3.7 + 4.6 + rotation 4.5, here 9.1 and 8.0 under the profiler; the step 865 and 761.  From six rows on the repeated norm costs more
-// than its launch did (kernels.NORM_GEMM_ROWS).
+// new residual, to another buffer than the one the others may still be reading.  Qwen2-0.5B, one row, under the profiler: norm 3.7 +
+// product 8.3 us and 3.7 + 4.6 + rotation 4.5, here 8.5 and 8.3; the step in a captured graph 867 and 774.  The norm is repeated by every
+// workgroup, in passes over the rows that its wavefronts hold at once: which sizes that pays for is kernels.norm_gemm_pays.
 #include "rope_common.h"
 #include "splitk.h"
 

@@ -1,21 +1,22 @@
 // Products of many rows: a workgroup per CU walks tiles of 256 x 256 outputs whose K blocks form one stream.
 //
 // What bounds it: the matrix cores and, on this part, their power: at 8192 x 8192 x 8192 the loop that this one replaced (a block
-// fetched, waited for and multiplied behind one barrier, 32 x 32 products) kept them 56 % busy at 1.76 GHz, the vendor library's
-// 87 % at 1.59.  What the loop spent beside them, from copies that leave one activity out (8192^3, us): whole 882, operands always
-// from the same cache lines 719, no LDS reads 716, no DMA 669, none of these and no barriers 505.  So
+// fetched, waited for and multiplied behind one barrier, 32 x 32 products) takes 1108 us with them 49 % busy, this one 866 with 65 %, the
+// vendor library 696 with 89 % (one machine, the chip warm; busy cycles per active one under the counters, where the clock is 1.4 - 1.9
+// GHz and lowest for the busiest).  What a form between the two spent beside the products, from copies that leave one activity out (us):
+// whole 882, operands always from the same cache lines 719, no LDS reads 716, no DMA 669, none of these and no barriers 505.  So
 //   * 16 x 16 x 32 products: a lane's results lie where whole 64-byte pieces of rows can be stored (14592 rows by 4096, K 1024: 143
 //     us with 32 x 32 products, 125 with these);
 //   * the barrier stands before the block's last step of K, whose fragments are in registers: behind it the first fragments of the
 //     next block are read under that step's products, and the buffer just left is refilled, one DMA instruction behind every few
-//     products (with all of them behind the reads: 846 us at 8192^3, so 796);
+//     products (with all of them behind the reads that form took 846 us at 8192^3, so 796);
 //   * the order of products, LDS reads and DMA is fixed in the source (sched_barrier); left alone, the compiler puts the reads
 //     behind two thirds of the products and waits for them at once;
 //   * workgroups stay: the first two blocks of the next tile are on their way while the results of a tile are stored, and nothing
 //     waits for those stores but the second block after them (14592 by 4096, K 1024: 129 us with a workgroup per tile, so 117).
 //     Their tiles are found once, by a thread each, and kept in LDS: found in the loop they cost it its registers.
-// Measured, before and after: sixteen experts, 32768 rows of them, gated up 2048 -> 2 x 3072 and down, the layer 1582 and 1428 us;
-// 16384 rows 2048 -> 6144 into fp32 429 and 372 us (1110 TFLOP/s).
+// Measured, before and after: sixteen experts, 32768 rows of them, gated up 2048 -> 2 x 3072 and down, the layer 1569 and 1401 us;
+// 16384 rows 2048 -> 6144 into fp32 473 and 380 us (1085 TFLOP/s).
 // LDS rows are 128 bytes, their 16-byte pieces dealt by XOR (through the DMA's source addresses) so that the 16 rows a read touches lie
 // in 16 bank groups.  Tiles go to the XCDs in contiguous eighths, within them in bands of eight row
 // tiles, so the 32 workgroups of an XCD share 8 row and 4 column panels in its L2.  A group's short last row tile stays in its band

@@ -332,9 +332,10 @@ def pick_split_k(M, N, K, wfmt=_C.W_INT4):
 
 
 # Rows from which a product goes through the vendor library (nv_gemm_lt) instead of nv_gemm's decode-shaped tiles:
-# prefill steps; from the same number on, what gemm_many_rows keeps on this library's own tiles.  Measured on the layer shapes of Qwen3-0.6B, Qwen2-0.5B and Qwen2-7B, weight expansion included
+# prefill steps.  Measured on the layer shapes of Qwen3-0.6B, Qwen2-0.5B and Qwen2-7B, weight expansion included
 # (scripts/r03_dense_prefill_gemm.py): at 1024 rows nv_gemm wins everywhere, at 2048 the two trade places by shape,
 # from 4096 on the library wins or ties (1.3-1.7 times faster from 8192).  NV_GEMM_LT_ROWS=0 switches the path off.
+# The streamed tiles (nv_gemm_stream) take part from the same number on, for gate/up from half of it, and are switched off with it.
 MANY_ROWS = int(os.environ.get("NV_GEMM_LT_ROWS", "4096"))
 LT_WORKSPACE_BYTES = 128 << 20
 
@@ -429,7 +430,7 @@ def gemm_many_rows(x, w, bias=None, out=None, silu_mul=False):
     """gemm() for prefill-sized x: the weight written out row-major into scratch and one vendor-library product, with a SiluAndMul pass
     over its result for gate/up weights; or, where that is not slower, this library's tiles (nv_gemm_stream).  Those have
      * gate/up weights of a K below 4096, or below 2048 where the weight has to be expanded, without a bias (16384 rows, both routes:
-       1024 -> 2 x 3072 217 and 197 us, int4 216 and 204; 2048 -> 2 x 6144 690 and 706, 6000 rows 351 and 271; 4096 rows 4096 -> 2 x
+       1024 -> 2 x 3072 217 and 197 us, int4 216 and 204; 14600 rows 220 and 190; 2048 -> 2 x 6144 690 and 706, 6000 rows 351 and 271; 4096 rows 4096 -> 2 x
        12288 645 and 651, int4 653 and 723);
      * products of 512 <= K < 1024 without a bias whose columns do not split into tiles and whose results fill 0.6 of their rounds, 0.8
        where the weight has to be expanded (tile_share; 16384 rows 896 -> 896, share 0.88: 43 and 30 us, int4 43 and 33; 11000 rows

@@ -166,8 +166,9 @@ int nv_gemm_lt(const void* x, int64_t x_row_stride, const void* w_rowmajor, cons
 /* The same many-row products on this library's own tiles, with what follows them; W in a 16-bit format of nv_gemm (NV_W_DENSE,
  * NV_W_DENSE_TILED), read as it lies.  nv_gemm_stream: out = x * W^T (+ bias), or with silu_mul the rows of nv_gemm's silu(gate)*up
  * epilogue (gate 2i, gate 2i+1, up 2i, up 2i+1; no bias; out [M, N / 2], nanovllm/layers/activation.py:10-13).
- * nv_gemm_stream_rope_kv_store: arguments and results of nv_gemm_rope_kv_store.  K >= 128, pointers 16-byte aligned, row strides
- * multiples of 8.  No workspace; may be captured. */
+ * nv_gemm_stream_rope_kv_store: arguments and results of nv_gemm_rope_kv_store.  K >= 128 and a multiple of 64 (tiled: 128), N a
+ * multiple of 16, pointers 16-byte aligned, row strides multiples of 8 that are no shorter than a row.  No workspace; may be captured;
+ * results are stored as without nv_set_result_policy. */
 int nv_gemm_stream(const void* x, int64_t x_row_stride, const void* w, const void* bias, void* out, int64_t out_row_stride,
                    int M, int N, int K, int wfmt, int silu_mul, int dtype, nv_stream_t stream);
 int nv_gemm_stream_rope_kv_store(const void* x, int64_t x_row_stride, const void* w, const void* bias, void* qkv,
@@ -178,7 +179,8 @@ int nv_gemm_stream_rope_kv_store(const void* x, int64_t x_row_stride, const void
 
 /* A residual add and RMSNorm (RMSNorm.add_rms_forward, nanovllm/layers/layernorm.py:31-41) inside the product that follows, for up to 16
  * rows.  x [M, K], or the fp32 slabs of a split-K product (x NULL); residual NULL: the norm alone; residual_out: another buffer than
- * residual.  w_tiled: NV_W_DENSE_TILED, K a multiple of 128 up to 2048, M rows of which fit 48 KB.
+ * residual.  w_tiled: NV_W_DENSE_TILED, K a multiple of 128 up to 2048, M rows of which fit 48 KB.  Results are stored as without
+ * nv_set_result_policy.
  * nv_norm_gemm_silu: gate/up rows as nv_gemm's silu(gate)*up epilogue wants them, out [M, N / 2];
  * nv_norm_gemm_rope_kv_store: the rest as in nv_gemm_rope_kv_store, `head_eps` for the per-head norms. */
 int nv_norm_gemm_silu(const void* x, const float* partials, int num_partials, const void* residual, void* residual_out,
