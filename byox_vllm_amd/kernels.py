@@ -430,8 +430,8 @@ def gemm_many_rows(x, w, bias=None, out=None, silu_mul=False):
     """gemm() for prefill-sized x: the weight written out row-major into scratch and one vendor-library product, with a SiluAndMul pass
     over its result for gate/up weights; or, where that is not slower, this library's tiles (nv_gemm_stream).  Those have
      * gate/up weights of a K below 4096, or below 2048 where the weight has to be expanded, without a bias (16384 rows, both routes:
-       1024 -> 2 x 3072 217 and 197 us, int4 216 and 204; 14600 rows 220 and 190; 2048 -> 2 x 6144 690 and 706, 6000 rows 351 and 271; 4096 rows 4096 -> 2 x
-       12288 645 and 651, int4 653 and 723);
+       1024 -> 2 x 3072 217 and 197 us, int4 216 and 204; 14600 rows 220 and 190; 2048 -> 2 x 6144 690
+       and 706, 6000 rows 351 and 271; 4096 rows 4096 -> 2 x 12288 645 and 651, int4 653 and 723);
      * products of 512 <= K < 1024 without a bias whose columns do not split into tiles and whose results fill 0.6 of their rounds, 0.8
        where the weight has to be expanded (tile_share; 16384 rows 896 -> 896, share 0.88: 43 and 30 us, int4 43 and 33; 11000 rows
        896 -> 640, 0.42: 21 and 27; whole tiles: 16384 rows 896 -> 8192 198 and 223, 2048 -> 1024 51 and 55)."""

@@ -117,7 +117,8 @@ def gated(y, act, cap=0.0):
 
 
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("M,N,K,act,biased", [(256 * 70 + 12, 520, 128, 0, True), (256 * 66, 512, 192, 1, False), (256 * 33 + 130, 1027, 128, 2, True),
+@pytest.mark.parametrize("M,N,K,act,biased", [(256 * 70 + 12, 520, 128, 0, True), (256 * 66, 512, 192, 1, False),
+                                              (256 * 33 + 130, 1027, 128, 2, True),
                                               (256 * 140 + 1, 256, 256, 0, False), (300, 136, 128, 1, True)])
 def test_streams_of_gated_tiles(M, N, K, act, biased, out_dtype, monkeypatch):
     """Gate and up rows side by side in a wavefront: 16-byte pieces of 16- and 32-bit results and columns that do not split into them, several
@@ -152,7 +153,8 @@ def test_streams_of_grouped_tiles(sizes, N, K, dtype, monkeypatch):
     assert tiles > 512
     x, token = torch.randn(T, K, device=DEV).to(dtype), torch.randint(0, T, (rows,), dtype=torch.int32, device=DEV)
     gu, scale = (torch.randn(E, 2 * N, K, device=DEV) * 0.1).to(dtype), torch.rand(rows, device=DEV) + 0.5
-    args = dict(rows=rows, a_rows=token, batch=E, group_offsets=off.to(DEV), max_group_rows=max(sizes), row_scale=scale, w_batch_stride=2 * N * K)
+    args = dict(rows=rows, a_rows=token, batch=E, group_offsets=off.to(DEV), max_group_rows=max(sizes), row_scale=scale,
+                w_batch_stride=2 * N * K)
     outs = [(o, kernels.linear(x, gu, epilogue=kernels.EPI_GLU, out_dtype=o, **args)) for o in (torch.bfloat16, torch.float32)]
     plain = kernels.linear(x, gu, out_dtype=torch.float32, n=2 * N, **args)
     for e in range(E):

@@ -118,7 +118,8 @@ def norm64(x, res, w, eps, dt):
 
 @pytest.mark.parametrize("name", ["bf16", "fp16"])
 @pytest.mark.parametrize("form", ["first", "rows", "slabs3"])
-@pytest.mark.parametrize("M,K,H,Hkv,D,inter", [(1, 896, 14, 2, 64, 4864), (4, 1024, 3, 1, 128, 520), (2, 2048, 2, 1, 64, 24), (3, 256, 1, 1, 128, 136)])
+@pytest.mark.parametrize("M,K,H,Hkv,D,inter", [(1, 896, 14, 2, 64, 4864), (4, 1024, 3, 1, 128, 520), (2, 2048, 2, 1, 64, 24),
+                                               (3, 256, 1, 1, 128, 136)])
 def test_against_float64(M, K, H, Hkv, D, inter, form, name):
     """Both products of normed rows, SiLU's and the rotation's ends, from the sums to the last rounding in float64."""
     from byox_vllm_amd import kernels

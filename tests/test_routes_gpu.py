@@ -76,7 +76,8 @@ OWN, OTHER, LT = ["nv_gemm_stream"], ["nv_gemm"], ["nv_weight_expand", "nv_gemm_
 
 @pytest.mark.parametrize("M,K,inter,fmt,want", [
     (2047, 512, 5120, None, OTHER), (2048, 512, 5120, None, OWN), (2048, 512, 2432, None, OTHER), (2048, 512, 2560, None, OWN),
-    (2048, 512, 5120, "w4a16", OTHER), (4095, 256, 512, None, OTHER), (4096, 256, 512, None, OWN), (4096, 256, 512, "w8a16", ["nv_weight_expand"] + OWN),
+    (2048, 512, 5120, "w4a16", OTHER), (4095, 256, 512, None, OTHER), (4096, 256, 512, None, OWN),
+    (4096, 256, 512, "w8a16", ["nv_weight_expand"] + OWN),
     (4096, 3968, 256, None, OWN), (4096, 4096, 256, None, LT), (4096, 1920, 256, "w4a16", ["nv_weight_expand"] + OWN),
     (4096, 2048, 256, "w4a16", LT)])
 def test_gate_up_of_many_rows(M, K, inter, fmt, want, launched):
