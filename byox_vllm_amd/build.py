@@ -93,11 +93,17 @@ def _has_all(sources) -> bool:
     return {os.path.basename(s) for s in sources} <= have
 
 
+def _with_needed(names):
+    """``names`` and what their sources call in others."""
+    needs = {"linear": ("linear_deep",)}
+    return list(dict.fromkeys(m for n in names for m in (n,) + needs.get(n, ())))
+
+
 def ensure(names) -> str:
     """Make sure a library with the kernels of csrc/<name>.hip, name in ``names``, is there.  An existing library is
     used as it is when it holds them and none of them is stale; otherwise exactly these sources are compiled and
     linked (beside whatever objects of an earlier partial build are current)."""
-    sources = [os.path.join(CSRC, n + ".hip") for n in names]
+    sources = [os.path.join(CSRC, n + ".hip") for n in _with_needed(names)]
     if os.path.exists(LIB) and _has_all(sources) and not _stale(LIB, sources + _headers()):
         return LIB
     objs = compile_sources(sources)

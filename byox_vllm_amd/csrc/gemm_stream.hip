@@ -9,7 +9,7 @@
 #include <type_traits>
 
 #include "rope_common.h"
-#include "stream_tiles.h"
+#include "stream_deep.h"
 
 namespace {
 
@@ -22,15 +22,14 @@ struct RowsArgs {
 
 enum { ROWS_PLAIN = 0, ROWS_SILU = 1, ROWS_ROPE = 2 };
 
-template <typename TT, int WHAT, int D, bool TILED>     // D: head size (ROWS_ROPE)
+template <typename TT, int WHAT, int D, bool TILED, bool FAR>     // D: head size (ROWS_ROPE); FAR: a tile's rows span 4 GiB and more
 struct RowsJob {
   typedef TT T;
   typedef std::conditional_t<WHAT == ROWS_SILU, std::conditional_t<TILED, StreamQuadsTiled, StreamQuads>,
                              std::conditional_t<TILED, StreamPairedTiled, StreamPaired>> Order;
   static constexpr bool SILU = WHAT == ROWS_SILU, ROPE = WHAT == ROWS_ROPE;
-  // a wavefront has whole heads, 128 columns, where their halves meet; else 64 columns and more rows
-  static constexpr int WN = ROPE ? 2 : 4, MT = 2 * WN, NT = 32 / WN / 2, NOUT = SILU ? 128 : 256;
-  static constexpr int NSTORE = MT * (SILU ? 1 : NT / 2);
+  static constexpr int NOUT = SILU ? 128 : 256, NSTORE_WAVE = SILU ? 16 : 32, EXTRA = ROPE ? 3072 : 0;
+  static constexpr bool FAR_A = FAR, FAR_W = FAR;
   RowsArgs p;
   RopeArgs ra;
   int K, rows, cols;      // row and column tiles
@@ -41,22 +40,25 @@ struct RowsJob {
     stream_order(tile, rows, cols, m_tile, n_tile);
     return StreamTile{m_tile * STREAM_BM, p.M, n_tile * NOUT, 0};
   }
-  __device__ __forceinline__ const void* a_base(const StreamTile&) const { return p.x; }
+  // the second half of a short tile has no rows and begins behind the last one
+  __device__ __forceinline__ static int first_row(const StreamTile& at) { return min(at.lo, at.hi - 1); }
+  __device__ __forceinline__ const void* a_base(const StreamTile& at) const { return reinterpret_cast<const uint16_t*>(p.x) + first_row(at) * p.xs; }
   __device__ __forceinline__ uint32_t a_stride() const { return (uint32_t)p.xs * 2; }
-  __device__ __forceinline__ uint32_t a_row(const StreamTile& at, int r) const { return (uint32_t)min(at.lo + r, at.hi - 1); }
-  __device__ __forceinline__ const void* w_base(const StreamTile&) const { return p.w; }
+  __device__ __forceinline__ uint32_t a_row(const StreamTile& at, int r) const { return (uint32_t)min(r, at.hi - 1 - first_row(at)); }
+  __device__ __forceinline__ const void* w_base(const StreamTile& at) const {
+    return reinterpret_cast<const uint16_t*>(p.w) + (int64_t)at.n0 * (SILU ? 2 : 1) * p.K;      // a row has K numbers in either layout
+  }
   __device__ __forceinline__ uint32_t w_stride() const { return (uint32_t)p.K * (TILED ? 32 : 2); }
   __device__ __forceinline__ uint32_t w_row(const StreamTile& at, int r) const {      // r: row, or 16-row tile
-    const int n = at.n0 * (SILU ? 2 : 1);
-    return TILED ? min((n >> 4) + r, (p.N >> 4) - 1) : min(n + r, p.N - 1);
+    const int left = p.N - at.n0 * (SILU ? 2 : 1);
+    return min(r, (TILED ? left >> 4 : left) - 1);
   }
   __device__ __forceinline__ uint32_t w_step() const { return TILED ? 2048 : 128; }
   __device__ __forceinline__ bool whole(const StreamTile& at) const {
     return at.lo + STREAM_BM <= at.hi && (at.n0 + NOUT) * (SILU ? 2 : 1) <= p.N;
   }
 
-  static __device__ __forceinline__ void widen(const uint16_t* at, float (&v)[8]) {
-    const u32x4 w = *reinterpret_cast<const u32x4*>(at);
+  static __device__ __forceinline__ void widen(const u32x4& w, float (&v)[8]) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       v[2 * e] = lo_f32<T>(w[e]);
@@ -68,122 +70,192 @@ struct RowsJob {
   }
   static __device__ __forceinline__ float rounded(float v) { return bits_to_f32<T>(f32_to_bits<T>(v)); }
 
-  __device__ __forceinline__ void store(const StreamTile& at, int row0, int wn, int lane, const f32x4 (&acc)[NT][MT]) const {
+  // -------- results: 64 rows of each half of the tile by 128 rows of W to a wavefront
+  __device__ __forceinline__ void fetch_extra(const StreamTile& at, int wv, int lane, unsigned char* extra) const {
+    if constexpr (ROPE) {      // the rows' positions (their low halves), cache rows, bias and norm weights, a tile ahead of their use
+      typedef __attribute__((address_space(1))) void global_void;
+      typedef __attribute__((address_space(3))) void lds_void;
+      const int t = min(at.lo + 64 * wv + lane, at.hi - 1);
+      __builtin_amdgcn_global_load_lds((global_void*)(ra.positions + t), (lds_void*)(extra + 256 * wv), 4, 0, 0);
+      if (ra.slots) __builtin_amdgcn_global_load_lds((global_void*)(ra.slots + t), (lds_void*)(extra + 1024 + 256 * wv), 4, 0, 0);
+      const uint16_t* norm = wv & 1 ? ra.kn_w : ra.qn_w;
+      const uint16_t* from = wv < 2 ? reinterpret_cast<const uint16_t*>(p.bias) : norm;      // two numbers to a lane
+      const int n = wv < 2 ? min(at.n0 + 128 * wv + 2 * lane, p.N - 2) : min(2 * lane, D - 2);
+      if (from) __builtin_amdgcn_global_load_lds((global_void*)(from + n), (lds_void*)(extra + 2048 + 256 * wv), 4, 0, 0);
+    }
+  }
+  __device__ __forceinline__ void finish(const StreamTile& at, int wm, int wn, int lane, bool live0, bool live1, const unsigned char* extra) const {
+    if constexpr (ROPE) {
+      if (at.n0 + 128 * wn < p.N) rotate(at, wm, at.n0 + 128 * wn, lane, live0, live1, extra);
+    } else {
+      if (live0) store<0>(at, at.lo + 64 * wm, wn, lane);
+      if (live1) store<1>(at, at.lo + 128 + 64 * wm, wn, lane);
+    }
+  }
+  template <int HALF>
+  __device__ __forceinline__ void store(const StreamTile& at, int row0, int wn, int lane) const {
     const int fr = lane & 15, g = lane >> 4;
+    constexpr int PIECES = SILU ? 2 : 4;
+    int n[PIECES];
+    u32x4 b[PIECES];      // ahead of the first store: loads and stores are counted in one order
     const uint16_t* bias = reinterpret_cast<const uint16_t*>(p.bias);
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      __builtin_amdgcn_sched_barrier(0);       // one row's results at a time: registers
+    for (int q = 0; q < PIECES; ++q) {
+      n[q] = at.n0 + (SILU ? 64 : 128) * wn + 32 * q + 8 * g;
+      if (!SILU && bias) b[q] = *reinterpret_cast<const u32x4*>(bias + min(n[q], p.N - 8));
+    }
+    if (!SILU && bias) {
+#pragma unroll
+      for (int q = 0; q < PIECES; ++q) asm volatile("" : "+v"(b[q]));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
       const int s = row0 + 16 * i + fr;
-      if constexpr (SILU) {
-        const int n = at.n0 + 32 * wn + 8 * g;        // a lane's eight results come from 16 rows of W: N is a multiple of that
-        if (s >= at.hi || 2 * n >= p.N) continue;
+      uint16_t* row = reinterpret_cast<uint16_t*>(p.out) + s * p.os;
+#pragma unroll
+      for (int q = 0; q < PIECES; ++q) {
+        __builtin_amdgcn_sched_barrier(0);       // a few results at a time: registers
         float v[8];
+        if constexpr (SILU) {      // a lane's eight results come from 16 rows of W: N is a multiple of that
+          f32x4 x[4];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          // dtype(dtype(silu(dtype(gate))) * dtype(up)), as nv_silu_mul takes it
-          const float gt = rounded(acc[e >> 2][i][e & 3]), up = rounded(acc[2 + (e >> 2)][i][e & 3]);
-          v[e] = rounded(gt / (1.0f + expf(-gt))) * up;
-        }
-        *reinterpret_cast<u32x4*>(reinterpret_cast<uint16_t*>(p.out) + s * p.os + n) = pack(v);
-      } else {
-        const int n0 = at.n0 + 16 * NT * wn;
-        uint16_t* row = reinterpret_cast<uint16_t*>(p.out) + s * p.os;
-        if constexpr (!ROPE) {
-          if (s >= at.hi) continue;
+          for (int j = 0; j < 4; ++j) x[j] = deep_take(HALF, 4 * q + j, i);
 #pragma unroll
-          for (int q = 0; q < NT / 2; ++q) {
-            const int n = n0 + 32 * q + 8 * g;
-            if (n >= p.N) continue;
-            float v[8], b[8] = {};
-            if (bias) widen(bias + n, b);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = acc[2 * q + (e >> 2)][i][e & 3] + b[e];
-            *reinterpret_cast<u32x4*>(row + n) = pack(v);
+          for (int e = 0; e < 8; ++e) {
+            // dtype(dtype(silu(dtype(gate))) * dtype(up)), as nv_silu_mul takes it
+            const float gt = rounded(x[e >> 2][e & 3]), up = rounded(x[2 + (e >> 2)][e & 3]);
+            v[e] = rounded(gt / (1.0f + expf(-gt))) * up;
           }
         } else {
+          f32x4 x[2];
 #pragma unroll
-          for (int h = 0; h < 128 / D; ++h) rope_row(s, s < at.hi, n0 + D * h, 8 * g, bias, row, acc, i, 2 * (D / 32) * h);
+          for (int j = 0; j < 2; ++j) x[j] = deep_take(HALF, 2 * q + j, i);
+          float w[8];
+          if (bias) widen(b[q], w);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = x[e >> 2][e & 3] + (bias ? w[e] : -0.0f);
         }
+        if (s < at.hi && n[q] * (SILU ? 2 : 1) < p.N) *reinterpret_cast<u32x4*>(row + n[q]) = pack(v);
       }
     }
   }
 
-  // One head of one token, spread over the four lanes g: `c` = 8 g, numbers 32 q + c .. + 7 from products j0 + 2 q and j0 + 2 q + 1.
-  // The arithmetic and its roundings are those of rope_finish.
-  __device__ __forceinline__ void rope_row(int64_t t, bool live, int n, int c, const uint16_t* bias, uint16_t* row,
-                                           const f32x4 (&acc)[NT][MT], int i, int j0) const {
-    constexpr int Q = D / 32;
-    if (n >= p.N) return;
-    const int hs = n / D;
-    const bool is_q = hs < ra.H, is_k = !is_q && hs < ra.H + ra.Hkv;
-    float x[Q][8];
+  // The heads of columns n0 .. n0 + 127 of the wavefront's rows: lane (fr, g) has numbers 32 q + 8 g .. + 7 of a head of row fr.  The
+  // arithmetic and its roundings are those of rope_finish.  A row's cosines and sines are asked for two rows ahead, before the stores of
+  // the row between: behind them they would be waited for with them.
+  __device__ __forceinline__ void rotate(const StreamTile& at, int wm, int n0, int lane, bool live0, bool live1, const unsigned char* extra) const {
+    constexpr int Q = D / 32, HEADS = 128 / D;
+    const int fr = lane & 15, c = 8 * (lane >> 4);
+    bool is_q[HEADS], is_k[HEADS];
+    int hs[HEADS];
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      float b[8] = {};
-      if (bias) widen(bias + n + 32 * q + c, b);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[q][e] = rounded(acc[j0 + 2 * q + (e >> 2)][i][e & 3] + b[e]);
+    for (int h = 0; h < HEADS; ++h) {
+      hs[h] = n0 / D + h;
+      is_q[h] = hs[h] < ra.H;
+      is_k[h] = !is_q[h] && hs[h] < ra.H + ra.Hkv;
     }
-    const int slot = ra.slots && live ? ra.slots[t] : -1;
-    const uint16_t* nw = is_q ? ra.qn_w : is_k ? ra.kn_w : nullptr;
-    if (nw) {
-      float ss = 0.f;
+    const bool turns = n0 < (ra.H + ra.Hkv) * D;
+    auto kept = [&](int r, int which) { return *reinterpret_cast<const uint32_t*>(extra + 1024 * which + 4 * (128 * (r >> 2) + 64 * wm + 16 * (r & 3) + fr)); };
+    f32x4 turn[2][2 * Q];      // cosines, then sines
+    auto ask = [&](int r) {
+      if (!turns) return;
+      const float* cs = ra.cos_sin + (int64_t)kept(r, 0) * D + c;
 #pragma unroll
-      for (int q = 0; q < Q; ++q)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) ss += x[q][e] * x[q][e];
-      float even, odd, lower, upper;
-      rows_pair16(ss, even, odd);
-      rows_pair32(even + odd, lower, upper);
-      const float inv = 1.0f / sqrtf((lower + upper) / (float)D + ra.eps);
-#pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        float w[8];
-        widen(nw + 32 * q + c, w);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[q][e] = rounded(rounded(x[q][e] * inv) * w[e]);
-      }
-    }
-    if (!live) return;
-    if (is_q || is_k) {
-      const float* cs = ra.cos_sin + ra.positions[t] * D + c;
-#pragma unroll
-      for (int q = 0; q < Q / 2; ++q) {
+      for (int q = 0; q < Q / 2; ++q)
 #pragma unroll
         for (int v = 0; v < 2; ++v) {
-          const f32x4 co = *reinterpret_cast<const f32x4*>(cs + 32 * q + 4 * v), si = *reinterpret_cast<const f32x4*>(cs + D / 2 + 32 * q + 4 * v);
+          turn[r & 1][2 * q + v] = *reinterpret_cast<const f32x4*>(cs + 32 * q + 4 * v);
+          turn[r & 1][Q + 2 * q + v] = *reinterpret_cast<const f32x4*>(cs + D / 2 + 32 * q + 4 * v);
+        }
+    };
+    ask(0);
+    ask(1);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float a = x[q][4 * v + e], b = x[q + Q / 2][4 * v + e];
-            x[q][4 * v + e] = __fsub_rn(__fmul_rn(a, co[e]), __fmul_rn(b, si[e]));
-            x[q + Q / 2][4 * v + e] = __fadd_rn(__fmul_rn(b, co[e]), __fmul_rn(a, si[e]));
+    for (int r = 0; r < 8; ++r) {
+      __builtin_amdgcn_sched_barrier(0);
+      const int64_t t = at.lo + 128 * (r >> 2) + 64 * wm + 16 * (r & 3) + fr;
+      u32x4 out[4];
+#pragma unroll
+      for (int h = 0; h < HEADS; ++h) {
+        f32x4 a[2 * Q];
+#pragma unroll
+        for (int j = 0; j < 2 * Q; ++j) a[j] = deep_take(r >> 2, 2 * Q * h + j, r & 3);
+        float x[Q][8];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+          float w[8];
+          if (p.bias) widen(*reinterpret_cast<const u32x4*>(extra + 2048 + 2 * (n0 - at.n0 + D * h + 32 * q + c)), w);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[q][e] = rounded(a[2 * q + (e >> 2)][e & 3] + (p.bias ? w[e] : 0.0f));
+        }
+        if (ra.qn_w && (is_q[h] || is_k[h])) {
+          float ss = 0.f;
+#pragma unroll
+          for (int q = 0; q < Q; ++q)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += x[q][e] * x[q][e];
+          float even, odd, lower, upper;
+          rows_pair16(ss, even, odd);
+          rows_pair32(even + odd, lower, upper);
+          const float inv = 1.0f / sqrtf((lower + upper) / (float)D + ra.eps);
+#pragma unroll
+          for (int q = 0; q < Q; ++q) {
+            float w[8];
+            widen(*reinterpret_cast<const u32x4*>(extra + (is_q[h] ? 2560 : 2816) + 2 * (32 * q + c)), w);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[q][e] = rounded(rounded(x[q][e] * inv) * w[e]);
           }
         }
-      }
-    }
-    uint16_t* cache = nullptr;
-    if (!is_q && slot >= 0 && ra.k_cache)
-      cache = (is_k ? ra.k_cache : ra.v_cache) + ((int64_t)slot * ra.Hkv + (hs - ra.H - (is_k ? 0 : ra.Hkv))) * D;
+        if (is_q[h] || is_k[h]) {
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      const u32x4 v = pack(x[q]);
-      *reinterpret_cast<u32x4*>(row + n + 32 * q + c) = v;
-      if (cache) *reinterpret_cast<u32x4*>(cache + 32 * q + c) = v;
+          for (int q = 0; q < Q / 2; ++q)
+#pragma unroll
+            for (int v = 0; v < 2; ++v) {
+              const f32x4 co = turn[r & 1][2 * q + v], si = turn[r & 1][Q + 2 * q + v];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const float lo = x[q][4 * v + e], hi = x[q + Q / 2][4 * v + e];
+                x[q][4 * v + e] = __fsub_rn(__fmul_rn(lo, co[e]), __fmul_rn(hi, si[e]));
+                x[q + Q / 2][4 * v + e] = __fadd_rn(__fmul_rn(hi, co[e]), __fmul_rn(lo, si[e]));
+              }
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) out[h * Q + q] = pack(x[q]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (r + 2 < 8) ask(r + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      if (t >= at.hi || !(r < 4 ? live0 : live1)) continue;
+      uint16_t* row = reinterpret_cast<uint16_t*>(p.out) + t * p.os + n0 + c;
+#pragma unroll
+      for (int h = 0; h < HEADS; ++h) {
+        if (n0 + D * h >= p.N) continue;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) *reinterpret_cast<u32x4*>(row + D * h + 32 * q) = out[h * Q + q];
+        if (is_q[h] || !ra.k_cache) continue;
+        const int slot = (int)kept(r, 1);
+        if (slot < 0) continue;
+        uint16_t* cache = (is_k[h] ? ra.k_cache : ra.v_cache) + ((int64_t)slot * ra.Hkv + (hs[h] - ra.H - (is_k[h] ? 0 : ra.Hkv))) * D + c;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) *reinterpret_cast<u32x4*>(cache + 32 * q) = out[h * Q + q];
+      }
     }
   }
 };
 
-template <typename T, int WHAT, int D, bool TILED>
+template <typename T, int WHAT, int D, bool TILED, bool FAR>
 hipError_t rows_go_as(const RowsArgs& p, const RopeArgs& ra, hipStream_t s) {
-  typedef RowsJob<T, WHAT, D, TILED> Job;
+  typedef RowsJob<T, WHAT, D, TILED, FAR> Job;
   const int n = WHAT == ROWS_SILU ? p.N / 2 : p.N;
   const Job job{p, ra, p.K, (p.M + STREAM_BM - 1) / STREAM_BM, (n + Job::NOUT - 1) / Job::NOUT};
-  return launch_stream_tiles<Job::WN>(job, (int64_t)job.rows * job.cols, s);
+  return launch_stream_deep(job, (int64_t)job.rows * job.cols, s);
 }
 template <typename T, int WHAT, int D>
 hipError_t rows_go(const RowsArgs& p, const RopeArgs& ra, hipStream_t s) {
-  return p.tiled ? rows_go_as<T, WHAT, D, true>(p, ra, s) : rows_go_as<T, WHAT, D, false>(p, ra, s);
+  if (p.xs >= (1 << 22) || p.K >= (1 << 22))
+    return p.tiled ? rows_go_as<T, WHAT, D, true, true>(p, ra, s) : rows_go_as<T, WHAT, D, false, true>(p, ra, s);
+  return p.tiled ? rows_go_as<T, WHAT, D, true, false>(p, ra, s) : rows_go_as<T, WHAT, D, false, false>(p, ra, s);
 }
 
 template <typename T>

@@ -4,9 +4,19 @@
 #pragma once
 #include <type_traits>
 
-#include "stream_tiles.h"
+#include "linear_args.h"
+#include "stream_deep.h"
 
-// value(s) of one output -> what is stored (bias, activation, gate); `gate`: the row's, where there is one for all of it
+// value(s) of one output, bias and scale included -> what the epilogue makes of it; `gate`: the row's
+template <int EPI, int ACT = -1>
+__device__ __forceinline__ float lin_epilogue(const LinArgs& p, float v, float u, float gate) {
+  if constexpr (EPI == EPI_GLU) return glu_act(v, u, ACT < 0 ? p.act : ACT, p.epi_c);
+  else if constexpr (EPI == EPI_SOFTCAP) return p.epi_c * tanhf(v / p.epi_c);
+  else if constexpr (EPI == EPI_ROW_GATE) return v * gate;
+  else if constexpr (EPI == EPI_ACT) return unary_act(v, ACT < 0 ? p.act : ACT, p.epi_ptr, p.epi_c);
+  else return v;
+}
+// the same with scale, bias and gate taken from memory here
 template <typename T, int EPI, int ACT = -1>
 __device__ __forceinline__ float lin_finish(const LinArgs& p, const T* bias, float v, float u, float rsc, float gate, int64_t s, int n,
                                             int z) {
@@ -15,15 +25,10 @@ __device__ __forceinline__ float lin_finish(const LinArgs& p, const T* bias, flo
   if constexpr (EPI == EPI_GLU) {
     u *= rsc;
     if (bias) u += ld_f32<T>(bias + p.N + n);
-    v = glu_act(v, u, p.act, p.epi_c);
-  } else if constexpr (EPI == EPI_SOFTCAP) {
-    v = p.epi_c * tanhf(v / p.epi_c);
-  } else if constexpr (EPI == EPI_ROW_GATE) {
-    v *= p.act ? sigmoid_f32(p.epi_ptr[s * p.epi_rs + (int64_t)z * p.N + n]) : gate;
-  } else if constexpr (EPI == EPI_ACT) {
-    v = unary_act(v, ACT < 0 ? p.act : ACT, p.epi_ptr, p.epi_c);
   }
-  return v;
+  if constexpr (EPI == EPI_ROW_GATE)
+    if (p.act) gate = sigmoid_f32(p.epi_ptr[s * p.epi_rs + (int64_t)z * p.N + n]);
+  return lin_epilogue<EPI, ACT>(p, v, u, gate);
 }
 
 // eight consecutive results of one row -> 16 bytes
@@ -102,52 +107,181 @@ struct LinearJob {
   __device__ __forceinline__ bool whole(const StreamTile& at) const {
     return vec && at.lo + BM <= at.hi && at.n0 + NOUT <= p.N;
   }
-  __device__ __forceinline__ void store(const StreamTile& at, int64_t row0, int wn, int lane, const f32x4 (&acc)[NT][MT]) const {
+  static constexpr int NSTORE_WAVE = 2 * NSTORE, EXTRA = 0;
+  static constexpr bool FAR_A = true, FAR_W = false;      // A's rows may lie anywhere; W: stream_takes
+  __device__ __forceinline__ void fetch_extra(const StreamTile&, int, int, unsigned char*) const {}
+  __device__ __forceinline__ void finish(const StreamTile& at, int wm, int wn, int lane, bool live0, bool live1, const unsigned char*) const {
+    if (live0) store_wave<0>(at, at.lo + 64 * wm, wn, lane);
+    if (live1) store_wave<1>(at, at.lo + 128 + 64 * wm, wn, lane);
+  }
+  // 64 rows by 128 rows of W of stream_deep.h.  What the results need of memory is fetched ahead of the first store: loads and stores
+  // are counted in one order, so a load behind a store is waited for behind it too.
+  template <int HALF>
+  __device__ __forceinline__ void store_wave(const StreamTile& at, int row0, int wn, int lane) const {
+    if (!vec || (EPI == EPI_ROW_GATE && p.act)) {
+      store<4>(at, row0, 2 * wn, lane, [](int j, int i) { return deep_take(HALF, j, i); });
+      store<4>(at, row0, 2 * wn + 1, lane, [](int j, int i) { return deep_take(HALF, 4 + j, i); });
+      return;
+    }
+    if constexpr (EPI == EPI_NONE) {
+      if (!p.bias && !p.row_scale) return store_ahead<HALF, -1, false>(at, row0, wn, lane);
+    }
+    if constexpr (EPI == EPI_ACT || EPI == EPI_GLU) {
+      switch (p.act) {
+        case 0: return store_ahead<HALF, 0, true>(at, row0, wn, lane);
+        case 1: return store_ahead<HALF, 1, true>(at, row0, wn, lane);
+        case 2: return store_ahead<HALF, 2, true>(at, row0, wn, lane);
+      }
+    }
+    if constexpr (EPI == EPI_ACT) {
+      if (p.act == 4) return store_ahead<HALF, 4, true>(at, row0, wn, lane);
+      return store_ahead<HALF, 3, true>(at, row0, wn, lane);
+    } else if constexpr (EPI != EPI_GLU) {
+      store_ahead<HALF, -1, true>(at, row0, wn, lane);
+    }
+  }
+  template <int HALF, int ACT, bool MORE>      // MORE: scale, bias or gate; 1 and -0, which change nothing, where there is none
+  __device__ __forceinline__ void store_ahead(const StreamTile& at, int row0, int wn, int lane) const {
+    constexpr int LEN = PAIRED ? 8 : 4, PIECES = (GLU ? 2 : 4) * 4 / LEN, UP = 2;
+    const int fr = lane & 15, g = lane >> 4;
+    float rsc[4], gate[4], bias[2][PIECES * LEN], up[GLU ? 2 : 1][GLU ? PIECES * LEN : 1];
+    int n[2][PIECES];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int q = 0; q < PIECES; ++q) n[h][q] = at.n0 + (GLU ? 32 : 64) * (2 * wn + h) + 4 * LEN * q + LEN * g;
+    if constexpr (MORE) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) rsc[i] = gate[i] = 1.0f;
+      if (p.row_scale) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rsc[i] = p.row_scale[min(row0 + 16 * i + fr, at.hi - 1)];
+      }
+      if constexpr (EPI == EPI_ROW_GATE) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gate[i] = p.epi_ptr[min(row0 + 16 * i + fr, at.hi - 1) * p.epi_rs + at.z];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gate[i] = sigmoid_f32(gate[i]);
+      }
+      // one branch for all of them, or each is waited for by itself
+      if (p.bias) {
+        const T* from = reinterpret_cast<const T*>(p.bias) + at.z * p.bias_bs;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int q = 0; q < PIECES; ++q)
+#pragma unroll
+            for (int e = 0; e < LEN; ++e) {
+              const int at_n = min(n[h][q], p.N - LEN) + e;
+              bias[h][q * LEN + e] = ld_f32<T>(from + at_n);
+              if constexpr (GLU) up[h][q * LEN + e] = ld_f32<T>(from + p.N + at_n);
+            }
+      } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int e = 0; e < PIECES * LEN; ++e) {
+            bias[h][e] = -0.0f;
+            if constexpr (GLU) up[h][e] = -0.0f;
+          }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(rsc[i]), "+v"(gate[i]));      // all of them waited for here
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < PIECES * LEN; ++e) {
+          asm volatile("" : "+v"(bias[h][e]));
+          if constexpr (GLU) asm volatile("" : "+v"(up[h][e]));
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int64_t s = row0 + 16 * i + fr;
+      TO* o = reinterpret_cast<TO*>(p.out) + at.z * p.out_bs + s * p.out_rs;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        __builtin_amdgcn_sched_barrier(0);       // one row's results at a time: registers
+        f32x4 x[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = deep_take(HALF, 4 * h + j, i);
+#pragma unroll
+        for (int q = 0; q < PIECES; ++q) {
+          float v[LEN];
+#pragma unroll
+          for (int e = 0; e < LEN; ++e) {
+            const int j = q * (LEN / 4) + e / 4;
+            float a = x[j][e & 3], u = GLU ? x[(j + UP) % NT][e & 3] : 0.0f;
+            if constexpr (MORE) {
+              a = a * rsc[i] + bias[h][q * LEN + e];
+              if constexpr (GLU) u = u * rsc[i] + up[h][q * LEN + e];
+            }
+            v[e] = lin_epilogue<EPI, ACT>(p, a, u, MORE ? gate[i] : 1.0f);
+          }
+          if (s < at.hi && n[h][q] < p.N) {
+            if constexpr (PAIRED) *reinterpret_cast<u32x4*>(o + n[h][q]) = pack8(v);
+            else *reinterpret_cast<f32x4*>(o + n[h][q]) = f32x4{v[0], v[1], v[2], v[3]};
+          }
+        }
+      }
+    }
+  }
+  template <int ROWS, typename Take>
+  __device__ __forceinline__ void store(const StreamTile& at, int64_t row0, int wn, int lane, Take take) const {
     if constexpr (EPI == EPI_ACT) {      // one function per copy: with the choice inside, the loops would not unroll
       switch (p.act) {
-        case 0: return store_as<0>(at, row0, wn, lane, acc);
-        case 1: return store_as<1>(at, row0, wn, lane, acc);
-        case 2: return store_as<2>(at, row0, wn, lane, acc);
-        case 4: return store_as<4>(at, row0, wn, lane, acc);
-        default: return store_as<3>(at, row0, wn, lane, acc);
+        case 0: return store_as<0, ROWS>(at, row0, wn, lane, take);
+        case 1: return store_as<1, ROWS>(at, row0, wn, lane, take);
+        case 2: return store_as<2, ROWS>(at, row0, wn, lane, take);
+        case 4: return store_as<4, ROWS>(at, row0, wn, lane, take);
+        default: return store_as<3, ROWS>(at, row0, wn, lane, take);
       }
     } else {
-      store_as<-1>(at, row0, wn, lane, acc);
+      store_as<-1, ROWS>(at, row0, wn, lane, take);
+    }
+  }
+  template <int ACT, int ROWS, typename Take>
+  __device__ __forceinline__ void store_as(const StreamTile& at, int64_t row0, int wn, int lane, Take take) const {
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+      __builtin_amdgcn_sched_barrier(0);       // one row's results at a time: registers
+      f32x4 x[NT];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) x[j] = take(j, i);
+      const int64_t s = row0 + 16 * i + (lane & 15);
+      if (s < at.hi) store_row<ACT>(at, s, wn, lane, x);
     }
   }
   template <int ACT>
-  __device__ __forceinline__ void store_as(const StreamTile& at, int64_t row0, int wn, int lane, const f32x4 (&acc)[NT][MT]) const {
-    const int fr = lane & 15, g = lane >> 4;
-    TO* O = reinterpret_cast<TO*>(p.out) + at.z * p.out_bs;
+  __device__ __forceinline__ void store_row(const StreamTile& at, int64_t s, int wn, int lane, const f32x4 (&x)[NT]) const {
+    const int g = lane >> 4;
     const T* bias = p.bias ? reinterpret_cast<const T*>(p.bias) + at.z * p.bias_bs : nullptr;
     constexpr int LEN = PAIRED ? 8 : 4, PIECES = (GLU ? 2 : 4) * 4 / LEN, UP = 2;
+    float rsc = 1.0f;
+    if (p.row_scale) {
+      rsc = p.row_scale[s];
+      asm volatile("" : "+v"(rsc));       // waited for here: pending on a path without its use, it would be waited for in the loop over blocks
+    }
+    const float gate = EPI == EPI_ROW_GATE && !p.act ? sigmoid_f32(p.epi_ptr[s * p.epi_rs + at.z]) : 1.0f;
+    auto result = [&](int q, int e, int n) {
+      const int j = q * (LEN / 4) + e / 4;
+      return lin_finish<T, EPI, ACT>(p, bias, x[j][e & 3], GLU ? x[(j + UP) % NT][e & 3] : 0.0f, rsc, gate, s, n + e, at.z);
+    };
+    TO* o = reinterpret_cast<TO*>(p.out) + at.z * p.out_bs + s * p.out_rs;
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      __builtin_amdgcn_sched_barrier(0);       // one row's results at a time: registers
-      const int64_t s = row0 + 16 * i + fr;
-      if (s >= at.hi) continue;
-      const float rsc = p.row_scale ? p.row_scale[s] : 1.0f;
-      const float gate = EPI == EPI_ROW_GATE && !p.act ? sigmoid_f32(p.epi_ptr[s * p.epi_rs + at.z]) : 1.0f;
-      auto result = [&](int q, int e, int n) {
-        const int j = q * (LEN / 4) + e / 4;
-        return lin_finish<T, EPI, ACT>(p, bias, acc[j][i][e & 3], GLU ? acc[(j + UP) % NT][i][e & 3] : 0.0f, rsc, gate, s, n + e, at.z);
-      };
-      TO* o = O + s * p.out_rs;
+    for (int q = 0; q < PIECES; ++q) {
+      const int n = at.n0 + (GLU ? 32 : 64) * wn + 4 * LEN * q + LEN * g;
+      if (vec) {
+        if (n >= p.N) continue;
+        float v[LEN];
 #pragma unroll
-      for (int q = 0; q < PIECES; ++q) {
-        const int n = at.n0 + (GLU ? 32 : 64) * wn + 4 * LEN * q + LEN * g;
-        if (vec) {
-          if (n >= p.N) continue;
-          float v[LEN];
+        for (int e = 0; e < LEN; ++e) v[e] = result(q, e, n);
+        if constexpr (PAIRED) *reinterpret_cast<u32x4*>(o + n) = pack8(v);
+        else *reinterpret_cast<f32x4*>(o + n) = f32x4{v[0], v[1], v[2], v[3]};
+      } else {
 #pragma unroll
-          for (int e = 0; e < LEN; ++e) v[e] = result(q, e, n);
-          if constexpr (PAIRED) *reinterpret_cast<u32x4*>(o + n) = pack8(v);
-          else *reinterpret_cast<f32x4*>(o + n) = f32x4{v[0], v[1], v[2], v[3]};
-        } else {
-#pragma unroll
-          for (int e = 0; e < LEN; ++e)
-            if (n + e < p.N) st_f32<TO>(o + n + e, result(q, e, n));
-        }
+        for (int e = 0; e < LEN; ++e)
+          if (n + e < p.N) st_f32<TO>(o + n + e, result(q, e, n));
       }
     }
   }
@@ -157,15 +291,19 @@ struct LinearJob {
 inline bool stream_takes(const LinArgs& p, int esz, int64_t total_rows, int batch, int cols) {
   const int64_t rows = p.group_off ? total_rows / 256 + batch : (p.M + 255) / 256 * batch;
   if (total_rows >= ((int64_t)1 << 31) || rows * ((cols + 255) / 256) > 256 * (STREAM_LIST - 2)) return false;
+  // a 16-bit tile's rows of W lie within 4 GiB of its first (the ups of a gated one N rows behind it)
+  if (esz == 2 && (cols + 256) * p.w_rs * esz >= ((int64_t)1 << 32)) return false;
   return p.K * esz >= 256 && p.K * esz % 128 == 0 && p.a_rs >= 0 && p.w_rs >= 0 && p.a_rs < ((int64_t)1 << 30) && p.w_rs < ((int64_t)1 << 30);
 }
 
 template <typename T, typename TO, int EPI>
-hipError_t launch_stream_epi(const LinArgs& p, int64_t total_rows, int batch, hipStream_t s) {
+LinearJob<T, TO, EPI> linear_job(const LinArgs& p, int batch) {
   typedef LinearJob<T, TO, EPI> Job;
   constexpr int64_t unit = sizeof(TO) == 2 ? 8 : 4;
   const int nt = (p.N + Job::NOUT - 1) / Job::NOUT;
   const int vec = p.N % unit == 0 && p.out_rs % unit == 0 && p.out_bs % unit == 0 && (uintptr_t)p.out % 16 == 0;
-  const Job job{p, p.K, p.group_off ? batch : 0, batch, nt, vec};
-  return launch_stream_tiles<4>(job, (p.group_off ? total_rows / Job::BM + batch : (p.M + Job::BM - 1) / Job::BM * batch) * nt, s);
+  return Job{p, p.K, p.group_off ? batch : 0, batch, nt, vec};
+}
+inline int64_t linear_job_tiles(const LinArgs& p, int nt, int64_t total_rows, int batch) {      // at most
+  return (p.group_off ? total_rows / STREAM_BM + batch : (p.M + STREAM_BM - 1) / STREAM_BM * batch) * nt;
 }

@@ -287,7 +287,14 @@ inline int pick_wide_tile(int64_t m, int64_t total_rows, int cols, int K, int ba
 
 template <typename T, typename TO, int EPI>
 hipError_t launch_wide_epi(const LinArgs& p, int64_t total_rows, int batch, int tile, hipStream_t s) {
-  if (tile == TILE_256) return launch_stream_epi<T, TO, EPI>(p, total_rows, batch, s);
+  if (tile == TILE_256) {
+    if constexpr (sizeof(T) == 2) {
+      return linear_deep_launch(p, EPI, sizeof(TO) == 2, total_rows, batch, s);
+    } else {
+      const auto job = linear_job<T, TO, EPI>(p, batch);
+      return launch_stream_tiles(job, linear_job_tiles(p, job.nt, total_rows, batch), s);
+    }
+  }
   if (tile == TILE_128) return launch_wide_one<T, TO, EPI, 2, 2, 2, 2>(p, total_rows, batch, s);
   return launch_wide_one<T, TO, EPI, 1, 2, 2, 3>(p, total_rows, batch, s);
 }

@@ -110,11 +110,11 @@ __device__ __forceinline__ int stream_lane() {
   return (int)__builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0));
 }
 
-template <int WN, typename Job>
+template <typename Job>
 __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef typename Job::T T;
-  constexpr int WM = 8 / WN, MT = STREAM_BM / 16 / WM, NT = STREAM_BN / 16 / WN;
+  constexpr int WN = 4, WM = 8 / WN, MT = STREAM_BM / 16 / WM, NT = STREAM_BN / 16 / WN;
   typedef typename Job::Order Order;
   constexpr int BM = STREAM_BM, BN = STREAM_BN, BO = STREAM_BUFFER;     // BO: bytes of one buffer
   constexpr int AG = BM / 64, WG = BN / 64, D = AG + WG;                // DMA instructions (8 rows each) of a wavefront per block
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
     left = blocks;
     if (live) {
   
-      job.store(at, at.lo + 16 * MT * wm, wn, stream_lane(), acc);
+      job.template store<MT>(at, at.lo + 16 * MT * wm, wn, stream_lane(), [&](int j, int i) { return acc[j][i]; });
       stored = job.whole(at);
       clear();
     }
@@ -301,14 +301,14 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
 #endif
 }
 
-template <int WN, typename Job>
+template <typename Job>
 hipError_t launch_stream_tiles(const Job& job, int64_t max_tiles, hipStream_t s) {
   constexpr size_t lds = 2 * STREAM_BUFFER + STREAM_LIST * sizeof(StreamTile);
   static std::atomic<uint64_t> devices{0};
-  const hipError_t e = allow_lds(reinterpret_cast<const void*>(&stream_tiles_kernel<WN, Job>), lds, devices);
+  const hipError_t e = allow_lds(reinterpret_cast<const void*>(&stream_tiles_kernel<Job>), lds, devices);
   if (e != hipSuccess) return e;
   // with few tiles there is a workgroup for each half of one
   const unsigned grid = (unsigned)(max_tiles < 128 ? (2 * max_tiles + 7) / 8 * 8 : 256);
-  stream_tiles_kernel<WN, Job><<<dim3(grid), dim3(512), lds, s>>>(job);
+  stream_tiles_kernel<Job><<<dim3(grid), dim3(512), lds, s>>>(job);
   return hipGetLastError();
 }
