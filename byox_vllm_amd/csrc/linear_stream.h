@@ -216,7 +216,8 @@ struct LinearJob {
               a = a * rsc[i] + bias[h][q * LEN + e];
               if constexpr (GLU) u = u * rsc[i] + up[h][q * LEN + e];
             }
-            v[e] = lin_epilogue<EPI, ACT>(p, a, u, MORE ? gate[i] : 1.0f);
+            if constexpr (GLU && ACT == 0 && PAIRED) v[e] = silu_16bit(a) * u;
+            else v[e] = lin_epilogue<EPI, ACT>(p, a, u, MORE ? gate[i] : 1.0f);
           }
           if (s < at.hi && n[h][q] < p.N) {
             if constexpr (PAIRED) *reinterpret_cast<u32x4*>(o + n[h][q]) = pack8(v);

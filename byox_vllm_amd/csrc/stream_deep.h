@@ -10,8 +10,9 @@
 //     (2816 cycles of products; the form before had 1000 - 2000).  The order of products, LDS reads and DMA is fixed in the source;
 //   * DMA a few at a time: eight products between two instructions; eight of them two apart queue up (8192^3: 756 against 730 us);
 //   * no branch between products in the loop for whole tiles (8192^3: 756 with one per half block, 710 without), and no vector address that
-//     moves with K: the tile's rows are offsets, K is in the scalar base.  A tile's first pair of blocks, where stores are still on their
-//     way, and tiles with wavefronts that have no rows take the other loop;
+//     moves with K: the tile's rows are offsets, K is in the scalar base.  A tile's first pair of blocks, whose products are
+//     added to nothing (256 registers less to clear) while stores are still on their way, and tiles with wavefronts that have no rows take
+//     the other loop;
 //   * a wavefront has rows 64 of each half of the tile, so a half of 128 rows, or a ragged tile, is half the work for each of them.
 // Results are those of stream_tiles.h, bit for bit: K in the same order.  Measured, before and after (us): the experts' layer of 16384 rows,
 // 2048 -> 2 x 3072 -> 2048, 1424 and 1185; 16384 rows 2048 -> 2 x 6144 with SiLU 738 and 646; 2048 -> 6144 into fp32 376 and 327; 14600
@@ -46,14 +47,18 @@
       "a224", "a225", "a226", "a227", "a228", "a229", "a230", "a231", "a232", "a233", "a234", "a235", "a236", "a237", "a238", "a239", \
       "a240", "a241", "a242", "a243", "a244", "a245", "a246", "a247", "a248", "a249", "a250", "a251", "a252", "a253", "a254", "a255"
 __device__ __forceinline__ constexpr int deep_at(int h, int j, int i) { return 4 * (32 * h + 4 * j + i); }
+template <bool NEW = false>      // NEW: the accumulators' first product, added to nothing
 __device__ __forceinline__ void deep_mma(int at, const u32x4& w, const u32x4& a, bf16_t) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], %0, %1, a[%2:%3]" ::"v"(w), "v"(a), "i"(at), "i"(at + 3));
+  if constexpr (NEW) asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], %0, %1, 0" ::"v"(w), "v"(a), "i"(at), "i"(at + 3));
+  else asm volatile("v_mfma_f32_16x16x32_bf16 a[%2:%3], %0, %1, a[%2:%3]" ::"v"(w), "v"(a), "i"(at), "i"(at + 3));
 #endif
 }
+template <bool NEW = false>      // NEW: the accumulators' first product, added to nothing
 __device__ __forceinline__ void deep_mma(int at, const u32x4& w, const u32x4& a, f16_t) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("v_mfma_f32_16x16x32_f16 a[%2:%3], %0, %1, a[%2:%3]" ::"v"(w), "v"(a), "i"(at), "i"(at + 3));
+  if constexpr (NEW) asm volatile("v_mfma_f32_16x16x32_f16 a[%2:%3], %0, %1, 0" ::"v"(w), "v"(a), "i"(at), "i"(at + 3));
+  else asm volatile("v_mfma_f32_16x16x32_f16 a[%2:%3], %0, %1, a[%2:%3]" ::"v"(w), "v"(a), "i"(at), "i"(at + 3));
 #endif
 }
 __device__ __forceinline__ f32x4 deep_take(int h, int j, int i) {
@@ -161,12 +166,6 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
     const int s = r >> 2, j = r & 3;
     fw[h][j][s] = *reinterpret_cast<const u32x4*>(lds_raw + bo + 2 * DEEP_PA + h * DEEP_PW + wat[s] + Order::off(j));
   };
-  auto clear = [&]() {
-#pragma unroll
-    for (int r = 0; r < 256; ++r) asm volatile("v_accvgpr_write_b32 a[%0], 0" ::"i"(r));
-    asm volatile("s_nop 7" ::: "memory", DEEP_REGISTERS);
-  };
-  clear();
   auto extra = [&](int n) { return lds_raw + 2 * DEEP_BUFFER + STREAM_LIST * sizeof(StreamTile) + (n & 1) * Job::EXTRA; };
   const int blocks = job.K / 64, pairs = (blocks + 1) / 2;
   const bool odd = blocks & 1;
@@ -192,7 +191,7 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
   // read and the pieces of LDS that were read before the barrier are filled again, in this order.  What is waited for was asked for
   // three halves before: sixteen operations are younger, and a tile's stores where they came between (`behind`).
   constexpr int BEHIND = 16 + Job::NSTORE_WAVE < 63 ? 16 + Job::NSTORE_WAVE : 63;
-  auto half = [&](auto plain, auto bb, auto ss, bool live, bool behind) {
+  auto half = [&](auto plain, auto bb, auto ss, bool live, bool fresh, bool behind) {
     constexpr bool PLAIN = decltype(plain)::value;
     constexpr int B = decltype(bb)::value, S = decltype(ss)::value, X = B, Y = 1 - B;
     constexpr int here = B * DEEP_BUFFER, there = (1 - B) * DEEP_BUFFER;
@@ -218,35 +217,41 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
         else fill_a(here, 1, k - 4);
       }
     };
-    auto product = [&](int m) {
+    auto product = [&](int m, auto is_new) {
       const int hw = (m < 32) == (S == 0) ? X : Y, s = (m >> 4) & 1, j = (m >> 2) & 3, i = m & 3;
-      deep_mma(deep_at(S, 4 * hw + j, i), fw[hw][j][s], fa[S][i][s], T{});
+      deep_mma<decltype(is_new)::value>(deep_at(S, 4 * hw + j, i), fw[hw][j][s], fa[S][i][s], T{});
     };
     if constexpr (PLAIN) {
 #pragma unroll
       for (int m = 0; m < 64; ++m) {
-        product(m);
+        product(m, std::false_type{});
         __builtin_amdgcn_sched_barrier(0);
         reads(m);
         if (m % 8 == 3) fills(m / 8);
         __builtin_amdgcn_sched_barrier(0);
       }
     } else {      // what is not for all wavefronts has no results but in the accumulators: nothing to be merged behind it
+      auto quarter = [&](int from) {
+        if (!live) return;
+        if (B == 0 && fresh) {
+#pragma unroll
+          for (int m = 0; m < 16; ++m) product(from + m, std::true_type{});
+        } else {
+#pragma unroll
+          for (int m = 0; m < 16; ++m) product(from + m, std::false_type{});
+        }
+#pragma unroll
+        for (int m = 16; m < 32; ++m) product(from + m, std::false_type{});
+      };
 #pragma unroll
       for (int m = 0; m < 32; ++m) reads(m);
 #pragma unroll
       for (int k = 0; k < 8; ++k) fills(k);
-      if (live) {
-#pragma unroll
-        for (int m = 0; m < 32; ++m) product(m);
-      }
+      quarter(0);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int m = 32; m < 64; ++m) reads(m);
-      if (live) {
-#pragma unroll
-        for (int m = 32; m < 64; ++m) product(m);
-      }
+      quarter(32);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -268,16 +273,16 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
   };
   for (;;) {
     // Each way reads its first fragments itself: handed from one to the other they would be moved between registers.
-    if (live0 && live1 && !stored && !odd) {
+    if (live0 && live1 && !odd && left < pairs) {
       const std::true_type plain;
       first();
       for (; left > 0; --left) {
         ask_ahead();
-        half(plain, I0, I0, true, false);
-        half(plain, I0, I1, true, false);
+        half(plain, I0, I0, true, false, false);
+        half(plain, I0, I1, true, false, false);
         next_block();
-        half(plain, I1, I0, true, false);
-        half(plain, I1, I1, true, false);
+        half(plain, I1, I0, true, false, false);
+        half(plain, I1, I1, true, false, false);
         next_block();
       }
     } else {
@@ -285,16 +290,16 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
       asm volatile("; not all" ::: "memory");      // or the reads of both ways become one, ahead of them
       first();
       ask_ahead();
-      half(plain, I0, I0, live0, stored);
-      half(plain, I0, I1, live1, stored);
+      half(plain, I0, I0, live0, left == pairs, stored);
+      half(plain, I0, I1, live1, left == pairs, stored);
       next_block();
       if (odd && left == 2) {      // the last pair has no second block: the first one again, unused
         abase -= 128;
         wbase -= w_step;
       }
       const bool full = !odd || left > 1;
-      half(plain, I1, I0, live0 && full, stored);
-      half(plain, I1, I1, live1 && full, false);
+      half(plain, I1, I0, live0 && full, false, stored);
+      half(plain, I1, I1, live1 && full, false, false);
       next_block();
       stored = false;
       --left;
@@ -302,9 +307,8 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
     if (left > 0) continue;
     left = pairs;
     asm volatile("s_nop 15\n\ts_nop 7" ::: "memory", DEEP_REGISTERS);      // the last products are through the matrix cores
-    job.finish(at, wm, wn, lane, live0, live1, extra(tile));
+    job.finish(at, wm, wn, stream_lane(), live0, live1, extra(tile));
     stored = job.whole(at);
-    clear();
     if (++tile == tiles) break;
     at = ahead;
     live0 = at.lo + 64 * wm < at.hi;
