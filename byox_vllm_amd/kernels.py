@@ -644,8 +644,7 @@ def linear(x, w, bias=None, out=None, out_dtype=None, *, rows=None, a_rows=None,
     #  * those with an epilogue that fill its rounds of 256 x 256 tiles (16384 rows 2048 -> 2 x 4096, SiLU, share 1.0: 489 us, the
     #    library and a pass 588; 6000 rows 4096 -> 2 x 1024, 0.73: 107 and 92; 4100 rows 1024 -> 1024, 0.29: 42 and 26; of 650 shapes
     #    above the line one is more than 3 % slower, by 3.1);
-    #  * plain ones of a short K whose columns do not split into the library's tiles (12300 rows 1024 -> 3088, share 0.79: 95 and 110;
-    #    5500 rows, 0.55: a layer 136 and 129; 12300 rows 2048 -> 4112: 325 and 290).
+    #  * plain ones where linear_streams says so.
     if (epilogue in (EPI_NONE, EPI_GLU, EPI_ACT) and M >= MANY_ROWS and batch == 1 and group_offsets is None and a_rows is None
             and (bias is None or (epilogue != EPI_NONE and (out_dtype or x.dtype) == x.dtype)) and out is None
             and row_scale is None and rows is None and x.dtype == torch.bfloat16
@@ -654,7 +653,7 @@ def linear(x, w, bias=None, out=None, out_dtype=None, *, rows=None, a_rows=None,
             and n % 8 == 0 and x.data_ptr() % 16 == 0):
         cols = 2 * n if epilogue == EPI_GLU else n
         if epilogue == EPI_NONE:
-            if not (K <= 1024 and n > 1024 and n % 256 and M <= LINEAR_ROWS and tile_share(M, n) >= 0.7):
+            if not linear_streams(M, n, K, out_dtype or x.dtype):
                 return _linear_many_rows(x, w, M, n, K, out_dtype or x.dtype)
         elif M > LINEAR_ROWS or tile_share(M, cols) < (0.7 if K <= 512 else 0.8):
             assert bias is None or (bias.dtype == x.dtype and bias.numel() == cols and bias.is_contiguous())
@@ -692,6 +691,23 @@ def linear(x, w, bias=None, out=None, out_dtype=None, *, rows=None, a_rows=None,
                                out_batch_stride, bias_stride, ptr(group_offsets), epilogue, act, ptr(gate), gate_stride,
                                cap, ptr(row_scale), M, _code32(x.dtype), stream()), "nv_linear_rows")
     return out
+
+
+def linear_streams(M, n, K, out_dtype) -> bool:
+    """Whether nv_linear forms a plain product of MANY_ROWS rows and more instead of the vendor library.  Both, us, library first:
+     * widths that do not split into the library's tiles, from a share of 0.7 (tile_share), 0.78 beyond K = 1024: 12300 rows 1024 -> 3088 into
+       fp32, share 0.79, 107 and 88; 16384 rows 2048 -> 4112, 0.83, 314 and 277; 6000 rows 1024 -> 3088, 0.60, 56 and 57.  Of 192 shapes of K
+       256 to 4096 above the line one is over 3 % slower (3.3), the mean is 1.36x;
+     * others only into fp32, which costs the library more beside 16 bits: K 512 to 1023 from a share of 0.7 (8192 rows 512 -> 4096: 56 and 45),
+       beyond 0.9 and up to 6144 columns (16384 rows 2048 -> 6144: 340 and 324, 2048 -> 2048 116 and 107; 24000 rows 1024 -> 8192 411 and 441).  Of
+       91 above the line one is 4 % slower, the mean is 1.13x.
+    """
+    if M > LINEAR_ROWS or n <= 1024 and n % 256:
+        return False
+    share = tile_share(M, n)
+    if n % 256:
+        return share >= (0.7 if K <= 1024 else 0.78)
+    return out_dtype == torch.float32 and K >= 512 and n <= 6144 and share >= (0.7 if K < 1024 else 0.9)
 
 
 def tile_share(M, n) -> float:
