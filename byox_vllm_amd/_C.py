@@ -129,6 +129,7 @@ _PROTOS = {
                                          _f, _i, _i, _p, _p, _i64, _i, _p, _sz, _i, _p]),
     "nv_qk_rotate_store": (_i, [_p, _p, _i64, _i, _i, _i, _p, _p, _i, _p, _p, _f, _i, _p, _i, _i, _f, _p, _i64, _p, _f, _f, _p,
                                 _p, _p, _i64, _i, _i, _i, _i, _i, _p]),
+    "nv_qkv_stream": (_i, [_p, _i64, _p, _i64, _i, _i, _p, _p, _i, _f, _f, _p, _p, _p, _p, _i64, _p, _i, _i, _i, _i, _p]),
     "nv_qk_conv_store_ok": (_i, [_p, _i64, _i, _i, _i, _p, _p, _p, _i, _i, _i]),
     "nv_qk_conv_store": (_i, [_p, _i64, _i, _i, _i, _p, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i, _i, _i, _i, _i, _i, _f, _f,
                               _i, _p]),

@@ -10,6 +10,7 @@ quantised formats, drops the dense copy.
 import torch
 import torch.distributed as dist
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from byox_vllm_amd import kernels
 from byox_vllm_amd.layers.quant import LinearWeight
@@ -367,6 +368,12 @@ class RowParallelLinear(LinearBase):
         if collectives_on(self.tp_size):
             tp_all_reduce(y)
         return y
+
+
+def called_plainly(module: nn.Module, cls: type) -> bool:
+    """Whether ``module`` is a ``cls`` whose call can be left out: no subclass, no forward of its own, nobody's hooks."""
+    return type(module) is cls and "forward" not in module.__dict__ and not (
+        module._forward_hooks or module._forward_pre_hooks or _has_any_global_hook())
 
 
 class DenseLinear(nn.Module):

@@ -8,14 +8,15 @@ of the sequence stay visible, a partial rotation, and one output gate per head:
 Kept tokens keep their place in the sequence: keys are rotated once, by their own position, when they are cached.  Pairs
 are (2i, 2i + 1) when ``interleaved``, else (i, i + rot_dims/2).  Cache rows [k: G * dim | v: G * vdim] live in pages of the
 engine's BlockManager in the model dtype; q | k | v | g are one merged projection left in fp32; rotation, scores, softmax
-and gate are fp32 (csrc/window_attn.hip: nv_qk_rotate_store, nv_paged_softmax_attn).  A mixer whose weights serve several
+and gate are fp32 (csrc/window_attn.hip: nv_qk_rotate_store, nv_paged_softmax_attn; prompts of many rows rotate and store
+behind the projection itself, csrc/qk_stream.hip).  A mixer whose weights serve several
 layers keeps one cache per layer run (``add_run``)."""
 
 import torch
 from torch import nn
 
 from byox_vllm_amd import kernels
-from byox_vllm_amd.layers.linear import DenseLinear
+from byox_vllm_amd.layers.linear import DenseLinear, called_plainly
 from byox_vllm_amd.layers.rotary_embedding import scaled_inv_freq
 from byox_vllm_amd.layers.sink_attention import CacheRun
 from byox_vllm_amd.utils.context import get_context
@@ -47,13 +48,18 @@ class SlidingAttention(nn.Module):
     def forward(self, h: torch.Tensor, positions: torch.Tensor, run: int = 0) -> torch.Tensor:
         ctx, own = get_context(), self.runs[run]
         H, G, d, dv = self.heads, self.kv_heads, self.dim, self.vdim
-        proj = self.inp(h, out_dtype=torch.float32)
-        q = kernels.qk_rotate_store(proj, (0, H * d, (H + G) * d), positions, self.scale, ctx.slot_mapping, own.cache, H, G, d,
-                                    dv, inv_freq=self.inv_freq, rot_dims=self.rot_dims, interleaved=self.interleaved,
-                                    mscale=self.magnitude)
+        if called_plainly(self.inp, DenseLinear) and own.cache.dtype == h.dtype and own.cache.data_ptr() % 8 == 0 and \
+                kernels.qkv_streams(h, self.inp.weight, H, G, d, dv, self.rot_dims, self.interleaved):
+            q, gates = kernels.qkv_project_store(h, self.inp.weight.data, positions, self.scale, ctx.slot_mapping, own.cache, H, G, d, dv,
+                                                 inv_freq=self.inv_freq, rot_dims=self.rot_dims, mscale=self.magnitude)
+        else:
+            proj = self.inp(h, out_dtype=torch.float32)
+            q = kernels.qk_rotate_store(proj, (0, H * d, (H + G) * d), positions, self.scale, ctx.slot_mapping, own.cache, H, G, d,
+                                        dv, inv_freq=self.inv_freq, rot_dims=self.rot_dims, interleaved=self.interleaved,
+                                        mscale=self.magnitude)
+            gates = proj[:, self.inp.offset("g"):]
         out = torch.empty(h.size(0), H * dv, dtype=h.dtype, device=h.device)
-        g = self.inp.offset("g")
         kernels.paged_softmax_attn(q, own.cache, ctx.block_tables, ctx.cu_seqlens_q, ctx.past_lens, ctx.seq_of_token,
                                    ctx.max_seqlen_q, H, G, d, dv, own.block_size, out, window=self.window,
-                                   keep_first=self.keep_first, gate=proj[:, g:g + H], gate_per_head=True)
+                                   keep_first=self.keep_first, gate=gates[:, :H], gate_per_head=True)
         return self.o(out, out_dtype=torch.float32)

@@ -16,7 +16,6 @@ import os
 
 import torch
 from torch import nn
-from torch.nn.modules.module import _has_any_global_hook
 
 from byox_vllm_amd import kernels
 from byox_vllm_amd._C import W_DENSE_TILED
@@ -25,14 +24,9 @@ from byox_vllm_amd.layers.attention import Attention
 from byox_vllm_amd.layers.embed_head import ParallelLMHead, VocabParallelEmbedding
 from byox_vllm_amd.layers.layernorm import RMSNorm
 from byox_vllm_amd.layers.linear import MergedColumnParallelLinear, QKVParallelLinear, RowParallelLinear
+from byox_vllm_amd.layers.linear import called_plainly as plain
 from byox_vllm_amd.layers.rotary_embedding import get_rope
 from byox_vllm_amd.utils.context import get_context
-
-
-def plain(module: nn.Module, cls: type) -> bool:
-    """Whether ``module`` is a ``cls`` whose call can be left out: no subclass, no forward of its own, nobody's hooks."""
-    return type(module) is cls and "forward" not in module.__dict__ and not (
-        module._forward_hooks or module._forward_pre_hooks or _has_any_global_hook())
 
 
 class Qwen3Attention(nn.Module):

@@ -105,7 +105,7 @@ class VasonexLayer(nn.Module):
 class VasonexForCausalLM(nn.Module):
     portioned = True          # steps through ModelRunner.run_portions: prompt pieces and decoded tokens in one batch
     prefix_cache = False      # portions extend a request's own pages; they do not look for another request's
-    kernel_sources = ("linear", "rowops", "window_attn", "moe", "misc", "gemm_lt")
+    kernel_sources = ("linear", "rowops", "window_attn", "qk_stream", "moe", "misc", "gemm_lt")
 
     @staticmethod
     def config_from_json(raw: dict, path: str | None):

@@ -655,6 +655,14 @@ int nv_qk_rotate_store(const float* proj, const void* bias, int64_t proj_row_str
                        const float* v_first, int64_t v_first_row_stride, const void* vmix, float scale, float eps,
                        const int32_t* slot_mapping, void* cache, float* q_out, int64_t tokens, int heads, int kv_heads,
                        int dim, int vdim, int dtype, nv_stream_t stream);
+/* The projection, rotation and store in one pass for many tokens (bf16): x [tokens, K] by w [N, K], whose rows are heads * dim queries, kv_heads
+ * * dim keys, kv_heads * vdim values and any others -> fp32 queries times scale in q_out [tokens, heads * dim], cache rows [k | v] of
+ * slot_mapping (negative: none), the other columns fp32 in rest [tokens, rest_row_stride].  The first rot_dims (0, 32, 64 or 128) numbers of
+ * every query and key head turn, i with i + rot_dims / 2; turns: room for tokens * rot_dims fp32.  dim 64 or 128, kv_heads * vdim a multiple
+ * of 16, K a multiple of 64 from 128 on; x, w, q_out and turns 16-byte aligned, cache 8. */
+int nv_qkv_stream(const void* x, int64_t x_row_stride, const void* w, int64_t tokens, int N, int K, const int64_t* positions,
+                  const float* inv_freq, int rot_dims, float mscale, float scale, const int32_t* slot_mapping, void* cache, float* q_out,
+                  float* rest, int64_t rest_row_stride, float* turns, int heads, int kv_heads, int dim, int vdim, nv_stream_t stream);
 /* nv_qk_conv_store: the store behind a short causal convolution (no bias) over time on every channel of q, k and v; w
  *   [H dim + G dim + G vdim, taps], state [slots, taps - 1, H dim + G dim + G vdim] keeps the last inputs; norm: every
  *   query and key head is then divided by its root mean square; q * scale to q_out, k and v to the cache.  Serves what
