@@ -1,11 +1,12 @@
-// The dense decoder's products of many rows (prefill) with what follows them, on the tiles of stream_tiles.h: bias; SiLU(gate) * up;
+// The dense decoder's products of many rows (prefill) with what follows them, on the tiles of stream_deep.h: bias; SiLU(gate) * up;
 // or bias, per-head norms, rotation and the KV-cache store.  16-bit weights, row-major or in nv_gemm's tiled layout, which the tiles'
 // DMA reads as it lies: nothing is written out first.
 //
 // What bounded these steps: the vendor library's product, then a pass over its whole result that moves it twice.  14.6 k rows of 1024
 // (Qwen3-0.6B): gate and up 157 us and SiluAndMul 53, q/k/v 105 and rotation with the store 61, and 5 - 7 us before each for the
-// weight as rows.  Here 190 and 151 us; SiLU by exp and quotient, as in the pass, is 20 of the first.  Which sizes this pays for:
-// kernels.gemm_many_rows and kernels.rotation_streams.
+// weight as rows.  Here 167 and 136 us (190 and 151 on the tiles of eight wavefronts).  What the results cost counts: with one wavefront to a
+// SIMD nothing hides it.  So SiLU in 11 instructions (anyt.h; exp and quotient: 177), roundings two at a time, and a row's cosines and sines,
+// norm weights and bias on their way before they are needed.  Which sizes this pays for: kernels.gemm_many_rows and kernels.rotation_streams.
 #include <type_traits>
 
 #include "anyt.h"

@@ -1,37 +1,32 @@
 // Products of many rows: a workgroup per CU walks tiles of 256 x 256 outputs whose K blocks form one stream.
 //
-// What bounds it: the matrix cores and, on this part, their power: at 8192 x 8192 x 8192 the loop that this one replaced (a block
-// fetched, waited for and multiplied behind one barrier, 32 x 32 products) takes 1108 us with them 49 % busy, this one 866 with 65 %, the
-// vendor library 696 with 89 % (one machine, the chip warm; busy cycles per active one under the counters, where the clock is 1.4 - 1.9
-// GHz and lowest for the busiest).  What a form between the two spent beside the products, from copies that leave one activity out (us):
-// whole 882, operands always from the same cache lines 719, no LDS reads 716, no DMA 669, none of these and no barriers 505.  So
-//   * 16 x 16 x 32 products: a lane's results lie where whole 64-byte pieces of rows can be stored (14592 rows by 4096, K 1024: 143
-//     us with 32 x 32 products, 125 with these);
+// Here: fp32, eight wavefronts of 128 x 64 each (16 bits: stream_deep.h, whose tiles, their order and W's rows in LDS are those of this file).
+//
+// What bounds it: the matrix cores (v_mfma_f32_16x16x4_f32).
+//   * 16-row products: a lane's results lie where whole 64-byte pieces of rows can be stored;
 //   * the barrier stands before the block's last step of K, whose fragments are in registers: behind it the first fragments of the
 //     next block are read under that step's products, and the buffer just left is refilled, one DMA instruction behind every few
-//     products (with all of them behind the reads that form took 846 us at 8192^3, so 796);
+//     products;
 //   * the order of products, LDS reads and DMA is fixed in the source (sched_barrier); left alone, the compiler puts the reads
 //     behind two thirds of the products and waits for them at once;
 //   * workgroups stay: the first two blocks of the next tile are on their way while the results of a tile are stored, and nothing
-//     waits for those stores but the second block after them (14592 by 4096, K 1024: 129 us with a workgroup per tile, so 117).
-//     Their tiles are found once, by a thread each, and kept in LDS: found in the loop they cost it its registers.
-// Measured, before and after: sixteen experts, 32768 rows of them, gated up 2048 -> 2 x 3072 and down, the layer 1569 and 1401 us;
-// 16384 rows 2048 -> 6144 into fp32 473 and 380 us (1085 TFLOP/s).
+//     waits for those stores but the second block after them.  Their tiles are found once, by a thread each, and kept in LDS.
+// Measured (us, this form and the 128 x 128 tiles): 2500 rows 1024 -> 6144 256 and 266, 8000 rows 512 -> 2048 137 and 149.
 // LDS rows are 128 bytes, their 16-byte pieces dealt by XOR (through the DMA's source addresses) so that the 16 rows a read touches lie
 // in 16 bank groups.  Tiles go to the XCDs in contiguous eighths, within them in bands of eight row
 // tiles, so the 32 workgroups of an XCD share 8 row and 4 column panels in its L2.  A group's short last row tile stays in its band
-// (at the end of everything, its column panels come from memory again: the experts' layer 1450 us against 1418).
+// (at the end of everything, its column panels come from memory again: sixteen experts in bf16 1450 us against 1418).
 //
 // Job (what is multiplied and what becomes of it) provides:
-//   T, Order (how W lies, below), NSTORE, K (elements, two blocks of 128 bytes at least)
+//   T, Order (how W lies, below; here in rows), NSTORE, K (elements, two blocks of 128 bytes at least)
 //   int count(lane)                       how many tiles there are
 //   StreamTile find(tile, lane)           which rows and columns the thread's tile has (every thread of a wavefront calls it)
 //   const void* a_base(tile); uint32_t a_row(tile, r); uint32_t a_stride()      row r of the tile's A rows (those past the end
 //                                         repeat a real one) lies at base + row * stride bytes, its K in 16-byte pieces
-//   w_base, w_row, w_stride, w_step()     the same of row r of the W tile in LDS, or of its 16-row tile r; bytes to the next K block
+//   w_base, w_row, w_stride, w_step()     the same of row r of the W tile in LDS (stream_deep.h: or of its 16-row tile r); bytes to the next K block
 //   bool whole(tile)                      NSTORE stores of a wavefront at least are executed for this tile
-//   void store(tile, first row, wn, lane, acc)   acc[j][i]: row 16 i + lane % 16 of the wavefront's, fragment row 4 (lane / 16) + r of product j
-// WN wavefronts lie along the columns, 8 / WN along the rows.
+//   void store<MT>(tile, first row, wn, lane, take)   take(j, i): row 16 i + lane % 16 of the wavefront's, fragment row 4 (lane / 16) + r of product j
+// Four wavefronts lie along the columns, two along the rows.
 #pragma once
 #include "anyt.h"
 #include "lds_limit.h"
@@ -42,14 +37,8 @@ struct alignas(16) StreamTile {
 };
 constexpr int STREAM_LIST = 512;      // tiles of one workgroup at most
 constexpr int STREAM_BM = 256, STREAM_BN = 256;
-constexpr int STREAM_BUFFER = (STREAM_BM + STREAM_BN) * 128 + 1024;      // a K block of both, and what lies between W's tiles
+constexpr int STREAM_BUFFER = (STREAM_BM + STREAM_BN) * 128;      // a K block of both
 
-__device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x4 c, bf16_t) {
-  return mfma16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c);
-}
-__device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x4 c, f16_t) {
-  return mfma16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c);
-}
 __device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x4 c, float) {
   // product e takes number 4 g + e of the sixteen that the four groups of lanes hold
 #pragma unroll
@@ -156,14 +145,13 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
   uint32_t arow[AG], wrow[WG];
   uint64_t apos, wpos;            // where the next K block begins, less what depends on the lane
   auto point = [&](const StreamTile& at) {
-
     const int r0 = 8 * wv + (stream_lane() >> 3);
 #pragma unroll
     for (int i = 0; i < AG; ++i) arow[i] = job.a_row(at, r0 + 64 * i);
 #pragma unroll
     for (int i = 0; i < AG; ++i) asm volatile("" : "+v"(arow[i]));      // a gathered row's number is waited for here, not at each fetch
 #pragma unroll
-    for (int i = 0; i < WG; ++i) wrow[i] = job.w_row(at, Order::TILED ? (wv >> 1) + 4 * i : r0 + 64 * i);
+    for (int i = 0; i < WG; ++i) wrow[i] = job.w_row(at, r0 + 64 * i);
     apos = reinterpret_cast<uint64_t>(job.a_base(at));
     wpos = reinterpret_cast<uint64_t>(job.w_base(at));
   };
@@ -172,12 +160,7 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
   auto lanes = [&]() {
     const int l = stream_lane(), r0 = 8 * wv + (l >> 3);
     alane = 16 * ((l & 7) ^ ((r0 >> 1) & 7));
-    if constexpr (Order::TILED) wlane = 1024 * (wv & 1) + 16 * l;
-    else wlane = 16 * ((l & 7) ^ Order::key(r0));
-  };
-  auto wplace = [&](int i) {
-    if constexpr (Order::TILED) return Order::place((wv >> 1) + 4 * i) + 1024 * (wv & 1);
-    else return 1024 * (wv + 8 * i);
+    wlane = 16 * ((l & 7) ^ Order::key(r0));
   };
   auto fill = [&](int bo, int i) {
     if (i < AG) {
@@ -187,7 +170,7 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
     } else {
       const int q = i < AG ? 0 : i - AG;
       __builtin_amdgcn_global_load_lds((global_void*)(wpos + (uint64_t)wrow[q] * w_stride + wlane),
-                                       (lds_void*)(lds_raw + bo + BM * 128 + wplace(q)), 16, 0, 0);
+                                       (lds_void*)(lds_raw + bo + (BM + 8 * (wv + 8 * q)) * 128), 16, 0, 0);
     }
     if (i == AG - 1) apos += 128;
     if (i == D - 1) wpos += w_step;
@@ -196,8 +179,7 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
   // starts at a multiple of 16 rows.
   auto fragments = [&](int bo, int step, int& wat, int& aat) {
     const int l = stream_lane(), fr = l & 15, in = bo + 16 * (((4 * step + (l >> 4)) ^ (fr >> 1)) & 7);
-    if constexpr (Order::TILED) wat = bo + BM * 128 + Order::place(NT * wn) + Order::frag(fr) + 1024 * step + 256 * (l >> 4);
-    else wat = in + (BM + 16 * NT * wn) * 128 + Order::frag(fr);
+    wat = in + (BM + 16 * NT * wn) * 128 + Order::frag(fr);
     aat = in + (16 * MT * wm + fr) * 128;
   };
   u32x4 wf[2][NT], af[2][MT];
@@ -285,7 +267,6 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
 
     left = blocks;
     if (live) {
-  
       job.template store<MT>(at, at.lo + 16 * MT * wm, wn, stream_lane(), [&](int j, int i) { return acc[j][i]; });
       stored = job.whole(at);
       clear();

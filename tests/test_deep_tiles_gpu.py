@@ -1,0 +1,79 @@
+"""16-bit products on the tiles of csrc/stream_deep.h where they can go wrong: an odd number of K blocks, one pair of blocks to a tile, halves
+of tiles in a last round, short tiles, weights in both layouts; and SiLU as it is formed behind them, for every gate."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def close(got, want, K, out_dtype):
+    tol = K * 2.0 ** -24 + (2.0 ** -8 if out_dtype == torch.bfloat16 else 2.0 ** -22)       # fp32 sums of K exact products, one rounding
+    off = ((got.double() - want).abs() / torch.maximum(want.pow(2).mean().sqrt(), want.abs())).max()
+    assert torch.isfinite(got).all() and off < tol, f"off by {off:.3g}, {tol:.3g} allowed"
+
+
+@pytest.mark.parametrize("K", [128, 192, 256, 320, 832])
+@pytest.mark.parametrize("M,N", [(1, 256), (65, 300), (128, 64), (129, 512), (256 * 33 + 5, 2000), (256 * 17 + 130, 4100), (256 * 70 + 1, 1000)])
+def test_blocks_and_tiles(M, N, K, monkeypatch):
+    from byox_vllm_amd import kernels
+    monkeypatch.setenv("NV_LINEAR_TILE", "2")
+    kernels.block_many_rows(True)
+    try:
+        torch.manual_seed(M + N + K)
+        x, w = torch.randn(max(M, 66), K, device=DEV).bfloat16(), (torch.randn(N, K, device=DEV) * 0.1).bfloat16()
+        bias, scale = torch.randn(N, device=DEV).bfloat16(), torch.rand(max(M, 66), device=DEV)
+        want = x.double() @ w.double().t()
+        for out_dtype in (torch.bfloat16, torch.float32):
+            close(kernels.linear(x, w, out_dtype=out_dtype), want, K, out_dtype)
+            close(kernels.linear(x, w, bias, out_dtype=out_dtype, row_scale=scale), want * scale.double()[:, None] + bias.double(), 2 * K, out_dtype)
+    finally:
+        kernels.block_many_rows(False)
+
+
+@pytest.mark.parametrize("tops", [[0, 0, 1000], [300, 1, 0, 129, 128, 257], [513] * 3])
+def test_gathered_groups(tops, monkeypatch):
+    """Groups that end anywhere in a tile, empty ones, rows from anywhere, gated."""
+    from byox_vllm_amd import kernels
+    monkeypatch.setenv("NV_LINEAR_TILE", "2")
+    torch.manual_seed(sum(tops))
+    T, K, n, E = 700, 320, 200, len(tops)
+    x, w = torch.randn(T, K, device=DEV).bfloat16(), (torch.randn(E, 2 * n, K, device=DEV) * 0.1).bfloat16()
+    rows = torch.randint(0, T, (sum(tops),), device=DEV, dtype=torch.int32)
+    off = torch.tensor([sum(tops[:i]) for i in range(E + 1)], dtype=torch.int32, device=DEV)
+    got = kernels.linear(x, w, rows=sum(tops), a_rows=rows, batch=E, w_batch_stride=2 * n * K, group_offsets=off, max_group_rows=max(max(tops), 65),
+                         epilogue=kernels.EPI_GLU, n=n)
+    at = 0
+    for e, m in enumerate(tops):
+        y = x[rows[at:at + m].long()].double() @ w[e].double().t()
+        if m:
+            close(got[at:at + m], torch.nn.functional.silu(y[:, :n]) * y[:, n:], 4 * K, torch.bfloat16)
+        at += m
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_silu_of_every_gate(dt):
+    """Gates of all 16-bit values against float64: SiLU's rounding and at most 4 units of fp32, which move it across a tie now and then."""
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.layers.quant import LinearWeight, interleave_gate_up
+    gates = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dt).to(DEV)
+    x = torch.zeros(65536, 128, device=DEV, dtype=dt)
+    x[:, 0], x[:, 1] = gates, 1.0
+    w = torch.zeros(512, 128, device=DEV, dtype=dt)
+    w[:256, 0] = 1.0          # every gate column is the gate, every up column 1
+    w[256:, 1] = 1.0
+    finite = torch.isfinite(gates)
+    x[~finite] = 0.0
+    got = kernels.gemm_stream(x, LinearWeight.make(interleave_gate_up(w), None), None, None, True)[:, 0][finite]
+    g = gates[finite].double()
+    want = torch.where(g < -700, -0.0, g / (1.0 + torch.exp(-g)))
+    tiny = 2.0 ** -126 if dt == torch.bfloat16 else 2.0 ** -24
+    eps = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
+    deep = g < -88.7                # exp overflows fp32, as it did: 0
+    assert (got[deep].abs().double() <= 2.0 ** -119).all()
+    err = (got.double() - want).abs()[~deep]
+    assert (err <= eps * want.abs()[~deep] * (1 + 2.0 ** -10) + tiny).all()
+    x[1, 0] = float("nan")          # what is not finite stays in its row
+    y = kernels.gemm_stream(x[:300], LinearWeight.make(interleave_gate_up(w), None), None, None, True)
+    assert torch.isnan(y[1]).all() and torch.isfinite(y[0]).all() and torch.isfinite(y[2:]).all()
