@@ -1244,7 +1244,8 @@ def qkv_streams(x, w, heads, kv_heads, dim, vdim, rot_dims, interleaved) -> bool
     M, N, K = x.size(0), w.size(0), w.size(1)
     return (M >= MANY_ROWS and x.dtype == w.dtype == torch.bfloat16 and x.dim() == 2 and x.stride(1) == 1 and w.is_contiguous()
             and x.size(1) == K and use_many_rows_path(M, K, 16) and K < 1 << 22 and N < 1 << 20 and dim in (64, 128)
-            and kv_heads * vdim % 16 == 0 and vdim > 0 and rot_dims in (0, 32, 64, 128) and rot_dims <= dim and not (interleaved and rot_dims)
+            and kv_heads > 0 and heads % kv_heads == 0 and kv_heads * vdim % 16 == 0 and vdim > 0
+            and rot_dims in (0, 32, 64, 128) and rot_dims <= dim and not (interleaved and rot_dims)
             and x.stride(0) % 8 == 0 and K <= x.stride(0) < 1 << 30 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and M <= LINEAR_ROWS and -(-M // 256) * -(-N // 256) <= 256 * 510 and tile_share(M, N) >= 0.7)
 

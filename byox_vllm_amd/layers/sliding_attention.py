@@ -48,8 +48,8 @@ class SlidingAttention(nn.Module):
     def forward(self, h: torch.Tensor, positions: torch.Tensor, run: int = 0) -> torch.Tensor:
         ctx, own = get_context(), self.runs[run]
         H, G, d, dv = self.heads, self.kv_heads, self.dim, self.vdim
-        if called_plainly(self.inp, DenseLinear) and own.cache.dtype == h.dtype and own.cache.data_ptr() % 8 == 0 and \
-                kernels.qkv_streams(h, self.inp.weight, H, G, d, dv, self.rot_dims, self.interleaved):
+        if called_plainly(self.inp, DenseLinear) and self.inp.bias is None and own.cache.dtype == h.dtype and \
+                own.cache.data_ptr() % 8 == 0 and kernels.qkv_streams(h, self.inp.weight, H, G, d, dv, self.rot_dims, self.interleaved):
             q, gates = kernels.qkv_project_store(h, self.inp.weight.data, positions, self.scale, ctx.slot_mapping, own.cache, H, G, d, dv,
                                                  inv_freq=self.inv_freq, rot_dims=self.rot_dims, mscale=self.magnitude)
         else:

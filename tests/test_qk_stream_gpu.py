@@ -63,6 +63,7 @@ def test_which_calls_take_it():
     assert not kernels.qkv_streams(x[:8192], w, 16, 2, 128, 128, 32, False)          # a share of 0.68
     assert not kernels.qkv_streams(x, w, 16, 2, 128, 128, 32, True)                  # pairs next to each other
     assert not kernels.qkv_streams(x, w, 32, 4, 32, 64, 32, False)                   # heads of 32
+    assert not kernels.qkv_streams(x, w, 15, 2, 128, 128, 32, False)                 # heads that do not divide: refused behind it
     assert not kernels.qkv_streams(x.float(), w.float(), 16, 2, 128, 128, 32, False)
     assert not kernels.qkv_streams(x, w, 16, 2, 128, 128, 16, False)                 # halves of 8
     from byox_vllm_amd.layers.linear import called_plainly
