@@ -369,13 +369,16 @@ def streams(x, w, *others):
 
 def rotation_streams(M, w) -> bool:
     """Whether gemm_stream_rope_kv_store is not slower than the library's product and rope_kv_store for M prefill rows: the results fill
-    their rounds of tiles (tile_share), by less where their width does not split into the library's; K up to 2048, 1024 where the weight
-    has to be expanded.  Both routes, us: 16384 rows 1024 -> 4096, share 1.0: 183 and 155; 14600 rows 896 -> 1152, 0.54: 69 and 62; 5000
-    rows, 0.40: 27 and 37; 4100 rows 2048 -> 4096, 0.54: 93 and 102; int4, 11000 rows 1024 -> 4096, 0.90: 140 and 123, 16384 rows
-    2048 -> 4096, 1.0: 249 and 255."""
+    their rounds of tiles (tile_share), by less where their width does not split into the library's and K is up to 2048; K up to 6144 for
+    more than 2048 columns, 2048 for fewer, 1024 where the weight has to be expanded.  Both routes, us: 16384 rows 1024 -> 4096, share 1.0:
+    183 and 155; 14600 rows 896 -> 1152, 0.54: 69 and 62; 5000 rows, 0.40: 27 and 37; 4100 rows 2048 -> 4096, 0.54: 93 and 102; 9959 rows
+    4224 -> 3072, 0.91: 213 and 198; 14170 rows 5888 -> 2048, 0.87: 273 and 286; 9591 rows 4096 -> 2304, 0.71: 180 and 196 (beyond 2048, of
+    34 above the line none is slower, 1.14x); int4, 11000 rows 1024 -> 4096, 0.90: 140 and 123, 10023 rows 4992 -> 3072, 0.92: 246 and 260."""
     N, odd = w.out_features, w.out_features % 256 != 0
     if w.fmt == _C.W_DENSE_TILED:
-        return w.in_features <= 2048 and tile_share(M, N) >= (0.5 if odd else 0.75)
+        if w.in_features > 2048:
+            return w.in_features <= 6144 and N > 2048 and tile_share(M, N) >= 0.8
+        return tile_share(M, N) >= (0.5 if odd else 0.75)
     return w.in_features <= 1024 and tile_share(M, N) >= (0.6 if odd else 0.8)
 
 
@@ -426,23 +429,40 @@ def gemm_stream(x, w, bias=None, out=None, silu_mul=False):
     return out
 
 
+def gemm_many_rows_streams(M, w, silu_mul) -> bool:
+    """Whether nv_gemm_stream is not slower than the vendor library's route for M rows without a bias.  Both, us, library first; share: tile_share.
+     * gate/up, weights in tiles: K below 4096, up to 8191 from a share of 0.8 (16384 rows 1024 -> 2 x 3072 232 and 175, 4096 rows
+       4096 -> 2 x 12288 667 and 564, 8192 rows 3584 -> 2 x 18944 1916 and 1527; 5402 rows 7040 -> 2 x 2048, 0.71, 276 and 309; 16249 rows
+       8192 -> 2 x 13056 5249 and 5429); of 73 shapes of K 2048 to 7680 above the line two are slower, by 0.5 %, the mean is 1.22x;
+     * gate/up, weights to be expanded: K below 2048, up to 8191 from a share of 0.85 where K is below 4608 or 6144 columns and more (int4: 8192
+       rows 3584 -> 2 x 18944 1937 and 1637; 7872 rows 6144 -> 2 x 1536, 0.78, 251 and 296; 4213 rows 6912 -> 2 x 1792 170 and 182): of 55 none is
+       slower, 1.14x;
+     * other products of more than 1024 columns, weights in tiles, which the library has to have written out: K 512 to 1023 from a share of
+       0.7, to 1536 of 0.74, to 3584 of 0.9 (13422 rows 512 -> 4864 87 and 71, 9741 rows 1024 -> 2560 58 and 54, 13741 rows 2048 -> 3584 153 and 148;
+       1024 columns tie: 16384 rows 2048 -> 1024 54 and 52, 14600 rows 3072 -> 1024, 0.89, 71 and 76; 6947 rows 1024 -> 2560, 0.57, 49 and 50; 14240 rows 4096 -> 8192 631 and 692): of 167 above the
+       line one is over 2 % slower (9), the mean is 1.21x;
+     * K 512 to 1023 and columns that do not split into tiles from a share of 0.6, 0.8 where the weight has to be expanded (16384 rows 896 -> 896,
+       0.88: 43 and 30, int4 43 and 33; 11000 rows 896 -> 640, 0.42: 21 and 27)."""
+    N, K, share = w.out_features, w.in_features, tile_share(M, w.out_features)
+    tiled = w.fmt == _C.W_DENSE_TILED
+    if silu_mul:
+        if tiled:
+            return K < 4096 or (K < 8192 and share >= 0.8)
+        return K < 2048 or (K < 8192 and share >= 0.85 and (K < 4608 or N >= 6144))
+    if K < 512:
+        return False
+    if K < 1024 and N % 256 != 0 and share >= (0.6 if tiled else 0.8):
+        return True
+    return tiled and N > 1024 and K <= 3584 and share >= (0.7 if K < 1024 else 0.74 if K <= 1536 else 0.9)
+
+
 def gemm_many_rows(x, w, bias=None, out=None, silu_mul=False):
     """gemm() for prefill-sized x: the weight written out row-major into scratch and one vendor-library product, with a SiluAndMul pass
-    over its result for gate/up weights; or, where that is not slower, this library's tiles (nv_gemm_stream).  Those have
-     * gate/up weights of a K below 4096, or below 2048 where the weight has to be expanded, without a bias (16384 rows, both routes:
-       1024 -> 2 x 3072 217 and 197 us, int4 216 and 204; 14600 rows 220 and 190; 2048 -> 2 x 6144 690
-       and 706, 6000 rows 351 and 271; 4096 rows 4096 -> 2 x 12288 645 and 651, int4 653 and 723);
-     * products of 512 <= K < 1024 without a bias whose columns do not split into tiles and whose results fill 0.6 of their rounds, 0.8
-       where the weight has to be expanded (tile_share; 16384 rows 896 -> 896, share 0.88: 43 and 30 us, int4 43 and 33; 11000 rows
-       896 -> 640, 0.42: 21 and 27; whole tiles: 16384 rows 896 -> 8192 198 and 223, 2048 -> 1024 51 and 55)."""
+    over its result for gate/up weights; or, where that is not slower, this library's tiles (nv_gemm_stream: gemm_many_rows_streams)."""
     M, K = x.shape
     N = w.out_features
     dev = x.device
-    if silu_mul:
-        own = bias is None and K < (4096 if w.fmt == _C.W_DENSE_TILED else 2048)
-    else:
-        own = bias is None and 512 <= K < 1024 and N % 256 != 0 and tile_share(M, N) >= (0.6 if w.fmt == _C.W_DENSE_TILED else 0.8)
-    if own and streams(x, w, bias, out) and _streams_into(out, x, N // 2 if silu_mul else N):
+    if bias is None and gemm_many_rows_streams(M, w, silu_mul) and streams(x, w, out) and _streams_into(out, x, N // 2 if silu_mul else N):
         return gemm_stream(x, w, bias, out, silu_mul)
     if w.fmt == _C.W_DENSE and not silu_mul:
         wr = w.data
