@@ -20,7 +20,7 @@
 // Job: as for stream_tiles.h, and
 //   bool FAR_A, FAR_W                     whether a tile's rows of A (W) may lie 4 GiB and more from its base
 //   NSTORE_WAVE                           stores of a wavefront of a whole tile, at least
-//   EXTRA, fetch_extra(tile, wv, lane, lds)   bytes of LDS a tile's results need of memory, and the DMA for them, a tile ahead
+//   EXTRA, fetch_extra(tile, wv, lane, lds)   bytes of LDS a tile's results need of memory (3 KB fit), and the DMA for them, a tile ahead
 //   finish(tile, wm, wn, lane, live0, live1, lds)   the results: rows 128 h + 64 wm .. of the tile, h = 0 and 1 as far as live, by rows 128 wn ..
 //                                         of W's tile; deep_take(h, j, i) has row 16 i + lane % 16, fragment row 4 (lane / 16) + r of product j of eight
 #pragma once
@@ -166,7 +166,9 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
     const int s = r >> 2, j = r & 3;
     fw[h][j][s] = *reinterpret_cast<const u32x4*>(lds_raw + bo + 2 * DEEP_PA + h * DEEP_PW + wat[s] + Order::off(j));
   };
-  auto extra = [&](int n) { return lds_raw + 2 * DEEP_BUFFER + STREAM_LIST * sizeof(StreamTile) + (n & 1) * Job::EXTRA; };
+  // What tile n's results need lies in one of four places.  Where a tile has one pair of blocks, no barrier stands between a wavefront's finish
+  // of tile n - 1 and another's DMA for n + 1, so three are in use at once.
+  auto extra = [&](int n) { return lds_raw + 2 * DEEP_BUFFER + STREAM_LIST * sizeof(StreamTile) + (n & 3) * Job::EXTRA; };
   const int blocks = job.K / 64, pairs = (blocks + 1) / 2;
   const bool odd = blocks & 1;
   StreamTile at = listed(0), ahead = at;
@@ -320,7 +322,8 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
 
 template <typename Job>
 hipError_t launch_stream_deep(const Job& job, int64_t max_tiles, hipStream_t s) {
-  constexpr size_t lds = 2 * DEEP_BUFFER + STREAM_LIST * sizeof(StreamTile) + 2 * Job::EXTRA;
+  constexpr size_t lds = 2 * DEEP_BUFFER + STREAM_LIST * sizeof(StreamTile) + 4 * Job::EXTRA;
+  static_assert(lds <= 160 * 1024, "LDS of a CU");
   static std::atomic<uint64_t> devices{0};
   const hipError_t e = allow_lds(reinterpret_cast<const void*>(&stream_deep_kernel<Job>), lds, devices);
   if (e != hipSuccess) return e;

@@ -111,6 +111,38 @@ def test_rope_kv_store(T, H, Hkv, D, norms, tiled, name):
     assert torch.equal(bare, got)
 
 
+@pytest.mark.parametrize("tiled", [True, False])
+@pytest.mark.parametrize("K", [128, 192, 256])
+@pytest.mark.parametrize("H,Hkv,D,norms", [(25, 4, 64, False), (9, 4, 128, True), (30, 2, 64, True)])
+def test_rope_kv_store_of_three_tiles_to_a_workgroup(H, Hkv, D, norms, K, tiled):
+    """Positions, cache rows and norm weights of one tile while others are fetched: with one pair of K blocks to a tile (K = 128) the
+    wavefronts without columns (33 heads of 64, 17 of 128) or with values alone are two tiles' fetches ahead of those that still read."""
+    from byox_vllm_amd import kernels
+    if tiled and K % 128:
+        pytest.skip("weights in tiles have K in 128s")
+    torch.manual_seed(K + H)
+    T, N, dt = 256 * 64 + 70, (H + 2 * Hkv) * D, torch.bfloat16
+    assert -(-T // 256) * -(-N // 256) > 512
+    x, w = torch.randn(T, K, device=DEV).to(dt), (torch.randn(N, K, device=DEV) * 0.1).to(dt)
+    bias = None if norms else torch.randn(N, device=DEV).to(dt)
+    qn, kn = ((torch.rand(D, device=DEV) + 0.5).to(dt) if norms else None for _ in range(2))
+    pos = torch.randint(0, 500, (T,), device=DEV)
+    cos_sin = torch.randn(500, D, device=DEV)
+    pages = -(-T // 16) + 1
+    slots = torch.randperm(pages * 16, device=DEV)[:T].int()
+    caches = [torch.zeros(pages, 16, Hkv, D, dtype=dt, device=DEV) for _ in range(4)]
+    args = dict(slot_mapping=slots, q_norm_w=qn, k_norm_w=kn, eps=1e-6)
+    qkv = kernels.gemm_stream(x, weight(w, tiled), bias)
+    want = kernels.rope_kv_store(qkv, pos, cos_sin, H, Hkv, D, k_cache=caches[2], v_cache=caches[3], **args)
+    for _ in range(3):
+        got = kernels.gemm_stream_rope_kv_store(x, weight(w, tiled), bias, pos, cos_sin, H, Hkv, D, k_cache=caches[0], v_cache=caches[1], **args)
+        for a, b in ((got, want), (caches[0], caches[2]), (caches[1], caches[3])):
+            # as in test_rope_kv_store: the norm's sum in another order, or the same numbers rounded once
+            scale = torch.finfo(dt).eps * 8.0 * 6.0 if norms else torch.finfo(dt).eps
+            assert ((a.double() - b.double()).abs() <= scale * (1 + b.double().abs())).all()
+            assert (a != b).float().mean() < 1e-3
+
+
 @pytest.mark.parametrize("M", [300, 2100, 4100])
 @pytest.mark.parametrize("inter", [24, 40])
 @pytest.mark.parametrize("fmt", [None, "w4a16"])
