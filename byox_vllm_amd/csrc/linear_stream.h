@@ -126,17 +126,21 @@ struct LinearJob {
     if constexpr (EPI == EPI_NONE) {
       if (!p.bias && !p.row_scale) return store_ahead<HALF, -1, false>(at, row0, wn, lane);
     }
-    if constexpr (EPI == EPI_ACT || EPI == EPI_GLU) {
+    if constexpr (EPI == EPI_GLU) {
+      switch (p.act) {      // as glu_act: what is neither GELU nor the clamped unit is SiLU
+        case 1: return store_ahead<HALF, 1, true>(at, row0, wn, lane);
+        case 2: return store_ahead<HALF, 2, true>(at, row0, wn, lane);
+        default: return store_ahead<HALF, 0, true>(at, row0, wn, lane);
+      }
+    } else if constexpr (EPI == EPI_ACT) {
       switch (p.act) {
         case 0: return store_ahead<HALF, 0, true>(at, row0, wn, lane);
         case 1: return store_ahead<HALF, 1, true>(at, row0, wn, lane);
         case 2: return store_ahead<HALF, 2, true>(at, row0, wn, lane);
+        case 4: return store_ahead<HALF, 4, true>(at, row0, wn, lane);
+        default: return store_ahead<HALF, 3, true>(at, row0, wn, lane);
       }
-    }
-    if constexpr (EPI == EPI_ACT) {
-      if (p.act == 4) return store_ahead<HALF, 4, true>(at, row0, wn, lane);
-      return store_ahead<HALF, 3, true>(at, row0, wn, lane);
-    } else if constexpr (EPI != EPI_GLU) {
+    } else {
       store_ahead<HALF, -1, true>(at, row0, wn, lane);
     }
   }

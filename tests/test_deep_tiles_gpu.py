@@ -52,6 +52,23 @@ def test_gathered_groups(tops, monkeypatch):
         at += m
 
 
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("act", [-1, 3, 7])
+def test_gated_products_without_an_activation_of_their_own(act, out_dtype, monkeypatch):
+    """What is neither GELU nor the clamped unit is SiLU, on these tiles as on the others."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(5)
+    K, n = 320, 300
+    x, w = torch.randn(700, K, device=DEV).bfloat16(), (torch.randn(2 * n, K, device=DEV) * 0.1).bfloat16()
+    y = x.double() @ w.double().t()
+    want = torch.nn.functional.silu(y[:, :n]) * y[:, n:]
+    for tile in ("0", "1", "2"):
+        monkeypatch.setenv("NV_LINEAR_TILE", tile)
+        got = kernels.linear(x, w, epilogue=kernels.EPI_GLU, act=act, out_dtype=out_dtype)
+        close(got, want, 4 * K, out_dtype)
+        assert torch.equal(got, kernels.linear(x, w, epilogue=kernels.EPI_GLU, out_dtype=out_dtype))
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 def test_silu_of_every_gate(dt):
     """Gates of all 16-bit values against float64: SiLU's rounding and at most 4 units of fp32, which move it across a tie now and then."""
