@@ -31,7 +31,7 @@ struct RowsJob {
                              std::conditional_t<TILED, StreamPairedTiled, StreamPaired>> Order;
   static constexpr bool SILU = WHAT == ROWS_SILU, ROPE = WHAT == ROWS_ROPE;
   static constexpr int NOUT = SILU ? 128 : 256, NSTORE_WAVE = SILU ? 16 : 32, EXTRA = ROPE ? 3072 : 0;
-  static constexpr bool FAR_A = FAR, FAR_W = FAR;
+  static constexpr bool FAR_A = FAR, FAR_W = FAR, UPS = false;
   RowsArgs p;
   RopeArgs ra;
   int K, rows, cols;      // row and column tiles

@@ -96,19 +96,22 @@ struct LinearJob {
     const int s = min(at.lo + r, at.hi - 1);
     return (uint32_t)(p.a_rows ? p.a_rows[s] : s);
   }
-  __device__ __forceinline__ const void* w_base(const StreamTile& at) const { return reinterpret_cast<const T*>(p.w) + at.z * p.w_bs; }
+  __device__ __forceinline__ const void* w_base(const StreamTile& at) const {
+    return reinterpret_cast<const T*>(p.w) + at.z * p.w_bs + at.n0 * p.w_rs;
+  }
   __device__ __forceinline__ uint32_t w_stride() const { return (uint32_t)p.w_rs * sizeof(T); }
+  __device__ __forceinline__ uint64_t w_ups() const { return (uint64_t)p.N * p.w_rs * sizeof(T); }
   __device__ __forceinline__ uint32_t w_row(const StreamTile& at, int r) const {
     // a wavefront's 64 rows: 64 columns, or 32 columns' gates and the same columns' ups
-    if constexpr (GLU) return min(at.n0 + 32 * (r >> 6) + (r & 31), p.N - 1) + ((r & 32) ? p.N : 0);
-    else return min(at.n0 + r, p.N - 1);
+    if constexpr (GLU) return min(32 * (r >> 6) + (r & 31), p.N - at.n0 - 1) + (!UPS && (r & 32) ? p.N : 0);
+    else return min(r, p.N - at.n0 - 1);
   }
   __device__ __forceinline__ uint32_t w_step() const { return 128; }
   __device__ __forceinline__ bool whole(const StreamTile& at) const {
     return vec && at.lo + BM <= at.hi && at.n0 + NOUT <= p.N;
   }
   static constexpr int NSTORE_WAVE = 2 * NSTORE, EXTRA = 0;
-  static constexpr bool FAR_A = true, FAR_W = false;      // A's rows may lie anywhere; W: stream_takes
+  static constexpr bool FAR_A = true, FAR_W = false, UPS = GLU && sizeof(T) == 2;      // A's rows may lie anywhere; W's: stream_takes
   __device__ __forceinline__ void fetch_extra(const StreamTile&, int, int, unsigned char*) const {}
   __device__ __forceinline__ void finish(const StreamTile& at, int wm, int wn, int lane, bool live0, bool live1, const unsigned char*) const {
     if (live0) store_wave<0>(at, at.lo + 64 * wm, wn, lane);
@@ -296,8 +299,7 @@ struct LinearJob {
 inline bool stream_takes(const LinArgs& p, int esz, int64_t total_rows, int batch, int cols) {
   const int64_t rows = p.group_off ? total_rows / 256 + batch : (p.M + 255) / 256 * batch;
   if (total_rows >= ((int64_t)1 << 31) || rows * ((cols + 255) / 256) > 256 * (STREAM_LIST - 2)) return false;
-  // a 16-bit tile's rows of W lie within 4 GiB of its first (the ups of a gated one N rows behind it)
-  if (esz == 2 && (cols + 256) * p.w_rs * esz >= ((int64_t)1 << 32)) return false;
+  if (esz == 2 && p.w_rs >= ((int64_t)1 << 23)) return false;      // a 16-bit tile's 256 rows of W lie within 4 GiB
   return p.K * esz >= 256 && p.K * esz % 128 == 0 && p.a_rs >= 0 && p.w_rs >= 0 && p.a_rs < ((int64_t)1 << 30) && p.w_rs < ((int64_t)1 << 30);
 }
 

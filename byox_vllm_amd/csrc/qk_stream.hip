@@ -26,7 +26,7 @@ template <int D, int HALF16>
 struct QkvJob {
   typedef bf16_t T;
   typedef StreamNatural Order;
-  static constexpr bool FAR_A = true, FAR_W = false;
+  static constexpr bool FAR_A = true, FAR_W = false, UPS = false;
   static constexpr int NSTORE_WAVE = 64, EXTRA = 0;
   QkvArgs p;
   int K, rows, cols;

@@ -19,6 +19,7 @@
 // rows 1024 -> 4096 121 and 105; gate/up of 1024 -> 2 x 3072 194 and 177, q/k/v with rotation 150 and 134.
 // Job: as for stream_tiles.h, and
 //   bool FAR_A, FAR_W                     whether a tile's rows of A (W) may lie 4 GiB and more from its base
+//   bool UPS, w_ups()                     whether W's rows 32 - 63 of every 64 lie another w_ups() bytes on (which may be 4 GiB and more)
 //   NSTORE_WAVE                           stores of a wavefront of a whole tile, at least
 //   EXTRA, fetch_extra(tile, wv, lane, lds)   bytes of LDS a tile's results need of memory (3 KB fit), and the DMA for them, a tile ahead
 //   finish(tile, wm, wn, lane, live0, live1, lds)   the results: rows 128 h + 64 wm .. of the tile, h = 0 and 1 as far as live, by rows 128 wn ..
@@ -117,7 +118,7 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
   // with K would be 32 registers, moved about wherever the ways through the loop below meet.)
   std::conditional_t<Job::FAR_A, uint64_t, uint32_t> ap[2][4];
   std::conditional_t<Job::FAR_W, uint64_t, uint32_t> wp[2][4];
-  uint64_t abase, wbase;
+  uint64_t abase, wbase, ubase = 0;
   auto point = [&](const StreamTile& at) {
     const int l = lane, r8 = 8 * wv + (l >> 3);
 #pragma unroll
@@ -135,6 +136,7 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
       }
     abase = reinterpret_cast<uint64_t>(job.a_base(at));
     wbase = reinterpret_cast<uint64_t>(job.w_base(at));
+    if constexpr (Job::UPS) ubase = wbase + job.w_ups();
   };
   auto fill_a = [&](int bo, int h, int q) {
     __builtin_amdgcn_global_load_lds((global_void*)(abase + ap[h][q]), (lds_void*)(lds_raw + bo + h * DEEP_PA + (wv + 4 * q) * 1024), 16, 0, 0);
@@ -143,11 +145,13 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
     int place;
     if constexpr (Order::TILED) place = Order::place((wv >> 1) + 2 * q) + 1024 * (wv & 1);
     else place = (wv + 4 * q) * 1024;
-    __builtin_amdgcn_global_load_lds((global_void*)(wbase + wp[h][q]), (lds_void*)(lds_raw + bo + 2 * DEEP_PA + h * DEEP_PW + place), 16, 0, 0);
+    const uint64_t base = Job::UPS && (q & 1) ? ubase : wbase;
+    __builtin_amdgcn_global_load_lds((global_void*)(base + wp[h][q]), (lds_void*)(lds_raw + bo + 2 * DEEP_PA + h * DEEP_PW + place), 16, 0, 0);
   };
   auto next_block = [&]() {
     abase += 128;
     wbase += w_step;
+    ubase += w_step;
   };
   u32x4 fa[2][4][2], fw[2][4][2];
   int aat[2], wat[2];
@@ -298,6 +302,7 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
       if (odd && left == 2) {      // the last pair has no second block: the first one again, unused
         abase -= 128;
         wbase -= w_step;
+        ubase -= w_step;
       }
       const bool full = !odd || left > 1;
       half(plain, I1, I0, live0 && full, false, stored);

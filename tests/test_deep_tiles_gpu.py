@@ -32,6 +32,24 @@ def test_blocks_and_tiles(M, N, K, monkeypatch):
         kernels.block_many_rows(False)
 
 
+@pytest.mark.parametrize("gated", [False, True])
+def test_weights_of_4_gib(gated, monkeypatch):
+    """Rows of W that lie 4 GiB and more from its first, and a gated product's ups as far from their gates."""
+    from byox_vllm_amd import kernels
+    monkeypatch.setenv("NV_LINEAR_TILE", "2")
+    torch.manual_seed(4)
+    M, K, n = 300, 4096, 2 ** 32 // 8192 + 696
+    x = torch.randn(M, K, device=DEV).bfloat16()
+    w = torch.empty((1 + gated) * n, K, device=DEV, dtype=torch.bfloat16).normal_(0.0, 0.1)
+    got = kernels.linear(x, w, epilogue=kernels.EPI_GLU if gated else kernels.EPI_NONE)
+    for at in (0, n // 2, n - 1000, n - 296):
+        c = slice(at, at + 296)
+        want = x.double() @ w[:n][c].double().t()
+        if gated:
+            want = torch.nn.functional.silu(want) * (x.double() @ w[n:][c].double().t())
+        close(got[:, c], want, 4 * K, torch.bfloat16)
+
+
 @pytest.mark.parametrize("tops", [[0, 0, 1000], [300, 1, 0, 129, 128, 257], [513] * 3])
 def test_gathered_groups(tops, monkeypatch):
     """Groups that end anywhere in a tile, empty ones, rows from anywhere, gated."""
