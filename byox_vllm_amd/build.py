@@ -9,6 +9,8 @@ import glob
 import os
 import subprocess
 
+from byox_vllm_amd import build_check
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "byox_vllm_amd", "csrc")
 LIB = os.path.join(ROOT, "byox_vllm_amd", "libnv_hip.so")
@@ -36,7 +38,7 @@ def _headers():
 
 
 def compile_sources(sources, force=False, jobs=None):
-    """hipcc -c each stale source (in parallel) -> the object files."""
+    """hipcc -c each stale source (in parallel) -> the object files, whose machine code is looked over where it has to be (build_check.py)."""
     jobs = jobs or max(1, min(16, os.cpu_count() or 1))
     headers = _headers()
     objs, todo = [], []
@@ -58,6 +60,13 @@ def compile_sources(sources, force=False, jobs=None):
             for _, q in running:
                 q.kill()
             raise RuntimeError(f"hipcc failed on {src}:\n{err.decode(errors='replace')[-4000:]}")
+        try:
+            build_check.check_object(src[:-4] + ".o")
+        except Exception:
+            os.remove(src[:-4] + ".o")      # not to be linked by a later call
+            for _, q in running:
+                q.kill()
+            raise
     return objs
 
 
