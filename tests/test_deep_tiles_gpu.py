@@ -1,5 +1,5 @@
 """16-bit products on the tiles of csrc/stream_deep.h where they can go wrong: an odd number of K blocks, one pair of blocks to a tile, halves
-of tiles in a last round, short tiles, weights in both layouts; and SiLU as it is formed behind them, for every gate."""
+of tiles in a last round, short tiles, a third tile to a workgroup; and SiLU as it is formed behind them, for every gate."""
 
 import pytest
 import torch
@@ -15,15 +15,18 @@ def close(got, want, K, out_dtype):
 
 
 @pytest.mark.parametrize("K", [128, 192, 256, 320, 832])
-@pytest.mark.parametrize("M,N", [(1, 256), (65, 300), (128, 64), (129, 512), (256 * 33 + 5, 2000), (256 * 17 + 130, 4100), (256 * 70 + 1, 1000)])
+@pytest.mark.parametrize("M,N", [(65, 300), (128, 64), (129, 512), (256 * 33 + 5, 2000), (256 * 17 + 130, 4100), (256 * 70 + 1, 1000),
+                                 (256 * 64 + 70, 2104)])
 def test_blocks_and_tiles(M, N, K, monkeypatch):
+    """The last of the sizes: 585 tiles, three to some workgroups, one column of wavefronts empty in every ninth.  One row alone in a tile:
+    256 * 70 + 1 here, and a group of one below."""
     from byox_vllm_amd import kernels
     monkeypatch.setenv("NV_LINEAR_TILE", "2")
     kernels.block_many_rows(True)
     try:
         torch.manual_seed(M + N + K)
-        x, w = torch.randn(max(M, 66), K, device=DEV).bfloat16(), (torch.randn(N, K, device=DEV) * 0.1).bfloat16()
-        bias, scale = torch.randn(N, device=DEV).bfloat16(), torch.rand(max(M, 66), device=DEV)
+        x, w = torch.randn(M, K, device=DEV).bfloat16(), (torch.randn(N, K, device=DEV) * 0.1).bfloat16()
+        bias, scale = torch.randn(N, device=DEV).bfloat16(), torch.rand(M, device=DEV)
         want = x.double() @ w.double().t()
         for out_dtype in (torch.bfloat16, torch.float32):
             close(kernels.linear(x, w, out_dtype=out_dtype), want, K, out_dtype)

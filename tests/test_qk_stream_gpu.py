@@ -71,3 +71,61 @@ def test_which_calls_take_it():
     assert called_plainly(layer, DenseLinear)
     layer.register_forward_hook(lambda *_: None)
     assert not called_plainly(layer, DenseLinear)
+
+
+@pytest.mark.parametrize("hook", [False, True])
+def test_layer_against_two_launches(hook, monkeypatch):
+    """SlidingAttention.forward over prompt pieces of five requests, its second run's cache: the projection with rotation and store in one pass,
+    and the two launches behind a product that a hook sees."""
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd.layers.sliding_attention import SlidingAttention
+    from byox_vllm_amd.utils.context import reset_context, set_context
+    torch.manual_seed(11)
+    width, H, G, d, page = 512, 16, 2, 128, 16
+    past, new = [0, 5, 64, 0, 300], [9000, 6000, 1, 1300, 83]
+    default = torch.get_default_dtype()
+    torch.set_default_dtype(torch.bfloat16)
+    try:
+        with torch.device(DEV):
+            layer = SlidingAttention(width, H, G, d, d, d ** -0.5, 256, 4, rot_dims=32)
+    finally:
+        torch.set_default_dtype(default)
+    for p in layer.parameters():
+        p.data.normal_(0.0, p.size(1) ** -0.5)
+    pages = [-(-(a + b) // page) for a, b in zip(past, new)]
+    order = torch.randperm(sum(pages)).tolist()
+    tables = [[order.pop() for _ in range(n)] for n in pages]
+    where = [(i, a + j) for i, (a, b) in enumerate(zip(past, new)) for j in range(b)]
+    ints = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    slots = ints([tables[i][t // page] * page + t % page for i, t in where])
+    positions = torch.tensor([t for _, t in where], device=DEV)
+    step = dict(cu_seqlens_q=ints([sum(new[:i]) for i in range(6)]), max_seqlen_q=max(new), slot_mapping=slots, past_lens=ints(past),
+                block_tables=ints([t + [0] * (max(pages) - len(t)) for t in tables]), seq_of_token=ints([i for i, _ in where]))
+    h = torch.randn(sum(new), width, device=DEV).bfloat16()
+    start = torch.randn(sum(pages) * page, G * 2 * d, device=DEV).bfloat16()
+    for _ in range(2):
+        layer.runs[layer.add_run()].block_size = page
+    calls, seen = [], []
+    one_pass, says = kernels.qkv_project_store, kernels.qkv_streams
+    monkeypatch.setattr(kernels, "qkv_project_store", lambda *a, **k: calls.append(1) or one_pass(*a, **k))
+    if hook:
+        layer.inp.register_forward_hook(lambda *_: seen.append(1))
+
+    def forward():
+        for own in layer.runs:
+            own.cache = start.clone()
+        set_context(True, **step)
+        y = layer(h, positions, run=1)
+        reset_context()
+        assert torch.equal(layer.runs[0].cache, start)
+        return y, layer.runs[1].cache
+    got, cache = forward()
+    assert len(calls) == (0 if hook else 1) and len(seen) == (1 if hook else 0)
+    monkeypatch.setattr(kernels, "qkv_streams", lambda *_: False)
+    want, cache2 = forward()
+    assert len(calls) == (0 if hook else 1) and says(h, layer.inp.weight, H, G, d, d, 32, False)
+    rest = torch.ones(start.size(0), dtype=torch.bool, device=DEV)
+    rest[slots.long()] = False
+    assert torch.equal(cache[rest], start[rest])
+    # the product behind a module is on the same tiles here (kernels.linear_streams), so the sums are the same
+    assert torch.equal(got, want) and torch.equal(cache, cache2)
