@@ -431,24 +431,26 @@ def gemm_stream(x, w, bias=None, out=None, silu_mul=False):
 
 def gemm_many_rows_streams(M, w, silu_mul) -> bool:
     """Whether nv_gemm_stream is not slower than the vendor library's route for M rows without a bias.  Both, us, library first; share: tile_share.
-     * gate/up, weights in tiles: K below 4096, up to 8191 from a share of 0.8 (16384 rows 1024 -> 2 x 3072 232 and 175, 4096 rows
-       4096 -> 2 x 12288 667 and 564, 8192 rows 3584 -> 2 x 18944 1916 and 1527; 5402 rows 7040 -> 2 x 2048, 0.71, 276 and 309; 16249 rows
-       8192 -> 2 x 13056 5249 and 5429); of 73 shapes of K 2048 to 7680 above the line two are slower, by 0.5 %, the mean is 1.22x;
-     * gate/up, weights to be expanded: K below 2048, up to 8191 from a share of 0.85 where K is below 4608 or 6144 columns and more (int4: 8192
-       rows 3584 -> 2 x 18944 1937 and 1637; 7872 rows 6144 -> 2 x 1536, 0.78, 251 and 296; 4213 rows 6912 -> 2 x 1792 170 and 182): of 55 none is
-       slower, 1.14x;
+     * gate/up, weights in tiles: K below 4096, below 7424 from a share of 0.8 (16384 rows 1024 -> 2 x 3072 233 and 188, 4096 rows
+       4096 -> 2 x 12288 660 and 553, 8192 rows 3584 -> 2 x 18944 1895 and 1526; 5402 rows 7040 -> 2 x 2048, 0.71, 269 and 304; 18351 rows
+       7424 -> 2 x 9216 3721 and 3973; 16249 rows 8192 -> 2 x 13056 5156 and 5397);
+     * gate/up, weights to be expanded: K below 2048, below 7424 from a share of 0.85 where K is below 4608 or 6144 columns and more (int4: 8192
+       rows 3584 -> 2 x 18944 1897 and 1634; 7872 rows 6144 -> 2 x 1536, 0.78, 244 and 288; 4213 rows 6912 -> 2 x 1792 165 and 179; int8, 20289
+       rows 8064 -> 2 x 8160 3849 and 4040).  Of 100 gate/up products of K 512 to 7423 above these lines, in all formats and both 16-bit types,
+       none is over 1 % slower, the mean is 1.20x;
      * other products of more than 1024 columns, weights in tiles, which the library has to have written out: K 512 to 1023 from a share of
        0.7, to 1536 of 0.74, to 3584 of 0.9 (13422 rows 512 -> 4864 87 and 71, 9741 rows 1024 -> 2560 58 and 54, 13741 rows 2048 -> 3584 153 and 148;
-       1024 columns tie: 16384 rows 2048 -> 1024 54 and 52, 14600 rows 3072 -> 1024, 0.89, 71 and 76; 6947 rows 1024 -> 2560, 0.57, 49 and 50; 14240 rows 4096 -> 8192 631 and 692): of 167 above the
-       line one is over 2 % slower (9), the mean is 1.21x;
+       1024 columns tie: 16384 rows 2048 -> 1024 54 and 52, 14600 rows 3072 -> 1024, 0.89, 71 and 76; 6947 rows 1024 -> 2560, 0.57, 49 and 50;
+       14240 rows 4096 -> 8192 631 and 692);
      * K 512 to 1023 and columns that do not split into tiles from a share of 0.6, 0.8 where the weight has to be expanded (16384 rows 896 -> 896,
-       0.88: 43 and 30, int4 43 and 33; 11000 rows 896 -> 640, 0.42: 21 and 27)."""
+       0.88: 43 and 30, int4 43 and 33; 11000 rows 896 -> 640, 0.42: 21 and 27).  Of 150 products of K 512 to 3584 above these two lines two are
+       over 3 % slower (14230 rows 2944 -> 9120 544 and 568; 24340 rows 3200 -> 3840 412 and 431), the mean is 1.22x."""
     N, K, share = w.out_features, w.in_features, tile_share(M, w.out_features)
     tiled = w.fmt == _C.W_DENSE_TILED
     if silu_mul:
         if tiled:
-            return K < 4096 or (K < 8192 and share >= 0.8)
-        return K < 2048 or (K < 8192 and share >= 0.85 and (K < 4608 or N >= 6144))
+            return K < 4096 or (K < 7424 and share >= 0.8)
+        return K < 2048 or (K < 7424 and share >= 0.85 and (K < 4608 or N >= 6144))
     if K < 512:
         return False
     if K < 1024 and N % 256 != 0 and share >= (0.6 if tiled else 0.8):
@@ -715,19 +717,19 @@ def linear(x, w, bias=None, out=None, out_dtype=None, *, rows=None, a_rows=None,
 
 def linear_streams(M, n, K, out_dtype) -> bool:
     """Whether nv_linear forms a plain product of MANY_ROWS rows and more instead of the vendor library.  Both, us, library first:
-     * widths that do not split into the library's tiles, from a share of 0.7 (tile_share), 0.78 beyond K = 1024: 12300 rows 1024 -> 3088 into
-       fp32, share 0.79, 107 and 88; 16384 rows 2048 -> 4112, 0.83, 314 and 277; 6000 rows 1024 -> 3088, 0.60, 56 and 57.  Of 192 shapes of K
-       256 to 4096 above the line one is over 3 % slower (3.3), the mean is 1.36x;
-     * others only into fp32, which costs the library more beside 16 bits: K 512 to 1023 from a share of 0.7 (8192 rows 512 -> 4096: 56 and 45),
-       beyond 0.9 and up to 6144 columns (16384 rows 2048 -> 6144: 340 and 324, 2048 -> 2048 116 and 107; 24000 rows 1024 -> 8192 411 and 441).  Of
-       91 above the line one is 4 % slower, the mean is 1.13x.
-    """
+     * widths that do not split into the library's tiles, from a share of 0.7 (tile_share), 0.78 for K 1025 to 4096: 12300 rows 1024 -> 3088 into
+       fp32, share 0.79, 107 and 88; 16384 rows 2048 -> 4112, 0.83, 314 and 277; 6000 rows 1024 -> 3088, 0.60, 56 and 57; 11517 rows 4864 ->
+       3248, 0.78, 276 and 312; 12812 rows 12160 -> 1168, 0.89, 275 and 297.  Of 101
+       of K 256 to 4096 above the line two are over 3 % slower (4), the mean is 1.22x;
+     * others of up to 6144 columns, and only into fp32, which costs the library more beside 16 bits: K 512 to 1023 from a share of 0.7 (8192 rows
+       512 -> 4096: 56 and 45), to 3584 from 0.9 (16384 rows 2048 -> 6144: 340 and 324, 2048 -> 2048 116 and 107; 24000 rows 1024 -> 8192 411
+       and 441; 20404 rows 3712 -> 4608 531 and 560).  Of 29 above the line none is slower, the mean is 1.11x."""
     if M > LINEAR_ROWS or n <= 1024 and n % 256:
         return False
     share = tile_share(M, n)
     if n % 256:
-        return share >= (0.7 if K <= 1024 else 0.78)
-    return out_dtype == torch.float32 and K >= 512 and n <= 6144 and share >= (0.7 if K < 1024 else 0.9)
+        return K <= 4096 and share >= (0.7 if K <= 1024 else 0.78)
+    return out_dtype == torch.float32 and 512 <= K <= 3584 and n <= 6144 and share >= (0.7 if K < 1024 else 0.9)
 
 
 def tile_share(M, n) -> float:
@@ -1258,16 +1260,18 @@ def qk_rotate_store(proj, offsets, positions, scale, slot_mapping, cache, heads,
 
 def qkv_streams(x, w, heads, kv_heads, dim, vdim, rot_dims, interleaved) -> bool:
     """Whether qkv_project_store takes these prompt rows and is not slower than a product and qk_rotate_store: bf16, heads of 64 or 128, a
-    rotation in halves of 16 numbers and more or none, and results that fill their rounds of tiles to 0.7 (tile_share).  Both, us: 16384 rows
-    2048 -> 4112, share 0.83, 389 and 259; 5000 rows 1536 -> 4632, 0.75, 104 and 98; 5000 rows 2048 -> 3104, 0.50, 88 and 110.  Of 84 shapes of
-    512 to 2048 columns of x above the line none is slower, the mean is 1.24x."""
+    rotation in halves of 16 numbers and more or none, K up to 12288, and results that fill their rounds of tiles (tile_share) to 0.7, beyond
+    K = 2048 to 0.78.  Both, us: 16384 rows 2048 -> 4112, share 0.83, 389 and 259; 5000 rows 1536 -> 4632, 0.75, 104 and 98; 5000 rows 2048 -> 3104,
+    0.50, 88 and 110; 18618 rows 8704 -> 4112, 0.91, 1148 and 1055; 9692 rows 10496 -> 3600, 0.73, 609 and 678.  Of 100 shapes of K
+    512 to 12288 above the line none is slower, the mean is 1.25x."""
     M, N, K = x.size(0), w.size(0), w.size(1)
     return (M >= MANY_ROWS and x.dtype == w.dtype == torch.bfloat16 and x.dim() == 2 and x.stride(1) == 1 and w.is_contiguous()
-            and x.size(1) == K and use_many_rows_path(M, K, 16) and K < 1 << 22 and N < 1 << 20 and dim in (64, 128)
+            and x.size(1) == K and use_many_rows_path(M, K, 16) and K <= 12288 and N < 1 << 20 and dim in (64, 128)
             and kv_heads > 0 and heads % kv_heads == 0 and kv_heads * vdim % 16 == 0 and vdim > 0
             and rot_dims in (0, 32, 64, 128) and rot_dims <= dim and not (interleaved and rot_dims)
             and x.stride(0) % 8 == 0 and K <= x.stride(0) < 1 << 30 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and M <= LINEAR_ROWS and -(-M // 256) * -(-N // 256) <= 256 * 510 and tile_share(M, N) >= 0.7)
+            and M <= LINEAR_ROWS and -(-M // 256) * -(-N // 256) <= 256 * 510
+            and tile_share(M, N) >= (0.7 if K <= 2048 else 0.78))
 
 
 def qkv_project_store(x, w, positions, scale, slot_mapping, cache, heads, kv_heads, dim, vdim, *, inv_freq=None, rot_dims=0, mscale=1.0):

@@ -11,15 +11,23 @@ TILED, INT4 = _C.W_DENSE_TILED, _C.W_INT4
 
 
 @pytest.mark.parametrize("M,N,K,fmt,silu,own", [
-    (4096, 24576, 3968, TILED, True, True), (8192, 16384, 8064, TILED, True, True), (8192, 16384, 8192, TILED, True, False),
+    (4096, 24576, 3968, TILED, True, True), (8192, 16384, 7296, TILED, True, True), (8192, 16384, 7424, TILED, True, False),
     (5402, 4096, 7040, TILED, True, False), (5402, 4096, 3968, TILED, True, True), (16384, 6144, 1920, INT4, True, True),
-    (8192, 37888, 3584, INT4, True, True), (7872, 3072, 6144, INT4, True, False), (4096, 3584, 4608, INT4, True, False),
+    (8192, 37888, 3584, INT4, True, True), (8192, 37888, 7296, INT4, True, True), (8192, 37888, 7424, INT4, True, False), (7872, 3072, 6144, INT4, True, False), (4096, 3584, 4608, INT4, True, False),
     (16384, 1024, 384, TILED, False, False), (16384, 2048, 3584, TILED, False, True), (16384, 2048, 3712, TILED, False, False),
     (14600, 1024, 3072, TILED, False, False), (16384, 1024, 1024, TILED, False, False), (16384, 896, 896, INT4, False, True),
     (16384, 2048, 1024, INT4, False, False)])
 def test_lines(M, N, K, fmt, silu, own):
     w = types.SimpleNamespace(out_features=N, in_features=K, fmt=fmt)
     assert kernels.gemm_many_rows_streams(M, w, silu) is own
+
+
+@pytest.mark.parametrize("M,n,K,dt,own", [
+    (16384, 4112, 4096, torch.bfloat16, True), (16384, 4112, 4224, torch.bfloat16, False), (16384, 4112, 4096, torch.float32, True),
+    (16384, 4112, 12288, torch.float32, False), (16384, 2048, 3584, torch.float32, True), (16384, 2048, 3712, torch.float32, False),
+    (16384, 2048, 2048, torch.bfloat16, False), (8192, 6144, 512, torch.float32, True), (8192, 8192, 512, torch.float32, False)])
+def test_plain_lines(M, n, K, dt, own):
+    assert kernels.linear_streams(M, n, K, dt) is own
 
 
 def test_rotation_lines():

@@ -62,6 +62,9 @@ def test_which_calls_take_it():
     assert not kernels.qkv_streams(x[:4095], w, 16, 2, 128, 128, 32, False)          # too few rows
     assert not kernels.qkv_streams(x[:8192], w, 16, 2, 128, 128, 32, False)          # a share of 0.68
     assert not kernels.qkv_streams(x, w, 16, 2, 128, 128, 32, True)                  # pairs next to each other
+    shapes = [kernels.qkv_streams(torch.empty(M, K, device=DEV, dtype=torch.bfloat16), torch.empty(2576, K, device=DEV, dtype=torch.bfloat16), 16, 2,
+                                  128, 128, 32, False) for M, K in ((9500, 2048), (9500, 2176), (16384, 12288), (16384, 12416))]
+    assert shapes == [True, False, True, False]      # beyond K = 2048 a share of 0.78 (9500 rows: 0.73), to 12288
     assert not kernels.qkv_streams(x, w, 32, 4, 32, 64, 32, False)                   # heads of 32
     assert not kernels.qkv_streams(x, w, 15, 2, 128, 128, 32, False)                 # heads that do not divide: refused behind it
     assert not kernels.qkv_streams(x.float(), w.float(), 16, 2, 128, 128, 32, False)
