@@ -36,7 +36,7 @@ __device__ __forceinline__ u32x4 pack8(const float* v) {
   return u32x4{pack2<bf16_t>(v[0], v[1]), pack2<bf16_t>(v[2], v[3]), pack2<bf16_t>(v[4], v[5]), pack2<bf16_t>(v[6], v[7])};
 }
 
-template <typename TT, typename TO, int EPI>
+template <typename TT, typename TO, int EPI, bool FAR_UPS = false>     // FAR_UPS: a gated product's ups lie 4 GiB and more from their gates
 struct LinearJob {
   typedef TT T;
   static constexpr int BM = STREAM_BM, MT = 8, NT = 4;              // four wavefronts along the columns
@@ -96,22 +96,25 @@ struct LinearJob {
     const int s = min(at.lo + r, at.hi - 1);
     return (uint32_t)(p.a_rows ? p.a_rows[s] : s);
   }
+  // W's rows from the tile's first on; gates and ups within 4 GiB from the matrix's first
+  static constexpr bool MOVES = !GLU || FAR_UPS;
   __device__ __forceinline__ const void* w_base(const StreamTile& at) const {
-    return reinterpret_cast<const T*>(p.w) + at.z * p.w_bs + at.n0 * p.w_rs;
+    return reinterpret_cast<const T*>(p.w) + at.z * p.w_bs + (MOVES ? at.n0 * p.w_rs : 0);
   }
   __device__ __forceinline__ uint32_t w_stride() const { return (uint32_t)p.w_rs * sizeof(T); }
   __device__ __forceinline__ uint64_t w_ups() const { return (uint64_t)p.N * p.w_rs * sizeof(T); }
   __device__ __forceinline__ uint32_t w_row(const StreamTile& at, int r) const {
+    const int n0 = MOVES ? 0 : at.n0, last = MOVES ? p.N - at.n0 - 1 : p.N - 1;
     // a wavefront's 64 rows: 64 columns, or 32 columns' gates and the same columns' ups
-    if constexpr (GLU) return min(32 * (r >> 6) + (r & 31), p.N - at.n0 - 1) + (!UPS && (r & 32) ? p.N : 0);
-    else return min(r, p.N - at.n0 - 1);
+    if constexpr (GLU) return min(n0 + 32 * (r >> 6) + (r & 31), last) + (!UPS && (r & 32) ? p.N : 0);
+    else return min(r, last);
   }
   __device__ __forceinline__ uint32_t w_step() const { return 128; }
   __device__ __forceinline__ bool whole(const StreamTile& at) const {
     return vec && at.lo + BM <= at.hi && at.n0 + NOUT <= p.N;
   }
   static constexpr int NSTORE_WAVE = 2 * NSTORE, EXTRA = 0;
-  static constexpr bool FAR_A = true, FAR_W = false, UPS = GLU && sizeof(T) == 2;      // A's rows may lie anywhere; W's: stream_takes
+  static constexpr bool FAR_A = true, FAR_W = false, UPS = FAR_UPS;      // A's rows may lie anywhere; W's: stream_takes
   __device__ __forceinline__ void fetch_extra(const StreamTile&, int, int, unsigned char*) const {}
   __device__ __forceinline__ void finish(const StreamTile& at, int wm, int wn, int lane, bool live0, bool live1, const unsigned char*) const {
     if (live0) store_wave<0>(at, at.lo + 64 * wm, wn, lane);
@@ -303,9 +306,9 @@ inline bool stream_takes(const LinArgs& p, int esz, int64_t total_rows, int batc
   return p.K * esz >= 256 && p.K * esz % 128 == 0 && p.a_rs >= 0 && p.w_rs >= 0 && p.a_rs < ((int64_t)1 << 30) && p.w_rs < ((int64_t)1 << 30);
 }
 
-template <typename T, typename TO, int EPI>
-LinearJob<T, TO, EPI> linear_job(const LinArgs& p, int batch) {
-  typedef LinearJob<T, TO, EPI> Job;
+template <typename T, typename TO, int EPI, bool FAR_UPS = false>
+LinearJob<T, TO, EPI, FAR_UPS> linear_job(const LinArgs& p, int batch) {
+  typedef LinearJob<T, TO, EPI, FAR_UPS> Job;
   constexpr int64_t unit = sizeof(TO) == 2 ? 8 : 4;
   const int nt = (p.N + Job::NOUT - 1) / Job::NOUT;
   const int vec = p.N % unit == 0 && p.out_rs % unit == 0 && p.out_bs % unit == 0 && (uintptr_t)p.out % 16 == 0;

@@ -11,8 +11,8 @@
 //   * DMA a few at a time: eight products between two instructions; eight of them two apart queue up (8192^3: 756 against 730 us);
 //   * no branch between products in the loop for whole tiles (8192^3: 756 with one per half block, 710 without), and no vector address that
 //     moves with K: the tile's rows are offsets, K is in the scalar base.  A tile's first pair of blocks, whose products are
-//     added to nothing (256 registers less to clear) while stores are still on their way, and tiles with wavefronts that have no rows take
-//     the other loop;
+//     added to nothing (256 registers less to clear) while stores are still on their way, the last pair of an odd number of blocks, and tiles
+//     with wavefronts that have no rows take the other loop (8192 rows 3008 -> 6144, 47 blocks: 205 us, all of them there 257);
 //   * a wavefront has rows 64 of each half of the tile, so a half of 128 rows, or a ragged tile, is half the work for each of them.
 // Results are those of stream_tiles.h, bit for bit: K in the same order.  Measured, before and after (us): the experts' layer of 16384 rows,
 // 2048 -> 2 x 3072 -> 2048, 1424 and 1185; 16384 rows 2048 -> 2 x 6144 with SiLU 738 and 646; 2048 -> 6144 into fp32 376 and 327; 14600
@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
   auto extra = [&](int n) { return lds_raw + 2 * DEEP_BUFFER + STREAM_LIST * sizeof(StreamTile) + (n & 3) * Job::EXTRA; };
   const int blocks = job.K / 64, pairs = (blocks + 1) / 2;
   const bool odd = blocks & 1;
-  StreamTile at = listed(0), ahead = at;
+  StreamTile at = listed(0);
   point(at);
   job.fetch_extra(at, wv, lane, extra(0));
 #pragma unroll
@@ -263,7 +263,7 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
   };
   const std::integral_constant<int, 0> I0;
   const std::integral_constant<int, 1> I1;
-  int left = pairs, tile = 0, next = 0;
+  int left = pairs, tile = 0;
   bool stored = false, live0 = at.lo + 64 * wm < at.hi, live1 = at.lo + 128 + 64 * wm < at.hi;
   auto first = [&]() {
 #pragma unroll
@@ -273,20 +273,20 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
   };
   auto ask_ahead = [&]() {      // with a tile's last pair the next one's first is fetched; behind the last tile that one's again, unused
     if (left > 1) return;
-    if (next + 1 < tiles) ahead = listed(++next);
+    const StreamTile ahead = listed(min(tile + 1, tiles - 1));
     point(ahead);
     job.fetch_extra(ahead, wv, lane, extra(tile + 1));
   };
   for (;;) {
     // Each way reads its first fragments itself: handed from one to the other they would be moved between registers.
-    if (live0 && live1 && !odd && left < pairs) {
+    if (live0 && live1 && left < pairs && left > odd) {
       const std::true_type plain;
       first();
-      for (; left > 0; --left) {
+      for (; left > odd; --left) {
         ask_ahead();
         half(plain, I0, I0, true, false, false);
         half(plain, I0, I1, true, false, false);
-        next_block();
+        if (!(odd && left == 2)) next_block();
         half(plain, I1, I0, true, false, false);
         half(plain, I1, I1, true, false, false);
         next_block();
@@ -298,12 +298,7 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
       ask_ahead();
       half(plain, I0, I0, live0, left == pairs, stored);
       half(plain, I0, I1, live1, left == pairs, stored);
-      next_block();
-      if (odd && left == 2) {      // the last pair has no second block: the first one again, unused
-        abase -= 128;
-        wbase -= w_step;
-        ubase -= w_step;
-      }
+      if (!(odd && left == 2)) next_block();      // the last pair has no second block: the first one again, unused
       const bool full = !odd || left > 1;
       half(plain, I1, I0, live0 && full, false, stored);
       half(plain, I1, I1, live1 && full, false, false);
@@ -317,7 +312,7 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
     job.finish(at, wm, wn, stream_lane(), live0, live1, extra(tile));
     stored = job.whole(at);
     if (++tile == tiles) break;
-    at = ahead;
+    at = listed(tile);
     live0 = at.lo + 64 * wm < at.hi;
     live1 = at.lo + 128 + 64 * wm < at.hi;
   }
