@@ -104,7 +104,7 @@ def _has_all(sources) -> bool:
 
 def _with_needed(names):
     """``names`` and what their sources call in others."""
-    needs = {"linear": ("linear_deep",)}
+    needs = {"linear": ("linear_deep", "linear_eight")}
     return list(dict.fromkeys(m for n in names for m in (n,) + needs.get(n, ())))
 
 

@@ -395,7 +395,7 @@ extern "C" int nv_linear_rows(const void* a, int64_t a_row_stride, const int32_t
     const int cols = epilogue == EPI_GLU ? 2 * N : N;
     const bool has_256 = stream_takes(p, (int)esz, total_rows, batch, cols);
     int tile = pick_wide_tile(M, total_rows, cols, K, batch, group_offsets != nullptr, dtype == NV_F32, has_256);
-    if (const char* force = getenv("NV_LINEAR_TILE")) tile = atoi(force) == TILE_256 && !has_256 ? TILE_128 : atoi(force);
+    if (const char* force = getenv("NV_LINEAR_TILE")) tile = atoi(force) >= TILE_256 && !has_256 ? TILE_128 : atoi(force);
     if (wide_tiles(64, 128, M, total_rows + 64 * batch, cols, batch, group_offsets != nullptr) < (1 << 30)) {
       hipError_t e;
       if (dtype == NV_BF16) {

@@ -40,3 +40,5 @@ __device__ __forceinline__ float unary_act(float v, int act, const float* prm, f
 
 // 16-bit products on the tiles of stream_deep.h (linear_deep.hip); total_rows: of all groups
 hipError_t linear_deep_launch(const LinArgs& p, int epilogue, bool out_16bit, int64_t total_rows, int batch, hipStream_t s);
+// the same on those of stream_tiles.h (linear_eight.hip)
+hipError_t linear_eight_launch(const LinArgs& p, int epilogue, bool out_16bit, int64_t total_rows, int batch, hipStream_t s);

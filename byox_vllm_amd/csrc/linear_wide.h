@@ -263,7 +263,7 @@ hipError_t launch_wide_one(const LinArgs& p, int64_t total_rows, int batch, hipS
 //   * 64 x 128 where they take fewer rounds per CU than two for each of 128 x 128 (2500 by 2048, K 1024, 3 and 2 x 2: 134, 135, 111;
 //     3135 by 4416, 7 and 2 x 4: 255, 265, 247);
 //   * else as in 16 bits.  Of 1430 shapes none is over 3 % slower than with the last rule alone.
-enum { TILE_256 = 2, TILE_128 = 1, TILE_64 = 0 };
+enum { TILE_256 = 2, TILE_128 = 1, TILE_64 = 0, TILE_256_EIGHT = 3, TILE_256_FOUR = 4 };      // the last two: 256 x 256 in 16 bits by so many wavefronts
 inline int64_t wide_tiles(int bm, int bn, int64_t m, int64_t total_rows, int cols, int batch, bool grouped) {
   // groups end inside a tile: half a tile each on average
   return (grouped ? (total_rows + bm - 1) / bm + batch / 2 : (m + bm - 1) / bm * batch) * ((cols + bn - 1) / bn);
@@ -288,9 +288,10 @@ inline int pick_wide_tile(int64_t m, int64_t total_rows, int cols, int K, int ba
 
 template <typename T, typename TO, int EPI>
 hipError_t launch_wide_epi(const LinArgs& p, int64_t total_rows, int batch, int tile, hipStream_t s) {
-  if (tile == TILE_256) {
+  if (tile >= TILE_256) {
     if constexpr (sizeof(T) == 2) {
-      return linear_deep_launch(p, EPI, sizeof(TO) == 2, total_rows, batch, s);
+      const bool four = tile == TILE_256 ? linear_four_wavefronts(p, EPI, sizeof(TO) == 2) : tile == TILE_256_FOUR;
+      return (four ? linear_deep_launch : linear_eight_launch)(p, EPI, sizeof(TO) == 2, total_rows, batch, s);
     } else {
       const auto job = linear_job<T, TO, EPI>(p, batch);
       return launch_stream_tiles(job, linear_job_tiles(p, job.nt, total_rows, batch), s);

@@ -1,8 +1,10 @@
 // Products of many rows: a workgroup per CU walks tiles of 256 x 256 outputs whose K blocks form one stream.
 //
-// Here: fp32, eight wavefronts of 128 x 64 each (16 bits: stream_deep.h, whose tiles, their order and W's rows in LDS are those of this file).
+// Here: eight wavefronts of 128 x 64 each, for fp32 and for 16-bit products whose results take long to form (linear_four_wavefronts); the other
+// 16-bit products: stream_deep.h, whose tiles, their order and W's rows in LDS are those of this file.
 //
-// What bounds it: the matrix cores (v_mfma_f32_16x16x4_f32).
+// What bounds it: the matrix cores (v_mfma_f32_16x16x4_f32; in 16 bits 852 us at 8192 x 8192 x 8192, stream_deep.h 705), two wavefronts to a
+// SIMD, of which one forms results while the other has products.
 //   * 16-row products: a lane's results lie where whole 64-byte pieces of rows can be stored;
 //   * the barrier stands before the block's last step of K, whose fragments are in registers: behind it the first fragments of the
 //     next block are read under that step's products, and the buffer just left is refilled, one DMA instruction behind every few
@@ -39,6 +41,9 @@ constexpr int STREAM_LIST = 512;      // tiles of one workgroup at most
 constexpr int STREAM_BM = 256, STREAM_BN = 256;
 constexpr int STREAM_BUFFER = (STREAM_BM + STREAM_BN) * 128;      // a K block of both
 
+__device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x4 c, bf16_t) {
+  return mfma16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c);
+}
 __device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x4 c, float) {
   // product e takes number 4 g + e of the sixteen that the four groups of lanes hold
 #pragma unroll

@@ -90,6 +90,38 @@ def test_gated_products_without_an_activation_of_their_own(act, out_dtype, monke
         assert torch.equal(got, kernels.linear(x, w, epilogue=kernels.EPI_GLU, out_dtype=out_dtype))
 
 
+@pytest.mark.parametrize("tile", ["3", "4", "2"])      # eight wavefronts, four, by the rule
+@pytest.mark.parametrize("n", [304, 300, 301])
+@pytest.mark.parametrize("biased", [False, True])
+def test_results_by_four_and_eight_wavefronts(tile, n, biased, monkeypatch):
+    """Every epilogue, whole pieces of 16 bytes and numbers one by one, over tiles with and without a neighbour."""
+    from byox_vllm_amd import kernels as k
+    F = torch.nn.functional
+    monkeypatch.setenv("NV_LINEAR_TILE", tile)
+    torch.manual_seed(n)
+    M, K = 700, 192
+    x, w = torch.randn(M, K, device=DEV).bfloat16(), (torch.randn(2 * n, K, device=DEV) * 0.1).bfloat16()
+    bias = torch.randn(2 * n, device=DEV).bfloat16() if biased else None
+    rows, gate, prm = torch.rand(M, device=DEV), torch.randn(M, n, device=DEV), torch.tensor([0.7, 0.4], device=DEV)
+    y = x.double() @ w.double().t() * rows.double()[:, None] + (bias.double() if biased else 0.0)
+    v, u, g = y[:, :n], y[:, n:], torch.sigmoid(gate.double())
+    xielu = torch.where(v > 0, prm[0].double() * v * v, prm[1].double() * (torch.expm1(v) - v)) + 0.5 * v
+    clamped = torch.clamp(v, max=2.0)
+    cases = [(dict(), v), (dict(epilogue=k.EPI_SOFTCAP, cap=3.0), 3.0 * torch.tanh(v / 3.0)),
+             (dict(epilogue=k.EPI_ROW_GATE, gate=gate[:, :1].contiguous(), gate_stride=1), v * g[:, :1]),
+             (dict(epilogue=k.EPI_ROW_GATE, act=k.GATE_PER_NUMBER, gate=gate, gate_stride=n), v * g),
+             (dict(epilogue=k.EPI_ACT, act=k.ACT_SILU), F.silu(v)), (dict(epilogue=k.EPI_ACT, act=k.ACT_GELU_TANH), F.gelu(v, approximate="tanh")),
+             (dict(epilogue=k.EPI_ACT, act=k.ACT_XIELU, gate=prm), xielu), (dict(epilogue=k.EPI_ACT, act=k.ACT_SCALE, cap=0.3), 0.3 * v),
+             (dict(epilogue=k.EPI_ACT, act=k.ACT_GELU_ERF), F.gelu(v)), (dict(epilogue=k.EPI_GLU, act=k.ACT_SILU), F.silu(v) * u),
+             (dict(epilogue=k.EPI_GLU, act=k.ACT_GELU_TANH), F.gelu(v, approximate="tanh") * u),
+             (dict(epilogue=k.EPI_GLU, act=k.GLU_CLAMPED, cap=2.0), clamped * torch.sigmoid(1.702 * clamped) * (torch.clamp(u, -2.0, 2.0) + 1.0))]
+    for args, want in cases:
+        gated = args.get("epilogue") == k.EPI_GLU
+        for out_dtype in (torch.bfloat16, torch.float32):
+            got = k.linear(x, w if gated else w[:n], bias if gated or not biased else bias[:n], out_dtype=out_dtype, row_scale=rows, **args)
+            close(got, want, 16 * K, out_dtype)      # as a product's, and a function that grows by 2 and more where its gate does
+
+
 @pytest.mark.parametrize("M,n,K", [(2100, 1000, 320), (700, 304, 128)])
 def test_silu_is_the_same_in_16_and_32_bits(M, n, K, monkeypatch):
     """Results in 16 bits are those in 32 bits, rounded: SiLU by exp and quotient in both."""
