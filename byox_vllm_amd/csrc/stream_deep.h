@@ -13,7 +13,9 @@
 //     moves with K: the tile's rows are offsets, K is in the scalar base.  A tile's first pair of blocks, whose products are
 //     added to nothing (256 registers less to clear) while stores are still on their way, the last pair of an odd number of blocks, and tiles
 //     with wavefronts that have no rows take the other loop (8192 rows 3008 -> 6144, 47 blocks: 205 us, all of them there 257);
-//   * a wavefront has rows 64 of each half of the tile, so a half of 128 rows, or a ragged tile, is half the work for each of them.
+//   * a wavefront has rows 64 of each half of the tile, so a half of 128 rows, or a ragged tile, is half the work for each of them, in a
+//     loop of its own: half of W's columns to a barrier, products above all reads and DMA (3000 rows 2048 -> 2048, 192 halves: 0.63 of the
+//     time in the loop with branches, where they were 1.07 of eight wavefronts' time; 8192 -> 2048 0.59 and 1.15).
 // Results are those of stream_tiles.h, bit for bit: K in the same order.  Measured, before and after (us): the experts' layer of 16384 rows,
 // 2048 -> 2 x 3072 -> 2048, 1424 and 1185; 16384 rows 2048 -> 2 x 6144 with SiLU 738 and 646; 2048 -> 6144 into fp32 376 and 327; 14600
 // rows 1024 -> 4096 121 and 105; gate/up of 1024 -> 2 x 3072 194 and 177, q/k/v with rotation 150 and 134.
@@ -162,9 +164,9 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
     if constexpr (Order::TILED) wat[s] = Order::place(4 * wn) + Order::frag(fr) + 1024 * s + 256 * g;
     else wat[s] = in + 64 * wn * 128 + Order::frag(fr);
   }
-  auto read_a = [&](int bo, int h, int r) {      // r: which of the eight
+  auto read_a = [&](int bo, int h, int r, int set) {      // r: which of the eight
     const int s = r >> 2, i = r & 3;
-    fa[h][i][s] = *reinterpret_cast<const u32x4*>(lds_raw + bo + h * DEEP_PA + aat[s] + 2048 * i);
+    fa[set][i][s] = *reinterpret_cast<const u32x4*>(lds_raw + bo + h * DEEP_PA + aat[s] + 2048 * i);
   };
   auto read_w = [&](int bo, int h, int r) {
     const int s = r >> 2, j = r & 3;
@@ -197,32 +199,37 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
   // read and the pieces of LDS that were read before the barrier are filled again, in this order.  What is waited for was asked for
   // three halves before: sixteen operations are younger, and a tile's stores where they came between (`behind`).
   constexpr int BEHIND = 16 + Job::NSTORE_WAVE < 63 ? 16 + Job::NSTORE_WAVE : 63;
+  auto arrive = [&](bool behind) {
+    if (behind) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BEHIND) : "memory");
+    else asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory", DEEP_REGISTERS);
+  };
+  auto refill = [&](auto bb, auto ss, int k) {
+    constexpr int B = decltype(bb)::value, S = decltype(ss)::value, here = B * DEEP_BUFFER;
+    if constexpr (S == 0) {
+      if (k < 4) fill_a(here, 0, k);
+      else fill_w(here, B, k - 4);
+    } else {
+      if (k < 4) fill_w(here, 1 - B, k);
+      else fill_a(here, 1, k - 4);
+    }
+  };
   auto half = [&](auto plain, auto bb, auto ss, bool live, bool fresh, bool behind) {
     constexpr bool PLAIN = decltype(plain)::value;
     constexpr int B = decltype(bb)::value, S = decltype(ss)::value, X = B, Y = 1 - B;
     constexpr int here = B * DEEP_BUFFER, there = (1 - B) * DEEP_BUFFER;
-    if (!PLAIN && behind) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BEHIND) : "memory");
-    else asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory", DEEP_REGISTERS);
+    arrive(!PLAIN && behind);
     auto reads = [&](int m) {
       if constexpr (S == 0) {
         if (m < 8) read_w(here, Y, m);
-        else if (m < 16) read_a(here, 1, m - 8);
+        else if (m < 16) read_a(here, 1, m - 8, 1);
       } else {
-        if (m < 8) read_a(there, 0, m);
+        if (m < 8) read_a(there, 0, m, 0);
         else if (m >= 32 && m < 40) read_w(there, Y, m - 32);
       }
     };
-    auto fills = [&](int k) {
-      if constexpr (S == 0) {
-        if (k < 4) fill_a(here, 0, k);
-        else fill_w(here, X, k - 4);
-      } else {
-        if (k < 4) fill_w(here, Y, k);
-        else fill_a(here, 1, k - 4);
-      }
-    };
+    auto fills = [&](int k) { refill(bb, ss, k); };
     auto product = [&](int m, auto is_new) {
       const int hw = (m < 32) == (S == 0) ? X : Y, s = (m >> 4) & 1, j = (m >> 2) & 3, i = m & 3;
       deep_mma<decltype(is_new)::value>(deep_at(S, 4 * hw + j, i), fw[hw][j][s], fa[S][i][s], T{});
@@ -261,13 +268,31 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
       __builtin_amdgcn_sched_barrier(0);
     }
   };
+  // The same for a wavefront that has rows in the tile's first half alone: half of W's columns in each half, so that reads and refills have
+  // products above them; A's fragments in either set by turns, W's behind the last of their products.
+  auto narrow = [&](auto bb, auto ss) {
+    constexpr int B = decltype(bb)::value, S = decltype(ss)::value, Y = 1 - B, hw = S == 0 ? B : Y;
+    constexpr int here = B * DEEP_BUFFER, there = (1 - B) * DEEP_BUFFER;
+    arrive(false);
+#pragma unroll
+    for (int m = 0; m < 32; ++m) {
+      const int s = m >> 4, j = (m >> 2) & 3, i = m & 3;
+      deep_mma(deep_at(0, 4 * hw + j, i), fw[hw][j][s], fa[B][i][s], T{});
+      __builtin_amdgcn_sched_barrier(0);
+      if (S == 0 && m < 8) read_w(here, Y, m);
+      if (S == 1 && m < 8) read_a(there, 0, m, 1 - B);
+      if (S == 1 && i == 3) read_w(there, Y, m >> 2);      // in place of the fragment that has been multiplied
+      if (m % 4 == 1) refill(bb, ss, m / 4);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
   const std::integral_constant<int, 0> I0;
   const std::integral_constant<int, 1> I1;
   int left = pairs, tile = 0;
   bool stored = false, live0 = at.lo + 64 * wm < at.hi, live1 = at.lo + 128 + 64 * wm < at.hi;
   auto first = [&]() {
 #pragma unroll
-    for (int r = 0; r < 8; ++r) read_a(0, 0, r);
+    for (int r = 0; r < 8; ++r) read_a(0, 0, r, 0);
 #pragma unroll
     for (int r = 0; r < 8; ++r) read_w(0, 0, r);
   };
@@ -291,9 +316,21 @@ __global__ __launch_bounds__(256, 1) void stream_deep_kernel(Job job) {
         half(plain, I1, I1, true, false, false);
         next_block();
       }
+    } else if (live0 && !live1 && left < pairs && left > odd) {
+      asm volatile("; half" ::: "memory");
+      first();
+      for (; left > odd; --left) {
+        ask_ahead();
+        narrow(I0, I0);
+        narrow(I0, I1);
+        if (!(odd && left == 2)) next_block();
+        narrow(I1, I0);
+        narrow(I1, I1);
+        next_block();
+      }
     } else {
       const std::false_type plain;
-      asm volatile("; not all" ::: "memory");      // or the reads of both ways become one, ahead of them
+      asm volatile("; not all" ::: "memory");      // or the reads of all ways become one, ahead of them
       first();
       ask_ahead();
       half(plain, I0, I0, live0, left == pairs, stored);
