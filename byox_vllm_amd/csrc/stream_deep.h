@@ -14,7 +14,7 @@
 //     added to nothing (256 registers less to clear) while stores are still on their way, the last pair of an odd number of blocks, and tiles
 //     with wavefronts that have no rows take the other loop (8192 rows 3008 -> 6144, 47 blocks: 205 us, all of them there 257);
 //   * a wavefront has rows 64 of each half of the tile, so a half of 128 rows, or a ragged tile, is half the work for each of them, in a
-//     loop of its own: half of W's columns to a barrier, products above all reads and DMA (3000 rows 2048 -> 2048, 192 halves: 0.63 of the
+//     loop of its own: half of W's columns to a barrier, products above all reads and DMA (3000 rows 2048 -> 2048, 192 halves: 0.67 of the
 //     time in the loop with branches, where they were 1.07 of eight wavefronts' time; 8192 -> 2048 0.59 and 1.15).
 // Results are those of stream_tiles.h, bit for bit: K in the same order.  Measured, before and after (us): the experts' layer of 16384 rows,
 // 2048 -> 2 x 3072 -> 2048, 1424 and 1185; 16384 rows 2048 -> 2 x 6144 with SiLU 738 and 646; 2048 -> 6144 into fp32 376 and 327; 14600
