@@ -4,8 +4,8 @@
 //
 // What bounded these steps: the vendor library's product, then a pass over its whole result that moves it twice.  14.6 k rows of 1024
 // (Qwen3-0.6B): gate and up 157 us and SiluAndMul 53, q/k/v 105 and rotation with the store 61, and 5 - 7 us before each for the
-// weight as rows.  Here 176 and 136 us (203 and 151 on the tiles of eight wavefronts).  What the results cost counts: with one wavefront to a
-// SIMD nothing hides it.  So SiLU in 17 instructions (anyt.h; with silu_f32's 27: 190), roundings two at a time, and a row's cosines and sines,
+// weight as rows.  Here 170 and 142 us (193 and 157 on the tiles of eight wavefronts).  What the results cost counts: with one wavefront to a
+// SIMD nothing hides it.  So SiLU in 17 instructions (anyt.h; silu_f32's 27: 8 % more), roundings two at a time, and a row's cosines and sines,
 // norm weights and bias on their way before they are needed.  Which sizes this pays for: kernels.gemm_many_rows and kernels.rotation_streams.
 #include <type_traits>
 

@@ -2,8 +2,8 @@
 // stream_deep.h, rotated, scaled and stored on the way: fp32 queries, cache rows [k | v] in bf16, the other columns in fp32.
 //
 // What bounded these steps: the projection was written in fp32 and read again.  16384 rows 2048 -> 16 + 8 + 8 heads of 128 and 16 gates: the
-// product 277 us and qk_pairs_store_kernel 110; here 259, the turns' cosines and sines, once per token, among them (the layer 636 and 532).  The
-// arithmetic is that of qk_pairs_store_kernel.  Which sizes it pays for: kernels.qkv_streams.
+// product 277 us and qk_pairs_store_kernel 110; here 240, the turns' cosines and sines, once per token, among them (the layer 670 and 516).  The
+// arithmetic is that of qk_pairs_store_kernel, over the same product bit for bit.  Which sizes it pays for: kernels.qkv_streams.
 #include "anyt.h"
 #include "stream_deep.h"
 

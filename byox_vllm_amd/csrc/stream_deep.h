@@ -16,9 +16,9 @@
 //   * a wavefront has rows 64 of each half of the tile, so a half of 128 rows, or a ragged tile, is half the work for each of them, in a
 //     loop of its own: half of W's columns to a barrier, products above all reads and DMA (3000 rows 2048 -> 2048, 192 halves: 0.67 of the
 //     time in the loop with branches, where they were 1.07 of eight wavefronts' time; 8192 -> 2048 0.59 and 1.15).
-// Results are those of stream_tiles.h, bit for bit: K in the same order.  Measured, before and after (us): the experts' layer of 16384 rows,
-// 2048 -> 2 x 3072 -> 2048, 1424 and 1185; 16384 rows 2048 -> 2 x 6144 with SiLU 738 and 646; 2048 -> 6144 into fp32 376 and 327; 14600
-// rows 1024 -> 4096 121 and 105; gate/up of 1024 -> 2 x 3072 194 and 177, q/k/v with rotation 150 and 134.
+// The sums are those of stream_tiles.h, bit for bit: K in the same order.  Measured, eight wavefronts and these (us): the experts' layer of 16384
+// rows, 2048 -> 2 x 3072 -> 2048, 1401 and 1143; 16384 rows 2048 -> 2 x 6144 with SiLU 734 and 607; 2048 -> 6144 into fp32 349 and 329; 14600 rows
+// 1024 -> 4096 114 and 105; gate/up of 1024 -> 2 x 3072 193 and 170, q/k/v with rotation 157 and 142.
 // Job: as for stream_tiles.h, and
 //   bool FAR_A, FAR_W                     whether a tile's rows of A (W) may lie 4 GiB and more from its base
 //   bool UPS, w_ups()                     whether W's rows 32 - 63 of every 64 lie another w_ups() bytes on (which may be 4 GiB and more)

@@ -1261,7 +1261,7 @@ def qk_rotate_store(proj, offsets, positions, scale, slot_mapping, cache, heads,
 def qkv_streams(x, w, heads, kv_heads, dim, vdim, rot_dims, interleaved) -> bool:
     """Whether qkv_project_store takes these prompt rows and is not slower than a product and qk_rotate_store: bf16, heads of 64 or 128, a
     rotation in halves of 16 numbers and more or none, K up to 12288, and results that fill their rounds of tiles (tile_share) to 0.7, beyond
-    K = 2048 to 0.78.  Both, us: 16384 rows 2048 -> 4112, share 0.83, 389 and 259; 5000 rows 1536 -> 4632, 0.75, 104 and 98; 5000 rows 2048 -> 3104,
+    K = 2048 to 0.78.  Both, us: 16384 rows 2048 -> 4112, share 0.83, 389 and 241; 5000 rows 1536 -> 4632, 0.75, 104 and 98; 5000 rows 2048 -> 3104,
     0.50, 88 and 110; 18618 rows 8704 -> 4112, 0.91, 1148 and 1055; 9692 rows 10496 -> 3600, 0.73, 609 and 678.  Of 100 shapes of K
     512 to 12288 above the line none is slower, the mean is 1.25x."""
     M, N, K = x.size(0), w.size(0), w.size(1)
