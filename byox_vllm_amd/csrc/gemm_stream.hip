@@ -171,7 +171,9 @@ struct RowsJob {
       is_k[h] = !is_q[h] && hs[h] < ra.H + ra.Hkv;
     }
     const bool turns = n0 < (ra.H + ra.Hkv) * D;
-    auto kept = [&](int r, int which) { return *reinterpret_cast<const uint32_t*>(extra + 1024 * which + 4 * (128 * (r >> 2) + 64 * wm + 16 * (r & 3) + fr)); };
+    auto kept = [&](int r, int which) {
+      return *reinterpret_cast<const uint32_t*>(extra + 1024 * which + 4 * (128 * (r >> 2) + 64 * wm + 16 * (r & 3) + fr));
+    };
     f32x4 turn[2][2 * Q];      // cosines, then sines
     auto ask = [&](int r) {
       if (!turns) return;

@@ -1,6 +1,6 @@
 // nv_linear for many rows: the products, groups and epilogues of LinArgs on the tiles of stream_tiles.h (fp32, and 16 bits in linear_eight.hip)
-// and stream_deep.h (16 bits, linear_deep.hip).  Groups (experts) of unknown size: every workgroup counts the tiles from the offsets with one wavefront-wide prefix
-// sum; a group that ends in the upper half of a tile's rows costs the half.
+// and stream_deep.h (16 bits, linear_deep.hip).  Groups (experts) of unknown size: every workgroup counts the tiles from the offsets with one
+// wavefront-wide prefix sum; a group that ends in the upper half of a tile's rows costs the half.
 #pragma once
 #include <type_traits>
 
@@ -302,7 +302,6 @@ struct LinearJob {
 inline bool stream_takes(const LinArgs& p, int esz, int64_t total_rows, int batch, int cols) {
   const int64_t rows = p.group_off ? total_rows / 256 + batch : (p.M + 255) / 256 * batch;
   if (total_rows >= ((int64_t)1 << 31) || rows * ((cols + 255) / 256) > 256 * (STREAM_LIST - 2)) return false;
-  if (esz == 2 && p.w_rs >= ((int64_t)1 << 23)) return false;      // a 16-bit tile's 256 rows of W lie within 4 GiB
   return p.K * esz >= 256 && p.K * esz % 128 == 0 && p.a_rs >= 0 && p.w_rs >= 0 && p.a_rs < ((int64_t)1 << 30) && p.w_rs < ((int64_t)1 << 30);
 }
 
@@ -311,13 +310,15 @@ inline bool stream_vec(const LinArgs& p, bool out_16bit) {      // whether a row
   return p.N % unit == 0 && p.out_rs % unit == 0 && p.out_bs % unit == 0 && (uintptr_t)p.out % 16 == 0;
 }
 
+// stream_deep.h has a tile's 256 rows of W within 4 GiB, stream_tiles.h anywhere
+inline bool stream_deep_takes(const LinArgs& p) { return p.w_rs < ((int64_t)1 << 23); }
+
 // Whether a 16-bit product's 256 x 256 tiles are four wavefronts' (stream_deep.h) or eight's (stream_tiles.h).  Four are faster over K (0.8 - 0.9 of
 // the time at long K), but alone on their SIMDs: nothing runs under the chains of instructions of a result's function, its gate or bias fetched for it
 // alone, stores of single numbers.  Results that eight take longer for, because they fetch a bias where it is added, are four's from the first
 // K on.  Four against eight, 16384 rows by 2048, bf16: plain K 192 0.97, 256 0.89 (6000 by 1536 1.09, 0.97); with a bias 0.61; SiLU 512 1.07, 1024
-// 1.01; GELU 2048 1.08, 4096 0.99, with a bias 512 1.05, 1024 1.01, gated 192 1.08, 512 0.95; xIELU 4096 1.07, 8192 0.91; soft cap 2048 1.05, 4096 0.97; a gate for every
-// number 4096 1.13, 8192 0.97; 2044 columns and a bias 4096 1.04, 8192 0.92, gated 2048 1.24, 8192 0.90.  Fewer than 128 tiles, where four are
-// slower beyond K = 2048, go to tiles of 128 x 128 (pick_wide_tile).
+// 1.01; GELU 2048 1.08, 4096 0.99, with a bias 512 1.05, 1024 1.01, gated 192 1.08, 512 0.95; xIELU 4096 1.07, 8192 0.91; soft cap 2048 1.05,
+// 4096 0.97; a gate for every number 4096 1.13, 8192 0.97; 2044 columns and a bias 4096 1.04, 8192 0.92, gated 2048 1.24, 8192 0.90.
 inline bool linear_four_wavefronts(const LinArgs& p, int epi, bool out_16bit) {
   static const int from[11][4] = {      // K from which four are faster: 16 bytes at a time, and a bias; numbers one by one, and a bias
       {256, 0, 512, 8192},              // plain

@@ -253,8 +253,8 @@ hipError_t launch_wide_one(const LinArgs& p, int64_t total_rows, int batch, hipS
 // Which tile: the one whose launch takes the fewest chip-wide rounds of tile area, each by what it reaches when the chip is
 // full (bf16, 32768 rows by 6144 columns of K 2048: 742 and 608 TFLOP/s in the tiles of 128 x 128 and 64 x 128, of which two share a CU; the
 // streams of 256 x 256, which have one to themselves, reach 1150 at the K of the smallest products that they are taken for and 1550 at the largest:
-// of 629 shapes of 256 to 8192 rows this picks the fastest within 0.5 % on average, 26 of them more than 5 % off).  A last round of 256 x 256 that half of the chip would have is dealt in halves and
-// costs 0.85 of a round (12000 rows by 2048, K 1024, 1.5 rounds: 65 us, 128 x 128 93, 64 x 128 88; 4096 by 2048, half a round:
+// of 629 shapes of 256 to 8192 rows this picks the fastest within 0.5 % on average, 26 of them more than 5 % off).  A last round of 256 x 256
+// that half of the chip would have is dealt in halves and costs 0.85 of a round, in 16 bits on four wavefronts less (12000 rows by 2048, K 1024, 1.5 rounds: 65 us, 128 x 128 93, 64 x 128 88; 4096 by 2048, half a round:
 // 29.4, 29.3, 33; 5000 by 1536, K 1536: 38, 34, 43).
 // fp32 is bound by its matrix instructions alone: a workgroup that has a CU to itself is twice as fast as one of two.  So, from K 256 on
 // (us of 256 x 256, 128 x 128 and 64 x 128; a tile's beginning and end weigh more below):
@@ -263,7 +263,7 @@ hipError_t launch_wide_one(const LinArgs& p, int64_t total_rows, int batch, hipS
 //   * 64 x 128 where they take fewer rounds per CU than two for each of 128 x 128 (2500 by 2048, K 1024, 3 and 2 x 2: 134, 135, 111;
 //     3135 by 4416, 7 and 2 x 4: 255, 265, 247);
 //   * else as in 16 bits.  Of 1430 shapes none is over 3 % slower than with the last rule alone.
-enum { TILE_256 = 2, TILE_128 = 1, TILE_64 = 0, TILE_256_EIGHT = 3, TILE_256_FOUR = 4 };      // the last two: 256 x 256 in 16 bits by so many wavefronts
+enum { TILE_256 = 2, TILE_128 = 1, TILE_64 = 0, TILE_256_EIGHT = 3, TILE_256_FOUR = 4 };      // the last two: in 16 bits by so many wavefronts
 inline int64_t wide_tiles(int bm, int bn, int64_t m, int64_t total_rows, int cols, int batch, bool grouped) {
   // groups end inside a tile: half a tile each on average
   return (grouped ? (total_rows + bm - 1) / bm + batch / 2 : (m + bm - 1) / bm * batch) * ((cols + bn - 1) / bn);
@@ -290,7 +290,7 @@ template <typename T, typename TO, int EPI>
 hipError_t launch_wide_epi(const LinArgs& p, int64_t total_rows, int batch, int tile, hipStream_t s) {
   if (tile >= TILE_256) {
     if constexpr (sizeof(T) == 2) {
-      const bool four = tile == TILE_256 ? linear_four_wavefronts(p, EPI, sizeof(TO) == 2) : tile == TILE_256_FOUR;
+      const bool four = stream_deep_takes(p) && (tile == TILE_256 ? linear_four_wavefronts(p, EPI, sizeof(TO) == 2) : tile == TILE_256_FOUR);
       return (four ? linear_deep_launch : linear_eight_launch)(p, EPI, sizeof(TO) == 2, total_rows, batch, s);
     } else {
       const auto job = linear_job<T, TO, EPI>(p, batch);

@@ -1226,8 +1226,8 @@ def qk_rotate_store(proj, offsets, positions, scale, slot_mapping, cache, heads,
     """fp32 projections [T, *] with q | k | v at ``offsets`` -> fp32 queries [T, heads * dim] times ``scale``; keys and
     values go to cache rows [G * dim | G * vdim] of ``slot_mapping``.  ``q_norm`` [heads * dim] / ``k_norm``
     [kv_heads * dim]: one RMS norm over all of a token's query numbers (and all of its key numbers) with a weight per
-    number; ``unit_heads``: every query and key head by its own root mean square, without weights.  ``rot_dims``: the first rot_dims numbers of every head turn by position * inv_freq[i], i with
-    i + rot_dims / 2 (``interleaved``: 2i with 2i + 1).  ``v_first`` fp32 [T, G * vdim] (a column slice is fine): the stored values are
+    number; ``unit_heads``: every query and key head by its own root mean square, without weights.  ``rot_dims``: the first rot_dims
+    numbers of every head turn by position * inv_freq[i], i with i + rot_dims / 2 (``interleaved``: 2i with 2i + 1).  ``v_first`` fp32 [T, G * vdim] (a column slice is fine): the stored values are
     (1 - vmix) v + vmix v_first."""
     require_gpu(proj, "qk_rotate_store")
     T = proj.size(0)

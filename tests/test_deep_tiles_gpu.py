@@ -53,6 +53,17 @@ def test_weights_of_4_gib(gated, monkeypatch):
         close(got[:, c], want, 4 * K, torch.bfloat16)
 
 
+@pytest.mark.parametrize("tile", ["2", "4"])
+def test_weight_rows_far_apart(tile, monkeypatch):
+    """Rows of W 16 MiB apart: 256 of them span 4 GiB, which the tiles of eight wavefronts take."""
+    from byox_vllm_amd import kernels
+    monkeypatch.setenv("NV_LINEAR_TILE", tile)
+    torch.manual_seed(6)
+    x, w = torch.randn(300, 320, device=DEV).bfloat16(), torch.empty(300, 2 ** 23, device=DEV, dtype=torch.bfloat16)[:, :320]
+    w.normal_(0.0, 0.1)
+    close(kernels.linear(x, w), x.double() @ w.double().t(), 320, torch.bfloat16)
+
+
 @pytest.mark.parametrize("tops", [[0, 0, 1000], [300, 1, 0, 129, 128, 257], [513] * 3])
 def test_gathered_groups(tops, monkeypatch):
     """Groups that end anywhere in a tile, empty ones, rows from anywhere, gated."""

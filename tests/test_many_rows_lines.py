@@ -13,7 +13,8 @@ TILED, INT4 = _C.W_DENSE_TILED, _C.W_INT4
 @pytest.mark.parametrize("M,N,K,fmt,silu,own", [
     (4096, 24576, 3968, TILED, True, True), (8192, 16384, 7296, TILED, True, True), (8192, 16384, 7424, TILED, True, False),
     (5402, 4096, 7040, TILED, True, False), (5402, 4096, 3968, TILED, True, True), (16384, 6144, 1920, INT4, True, True),
-    (8192, 37888, 3584, INT4, True, True), (8192, 37888, 7296, INT4, True, True), (8192, 37888, 7424, INT4, True, False), (7872, 3072, 6144, INT4, True, False), (4096, 3584, 4608, INT4, True, False),
+    (8192, 37888, 3584, INT4, True, True), (8192, 37888, 7296, INT4, True, True), (8192, 37888, 7424, INT4, True, False),
+    (7872, 3072, 6144, INT4, True, False), (4096, 3584, 4608, INT4, True, False),
     (16384, 1024, 384, TILED, False, False), (16384, 2048, 3584, TILED, False, True), (16384, 2048, 3712, TILED, False, False),
     (14600, 1024, 3072, TILED, False, False), (16384, 1024, 1024, TILED, False, False), (16384, 896, 896, INT4, False, True),
     (16384, 2048, 1024, INT4, False, False)])
