@@ -104,7 +104,7 @@ def _has_all(sources) -> bool:
 
 def _with_needed(names):
     """``names`` and what their sources call in others."""
-    needs = {"linear": ("linear_deep", "linear_eight")}
+    needs = {"linear": ("linear_deep", "linear_eight", "linear_split")}
     return list(dict.fromkeys(m for n in names for m in (n,) + needs.get(n, ())))
 
 

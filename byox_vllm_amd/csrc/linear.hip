@@ -3,8 +3,8 @@
 // (nv_gemm) does not take: K or N that are no multiples of its tiles, fp32 models, batched products with one weight
 // per head, grouped products with one weight per expert over gathered rows, and the gated epilogues.
 //
-// linear_stream.h and linear_wide.h serve more than 64 rows whose K splits into 128-byte blocks, linear_short.h many rows by a K below
-// that, linear_few.h up to 64 rows; linear_tile_kernel below the other aligned bf16 products of many rows, linear_kernel the rest.
+// linear_stream.h, linear_wide.h and, in fp32, linear_split.hip serve more than 64 rows whose K splits into 128-byte blocks, linear_short.h
+// many rows by a K below that, linear_few.h up to 64 rows; linear_tile_kernel below the other aligned bf16 products of many rows, linear_kernel the rest.
 //
 // linear_kernel: a workgroup owns a 64 x 64 tile of the output: wavefront w the 16 columns n0 + 16 w .. and all four 16-row
 // sub-tiles.  Operands go from memory straight into MFMA fragments (both are K-contiguous rows, which is the fragment
@@ -382,29 +382,26 @@ extern "C" int nv_linear_rows(const void* a, int64_t a_row_stride, const int32_t
     NV_CHECK_LAUNCH();
     return NV_OK;
   }
-  // more than 64 rows that split into K blocks of 128 bytes: the wide tiles.  In fp32 a wide tile costs whatever of it is used, and its
+  // more than 64 rows that split into K blocks of 128 bytes: the wide tiles.  In fp32 a tile costs whatever of it is used, and its
   // wavefronts form twice as many results each as those of linear_kernel, so two kinds of product stay there: at most 32 columns
-  // whose short K brings more tiles than the chip holds (32 heads of 32 columns, 4000 rows, K = 128: 33.8 us there, 50 in wide tiles;
-  // 1000 rows, 512 tiles: 15.7 and 14.9), and element-wise functions of a product of two K blocks that leaves CUs idle (130 rows by
-  // 1500 columns, K = 64, soft cap: 11.4 and 13.9; K = 128: 15.3 and 16.2; 4000 rows by 512: 14.4 and 13.0).
+  // whose short K brings more tiles than the chip holds (32 heads of 32 columns, 4000 rows, K = 128: 32.2 us there, 42.3 in tiles;
+  // 1000 rows, 512 tiles: 14.8 and 10.3), and element-wise functions of a product of two K blocks that leaves CUs idle (130 rows by
+  // 1500 columns, K = 64: 11.4 and 12.7; soft cap 10.8 in both; 4000 rows by 512: 13.7 and 13.7).
   const int64_t tiles64 = wide_tiles(64, 128, M, total_rows, epilogue == EPI_GLU ? 2 * N : N, batch, group_offsets != nullptr);
   const bool stays = dtype == NV_F32 && !group_offsets && epilogue != EPI_GLU &&
                      (N <= 32 ? K <= 128 && tiles64 > 512
                               : (epilogue == EPI_SOFTCAP || epilogue == EPI_ACT) && K <= 64 && tiles64 < 96);
   if (M > 64 && p.vec_a && p.vec_w && (K * esz) % 128 == 0 && !stays && getenv("NV_LINEAR_TILE_OFF") == nullptr) {
     const int cols = epilogue == EPI_GLU ? 2 * N : N;
-    const bool has_256 = stream_takes(p, (int)esz, total_rows, batch, cols);
-    int tile = pick_wide_tile(M, total_rows, cols, K, batch, group_offsets != nullptr, dtype == NV_F32, has_256);
-    if (const char* force = getenv("NV_LINEAR_TILE")) tile = atoi(force) >= TILE_256 && !has_256 ? TILE_128 : atoi(force);
+    const bool has_256 = dtype == NV_BF16 && stream_takes(p, (int)esz, total_rows, batch, cols);
+    int tile = dtype == NV_F32 ? pick_split_tile(M, total_rows, cols, K, batch, group_offsets != nullptr)
+                               : pick_wide_tile(M, total_rows, cols, batch, group_offsets != nullptr, has_256);
+    if (const char* force = getenv("NV_LINEAR_TILE")) tile = dtype == NV_BF16 && atoi(force) >= TILE_256 && !has_256 ? TILE_128 : atoi(force);
     if (wide_tiles(64, 128, M, total_rows + 64 * batch, cols, batch, group_offsets != nullptr) < (1 << 30)) {
       hipError_t e;
-      if (dtype == NV_BF16) {
-        e = out_dtype == NV_BF16 ? launch_wide<bf16_t, bf16_t>(p, epilogue, total_rows, batch, tile, s)
-                                 : launch_wide<bf16_t, float>(p, epilogue, total_rows, batch, tile, s);
-      } else {
-        e = out_dtype == NV_BF16 ? launch_wide<float, bf16_t>(p, epilogue, total_rows, batch, tile, s)
-                                 : launch_wide<float, float>(p, epilogue, total_rows, batch, tile, s);
-      }
+      if (dtype == NV_F32) e = linear_split_launch(p, epilogue, out_dtype == NV_BF16, total_rows, batch, tile, s);
+      else if (out_dtype == NV_BF16) e = launch_wide<bf16_t>(p, epilogue, total_rows, batch, tile, s);
+      else e = launch_wide<float>(p, epilogue, total_rows, batch, tile, s);
       if (e != hipSuccess) {
         nv_set_error("nv_linear: %s", hipGetErrorString(e));
         return NV_ERR_LAUNCH;

@@ -42,3 +42,6 @@ __device__ __forceinline__ float unary_act(float v, int act, const float* prm, f
 hipError_t linear_deep_launch(const LinArgs& p, int epilogue, bool out_16bit, int64_t total_rows, int batch, hipStream_t s);
 // the same on those of stream_tiles.h (linear_eight.hip)
 hipError_t linear_eight_launch(const LinArgs& p, int epilogue, bool out_16bit, int64_t total_rows, int batch, hipStream_t s);
+// fp32 products as sums of 16-bit ones (linear_split.hip), in tiles of 64, 128 or 256 rows by 128 columns
+enum { SPLIT_64 = 0, SPLIT_128 = 1, SPLIT_256 = 2 };
+hipError_t linear_split_launch(const LinArgs& p, int epilogue, bool out_16bit, int64_t total_rows, int batch, int tile, hipStream_t s);

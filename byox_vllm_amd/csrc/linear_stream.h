@@ -1,5 +1,5 @@
-// nv_linear for many rows: the products, groups and epilogues of LinArgs on the tiles of stream_tiles.h (fp32, and 16 bits in linear_eight.hip)
-// and stream_deep.h (16 bits, linear_deep.hip).  Groups (experts) of unknown size: every workgroup counts the tiles from the offsets with one
+// nv_linear for many rows: the products, groups and epilogues of LinArgs in 16 bits on the tiles of stream_tiles.h (linear_eight.hip)
+// and stream_deep.h (linear_deep.hip).  Groups (experts) of unknown size: every workgroup counts the tiles from the offsets with one
 // wavefront-wide prefix sum; a group that ends in the upper half of a tile's rows costs the half.
 #pragma once
 #include <type_traits>

@@ -1,10 +1,10 @@
 // Products of many rows: a workgroup per CU walks tiles of 256 x 256 outputs whose K blocks form one stream.
 //
-// Here: eight wavefronts of 128 x 64 each, for fp32 and for 16-bit products whose results take long to form (linear_four_wavefronts); the other
-// 16-bit products: stream_deep.h, whose tiles, their order and W's rows in LDS are those of this file.
+// Here: eight wavefronts of 128 x 64 each, for 16-bit products whose results take long to form (linear_four_wavefronts); the others:
+// stream_deep.h, whose tiles, their order and W's rows in LDS are those of this file.
 //
-// What bounds it: the matrix cores (v_mfma_f32_16x16x4_f32; in 16 bits 852 us at 8192 x 8192 x 8192, stream_deep.h 705), two wavefronts to a
-// SIMD, of which one forms results while the other has products.
+// What bounds it: the matrix cores (852 us at 8192 x 8192 x 8192, stream_deep.h 705), two wavefronts to a SIMD, of which one forms results
+// while the other has products.
 //   * 16-row products: a lane's results lie where whole 64-byte pieces of rows can be stored;
 //   * the barrier stands before the block's last step of K, whose fragments are in registers: behind it the first fragments of the
 //     next block are read under that step's products, and the buffer just left is refilled, one DMA instruction behind every few
@@ -13,7 +13,6 @@
 //     behind two thirds of the products and waits for them at once;
 //   * workgroups stay: the first two blocks of the next tile are on their way while the results of a tile are stored, and nothing
 //     waits for those stores but the second block after them.  Their tiles are found once, by a thread each, and kept in LDS.
-// Measured (us, this form and the 128 x 128 tiles): 2500 rows 1024 -> 6144 256 and 266, 8000 rows 512 -> 2048 137 and 149.
 // LDS rows are 128 bytes, their 16-byte pieces dealt by XOR (through the DMA's source addresses) so that the 16 rows a read touches lie
 // in 16 bank groups.  Tiles go to the XCDs in contiguous eighths, within them in bands of eight row
 // tiles, so the 32 workgroups of an XCD share 8 row and 4 column panels in its L2.  A group's short last row tile stays in its band
@@ -43,12 +42,6 @@ constexpr int STREAM_BUFFER = (STREAM_BM + STREAM_BN) * 128;      // a K block o
 
 __device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x4 c, bf16_t) {
   return mfma16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c);
-}
-__device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x4 c, float) {
-  // product e takes number 4 g + e of the sixteen that the four groups of lanes hold
-#pragma unroll
-  for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[e]), __uint_as_float(b[e]), c, 0, 0, 0);
-  return c;
 }
 
 // Where W lies in LDS and which of its rows a fragment has.  W stays in the order it has in memory, so that neighbouring lanes of a
