@@ -98,14 +98,23 @@ __device__ __forceinline__ void prompt_rows_again(const WAttnArgs& a, uint32_t r
   }
 }
 
+// 16 bytes to a lane into LDS at `dst` + 16 * lane.  Not the builtin: the compiler waits for every DMA under way ahead of a transposing
+// read, for the next tile's too; what has to be waited for is said at the tile's beginning.
+__device__ __forceinline__ void pa_dma(const void* src, uint32_t dst) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src) : "memory");
+}
+__device__ __forceinline__ void pa_dma(const void* base, uint32_t off, uint32_t dst) {      // one base for the wavefront
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory");
+}
+
 template <int D, bool EXT>
 __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int tiles, int num_seqs, int bs_shift) {
   constexpr int KS = D / 16, DT = D / 32, ROWB = 2 * D, TILE = PA_KEYS * ROWB;      // bytes of one operand's tile
   constexpr int RPI = 1024 / ROWB, NI = PA_KEYS / RPI / 4;                          // rows per DMA instruction; instructions per wavefront
   constexpr float L2E = 1.4426950408889634f;
   __shared__ __attribute__((aligned(1024))) unsigned char lds[2][2 * TILE];
-  typedef __attribute__((address_space(1))) const void global_void;
-  typedef __attribute__((address_space(3))) void lds_void;
+  typedef __attribute__((address_space(3))) unsigned char lds_byte;
+  const uint32_t lds_at = (uint32_t)(uintptr_t)(lds_byte*)&lds[0][0];
   typedef short v4s __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) v4s lds_v4s;
   // tiles that share keys run on one XCD; late tiles of a request, which see the most keys, first
@@ -121,11 +130,11 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
   const int lr = lane & 31, lh = lane >> 5;
   // the tile's tokens: of one request where their number is known, else of as many as have tokens there
   int64_t t_begin = (int64_t)tile * p.TQ, t_end = min(p.tokens, t_begin + p.TQ);
-  int owner = -1;
+  int owner = -1, owner_pos = 0;       // the request and the position of the tile's first token
   if (num_seqs > 1) {
     for (int base = 0, before = 0; base < num_seqs && owner < 0; base += 64) {
       const int i = min(base + lane, num_seqs - 1);
-      const int first = (int)min((int64_t)p.cu_q[i], p.tokens), end = (int)min((int64_t)p.cu_q[i + 1], p.tokens);
+      const int first = (int)min((int64_t)p.cu_q[i], p.tokens), end = (int)min((int64_t)p.cu_q[i + 1], p.tokens), ahead = p.past[i];
       const int mine = base + lane < num_seqs ? (end - first + p.TQ - 1) / p.TQ : 0;
       int upto = mine;
 #pragma unroll
@@ -140,6 +149,7 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
         owner = base + l;
         t_begin = __builtin_amdgcn_readlane(first, l) + (int64_t)local * p.TQ;
         t_end = min((int64_t)__builtin_amdgcn_readlane(end, l), t_begin + p.TQ);
+        owner_pos = __builtin_amdgcn_readlane(ahead, l) + local * p.TQ;
       }
       before += __builtin_amdgcn_readlane(upto, 63);
     }
@@ -148,6 +158,7 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
   const char* k_base = reinterpret_cast<const char*>(p.cache) + (int64_t)g * ROWB;
   const char* v_base = reinterpret_cast<const char*>(p.cache) + ((int64_t)p.v_col + (int64_t)g * D) * 2;
   const int64_t row_bytes = (int64_t)p.cw * 2;
+  const bool whole_tiles = p.block_size % PA_KEYS == 0 && p.cw < (1 << 24);
   const bf16_t* sink = reinterpret_cast<const bf16_t*>(p.sink);
   auto k_swz = [](int r) { return D == 128 ? r & 15 : (r >> 1) & 7; };
   auto v_swz = [](int r) { return D == 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); };
@@ -155,10 +166,11 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
   // this lane's part of the DMA: row RPI * (wv * NI + i) + lane / (64 / RPI) of the tile, piece lane % (64 / RPI)
   constexpr int PIECES = 64 / RPI;                 // 16-byte pieces of a row
   const int dma_r = lane / PIECES, dma_p = lane % PIECES;
-  int k_off[NI], v_off[NI];
+  uint32_t row_off[NI], k_off[NI], v_off[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int r = RPI * (wv * NI + i) + dma_r;
+    row_off[i] = (uint32_t)r * (uint32_t)row_bytes;
     k_off[i] = (dma_p ^ k_swz(r)) << 4;
     v_off[i] = (dma_p ^ v_swz(r)) << 4;
   }
@@ -170,14 +182,75 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
 
   for (int64_t ts = t_begin; ts < t_end;) {
     const int b = owner >= 0 ? owner : p.seq_of[ts];
-    const int64_t te = min(t_end, (int64_t)p.cu_q[b + 1]);
+    const int64_t te = owner >= 0 ? t_end : min(t_end, (int64_t)p.cu_q[b + 1]);
     const int nq = (int)(te - ts), rows = nq * R;
-    const int p0 = p.past[b] + (int)(ts - p.cu_q[b]);
+    const int p0 = owner >= 0 ? owner_pos : p.past[b] + (int)(ts - p.cu_q[b]);
     const int32_t* table = p.tables + (int64_t)b * p.table_cols;
     const int row0 = 32 * wv, rr = row0 + lr;
     const bool valid = rr < rows, wave_on = row0 < rows;
     const int tok = valid ? rr / R : 0, head = g * R + (valid ? rr % R : 0);
     const int pos = p0 + tok;
+    f32x16 o[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[dt][r] = 0.0f;
+    float m_run = -INFINITY, l_run = 0.0f;
+    const int wpos_lo = p0 + row0 / R, wpos_hi = p0 + min(rows - 1, row0 + 31) / R;
+
+    // The walk is over tiles of 64 keys from multiples of 64 on: those with kept keys (of which the first sees them all), then those from
+    // the first key of the tile's first row to the last key of its last.
+    auto first_of = [&](int at) { return max(p.window > 0 ? at - p.window + 1 : 0, EXT && p.chunk > 0 ? at / p.chunk * p.chunk : 0); };
+    const int low = first_of(pos), hi = p0 + nq - 1, wlow_lo = first_of(wpos_lo), wlow_hi = first_of(wpos_hi);
+    const int kept_tiles = EXT ? (min(p.keep, first_of(p0)) + PA_KEYS - 1) / PA_KEYS : 0;
+    const int skipped = max(first_of(p0) / PA_KEYS - kept_tiles, 0), count = hi / PA_KEYS + 1 - skipped;
+    auto tile_key = [&](int it) { return PA_KEYS * (it < kept_tiles ? it : it + skipped); };
+    // Where its rows are.  Blocks of a multiple of 64 hold whole tiles: one page number for all lanes, asked for a tile ahead (as a vector
+    // load: what waits for a scalar one waits for all reads of LDS too), and every lane's place in a tile is the same each time.  Else every
+    // lane looks its rows up.  Places past the last key repeat it: they are masked, and what nobody has written there may be a NaN.
+    int page[NI], in_page[NI], no_lane;
+    asm volatile("v_mov_b32 %0, 0" : "=v"(no_lane));
+    auto look_up = [&](int it) {
+      const int j0 = tile_key(min(it, count - 1));
+      if (whole_tiles) {
+        page[0] = table[(bs_shift >= 0 ? j0 >> bs_shift : j0 / p.block_size) + no_lane];
+        return;
+      }
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int kp = min(j0 + RPI * (wv * NI + i) + dma_r, hi);
+        const int n = bs_shift >= 0 ? kp >> bs_shift : kp / p.block_size;
+        in_page[i] = kp - n * p.block_size;
+        page[i] = table[n];
+      }
+    };
+    auto fill = [&](int buf, int it) {
+      const uint32_t dst = lds_at + buf * 2 * TILE + wv * NI * 1024;
+      if (whole_tiles) {
+        const int j0 = tile_key(it), n = bs_shift >= 0 ? j0 >> bs_shift : j0 / p.block_size;
+        const int64_t at = ((int64_t)__builtin_amdgcn_readfirstlane(page[0]) * p.block_size + (j0 - n * p.block_size)) * row_bytes;
+        const bool ends = hi - j0 < PA_KEYS - 1;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          const uint32_t row = ends ? (uint32_t)min(RPI * (wv * NI + i) + dma_r, hi - j0) * (uint32_t)row_bytes : row_off[i];
+          pa_dma(k_base + at, row + k_off[i], dst + i * 1024);
+          pa_dma(v_base + at, row + v_off[i], dst + i * 1024 + TILE);
+        }
+        return;
+      }
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int64_t at = ((int64_t)page[i] * p.block_size + in_page[i]) * row_bytes;
+        pa_dma(k_base + at + k_off[i], dst + i * 1024);
+        pa_dma(v_base + at + v_off[i], dst + i * 1024 + TILE);
+      }
+    };
+    __builtin_amdgcn_s_barrier();            // an earlier request's walk through this tile has read its last buffer
+    look_up(0);
+    const float* gates = p.gate ? p.gate + (ts + tok) * p.gate_rs : nullptr;
+    const float head_gate = EXT && p.gate_head && gates ? gates[head] : 0.0f;      // waited for at the end
+    fill(0, 0);
+    look_up(1);
     // queries: lane holds numbers 16 ks + 8 lh .. + 7 of its row
     bf16x8 qf[KS];
     {
@@ -192,96 +265,63 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
         }
       }
     }
-    f32x16 o[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) o[dt][r] = 0.0f;
-    float m_run = -INFINITY, l_run = 0.0f;
-    // first key of the row's window or chunk
-    const int low = max(p.window > 0 ? pos - p.window + 1 : 0, EXT && p.chunk > 0 ? pos / p.chunk * p.chunk : 0);
-    const int wpos_lo = p0 + row0 / R, wpos_hi = p0 + min(rows - 1, row0 + 31) / R;
-
-    const int lo_w = p.window > 0 ? max(0, p0 - p.window + 1) : 0;
-    const int lo = EXT && p.chunk > 0 ? max(lo_w, p0 / p.chunk * p.chunk) : lo_w, hi = p0 + nq - 1;
-    // kept keys: the walk is over c = c_first .. hi; c < lo means key c - c_first (those ahead of the window), else key c
-    const int c_first = EXT ? lo - min(p.keep, lo) : lo;
-    auto key_of = [&](int c) { return EXT && c < lo ? c - c_first : c; };
-    // pages of this lane's part of a tile (places past the last key repeat it: they are masked).  They are asked for a tile
-    // ahead and turned into addresses only when the tile is fetched, so nothing waits for them.
-    int page[NI], in_page[NI];
-    auto look_up = [&](int j0) {
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int kp = key_of(min(j0 + RPI * (wv * NI + i) + dma_r, hi));
-        const int n = bs_shift >= 0 ? kp >> bs_shift : kp / p.block_size;
-        in_page[i] = kp - n * p.block_size;
-        page[i] = table[n];
-      }
-    };
-    auto fill = [&](int buf) {
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int64_t at = ((int64_t)page[i] * p.block_size + in_page[i]) * row_bytes;
-        unsigned char* dst = lds[buf] + (wv * NI + i) * 1024;
-        __builtin_amdgcn_global_load_lds((global_void*)(k_base + at + k_off[i]), (lds_void*)dst, 16, 0, 0);
-        __builtin_amdgcn_global_load_lds((global_void*)(v_base + at + v_off[i]), (lds_void*)(dst + TILE), 16, 0, 0);
-      }
-    };
-    __builtin_amdgcn_s_barrier();            // an earlier request's walk through this tile has read its last buffer
-    look_up(c_first);
-    fill(0);
-    look_up(c_first + PA_KEYS);              // page numbers a tile ahead of their use
     int buf = 0;
-    for (int j0 = c_first; j0 <= hi; j0 += PA_KEYS, buf ^= 1) {
+    for (int it = 0; it < count; ++it, buf ^= 1) {
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      if (j0 + PA_KEYS <= hi) {
-        fill(buf ^ 1);
-        look_up(j0 + 2 * PA_KEYS);
+      if (it + 1 < count) {
+        fill(buf ^ 1, it + 1);
+        look_up(it + 2);
       }
-      // keys that this wavefront's rows can see at all, and whether all its rows see all of the tile
-      bool need = wave_on && j0 <= wpos_hi && (p.window <= 0 || j0 + PA_KEYS - 1 > wpos_lo - p.window);
-      bool all = j0 + PA_KEYS - 1 <= wpos_lo && (p.window <= 0 || wpos_hi - j0 < p.window);
-      if constexpr (EXT) {
-        need = wave_on && key_of(j0) <= wpos_hi && (need || key_of(j0) < p.keep) &&
-               (p.chunk <= 0 || j0 + PA_KEYS - 1 >= wpos_lo / p.chunk * p.chunk);
-        all = all && j0 >= lo && (p.chunk <= 0 || j0 >= wpos_hi / p.chunk * p.chunk);
-      }
-      if (!need) continue;
+      // keys that this wavefront's rows can see at all, and whether some row sees none of the first or none of the last of them
+      const int j0 = tile_key(it), j1 = j0 + PA_KEYS - 1;
+      if (!wave_on || j0 > wpos_hi || (j1 < wlow_lo && (!EXT || j0 >= p.keep))) continue;
+      const bool cut_low = wlow_hi > j0 && (!EXT || j1 >= p.keep), cut_high = j1 > wpos_lo;
       const unsigned char* kt = lds[buf];
       f32x16 s[2];
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
+      for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) s[t][r] = 0.0f;
+      // every product has its fragment read AHEAD products before it, in the order written here: left alone, the compiler reads each
+      // right before its product and waits for it
+      constexpr int AHEAD = 4, QK = 2 * KS, PV = 4 * DT;
+      bf16x8 kf[QK], vf[PV];
+      auto k_read = [&](int f) { kf[f] = *reinterpret_cast<const bf16x8*>(kt + (32 * (f & 1) + lr) * ROWB + (((f & ~1) + lh) ^ ksw) * 16); };
+      auto v_read = [&](int f) {
+        const unsigned char* a = kt + TILE + 16 * (f / DT) * ROWB + v_at(f % DT);
+        const u32x2 x = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)a));
+        const u32x2 y = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(a + 8 * ROWB)));
+        vf[f] = __builtin_bit_cast(bf16x8, u32x4{x[0], x[1], y[0], y[1]});
+      };
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          const bf16x8 kf = *reinterpret_cast<const bf16x8*>(kt + (32 * t + lr) * ROWB + (((2 * ks + lh) ^ ksw) << 4));
-          s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], s[t], 0, 0, 0);
-        }
-      }
-      // four fragments ahead of the products that use them
-      __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+      for (int f = 0; f < AHEAD; ++f) k_read(f);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < 2 * KS; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (i < 2 * KS - 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      for (int f = 0; f < QK; ++f) {
+        s[f & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[f], qf[f >> 1], s[f & 1], 0, 0, 0);
+        if (f + AHEAD < QK) k_read(f + AHEAD);
+        else v_read(f + AHEAD - QK);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      if (!all) {
-        // place k of the lane's keys shows key c = j0 + 4 lh + k of the walk: kept keys (c < lo), then those from the row's
-        // first to its own position, or below `keep`
-        const int c0 = j0 + 4 * lh, last = pos - c0, first = low - c0, kept = (EXT ? lo : 0) - c0, low_kept = p.keep - c0;
+      // place k of the lane's keys is key c0 + k
+      const int c0 = j0 + 4 * lh, last = pos - c0, first = low - c0, kept = p.keep - c0;
+      if (cut_low) {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const int k = 32 * t + 8 * (r >> 2) + (r & 3);
-            bool vis = k <= last && k >= first;
-            if constexpr (EXT) vis = vis || k < kept || (k < low_kept && k <= last);
-            s[t][r] = vis ? s[t][r] : -INFINITY;
+            bool vis = k >= first;
+            if constexpr (EXT) vis = vis || k < kept;
+            s[t][r] = vis && k <= last ? s[t][r] : -INFINITY;
           }
+      } else if (cut_high) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s[t][r] = 32 * t + 8 * (r >> 2) + (r & 3) <= last ? s[t][r] : -INFINITY;
       }
       float mx[4];
 #pragma unroll
@@ -303,35 +343,30 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
         l_run *= corr;
         m_run = m_new;
       }
+      // weights of sixteen keys at a time, under the products of the sixteen before
       float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
       bf16x8 pf[4];
+      auto weights = [&](int ss, int from, int to) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
+        for (int i = 0; i < 8; ++i) {
+          if (i < from || i >= to) continue;
+          const int t = ss >> 1, r = 8 * (ss & 1) + i;
           const float e = __builtin_amdgcn_exp2f(fmaf(s[t][r], L2E, -m_use));
           sum[r & 3] += e;
-          pf[2 * t + (r >> 3)][r & 7] = (bf16_t)e;
+          pf[ss][i] = (bf16_t)e;
         }
-      l_run += (sum[0] + sum[1]) + (sum[2] + sum[3]);
-      const unsigned char* vt = kt + TILE;
+      };
+      weights(0, 0, 8);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int ss = 0; ss < 4; ++ss)
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          const unsigned char* a = vt + 16 * ss * ROWB + v_at(dt);
-          const v4s x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)a);
-          const v4s y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(a + 8 * ROWB));
-          const u32x2 x2 = __builtin_bit_cast(u32x2, x), y2 = __builtin_bit_cast(u32x2, y);
-          const bf16x8 vf = __builtin_bit_cast(bf16x8, u32x4{x2[0], x2[1], y2[0], y2[1]});
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[ss], o[dt], 0, 0, 0);
-        }
-      __builtin_amdgcn_sched_group_barrier(0x100, 6, 1);
-#pragma unroll
-      for (int i = 0; i < 4 * DT; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
-        if (i < 4 * DT - 3) __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
+      for (int f = 0; f < PV; ++f) {
+        const int ss = f / DT, dt = f % DT;
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[f], pf[ss], o[dt], 0, 0, 0);
+        if (f + AHEAD < PV) v_read(f + AHEAD);
+        if (ss < 3) weights(ss + 1, 8 / DT * dt, 8 / DT * (dt + 1));
+        __builtin_amdgcn_sched_barrier(0);
       }
+      l_run += (sum[0] + sum[1]) + (sum[2] + sum[3]);
     }
     if (wave_on) {
       float none[4] = {0.0f, 0.0f, 0.0f, 0.0f};       // 0 times every number: NaN where one is not finite
@@ -347,9 +382,9 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
         float fs, den;
         close_softmax(m_run, l_lo + l_hi, sink != nullptr, sink ? ld_f32<bf16_t>(sink + head) : 0.0f, fs, den);
         float f = p.out_scale * fs / den;
-        const float* grow = p.gate ? p.gate + (ts + tok) * p.gate_rs : nullptr;
+        const float* grow = gates;
         if (EXT && p.gate_head) {
-          if (grow) f *= sigmoid_f32(grow[head]);
+          if (grow) f *= sigmoid_f32(head_gate);
           grow = nullptr;
         }
         bf16_t* orow = reinterpret_cast<bf16_t*>(p.out) + (ts + tok) * p.out_rs + (int64_t)head * D + 4 * lh;
