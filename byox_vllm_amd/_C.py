@@ -110,6 +110,7 @@ _PROTOS = {
     "nv_latent_attn_split": (_i, [_p, _p, _p, _i, _p, _p, _p, _p, _i64, _i, _i, _i, _i, _i, _i, _f, _i, _p, _sz, _i, _p]),
     "nv_latent_attn_workspace_bytes": (_sz, [_i64, _i, _i, _i]),
     "nv_latent_q_rows": (_i, [_p, _i64, _p, _p, _f, _p, _i64, _i, _i, _i, _i, _i, _i, _i, _f, _i, _p]),
+    "nv_latent_q_rows_as": (_i, [_p, _i64, _p, _p, _f, _p, _i, _i64, _i, _i, _i, _i, _i, _i, _i, _f, _i, _p]),
     "nv_latent_gather": (_i, [_p, _p, _i, _p, _p, _p, _i, _i, _i, _p, _i64, _i, _p]),
     "nv_latent_expand": (_i, [_p, _p, _p, _i64, _i, _i, _i, _i, _i, _i, _p]),
     "nv_moe_route": (_i, [_p, _i64, _p, _p, _i64, _i, _i, _i, _p]),
@@ -127,9 +128,13 @@ _PROTOS = {
                                    _i, _p, _p, _i64, _i, _p, _sz, _i, _p]),
     "nv_paged_softmax_attn_batch": (_i, [_p, _p, _p, _i, _p, _p, _p, _p, _i64, _i64, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _f,
                                          _f, _i, _i, _p, _p, _i64, _i, _p, _sz, _i, _p]),
+    "nv_paged_softmax_attn_q": (_i, [_p, _i, _p, _p, _i, _p, _p, _p, _p, _i64, _i64, _i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _f,
+                                         _f, _i, _i, _p, _p, _i64, _i, _p, _sz, _i, _p]),
+    "nv_paged_softmax_attn_takes_q16": (_i, [_p, _i64, _i64, _i, _i, _i, _i, _i, _i, _f, _i, _i]),
     "nv_qk_rotate_store": (_i, [_p, _p, _i64, _i, _i, _i, _p, _p, _i, _p, _p, _f, _i, _p, _i, _i, _f, _p, _i64, _p, _f, _f, _p,
                                 _p, _p, _i64, _i, _i, _i, _i, _i, _p]),
     "nv_qkv_stream": (_i, [_p, _i64, _p, _i64, _i, _i, _p, _p, _i, _f, _f, _p, _p, _p, _p, _i64, _p, _i, _i, _i, _i, _p]),
+    "nv_qkv_stream_as": (_i, [_p, _i64, _p, _i64, _i, _i, _p, _p, _i, _f, _f, _p, _p, _p, _i, _p, _i64, _p, _i, _i, _i, _i, _p]),
     "nv_qk_conv_store_ok": (_i, [_p, _i64, _i, _i, _i, _p, _p, _p, _i, _i, _i]),
     "nv_qk_conv_store": (_i, [_p, _i64, _i, _i, _i, _p, _i, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i, _i, _i, _i, _i, _i, _f, _f,
                               _i, _p]),

@@ -130,11 +130,11 @@ constexpr int TURNS = 256;
 // they were most of the kernel), the numbers in front in fours where rows split into them (`quads`).  53 us for 11013 tokens of 16
 // heads of 96 + 32 then, 38 now (135 MB).  With one number per thread the table and its barrier only cost: 16384 tokens of 4 such
 // heads 21.2 us with it, 18.7 without.
-template <typename T>
+template <typename T, typename TO>
 __global__ __launch_bounds__(256) void latent_q_rope_kernel(const T* __restrict__ q, int64_t q_rs,
                                                             const int64_t* __restrict__ positions,
                                                             const float* __restrict__ inv_freq, float mscale,
-                                                            float* __restrict__ qa, int H, int dim, int rot_dim,
+                                                            TO* __restrict__ qa, int H, int dim, int rot_dim,
                                                             int rot_dims, int rank, int interleaved, int copy_front,
                                                             float factor, int quads) {
   __shared__ float2 turn[TURNS];
@@ -155,12 +155,12 @@ __global__ __launch_bounds__(256) void latent_q_rope_kernel(const T* __restrict_
       f32x4 v = Pack4<T>::widen(*reinterpret_cast<const typename Pack4<T>::type*>(q + t * q_rs + (int64_t)h * (dim + rot_dim) + j));
 #pragma unroll
       for (int r = 0; r < 4; ++r) v[r] *= factor;
-      *reinterpret_cast<f32x4*>(qa + (t * H + h) * (rank + rot_dim) + j) = v;
+      *reinterpret_cast<typename Pack4<TO>::type*>(qa + (t * H + h) * (rank + rot_dim) + j) = Pack4<TO>::narrow(v);
     }
   } else if (copy_front) {
     for (int idx = threadIdx.x; idx < H * dim; idx += blockDim.x) {
       const int h = idx / dim, j = idx % dim;
-      qa[(t * H + h) * (rank + rot_dim) + j] = ld_f32<T>(q + t * q_rs + (int64_t)h * (dim + rot_dim) + j) * factor;
+      st_f32<TO>(qa + (t * H + h) * (rank + rot_dim) + j, ld_f32<T>(q + t * q_rs + (int64_t)h * (dim + rot_dim) + j) * factor);
     }
   }
   if (table) __syncthreads();
@@ -175,7 +175,7 @@ __global__ __launch_bounds__(256) void latent_q_rope_kernel(const T* __restrict_
       const float other = ld_f32<T>(src + (interleaved ? j ^ 1 : (first ? j + half : j - half)));
       v = first ? v * a.x - other * a.y : v * a.x + other * a.y;
     }
-    qa[(t * H + h) * (rank + rot_dim) + rank + j] = v * factor;
+    st_f32<TO>(qa + (t * H + h) * (rank + rot_dim) + rank + j, v * factor);
   }
 }
 
@@ -643,6 +643,14 @@ extern "C" int nv_latent_q_rope(const void* q, int64_t q_row_stride, const int64
 extern "C" int nv_latent_q_rows(const void* q, int64_t q_row_stride, const int64_t* positions, const float* inv_freq,
                                 float mscale, float* qa, int64_t tokens, int heads, int dim, int rot_dim, int rot_dims,
                                 int interleaved, int rank, int copy_front, float factor, int dtype, nv_stream_t stream) {
+  return nv_latent_q_rows_as(q, q_row_stride, positions, inv_freq, mscale, qa, NV_F32, tokens, heads, dim, rot_dim, rot_dims, interleaved,
+                             rank, copy_front, factor, dtype, stream);
+}
+
+extern "C" int nv_latent_q_rows_as(const void* q, int64_t q_row_stride, const int64_t* positions, const float* inv_freq,
+                                   float mscale, void* qa, int qa_dtype, int64_t tokens, int heads, int dim, int rot_dim, int rot_dims,
+                                   int interleaved, int rank, int copy_front, float factor, int dtype, nv_stream_t stream) {
+  NV_CHECK_ARG(qa_dtype == NV_F32 || qa_dtype == NV_BF16, "nv_latent_q_rope: bad dtype %d of the rows", qa_dtype);
   NV_CHECK_ARG(!copy_front || rank == dim, "nv_latent_q_rows: whole query rows have the unrotated numbers in front");
   NV_CHECK_ARG(q && positions && inv_freq && qa, "nv_latent_q_rope: null pointer");
   NV_CHECK_ARG(dtype == NV_BF16 || dtype == NV_F32, "nv_latent_q_rope: bad dtype %d", dtype);
@@ -651,9 +659,14 @@ extern "C" int nv_latent_q_rows(const void* q, int64_t q_row_stride, const int64
   if (tokens == 0 || (rot_dim == 0 && !copy_front)) return NV_OK;
   const int quads = dim % 4 == 0 && rot_dim % 4 == 0 && q_row_stride % 4 == 0 && (uintptr_t)qa % 16 == 0 &&
                     (uintptr_t)q % (dtype == NV_BF16 ? 8 : 16) == 0;
-  NV_DISPATCH_T(dtype, latent_q_rope_kernel<T><<<dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream>>>(
-                           (const T*)q, q_row_stride, positions, inv_freq, mscale, qa, heads, dim, rot_dim, rot_dims, rank,
-                           interleaved, copy_front, factor, quads));
+  if (qa_dtype == NV_F32)
+    NV_DISPATCH_T(dtype, latent_q_rope_kernel<T, float><<<dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream>>>(
+                             (const T*)q, q_row_stride, positions, inv_freq, mscale, (float*)qa, heads, dim, rot_dim, rot_dims, rank,
+                             interleaved, copy_front, factor, quads));
+  else
+    NV_DISPATCH_T(dtype, latent_q_rope_kernel<T, bf16_t><<<dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream>>>(
+                             (const T*)q, q_row_stride, positions, inv_freq, mscale, (bf16_t*)qa, heads, dim, rot_dim, rot_dims, rank,
+                             interleaved, copy_front, factor, quads));
   NV_CHECK_LAUNCH();
   return NV_OK;
 }

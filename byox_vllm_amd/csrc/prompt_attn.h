@@ -16,9 +16,17 @@
 // with one prefix sum over the requests.  A layer of 16 heads of 128 over 64 requests of 2048 cached tokens, one new token each, and
 // a prompt of 512: 8900 us in the older kernel, 4430 with tiles over several requests, 302 now; two heads per key head and a window
 // of 512: 1495, 1515, 109; prompts alone as before (8 x 2048 ragged: 589 and 577).
-// Scores, maxima, sums and outputs are fp32; q and P enter the products as bf16, as before.  Measured, 8 prompts of 2048
-// tokens, 16 heads of 128: window 512 beside 16 kept keys, two heads per key head, 554 -> 179 us; 16 key heads, ragged, every
-// earlier key, 549 -> 181 us.  What is left is the softmax: about 250 VALU instructions per 32 matrix instructions.
+// Scores, maxima, sums and outputs are fp32; q and P enter the products as bf16, so queries may come in bf16 as well (half the bytes of the
+// rows that a workgroup begins with).  Of what held the walk up besides its softmax:
+//   * the compiler put every fragment's read right before its product, and ahead of the first transposing read waited for the next tile's
+//     DMA: both are placed by hand, fragments four products ahead, weights of sixteen keys under the products of the sixteen before;
+//   * page numbers and addresses were a lane's own, 200 of a tile's 500 vector instructions: tiles begin at multiples of 64, so that blocks
+//     of a multiple of 64 hold whole tiles at a place that one scalar gives.  In one kernel with the lanes' own the registers did not suffice;
+//   * a tile's request and first position were looked up in turn, ahead of its queries.
+// Measured, 8 prompts of 2048 tokens, 16 heads of 128: window 512 beside 16 kept keys, two heads per key head, 554 us in the older kernel,
+// 179, now 145; 16 key heads, ragged, every earlier key, 549, 181, now 155.  Heads of 64 have three wavefronts to a SIMD; with two, kept keys
+// and a window of 700 took 3 % more of a layer.  What is left: the queries' and results' bytes, which nothing overlaps at a workgroup's
+// beginning and end (40 us), and 330 vector instructions per 32 products.
 #pragma once
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -40,7 +48,10 @@ __device__ __forceinline__ void prompt_rows_again(const WAttnArgs& a, uint32_t r
     const int row = row0 + __ffs(rest) - 1, row_tok = row / heads, row_head = g * heads + row % heads, row_pos = first_pos + row_tok;
     const int first = max(a.window > 0 ? row_pos - a.window + 1 : 0, EXT && a.chunk > 0 ? row_pos / a.chunk * a.chunk : 0);
     const int from = max(first, 0), kept = EXT ? min(a.keep, from) : 0, count = kept + row_pos + 1 - from;
-    const float* qrow = a.q + ((ts + row_tok) * a.H + row_head) * D;
+    const int64_t q_at = ((ts + row_tok) * a.H + row_head) * D;
+    auto query = [&](int e) {
+      return a.q16 ? (float)reinterpret_cast<const bf16_t*>(a.q)[q_at + e] : (float)(bf16_t)reinterpret_cast<const float*>(a.q)[q_at + e];
+    };
     auto row_at = [&](int c) {             // byte offset of the row's c-th visible key
       const int key = c < kept ? c : from + c - kept, n = bs_shift >= 0 ? key >> bs_shift : key / a.block_size;
       return ((int64_t)table[n] * a.block_size + (key - n * a.block_size)) * (2 * (int64_t)a.cw);
@@ -52,7 +63,7 @@ __device__ __forceinline__ void prompt_rows_again(const WAttnArgs& a, uint32_t r
       for (int e = 0; e < D; e += 8) {
         const bf16x8 x = *reinterpret_cast<const bf16x8*>(k + 2 * e);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) sum = fmaf((float)(bf16_t)qrow[e + j], (float)x[j], sum);
+        for (int j = 0; j < 8; ++j) sum = fmaf(query(e + j), (float)x[j], sum);
       }
       return sum;
     };
@@ -107,8 +118,9 @@ __device__ __forceinline__ void pa_dma(const void* base, uint32_t off, uint32_t 
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory");
 }
 
-template <int D, bool EXT>
-__global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int tiles, int num_seqs, int bs_shift) {
+// WHOLE: blocks of a multiple of 64 hold whole tiles (and rows of less than 32 MB, so that a place in a tile is 32 bits)
+template <int D, bool EXT, bool WHOLE>
+__global__ __launch_bounds__(256, D == 64 && EXT ? 3 : 2) void prompt_attn_kernel(WAttnArgs p, int tiles, int num_seqs, int bs_shift) {
   constexpr int KS = D / 16, DT = D / 32, ROWB = 2 * D, TILE = PA_KEYS * ROWB;      // bytes of one operand's tile
   constexpr int RPI = 1024 / ROWB, NI = PA_KEYS / RPI / 4;                          // rows per DMA instruction; instructions per wavefront
   constexpr float L2E = 1.4426950408889634f;
@@ -158,7 +170,6 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
   const char* k_base = reinterpret_cast<const char*>(p.cache) + (int64_t)g * ROWB;
   const char* v_base = reinterpret_cast<const char*>(p.cache) + ((int64_t)p.v_col + (int64_t)g * D) * 2;
   const int64_t row_bytes = (int64_t)p.cw * 2;
-  const bool whole_tiles = p.block_size % PA_KEYS == 0 && p.cw < (1 << 24);
   const bf16_t* sink = reinterpret_cast<const bf16_t*>(p.sink);
   auto k_swz = [](int r) { return D == 128 ? r & 15 : (r >> 1) & 7; };
   auto v_swz = [](int r) { return D == 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); };
@@ -166,13 +177,15 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
   // this lane's part of the DMA: row RPI * (wv * NI + i) + lane / (64 / RPI) of the tile, piece lane % (64 / RPI)
   constexpr int PIECES = 64 / RPI;                 // 16-byte pieces of a row
   const int dma_r = lane / PIECES, dma_p = lane % PIECES;
-  uint32_t row_off[NI], k_off[NI], v_off[NI];
+  uint32_t k_off[NI], v_off[NI];      // WHOLE: from the tile's first row, else from its own
+  auto row_of = [&](int i) { return RPI * (wv * NI + i) + dma_r; };
+  auto k_piece = [&](int i) { return (uint32_t)(dma_p ^ k_swz(row_of(i))) << 4; };
+  auto v_piece = [&](int i) { return (uint32_t)(dma_p ^ v_swz(row_of(i))) << 4; };
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int r = RPI * (wv * NI + i) + dma_r;
-    row_off[i] = (uint32_t)r * (uint32_t)row_bytes;
-    k_off[i] = (dma_p ^ k_swz(r)) << 4;
-    v_off[i] = (dma_p ^ v_swz(r)) << 4;
+    const uint32_t row = WHOLE ? (uint32_t)row_of(i) * (uint32_t)row_bytes : 0;
+    k_off[i] = row + k_piece(i);
+    v_off[i] = row + v_piece(i);
   }
   // fragment addresses inside a tile: K row lr of a 32-row tile, piece 2 ks + lh; V^T: four tokens by sixteen numbers per
   // sixteen lanes, rows 4 lh + (lane & 15) / 4 (and 8 further), numbers 16 (lr >> 4) + 4 (lane & 3)
@@ -198,11 +211,13 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
     float m_run = -INFINITY, l_run = 0.0f;
     const int wpos_lo = p0 + row0 / R, wpos_hi = p0 + min(rows - 1, row0 + 31) / R;
 
-    // The walk is over tiles of 64 keys from multiples of 64 on: those with kept keys (of which the first sees them all), then those from
-    // the first key of the tile's first row to the last key of its last.
+    // The walk is over tiles of 64 keys from multiples of 64 on: those with kept keys, then those from the first key of the tile's first row
+    // to the last key of its last.  Kept keys that fit the places ahead of that first key lie there instead of in a tile of their own.
     auto first_of = [&](int at) { return max(p.window > 0 ? at - p.window + 1 : 0, EXT && p.chunk > 0 ? at / p.chunk * p.chunk : 0); };
     const int low = first_of(pos), hi = p0 + nq - 1, wlow_lo = first_of(wpos_lo), wlow_hi = first_of(wpos_hi);
-    const int kept_tiles = EXT ? (min(p.keep, first_of(p0)) + PA_KEYS - 1) / PA_KEYS : 0;
+    const int kept_keys = EXT ? min(p.keep, first_of(p0)) : 0;
+    const int merged = EXT && first_of(p0) >= PA_KEYS && kept_keys <= first_of(p0) % PA_KEYS ? kept_keys : 0;
+    const int kept_tiles = merged > 0 ? 0 : (kept_keys + PA_KEYS - 1) / PA_KEYS;
     const int skipped = max(first_of(p0) / PA_KEYS - kept_tiles, 0), count = hi / PA_KEYS + 1 - skipped;
     auto tile_key = [&](int it) { return PA_KEYS * (it < kept_tiles ? it : it + skipped); };
     // Where its rows are.  Blocks of a multiple of 64 hold whole tiles: one page number for all lanes, asked for a tile ahead (as a vector
@@ -212,56 +227,83 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
     asm volatile("v_mov_b32 %0, 0" : "=v"(no_lane));
     auto look_up = [&](int it) {
       const int j0 = tile_key(min(it, count - 1));
-      if (whole_tiles) {
+      if constexpr (WHOLE) {
         page[0] = table[(bs_shift >= 0 ? j0 >> bs_shift : j0 / p.block_size) + no_lane];
-        return;
-      }
+        if (EXT && merged > 0 && it == 0) page[1] = table[no_lane];
+      } else {
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int kp = min(j0 + RPI * (wv * NI + i) + dma_r, hi);
-        const int n = bs_shift >= 0 ? kp >> bs_shift : kp / p.block_size;
-        in_page[i] = kp - n * p.block_size;
-        page[i] = table[n];
+        for (int i = 0; i < NI; ++i) {
+          const int r = row_of(i), kp = EXT && it == 0 && r < merged ? r : min(j0 + r, hi);
+          const int n = bs_shift >= 0 ? kp >> bs_shift : kp / p.block_size;
+          in_page[i] = kp - n * p.block_size;
+          page[i] = table[n];
+        }
       }
     };
     auto fill = [&](int buf, int it) {
       const uint32_t dst = lds_at + buf * 2 * TILE + wv * NI * 1024;
-      if (whole_tiles) {
+      if constexpr (WHOLE) {
         const int j0 = tile_key(it), n = bs_shift >= 0 ? j0 >> bs_shift : j0 / p.block_size;
         const int64_t at = ((int64_t)__builtin_amdgcn_readfirstlane(page[0]) * p.block_size + (j0 - n * p.block_size)) * row_bytes;
         const bool ends = hi - j0 < PA_KEYS - 1;
+        if (EXT && merged > 0 && it == 0) {
+          const int64_t at_kept = (int64_t)__builtin_amdgcn_readfirstlane(page[1]) * p.block_size * row_bytes;
+#pragma unroll
+          for (int i = 0; i < NI; ++i) {
+            const int r = row_of(i);
+            const int64_t row = r < merged ? at_kept + r * row_bytes : at + min(r, hi - j0) * row_bytes;
+            pa_dma(k_base + row + k_piece(i), dst + i * 1024);
+            pa_dma(v_base + row + v_piece(i), dst + i * 1024 + TILE);
+          }
+          return;
+        }
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
-          const uint32_t row = ends ? (uint32_t)min(RPI * (wv * NI + i) + dma_r, hi - j0) * (uint32_t)row_bytes : row_off[i];
-          pa_dma(k_base + at, row + k_off[i], dst + i * 1024);
-          pa_dma(v_base + at, row + v_off[i], dst + i * 1024 + TILE);
+          uint32_t k = k_off[i], v = v_off[i];
+          if (ends) {
+            const uint32_t row = (uint32_t)min(row_of(i), hi - j0) * (uint32_t)row_bytes;
+            k = row + k_piece(i);
+            v = row + v_piece(i);
+          }
+          pa_dma(k_base + at, k, dst + i * 1024);
+          pa_dma(v_base + at, v, dst + i * 1024 + TILE);
         }
-        return;
-      }
+      } else {
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int64_t at = ((int64_t)page[i] * p.block_size + in_page[i]) * row_bytes;
-        pa_dma(k_base + at + k_off[i], dst + i * 1024);
-        pa_dma(v_base + at + v_off[i], dst + i * 1024 + TILE);
+        for (int i = 0; i < NI; ++i) {
+          const int64_t at = ((int64_t)page[i] * p.block_size + in_page[i]) * row_bytes;
+          pa_dma(k_base + at + k_off[i], dst + i * 1024);
+          pa_dma(v_base + at + v_off[i], dst + i * 1024 + TILE);
+        }
       }
     };
     __builtin_amdgcn_s_barrier();            // an earlier request's walk through this tile has read its last buffer
     look_up(0);
-    const float* gates = p.gate ? p.gate + (ts + tok) * p.gate_rs : nullptr;
-    const float head_gate = EXT && p.gate_head && gates ? gates[head] : 0.0f;      // waited for at the end
+    const float head_gate = EXT && p.gate_head && p.gate ? p.gate[(ts + tok) * p.gate_rs + head] : 0.0f;      // waited for at the end
     fill(0, 0);
     look_up(1);
     // queries: lane holds numbers 16 ks + 8 lh .. + 7 of its row
     bf16x8 qf[KS];
     {
-      const float* qrow = p.q + ((ts + tok) * p.H + head) * D + 8 * lh;
+      const int64_t at = ((ts + tok) * p.H + head) * D + 8 * lh;
+      if (p.q16) {
+        const bf16_t* qrow = reinterpret_cast<const bf16_t*>(p.q) + at;
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const f32x4 a = *reinterpret_cast<const f32x4*>(qrow + 16 * ks), c = *reinterpret_cast<const f32x4*>(qrow + 16 * ks + 4);
+        for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(qrow + 16 * ks);
+        if (!valid) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          qf[ks][e] = (bf16_t)(valid ? a[e] : 0.0f);
-          qf[ks][4 + e] = (bf16_t)(valid ? c[e] : 0.0f);
+          for (int ks = 0; ks < KS; ++ks) qf[ks] = __builtin_bit_cast(bf16x8, u32x4{0, 0, 0, 0});
+        }
+      } else {
+        const float* qrow = reinterpret_cast<const float*>(p.q) + at;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const f32x4 a = *reinterpret_cast<const f32x4*>(qrow + 16 * ks), c = *reinterpret_cast<const f32x4*>(qrow + 16 * ks + 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            qf[ks][e] = (bf16_t)(valid ? a[e] : 0.0f);
+            qf[ks][4 + e] = (bf16_t)(valid ? c[e] : 0.0f);
+          }
         }
       }
     }
@@ -276,7 +318,8 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
       }
       // keys that this wavefront's rows can see at all, and whether some row sees none of the first or none of the last of them
       const int j0 = tile_key(it), j1 = j0 + PA_KEYS - 1;
-      if (!wave_on || j0 > wpos_hi || (j1 < wlow_lo && (!EXT || j0 >= p.keep))) continue;
+      const bool with_kept = EXT && merged > 0 && it == 0;
+      if (!wave_on || j0 > wpos_hi || (j1 < wlow_lo && (!EXT || (j0 >= p.keep && !with_kept)))) continue;
       const bool cut_low = wlow_hi > j0 && (!EXT || j1 >= p.keep), cut_high = j1 > wpos_lo;
       const unsigned char* kt = lds[buf];
       f32x16 s[2];
@@ -286,7 +329,7 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
         for (int r = 0; r < 16; ++r) s[t][r] = 0.0f;
       // every product has its fragment read AHEAD products before it, in the order written here: left alone, the compiler reads each
       // right before its product and waits for it
-      constexpr int AHEAD = 4, QK = 2 * KS, PV = 4 * DT;
+      constexpr int AHEAD = D == 64 ? 3 : 4, QK = 2 * KS, PV = 4 * DT;
       bf16x8 kf[QK], vf[PV];
       auto k_read = [&](int f) { kf[f] = *reinterpret_cast<const bf16x8*>(kt + (32 * (f & 1) + lr) * ROWB + (((f & ~1) + lh) ^ ksw) * 16); };
       auto v_read = [&](int f) {
@@ -306,7 +349,7 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
         __builtin_amdgcn_sched_barrier(0);
       }
       // place k of the lane's keys is key c0 + k
-      const int c0 = j0 + 4 * lh, last = pos - c0, first = low - c0, kept = p.keep - c0;
+      const int c0 = j0 + 4 * lh, last = pos - c0, first = low - c0, kept = with_kept ? merged - 4 * lh : p.keep - c0;
       if (cut_low) {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -378,7 +421,11 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(WAttnArgs p, int ti
       const uint64_t odd_lanes = __ballot(odd && valid);
       float l_lo, l_hi;
       rows_pair32(l_run, l_lo, l_hi);
-      if (valid) {
+      int again = rr;                           // what the walk does not need is formed anew: registers
+      asm volatile("" : "+v"(again));
+      if (again < rows) {
+        const int tok = again / R, head = g * R + again % R;
+        const float* gates = p.gate ? p.gate + (ts + tok) * p.gate_rs : nullptr;
         float fs, den;
         close_softmax(m_run, l_lo + l_hi, sink != nullptr, sink ? ld_f32<bf16_t>(sink + head) : 0.0f, fs, den);
         float f = p.out_scale * fs / den;
@@ -420,13 +467,13 @@ hipError_t launch_prompt_attn(WAttnArgs p, int num_seqs, hipStream_t s) {
   if ((p.block_size & (p.block_size - 1)) == 0)
     for (shift = 0; (1 << shift) < p.block_size;) ++shift;
   const dim3 grid((unsigned)((tiles * p.G + 7) / 8 * 8));
-  if (p.chunk > 0 || p.keep > 0 || (p.gate && p.gate_head)) prompt_attn_kernel<D, true><<<grid, dim3(256), 0, s>>>(p, (int)tiles, num_seqs, shift);
-  else prompt_attn_kernel<D, false><<<grid, dim3(256), 0, s>>>(p, (int)tiles, num_seqs, shift);
+  const bool whole = p.block_size % PA_KEYS == 0 && p.cw < (1 << 24);
+  if (p.chunk > 0 || p.keep > 0 || (p.gate && p.gate_head)) {
+    if (whole) prompt_attn_kernel<D, true, true><<<grid, dim3(256), 0, s>>>(p, (int)tiles, num_seqs, shift);
+    else prompt_attn_kernel<D, true, false><<<grid, dim3(256), 0, s>>>(p, (int)tiles, num_seqs, shift);
+  } else {
+    if (whole) prompt_attn_kernel<D, false, true><<<grid, dim3(256), 0, s>>>(p, (int)tiles, num_seqs, shift);
+    else prompt_attn_kernel<D, false, false><<<grid, dim3(256), 0, s>>>(p, (int)tiles, num_seqs, shift);
+  }
   return hipGetLastError();
-}
-
-// The kernel's sizes: heads of 64 or 128 for keys and values alike, 16-byte rows, scores without cap and distance term.
-inline bool prompt_attn_serves(const WAttnArgs& p) {
-  return (p.d == 64 || p.d == 128) && p.dv == p.d && p.H / p.G <= PA_ROWS && p.softcap <= 0.0f && !p.slope_on &&
-         (uintptr_t)p.q % 16 == 0 && (uintptr_t)p.out % 8 == 0 && p.out_rs % 4 == 0;
 }

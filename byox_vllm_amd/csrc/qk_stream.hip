@@ -1,5 +1,5 @@
 // q/k/v of attention over its own paged rows, for prompts: the projection (and the columns behind it, gates and the like) on the tiles of
-// stream_deep.h, rotated, scaled and stored on the way: fp32 queries, cache rows [k | v] in bf16, the other columns in fp32.
+// stream_deep.h, rotated, scaled and stored on the way: queries in fp32 or bf16, cache rows [k | v] in bf16, the other columns in fp32.
 //
 // What bounded these steps: the projection was written in fp32 and read again.  16384 rows 2048 -> 16 + 8 + 8 heads of 128 and 16 gates: the
 // product 277 us and qk_pairs_store_kernel 110; here 240, the turns' cosines and sines, once per token, among them (the layer 670 and 516).  The
@@ -15,10 +15,12 @@ struct QkvArgs {
   const float* turns;         // [tokens, 2 * half]: cosines, then sines
   const int32_t* slots;
   uint16_t* cache;            // [rows, nkv]
-  float *q, *rest;            // [tokens, nq], [tokens, rest_rs]
+  void* q;                    // [tokens, nq]
+  float* rest;                // [tokens, rest_rs]
   int64_t rest_rs;
   int M, N, K, nq, nk, nkv;
   float scale;
+  int q16;                    // queries in bf16
 };
 
 // HALF16: a head's rotated numbers are 2 * 16 * HALF16, i with i + 16 * HALF16; 0: none
@@ -110,7 +112,9 @@ struct QkvJob {
           f32x4 v = x[j];
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] *= p.scale;
-          *reinterpret_cast<f32x4*>(p.q + (int64_t)t * p.nq + n + 4 * g) = v;
+          const int64_t to = (int64_t)t * p.nq + n + 4 * g;
+          if (p.q16) *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(p.q) + to) = Pack4<bf16_t>::narrow(v);
+          else *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.q) + to) = v;
         } else if (n < p.nq + p.nkv) {
           if (slot[r] >= 0)
             *reinterpret_cast<uint2*>(p.cache + (int64_t)slot[r] * p.nkv + (n - p.nq) + 4 * g) = Pack4<bf16_t>::narrow(x[j]);
@@ -149,6 +153,15 @@ extern "C" int nv_qkv_stream(const void* x, int64_t x_row_stride, const void* w,
                              const float* inv_freq, int rot_dims, float mscale, float scale, const int32_t* slot_mapping, void* cache,
                              float* q_out, float* rest, int64_t rest_row_stride, float* turns, int heads, int kv_heads, int dim, int vdim,
                              nv_stream_t stream) {
+  return nv_qkv_stream_as(x, x_row_stride, w, tokens, N, K, positions, inv_freq, rot_dims, mscale, scale, slot_mapping, cache, q_out, NV_F32,
+                          rest, rest_row_stride, turns, heads, kv_heads, dim, vdim, stream);
+}
+
+extern "C" int nv_qkv_stream_as(const void* x, int64_t x_row_stride, const void* w, int64_t tokens, int N, int K, const int64_t* positions,
+                                const float* inv_freq, int rot_dims, float mscale, float scale, const int32_t* slot_mapping, void* cache,
+                                void* q_out, int q_dtype, float* rest, int64_t rest_row_stride, float* turns, int heads, int kv_heads,
+                                int dim, int vdim, nv_stream_t stream) {
+  NV_CHECK_ARG(q_dtype == NV_F32 || q_dtype == NV_BF16, "nv_qkv_stream: bad dtype %d of the queries", q_dtype);
   NV_CHECK_ARG(x && w && slot_mapping && cache && q_out, "nv_qkv_stream: null pointer");
   NV_CHECK_ARG(dim == 64 || dim == 128, "nv_qkv_stream: head_dim %d not in {64, 128}", dim);
   NV_CHECK_ARG(heads > 0 && kv_heads > 0 && heads <= 65536 && kv_heads <= 65536 && vdim > 0 && vdim <= 65536 && kv_heads * vdim % 16 == 0,
@@ -172,7 +185,7 @@ extern "C" int nv_qkv_stream(const void* x, int64_t x_row_stride, const void* w,
     NV_CHECK_LAUNCH();
   }
   const QkvArgs p{(const uint16_t*)x, (const uint16_t*)w, x_row_stride, turns, slot_mapping, (uint16_t*)cache, q_out, rest, rest_row_stride,
-                  (int)tokens, N, K, (int)nq, (int)nk, (int)nkv, scale};
+                  (int)tokens, N, K, (int)nq, (int)nk, (int)nkv, scale, q_dtype == NV_BF16};
   hipError_t e;
   if (dim == 64) e = rot_dims == 0 ? qkv_go<64, 0>(p, s) : rot_dims == 32 ? qkv_go<64, 1>(p, s) : qkv_go<64, 2>(p, s);
   else e = rot_dims == 0 ? qkv_go<128, 0>(p, s) : rot_dims == 32 ? qkv_go<128, 1>(p, s) : rot_dims == 64 ? qkv_go<128, 2>(p, s) : qkv_go<128, 4>(p, s);

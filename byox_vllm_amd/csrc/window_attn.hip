@@ -345,7 +345,7 @@ __global__ __launch_bounds__(256) void qk_conv_store_kernel(QkConvArgs p, int TT
 }
 
 struct WAttnArgs {
-  const float* q;          // [tokens, H * d]
+  const float* q;          // [tokens, H * d]; q16: bf16 in fact (prompt_attn_kernel alone)
   const void* cache;       // [rows, G * (d + dv)]
   const int32_t* tables;   // [B, table_cols]
   int table_cols;
@@ -367,6 +367,7 @@ struct WAttnArgs {
   int keep;                // the first `keep` keys stay visible behind the window (0: none; not together with chunk)
   int ksplit;              // SPLIT only: workgroups that share a token's keys (blockIdx.z); > 1: results go to `partial`
   float* partial;          // [tokens, H, ksplit, dv + 2]: unnormalised output, then maximum and sum
+  int q16;
 };
 
 // (factor for the accumulated values, denominator) once the walk over the keys is over: the sink joins the sum
@@ -1164,7 +1165,37 @@ extern "C" int nv_paged_softmax_attn(const float* q, const void* cache, const in
                                      workspace, workspace_bytes, dtype, stream);
 }
 
+// Whether a step goes to prompt_attn_kernel, whose queries enter the products in bf16
+static bool prompt_attn_step(const void* cache, int64_t out_row_stride, int64_t tokens, int max_q, int heads, int kv_heads, int dim, int vdim,
+                             int values_are_keys, float softcap, int distance_term, int dtype) {
+  const int cw = values_are_keys ? kv_heads * dim : kv_heads * (dim + vdim), v_col = values_are_keys ? 0 : kv_heads * dim;
+  return dtype == NV_BF16 && (dim == 64 || dim == 128) && vdim == dim && heads / kv_heads <= 64 && kv_heads <= 65535 &&
+         (uintptr_t)cache % 16 == 0 && cw % 8 == 0 && v_col % 8 == 0 && max_q > 1 && softcap <= 0.0f && !distance_term &&
+         out_row_stride % 4 == 0 && (tokens * (int64_t)kv_heads + 7) / 8 * 8 < (1 << 30) && getenv("NV_WINDOW_ATTN_MFMA_OFF") == nullptr &&
+         getenv("NV_WINDOW_ATTN_PROMPT_OFF") == nullptr;
+}
+
+extern "C" int nv_paged_softmax_attn_takes_q16(const void* cache, int64_t out_row_stride, int64_t tokens, int max_q, int heads, int kv_heads,
+                                               int dim, int vdim, int values_are_keys, float softcap, int distance_term, int dtype) {
+  return heads > 0 && kv_heads > 0 && heads % kv_heads == 0 &&
+         prompt_attn_step(cache, out_row_stride, tokens, max_q, heads, kv_heads, dim, vdim, values_are_keys, softcap, distance_term, dtype);
+}
+
 extern "C" int nv_paged_softmax_attn_batch(const float* q, const void* cache, const int32_t* block_tables, int table_cols,
+                                           const int32_t* cu_q, const int32_t* past_lens, const int32_t* seq_of_token,
+                                           void* out, int64_t out_row_stride, int64_t tokens, int num_seqs, int max_q,
+                                           int heads, int kv_heads, int dim, int vdim, int block_size, int window, int chunk,
+                                           int keep_first, float softcap, float out_scale, int distance_term,
+                                           int values_are_keys, const void* sink, const float* gate, int64_t gate_row_stride,
+                                           int gate_per_head, void* workspace, size_t workspace_bytes, int dtype,
+                                           nv_stream_t stream) {
+  return nv_paged_softmax_attn_q(q, NV_F32, cache, block_tables, table_cols, cu_q, past_lens, seq_of_token, out, out_row_stride, tokens,
+                                 num_seqs, max_q, heads, kv_heads, dim, vdim, block_size, window, chunk, keep_first, softcap, out_scale,
+                                 distance_term, values_are_keys, sink, gate, gate_row_stride, gate_per_head, workspace, workspace_bytes,
+                                 dtype, stream);
+}
+
+extern "C" int nv_paged_softmax_attn_q(const void* q, int q_dtype, const void* cache, const int32_t* block_tables, int table_cols,
                                            const int32_t* cu_q, const int32_t* past_lens, const int32_t* seq_of_token,
                                            void* out, int64_t out_row_stride, int64_t tokens, int num_seqs, int max_q,
                                            int heads, int kv_heads, int dim, int vdim, int block_size, int window, int chunk,
@@ -1180,6 +1211,9 @@ extern "C" int nv_paged_softmax_attn_batch(const float* q, const void* cache, co
                    block_size > 0 && window >= 0 && chunk >= 0 && keep_first >= 0 && table_cols > 0 && num_seqs >= 0,
                "nv_window_attn: bad shape");
   NV_CHECK_ARG(chunk == 0 || keep_first == 0, "nv_window_attn: chunks and kept first keys exclude each other");
+  const bool prompt = prompt_attn_step(cache, out_row_stride, tokens, max_q, heads, kv_heads, dim, vdim, values_are_keys, softcap,
+                                       distance_term, dtype) && (uintptr_t)q % 16 == 0 && (uintptr_t)out % 8 == 0;
+  NV_CHECK_ARG(q_dtype == NV_F32 || (q_dtype == NV_BF16 && prompt), "nv_window_attn: this step does not take queries of dtype %d", q_dtype);
   if (tokens == 0) return NV_OK;
   const int R = heads / kv_heads;
   // bf16 caches with 16-byte-aligned heads of up to 256 numbers: the matrix-core kernel
@@ -1196,14 +1230,14 @@ extern "C" int nv_paged_softmax_attn_batch(const float* q, const void* cache, co
       int ksplit = split || rows ? window_attn_key_splits(tokens, kv_heads) : 1;
       if (ksplit > 1 && (!workspace || workspace_bytes < (size_t)tokens * heads * ksplit * (vdim + 2) * sizeof(float)))
         ksplit = 1;
-      WAttnArgs pm{q, cache, block_tables, table_cols, cu_q, past_lens, seq_of_token, out, out_row_stride, tokens, heads,
+      WAttnArgs pm{reinterpret_cast<const float*>(q), cache, block_tables, table_cols, cu_q, past_lens, seq_of_token, out, out_row_stride, tokens, heads,
                    kv_heads, dim, vdim, block_size, window, TQm, MA_KEYS, softcap, out_scale, cw, v_col, distance_term, sink,
-                   gate, gate_row_stride, gate_per_head, chunk, keep_first, ksplit, reinterpret_cast<float*>(workspace)};
+                   gate, gate_row_stride, gate_per_head, chunk, keep_first, ksplit, reinterpret_cast<float*>(workspace),
+                   q_dtype == NV_BF16};
       dim3 gridm((unsigned)((tokens + TQm - 1) / TQm), (unsigned)kv_heads, (unsigned)ksplit);
       hipStream_t st = (hipStream_t)stream;
       const int wide = dim > vdim ? dim : vdim;
-      if (max_q > 1 && prompt_attn_serves(pm) && (tokens * (int64_t)kv_heads + 7) / 8 * 8 < (1 << 30) &&
-          getenv("NV_WINDOW_ATTN_PROMPT_OFF") == nullptr) {
+      if (prompt) {
         const hipError_t e = dim == 64 ? launch_prompt_attn<64>(pm, num_seqs, st) : launch_prompt_attn<128>(pm, num_seqs, st);
         if (e != hipSuccess) {
           nv_set_error("nv_window_attn: %s", hipGetErrorString(e));
@@ -1239,7 +1273,7 @@ extern "C" int nv_paged_softmax_attn_batch(const float* q, const void* cache, co
   while (TQ > 1 && (need(TQ, TK) > budget || TQ * R > 256)) TQ /= 2;
   NV_CHECK_ARG(R <= 256 && kv_heads <= 65535, "nv_window_attn: %d query heads per key head exceed a workgroup", R);
   const int64_t tiles = (tokens + TQ - 1) / TQ;
-  WAttnArgs p{q, cache, block_tables, table_cols, cu_q, past_lens, seq_of_token, out, out_row_stride, tokens, heads,
+  WAttnArgs p{reinterpret_cast<const float*>(q), cache, block_tables, table_cols, cu_q, past_lens, seq_of_token, out, out_row_stride, tokens, heads,
               kv_heads, dim, vdim, block_size, window, TQ, TK, softcap, out_scale, cw, v_col, distance_term, sink, gate,
               gate_row_stride, gate_per_head, chunk, keep_first, 1, nullptr};
   dim3 grid((unsigned)tiles, (unsigned)kv_heads);

@@ -989,14 +989,14 @@ def latent_q_rope(q, positions, inv_freq, mscale, qa, heads, dim, rot_dim, rot_d
           "nv_latent_q_rope")
 
 
-def latent_q_rows(q, positions, inv_freq, mscale, heads, dim, rot_dim, rot_dims, factor, interleaved=False):
-    """q [T, heads * (dim + rot_dim)] -> fp32 rows of the same layout, the rotated part turned, everything times
+def latent_q_rows(q, positions, inv_freq, mscale, heads, dim, rot_dim, rot_dims, factor, interleaved=False, out_dtype=torch.float32):
+    """q [T, heads * (dim + rot_dim)] -> rows of the same layout in ``out_dtype``, the rotated part turned, everything times
     ``factor``."""
     require_gpu(q, "latent_q_rows")
     assert q.stride(1) == 1 and q.size(1) == heads * (dim + rot_dim) and positions.dtype == torch.int64
-    out = torch.empty(q.size(0), heads * (dim + rot_dim), dtype=torch.float32, device=q.device)
-    check(lib().nv_latent_q_rows(ptr(q), q.stride(0), ptr(positions), ptr(inv_freq), mscale, ptr(out), q.size(0), heads,
-                                 dim, rot_dim, rot_dims, int(interleaved), dim, 1, factor, _code32(q.dtype), stream()),
+    out = torch.empty(q.size(0), heads * (dim + rot_dim), dtype=out_dtype, device=q.device)
+    check(lib().nv_latent_q_rows_as(ptr(q), q.stride(0), ptr(positions), ptr(inv_freq), mscale, ptr(out), _code32(out_dtype), q.size(0), heads,
+                                    dim, rot_dim, rot_dims, int(interleaved), dim, 1, factor, _code32(q.dtype), stream()),
           "nv_latent_q_rows")
     return out
 
@@ -1274,9 +1274,10 @@ def qkv_streams(x, w, heads, kv_heads, dim, vdim, rot_dims, interleaved) -> bool
             and tile_share(M, N) >= (0.7 if K <= 2048 else 0.78))
 
 
-def qkv_project_store(x, w, positions, scale, slot_mapping, cache, heads, kv_heads, dim, vdim, *, inv_freq=None, rot_dims=0, mscale=1.0):
-    """linear(x, w) into fp32 and qk_rotate_store in one pass (qkv_streams) -> the fp32 queries [T, heads * dim], and the columns of w behind
-    q | k | v, fp32 [T, *]."""
+def qkv_project_store(x, w, positions, scale, slot_mapping, cache, heads, kv_heads, dim, vdim, *, inv_freq=None, rot_dims=0, mscale=1.0,
+                      q_dtype=torch.float32):
+    """linear(x, w) into fp32 and qk_rotate_store in one pass (qkv_streams) -> the queries [T, heads * dim] in ``q_dtype``, and the columns of w
+    behind q | k | v, fp32 [T, *]."""
     require_gpu(x, "qkv_project_store")
     T, N = x.size(0), w.size(0)
     rest_cols = N - heads * dim - kv_heads * (dim + vdim)
@@ -1285,12 +1286,13 @@ def qkv_project_store(x, w, positions, scale, slot_mapping, cache, heads, kv_hea
     assert positions.dtype == torch.int64 and positions.numel() == T and positions.is_contiguous()
     if rot_dims:
         assert inv_freq.dtype == torch.float32 and inv_freq.is_contiguous() and inv_freq.numel() * 2 >= rot_dims and inv_freq.is_cuda
-    q = torch.empty(T, heads * dim, dtype=torch.float32, device=x.device)
+    q = torch.empty(T, heads * dim, dtype=q_dtype, device=x.device)
     rest = torch.empty(T, rest_cols, dtype=torch.float32, device=x.device)
     turns = torch.empty(T, rot_dims, dtype=torch.float32, device=x.device) if rot_dims else None
-    check(lib().nv_qkv_stream(ptr(x), x.stride(0), ptr(w), T, N, w.size(1), ptr(positions), ptr(inv_freq) if rot_dims else None, int(rot_dims),
-                              float(mscale), float(scale), ptr(slot_mapping), ptr(cache), ptr(q), ptr(rest) if rest_cols else None,
-                              max(1, rest_cols), ptr(turns), heads, kv_heads, dim, vdim, stream()), "nv_qkv_stream")
+    check(lib().nv_qkv_stream_as(ptr(x), x.stride(0), ptr(w), T, N, w.size(1), ptr(positions), ptr(inv_freq) if rot_dims else None,
+                                 int(rot_dims), float(mscale), float(scale), ptr(slot_mapping), ptr(cache), ptr(q), _code32(q_dtype),
+                                 ptr(rest) if rest_cols else None, max(1, rest_cols), ptr(turns), heads, kv_heads, dim, vdim, stream()),
+          "nv_qkv_stream")
     return q, rest
 
 
@@ -1343,6 +1345,14 @@ def qk_store(proj, offsets, positions, scale, slot_mapping, cache, heads, kv_hea
     return q
 
 
+def prompt_query_dtype(cache, tokens, max_q, heads, kv_heads, dim, vdim):
+    """The dtype in which paged_softmax_attn takes the queries of a step without cap, distance term or keys that are the values, into a
+    contiguous result: bf16 where they enter the products in bf16 in any case, which half of the bytes then say as well."""
+    takes = lib().nv_paged_softmax_attn_takes_q16(ptr(cache), heads * vdim, tokens, max_q, heads, kv_heads, dim, vdim, 0, 0.0, 0,
+                                                  _code32(cache.dtype))
+    return torch.bfloat16 if takes else torch.float32
+
+
 def paged_softmax_attn(q, cache, block_tables, cu_q, past_lens, seq_of_token, max_q, heads, kv_heads, dim, vdim, block_size,
                        out, window=0, softcap=0.0, out_scale=1.0, distance_term=False, values_are_keys=False, sink=None,
                        gate=None, chunk=0, gate_per_head=False, keep_first=0):
@@ -1350,10 +1360,10 @@ def paged_softmax_attn(q, cache, block_tables, cu_q, past_lens, seq_of_token, ma
     serve as values too, a sink logit per head in the denominator, a sigmoid gate (fp32 logits laid out like the
     output, or with ``gate_per_head`` one per head) folded into the store, and ``chunk`` > 0: a query sees the keys
     of its own chunk of the sequence only; ``keep_first`` > 0: the first keys of the sequence stay visible
-    beside the window."""
+    beside the window.  ``q`` in fp32, or in bf16 where prompt_query_dtype says so."""
     require_gpu(q, "paged_softmax_attn")
     T = q.size(0)
-    assert q.dtype == torch.float32 and q.is_contiguous() and q.size(1) == heads * dim and cache.is_contiguous()
+    assert q.dtype in (torch.float32, torch.bfloat16) and q.is_contiguous() and q.size(1) == heads * dim and cache.is_contiguous()
     assert cache.size(-1) == (kv_heads * dim if values_are_keys else kv_heads * (dim + vdim))
     assert block_tables.dtype == torch.int32 and block_tables.is_contiguous() and block_tables.dim() == 2
     assert cu_q.dtype == past_lens.dtype == seq_of_token.dtype == torch.int32 and seq_of_token.numel() == T
@@ -1365,14 +1375,14 @@ def paged_softmax_attn(q, cache, block_tables, cu_q, past_lens, seq_of_token, ma
     # by the warm-up run of the same shape)
     nbytes = lib().nv_paged_softmax_attn_workspace_bytes(T, max_q, heads, kv_heads, vdim) if cache.dtype == torch.bfloat16 else 0
     ws = workspace(nbytes, q.device, "paged_softmax_attn") if nbytes else None
-    check(lib().nv_paged_softmax_attn_batch(ptr(q), ptr(cache), ptr(block_tables), block_tables.size(1), ptr(cu_q),
-                                            ptr(past_lens), ptr(seq_of_token), ptr(out), out.stride(0), T,
-                                            min(cu_q.numel() - 1, past_lens.numel()), max_q, heads, kv_heads, dim, vdim,
-                                            block_size, window, int(chunk), int(keep_first), float(softcap or 0.0), out_scale,
-                                            int(distance_term), int(values_are_keys), ptr(sink), ptr(gate),
-                                            gate.stride(0) if gate is not None else 0, int(gate_per_head), ptr(ws), nbytes,
-                                            _code32(cache.dtype), stream()),
-          "nv_paged_softmax_attn_batch")
+    check(lib().nv_paged_softmax_attn_q(ptr(q), _code32(q.dtype), ptr(cache), ptr(block_tables), block_tables.size(1), ptr(cu_q),
+                                        ptr(past_lens), ptr(seq_of_token), ptr(out), out.stride(0), T,
+                                        min(cu_q.numel() - 1, past_lens.numel()), max_q, heads, kv_heads, dim, vdim,
+                                        block_size, window, int(chunk), int(keep_first), float(softcap or 0.0), out_scale,
+                                        int(distance_term), int(values_are_keys), ptr(sink), ptr(gate),
+                                        gate.stride(0) if gate is not None else 0, int(gate_per_head), ptr(ws), nbytes,
+                                        _code32(cache.dtype), stream()),
+          "nv_paged_softmax_attn_q")
     return out
 
 

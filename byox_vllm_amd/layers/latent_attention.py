@@ -113,8 +113,8 @@ class LatentAttention(nn.Module):
         cols = ctx.context_rows // bs          # at most: one request owns every block
         tables = (torch.div(ctx.cu_context[:B], bs, rounding_mode="floor")[:, None]
                   + torch.arange(cols, dtype=torch.int32, device=q.device)[None]).to(torch.int32).contiguous()
-        qf = kernels.latent_q_rows(q, positions, inv_freq, self.magnitude, H, d, r, self.rot_dims, self.scale,
-                                   self.interleaved)
+        qf = kernels.latent_q_rows(q, positions, inv_freq, self.magnitude, H, d, r, self.rot_dims, self.scale, self.interleaved,
+                                   kernels.prompt_query_dtype(rows, q.size(0), ctx.max_seqlen_q, H, H, d + r, dv))
         out = torch.empty(q.size(0), H * dv, dtype=q.dtype, device=q.device)
         g = self.down.offset("g")
         if self.gate_per_number:

@@ -51,7 +51,8 @@ class SlidingAttention(nn.Module):
         if called_plainly(self.inp, DenseLinear) and self.inp.bias is None and own.cache.dtype == h.dtype and \
                 own.cache.data_ptr() % 8 == 0 and kernels.qkv_streams(h, self.inp.weight, H, G, d, dv, self.rot_dims, self.interleaved):
             q, gates = kernels.qkv_project_store(h, self.inp.weight.data, positions, self.scale, ctx.slot_mapping, own.cache, H, G, d, dv,
-                                                 inv_freq=self.inv_freq, rot_dims=self.rot_dims, mscale=self.magnitude)
+                                                 inv_freq=self.inv_freq, rot_dims=self.rot_dims, mscale=self.magnitude,
+                                                 q_dtype=kernels.prompt_query_dtype(own.cache, h.size(0), ctx.max_seqlen_q, H, G, d, dv))
         else:
             proj = self.inp(h, out_dtype=torch.float32)
             q = kernels.qk_rotate_store(proj, (0, H * d, (H + G) * d), positions, self.scale, ctx.slot_mapping, own.cache, H, G, d,

@@ -534,6 +534,10 @@ int nv_latent_q_rope(const void* q, int64_t q_row_stride, const int64_t* positio
 int nv_latent_q_rows(const void* q, int64_t q_row_stride, const int64_t* positions, const float* inv_freq, float mscale,
                      float* qa, int64_t tokens, int heads, int dim, int rot_dim, int rot_dims, int interleaved, int rank,
                      int copy_front, float factor, int dtype, nv_stream_t stream);
+/* nv_latent_q_rows_as: the rows in qa_dtype (NV_F32, NV_BF16). */
+int nv_latent_q_rows_as(const void* q, int64_t q_row_stride, const int64_t* positions, const float* inv_freq, float mscale,
+                        void* qa, int qa_dtype, int64_t tokens, int heads, int dim, int rot_dim, int rot_dims, int interleaved, int rank,
+                        int copy_front, float factor, int dtype, nv_stream_t stream);
 int nv_latent_gather(const void* cache, const int32_t* block_tables, int table_cols, const int32_t* cu_k,
                      const int32_t* cu_q, const int32_t* past_lens, int num_seqs, int block_size, int row_width, void* out,
                      int64_t rows, int dtype, nv_stream_t stream);
@@ -649,6 +653,17 @@ int nv_paged_softmax_attn_batch(const float* q, const void* cache, const int32_t
                                 float out_scale, int distance_term, int values_are_keys, const void* sink, const float* gate,
                                 int64_t gate_row_stride, int gate_per_head, void* workspace, size_t workspace_bytes, int dtype,
                                 nv_stream_t stream);
+/* nv_paged_softmax_attn_q: queries in q_dtype.  NV_BF16 where nv_paged_softmax_attn_takes_q16 (prompts in bf16, heads of 64 or 128 for keys and
+ * values alike, scores without cap and distance term; q 16-byte, out 8-byte aligned): there they enter the products in bf16 in any case. */
+int nv_paged_softmax_attn_takes_q16(const void* cache, int64_t out_row_stride, int64_t tokens, int max_q, int heads, int kv_heads, int dim,
+                                    int vdim, int values_are_keys, float softcap, int distance_term, int dtype);
+int nv_paged_softmax_attn_q(const void* q, int q_dtype, const void* cache, const int32_t* block_tables, int table_cols,
+                                const int32_t* cu_q, const int32_t* past_lens, const int32_t* seq_of_token, void* out,
+                                int64_t out_row_stride, int64_t tokens, int num_seqs, int max_q, int heads, int kv_heads,
+                                int dim, int vdim, int block_size, int window, int chunk, int keep_first, float softcap,
+                                float out_scale, int distance_term, int values_are_keys, const void* sink, const float* gate,
+                                int64_t gate_row_stride, int gate_per_head, void* workspace, size_t workspace_bytes, int dtype,
+                                nv_stream_t stream);
 int nv_qk_rotate_store(const float* proj, const void* bias, int64_t proj_row_stride, int q_off, int k_off, int v_off,
                        const void* q_norm, const void* k_norm, int norm_whole, const void* temp, const int64_t* positions,
                        float temp_coef, int temp_every, const float* inv_freq, int rot_dims, int interleaved, float mscale,
@@ -663,6 +678,11 @@ int nv_qk_rotate_store(const float* proj, const void* bias, int64_t proj_row_str
 int nv_qkv_stream(const void* x, int64_t x_row_stride, const void* w, int64_t tokens, int N, int K, const int64_t* positions,
                   const float* inv_freq, int rot_dims, float mscale, float scale, const int32_t* slot_mapping, void* cache, float* q_out,
                   float* rest, int64_t rest_row_stride, float* turns, int heads, int kv_heads, int dim, int vdim, nv_stream_t stream);
+/* nv_qkv_stream_as: the queries in q_dtype (NV_F32, NV_BF16). */
+int nv_qkv_stream_as(const void* x, int64_t x_row_stride, const void* w, int64_t tokens, int N, int K, const int64_t* positions,
+                     const float* inv_freq, int rot_dims, float mscale, float scale, const int32_t* slot_mapping, void* cache, void* q_out,
+                     int q_dtype, float* rest, int64_t rest_row_stride, float* turns, int heads, int kv_heads, int dim, int vdim,
+                     nv_stream_t stream);
 /* nv_qk_conv_store: the store behind a short causal convolution (no bias) over time on every channel of q, k and v; w
  *   [H dim + G dim + G vdim, taps], state [slots, taps - 1, H dim + G dim + G vdim] keeps the last inputs; norm: every
  *   query and key head is then divided by its root mean square; q * scale to q_out, k and v to the cache.  Serves what
