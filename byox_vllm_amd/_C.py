@@ -99,6 +99,8 @@ _PROTOS = {
     "nv_matrix_memory_state_size": (_i64, [_i, _i, _i]),
     "nv_matrix_memory": (_i, [_p, _i64, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _i64, _i, _i, _i, _i, _i, _i, _f, _f,
                               _p, _i, _f, _i, _i, _p]),
+    "nv_matrix_memory_batch": (_i, [_p, _i64, _i, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i, _i, _i, _i, _i, _i, _f, _f,
+                                    _p, _i, _f, _i, _i, _p]),
     "nv_retention_step_ok": (_i, [_p, _i64, _i, _i, _i, _i, _p, _p, _i64, _i, _i]),
     "nv_retention_step": (_i, [_p, _i64, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p, _i, _f, _f, _f, _i, _p, _i64, _i, _i, _i, _i, _i,
                                _p]),
@@ -146,6 +148,8 @@ _PROTOS = {
     "nv_mingru_scan": (_i, [_p, _i64, _i, _i, _i, _p, _p, _p, _p, _p, _p, _p, _i64, _i, _i, _i, _p]),
     "nv_ssd_scan": (_i, [_p, _i64, _p, _i64, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _p, _sz, _i,
                          _p]),
+    "nv_ssd_scan_batch": (_i, [_p, _i64, _p, _i64, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _i64, _i, _i, _i, _i, _i, _i, _p, _sz, _i,
+                               _p]),
     "nv_ssd_scan_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
 }
 

@@ -16,6 +16,7 @@
 // m of a four-number sum taking the numbers {16 kk + 4 g + m}, an accumulator of S (rows 4 g + m of tile kk, column c) IS
 // the operand fragment of the next chunk's q . S.  The serial chain of a prompt is one chunk of about 40 matrix
 // instructions per wavefront; the walk it replaces is bound by the issue of 2 dim FMAs per column and token.
+// Prompts with a decay per head and token take chunk_parts.h instead, but for steps of few tokens to a request.
 //
 // Measured against that walk: channel decays, 8 x 2048 tokens, 16 heads of 64 x 128: 2560 us then, 316 now (542 MB of operands:
 // 1.7 TB/s); exponential gates, 64 requests of about 256 tokens, 8 heads of 64 x 128: 477 and 82; one decay per token, 4 requests
@@ -58,6 +59,7 @@ struct Args {
   float* ws_state;       // [B * H * runs][dim * vdim] state at the end of each run
   float* ws_decay;       // SSD [B * H * runs], GLA [B * H * runs][dim]: product of the run's decays
   int runs, run_len, pass;
+  int in_parts;          // EXPGATE, SSD: the kernel of chunk_parts.h
 };
 
 constexpr int TOK = 16, CP = 20;
@@ -612,16 +614,36 @@ __global__ __launch_bounds__(64 * NW, D <= 64 || (MODE == SSD && NW == 8) ? 4 : 
   }
 }
 
+}  // namespace chunk_scan
+
+#include "chunk_parts.h"
+
+namespace chunk_scan {
+
+// Scalar decays in chunks of thirty-two from twenty tokens to a request of the step on: below, most of its chunks would be empty places (us,
+// both, state-space layers of 16 heads of 128 x 64 and exponential gates of 64 x 128: 24 requests of 33 tokens 22.8 and 20.4, 21.7 and
+// 21.8, of 16 12.5 and 13.7, 12.6 and 15.1; 64 single tokens beside a piece of 40 37.4 and 35.2, 29.3 and 33.5).
+inline bool in_parts(int64_t tokens, int num_seqs) { return tokens >= 20 * (int64_t)num_seqs; }
+
 template <int MODE, typename T, int D, int NW>
 hipError_t launch_one(const Args& p, int num_seqs, int runs, hipStream_t s) {
-  constexpr size_t lds = lds_floats<D, NW>() * sizeof(float);
-  static_assert(lds <= 160 * 1024, "the chunk fits the LDS");
+  void (*kernel)(Args) = chunk_scan_kernel<MODE, T, D, NW>;
+  size_t lds = lds_floats<D, NW>() * sizeof(float);
+  static std::atomic<uint64_t> devices[2] = {{0}, {0}};
+  int form = 0;
+  if constexpr (MODE != GLA) {
+    if (p.in_parts) {
+      kernel = chunk_parts_kernel<MODE, T, D, NW>;
+      lds = PartsPlan<MODE, D, NW>::BYTES;
+      form = 1;
+    }
+  }
+  static_assert(lds_floats<D, NW>() * sizeof(float) <= 160 * 1024, "the chunk fits the LDS");
   if (lds > 64 * 1024) {
-    static std::atomic<uint64_t> devices{0};
-    const hipError_t e = allow_lds(reinterpret_cast<const void*>(&chunk_scan_kernel<MODE, T, D, NW>), lds, devices);
+    const hipError_t e = allow_lds(reinterpret_cast<const void*>(kernel), lds, devices[form]);
     if (e != hipSuccess) return e;
   }
-  chunk_scan_kernel<MODE, T, D, NW><<<dim3(p.H, num_seqs, runs), dim3(64 * NW), lds, s>>>(p);
+  kernel<<<dim3(p.H, num_seqs, runs), dim3(64 * NW), lds, s>>>(p);
   return hipGetLastError();
 }
 

@@ -671,6 +671,17 @@ extern "C" int nv_matrix_memory(const float* proj, int64_t proj_row_stride, int 
                                 int num_seqs, int heads, int dim, int vdim, int mode, int silu, float q_scale,
                                 float k_scale, const float* rot, int rot_dims, float cap, int max_q, int dtype,
                                 nv_stream_t stream) {
+  return nv_matrix_memory_batch(proj, proj_row_stride, q_off, k_off, v_off, i_off, f_off, bias, decay, state, cu_q, past_lens, state_slots,
+                                out, out_row_stride, 0, num_seqs, heads, dim, vdim, mode, silu, q_scale, k_scale, rot, rot_dims, cap, max_q,
+                                dtype, stream);
+}
+
+extern "C" int nv_matrix_memory_batch(const float* proj, int64_t proj_row_stride, int q_off, int k_off, int v_off, int i_off,
+                                      int f_off, const void* bias, const float* decay, float* state, const int32_t* cu_q,
+                                      const int32_t* past_lens, const int32_t* state_slots, float* out, int64_t out_row_stride,
+                                      int64_t tokens, int num_seqs, int heads, int dim, int vdim, int mode, int silu, float q_scale,
+                                      float k_scale, const float* rot, int rot_dims, float cap, int max_q, int dtype,
+                                      nv_stream_t stream) {
   NV_CHECK_ARG(proj && state && cu_q && past_lens && state_slots && out, "nv_matrix_memory: null pointer");
   NV_CHECK_ARG(dtype == NV_BF16 || dtype == NV_F32, "nv_matrix_memory: bad dtype %d", dtype);
   NV_CHECK_ARG(mode == MEM_CONST || mode == MEM_EXPGATE, "nv_matrix_memory: bad mode %d", mode);
@@ -718,7 +729,7 @@ extern "C" int nv_matrix_memory(const float* proj, int64_t proj_row_stride, int 
     }
     return NV_OK;
   }
-  // prompts in the gated form: sixteen tokens at a time (two tokens already cost the walk a whole staged chunk)
+  // prompts in the gated form: chunks of tokens (two tokens already cost the walk a whole staged chunk)
   if (mode == MEM_EXPGATE && max_q > 1 && !silu && rot_dims == 0 && getenv("NV_MATRIX_MEMORY_STEPS") == nullptr &&
       getenv("NV_MATRIX_MEMORY_GENERIC") == nullptr) {
     chunk_scan::Args c{};
@@ -745,6 +756,7 @@ extern "C" int nv_matrix_memory(const float* proj, int64_t proj_row_stride, int 
     c.q_scale = q_scale;
     c.k_scale = k_scale;
     c.c0 = cap;
+    c.in_parts = chunk_scan::in_parts(tokens, num_seqs);
     if (chunk_scan::serves(c)) {
       hipError_t e;
       NV_DISPATCH_T(dtype, e = chunk_scan::launch<chunk_scan::EXPGATE, T>(c, num_seqs, (hipStream_t)stream));

@@ -577,6 +577,15 @@ extern "C" int nv_ssd_scan(const float* xbc, int64_t xbc_row_stride, const float
                            const int32_t* cu_q, const int32_t* past_lens, const int32_t* state_slots, float* out,
                            int num_seqs, int heads, int groups, int state_size, int vdim, int max_q, void* workspace,
                            size_t workspace_bytes, int dtype, nv_stream_t stream) {
+  return nv_ssd_scan_batch(xbc, xbc_row_stride, z, z_row_stride, dt, dt_row_stride, dt_bias, A_log, D, state, cu_q, past_lens, state_slots,
+                           out, 0, num_seqs, heads, groups, state_size, vdim, max_q, workspace, workspace_bytes, dtype, stream);
+}
+
+extern "C" int nv_ssd_scan_batch(const float* xbc, int64_t xbc_row_stride, const float* z, int64_t z_row_stride, const float* dt,
+                                 int64_t dt_row_stride, const void* dt_bias, const void* A_log, const void* D, float* state,
+                                 const int32_t* cu_q, const int32_t* past_lens, const int32_t* state_slots, float* out, int64_t tokens,
+                                 int num_seqs, int heads, int groups, int state_size, int vdim, int max_q, void* workspace,
+                                 size_t workspace_bytes, int dtype, nv_stream_t stream) {
   NV_CHECK_ARG(xbc && z && dt && dt_bias && A_log && D && state && cu_q && past_lens && state_slots && out,
                "nv_ssd_scan: null pointer");
   NV_CHECK_ARG(dtype == NV_BF16 || dtype == NV_F32, "nv_ssd_scan: bad dtype %d", dtype);
@@ -633,6 +642,7 @@ extern "C" int nv_ssd_scan(const float* xbc, int64_t xbc_row_stride, const float
     c.ws_decay = decays(runs);
     c.runs = runs;
     c.run_len = run_len;
+    c.in_parts = chunk_scan::in_parts(tokens, num_seqs);
     if (chunk_scan::serves(c)) {
       hipError_t e;
       NV_DISPATCH_T(dtype, e = chunk_scan::launch_runs<chunk_scan::SSD, T>(c, num_seqs, (hipStream_t)stream));

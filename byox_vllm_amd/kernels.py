@@ -901,10 +901,10 @@ def matrix_memory(proj, offsets, state, cu_q, past_lens, state_slots, heads, dim
             dt = bias.dtype
     out = torch.empty(T, heads * vdim, dtype=torch.float32, device=proj.device) if out is None else out
     assert out.dtype == torch.float32 and out.stride(1) == 1 and out.size(0) == T and out.size(1) >= heads * vdim
-    check(lib().nv_matrix_memory(ptr(proj), proj.stride(0), q_off, k_off, v_off, i_off, f_off, ptr(bias), ptr(decay),
-                                 ptr(state), ptr(cu_q), ptr(past_lens), ptr(state_slots), ptr(out), out.stride(0), B, heads,
-                                 dim, vdim, mode, int(silu), q_scale, k_scale, ptr(rot), rot.size(1) if rot is not None else 0, cap,
-                                 int(max_q), _code32(dt), stream()), "nv_matrix_memory")
+    check(lib().nv_matrix_memory_batch(ptr(proj), proj.stride(0), q_off, k_off, v_off, i_off, f_off, ptr(bias), ptr(decay),
+                                       ptr(state), ptr(cu_q), ptr(past_lens), ptr(state_slots), ptr(out), out.stride(0), T, B, heads,
+                                       dim, vdim, mode, int(silu), q_scale, k_scale, ptr(rot), rot.size(1) if rot is not None else 0, cap,
+                                       int(max_q), _code32(dt), stream()), "nv_matrix_memory")
     return out
 
 
@@ -1444,9 +1444,9 @@ def ssd_scan(xbc, z, dt, dt_bias, A_log, D, state, cu_q, past_lens, state_slots,
     B = past_lens.numel()
     nbytes = lib().nv_ssd_scan_workspace_bytes(B, heads, state_size, vdim, max_q)
     ws = workspace(nbytes, xbc.device, "ssd_scan") if nbytes else None
-    check(lib().nv_ssd_scan(ptr(xbc), xbc.stride(0), ptr(z), z.stride(0), ptr(dt), dt.stride(0), ptr(dt_bias), ptr(A_log),
-                            ptr(D), ptr(state), ptr(cu_q), ptr(past_lens), ptr(state_slots), ptr(out), B,
-                            heads, groups, state_size, vdim, max_q, ptr(ws), nbytes, _code32(dt_bias.dtype), stream()),
+    check(lib().nv_ssd_scan_batch(ptr(xbc), xbc.stride(0), ptr(z), z.stride(0), ptr(dt), dt.stride(0), ptr(dt_bias), ptr(A_log),
+                                  ptr(D), ptr(state), ptr(cu_q), ptr(past_lens), ptr(state_slots), ptr(out), xbc.size(0), B,
+                                  heads, groups, state_size, vdim, max_q, ptr(ws), nbytes, _code32(dt_bias.dtype), stream()),
           "nv_ssd_scan")
     return out
 

@@ -497,6 +497,12 @@ int nv_matrix_memory(const float* proj, int64_t proj_row_stride, int q_off, int 
                      const int32_t* state_slots, float* out, int64_t out_row_stride, int num_seqs, int heads, int dim,
                      int vdim, int mode, int silu, float q_scale, float k_scale, const float* rot, int rot_dims, float cap,
                      int max_q, int dtype, nv_stream_t stream);
+/* nv_matrix_memory_batch: with the number of the step's tokens (0: unknown), by which it chooses between its forms for prompts. */
+int nv_matrix_memory_batch(const float* proj, int64_t proj_row_stride, int q_off, int k_off, int v_off, int i_off, int f_off,
+                     const void* bias, const float* decay, float* state, const int32_t* cu_q, const int32_t* past_lens,
+                     const int32_t* state_slots, float* out, int64_t out_row_stride, int64_t tokens, int num_seqs, int heads, int dim,
+                     int vdim, int mode, int silu, float q_scale, float k_scale, const float* rot, int rot_dims, float cap,
+                     int max_q, int dtype, nv_stream_t stream);
 /* Steps of one token per request in mode 0 with what follows per head, in one launch: o divided by its root mean square,
  * times sigmoid (gate_silu: SiLU) of the gate logits at columns g_off + h * vdim of proj, rows in the storage type.  Serves
  * what nv_retention_step_ok admits (value sizes of a multiple of 4, 16-byte aligned arrays). */
@@ -731,6 +737,12 @@ int nv_mingru_scan(const float* proj, int64_t proj_row_stride, int z_off, int u_
 int nv_ssd_scan(const float* xbc, int64_t xbc_row_stride, const float* z, int64_t z_row_stride, const float* dt,
                 int64_t dt_row_stride, const void* dt_bias, const void* A_log, const void* D, float* state,
                 const int32_t* cu_q, const int32_t* past_lens, const int32_t* state_slots, float* out, int num_seqs,
+                int heads, int groups, int state_size, int vdim, int max_q, void* workspace, size_t workspace_bytes,
+                int dtype, nv_stream_t stream);
+/* nv_ssd_scan_batch: with the number of the step's tokens (0: unknown), by which it chooses between its forms for prompts. */
+int nv_ssd_scan_batch(const float* xbc, int64_t xbc_row_stride, const float* z, int64_t z_row_stride, const float* dt,
+                int64_t dt_row_stride, const void* dt_bias, const void* A_log, const void* D, float* state,
+                const int32_t* cu_q, const int32_t* past_lens, const int32_t* state_slots, float* out, int64_t tokens, int num_seqs,
                 int heads, int groups, int state_size, int vdim, int max_q, void* workspace, size_t workspace_bytes,
                 int dtype, nv_stream_t stream);
 /* Bytes nv_ssd_scan needs when no request brings more than max_q tokens (0 for short steps: long prompts are cut into

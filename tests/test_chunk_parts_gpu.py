@@ -1,0 +1,113 @@
+"""Scalar decays in chunks of thirty-two tokens (csrc/chunk_parts.h), which the launches take where they know of twenty tokens and more to
+a request, against the chunks of sixteen, which they take where they know nothing; at the edges of both, and which steps go where."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+LENS = [1, 31, 32, 33, 63, 64, 65, 97]
+# fp32 products and sums of up to 128 terms in two orders, and exponentials of sums of 32 and of 16 log decays: twice that of one against
+# float64 (test_chunk_scan_gpu.py)
+TOL = 2 * 4 * (128 + 32) * 2.0 ** -24
+
+
+def i32(v):
+    return torch.tensor(v, dtype=torch.int32, device=DEV)
+
+
+def close(got, want, magnified=1.0):
+    got, want = got.double(), want.double()
+    off = ((got - want).abs() / torch.maximum(want.pow(2).mean().sqrt(), want.abs()) / magnified).max().item()
+    assert torch.isfinite(got).all() and off < TOL, off
+
+
+def both(run, lens, state):
+    """``run(tokens, state, ints)`` -> rows; without the number of tokens and with it."""
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    past = [0 if i % 3 else 7 for i in range(len(lens))]
+    ints = [i32(cu), i32(past), i32([len(lens) - 1 - i for i in range(len(lens))])]
+    results = []
+    for tokens in (0, cu[-1]):
+        s = state.clone()
+        results.append((run(tokens, s, ints), s))
+    return results
+
+
+@pytest.mark.parametrize("H,G,n,dv", [(4, 1, 128, 64), (4, 2, 64, 64), (2, 2, 16, 128), (2, 1, 20, 24), (3, 3, 4, 4), (2, 1, 100, 68),
+                                      (2, 1, 128, 128)])
+@pytest.mark.parametrize("lens", [LENS, [300, 257]])       # the last: runs side by side
+def test_state_space(H, G, n, dv, lens):
+    from byox_vllm_amd._C import check, lib, ptr, stream
+    from byox_vllm_amd.kernels import workspace
+    torch.manual_seed(n + dv)
+    T, inner = sum(lens), H * dv
+    xbc, z, dt = (torch.randn(T, c, device=DEV) for c in (inner + 2 * G * n, inner, H))
+    dt_bias, A_log, D = (torch.randn(H, device=DEV) for _ in range(3))
+    need = lib().nv_ssd_scan_workspace_bytes(len(lens), H, n, dv, max(lens))
+    ws = workspace(need, torch.device(DEV, 0), "ssd_scan") if need else None
+
+    def run(tokens, state, ints):
+        out = torch.empty(T, inner, device=DEV)
+        check(lib().nv_ssd_scan_batch(ptr(xbc), xbc.stride(0), ptr(z), z.stride(0), ptr(dt), dt.stride(0), ptr(dt_bias), ptr(A_log), ptr(D),
+                                      ptr(state), *map(ptr, ints), ptr(out), tokens, len(lens), H, G, n, dv, max(lens), ptr(ws), need, 2,
+                                      stream()), "nv_ssd_scan_batch")
+        return out
+    (rows, state), (rows_parts, state_parts) = both(run, lens, torch.randn(len(lens), H, n, dv, device=DEV))
+    close(rows_parts, rows)
+    close(state_parts, state)
+    assert not torch.equal(rows_parts, rows)       # two forms indeed
+
+
+@pytest.mark.parametrize("H,d,dv", [(2, 64, 128), (1, 128, 128), (3, 32, 64), (2, 20, 24), (1, 4, 4), (2, 100, 68), (1, 36, 128), (2, 64, 64)])
+@pytest.mark.parametrize("forget", [4.0, -30.0])
+def test_exponential_gates(H, d, dv, forget):
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd._C import check, lib, ptr, stream
+    torch.manual_seed(d + dv)
+    T, cols = sum(LENS), 2 * H * d + H * dv
+    proj = torch.randn(T, cols + 2 * H + (-(cols + 2 * H)) % 4, device=DEV)
+    proj[:, cols:] *= 3.0
+    bias = torch.zeros(cols + 2 * H, device=DEV)
+    bias[cols:cols + H], bias[cols + H:] = -1.0, forget
+    per_head = kernels.matrix_memory_state_size(kernels.MEM_EXPGATE, d, dv)
+    state = torch.randn(len(LENS), H, per_head, device=DEV)
+    slices = -(-dv // 64)
+    for c in range(1, slices):      # the normaliser and the maximum lie there once per slice of 64 columns
+        state[..., d * dv + c * (d + 1):d * dv + (c + 1) * (d + 1)] = state[..., d * dv:d * dv + d + 1]
+
+    def run(tokens, s, ints):
+        out = torch.empty(T, H * dv, device=DEV)
+        check(lib().nv_matrix_memory_batch(ptr(proj), proj.stride(0), 0, H * d, 2 * H * d, cols, cols + H, ptr(bias), None, ptr(s),
+                                           *map(ptr, ints), ptr(out), out.stride(0), tokens, len(LENS), H, d, dv, kernels.MEM_EXPGATE, 0,
+                                           d ** -0.5, 1.0, None, 0, 15.0, max(LENS), 2, stream()), "nv_matrix_memory_batch")
+        return out
+    (rows, end), (rows_parts, end_parts) = both(run, LENS, state)
+    # a row is divided by a sum n . q that may nearly cancel, which enlarges its errors: rows of like size
+    calm = (rows.abs() < 8.0).view(T, H, dv).all(-1, keepdim=True).expand(-1, -1, dv).reshape(T, -1)
+    assert calm.float().mean() > 0.5
+    close(torch.where(calm, rows_parts, 0.0), torch.where(calm, rows, 0.0), 16.0)
+    close(end_parts, end)
+    assert not torch.equal(rows_parts, rows)
+
+
+def test_the_line_between_them():
+    """Steps of 20 tokens to a request on average and more."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(1)
+    H, n, dv = 2, 64, 64
+    for lens, parts in (([20, 20], True), ([20, 19], False), ([59, 1], True), ([58, 1, 1], True), ([57, 1, 1], False)):
+        T, B = sum(lens), len(lens)
+        cu = [0]
+        for m in lens:
+            cu.append(cu[-1] + m)
+        data = [torch.randn(s, device=DEV) for s in ((T, H * dv + 2 * n), (T, H * dv), (T, H), (H,), (H,), (H,))]
+        state, ints = torch.randn(B, H, n, dv, device=DEV), (i32(cu), i32([3] * B), i32(list(range(B))))
+        got = kernels.ssd_scan(*data, state.clone(), *ints, H, 1, n, dv, max_q=max(lens))
+        from byox_vllm_amd._C import check, lib, ptr, stream
+        sixteen, s = torch.empty_like(got), state.clone()
+        check(lib().nv_ssd_scan(*(a for x in data[:3] for a in (ptr(x), x.stride(0))), *map(ptr, data[3:]), ptr(s), *map(ptr, ints),
+                                ptr(sixteen), B, H, 1, n, dv, max(lens), None, 0, 2, stream()), "nv_ssd_scan")
+        assert torch.equal(got, sixteen) != parts, lens
