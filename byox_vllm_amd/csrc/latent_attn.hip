@@ -179,6 +179,60 @@ __global__ __launch_bounds__(256) void latent_q_rope_kernel(const T* __restrict_
   }
 }
 
+// Whole query rows in fours, up to QT tokens to a workgroup: all of their cosines and sines into LDS by as many lanes at once, then four numbers to a
+// lane, whose partners of the rotation are four others half a turn on or, interleaved, among them.  Rows, heads and both halves split into fours.
+// What bounded one token to a workgroup: a wavefront's cosines ahead of everybody's barrier, single numbers with two divisions each.
+// 11013 tokens of 16 heads of 96 + 32, bf16 into bf16, 27.3 us there, 19.8 here (4.6 TB/s), 16384 of 4 heads 17.7 and 11.6, 100 of 16 3.7 and 3.2.
+// One token to a workgroup up to 2048 (300 tokens 3.6, 4.0 with two, 5.7 with four; 2000 5.8, 6.2, 7.5), then two (3000 7.6, 7.3, 8.4; 11013 21.8,
+// 19.8, 20.1), or four where a row has fours for half of the lanes at most (4 heads, 16384 tokens 16.8, 13.0, 11.6).
+constexpr int QT = 4;
+template <typename T, typename TO>
+__global__ __launch_bounds__(256) void latent_q_rows_kernel(const T* __restrict__ q, int64_t q_rs, const int64_t* __restrict__ positions,
+                                                            const float* __restrict__ inv_freq, float mscale, TO* __restrict__ out, int tokens, int per,
+                                                            int H, int dim, int rot_dim, int rot_dims, int interleaved, float factor) {
+  __shared__ float2 turn[QT * TURNS];
+  const int t0 = blockIdx.x * per, n = min(per, tokens - t0), half = rot_dims / 2, row4 = (dim + rot_dim) / 4, step_h = 256 / row4,
+            step_r = 256 % row4;
+  for (int i = threadIdx.x; i < n * half; i += 256) {
+    const int t = i / half;
+    const float a = (float)positions[t0 + t] * inv_freq[i - t * half];
+    turn[i] = make_float2(cosf(a) * mscale, sinf(a) * mscale);
+  }
+  __syncthreads();
+  for (int t = 0; t < n; ++t) {
+    const T* from = q + (int64_t)(t0 + t) * q_rs;
+    TO* to = out + (int64_t)(t0 + t) * H * (4 * row4);
+    const float2* by = turn + t * half;
+    int h = threadIdx.x / row4, r = threadIdx.x % row4;
+    for (; h < H; h += step_h, r += step_r) {
+      if (r >= row4) {
+        r -= row4;
+        if (++h >= H) break;
+      }
+      const int j = 4 * r - dim;           // place in the rotated part
+      const T* src = from + h * (4 * row4) + 4 * r;
+      f32x4 v = Pack4<T>::widen(*reinterpret_cast<const typename Pack4<T>::type*>(src));
+      if (j >= 0 && j < rot_dims) {
+        if (interleaved) {
+          const float2 a = by[j / 2], b = by[j / 2 + 1];
+          v = f32x4{v[0] * a.x - v[1] * a.y, v[1] * a.x + v[0] * a.y, v[2] * b.x - v[3] * b.y, v[3] * b.x + v[2] * b.y};
+        } else {
+          const bool first = j < half;
+          const f32x4 o = Pack4<T>::widen(*reinterpret_cast<const typename Pack4<T>::type*>(first ? src + half : src - half));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float2 a = by[(first ? j : j - half) + e];
+            v[e] = first ? v[e] * a.x - o[e] * a.y : v[e] * a.x + o[e] * a.y;
+          }
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] *= factor;
+      *reinterpret_cast<typename Pack4<TO>::type*>(to + h * (4 * row4) + 4 * r) = Pack4<TO>::narrow(v);
+    }
+  }
+}
+
 // The cache rows of every request of a step, in order of position, into one buffer: request b's row j goes to row
 // cu_k[b] + j (cu_k: starts padded to whole blocks; rows past the request's end are zero).
 template <typename T>
@@ -659,6 +713,21 @@ extern "C" int nv_latent_q_rows_as(const void* q, int64_t q_row_stride, const in
   if (tokens == 0 || (rot_dim == 0 && !copy_front)) return NV_OK;
   const int quads = dim % 4 == 0 && rot_dim % 4 == 0 && q_row_stride % 4 == 0 && (uintptr_t)qa % 16 == 0 &&
                     (uintptr_t)q % (dtype == NV_BF16 ? 8 : 16) == 0;
+  // whole rows whose rotation is in fours as well
+  if (quads && copy_front && rot_dims % (interleaved ? 4 : 8) == 0 && rot_dims <= 2 * TURNS && tokens < (1 << 30)) {
+    const int per = tokens <= 2048 ? 1 : heads * (dim + rot_dim) <= 512 ? QT : 2;
+    const dim3 g((unsigned)((tokens + per - 1) / per));
+    if (qa_dtype == NV_F32)
+      NV_DISPATCH_T(dtype, latent_q_rows_kernel<T, float><<<g, dim3(256), 0, (hipStream_t)stream>>>(
+                               (const T*)q, q_row_stride, positions, inv_freq, mscale, (float*)qa, (int)tokens, per, heads, dim, rot_dim, rot_dims,
+                               interleaved, factor));
+    else
+      NV_DISPATCH_T(dtype, latent_q_rows_kernel<T, bf16_t><<<g, dim3(256), 0, (hipStream_t)stream>>>(
+                               (const T*)q, q_row_stride, positions, inv_freq, mscale, (bf16_t*)qa, (int)tokens, per, heads, dim, rot_dim, rot_dims,
+                               interleaved, factor));
+    NV_CHECK_LAUNCH();
+    return NV_OK;
+  }
   if (qa_dtype == NV_F32)
     NV_DISPATCH_T(dtype, latent_q_rope_kernel<T, float><<<dim3((unsigned)tokens), dim3(256), 0, (hipStream_t)stream>>>(
                              (const T*)q, q_row_stride, positions, inv_freq, mscale, (float*)qa, heads, dim, rot_dim, rot_dims, rank,
