@@ -82,18 +82,13 @@ struct KvRows {
   int interleaved;
 };
 
+// ... a token's rotated part, by `threads` threads
 template <typename T>
-__device__ __forceinline__ void latent_kv_store(const KvRows& p, bool quads, float* red) {
-  const int64_t t = blockIdx.x;
-  const int32_t slot = p.slots[t];
-  const float* row = p.kv + t * p.rs;
+__device__ __forceinline__ void latent_rot_store(const KvRows& p, int64_t t, const float* row, T* dst, int thread, int threads) {
   const int rank = p.rank, rot_dims = p.rot_dims;
-  T* dst = reinterpret_cast<T*>(p.cache) + (int64_t)(slot < 0 ? 0 : slot) * (rank + p.rot_dim);
-  norm_row<T>(row, reinterpret_cast<const T*>(p.w), dst, rank, p.eps, quads, slot >= 0, red);
-  if (slot < 0) return;
   const float pos = (float)p.positions[t];
   const int half = rot_dims / 2;
-  for (int j = threadIdx.x; j < p.rot_dim; j += blockDim.x) {
+  for (int j = thread; j < p.rot_dim; j += threads) {
     float v = row[rank + j];
     if (j < rot_dims) {
       const bool first = p.interleaved ? (j & 1) == 0 : j < half;
@@ -105,6 +100,16 @@ __device__ __forceinline__ void latent_kv_store(const KvRows& p, bool quads, flo
     }
     st_f32<T>(dst + rank + j, v);
   }
+}
+
+template <typename T>
+__device__ __forceinline__ void latent_kv_store(const KvRows& p, bool quads, float* red) {
+  const int64_t t = blockIdx.x;
+  const int32_t slot = p.slots[t];
+  const float* row = p.kv + t * p.rs;
+  T* dst = reinterpret_cast<T*>(p.cache) + (int64_t)(slot < 0 ? 0 : slot) * (p.rank + p.rot_dim);
+  norm_row<T>(row, reinterpret_cast<const T*>(p.w), dst, p.rank, p.eps, quads, slot >= 0, red);
+  if (slot >= 0) latent_rot_store<T>(p, t, row, dst, threadIdx.x, blockDim.x);
 }
 
 template <typename T, bool QUADS>
@@ -177,6 +182,48 @@ __global__ __launch_bounds__(256) void latent_q_rope_kernel(const T* __restrict_
     }
     st_f32<TO>(qa + (t * H + h) * (rank + rot_dim) + rank + j, v * factor);
   }
+}
+
+// Both norms, a wavefront to a row of fours of at most 1024 numbers.  In latent_norms_kernel rows of less than 1024 leave wavefronts idle that
+// wait at two barriers all the same: 11013 tokens of 768 and 512 + 32 numbers, bf16, 26.3 us there, 17.5 here (5.0 TB/s), of 256 and 128 + 32
+// 22.4 and 9.5, 1024 tokens 4.2 and 3.9, 8 tokens 3.4 and 3.3.
+template <typename T>
+__global__ __launch_bounds__(256) void latent_norm_rows_kernel(KvRows p, NormRows q, int64_t tokens) {
+  typedef typename Pack4<T>::type P;
+  const int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (t >= tokens) return;
+  const int lane = threadIdx.x & 63, n = blockIdx.y ? q.n : p.rank, slot = blockIdx.y ? 0 : p.slots[t];
+  if (slot < 0) return;
+  const float* x = blockIdx.y ? q.x + t * q.rs : p.kv + t * p.rs;
+  const T* w = reinterpret_cast<const T*>(blockIdx.y ? q.w : p.w);
+  T* out = blockIdx.y ? reinterpret_cast<T*>(q.out) + t * n : reinterpret_cast<T*>(p.cache) + (int64_t)slot * (n + p.rot_dim);
+  f32x4 v[4];
+  P f[4];
+  float ss = 0.0f;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int j = 4 * (lane + 64 * k);
+    v[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (j < n) {
+      v[k] = *reinterpret_cast<const f32x4*>(x + j);
+      f[k] = *reinterpret_cast<const P*>(w + j);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) ss += v[k][r] * v[k][r];
+  const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)n + p.eps);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int j = 4 * (lane + 64 * k);
+    if (j >= n) continue;
+    const f32x4 g = Pack4<T>::widen(f[k]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[k][r] = v[k][r] * inv * g[r];
+    *reinterpret_cast<P*>(out + j) = Pack4<T>::narrow(v[k]);
+  }
+  if (!blockIdx.y) latent_rot_store<T>(p, t, x, out, lane, 64);
 }
 
 // Whole query rows in fours, up to QT tokens to a workgroup: all of their cosines and sines into LDS by as many lanes at once, then four numbers to a
@@ -680,7 +727,9 @@ extern "C" int nv_latent_norms(const float* kv, int64_t kv_row_stride, const voi
   const dim3 grid((unsigned)tokens, q ? 2 : 1);
   hipStream_t s = (hipStream_t)stream;
   // alone, fours pay from 512 numbers on (16000 tokens of 64: 16.7 us in fours, 13.9 one at a time; of 512: 21.1 and 25.4)
-  if (q) NV_DISPATCH_T(dtype, latent_norms_kernel<T><<<grid, dim3(256), 0, s>>>(p, kv_quads, rows));
+  if (q && kv_quads && rows.quads && rank <= 1024 && q_rank <= 1024)
+    NV_DISPATCH_T(dtype, latent_norm_rows_kernel<T><<<dim3((unsigned)((tokens + 3) / 4), 2), dim3(256), 0, s>>>(p, rows, tokens));
+  else if (q) NV_DISPATCH_T(dtype, latent_norms_kernel<T><<<grid, dim3(256), 0, s>>>(p, kv_quads, rows));
   else if (kv_quads && rank >= 512) NV_DISPATCH_T(dtype, latent_kv_store_kernel<T, true><<<grid, dim3(256), 0, s>>>(p));
   else NV_DISPATCH_T(dtype, latent_kv_store_kernel<T, false><<<grid, dim3(256), 0, s>>>(p));
   NV_CHECK_LAUNCH();

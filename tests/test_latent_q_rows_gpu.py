@@ -1,4 +1,4 @@
-"""Whole query rows of latent attention (csrc/latent_attn.hip, latent_q_rows_kernel) against float64: one, two and four tokens to a workgroup, last
+"""Query rows and norms of latent attention (csrc/latent_attn.hip) against float64.  Whole query rows: one, two and four tokens to a workgroup, last
 workgroups with fewer, rows shorter and longer than a workgroup's lanes, rotations that end inside the rotated part."""
 
 import pytest
@@ -29,3 +29,36 @@ def test_rows(T, H, d, r, rot, interleaved, dtype, out_dtype):
     assert got.dtype == out_dtype
     # cosines within 2 units of 2^-24, two products and their sum of numbers below 6; then one rounding of the result
     assert ((got.double().cpu() - want).abs() <= 2.0 ** -20 + (2.0 ** -8 * want.abs() if out_dtype == torch.bfloat16 else 0.0)).all()
+
+
+@pytest.mark.parametrize("T", [1, 3, 9])
+@pytest.mark.parametrize("q_rank,rank,r", [(4, 8, 8), (256, 260, 16), (260, 256, 0), (1024, 1020, 64), (1028, 512, 32), (768, 1028, 32)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_both_norms(T, q_rank, rank, r, dtype):
+    """A wavefront to a row, and (more than 1024 numbers) a workgroup to a row; one token has no place in the cache."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(T + rank)
+    x = torch.randn(T, q_rank + rank + r + 4) * 2.0
+    qw, w, positions = torch.randn(q_rank).to(dtype), torch.randn(rank).to(dtype), torch.randint(0, 100, (T,))
+    freq = 10000.0 ** (-torch.arange(0, max(r, 2), 2).float() / max(r, 2))
+    slots = [T + 1 - i for i in range(T)]
+    slots[T // 2] = -1
+    cache = torch.full((T + 2, rank + r), 7.0, dtype=dtype, device=DEV)
+    d = x.to(DEV)
+    got = kernels.latent_kv_store(d[:, q_rank:q_rank + rank + r], w.to(DEV), positions.to(DEV), freq.to(DEV), 1.0,
+                                  torch.tensor(slots, dtype=torch.int32, device=DEV), cache, rank, r, r, 1e-5, False, q=d[:, :q_rank],
+                                  q_norm_w=qw.to(DEV))
+    def norm(v, f):
+        return v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + 1e-5) * f.double()
+    a, b = x[:, q_rank + rank:q_rank + rank + r].double().chunk(2, -1)
+    angle = (positions.float()[:, None] * freq[:r // 2]).double()
+    turned = torch.cat([a * angle.cos() - b * angle.sin(), b * angle.cos() + a * angle.sin()], -1)
+    want = torch.full((T + 2, rank + r), 7.0, dtype=torch.float64)
+    rows = torch.cat([norm(x[:, q_rank:q_rank + rank].double(), w), turned], -1)
+    for i, s in enumerate(slots):
+        if s >= 0:
+            want[s] = rows[i]
+    for have, should in ((got, norm(x[:, :q_rank].double(), qw)), (cache, want)):
+        # a sum of squares of 1028 numbers (its error halved by the root), root, quotient and two products; then one rounding
+        bound = (1028 / 64 + 8) * 2.0 ** -24 * should.abs() + 2.0 ** -20 + (2.0 ** -8 * should.abs() if dtype == torch.bfloat16 else 0.0)
+        assert ((have.double().cpu() - should).abs() <= bound).all()
