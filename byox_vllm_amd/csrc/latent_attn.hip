@@ -281,27 +281,34 @@ __global__ __launch_bounds__(256) void latent_q_rows_kernel(const T* __restrict_
 }
 
 // The cache rows of every request of a step, in order of position, into one buffer: request b's row j goes to row
-// cu_k[b] + j (cu_k: starts padded to whole blocks; rows past the request's end are zero).
-template <typename T>
-__global__ __launch_bounds__(256) void latent_gather_kernel(const T* __restrict__ cache, const int32_t* __restrict__ tables,
+// cu_k[b] + j (cu_k: starts padded to whole blocks; rows past the request's end are zero).  U: what a lane moves at once, a number or 16 bytes
+// (rows that split into them).  What bounded it: a row's request, looked for in one start after the other; now 64 starts at once.
+// Pages of 256 and 544 numbers of bf16: 128 requests of 100 tokens (288 numbers) 78 and 8.8 us, 64 of 200 25.6 and 7.3, 8 of 1500 8.3 and 6.3.
+template <typename U>
+__global__ __launch_bounds__(256) void latent_gather_kernel(const U* __restrict__ cache, const int32_t* __restrict__ tables,
                                                             int table_cols, const int32_t* __restrict__ cu_k,
                                                             const int32_t* __restrict__ cu_q,
                                                             const int32_t* __restrict__ past, int B, int block_size,
-                                                            int Dk, T* __restrict__ out) {
+                                                            int width, U* __restrict__ out) {
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= cu_k[B]) return;
   const int lane = threadIdx.x & 63;
-  int b = 0;
-  while (b + 1 < B && row >= cu_k[b + 1]) ++b;
+  int b = 0;                     // the starts behind the first that are not past the row
+  for (int i = 0; i < B - 1; i += 64) {
+    const uint64_t m = __ballot(i + lane < B - 1 && row >= cu_k[min(i + lane, B - 2) + 1]);
+    b += __popcll(m);
+    if (~m != 0) break;
+  }
+  b = __builtin_amdgcn_readfirstlane(b);
   const int j = (int)(row - cu_k[b]);
   const int len = past[b] + cu_q[b + 1] - cu_q[b];
-  T* dst = out + row * Dk;
+  U* dst = out + row * width;
   if (j >= len) {
-    for (int e = lane; e < Dk; e += 64) dst[e] = (T)0.0f;
+    for (int e = lane; e < width; e += 64) dst[e] = U{};
     return;
   }
-  const T* src = cache + ((int64_t)tables[(int64_t)b * table_cols + j / block_size] * block_size + j % block_size) * Dk;
-  for (int e = lane; e < Dk; e += 64) dst[e] = src[e];
+  const U* src = cache + ((int64_t)tables[(int64_t)b * table_cols + j / block_size] * block_size + j % block_size) * width;
+  for (int e = lane; e < width; e += 64) dst[e] = src[e];
 }
 
 // Expanded key/value rows [k: H * (dim + rot_dim) | v: H * vdim] from the up-projections kv [rows, H * dim | H * vdim]
@@ -911,9 +918,15 @@ extern "C" int nv_latent_gather(const void* cache, const int32_t* block_tables, 
   NV_CHECK_ARG(dtype == NV_BF16 || dtype == NV_F32, "nv_latent_gather: bad dtype %d", dtype);
   NV_CHECK_ARG(num_seqs > 0 && block_size > 0 && row_width > 0 && rows >= 0 && table_cols > 0, "nv_latent_gather: bad shape");
   if (rows == 0) return NV_OK;
-  NV_DISPATCH_T(dtype, latent_gather_kernel<T><<<dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, (hipStream_t)stream>>>(
-                           (const T*)cache, block_tables, table_cols, cu_k, cu_q, past_lens, num_seqs, block_size,
-                           row_width, (T*)out));
+  const dim3 g((unsigned)((rows + 3) / 4));
+  const int bytes = row_width * (dtype == NV_BF16 ? 2 : 4);
+  if (bytes % 16 == 0 && ((uintptr_t)cache | (uintptr_t)out) % 16 == 0)
+    latent_gather_kernel<u32x4><<<g, dim3(256), 0, (hipStream_t)stream>>>((const u32x4*)cache, block_tables, table_cols, cu_k, cu_q, past_lens,
+                                                                          num_seqs, block_size, bytes / 16, (u32x4*)out);
+  else
+    NV_DISPATCH_T(dtype, latent_gather_kernel<T><<<g, dim3(256), 0, (hipStream_t)stream>>>(
+                             (const T*)cache, block_tables, table_cols, cu_k, cu_q, past_lens, num_seqs, block_size,
+                             row_width, (T*)out));
   NV_CHECK_LAUNCH();
   return NV_OK;
 }

@@ -62,3 +62,33 @@ def test_both_norms(T, q_rank, rank, r, dtype):
         # a sum of squares of 1028 numbers (its error halved by the root), root, quotient and two products; then one rounding
         bound = (1028 / 64 + 8) * 2.0 ** -24 * should.abs() + 2.0 ** -20 + (2.0 ** -8 * should.abs() if dtype == torch.bfloat16 else 0.0)
         assert ((have.double().cpu() - should).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("B", [1, 2, 64, 65, 66, 131])
+@pytest.mark.parametrize("width,dtype", [(24, torch.bfloat16), (544, torch.bfloat16), (20, torch.bfloat16), (12, torch.float32), (7, torch.float32)])
+def test_rows_gathered_from_pages(B, width, dtype):
+    """Requests found 64 starts at a time, some without tokens; rows in pieces of 16 bytes and in single numbers."""
+    from byox_vllm_amd._C import check, dtype_code, lib, ptr, stream
+    torch.manual_seed(B + width)
+    block = 16
+    past, new = torch.randint(0, 40, (B,)).tolist(), torch.randint(0, 30, (B,)).tolist()
+    past[0], new[0] = 3, 2
+    if B > 1:
+        past[1] = new[1] = 0
+    pages = [-(-(a + b) // block) for a, b in zip(past, new)]
+    order = torch.randperm(sum(pages)).tolist()
+    tables, cu_k, cu_q = torch.zeros(B, max(pages), dtype=torch.int32), [0], [0]
+    cache = torch.randn(sum(pages) * block, width).to(dtype)
+    want = torch.zeros(sum(pages) * block, width, dtype=dtype)
+    for b in range(B):
+        for i in range(pages[b]):
+            tables[b, i] = p = order.pop()
+            filled = min(block, past[b] + new[b] - i * block)
+            want[cu_k[b] + i * block:cu_k[b] + i * block + filled] = cache[p * block:p * block + filled]
+        cu_k.append(cu_k[-1] + pages[b] * block)
+        cu_q.append(cu_q[-1] + new[b])
+    out = torch.full_like(want, 9.0).to(DEV)
+    args = [t.to(DEV) for t in (cache, tables, *(torch.tensor(v, dtype=torch.int32) for v in (cu_k, cu_q, past)))]
+    check(lib().nv_latent_gather(ptr(args[0]), ptr(args[1]), tables.size(1), *map(ptr, args[2:]), B, block, width, ptr(out), cu_k[-1],
+                                 dtype_code(dtype, allow_f32=True), stream()), "nv_latent_gather")
+    assert torch.equal(out.cpu(), want)
