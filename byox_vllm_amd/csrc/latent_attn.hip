@@ -186,7 +186,7 @@ __global__ __launch_bounds__(256) void latent_q_rope_kernel(const T* __restrict_
 
 // Both norms, a wavefront to a row of fours of at most 1024 numbers.  In latent_norms_kernel rows of less than 1024 leave wavefronts idle that
 // wait at two barriers all the same: 11013 tokens of 768 and 512 + 32 numbers, bf16, 26.3 us there, 17.5 here (5.0 TB/s), of 256 and 128 + 32
-// 22.4 and 9.5, 1024 tokens 4.2 and 3.9, 8 tokens 3.4 and 3.3.
+// 22.4 and 8.7, 1024 tokens 4.2 and 3.8, 8 tokens 3.4 and 3.3.
 template <typename T>
 __global__ __launch_bounds__(256) void latent_norm_rows_kernel(KvRows p, NormRows q, int64_t tokens) {
   typedef typename Pack4<T>::type P;
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(256) void latent_norm_rows_kernel(KvRows p, NormRow
   T* out = blockIdx.y ? reinterpret_cast<T*>(q.out) + t * n : reinterpret_cast<T*>(p.cache) + (int64_t)slot * (n + p.rot_dim);
   f32x4 v[4];
   P f[4];
-  float ss = 0.0f;
+  float ss;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const int j = 4 * (lane + 64 * k);
@@ -209,11 +209,24 @@ __global__ __launch_bounds__(256) void latent_norm_rows_kernel(KvRows p, NormRow
       f[k] = *reinterpret_cast<const P*>(w + j);
     }
   }
+  // The squares of 256 numbers at a time, as norm_row adds them: the same numbers from either.  wave_sum's pairs without the LDS crossbar,
+  // through which four such sums took 0.2 - 0.5 us.
+  auto squares = [&](int k) {
+    float x = 0.0f, a, b;
 #pragma unroll
-  for (int k = 0; k < 4; ++k)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) ss += v[k][r] * v[k][r];
-  const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)n + p.eps);
+    for (int r = 0; r < 4; ++r) x += v[k][r] * v[k][r];
+    rows_pair32(x, a, b);
+    rows_pair16(a + b, a, b);
+    x = a + b;
+    x += dpp_f32<0x128>(x);          // row_ror 8, 4, 2, 1
+    x += dpp_f32<0x124>(x);
+    x += dpp_f32<0x122>(x);
+    x += dpp_f32<0x121>(x);
+    return x;
+  };
+  ss = squares(0);
+  if (n > 256) ss = ss + squares(1) + squares(2) + squares(3);
+  const float inv = 1.0f / sqrtf(ss / (float)n + p.eps);
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const int j = 4 * (lane + 64 * k);

@@ -64,6 +64,21 @@ def test_both_norms(T, q_rank, rank, r, dtype):
         assert ((have.double().cpu() - should).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("rank", [512, 516, 768, 1020, 1024])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_norms_add_their_squares_in_one_order(rank, dtype):
+    """A row's norm is the same number whether a wavefront takes it (beside the query's) or a workgroup (alone): to the last bit."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(rank)
+    T, r = 301, 32
+    x, w = (torch.randn(T, rank + r) * 2.0).to(DEV), torch.randn(rank).to(dtype).to(DEV)
+    rest = (torch.arange(T).to(DEV), torch.rand(r // 2).to(DEV), 1.0, torch.arange(T, dtype=torch.int32).to(DEV))
+    alone, beside = (torch.empty(T, rank + r, dtype=dtype, device=DEV) for _ in range(2))
+    kernels.latent_kv_store(x, w, *rest, alone, rank, r, r, 1e-5)
+    got = kernels.latent_kv_store(x, w, *rest, beside, rank, r, r, 1e-5, q=x[:, :rank], q_norm_w=w)
+    assert torch.equal(beside, alone) and torch.equal(got, alone[:, :rank])
+
+
 @pytest.mark.parametrize("B", [1, 2, 64, 65, 66, 131])
 @pytest.mark.parametrize("width,dtype", [(24, torch.bfloat16), (544, torch.bfloat16), (20, torch.bfloat16), (12, torch.float32), (7, torch.float32)])
 def test_rows_gathered_from_pages(B, width, dtype):
