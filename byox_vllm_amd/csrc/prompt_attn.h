@@ -215,14 +215,16 @@ __global__ __launch_bounds__(256, D == 64 && EXT ? 3 : 2) void prompt_attn_kerne
     // to the last key of its last.  Kept keys that fit the places ahead of that first key lie there instead of in a tile of their own.
     auto first_of = [&](int at) { return max(p.window > 0 ? at - p.window + 1 : 0, EXT && p.chunk > 0 ? at / p.chunk * p.chunk : 0); };
     const int low = first_of(pos), hi = p0 + nq - 1, wlow_lo = first_of(wpos_lo), wlow_hi = first_of(wpos_hi);
-    const int kept_keys = EXT ? min(p.keep, first_of(p0)) : 0;
-    const int merged = EXT && first_of(p0) >= PA_KEYS && kept_keys <= first_of(p0) % PA_KEYS ? kept_keys : 0;
+    const int first_key = first_of(p0), kept_keys = EXT ? min(p.keep, first_key) : 0;
+    const int merged = EXT && first_key >= PA_KEYS && kept_keys <= first_key % PA_KEYS ? kept_keys : 0;
     const int kept_tiles = merged > 0 ? 0 : (kept_keys + PA_KEYS - 1) / PA_KEYS;
-    const int skipped = max(first_of(p0) / PA_KEYS - kept_tiles, 0), count = hi / PA_KEYS + 1 - skipped;
+    const int skipped = max(first_key / PA_KEYS - kept_tiles, 0), count = hi / PA_KEYS + 1 - skipped;
     auto tile_key = [&](int it) { return PA_KEYS * (it < kept_tiles ? it : it + skipped); };
     // Where its rows are.  Blocks of a multiple of 64 hold whole tiles: one page number for all lanes, asked for a tile ahead (as a vector
     // load: what waits for a scalar one waits for all reads of LDS too), and every lane's place in a tile is the same each time.  Else every
-    // lane looks its rows up.  Places past the last key repeat it: they are masked, and what nobody has written there may be a NaN.
+    // lane looks its rows up.  Places past the last key repeat it: they are masked, and what nobody has written there may be a NaN.  Places
+    // between the kept keys and the first key of the tile's first row, masked as well, repeat that key: their blocks may be anybody's by now,
+    // and their entries of the table are not read (with whole tiles in a block, the entry is that of a key that is seen).
     int page[NI], in_page[NI], no_lane;
     asm volatile("v_mov_b32 %0, 0" : "=v"(no_lane));
     auto look_up = [&](int it) {
@@ -233,7 +235,7 @@ __global__ __launch_bounds__(256, D == 64 && EXT ? 3 : 2) void prompt_attn_kerne
       } else {
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
-          const int r = row_of(i), kp = EXT && it == 0 && r < merged ? r : min(j0 + r, hi);
+          const int r = row_of(i), key = min(j0 + r, hi), kp = EXT && it == 0 && r < merged ? r : key < kept_keys ? key : max(key, first_key);
           const int n = bs_shift >= 0 ? kp >> bs_shift : kp / p.block_size;
           in_page[i] = kp - n * p.block_size;
           page[i] = table[n];

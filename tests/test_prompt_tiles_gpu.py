@@ -70,3 +70,38 @@ def test_queries_in_16_bits_are_refused_elsewhere():
         with pytest.raises(RuntimeError, match="does not take queries"):
             kernels.paged_softmax_attn(torch.zeros(3, 64, dtype=torch.bfloat16, device=DEV), *args, max_q, 1, 1, 64, 64, 256,
                                        torch.empty(3, 64, dtype=torch.bfloat16, device=DEV), **options)
+
+
+@pytest.mark.parametrize("block", [16, 32, 48, 64, 80, 128])
+@pytest.mark.parametrize("D,R", [(64, 1), (64, 4), (128, 2)])
+@pytest.mark.parametrize("window,keep,chunk", [(64, 0, 0), (100, 1, 0), (65, 63, 0), (90, 64, 0), (70, 130, 0), (33, 16, 0), (0, 0, 100)])
+def test_entries_of_the_table_that_nobody_sees_are_not_read(D, R, window, keep, chunk, block):
+    """Blocks without a kept key and without one from the first new token's window on may have been given away: their entries are -1, and
+    the page ahead of the cache, which such an entry stands for, holds NaNs that a read would carry into the results."""
+    from byox_vllm_amd import kernels
+    torch.manual_seed(window + keep + chunk + D)
+    new, past, G = [130, 1, 70, 200], [0, 511, 301, 64 * 5 + 33], 2
+    H, pages, T = R * G, [-(-(a + b) // block) for a, b in zip(new, past)], sum(new)
+    held = torch.full(((sum(pages) + 1) * block, 2 * G * D), float("nan"), dtype=torch.bfloat16)
+    cache = held[block:]
+    cache[:] = torch.randn(cache.shape)
+    order, tables, left = torch.randperm(sum(pages)).tolist(), [], []
+    for n, before in zip(pages, past):
+        tables.append([order.pop() for _ in range(n)])
+        first = max(before - window + 1 if window else 0, before // chunk * chunk if chunk else 0, 0)
+        left.append([page if (i + 1) * block > first or i * block < keep else -1 for i, page in enumerate(tables[-1])])
+    assert any(-1 in t for t in left)
+    cu = [0]
+    for n in new:
+        cu.append(cu[-1] + n)
+    q = (torch.randn(T, H * D) * 2.0 * D ** -0.5).to(DEV)
+    rows = held.to(DEV)[block:]
+    results = []
+    for shown in (tables, left):
+        out = torch.empty(T, H * D, dtype=torch.bfloat16, device=DEV)
+        kernels.paged_softmax_attn(q, rows, i32([t + [-1] * (max(pages) - len(t)) for t in shown]), i32(cu), i32(past),
+                                   i32([b for b, n in enumerate(new) for _ in range(n)]), max(new), H, G, D, D, block, out,
+                                   window=window, keep_first=keep, chunk=chunk)
+        results.append(out)
+    assert torch.isfinite(results[0]).all()
+    assert torch.equal(*results)
