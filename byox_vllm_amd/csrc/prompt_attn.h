@@ -112,10 +112,10 @@ __device__ __forceinline__ void prompt_rows_again(const WAttnArgs& a, uint32_t r
 // 16 bytes to a lane into LDS at `dst` + 16 * lane.  Not the builtin: the compiler waits for every DMA under way ahead of a transposing
 // read, for the next tile's too; what has to be waited for is said at the tile's beginning.
 __device__ __forceinline__ void pa_dma(const void* src, uint32_t dst) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src) : "memory", "m0");
 }
 __device__ __forceinline__ void pa_dma(const void* base, uint32_t off, uint32_t dst) {      // one base for the wavefront
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(off), "s"(base) : "memory", "m0");
 }
 
 // WHOLE: blocks of a multiple of 64 hold whole tiles (and rows of less than 32 MB, so that a place in a tile is 32 bits)
