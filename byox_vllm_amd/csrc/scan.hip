@@ -37,7 +37,7 @@ struct ConvArgs {
   void* out_t;            // [tokens, ot_rs] in the storage type, or null
   int64_t ot_rs;
   int C, taps, act;       // act 0: none, 1: SiLU, 2: none, and the token's own input is added to the result
-  int heads_only;         // 1: blockIdx.x counts requests; only the tokens that reach back over a portion's start are served
+  int heads_only;         // 1: blockIdx.x counts requests, whose tokens a workgroup serves one after the other
   int64_t tokens;
 };
 
@@ -101,7 +101,11 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(ConvArgs p) {
   if (c >= p.C) return;
   if (p.heads_only && p.cu_q[blockIdx.x + 1] <= p.cu_q[blockIdx.x]) return;
   const int64_t t = p.heads_only ? p.cu_q[blockIdx.x] : blockIdx.x;
-  conv_token<T>(p, c, t, p.heads_only ? blockIdx.x : p.seq_of[t]);
+  const int b = p.heads_only ? blockIdx.x : p.seq_of[t];
+  conv_token<T>(p, c, t, b);
+  if (!p.heads_only) return;
+  // steps of no more tokens than requests: a request has more than one of them where others have none
+  for (int64_t u = t + max(p.taps - 1, 1), end = p.cu_q[b + 1]; u < end; ++u) conv_token<T>(p, c, u, b);
 }
 
 // The tokens that lie at least taps - 1 rows behind their portion's start need no slot: a thread takes four channels

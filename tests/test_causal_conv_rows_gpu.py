@@ -12,7 +12,8 @@ def i32(v):
     return torch.tensor(v, dtype=torch.int32, device=DEV)
 
 
-@pytest.mark.parametrize("lens", [[2], [8, 1, 7], [1, 2, 3, 0, 9, 16, 31], [1] * 5 + [65]])
+# the last three: no more tokens than requests, not all of which have one
+@pytest.mark.parametrize("lens", [[2], [8, 1, 7], [1, 2, 3, 0, 9, 16, 31], [1] * 5 + [65], [0, 0, 0, 0, 0, 6], [0, 2], [0, 9, 0, 1] + [0] * 9])
 @pytest.mark.parametrize("taps", [1, 2, 3, 4, 5, 8])
 @pytest.mark.parametrize("C,dtype", [(4, torch.float32), (260, torch.bfloat16), (1028, torch.float32), (1540, torch.bfloat16)])
 @pytest.mark.parametrize("act", [0, 1, 2])
