@@ -46,10 +46,11 @@ __device__ __forceinline__ double from_lane31(double x) {
   const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)u, 31), hi = __builtin_amdgcn_readlane((uint32_t)(u >> 32), 31);
   return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
-__device__ __forceinline__ float bf16_bits(uint16_t u) { return __uint_as_float((uint32_t)u << 16); }
 
 // ---- fp32 products on the 16-bit matrix instructions: a number is the sum of three of bf16, and the six largest of the nine products of two
-// such sums are added up in fp32 (off by less than 2^-25 of the product)
+// such sums are added up in fp32 (off by less than 2^-25 of the product).
+// Infinities, and numbers that bf16 rounds to one, have no parts.  They leave a result that is not finite, and then the workgroup walks its
+// tokens again as chunk_scan_kernel does: its rows and states are that kernel's, and cost twice.
 struct Parts { u32x4 p[3]; };      // eight numbers
 __device__ __forceinline__ void split2(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
   asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(h) : "v"(x), "v"(y));
@@ -84,7 +85,8 @@ struct PartsPlan {
   static constexpr int RB = 2 * D + 16, PLANE = PTOK * RB, PRB = 2 * PTOK + 16, PPLANE = PTOK * PRB;      // bytes
   static constexpr int Q = 0, K = 3 * PLANE, P = 6 * PLANE, F = P + 3 * PPLANE;                         // parts of q, of k, of the scores; doubles
   static constexpr int E = F + 2 * PTOK * 8;                                                             // floats from here on
-  static constexpr int NQ = E + 3 * PTOK * 4, PN = NQ + (MODE == EXPGATE ? NW * PTOK * 4 : 0), BYTES = PN + (MODE == EXPGATE ? 3 * PTOK * 4 : 0);
+  static constexpr int NQ = E + 3 * PTOK * 4, PN = NQ + (MODE == EXPGATE ? NW * PTOK * 4 : 0), END = PN + (MODE == EXPGATE ? 3 * PTOK * 4 : 0);
+  static constexpr int WALK = (int)(lds_floats<D, NW>() * sizeof(float)), BYTES = END > WALK ? END : WALK;
 };
 
 template <int MODE, typename T, int D, int NW>
@@ -179,7 +181,7 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
   const float *q_p = p.q + t0 * p.q_rs + hq * d, *k_p = p.k + t0 * p.k_rs + hq * d, *v_p = p.v + t0 * p.v_rs + h * vd;
   const float* g_p = MODE != EXPGATE ? p.g + t0 * p.g_rs + h * vd : nullptr;
   auto fetch = [&](int c0) {
-    const int last = min(PTOK, t1 - c0) - 1;      // 64 rows within 2 GB: 32 bits hold every size
+    const int last = min(PTOK, t1 - c0) - 1;      // 64 rows within 2 GB (serves): 32 bits hold every size
     if (emit) load_n(q, rows_of(q_p, (last * (int)p.q_rs + d) * 4), qk_at[0], left);
     load_n(k, rows_of(k_p, (last * (int)p.k_rs + d) * 4), qk_at[1], left);
     q_p += PTOK * p.q_rs;
@@ -265,6 +267,7 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
     v_p += PTOK * p.v_rs;
   };
   if constexpr (EARLY) fetch_v(t0);
+  float finite = 0.0f;                   // NaN once a result was not
   int second = 0;
   for (int c0 = t0; c0 < t1; c0 += PTOK, second ^= 1) {
     const int n = min(PTOK, t1 - c0);
@@ -394,10 +397,6 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
       }
     }
     // -------- the state behind the chunk
-    bool odd = false;                    // of this wavefront's values, is one not finite?
-#pragma unroll
-    for (int e = 0; e < 8; ++e) odd |= __builtin_amdgcn_classf(v[e >> 2][e & 3], 0x207);         // NaNs and infinities
-    odd = __any(odd);
     Parts vp;
     {
       f32x4 x[2];
@@ -425,33 +424,15 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
     __syncthreads();                     // the scores are there; the parts of q and k may be overwritten
     if (!emit) continue;
     // -------- what the chunk's own tokens contribute
-    // A score of a later token is 0, but 0 times an infinity or a NaN is not: with such a value in the chunk its terms are summed one
-    // by one, so that a token's row depends on the tokens up to it alone.
-    if (!odd) {
+    // A score of a later token is 0, but 0 times an infinity or a NaN is not: with such a value in the chunk the tokens are walked again.
 #pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        Parts P;
+    for (int a = 0; a < 2; ++a) {
+      Parts P;
 #pragma unroll
-        for (int t = 0; t < 3; ++t) P.p[t] = *reinterpret_cast<const u32x4*>(lds + L::P + t * L::PPLANE + (16 * a + lc) * L::PRB + 16 * lg);
-        o[a] = mma6(P, vp, o[a]);
-      }
-    } else {
-      f32x4 again[2];                    // not held until here
-      column8(again, v_p - (EARLY && MODE != SSD ? 2 : 1) * PTOK * p.v_rs, n - 1, p.v_rs, v_at);
-#pragma unroll 1
-      for (int s = 0; s < PTOK; ++s) {
-        const f32x4 x = s < 16 ? again[0] : again[1];
-        const float vs = __shfl(s & 2 ? (s & 1 ? x[3] : x[2]) : (s & 1 ? x[1] : x[0]), 16 * ((s >> 2) & 3) + lc, 64);
+      for (int t = 0; t < 3; ++t) P.p[t] = *reinterpret_cast<const u32x4*>(lds + L::P + t * L::PPLANE + (16 * a + lc) * L::PRB + 16 * lg);
+      o[a] = mma6(P, vp, o[a]);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int t = 4 * lg + row8(e);
-          float ps = 0.0f;
-#pragma unroll
-          for (int i = 0; i < 3; ++i)
-            ps += bf16_bits(*reinterpret_cast<const uint16_t*>(lds + L::P + i * L::PPLANE + t * L::PRB + 2 * score_place(s)));
-          if (s <= t) o[e >> 2][e & 3] = fmaf(ps, vs, o[e >> 2][e & 3]);
-        }
-      }
+      for (int r = 0; r < 4; ++r) finite = fmaf(o[a][r], 0.0f, finite);
     }
     const auto ro = rows_of(out_p, ((n - 1) * (int)p.out_rs + vd) * 4);
     uint32_t out_at = o_at;
@@ -460,6 +441,7 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
     if constexpr (MODE == EXPGATE) {
       // n_t . q_t of token tl: its scores and the normaliser ahead of the chunk
       const float nq = (tl < 16 ? spn[tl] : spn[PTOK + tl] + spn[2 * PTOK + tl]) + ahead * row_ahead;
+      finite = fmaf(nq, 0.0f, finite);
       const float under = 1.0f / (fmaxf(fabsf(nq), floor_t) + 1e-6f);
 #pragma unroll
       for (int e = 0; e < 8; ++e) store_1<float>(ro, (int)(out_at + row8(e) * o_step), o[e >> 2][e & 3] * __shfl(under, 4 * lg + row8(e), 64));
@@ -470,6 +452,30 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
       if constexpr (EARLY) fetch_v(c0 + PTOK);
     }
   }
+#pragma unroll
+  for (int i = 0; i < DT; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) finite = fmaf(S[i][r], 0.0f, finite);
+  if constexpr (MODE == EXPGATE) {
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) finite = fmaf(n0[i], 0.0f, finite);
+  }
+  int* again = reinterpret_cast<int*>(lds);
+  __syncthreads();                       // everybody is through with the last chunk
+  if (lane == 0) again[wv] = 0;
+  if (finite != 0.0f) again[wv] = 1;
+  __syncthreads();
+  int any = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) any |= again[w];
+  if (__builtin_expect(any, 0)) {
+    __syncthreads();
+    uint64_t args = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    int thread = threadIdx.x;
+    asm volatile("" : "+s"(args), "+v"(thread));       // formed anew from here on: kept until here, 10 to 20 registers in the loop above
+    chunk_walk<MODE, T, D, NW>(*reinterpret_cast<const Args*>(args), thread);
+    return;
+  }
   if (own) {
     const bool to_slot = emit && t1 == t_end, to_ws = MODE != EXPGATE && p.runs > 1 && p.pass == 1 && t1 < t_end;
     float* E = p.ws_state + (run0 + j) * d * vd;
@@ -479,8 +485,9 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
       for (int r = 0; r < 4; ++r) {
         const int row = 16 * i + 4 * lg + r;
         if (row < d) {
-          if (to_slot) S_g[(int64_t)row * vd + col] = S[i][r];
-          if (to_ws) E[(int64_t)row * vd + col] = S[i][r];
+          const float x = S[i][r];
+          if (to_slot) S_g[(int64_t)row * vd + col] = x;
+          if (to_ws) E[(int64_t)row * vd + col] = x;
         }
       }
     if (MODE == SSD && to_ws && tid == 0) p.ws_decay[run0 + j] = expf((float)run_lf);

@@ -175,7 +175,7 @@ __device__ __forceinline__ float silu(float z) {
 }
 
 template <int MODE, typename T, int D, int NW>
-__global__ __launch_bounds__(64 * NW, D <= 64 || (MODE == SSD && NW == 8) ? 4 : 1) void chunk_scan_kernel(Args p) {
+__device__ __forceinline__ void chunk_walk(const Args& p, int tid) {
   constexpr int DP = D + 4, DT = D / 16, CPL = D / (4 * NW), NP = DT < 2 ? 2 : DT;
   static_assert(CPL >= 1 && CPL <= 8 && NW % 4 == 0 && D * CP >= TOK * DP, "every lane stages whole channels");
   constexpr int BUF = 2 * TOK * DP + D * CP + D + 6 * TOK;
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(64 * NW, D <= 64 || (MODE == SSD && NW == 8) ? 4 : 
   float* snq = sred + NW * TOK;          // [2][NW][16] EXPGATE: shares of n . q
   float* sflag = snq + 2 * NW * TOK;     // [2][NW] GLA: this wavefront's channels decay out of the scores' range
   const int h = blockIdx.x, b = blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, lc = lane & 15, lg = lane >> 4;
+  const int lane = tid & 63, wv = tid >> 6, lc = lane & 15, lg = lane >> 4;
   int t0 = p.cu_q[b], t1 = p.cu_q[b + 1];
   const int t_end = t1, j = MODE != EXPGATE ? (int)blockIdx.z + (p.pass == 2 ? 1 : 0) : 0;
   if constexpr (MODE != EXPGATE) {
@@ -612,6 +612,11 @@ __global__ __launch_bounds__(64 * NW, D <= 64 || (MODE == SSD && NW == 8) ? 4 : 
       if (tid == 0) n_g[d] = m_run;
     }
   }
+}
+
+template <int MODE, typename T, int D, int NW>
+__global__ __launch_bounds__(64 * NW, D <= 64 || (MODE == SSD && NW == 8) ? 4 : 1) void chunk_scan_kernel(Args p) {
+  chunk_walk<MODE, T, D, NW>(p, threadIdx.x);
 }
 
 }  // namespace chunk_scan

@@ -22,6 +22,36 @@ def close(got, want, magnified=1.0):
     assert torch.isfinite(got).all() and off < TOL, off
 
 
+def state_space(xbc, z, dt, dt_bias, A_log, D, state, ints, lens, H, G, n, dv, tokens, runs=False):
+    """nv_ssd_scan_batch -> rows; the state in place."""
+    from byox_vllm_amd._C import check, lib, ptr, stream
+    from byox_vllm_amd.kernels import workspace
+    need = lib().nv_ssd_scan_workspace_bytes(len(lens), H, n, dv, max(lens)) if runs else 0
+    ws = workspace(need, torch.device(DEV, 0), "ssd_scan") if need else None
+    out = torch.empty(xbc.size(0), H * dv, device=DEV)
+    check(lib().nv_ssd_scan_batch(ptr(xbc), xbc.stride(0), ptr(z), z.stride(0), ptr(dt), dt.stride(0), ptr(dt_bias), ptr(A_log), ptr(D),
+                                  ptr(state), *map(ptr, ints), ptr(out), tokens, len(lens), H, G, n, dv, max(lens), ptr(ws), need, 2,
+                                  stream()), "nv_ssd_scan_batch")
+    return out
+
+
+def gated(proj, bias, state, ints, lens, H, d, dv, tokens, q_scale=1.0):
+    """nv_matrix_memory_batch with exponential gates, rows q | k | v | i | f -> rows; the state in place."""
+    from byox_vllm_amd import kernels
+    from byox_vllm_amd._C import check, lib, ptr, stream
+    cols, out = 2 * H * d + H * dv, torch.empty(proj.size(0), H * dv, device=DEV)
+    check(lib().nv_matrix_memory_batch(ptr(proj), proj.stride(0), 0, H * d, 2 * H * d, cols, cols + H, ptr(bias), None, ptr(state),
+                                       *map(ptr, ints), ptr(out), out.stride(0), tokens, len(lens), H, d, dv, kernels.MEM_EXPGATE, 0,
+                                       q_scale, 1.0, None, 0, 15.0, max(lens), 2, stream()), "nv_matrix_memory_batch")
+    return out
+
+
+def padded(*columns):
+    """Columns side by side, rows of a multiple of four numbers."""
+    x = torch.cat(columns, 1)
+    return torch.cat([x, x.new_zeros(x.size(0), -x.size(1) % 4)], 1).to(DEV)
+
+
 def both(run, lens, state):
     """``run(tokens, state, ints)`` -> rows; without the number of tokens and with it."""
     cu = [0]
@@ -111,3 +141,101 @@ def test_the_line_between_them():
         check(lib().nv_ssd_scan(*(a for x in data[:3] for a in (ptr(x), x.stride(0))), *map(ptr, data[3:]), ptr(s), *map(ptr, ints),
                                 ptr(sixteen), B, H, 1, n, dv, max(lens), None, 0, 2, stream()), "nv_ssd_scan")
         assert torch.equal(got, sixteen) != parts, lens
+
+
+def same(a, b):
+    return torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(0.0), b.nan_to_num(0.0))
+
+
+PLACES = [("q", float("inf")), ("k", float("-inf")), ("v", float("inf")), ("v", float("nan")), ("v", 3.4e38), ("k", 3.4e38), ("state", float("inf")), ("state", 3.4e38)]
+
+
+def numbers_without_parts(place, value, run, H, of):
+    """``run(tokens, put)`` -> rows [T, H, *], states [B, H, *] with ``put`` ahead of it: one number of one request's second head.  That
+    head's rows and states are those of the sixteen-token chunks, all others what they are without it."""
+    clean, dirty, sixteen = (run(t, p) for t, p in ((True, False), (True, True), (False, True)))
+    for (a, b, c), mine in zip(zip(clean, dirty, sixteen), of):
+        mine = torch.stack([torch.zeros_like(mine), mine], 1).view(b.size(0), H)
+        assert same(b[~mine], a[~mine]) and same(b[mine], c[mine]) and not same(b[mine], a[mine])
+    assert not all(x.isfinite().all() for x in dirty) or abs(value) < float("inf")
+
+
+@pytest.mark.parametrize("n,dv", [(64, 64), (128, 64), (128, 128), (32, 24)])
+@pytest.mark.parametrize("place,value", PLACES)
+def test_state_space_numbers_without_parts(n, dv, place, value):
+    torch.manual_seed(n + dv)
+    H, lens, hit = 2, [1, 97, 65, 40], 2
+    B, T, inner, at = len(lens), sum(lens), H * dv, sum(lens[:hit]) + 37
+    xbc, z, dt = (torch.randn(T, c, device=DEV) for c in (inner + 2 * H * n, inner, H))
+    head, state = [torch.randn(H, device=DEV) for _ in range(3)], torch.randn(B, H, n, dv, device=DEV)
+    cu = [sum(lens[:i]) for i in range(B + 1)]
+    ints = [i32(cu), i32([3] * B), i32(list(range(B)))]
+
+    def run(tokens, put):
+        x, s = xbc.clone(), state.clone()
+        if put and place == "state":
+            s[hit, 1, 3, 5] = value
+        elif put:
+            x[at, {"v": dv, "k": inner + n, "q": inner + H * n + n}[place] + 5] = value
+        rows = state_space(x, z, dt, *head, s, ints, lens, H, H, n, dv, T if tokens else 0)
+        return rows.view(T, H, dv), s
+    seq = torch.tensor([b for b, m in enumerate(lens) for _ in range(m)], device=DEV)
+    request = torch.arange(B, device=DEV) == hit
+    if place == "q":      # the state does not depend on it
+        clean, dirty = run(True, False), run(True, True)
+        assert same(dirty[1][request][:, 1], run(False, True)[1][request][:, 1]) and same(dirty[0][:, 0], clean[0][:, 0])
+        assert same(dirty[0][seq == hit][:, 1], run(False, True)[0][seq == hit][:, 1]) and not same(dirty[0], clean[0])
+        return
+    numbers_without_parts(place, value, run, H, (seq == hit, request))
+
+
+@pytest.mark.parametrize("d,dv", [(64, 64), (128, 64), (64, 128), (128, 128), (32, 24)])
+@pytest.mark.parametrize("place,value", PLACES)
+def test_exponential_gates_numbers_without_parts(d, dv, place, value):
+    from byox_vllm_amd import kernels
+    torch.manual_seed(d + dv)
+    H, lens, hit = 2, [1, 97, 65, 40], 2
+    B, T, at = len(lens), sum(lens), sum(lens[:hit]) + 37
+    proj = padded(torch.randn(T, 2 * H * d + H * dv + 2 * H))
+    state = torch.randn(B, H, kernels.matrix_memory_state_size(kernels.MEM_EXPGATE, d, dv), device=DEV)
+    cu = [sum(lens[:i]) for i in range(B + 1)]
+    ints = [i32(cu), i32([3] * B), i32(list(range(B)))]
+
+    def run(tokens, put):
+        x, s = proj.clone(), state.clone()
+        if put and place == "state":
+            s[hit, 1, 3 * dv + 5] = value
+        elif put:
+            x[at, {"q": d, "k": H * d + d, "v": 2 * H * d + dv}[place] + 5] = value
+        rows = gated(x, None, s, ints, lens, H, d, dv, T if tokens else 0)
+        return rows.view(T, H, dv), s
+    seq = torch.tensor([b for b, m in enumerate(lens) for _ in range(m)], device=DEV)
+    request = torch.arange(B, device=DEV) == hit
+    if place == "q":
+        clean, dirty, sixteen = run(True, False), run(True, True), run(False, True)
+        assert same(dirty[1][request][:, 1], sixteen[1][request][:, 1]) and same(dirty[0][:, 0], clean[0][:, 0])
+        assert same(dirty[0][seq == hit][:, 1], sixteen[0][seq == hit][:, 1]) and not same(dirty[0], clean[0])
+        return
+    numbers_without_parts(place, value, run, H, (seq == hit, request))
+
+
+@pytest.mark.parametrize("place", ["k", "v", "state"])
+def test_infinities_in_runs_side_by_side(place):
+    """A run that meets one is walked again; what it leaves reaches the runs behind it."""
+    torch.manual_seed(7)
+    H, n, dv, lens = 2, 64, 64, [300, 257]
+    T, inner = sum(lens), H * dv
+    xbc, z, dt = (torch.randn(T, c, device=DEV) for c in (inner + 2 * H * n, inner, H))
+    head, state = [torch.randn(H, device=DEV) - 2.0 for _ in range(3)], torch.randn(2, H, n, dv, device=DEV)
+    if place == "state":
+        state[0, 0, 5, 7] = float("inf")
+    else:
+        xbc[120, 7 if place == "v" else inner + 5] = float("inf")
+    results = []
+    for tokens in (T, 0):
+        s = state.clone()
+        results.append((state_space(xbc, z, dt, *head, s, [i32([0, 300, 557]), i32([3, 3]), i32([0, 1])], lens, H, H, n, dv, tokens, True), s))
+    for got, want in zip(*results):
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf()) and not want.isfinite().all()
+        assert torch.equal(got[got.isinf()], want[want.isinf()])
+        close(torch.where(want.isfinite(), got, 0.0), torch.where(want.isfinite(), want, 0.0))
