@@ -49,8 +49,12 @@ __device__ __forceinline__ double from_lane31(double x) {
 
 // ---- fp32 products on the 16-bit matrix instructions: a number is the sum of three of bf16, and the six largest of the nine products of two
 // such sums are added up in fp32 (off by less than 2^-25 of the product).
-// Infinities, and numbers that bf16 rounds to one, have no parts.  They leave a result that is not finite, and then the workgroup walks its
-// tokens again as chunk_scan_kernel does: its rows and states are that kernel's, and cost twice.
+// The third part of a number below 2^-110 is below the least number of bf16, so q, k and the values enter times SCALE, which brings the last
+// bit of every number of fp32 above that; the state and the scores are kept times SCALE^2 and what they form times SCALE^3.  Rows and states of
+// 97 tokens, 128 x 64, positive numbers whose parts are as large as can be: 0.6 to 2.7e-7 of the norm off float64, wherever in fp32's range.
+// Infinities and numbers too large for that have no parts.  They leave a result that is not finite, and then the workgroup walks its tokens
+// again as chunk_scan_kernel does: its rows and states are that kernel's, and cost twice.
+constexpr float SCALE = 16777216.0f, SCALE2 = SCALE * SCALE, SCALE3 = SCALE2 * SCALE;      // 2^24
 struct Parts { u32x4 p[3]; };      // eight numbers
 __device__ __forceinline__ void split2(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
   asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(h) : "v"(x), "v"(y));
@@ -146,7 +150,7 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
 #pragma unroll
     for (int i = 0; i < DT; ++i)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) S[i][r] = load_1(r_s, s_at + (16 * i + r) * vd * 4);
+      for (int r = 0; r < 4; ++r) S[i][r] = SCALE2 * load_1(r_s, s_at + (16 * i + r) * vd * 4);
   }
   if (MODE != EXPGATE && p.pass == 2) {       // what the runs ahead left: S <- D_i S + E_i in turn
     for (int64_t run = run0; run < run0 + j; ++run) {
@@ -155,7 +159,7 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
 #pragma unroll
       for (int i = 0; i < DT; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) S[i][r] = f * S[i][r] + load_1(r_s, s_at + (16 * i + r) * vd * 4);
+        for (int r = 0; r < 4; ++r) S[i][r] = f * S[i][r] + SCALE2 * load_1(r_s, s_at + (16 * i + r) * vd * 4);
     }
   }
   double run_lf = 0.0;                   // SSD: the run's log decay
@@ -302,13 +306,13 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
     float nq = 0.0f;
 #pragma unroll
     for (int i = 0; i < CPL; ++i) {
-      q[i] *= p.q_scale;
-      k[i] *= p.k_scale;
+      q[i] *= SCALE * p.q_scale;
+      k[i] *= SCALE * p.k_scale;
       if constexpr (MODE == EXPGATE) {
         nq += q[i] * n0[i];
         float a, c;
         rows_pair16(lanes_sum<16>(k[i] * w), a, c);
-        n0[i] = whole * n0[i] + (a + c);
+        n0[i] = whole * n0[i] + (a + c) * (1.0f / SCALE);
       }
     }
     if (emit) put(L::Q, q);
@@ -330,7 +334,7 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
         sf[PTOK + tl] = in_gate;
       }
       sf[tl] = rowf;
-      sf[2 * PTOK + tl] = w;
+      sf[2 * PTOK + tl] = SCALE * w;
     }
     m_run = m_end;
     __syncthreads();
@@ -414,7 +418,7 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
         S[i] = mma6(columns16(i), vw, S[i]);
         if (i % 2 == 1) __builtin_amdgcn_sched_barrier(0);
       }
-      vp = split8(v[0], v[1]);
+      vp = split8(v[0] * SCALE, v[1] * SCALE);
     }
     if constexpr (MODE != EXPGATE && !EARLY) {
       if (emit) column8(gate, g_p, n - 1, p.g_rs, g_at);
@@ -432,7 +436,10 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
       for (int t = 0; t < 3; ++t) P.p[t] = *reinterpret_cast<const u32x4*>(lds + L::P + t * L::PPLANE + (16 * a + lc) * L::PRB + 16 * lg);
       o[a] = mma6(P, vp, o[a]);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) finite = fmaf(o[a][r], 0.0f, finite);
+      for (int r = 0; r < 4; ++r) {
+        finite = fmaf(o[a][r], 0.0f, finite);
+        o[a][r] *= 1.0f / SCALE3;
+      }
     }
     const auto ro = rows_of(out_p, ((n - 1) * (int)p.out_rs + vd) * 4);
     uint32_t out_at = o_at;
@@ -440,7 +447,7 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
     out_p += PTOK * p.out_rs * 4;
     if constexpr (MODE == EXPGATE) {
       // n_t . q_t of token tl: its scores and the normaliser ahead of the chunk
-      const float nq = (tl < 16 ? spn[tl] : spn[PTOK + tl] + spn[2 * PTOK + tl]) + ahead * row_ahead;
+      const float nq = (tl < 16 ? spn[tl] : spn[PTOK + tl] + spn[2 * PTOK + tl]) * (1.0f / SCALE2) + ahead * (1.0f / SCALE) * row_ahead;
       finite = fmaf(nq, 0.0f, finite);
       const float under = 1.0f / (fmaxf(fabsf(nq), floor_t) + 1e-6f);
 #pragma unroll
@@ -485,7 +492,7 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
       for (int r = 0; r < 4; ++r) {
         const int row = 16 * i + 4 * lg + r;
         if (row < d) {
-          const float x = S[i][r];
+          const float x = S[i][r] * (1.0f / SCALE2);
           if (to_slot) S_g[(int64_t)row * vd + col] = x;
           if (to_ws) E[(int64_t)row * vd + col] = x;
         }

@@ -4,6 +4,8 @@ a request, against the chunks of sixteen, which they take where they know nothin
 import pytest
 import torch
 
+import chunk_parts_cases as C
+
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 LENS = [1, 31, 32, 33, 63, 64, 65, 97]
@@ -143,11 +145,48 @@ def test_the_line_between_them():
         assert torch.equal(got, sixteen) != parts, lens
 
 
+# powers of two that q, k and v are multiplied by: numbers whose second and third parts would lie below the range of bf16
+SCALES = [(0, 0, 0), (110, -118, 0), (-118, 60, 0), (0, 0, -119), (100, -70, -60)]
+
+
+@pytest.mark.parametrize("scales", SCALES)
+@pytest.mark.parametrize("weighted", [False, True])
+def test_state_space_as_close_as_fp32(scales, weighted):
+    q, k, v, state, dt, bias, A_log = C.state_space_case(weighted)
+    a, b, c = (2.0 ** e for e in scales)
+    q, k, v, state = q * a, k * b, v * c, state * b * c
+    step, lf = C.steps_and_decays(dt, bias, A_log)
+    want, end = C.recurrence(q, k, v, state, lf, step, False)
+    T, (d, dv) = q.size(0), state.shape
+    z, s = torch.ones(T, dv, device=DEV), state.to(DEV).view(1, 1, d, dv).clone()
+    got = state_space(padded(v, k, q), z, dt.view(T, 1).to(DEV), bias.view(1).to(DEV), A_log.view(1).to(DEV), torch.zeros(1, device=DEV), s,
+                      [i32([0, T]), i32([5]), i32([0])], [T], 1, 1, d, dv, T)
+    errors = C.error(got, want * torch.nn.functional.silu(torch.ones((), dtype=torch.float64))), C.error(s.view(d, dv), end)
+    assert max(errors) < C.BOUND, errors
+
+
+@pytest.mark.parametrize("scales", SCALES)
+@pytest.mark.parametrize("weighted", [False, True])
+def test_exponential_gates_as_close_as_fp32(scales, weighted):
+    q, k, v, state, n, m, i, f, cap = C.gates_case(weighted)
+    a, b, c = (2.0 ** e for e in scales)
+    q, k, v, state, n = q * a, k * b, v * c, state * b * c, n * b
+    gate, lf = C.capped_gates(i, f, cap)
+    want, end, n_end, m_end = C.recurrence(q, k, v, state, lf, gate, True, m.double(), n)
+    T, (d, dv) = q.size(0), state.shape
+    s = torch.cat([state.reshape(-1), n, m.view(1)]).to(DEV).view(1, 1, -1).clone()
+    got = gated(padded(q, k, v, i.view(T, 1), f.view(T, 1)), None, s, [i32([0, T]), i32([5]), i32([0])], [T], 1, d, dv, T)
+    s = s.view(-1)
+    errors = C.error(got, want), C.error(s[:d * dv].view(d, dv), end), C.error(s[d * dv:-1], n_end)
+    assert max(errors) < C.BOUND and abs(s[-1].item() - m_end.item()) < 2.0 ** -20, errors
+
+
 def same(a, b):
     return torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(0.0), b.nan_to_num(0.0))
 
 
-PLACES = [("q", float("inf")), ("k", float("-inf")), ("v", float("inf")), ("v", float("nan")), ("v", 3.4e38), ("k", 3.4e38), ("state", float("inf")), ("state", 3.4e38)]
+PLACES = [("q", float("inf")), ("k", float("-inf")), ("v", float("inf")), ("v", float("nan")), ("v", 3.4e38), ("k", 3.4e38), ("q", 1e34),
+          ("state", float("inf")), ("state", 3.4e38)]
 
 
 def numbers_without_parts(place, value, run, H, of):
