@@ -185,7 +185,7 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 2 : NW == 8 ? 4 : 3) void chunk_p
   const float *q_p = p.q + t0 * p.q_rs + hq * d, *k_p = p.k + t0 * p.k_rs + hq * d, *v_p = p.v + t0 * p.v_rs + h * vd;
   const float* g_p = MODE != EXPGATE ? p.g + t0 * p.g_rs + h * vd : nullptr;
   auto fetch = [&](int c0) {
-    const int last = min(PTOK, t1 - c0) - 1;      // 64 rows within 2 GB (serves): 32 bits hold every size
+    const int last = min(PTOK, t1 - c0) - 1;      // 64 rows lie within 2 GB (serves): 32 bits hold every size
     if (emit) load_n(q, rows_of(q_p, (last * (int)p.q_rs + d) * 4), qk_at[0], left);
     load_n(k, rows_of(k_p, (last * (int)p.k_rs + d) * 4), qk_at[1], left);
     q_p += PTOK * p.q_rs;

@@ -4,7 +4,7 @@
 
 template <typename TO, int EPI, bool FAR_UPS = false>
 static hipError_t linear_deep_as(const LinArgs& p, int64_t total_rows, int batch, hipStream_t s) {
-  const auto job = linear_job<bf16_t, TO, EPI, FAR_UPS>(p, batch);
+  const auto job = linear_job<TO, EPI, FAR_UPS>(p, batch);
   return launch_stream_deep(job, linear_job_tiles(p, job.nt, total_rows, batch), s);
 }
 template <typename TO>

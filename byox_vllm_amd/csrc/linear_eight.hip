@@ -4,7 +4,7 @@
 
 template <typename TO, int EPI>
 static hipError_t linear_eight_as(const LinArgs& p, int64_t total_rows, int batch, hipStream_t s) {
-  const auto job = linear_job<bf16_t, TO, EPI>(p, batch);
+  const auto job = linear_job<TO, EPI>(p, batch);
   return launch_stream_tiles(job, linear_job_tiles(p, job.nt, total_rows, batch), s);
 }
 template <typename TO>

@@ -36,9 +36,9 @@ __device__ __forceinline__ u32x4 pack8(const float* v) {
   return u32x4{pack2<bf16_t>(v[0], v[1]), pack2<bf16_t>(v[2], v[3]), pack2<bf16_t>(v[4], v[5]), pack2<bf16_t>(v[6], v[7])};
 }
 
-template <typename TT, typename TO, int EPI, bool FAR_UPS = false>     // FAR_UPS: a gated product's ups lie 4 GiB and more from their gates
+template <typename TO, int EPI, bool FAR_UPS = false>     // FAR_UPS: a gated product's ups lie 4 GiB and more from their gates
 struct LinearJob {
-  typedef TT T;
+  typedef bf16_t T;
   static constexpr int BM = STREAM_BM, MT = 8, NT = 4;              // four wavefronts along the columns
   static constexpr bool GLU = EPI == EPI_GLU, PAIRED = sizeof(TO) == 2;
   typedef std::conditional_t<PAIRED, StreamPaired, StreamNatural> Order;
@@ -336,9 +336,9 @@ inline bool linear_four_wavefronts(const LinArgs& p, int epi, bool out_16bit) {
   return p.K >= from[what][(stream_vec(p, out_16bit) ? 0 : 2) + (p.bias ? 1 : 0)];
 }
 
-template <typename T, typename TO, int EPI, bool FAR_UPS = false>
-LinearJob<T, TO, EPI, FAR_UPS> linear_job(const LinArgs& p, int batch) {
-  typedef LinearJob<T, TO, EPI, FAR_UPS> Job;
+template <typename TO, int EPI, bool FAR_UPS = false>
+LinearJob<TO, EPI, FAR_UPS> linear_job(const LinArgs& p, int batch) {
+  typedef LinearJob<TO, EPI, FAR_UPS> Job;
   const int nt = (p.N + Job::NOUT - 1) / Job::NOUT;
   return Job{p, p.K, p.group_off ? batch : 0, batch, nt, stream_vec(p, sizeof(TO) == 2)};
 }

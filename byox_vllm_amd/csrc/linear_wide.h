@@ -135,7 +135,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void linear_wide_kernel(LinArgs p,
   typedef bf16_t T;
   constexpr bool GLU = EPI == EPI_GLU;
   constexpr int NW = WM * WN, BM = 32 * MT * WM, BN = 64 * WN, NOUT = GLU ? BN / 2 : BN;
-  constexpr int PER = 16 / sizeof(T), BK = 8 * PER;                 // numbers per 16-byte piece; per K block
+  constexpr int PER = 8, BK = 8 * PER;                              // numbers per 16-byte piece; per K block
   constexpr int AG = BM / 8 / NW, WG = BN / 8 / NW;                 // DMA instructions (8 rows each) per wavefront
   static_assert(AG >= 1 && WG >= 1 && AG * 8 * NW == BM && WG * 8 * NW == BN, "the tile splits into whole DMA instructions");
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];

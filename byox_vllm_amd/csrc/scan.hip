@@ -9,8 +9,8 @@
 // mingru_scan:  z = sigmoid(zl),  S = (1 - z) S + z c(u),  c(u) = u + 1/2 for u >= 0 and sigmoid(u) below,
 //               out = S * silu(g): the minimal gated recurrent unit, whose gates read the current token only.
 // ssd_scan:     per head, S [N, P]:  S = exp(-exp(A_log) dt) S + dt B x^T,  y = S^T C + D x,  dt = softplus(raw + bias);
-//               out = y * silu(z): the selective state-space recurrence of Mamba-2.  Prompts run sixteen tokens at a time on
-//               the matrix cores (chunk_scan.h); single tokens and sizes that kernel does not serve walk token by token.
+//               out = y * silu(z): the selective state-space recurrence of Mamba-2.  Prompts run sixteen or thirty-two tokens at a
+//               time on the matrix cores (chunk_scan.h, chunk_parts.h); single tokens and sizes that kernel does not serve walk token by token.
 #include <algorithm>
 
 #include "chunk_scan.h"

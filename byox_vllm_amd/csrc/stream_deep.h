@@ -1,5 +1,5 @@
 // Products of many rows in 16 bits: tiles of 256 x 256 outputs by four wavefronts of 128 x 128 each, their K blocks one stream (the tiles
-// and their order are those of stream_tiles.h, which keeps fp32).
+// and their order are those of stream_tiles.h, which keeps the products whose results take long to form).
 //
 // What bounds it: the matrix cores and their power.  The eight wavefronts of 128 x 64 that this form replaced read 192 KB of LDS per K
 // block of 64 for 128 KB here, asked for a block about half a block's products before it was waited for, and took 852 us at 8192 x 8192

@@ -19,7 +19,7 @@
 // (at the end of everything, its column panels come from memory again: sixteen experts in bf16 1450 us against 1418).
 //
 // Job (what is multiplied and what becomes of it) provides:
-//   T, Order (how W lies, below; here in rows), NSTORE, K (elements, two blocks of 128 bytes at least)
+//   T (stream_deep.h: what is multiplied), Order (how W lies, below; here in rows), NSTORE, K (elements, two blocks of 128 bytes at least)
 //   int count(lane)                       how many tiles there are
 //   StreamTile find(tile, lane)           which rows and columns the thread's tile has (every thread of a wavefront calls it)
 //   const void* a_base(tile); uint32_t a_row(tile, r); uint32_t a_stride()      row r of the tile's A rows (those past the end
@@ -40,7 +40,7 @@ constexpr int STREAM_LIST = 512;      // tiles of one workgroup at most
 constexpr int STREAM_BM = 256, STREAM_BN = 256;
 constexpr int STREAM_BUFFER = (STREAM_BM + STREAM_BN) * 128;      // a K block of both
 
-__device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x4 c, bf16_t) {
+__device__ __forceinline__ f32x4 stream_mma(const u32x4& a, const u32x4& b, f32x4 c) {
   return mfma16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c);
 }
 
@@ -100,7 +100,6 @@ __device__ __forceinline__ int stream_lane() {
 template <typename Job>
 __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  typedef typename Job::T T;
   constexpr int WN = 4, WM = 8 / WN, MT = STREAM_BM / 16 / WM, NT = STREAM_BN / 16 / WN;
   typedef typename Job::Order Order;
   constexpr int BM = STREAM_BM, BN = STREAM_BN, BO = STREAM_BUFFER;     // BO: bytes of one buffer
@@ -195,7 +194,7 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
   };
   clear();
 
-  const int blocks = job.K / (128 / (int)sizeof(T));
+  const int blocks = job.K / 64;
   StreamTile at = listed(0), ahead = at;
   point(at);
   lanes();
@@ -223,7 +222,7 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
       fragments(bo, 1, wat, aat);
 #pragma unroll
       for (int m = 0; m < P; ++m) {
-        acc[m % NT][m / NT] = stream_mma(wf[0][m % NT], af[0][m / NT], acc[m % NT][m / NT], T{});
+        acc[m % NT][m / NT] = stream_mma(wf[0][m % NT], af[0][m / NT], acc[m % NT][m / NT]);
         if (m == 0) __builtin_amdgcn_sched_barrier(0);       // or the first product waits for the first of these reads
         if (m < R) read(wat, aat, m, 1);
         __builtin_amdgcn_sched_barrier(0);
@@ -246,7 +245,7 @@ __global__ __launch_bounds__(512, 2) void stream_tiles_kernel(Job job) {
       constexpr int EVERY = P / D;
 #pragma unroll
       for (int m = 0; m < P; ++m) {
-        acc[m % NT][m / NT] = stream_mma(wf[1][m % NT], af[1][m / NT], acc[m % NT][m / NT], T{});
+        acc[m % NT][m / NT] = stream_mma(wf[1][m % NT], af[1][m / NT], acc[m % NT][m / NT]);
         if (m == 0) __builtin_amdgcn_sched_barrier(0);       // or the first product waits for the first of these reads
         if (m < R) read(wat, aat, m, 0);
         if (m % EVERY == 0 && m / EVERY < D) fill(bo, m / EVERY);
