@@ -173,47 +173,45 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_split_kernel(LinArgs p, i
   }
 
   // -------- An infinity, a NaN and a number of 2^88 and more have no such parts and leave a result that is not finite, as a sum of 2^48 and
-  // more does: these products are formed again as they are.
-  float finite = 0.0f;
+  // more does: these results, and only these, are formed again from the numbers as they are, so that no result depends on other rows and columns.
+  // 3135 rows 1024 -> 4416: 178 us, 233 with an infinity in one row, 695 where no result can be kept; 2048 -> 1024 80, 211, 354.
+  constexpr float BACK = 1.0f / (SCALE * SCALE);
+  auto odd = [&](int j, int i) {
+    float finite = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) finite = fmaf(acc[j][i][r], 0.0f, finite);
+    return finite != 0.0f;
+  };
+  bool any = false;
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int i = 0; i < MT; ++i) any |= odd(j, i);
+  if (__builtin_expect(__any(any), 0)) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) finite = fmaf(acc[j][i][r], 0.0f, finite);
-  float back = 1.0f / (SCALE * SCALE);
-  if (__any(finite != 0.0f)) {
-    back = 1.0f;
-    const float *ap[MT], *wp[2];
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int i = 0; i < MT; ++i) ap[i] = a_row(32 * (MT * wm + i) + fr) + 4 * fh;
+      for (int i = 0; i < MT; ++i) {
+        f32x16 again = acc[j][i];
+        if (__any(odd(j, i))) {
+          const float *ap = a_row(32 * (MT * wm + i) + fr) + 4 * fh, *wp = w_row(w_tile(j) + fr) + 4 * fh;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) wp[j] = w_row(w_tile(j) + fr) + 4 * fh;
+          for (int r = 0; r < 16; ++r) again[r] = 0.0f;
+#pragma unroll 1
+          for (int k = 0; k < p.K; k += 8)
+            again = mma32(*reinterpret_cast<const u32x4*>(wp + k), *reinterpret_cast<const u32x4*>(ap + k), again, 0.0f);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[j][i][r] = __builtin_isfinite(acc[j][i][r]) ? acc[j][i][r] * BACK : again[r];
+      }
+  } else {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[j][i][r] = 0.0f;
-#pragma unroll 1
-    for (int k = 0; k < p.K; k += 8) {
-      u32x4 w[2], a[MT];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) w[j] = *reinterpret_cast<const u32x4*>(wp[j] + k);
-#pragma unroll
-      for (int i = 0; i < MT; ++i) a[i] = *reinterpret_cast<const u32x4*>(ap[i] + k);
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[j][i] = mma32(w[j], a[i], acc[j][i], 0.0f);
-    }
+        for (int r = 0; r < 16; ++r) acc[j][i][r] *= BACK;
   }
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[j][i][r] *= back;
   wide_results<float, TO, EPI, MT>(p, acc, at.z, mbase + 32 * MT * wm, hi, n0, wn, fr, fh);
 }
 

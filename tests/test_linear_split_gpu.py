@@ -54,3 +54,22 @@ def test_values_without_parts(tile, monkeypatch):
     finite = want.isfinite()
     finite[:, 269] = False      # 1e38 times normal values: its own scale
     assert (got - want)[finite].abs().max() < 256 * 2.0 ** -24 * 16
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 1e30, 2.0 ** 60])
+def test_results_without_parts_leave_the_others_alone(tile, value, monkeypatch):
+    """A row of x and a column of results that are formed again: every other result is the same to the last bit."""
+    from byox_vllm_amd import kernels
+    monkeypatch.setenv("NV_LINEAR_TILE", tile)
+    torch.manual_seed(4)
+    x, w = torch.randn(300, 256, device=DEV), torch.randn(270, 256, device=DEV)
+    clean = kernels.linear(x, w)
+    x[77, 9], w[130, 200] = value, value
+    got, rows, columns = kernels.linear(x, w), torch.arange(300) != 77, torch.arange(270) != 130
+    assert torch.equal(got[rows][:, columns], clean[rows][:, columns])
+    want = (x.double() @ w.double().t()).float()
+    for a, b in ((got[77], want[77]), (got[:, 130], want[:, 130])):
+        assert torch.equal(a.isfinite(), b.isfinite())
+        a, b = (torch.where(b.isfinite(), c, 0.0) for c in (a, b))
+        assert (a - b).abs().max() <= 256 * 2.0 ** -24 * b.abs().max()      # 256 additions, one of them next to all of the sum
