@@ -8,7 +8,8 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-@pytest.mark.parametrize("T", [1, 5, 2048, 2049, 2051])
+# the line between the two forms: 1024 tokens below 32 rotated numbers, 4096 without one
+@pytest.mark.parametrize("T", [1, 5, 1024, 1025, 2048, 2049, 2051, 4096, 4097])
 @pytest.mark.parametrize("H,d,r,rot", [(1, 4, 8, 8), (3, 32, 16, 8), (4, 96, 32, 32), (5, 96, 32, 32), (9, 100, 28, 24), (2, 64, 0, 0)])
 @pytest.mark.parametrize("interleaved", [False, True])
 @pytest.mark.parametrize("dtype,out_dtype", [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.float32, torch.float32)])
