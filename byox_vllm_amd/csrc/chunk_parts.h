@@ -12,7 +12,7 @@
 //     which makes them the operand as they are.
 //   * The three tiles of scores on and below the diagonal are three wavefronts', who form k q^T: a lane then holds four keys of one query.
 // Measured: whole fp32 layers of 4 requests of about 1000 tokens, 32 heads of 128 x 64 433 and 380 us, 8 requests of 2048 tokens in bf16 1250 and
-// 1040; exponential gates, 3 requests of 1500 tokens, 8 heads of 128 x 128 458 and 318, 64 of about 256 tokens, 64 x 128 228 and 215.  What
+// 1040; exponential gates, 3 requests of 1500 tokens, 8 heads of 128 x 128 458 and 318, 64 of about 256 tokens, 64 x 128 229 and 210.  What
 // bounds it now: waiting, 60 % of the wavefronts' time with two or three to a SIMD, at the chunk's two barriers and for its rows.
 // Channel decays in this form (exponents taken from the chunk's middle, per-channel factors around the products) were 5 % slower than there:
 // their second form for chunks that decay far takes the registers that keep two workgroups on a CU.

@@ -113,7 +113,8 @@ __global__ __launch_bounds__(256) void causal_conv_kernel(ConvArgs p) {
 // access.  The others, and the slots, are those of the first 4 num_seqs workgroups along x, a channel to a thread.  C % 4 == 0, aligned rows.
 // What bounded it: a token's row, its request and that one's first token, asked for in turn eight times over, and the slots' tokens in a launch
 // of their own ahead (6 us).  Now a tile's rows are asked for at once.  SiLU into fp32, taps of 4, 2304 channels: 4 requests of 3135 tokens
-// together 34.4 and 20.5 us, 8 of 2048 116.7 and 86.3 (3.5 TB/s), 64 single tokens beside a piece of 512 16.4 and 9.9.
+// together 34.4 and 20.5 us, 8 of 2048 116.7 and 86.3 (3.5 TB/s), 64 single tokens beside a piece of 512 16.4 and 9.9; taps of 6, 100 of about
+// 150, 512 channels 38.2 and 31.8, of 8, 8 of 3 17.4 and 8.7.
 constexpr int CONV_TT = 8;
 
 template <typename T, int TAPS>      // at least p.taps
